@@ -1,0 +1,363 @@
+// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float for more than 16 rows, on the bfloat16 matrix
+// instruction (v_mfma_f32_32x32x16_bf16): the 32-bit path's product of prompts and large batches.
+//
+// A float is exactly the sum of three bfloat16 numbers (8 + 8 + 8 significant bits; each is the rest of the
+// one before, rounded to nearest, so the rests have either sign).  Of the nine partial products of two such
+// sums the six that reach 2^-18 of the largest are taken, small ones first, each exact in the instruction's
+// float sums; the three left out are below 2^-26 of the product they belong to, a quarter of the rounding
+// that a float product itself has.  Six bfloat16 products take 6 / 16 of the matrix cores' time of one on
+// the float instruction (2.5 PFLOP/s against 157 TFLOP/s), and the sums have fewer roundings: at 2,048 rows and
+// K = 18,944 the result is 5.4e-7 off the exact one where the float instruction's was 2.5e-6 (3,584: 4.8e-7 and 1.1e-6).
+//
+// What is split where: the rows of A once, by a pass of its own, into the order in which the product reads
+// them (fs_split_kernel: 4 bytes read and 6 written per value); W, which may be most of the GPU's memory,
+// stays float and is split in registers by the wave that owns its columns, from the matrix-core ordered copy
+// that the few-row product streams as well.  A wave owns 32 or 64 columns and all the rows of its work-group
+// (up to 128): 44 vector instructions per 32 columns beside 6 matrix instructions per 32 x 32 block and 16 k.
+//
+// Per step of 16 k a work-group holds 3 KB of A per 32 rows and 2 KB of W per 32 columns of a wave in LDS, in the
+// layout the fragments are read in (a fragment is 1 KB, lane after lane: no bank conflicts), fetched one or two
+// steps ahead by global_load_lds; one barrier per step.  What bounds it: the matrix cores are busy half of the time
+// (197 TFLOP/s are 1.18 PFLOP/s of bfloat16 products), the rest is the splitting of W, which does not overlap with them,
+// and LDS reads (a fragment of A feeds six products of a column block).
+//
+// One output element is summed in one fixed order whatever the number of rows or the tile: k in segments of
+// FS_SEG at absolute k, within a segment steps of 16 upwards with the six partial products of a step in one
+// order, the segments' sums added in ascending order.  Few tiles (few rows of a narrow matrix) are spread
+// over the GPU by segments, whose sums a second kernel adds in the same order.
+//
+// Values that are not finite, and those so large that they round to infinity as bfloat16, make the split
+// itself infinity minus infinity: an element that comes out as NaN is computed again with plain float
+// multiply-adds, so infinities and NaN give what they give there.
+#include "common.h"
+
+typedef __bf16 fs_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 fs_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float fs_f32x2 __attribute__((ext_vector_type(2)));
+typedef float fs_f32x16 __attribute__((ext_vector_type(16)));
+
+#define FS_STEP 16
+#define FS_SEG 2048                      // k per segment
+#define FS_SEG_STEPS (FS_SEG / FS_STEP)
+#define FS_WAVES 4
+#define FS_CUS 256
+
+// two floats as two bfloat16, rounded to nearest even, and what is left of each
+__device__ __forceinline__ uint32_t fs_take(float& a, float& b) {
+    const fs_f32x2 v = {a, b};
+    const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, fs_bf16x2));
+    a -= __uint_as_float(p << 16);
+    b -= __uint_as_float(p & 0xffff0000u);
+    return p;
+}
+// eight floats as three times eight bfloat16
+__device__ __forceinline__ void fs_split8(float4 x, float4 y, uint4& hi, uint4& mid, uint4& lo) {
+    hi = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
+    mid = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
+    lo = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
+}
+
+// A as the product reads it: [ceil(M/32) blocks][ceil(K/16) steps][3 parts][64 lanes][8 values], lane l the row
+// l % 32 of the block at k = 16 step + 8 (l / 32) .. + 8; zero beyond M and K.  A wave per (block, step).
+__global__ __launch_bounds__(256) void fs_split_kernel(const float* __restrict__ A, uint4* __restrict__ out, int M, int K, int lda,
+                                                       int steps, int vec) {
+    const int lane = threadIdx.x & 63, step = blockIdx.x * 4 + (threadIdx.x >> 6), block = blockIdx.y;
+    if (step >= steps) return;
+    const int row = block * 32 + (lane & 31), k = step * FS_STEP + 8 * (lane >> 5);
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f), y = x;
+    if (row < M) {
+        const float* p = A + (size_t)row * lda + k;
+        if (vec && k + 8 <= K) {
+            x = *reinterpret_cast<const float4*>(p);
+            y = *reinterpret_cast<const float4*>(p + 4);
+        } else {
+            x.x = k < K ? p[0] : 0.f;
+            x.y = k + 1 < K ? p[1] : 0.f;
+            x.z = k + 2 < K ? p[2] : 0.f;
+            x.w = k + 3 < K ? p[3] : 0.f;
+            y.x = k + 4 < K ? p[4] : 0.f;
+            y.y = k + 5 < K ? p[5] : 0.f;
+            y.z = k + 6 < K ? p[6] : 0.f;
+            y.w = k + 7 < K ? p[7] : 0.f;
+        }
+    }
+    uint4 hi, mid, lo;
+    fs_split8(x, y, hi, mid, lo);
+    uint4* o = out + ((size_t)block * steps + step) * 192 + lane;
+    o[0] = hi;
+    o[64] = mid;
+    o[128] = lo;
+}
+
+// 16 bytes per lane from memory straight into LDS at lds_base + 16 * lane.  Written as assembly so that the
+// compiler does not make every LDS read wait for it: the loads are waited for where FS_LANDED says so.
+__device__ __forceinline__ void fs_load_to_lds(const void* g, void* lds_base) {
+    const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds_base);
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "s"(base), "v"(g)
+        : "memory");
+}
+// at most N of this wave's loads are still on their way, and its LDS reads are done
+#define FS_LANDED(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory")
+
+// one element (or one segment of it) with float multiply-adds, from the values themselves
+__device__ float fs_plain(const float* __restrict__ A, const float* __restrict__ Ws, int lda, int steps, int m, int n, int k0, int k1) {
+    float sum = 0.f;
+    for (int k = k0; k < k1 && sum == sum; ++k)
+        sum = fmaf(A[(size_t)m * lda + k],
+                   Ws[(((size_t)(n >> 4) * steps + (k >> 4)) * 64 + ((k >> 2) & 3) * 16 + (n & 15)) * 4 + (k & 3)], sum);
+    return sum;
+}
+
+// MB blocks of 32 rows, FS_WAVES waves side by side with NB blocks of 32 columns each.  PARTS: blockIdx.y is a segment
+// of K and C the workspace [segments][M][N]; else the whole K, C holding the sum of the segments so far (a lane reads
+// and writes its own elements only).
+// Work-groups of one XCD (every eighth in the order of their ids) take the row tiles of one column tile in turn, so
+// that W is fetched into an L2 once and the rows are what its work-groups share at a time.
+template <int MB, int NB, int STAGES, bool PARTS>
+__global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_kernel(
+    const uint4* __restrict__ As, const float* __restrict__ A, const float* __restrict__ Ws, const float* __restrict__ bias,
+    float* __restrict__ C, int M, int N, int K, int lda, int ldc, int steps) {
+    extern __shared__ uint4 fs_lds[];
+    constexpr int CHUNKS = MB * 3, LA = (CHUNKS + FS_WAVES - 1) / FS_WAVES, LW = NB * 2, STAGE = (CHUNKS + FS_WAVES * LW) * 64;
+    constexpr int BN = FS_WAVES * NB * 32;
+    const int blocks = (M + 31) / 32, mtiles = (blocks + MB - 1) / MB, ntiles = (N + BN - 1) / BN;
+    const int local = blockIdx.x >> 3;
+    const int nt = (local / mtiles) * 8 + (blockIdx.x & 7), mt = local % mtiles;
+    if (nt >= ntiles) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b0 = mt * MB, n0 = (nt * FS_WAVES + wave) * NB * 32;
+    const int first = PARTS ? blockIdx.y * FS_SEG_STEPS : 0;
+    const int last = PARTS ? min(first + FS_SEG_STEPS, steps) : steps;
+
+    const uint4* ap[LA];
+    const uint4* wp[LW];
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+        const int c = min(wave + i * FS_WAVES, CHUNKS - 1);            // a wave without a piece of its own repeats the last one
+        ap[i] = As + ((size_t)min(b0 + c / 3, blocks - 1) * steps + first) * 192 + (c % 3) * 64 + lane;
+    }
+#pragma unroll
+    for (int j = 0; j < LW; ++j)
+        wp[j] = reinterpret_cast<const uint4*>(Ws) + ((size_t)min(n0 / 16 + j, (N + 15) / 16 - 1) * steps + first) * 64 + lane;
+    int ahead = first;                   // the step that is fetched next; the last one again at the end
+    auto fetch = [&](int buf) {
+        uint4* stage = fs_lds + buf * STAGE;
+#pragma unroll
+        for (int i = 0; i < LA; ++i) fs_load_to_lds(ap[i], stage + min(wave + i * FS_WAVES, CHUNKS - 1) * 64);
+#pragma unroll
+        for (int j = 0; j < LW; ++j) fs_load_to_lds(wp[j], stage + (CHUNKS + wave * LW + j) * 64);
+        if (++ahead < last) {
+#pragma unroll
+            for (int i = 0; i < LA; ++i) ap[i] += 192;
+#pragma unroll
+            for (int j = 0; j < LW; ++j) wp[j] += 64;
+        }
+    };
+    fs_f32x16 acc[MB][NB];
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    };
+    // this lane holds rows 8 (r / 4) + 4 (lane / 32) + r % 4 of a block and one column
+    float* out = PARTS ? C + (size_t)blockIdx.y * M * N : C;
+    const size_t ld = PARTS ? N : ldc;
+    const int row0 = b0 * 32 + 4 * (lane >> 5);
+    bool nan_seen = false;
+    auto store = [&](bool first_seg, bool last_seg) {
+        int row = row0, col = n0 + (lane & 31);
+        asm volatile("" : "+v"(row), "+v"(col));       // addresses and bounds are made here, not kept through the loop over k
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            const int n = col + j * 32;
+            const float b = !PARTS && bias && last_seg && n < N ? bias[n] : 0.f;
+            float* o = out + (size_t)row * ld + n;
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {          // four rows at a time: a few addresses and sums in registers
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        float v = acc[i][j][4 * q + r];
+                        if (n < N && row + i * 32 + 8 * q + r < M) {
+                            if (!PARTS && !first_seg) v = o[r * ld] + v;
+                            nan_seen |= v != v;
+                            o[r * ld] = v + b;
+                        }
+                    }
+                    o += 8 * ld;
+                    asm volatile("" ::: "memory");
+                }
+        }
+    };
+    clear();
+    for (int i = 0; i < STAGES - 1; ++i) fetch(i);
+    int buf = 0;
+    const int wfrag = (CHUNKS + wave * LW) * 64 + ((lane >> 4) & 1) * 64 + (lane >> 5) * 32 + (lane & 15);
+    for (int s = first; s < last; ++s) {
+        FS_LANDED((STAGES - 2) * (LA + LW));   // step s is here; later ones may be on their way
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        fetch(buf == 0 ? STAGES - 1 : buf - 1);   // the buffer of step s - 1, which every wave has read
+        const uint4* stage = fs_lds + buf * STAGE;
+        uint4 w[NB][3];
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            fs_split8(__builtin_bit_cast(float4, stage[wfrag + j * 128]), __builtin_bit_cast(float4, stage[wfrag + j * 128 + 16]),
+                      w[j][0], w[j][1], w[j][2]);
+        // two blocks' products in turn, so that none waits for the one before it
+        constexpr int IB = NB > 1 || MB == 1 ? 1 : 2;
+#pragma unroll
+        for (int i = 0; i < MB; i += IB) {
+            uint4 a[IB][3];
+#pragma unroll
+            for (int b = 0; b < IB; ++b)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) a[b][p] = stage[((i + b) * 3 + p) * 64 + lane];
+#define FS_MUL(PA, PW)                                                                                                       \
+    _Pragma("unroll") for (int b = 0; b < IB; ++b) _Pragma("unroll") for (int j = 0; j < NB; ++j) acc[i + b][j] =              \
+        __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fs_bf16x8, a[b][PA]), __builtin_bit_cast(fs_bf16x8, w[j][PW]), \
+                                                acc[i + b][j], 0, 0, 0);
+            FS_MUL(0, 2)
+            FS_MUL(2, 0)
+            FS_MUL(1, 1)
+            FS_MUL(0, 1)
+            FS_MUL(1, 0)
+            FS_MUL(0, 0)
+#undef FS_MUL
+        }
+        if (!PARTS && (s + 1) % FS_SEG_STEPS == 0 && s + 1 < last) {
+            store(s < FS_SEG_STEPS, false);
+            clear();
+        }
+        buf = buf == STAGES - 1 ? 0 : buf + 1;
+    }
+    FS_LANDED(0);                        // nothing may land in LDS that is no longer this work-group's
+    store(last <= FS_SEG_STEPS, true);
+    if (!nan_seen) return;
+    for (int j = 0; j < NB; ++j) {
+        const int n = n0 + j * 32 + (lane & 31);
+        for (int i = 0; n < N && i < MB * 16; ++i) {
+            const int m = row0 + 8 * (i >> 2) + (i & 3);
+            if (m >= M || out[(size_t)m * ld + n] == out[(size_t)m * ld + n]) continue;
+            out[(size_t)m * ld + n] = fs_plain(A, Ws, lda, steps, m, n, first * FS_STEP, min(last * FS_STEP, K)) + (!PARTS && bias ? bias[n] : 0.f);
+        }
+    }
+}
+
+// The segments' sums in ascending order, as the product adds them where it has the whole K.  VEC: four columns a
+// thread (N and ldc multiples of four, everything aligned).
+template <bool VEC>
+__global__ __launch_bounds__(256) void fs_add_kernel(const float* __restrict__ parts, const float* __restrict__ bias,
+                                                     float* __restrict__ C, int M, int N, int ldc, int nseg) {
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * (VEC ? 4 : 1), all = (size_t)M * N;
+    if (i >= all) return;
+    const int m = (int)(i / N), n = (int)(i - (size_t)m * N);
+    if (VEC) {
+        float4 sum = *reinterpret_cast<const float4*>(parts + i);
+        for (int g = 1; g < nseg; ++g) {
+            const float4 p = *reinterpret_cast<const float4*>(parts + (size_t)g * all + i);
+            sum.x += p.x, sum.y += p.y, sum.z += p.z, sum.w += p.w;
+        }
+        if (bias) sum.x += bias[n], sum.y += bias[n + 1], sum.z += bias[n + 2], sum.w += bias[n + 3];
+        *reinterpret_cast<float4*>(C + (size_t)m * ldc + n) = sum;
+    } else {
+        float sum = parts[i];
+        for (int g = 1; g < nseg; ++g) sum += parts[(size_t)g * all + i];
+        C[(size_t)m * ldc + n] = sum + (bias ? bias[n] : 0.f);
+    }
+}
+
+// The tiles (row blocks and column blocks of a wave) with what was measured on the products of 7B and 0.5B models: a step of
+// 16 k takes a work-group `alone` us when its CU has nothing else (the chain barrier - reads - products), and a CU gets
+// through one in `shared` us when it holds as many as fit.  The tile, and whether K is dealt out by segments, is the
+// least estimate; e.g. at 2,048 rows gate/up (37,888 x 3,584) 2.8 ms in tiles of 128 x 256 (197 TFLOP/s; tiles of 256 rows
+// 3.1, of 128 x 128 3.0), down (3,584 x 18,944) 1.66 ms with K dealt out against 1.72, where the float instruction took 4.9 and
+// 2.8; at 40 rows down takes 97 us dealt out against 480.
+struct FsTile {
+    int mb, nb, fit;
+    double alone, shared;
+};
+static const FsTile fs_tiles[] = {{4, 2, 2, 1.90, 1.36}, {4, 1, 2, 0.95, 0.71}, {2, 1, 3, 0.56, 0.41}, {1, 1, 4, 0.43, 0.26}};
+
+static int fs_choose(int M, int N, int K, bool* parts) {
+    const int blocks = tl_ceil_div(M, 32), steps = tl_ceil_div(K, FS_STEP), nseg = tl_ceil_div(K, FS_SEG);
+    int best = 3;
+    double cost = 1e300;
+    for (int t = 0; t < 4; ++t) {
+        const FsTile& z = fs_tiles[t];
+        if (z.mb > 1 && z.mb / 2 >= blocks) continue;                  // half of it holds all the rows
+        const double tiles = (double)tl_ceil_div(blocks, z.mb) * tl_ceil_div(N, FS_WAVES * 32 * z.nb);
+        for (int cut = 0; cut < (nseg > 1 && nseg <= 65535 ? 2 : 1); ++cut) {
+            const double each = tiles * (cut ? nseg : 1) / FS_CUS, whole = (double)(long long)(each + 0.999999);
+            const double on_a_cu = whole < 4 ? whole : each + 0.5, turns = (double)(long long)((whole + z.fit - 1) / z.fit);
+            const double step = turns * z.alone > on_a_cu * z.shared ? turns * z.alone : on_a_cu * z.shared;
+            const double us = step * steps / (cut ? nseg : 1) + (cut ? 4.0 + 8.0 * M * N * nseg / 6e6 : 0.0);
+            if (us < cost) cost = us, best = t, *parts = cut != 0;
+        }
+    }
+    return best;
+}
+
+// Floats of workspace that tl_gemm_float_split needs for the segments' sums (0: none).
+extern "C" long long tl_gemm_float_split_workspace(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    bool parts = false;
+    fs_choose(M, N, K, &parts);
+    return parts ? (long long)tl_ceil_div(K, FS_SEG) * M * N : 0;
+}
+
+// A float [M, K] with row stride lda; Ws float [ceil(N/16), ceil(K/16), 64, 4] (the matrix-core ordered copy of W, zero
+// where it pads); split: workspace of ceil(M/32) * ceil(K/16) * 3 KB; ws: tl_gemm_float_split_workspace floats.
+extern "C" int tl_gemm_float_split(const float* A, const float* Ws, const float* bias, float* C, void* split, float* ws, int M,
+                                   int N, int K, int lda, int ldc, hipStream_t stream) {
+    TL_CHECK_ARG(M >= 0 && N > 0 && K > 0, "tl_gemm_float_split: bad sizes M=%d N=%d K=%d", M, N, K);
+    TL_CHECK_ARG(lda >= K && ldc >= N, "tl_gemm_float_split: row strides lda=%d ldc=%d too small for K=%d N=%d", lda, ldc, K, N);
+    TL_CHECK_ARG((uintptr_t)Ws % 16 == 0 && (uintptr_t)split % 16 == 0, "tl_gemm_float_split: the weight copy and the workspace must be 16-byte aligned");
+    if (M == 0) return 0;
+    const int steps = tl_ceil_div(K, FS_STEP), blocks = tl_ceil_div(M, 32), nseg = tl_ceil_div(K, FS_SEG);
+    TL_CHECK_ARG(blocks <= 65535, "tl_gemm_float_split: %d rows are too many for one launch", M);
+    bool parts = false;
+    const int tile = fs_choose(M, N, K, &parts);
+    const int mtiles = tl_ceil_div(blocks, fs_tiles[tile].mb), ntiles = tl_ceil_div(N, FS_WAVES * 32 * fs_tiles[tile].nb);
+    const long long grid = (long long)mtiles * tl_ceil_div(ntiles, 8) * 8;
+    TL_CHECK_ARG(grid < (1ll << 31), "tl_gemm_float_split: M=%d N=%d are too many tiles for one launch", M, N);
+    TL_CHECK_ARG(!parts || ws, "tl_gemm_float_split: no workspace for the segments' sums");
+    const int vec = ((uintptr_t)A % 16 == 0 && lda % 4 == 0) ? 1 : 0;
+    hipLaunchKernelGGL(fs_split_kernel, dim3(tl_ceil_div(steps, 4), blocks), dim3(256), 0, stream, A, (uint4*)split, M, K, lda, steps, vec);
+#define FS_GO(MB, NB, ST, P)                                                                                                     \
+    hipLaunchKernelGGL((fs_gemm_kernel<MB, NB, ST, P>), dim3((unsigned)grid, P ? nseg : 1), dim3(FS_WAVES * 64),                 \
+                       ST * (MB * 3 + FS_WAVES * NB * 2) * 1024, stream, (const uint4*)split, A, Ws, bias, P ? ws : C, M, N, K, \
+                       lda, ldc, steps)
+#define FS_GO_P(MB, NB, ST)             \
+    if (parts) FS_GO(MB, NB, ST, true); \
+    else FS_GO(MB, NB, ST, false)
+    if (tile == 0) {
+        FS_GO_P(4, 2, 2);
+    } else if (tile == 1) {
+        FS_GO_P(4, 1, 3);
+    } else if (tile == 2) {
+        FS_GO_P(2, 1, 3);
+    } else {
+        FS_GO_P(1, 1, 3);
+    }
+#undef FS_GO_P
+#undef FS_GO
+    if (parts) {
+        const long long all = (long long)M * N;
+        TL_CHECK_ARG((all + 255) / 256 < (1ll << 31), "tl_gemm_float_split: M=%d N=%d are too many sums for one launch", M, N);
+        if (N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0 && (uintptr_t)ws % 16 == 0)
+            hipLaunchKernelGGL(fs_add_kernel<true>, dim3((unsigned)((all / 4 + 255) / 256)), dim3(256), 0, stream, ws, bias, C, M, N, ldc, nseg);
+        else
+            hipLaunchKernelGGL(fs_add_kernel<false>, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, stream, ws, bias, C, M, N, ldc, nseg);
+    }
+    TL_CHECK_LAUNCH("tl_gemm_float_split");
+    return 0;
+}

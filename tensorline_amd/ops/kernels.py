@@ -43,6 +43,7 @@ def library() -> ctypes.CDLL:
                 except OSError as e:
                     raise KernelError(f"cannot load the HIP kernel library {path}: {e}") from e
                 lib.tl_last_error.restype = ctypes.c_char_p
+                lib.tl_gemm_float_split_workspace.restype = ctypes.c_longlong
                 _lib = lib
     return _lib
 
@@ -562,6 +563,7 @@ MFMA_HEAD_DIMS = (32, 64, 128, 256)   # head sizes of the bfloat16 matrix-core a
 GENERIC_SPLIT_KEYS = 256  # keys per split of the any-shape attention kernel in steps of one token per sequence
 SKINNY_MAX_ROWS = 16     # rows the few-row kernel serves (one 16-row MFMA tile)
 ROWS64_MAX_ROWS = 64     # rows the 17..64-row kernel serves; above that the library
+FLOAT_SPLIT_MAX_ROWS = 65535 * 32   # rows one launch of the float product of more than 16 rows takes
 
 
 def _skinny_ok(a: torch.Tensor, shuffled: torch.Tensor | None, M: int, K: int, lda: int) -> bool:
@@ -587,6 +589,19 @@ def _few_rows_go_to_rows64(N: int, K: int) -> bool:
     return 2 <= rounds <= 3 and tiles < 0.75 * rounds * 256 and rounds * steps >= 150
 
 
+def _float_split(a, shuffled, bias, out, M, N, K, lda, ldc):
+    """More than 16 float rows: every float as the sum of three bfloat16 numbers on the bfloat16 matrix instruction,
+    the weight from its matrix-core ordered copy.  Every matrix that has the copy goes here, whatever its rows beyond 16, so
+    that a row's bits do not depend on how many others come along: at 33 rows and more it is the faster kernel at every K
+    (300 rows, N = 1,152: K = 64 8.2 us against 16, 896 29 against 89), at 17 to 32 rows it is level from K = 896 on and its
+    second launch costs 2 us below (K = 128: 7.8 against 5.7)."""
+    split = torch.empty(-(-M // 32) * -(-K // 16) * 1536, dtype=torch.int16, device=a.device)
+    floats = library().tl_gemm_float_split_workspace(M, N, K)
+    ws = torch.empty(floats, dtype=torch.float32, device=a.device) if floats else None
+    _call("tl_gemm_float_split", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), _ptr(split), _ptr(ws), M, N, K, lda, ldc, _stream())
+    return out
+
+
 def _rows64(a, shuffled, bias, out, M, N, K, lda, ldc, swiglu: bool, norm=None):
     """17 to 64 rows: a 16-column tile per wave, rows shared through LDS, K split over the grid."""
     shares = library().tl_gemm_rows64_shares(M, N, K)
@@ -610,6 +625,9 @@ def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None) -> 
             and M <= SKINNY_MAX_ROWS and library().tl_gemm_fewrows_takes(K)):
         _call("tl_gemm_fewrows_shuffled", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), M, N, K, lda, ldc, _stream())
         return out
+    if (shuffled is not None and shuffled.dtype == torch.float32 and a.dtype == torch.float32 and out.dtype == torch.float32
+            and SKINNY_MAX_ROWS < M <= FLOAT_SPLIT_MAX_ROWS):
+        return _float_split(a, shuffled, bias, out, M, N, K, lda, ldc)
     _call("tl_gemm_generic", _ptr(a), _code(a, "linear input"), _ptr(weight), _code(weight, "linear weight"),
           _ptr(bias), _ptr(out), _code(out, "linear output"), M, N, K, lda, ldc, _stream())
     return out

@@ -141,6 +141,43 @@ def test_linear_few_rows_float32(M, N, Kd):
     torch.testing.assert_close(K().linear(strided, w, b, shuffled=ws), K().linear(strided, w, b), atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 70, 129, 300])
+@pytest.mark.parametrize("N,Kd", [(1, 1), (31, 15), (33, 16), (130, 17), (257, 2047), (96, 2048), (132, 2049), (40, 4100), (1152, 896)])
+def test_linear_float_by_three_bfloat16(M, N, Kd):
+    """The float product of more than 16 rows (every float as the sum of three bfloat16): tiles' and segments' edges,
+    rows neither aligned nor contiguous, columns that the segments' adding kernel takes four at a time or one.  The bound is
+    that of K float multiply-adds in any order.  A row has the same bits whatever rows come along."""
+    torch.manual_seed(M + N)
+    w = torch.randn(N, Kd, device=DEV)
+    b = torch.randn(N, device=DEV)
+    ws = K().shuffle_weight_float(w)
+    for a in (torch.randn(M, Kd, device=DEV), torch.randn(M, Kd + 5, device=DEV)[:, 1:Kd + 1]):
+        want = a.double() @ w.double().T + b.double()
+        size = a.double().abs() @ w.double().abs().T + b.double().abs()
+        got = K().linear(a, w, b, shuffled=ws)
+        assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())
+        few = K().linear(a[M - 17:], w, b, shuffled=ws)
+        assert torch.equal(few, got[M - 17:])
+        wide = torch.full((M, N + 3), 7.0, device=DEV)
+        K().linear(a, w, b, out=wide[:, 1:N + 1], shuffled=ws)
+        assert torch.equal(wide[:, 1:N + 1], got) and bool((wide[:, [0, N + 1, N + 2]] == 7.0).all())
+
+
+def test_linear_float_by_three_bfloat16_not_finite():
+    """Infinities, NaN and values that round to infinity as bfloat16, on either side and across segments: what plain float
+    arithmetic gives."""
+    torch.manual_seed(3)
+    a, w = torch.randn(40, 2100, device=DEV), torch.randn(70, 2100, device=DEV)
+    a[3, 5], a[7, 2070], a[9, 1], w[5, 2], w[6, 2090] = float("inf"), float("nan"), 3.4e38, float("-inf"), 3.4e38
+    w[:, 1] *= 1e-3
+    got = K().linear(a, w, shuffled=K().shuffle_weight_float(w)).cpu()
+    want = (a.cpu().double() @ w.cpu().double().T).float()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    torch.testing.assert_close(got[fine], want[fine], atol=1e-3, rtol=1e-5)
+
+
 @pytest.mark.parametrize("M", [1, 2, 8, 16, 17, 33, 48, 64])
 @pytest.mark.parametrize("N,Kd", [(1000, 1184), (4608, 3584), (136, 8), (50, 264), (3584, 18944), (5120, 1184), (2090, 72),
                                   (5120, 9728)])
