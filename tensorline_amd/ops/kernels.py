@@ -1791,6 +1791,21 @@ def moe_tile_rows(pairs: int, experts: int) -> int:
     return 16 if pairs <= 16 * experts else 64
 
 
+MOE_WIDE_TILE = 256      # rows at most of a tile of the grouped bfloat16 product of many rows per expert
+
+
+def _moe_takes_wide_tiles(pairs: int, experts: int, ff: int) -> bool:
+    """Whether the experts' products run in tiles of up to 256 rows by 256 matrix rows (a work-group of one per CU) and not in
+    tiles of 64 by 128.  They fetch each matrix once and the rows half as often, which pays from few rows on where there are
+    twice as many tiles as CUs (64 experts of 4,096 x 2,048, both products: 18 rows per expert 647 against 693 us, 90: 754
+    against 932, 192: 1,066 against 1,475; of 2,048 x 1,408: 18 rows 239 against 246, 192: 433 against 616); between one and two
+    tiles per CU only where they are full (32 experts of 1,024 x 512: 384 rows 109 against 124 us, 188 rows, with half a
+    tile per CU, 101 against 75)."""
+    rows = -(-pairs // experts)
+    tiles = experts * -(-rows // MOE_WIDE_TILE) * -(-ff // 128)
+    return tiles >= 512 or (tiles >= 256 and rows >= MOE_WIDE_TILE)
+
+
 def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
                 limit: float, alpha: float, shared: torch.Tensor | None = None, shift: float = 1.0,
                 gated: bool = True, shared_gate: torch.Tensor | None = None, keep_rows: bool = False) -> "torch.Tensor | ExpertRows":
@@ -1814,17 +1829,21 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
         _f32(shared, "moe_experts shared", T * N)
     P = T * top
     BM = moe_tile_rows(P, E)
+    if (BM == 64 and _moe_takes_wide_tiles(P, E, F) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
+            and library().tl_moe_gemm_takes_wide(F) and (T == 1 or h.stride(0) % 8 == 0)
+            and (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0):
+        BM = MOE_WIDE_TILE
     max_tiles = P // BM + E
     order = torch.empty(P, dtype=torch.int32, device=h.device)
     tiles = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=h.device)
     _call("tl_moe_sort", _ptr(ids), _ptr(order), _ptr(tiles), P, E, BM, _stream())
     act = torch.empty(P, F, dtype=h.dtype, device=h.device)
     _call("tl_moe_gemm", _ptr(h), _code(h, "moe_experts input"), h.stride(0) if T > 1 else K, _ptr(gate_up),
-          _code(gate_up, "moe_experts weights"), _ptr(act), _code(act, "moe_experts"), F, _ptr(order), _ptr(tiles), max_tiles, BM,
+          _code(gate_up, "moe_experts weights"), _ptr(act), _code(act, "moe_experts"), F, _ptr(order), _ptr(tiles), max_tiles, E, BM,
           top, F, K, 1 if gated else 2, ctypes.c_float(limit), ctypes.c_float(alpha), ctypes.c_float(shift), _stream())
     y = torch.empty(P, N, dtype=torch.float32, device=h.device)
     _call("tl_moe_gemm", _ptr(act), _code(act, "moe_experts"), F, _ptr(down), _code(down, "moe_experts weights"), _ptr(y), F32, N,
-          _ptr(order), _ptr(tiles), max_tiles, BM, top, N, F, 0, ctypes.c_float(0.0), ctypes.c_float(0.0), ctypes.c_float(0.0),
+          _ptr(order), _ptr(tiles), max_tiles, E, BM, top, N, F, 0, ctypes.c_float(0.0), ctypes.c_float(0.0), ctypes.c_float(0.0),
           _stream())
     if keep_rows:
         _check(shared is None, "moe_experts: the experts' rows are handed on without a shared expert only")

@@ -1060,3 +1060,55 @@ def test_bias_at_every_distance_with_windows_and_kept_keys(path, dtype, window, 
             got, want = _attention_case(dtype, 4, 2, 64, 16, lens, q_lens, seed=at, path=path, window=window, keep_first=keep_first,
                                         softcap=9.0, sink=True, bias=bias)
             torch.testing.assert_close(got, want, **tol(dtype, 3e-5, 2e-2))
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("Kd,F,N", [(64, 64, 64), (320, 192, 320), (1024, 448, 1024)])
+def test_experts_in_wide_tiles(gated, Kd, F, N, monkeypatch):
+    """The grouped product's tiles of up to 256 rows: experts of no pair, one, a tile's edges and several tiles, matrices of
+    fewer rows than a tile, input rows wider than K: against the sums in float64, and bit for bit what tiles of 64 rows give."""
+    torch.manual_seed(F)
+    loads = [0, 1, 63, 64, 65, 130, 193, 255, 256, 257, 300, 513]
+    E, top = len(loads), 1
+    ids = torch.tensor([e for e, n in enumerate(loads) for _ in range(n)], dtype=torch.int32)
+    ids = ids[torch.randperm(len(ids))].to(DEV)[:, None].contiguous()
+    T = ids.shape[0]
+    h = torch.randn(T, Kd + 8, device=DEV).to(torch.bfloat16)[:, :Kd]
+    up = (torch.randn(E, (2 if gated else 1) * F, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    down = (torch.randn(E, N, F, device=DEV) / math.sqrt(F)).to(torch.bfloat16)
+    weights = torch.rand(T, top, device=DEV)
+    got = {}
+    for wide in (True, False):
+        monkeypatch.setattr(K(), "_moe_takes_wide_tiles", lambda *a: wide)
+        got[wide] = K().moe_experts(h, up, down, ids, weights, 7.0 if gated else float("inf"), 1.702 if gated else 1.0, gated=gated)
+    assert torch.equal(got[True], got[False])
+    want = torch.zeros(T, N, dtype=torch.float64, device=DEV)
+    for e in range(E):
+        rows = (ids[:, 0] == e).nonzero()[:, 0]
+        z = h[rows].double() @ up[e].double().T
+        if gated:
+            g = z[:, :F].clamp(max=7.0)
+            act = g * torch.sigmoid(1.702 * g) * (z[:, F:].clamp(-7.0, 7.0) + 1.0)
+        else:
+            act = z.clamp(min=0) ** 2
+        # the activations are kept as bfloat16 (2^-9 of each at most): what that can move in a sum of F products
+        want[rows] = weights[rows].double() * (act @ down[e].double().T)
+        slack = weights[rows].double() * ((act.abs() * 2.0 ** -8 + 1e-4) @ down[e].double().abs().T) + 1e-4
+        assert bool(((got[True][rows].double() - want[rows]).abs() <= slack).all()), e
+
+
+@pytest.mark.parametrize("P,E,BM", [(1, 1, 16), (7, 3, 256), (1000, 70, 16), (5000, 64, 256), (12288, 64, 64), (9000, 200, 256), (3000, 1024, 16)])
+def test_pairs_in_tiles_by_expert(P, E, BM):
+    """The order of the pairs and the tiles made of it: every pair once, in a tile of its expert, tiles within BM rows."""
+    torch.manual_seed(P)
+    ids = (torch.rand(P, device=DEV) ** 2 * E).to(torch.int32).clamp(max=E - 1)
+    order, tiles = torch.full((P,), -1, dtype=torch.int32, device=DEV), torch.zeros(1 + 3 * (P // BM + E), dtype=torch.int32, device=DEV)
+    K()._call("tl_moe_sort", K()._ptr(ids), K()._ptr(order), K()._ptr(tiles), P, E, BM, K()._stream())
+    order, tiles, ids = order.tolist(), tiles.tolist(), ids.tolist()
+    assert sorted(order) == list(range(P)) and 0 < tiles[0] <= P // BM + E
+    at = 0
+    for t in range(tiles[0]):
+        e, first, rows = tiles[1 + 3 * t:4 + 3 * t]
+        assert first == at and 0 < rows <= BM and all(ids[order[p]] == e for p in range(first, first + rows))
+        at += rows
+    assert at == P
