@@ -568,11 +568,12 @@ __device__ __forceinline__ void am_tile_lds(const uint4* kt, const uint4* vt, in
 __device__ __forceinline__ int at_lds_key(int row) {
     return (row & 35) + ((row & 16) >> 2) + ((row & 12) << 1);
 }
-// Where unit u of a row lies in it: u ^ swizzle(row).  A K row has UPK = 4, 8 or 16 units, so 16 /
-// UPK rows span the 256 bytes over which the banks repeat; the swizzle steps once per such span.  A
+// Where unit u of a row lies in it: u ^ swizzle(row).  A K row has UPK = 4, 8, 16 or 32 units, so 16 /
+// UPK rows span the 256 bytes over which the banks repeat; the swizzle steps once per such span (once per row of
+// 16 or 32 units).  A
 // V^T row has 8 units.  Both depend only on the row modulo 16 (the lane's c in a fragment read).
 template <int UPK>
-__device__ __forceinline__ int at_k_swizzle(int row) { return ((row & 15) * UPK) >> 4; }
+__device__ __forceinline__ int at_k_swizzle(int row) { return ((row & 15) * (UPK < 16 ? UPK : 16)) >> 4; }
 __device__ __forceinline__ int at_v_swizzle(int row) { return (row >> 1) & 7; }
 
 // 16 bytes per lane from memory straight into LDS at lds_base + 16 * lane (lds_base is the same for
@@ -597,8 +598,11 @@ __device__ __forceinline__ void at_load_to_lds(const void* g, void* lds_base) {
 // work-group per CU (a short portion behind a long context), where the longest walk sets the time and
 // a lone work-group leaves part of its CU unused.  The chains share the barrier, so they pass a
 // tile's phases together and gain less than two work-groups that drift apart would: 10 to 17%.
+// A head size of 256 (DC = 8: latent attention, whose query heads share one key/value head) has 128 KB of tiles and up to
+// 256 registers a wave: one work-group per CU.  2,048 fresh tokens of 32 heads take 98 us, where independent
+// waves, each fetching its own fragments for 16 columns, took 457 (512 behind 3,500: 130 against 357).
 template <int DC, int NT, int WAVES, int CH, int MODE>
-__global__ __launch_bounds__(CH * WAVES * 64, 32 / WAVES) void attn_tile_kernel(
+__global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void attn_tile_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int32_t* __restrict__ tables, int NB, const int32_t* __restrict__ q_start,
     const int32_t* __restrict__ ctx_start, bf16_t* __restrict__ out, int out_stride, int S, int nq, int nkv, int bs,
@@ -673,11 +677,11 @@ __global__ __launch_bounds__(CH * WAVES * 64, 32 / WAVES) void attn_tile_kernel(
     // work-group i + 256 on the CU of work-group i (256 CUs, two work-groups each), so when the
     // grid has more than 256 and at most 512 work-groups the groups after the first 256 / nkv are
     // taken from the light end instead: the heaviest shares its CU with the lightest, and the CUs
-    // finish together instead of the first ones last.
+    // finish together instead of the first ones last.  (With one work-group per CU the heaviest first is the order.)
     int group = ngroups - 1 - flat;
     {
         const int total = (int)(gridDim.x * gridDim.y), first = AT_CUS / (int)gridDim.x;
-        if (CH == 1 && total > AT_CUS && total <= 2 * AT_CUS && flat >= first) group = flat - first;
+        if (CH == 1 && DC < 8 && total > AT_CUS && total <= 2 * AT_CUS && flat >= first) group = flat - first;
     }
     const int wg_col0 = group * 128;
     const int col0 = wg_col0 + wave * WCOLS;
@@ -1088,9 +1092,8 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
     dim3 grid(S_run, nkv, (unsigned)((waves + wg_waves - 1) / wg_waves));
     const bf16_t *qq = (const bf16_t*)q, *kk = (const bf16_t*)k_cache, *vv = (const bf16_t*)v_cache;
     const bool pow2 = (bs & (bs - 1)) == 0;
-    // (a head size of 256 has the independent waves only: its tiles of keys and values would not leave
-    // LDS for a second work-group per CU)
-    if (NT == 2 && nsplit == 1 && shared && pow2 && !seq_list && total_groups128 > 0 && d != 256 &&
+    // (a head size of 256 comes with NT = 1, its column tiles where the waves are independent; one chain of tiles fills LDS)
+    if ((NT == 2 || d == 256) && nsplit == 1 && shared && pow2 && !seq_list && total_groups128 > 0 &&
         at_lds_bytes(d / 32, NB, S, bias_floats) <= 160 * 1024) {
         // 128 columns per work-group, keys and values shared through LDS; shared == 2 asks for two
         // chains per work-group where their tiles fit LDS
@@ -1098,7 +1101,7 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
         while ((1 << bs_shift) < bs) ++bs_shift;
         TL_CHECK_ARG(total_groups128 <= 65535, "tl_attention_mfma: %d column groups are more than a launch takes", total_groups128);
         dim3 sgrid(nkv, (unsigned)total_groups128, 1);
-        const int chains = (shared == 2 && at_lds_bytes(d / 32, NB, S, bias_floats, 2) <= 160 * 1024) ? 2 : 1;
+        const int chains = (shared == 2 && d != 256 && at_lds_bytes(d / 32, NB, S, bias_floats, 2) <= 160 * 1024) ? 2 : 1;
         const size_t lds = at_lds_bytes(d / 32, NB, S, bias_floats, chains);
 #define TL_TILE_CASE(DCV)                                                                                             \
     do {                                                                                                              \
@@ -1106,20 +1109,27 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
         else if (softcap > 0.f) TL_TILE_GO(DCV, 1);                                                                   \
         else TL_TILE_GO(DCV, 0);                                                                                      \
     } while (0)
+#define TL_TILE_CASE_256()                                                                                            \
+    do {                                                                                                              \
+        if (bias_table) TL_TILE_GO_(8, 1, 2);                                                                         \
+        else if (softcap > 0.f) TL_TILE_GO_(8, 1, 1);                                                                 \
+        else TL_TILE_GO_(8, 1, 0);                                                                                    \
+    } while (0)
 #define TL_TILE_GO(DCV, MODEV)                                                                                        \
     do {                                                                                                              \
-        if (chains == 2)                                                                                              \
-            hipLaunchKernelGGL((attn_tile_kernel<DCV, AT_NT, 8 / AT_NT, 2, MODEV>), sgrid, dim3(2 * 64 * 8 / AT_NT), lds,    \
-                               stream, qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride, \
-                               S, nq, nkv, bs, bs_shift, mask, scale, skip_single, sinks, softcap, bias);                              \
-        else                                                                                                          \
-            hipLaunchKernelGGL((attn_tile_kernel<DCV, AT_NT, 8 / AT_NT, 1, MODEV>), sgrid, dim3(64 * 8 / AT_NT), lds,        \
-                               stream, qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride, \
-                               S, nq, nkv, bs, bs_shift, mask, scale, skip_single, sinks, softcap, bias);                              \
+        if (chains == 2) TL_TILE_GO_(DCV, 2, MODEV);                                                                  \
+        else TL_TILE_GO_(DCV, 1, MODEV);                                                                              \
     } while (0)
+#define TL_TILE_GO_(DCV, CHV, MODEV)                                                                                  \
+    hipLaunchKernelGGL((attn_tile_kernel<DCV, AT_NT, 8 / AT_NT, CHV, MODEV>), sgrid, dim3(CHV * 64 * 8 / AT_NT), lds, stream, \
+                       qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride, S, nq, nkv, bs, \
+                       bs_shift, mask, scale, skip_single, sinks, softcap, bias)
         if (d == 32) TL_TILE_CASE(1);
         else if (d == 64) TL_TILE_CASE(2);
-        else TL_TILE_CASE(4);
+        else if (d == 128) TL_TILE_CASE(4);
+        else TL_TILE_CASE_256();
+#undef TL_TILE_CASE_256
+#undef TL_TILE_GO_
 #undef TL_TILE_GO
 #undef TL_TILE_CASE
         TL_CHECK_LAUNCH("tl_attention_mfma tiles");

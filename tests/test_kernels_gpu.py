@@ -1112,3 +1112,19 @@ def test_pairs_in_tiles_by_expert(P, E, BM):
         assert first == at and 0 < rows <= BM and all(ids[order[p]] == e for p in range(first, first + rows))
         at += rows
     assert at == P
+
+
+@pytest.mark.parametrize("nq,nkv,bs,lens,q_lens,kw", [
+    (4, 1, 16, [300, 65, 64, 2], [300, 64, 17, 2], {}),                              # tiles' edges; fewer columns than a wave, a work-group
+    (32, 1, 8, [700, 130], [41, 130], {}),                                           # a portion behind cached tokens, pages of 8
+    (16, 2, 64, [257, 900], [257, 3], dict(window=100)),                             # two key/value heads, a window
+    (8, 1, 16, [900, 64], [500, 64], dict(window=70, keep_first=5)),
+    (8, 1, 16, [900, 200], [300, 200], dict(chunk=96, softcap=20.0)),
+    (8, 1, 32, [400, 1, 300], [200, 1, 1], dict(sink=True)),                         # one-token requests beside a portion
+    (8, 1, 24, [300], [100], {}),                                                    # pages that are no power of two: independent waves
+])
+def test_attention_tiles_at_head_size_256(nq, nkv, bs, lens, q_lens, kw):
+    """Prompt portions at a head size of 256 on the kernel that shares key tiles through LDS (probabilities are rounded to
+    bfloat16 ahead of their product with the values: 2^-9 of each, as at the other head sizes)."""
+    got, want = _attention_case(torch.bfloat16, nq, nkv, 256, bs, lens, q_lens, seed=9, **kw)
+    torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
