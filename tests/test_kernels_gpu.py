@@ -1128,3 +1128,21 @@ def test_attention_tiles_at_head_size_256(nq, nkv, bs, lens, q_lens, kw):
     bfloat16 ahead of their product with the values: 2^-9 of each, as at the other head sizes)."""
     got, want = _attention_case(torch.bfloat16, nq, nkv, 256, bs, lens, q_lens, seed=9, **kw)
     torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
+
+
+@pytest.mark.parametrize("T", [1, 17, 32, 33, 130])
+@pytest.mark.parametrize("B,N,Kd", [(3, 1, 8), (2, 63, 24), (3, 64, 40), (2, 65, 192), (2, 192, 128), (1, 70, 1024), (2, 40, 1032)])
+def test_batched_linear_bfloat16(T, B, N, Kd):
+    """The product per head: remainders of rows, columns and k, operands that are column blocks of wider rows, a K too long
+    for the kernel without LDS, and rows that are not aligned (the any-shape kernel)."""
+    torch.manual_seed(T + N)
+    w = torch.randn(B, N, Kd, device=DEV).to(torch.bfloat16)
+    for off in (0, 8, 1):
+        a = torch.randn(T, B, Kd + 16, device=DEV).to(torch.bfloat16)[:, :, off:off + Kd]
+        wide = torch.full((T, B, N + 3), 7.0, dtype=torch.bfloat16, device=DEV)
+        got = K().batched_linear(a, w, wide[:, :, 2:N + 2])
+        want = torch.stack([a[:, b].double() @ w[b].double().T for b in range(B)], 1)
+        size = torch.stack([a[:, b].double().abs() @ w[b].double().abs().T for b in range(B)], 1)
+        # a float sum of Kd products in any order, then one rounding to bfloat16
+        assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + (Kd + 8) * 2.0 ** -24 * size).all())
+        assert bool((wide[:, :, [0, 1, N + 2]] == 7.0).all())
