@@ -1799,12 +1799,10 @@ def _moe_takes_wide_tiles(pairs: int, experts: int, ff: int) -> bool:
     """Whether the experts' products run in tiles of up to 256 rows by 256 matrix rows (a work-group of one per CU) and not in
     tiles of 64 by 128.  They fetch each matrix once and the rows half as often, which pays from few rows on where there are
     twice as many tiles as CUs (64 experts of 4,096 x 2,048, both products: 18 rows per expert 647 against 693 us, 90: 754
-    against 932, 192: 1,066 against 1,475; of 2,048 x 1,408: 18 rows 239 against 246, 192: 433 against 616); between one and two
-    tiles per CU only where they are full (32 experts of 1,024 x 512: 384 rows 109 against 124 us, 188 rows, with half a
-    tile per CU, 101 against 75)."""
+    against 932, 192: 1,066 against 1,475; of 2,048 x 1,408: 18 rows 239 against 246, 192: 433 against 616), and not where there
+    are fewer (32 experts of 1,024 x 512: 188 rows, with half a tile per CU, 101 against 75 us, 562 rows 183 against 169)."""
     rows = -(-pairs // experts)
-    tiles = experts * -(-rows // MOE_WIDE_TILE) * -(-ff // 128)
-    return tiles >= 512 or (tiles >= 256 and rows >= MOE_WIDE_TILE)
+    return experts * -(-rows // MOE_WIDE_TILE) * -(-ff // 128) >= 512
 
 
 def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
