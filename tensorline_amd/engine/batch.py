@@ -40,6 +40,8 @@ class StepFacts:
     # The longest context the engine will ever run, if the caller knows it (0: unknown).  Choices
     # that must be the same in every step of an engine are made for it.
     fit_context: int = 0
+    # what a part worked out from the facts above for one layer of the step, by a key of its own, for the step's other layers
+    worked_out: dict = field(default_factory=dict, compare=False, repr=False)
 
 
 @dataclass

@@ -14,6 +14,7 @@ import tempfile
 import threading
 import warnings
 from dataclasses import dataclass
+from typing import NamedTuple
 
 import torch
 
@@ -63,15 +64,19 @@ def require_gpu(device) -> torch.device:
     return dev
 
 
+_entry_points: dict[str, object] = {}
+
+
 def _call(name: str, *args) -> None:
-    fn = getattr(library(), name)
-    rc = fn(*args)
-    if rc != 0:
+    fn = _entry_points.get(name)
+    if fn is None:
+        fn = _entry_points[name] = getattr(library(), name)
+    if fn(*args) != 0:
         raise KernelError(library().tl_last_error().decode("utf-8", "replace"))
 
 
 def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
@@ -91,19 +96,26 @@ def _check(cond: bool, msg: str) -> None:
 
 
 def _on_gpu(*tensors: torch.Tensor | None) -> None:
-    dev = None
+    """Every tensor is on one and the same GPU.  (Called before every launch: messages are made only where one is raised.)"""
+    first = None
     for t in tensors:
         if t is None:
             continue
-        _check(t.is_cuda, f"tensor of shape {tuple(t.shape)} is on {t.device}, not on the GPU")
-        dev = dev or t.device
-        _check(t.device == dev, "tensors are on different devices")
+        index = t.get_device()                       # -1 on the CPU
+        if index != first:
+            if index < 0 or not t.is_cuda:
+                raise KernelError(f"tensor of shape {tuple(t.shape)} is on {t.device}, not on the GPU")
+            if first is not None:
+                raise KernelError("tensors are on different devices")
+            first = index
 
 
 def _i32(t: torch.Tensor, what: str, n: int | None = None) -> None:
-    _check(t.dtype == torch.int32 and t.is_contiguous(), f"{what} must be a contiguous int32 tensor")
+    if not (t.dtype == torch.int32 and t.is_contiguous()):
+        raise KernelError(f"{what} must be a contiguous int32 tensor")
     if n is not None:
-        _check(t.numel() >= n, f"{what} has {t.numel()} entries, {n} are needed")
+        if not (t.numel() >= n):
+            raise KernelError(f"{what} has {t.numel()} entries, {n} are needed")
 
 
 # ---------------------------------------------------------------------------------------------
@@ -337,8 +349,8 @@ def add_rmsnorm(x: torch.Tensor, residual: "torch.Tensor | ShareSum | None", wei
     _on_gpu(x, residual, weight, rows, out)
     _check(x.dtype == torch.float32 and x.dim() == 2 and x.is_contiguous(), "add_rmsnorm: x must be contiguous float32 [T, H]")
     T, H = x.shape
-    _check(weight.dtype == torch.float32 and weight.is_contiguous() and weight.numel() == H,
-           f"add_rmsnorm: weight must be float32 of {H} entries")
+    if not (weight.dtype == torch.float32 and weight.is_contiguous() and weight.numel() == H):
+        raise KernelError(f"add_rmsnorm: weight must be float32 of {H} entries")
     res_code = F32
     if residual is not None:
         _check(residual.is_contiguous() and tuple(residual.shape) == (T, H), "add_rmsnorm: residual must match x")
@@ -391,12 +403,12 @@ def shuffle_weight_float(weight: torch.Tensor) -> torch.Tensor | None:
 
 def _check_shuffled(shuffled: torch.Tensor, N: int, K: int) -> None:
     if shuffled.dtype == torch.float32:
-        _check(shuffled.is_contiguous() and tuple(shuffled.shape) == (-(-N // 16), -(-K // 16), 4, 16, 4),
-               f"linear: the shuffled float weight copy does not belong to a [{N}, {K}] matrix")
+        if not (shuffled.is_contiguous() and tuple(shuffled.shape) == (-(-N // 16), -(-K // 16), 4, 16, 4)):
+            raise KernelError(f"linear: the shuffled float weight copy does not belong to a [{N}, {K}] matrix")
         return
-    _check(shuffled.dtype == torch.bfloat16 and shuffled.is_contiguous()
-           and tuple(shuffled.shape) == (-(-N // 16), -(-K // 32), 4, 16, 8),
-           f"linear: the shuffled weight copy does not belong to a [{N}, {K}] matrix")
+    if not (shuffled.dtype == torch.bfloat16 and shuffled.is_contiguous()
+            and tuple(shuffled.shape) == (-(-N // 16), -(-K // 32), 4, 16, 8)):
+        raise KernelError(f"linear: the shuffled weight copy does not belong to a [{N}, {K}] matrix")
 
 
 @dataclass
@@ -467,10 +479,10 @@ def _norm_args(owed: NormedRows | None, sink: NormSink | None, M: int, N: int, d
     if sink is not None:
         r, w = sink.resid, sink.weight
         _on_gpu(r, w)
-        _check(r.dtype == torch.float32 and tuple(r.shape) == (M, N) and r.stride(1) == 1,
-               f"residual sink: the residual must be float32 [{M}, {N}]")
-        _check(w.dtype == torch.float32 and w.is_contiguous() and w.numel() == N,
-               f"residual sink: the norm weight must be float32 of {N} entries")
+        if not (r.dtype == torch.float32 and tuple(r.shape) == (M, N) and r.stride(1) == 1):
+            raise KernelError(f"residual sink: the residual must be float32 [{M}, {N}]")
+        if not (w.dtype == torch.float32 and w.is_contiguous() and w.numel() == N):
+            raise KernelError(f"residual sink: the norm weight must be float32 of {N} entries")
         parts = -(-N // columns_per_partial)
         produced = NormedRows(torch.empty(M, N, dtype=torch.bfloat16, device=device),
                               torch.empty(parts, M, dtype=torch.float32, device=device), N, float(sink.eps))
@@ -501,11 +513,12 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
                 and not _few_rows_go_to_rows64(weight.shape[0], K)):
             _on_gpu(a, weight, bias, shuffled)
             N = weight.shape[0]
-            _check(weight.shape[1] == K, f"linear: input has K={K}, weight has K={weight.shape[1]}")
+            if not (weight.shape[1] == K):
+                raise KernelError(f"linear: input has K={K}, weight has K={weight.shape[1]}")
             _check_shuffled(shuffled, N, K)
             if bias is not None:
-                _check(bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == N,
-                       f"linear: bias must be float32 of {N} entries")
+                if not (bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == N):
+                    raise KernelError(f"linear: bias must be float32 of {N} entries")
             na = _NormArgs()
             na.act = 1
             res = torch.empty(M, N, dtype=out_dtype or a.dtype, device=a.device)
@@ -521,10 +534,11 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
     _check(weight.dim() == 2 and weight.is_contiguous(), "linear: weight must be a contiguous [N, K] matrix")
     M, K = a.shape
     N = weight.shape[0]
-    _check(weight.shape[1] == K, f"linear: input has K={K}, weight has K={weight.shape[1]}")
+    if not (weight.shape[1] == K):
+        raise KernelError(f"linear: input has K={K}, weight has K={weight.shape[1]}")
     if bias is not None:
-        _check(bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == N,
-               f"linear: bias must be float32 of {N} entries")
+        if not (bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == N):
+            raise KernelError(f"linear: bias must be float32 of {N} entries")
     out_dtype = out_dtype or a.dtype
     if owed is not None or sink is not None:
         lda = a.stride(0) if M > 1 else K
@@ -733,7 +747,8 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
     few-row bfloat16 batches (it streams the ``shuffled`` copy), product then SiLU-multiply otherwise.
     ``h`` may be :class:`NormedRows` (few-row kernel only).  ``activation`` "gelu_tanh": the tanh form of GELU
     passes the gate instead of SiLU (in the streaming kernels' epilogues, or by a pass over the product)."""
-    _check(activation in GLU_ACTIVATIONS, f"swiglu_gate_up: unknown activation {activation!r}")
+    if not (activation in GLU_ACTIVATIONS):
+        raise KernelError(f"swiglu_gate_up: unknown activation {activation!r}")
     if activation != "silu":
         _check(not isinstance(h, NormedRows), "swiglu_gate_up: only SiLU rides on a product that carries a norm")
         M, K = h.shape
@@ -782,13 +797,12 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
 
 def _check_caches(k_cache, v_cache, dtype, num_kv_heads, head_dim, who: str) -> None:
     """Keys are paged as [pages, page, nkv, d]; values as [pages, nkv, d, page] (transposed in the page)."""
-    _check(k_cache.dtype == dtype and k_cache.is_contiguous() and k_cache.dim() == 4
-           and k_cache.shape[2] == num_kv_heads and k_cache.shape[3] == head_dim,
-           f"{who}: key cache must be contiguous [pages, page, nkv, d] of the activation dtype")
+    if not (k_cache.dtype == dtype and k_cache.is_contiguous() and k_cache.dim() == 4
+            and k_cache.shape[2] == num_kv_heads and k_cache.shape[3] == head_dim):
+        raise KernelError(f"{who}: key cache must be contiguous [pages, page, nkv, d] of the activation dtype")
     pages, page = k_cache.shape[0], k_cache.shape[1]
-    _check(v_cache.dtype == dtype and v_cache.is_contiguous()
-           and tuple(v_cache.shape) == (pages, num_kv_heads, head_dim, page),
-           f"{who}: value cache must be contiguous [pages, nkv, d, page] matching the key cache")
+    if not (v_cache.dtype == dtype and v_cache.is_contiguous() and tuple(v_cache.shape) == (pages, num_kv_heads, head_dim, page)):
+        raise KernelError(f"{who}: value cache must be contiguous [pages, nkv, d, page] matching the key cache")
 
 
 def qkv_rope_store(h: torch.Tensor | NormedRows, shuffled: torch.Tensor, bias: torch.Tensor | None, pos: torch.Tensor,
@@ -848,14 +862,15 @@ def rope_store(qkv: torch.Tensor, pos: torch.Tensor, inv_freq: torch.Tensor | No
                "rope_store: the bias must be float32 with one entry per column")
     T = qkv.shape[0]
     width = (num_heads + 2 * num_kv_heads) * head_dim
-    _check(qkv.dim() == 2 and qkv.is_contiguous() and qkv.shape[1] == width,
-           f"rope_store: qkv must be contiguous [T, {width}], got {tuple(qkv.shape)}")
+    if not (qkv.dim() == 2 and qkv.is_contiguous() and qkv.shape[1] == width):
+        raise KernelError(f"rope_store: qkv must be contiguous [T, {width}], got {tuple(qkv.shape)}")
     _i32(pos, "pos", T)
     rot = 0
     if inv_freq is not None:
         _check(inv_freq.dtype == torch.float32 and inv_freq.is_contiguous(), "rope_store: inv_freq must be float32")
         rot = 2 * inv_freq.numel()
-        _check(rot <= head_dim, f"rope_store: rotary width {rot} exceeds the head size {head_dim}")
+        if not (rot <= head_dim):
+            raise KernelError(f"rope_store: rotary width {rot} exceeds the head size {head_dim}")
     write = k_cache is not None
     if write:
         _check(v_cache is not None and slots is not None, "rope_store: cache write needs k_cache, v_cache and slots")
@@ -957,6 +972,53 @@ def _tile32_waves(q_lens, starts, num_heads: int) -> int:
     return 8 if keys >= 4096 and cols * num_heads >= 128 * 256 else 0          # at least 128 such work-groups
 
 
+class _AttentionLaunch(NamedTuple):
+    """What the host-side facts of a step say about the launches of the matrix-core attention."""
+    singles: int                   # one-token sequences that could get a launch of their own
+    own_split: tuple | None        # (keys per split, splits) of that launch, if they get it
+    nt: int                        # column tiles of 16 per wave
+    max_groups: int                # independent waves: the most a sequence has
+    total128: int                  # work-groups of 128 columns
+    total32: int                   # work-groups of the kernel with 32 columns per wave
+    split_len: int                 # keys per split and their number (0, 1: none)
+    nsplit: int
+    waves32: int                   # waves of the kernel with 32 columns per wave, 0: not that kernel
+    chains: int                    # chains of tiles per work-group, 0: independent waves
+
+
+def _attention_launch(plan, S: int, num_heads: int, num_kv_heads: int, head_dim: int, window: int, keep_first: int, chunk: int,
+                      path, split_keys, route_singles, has_singles: bool) -> _AttentionLaunch:
+    G = num_heads // num_kv_heads
+    singles = one_token_sequences(plan) if has_singles and split_keys is None and route_singles is not False else []
+    own = None
+    if singles:
+        ctx1 = max([plan.starts[s] + 1 for s in singles if s < len(plan.starts)] + [1])
+        split_len, nsplit = _key_splits(len(singles), num_kv_heads, ctx1, plan.fit_context)
+        if route_singles or (route_singles is None and nsplit > 1 and _singles_get_own_launch(
+                plan, singles, num_heads, num_kv_heads, head_dim,
+                (window + keep_first) if window else chunk)):               # the most keys such a token reads
+            own = (split_len, nsplit)
+    q_lens = [n for n in plan.q_lens if n > 1] if own else plan.q_lens
+    nt = 1 if plan.max_query_len * G <= 16 or head_dim == 256 else 2
+    groups = [-(-n * G // (16 * nt)) for n in q_lens]
+    pads = 0 if own else max(0, S - len(groups))            # padding sequences bring one token each
+    total128 = sum(-(-n * G // 128) for n in q_lens) + pads
+    # Splits are fixed runs of keys aligned to absolute positions, so the same keys are summed
+    # together whatever the context length or the launch shape.  Pure decode steps split by the
+    # batch size rounded up to a power of two (what a graph bucket pads to); steps with prompt
+    # portions have enough columns and do not split.
+    split_len, nsplit = 0, 1
+    if split_keys is not None:
+        split_len, nsplit = _fit_key_splits(int(split_keys), plan.max_context, plan.fit_context)
+    elif plan.decode_only:
+        split_len, nsplit = _key_splits(S, num_kv_heads, plan.max_context, plan.fit_context)
+    waves = 8 if path == "mfma-tile32" else _tile32_waves(plan.q_lens, plan.starts, num_heads) if path in (None, "mfma") else 0
+    chains = 0 if path == "mfma-direct" or (head_dim == 256 and plan.max_query_len == 1) \
+        else _tile16_chains(total128, num_kv_heads, path, plan.max_context)
+    return _AttentionLaunch(len(singles), own, nt, max(groups + [1]), total128,
+                            sum(-(-n * G // (32 * waves)) for n in q_lens) + pads if waves else 0, split_len, nsplit, waves, chains)
+
+
 def attention_takes_head_dim(head_dim: int) -> bool:
     """The head sizes the attention kernels take: multiples of 16 up to 256 (32, 64 and 128 on the
     bfloat16 MFMA kernels, the others on the any-shape kernel)."""
@@ -1038,62 +1100,48 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         _i32(q_start, "q_start", S + 1)
         _i32(ctx_start, "ctx_start", S)
         G = num_heads // num_kv_heads
-        skip_single = 0
-        singles = one_token_sequences(plan) if single_seqs is not None and split_keys is None else []
-        if singles and route_singles is not False:
-            _i32(single_seqs, "single_seqs", len(singles))
-            ctx1 = max([plan.starts[s] + 1 for s in singles if s < len(plan.starts)] + [1])
-            split_len, nsplit = _key_splits(len(singles), num_kv_heads, ctx1, plan.fit_context)
-            if route_singles or (route_singles is None and nsplit > 1 and _singles_get_own_launch(
-                    plan, singles, num_heads, num_kv_heads, head_dim,
-                    (int(window) + keep_first) if window else chunk)):      # the most keys such a token reads
-                nt1 = 1 if G <= 16 or head_dim == 256 else 2      # a head size of 256: one column tile per wave (registers)
-                ws = torch.empty(len(singles) * num_heads * nsplit * (head_dim + 2), dtype=torch.float32, device=q.device)
-                n_o = len(singles) * num_heads * nsplit * head_dim
-                _call("tl_attention_mfma", _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(tables), tables.shape[1],
-                      _ptr(q_start), _ptr(ctx_start), _ptr(pos), _ptr(out), o_stride, _ptr(ws[:n_o]), _ptr(ws[n_o:]), T, S,
-                      num_heads, num_kv_heads, head_dim, page, int(window), ctypes.c_float(scale), nt1,
-                      -(-G // (16 * nt1)), nsplit, max(split_len // 32, 1), 0, 0, _ptr(single_seqs), len(singles), 0,
-                      _ptr(sink), cap, keep_first, chunk, _ptr(bias), reach, _stream())
-                skip_single = 1
-        q_lens = [n for n in plan.q_lens if n > 1] if skip_single else plan.q_lens
-        nt = 1 if plan.max_query_len * G <= 16 or head_dim == 256 else 2
-        groups = [-(-n * G // (16 * nt)) for n in q_lens]
-        pads = 0 if skip_single else max(0, S - len(groups))    # padding sequences bring one token each
-        max_groups = max(groups + [1])
-        total128 = sum(-(-n * G // 128) for n in q_lens) + pads
-        # Splits are fixed runs of keys aligned to absolute positions, so the same keys are summed
-        # together whatever the context length or the launch shape.  Pure decode steps split by the
-        # batch size rounded up to a power of two (what a graph bucket pads to); steps with prompt
-        # portions have enough columns and do not split.
-        split_len, nsplit = 0, 1
         if split_keys is not None:
             _check(int(split_keys) % 32 == 0, "paged_attention: a split is a multiple of 32 keys")
-            split_len, nsplit = _fit_key_splits(int(split_keys), plan.max_context, plan.fit_context)
-        elif plan.decode_only:
-            split_len, nsplit = _key_splits(S, num_kv_heads, plan.max_context, plan.fit_context)
+        # the choices are the same for every layer of a step that has these heads and this mask
+        key = (S, num_heads, num_kv_heads, head_dim, window, keep_first, chunk, path, split_keys, route_singles,
+               single_seqs is not None)
+        memo, memo_key = getattr(plan, "worked_out", {}), key + (plan.max_context, plan.fit_context, plan.decode_only)
+        launch = memo.get(memo_key)
+        if launch is None:
+            launch = memo[memo_key] = _attention_launch(plan, *key)
+        if launch.singles:
+            _i32(single_seqs, "single_seqs", launch.singles)
+        if launch.own_split:
+            split_len, nsplit = launch.own_split
+            nt1 = 1 if G <= 16 or head_dim == 256 else 2      # a head size of 256: one column tile per wave (registers)
+            ws = torch.empty(launch.singles * num_heads * nsplit * (head_dim + 2), dtype=torch.float32, device=q.device)
+            n_o = launch.singles * num_heads * nsplit * head_dim
+            _call("tl_attention_mfma", _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(tables), tables.shape[1],
+                  _ptr(q_start), _ptr(ctx_start), _ptr(pos), _ptr(out), o_stride, _ptr(ws[:n_o]), _ptr(ws[n_o:]), T, S,
+                  num_heads, num_kv_heads, head_dim, page, int(window), ctypes.c_float(scale), nt1,
+                  -(-G // (16 * nt1)), nsplit, max(split_len // 32, 1), 0, 0, _ptr(single_seqs), launch.singles, 0,
+                  _ptr(sink), cap, keep_first, chunk, _ptr(bias), reach, _stream())
+        skip_single, nt, max_groups, total128 = 1 if launch.own_split else 0, launch.nt, launch.max_groups, launch.total128
+        split_len, nsplit = launch.split_len, launch.nsplit
         split_blocks = max(split_len // 32, 1)
         ws_o = ws_ml = None
         if nsplit > 1:
             ws = torch.empty(T * num_heads * nsplit * (head_dim + 2), dtype=torch.float32, device=q.device)
             ws_o, ws_ml = ws[:T * num_heads * nsplit * head_dim], ws[T * num_heads * nsplit * head_dim:]
-        waves = 8 if path == "mfma-tile32" else _tile32_waves(plan.q_lens, plan.starts, num_heads) if path in (None, "mfma") else 0
+        waves = launch.waves32
         if (waves and nt == 2 and nsplit == 1 and total128 > 0
                 and library().tl_attention_tile32_takes(head_dim, page, tables.shape[1], S, waves, G * (reach + 1) if bias is not None else 0)):
             # prompt portions behind many keys, head size 64 or 128: 32 columns per wave on the 32x32
             # matrix-core instruction, work-groups of 256 columns
-            cols = 32 * waves
-            total = sum(-(-n * G // cols) for n in q_lens) + pads
             _call("tl_attention_tile32", _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(tables), tables.shape[1],
                   _ptr(q_start), _ptr(ctx_start), _ptr(out), o_stride, T, S, num_heads, num_kv_heads, head_dim, page,
-                  int(window), ctypes.c_float(scale), waves, total, skip_single, _ptr(sink), cap, keep_first, chunk,
+                  int(window), ctypes.c_float(scale), waves, launch.total32, skip_single, _ptr(sink), cap, keep_first, chunk,
                   _ptr(bias), reach, _stream())
             return out
         _call("tl_attention_mfma", _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(tables), tables.shape[1],
               _ptr(q_start), _ptr(ctx_start), _ptr(pos), _ptr(out), o_stride, _ptr(ws_o), _ptr(ws_ml), T, S, num_heads,
               num_kv_heads, head_dim, page, int(window), ctypes.c_float(scale), nt, max_groups, nsplit, split_blocks,
-              0 if path == "mfma-direct" or (head_dim == 256 and plan.max_query_len == 1)
-              else _tile16_chains(total128, num_kv_heads, path, plan.max_context), total128,
+              launch.chains, total128,
               _ptr(None), 0,
               skip_single, _ptr(sink), cap, keep_first, chunk, _ptr(bias), reach, _stream())
         return out
@@ -1109,8 +1157,10 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         q_start[1:] = torch.cumsum(counts, 0)
         max_query_len = int(counts.max().item()) if T else 1
         # a row of a sequence the table does not have would be computed by nobody and merged from nothing
-        _check(int(counts.sum().item()) == T, f"paged_attention: seq_of_token names sequences outside the {S} of the page table")
-    _check(attention_takes_head_dim(head_dim), f"paged_attention: head size {head_dim} must be a multiple of 16, at most 256")
+        if not (int(counts.sum().item()) == T):
+            raise KernelError(f"paged_attention: seq_of_token names sequences outside the {S} of the page table")
+    if not (attention_takes_head_dim(head_dim)):
+        raise KernelError(f"paged_attention: head size {head_dim} must be a multiple of 16, at most 256")
     # Steps of one token per sequence split the keys into runs of GENERIC_SPLIT_KEYS at absolute positions
     # (longer runs only where the longest context the engine ever runs would need more splits than a launch
     # takes), whatever the batch: one work-group per sequence and key/value head would walk a long context alone.
@@ -1173,7 +1223,8 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.Tensor,
     _check(logits.dim() == 2 and logits.dtype == torch.float32 and logits.stride(1) == 1, "sample: logits must be float32 [R, V]")
     R, V = logits.shape
     for name, t in (("temperature", temperature), ("top_p", top_p), ("uniform", uniform)):
-        _check(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == R, f"sample: {name} must be float32 [R]")
+        if not (t.dtype == torch.float32 and t.is_contiguous() and t.numel() == R):
+            raise KernelError(f"sample: {name} must be float32 [R]")
     if out is None:
         out = torch.empty(R, dtype=torch.int32, device=logits.device)
     _i32(out, "sample output", R)
@@ -1190,9 +1241,11 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.Tensor,
 # ---------------------------------------------------------------------------------------------
 # Norms without statistics, gated and grouped norms, token shift, per-layer token input
 def _f32(t: torch.Tensor, what: str, n: int | None = None) -> None:
-    _check(t.dtype == torch.float32 and t.is_contiguous(), f"{what} must be a contiguous float32 tensor")
+    if not (t.dtype == torch.float32 and t.is_contiguous()):
+        raise KernelError(f"{what} must be a contiguous float32 tensor")
     if n is not None:
-        _check(t.numel() == n, f"{what} has {t.numel()} entries, {n} are needed")
+        if not (t.numel() == n):
+            raise KernelError(f"{what} has {t.numel()} entries, {n} are needed")
 
 
 def add_dyt(x: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor, bias: torch.Tensor, alpha: torch.Tensor,
@@ -1287,7 +1340,8 @@ GLU_ACTIVATIONS = {"silu": 0, "gelu_tanh": 1}
 def glu(gate_up: torch.Tensor, activation: str, out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """For a fused [T, 2F] projection (gate columns first): ``act(gate) * up`` [T, F], ``act`` "silu" or
     "gelu_tanh" (``0.5 z (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3)))``), computed in float32."""
-    _check(activation in GLU_ACTIVATIONS, f"glu: unknown activation {activation!r}")
+    if not (activation in GLU_ACTIVATIONS):
+        raise KernelError(f"glu: unknown activation {activation!r}")
     _on_gpu(gate_up)
     _check(gate_up.dim() == 2 and gate_up.is_contiguous() and gate_up.shape[1] % 2 == 0, "glu: input must be contiguous [T, 2F]")
     T, F2 = gate_up.shape
@@ -1480,10 +1534,11 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ctx, st
     _on_gpu(q, k, v, state, decay, wlog, bonus, steps, rate_log, step_bias, skip)
     T = q.shape[0]
     share = int(share) if steps is not None else 1
-    _check(share >= 1 and heads % share == 0, f"linear_recurrence: {heads} heads do not share queries in groups of {share}")
+    if not (share >= 1 and heads % share == 0):
+        raise KernelError(f"linear_recurrence: {heads} heads do not share queries in groups of {share}")
     for name, t, n in (("q", q, heads // share * dk), ("k", k, heads // share * dk), ("v", v, heads * dv)):
-        _check(t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, n),
-               f"linear_recurrence: {name} must be float32 [T, {n}]")
+        if not (t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, n)):
+            raise KernelError(f"linear_recurrence: {name} must be float32 [T, {n}]")
     per_token = 2 if steps is not None else 1 if wlog is not None else 0
     if per_token == 2:
         _check(steps.dtype == torch.float32 and steps.dim() == 2 and steps.stride(1) == 1 and tuple(steps.shape) == (T, heads)
@@ -1589,7 +1644,8 @@ def conv_unit(x: torch.Tensor, taps: torch.Tensor, ctx, state: torch.Tensor, off
     T, C = x.shape
     K = taps.shape[0]
     _check(x.dtype == torch.float32 and x.stride(1) == 1, "conv_unit: the input must be float32 [T, C]")
-    _check(taps.dim() == 2 and taps.shape[1] == C and 1 <= K <= CONV_MAX_TAPS, f"conv_unit: taps must be [up to {CONV_MAX_TAPS}, C]")
+    if not (taps.dim() == 2 and taps.shape[1] == C and 1 <= K <= CONV_MAX_TAPS):
+        raise KernelError(f"conv_unit: taps must be [up to {CONV_MAX_TAPS}, C]")
     _f32(taps, "conv_unit taps")
     _check(offset + (K - 1) * C <= state.shape[1], "conv_unit: the kept inputs do not fit the state")
     kept, stride = _state_ptr(state, offset)
@@ -1619,10 +1675,11 @@ def delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, b: torch.Tenso
     _on_gpu(q, k, v, b, a, rate_log, step_bias, state)
     T = q.shape[0]
     share = int(share)
-    _check(share >= 1 and heads % share == 0, f"delta_rule: {heads} heads do not share queries in groups of {share}")
+    if not (share >= 1 and heads % share == 0):
+        raise KernelError(f"delta_rule: {heads} heads do not share queries in groups of {share}")
     for name, t, n in (("q", q, heads // share * dk), ("k", k, heads // share * dk), ("v", v, heads * dv), ("b", b, heads), ("a", a, heads)):
-        _check(t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, n),
-               f"delta_rule: {name} must be float32 [T, {n}]")
+        if not (t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, n)):
+            raise KernelError(f"delta_rule: {name} must be float32 [T, {n}]")
     _f32(rate_log, "delta_rule rate_log", heads)
     if step_bias is not None:
         _f32(step_bias, "delta_rule step_bias", heads)
@@ -1675,8 +1732,8 @@ def matrix_lstm(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_in: torc
     T = q.shape[0]
     for name, t, n in (("q", q, heads * dk), ("k", k, heads * dk), ("v", v, heads * dv), ("gate_in", gate_in, heads),
                        ("gate_forget", gate_forget, heads)):
-        _check(t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, n),
-               f"matrix_lstm: {name} must be float32 [T, {n}]")
+        if not (t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, n)):
+            raise KernelError(f"matrix_lstm: {name} must be float32 [T, {n}]")
     for name, t in (("bias_in", bias_in), ("bias_forget", bias_forget)):
         if t is not None:
             _f32(t, "matrix_lstm " + name, heads)
@@ -1723,8 +1780,8 @@ def selective_scan(dt_raw: torch.Tensor, dt_bias: torch.Tensor | None, x: torch.
     T, inner = x.shape
     N = a2.shape[0]
     for name, t, n in (("dt", dt_raw, inner), ("z", z, inner), ("[B | C]", bc, 2 * N)):
-        _check(t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, n),
-               f"selective_scan: {name} must be float32 [T, {n}]")
+        if not (t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, n)):
+            raise KernelError(f"selective_scan: {name} must be float32 [T, {n}]")
     _check(x.stride(1) == 1 and tuple(a2.shape) == (N, inner) and N <= SELECTIVE_SCAN_MAX_STATE, "selective_scan: bad x or A")
     _f32(a2, "selective_scan A")
     _f32(skip, "selective_scan D", inner)
@@ -1763,7 +1820,8 @@ def moe_route(logits: torch.Tensor, top: int, weighting: str = "softmax_top", sc
     their scores divided by their sum; with ``correction`` (float32 [E]) groups and experts are chosen by score +
     correction, the weights made of the scores alone.  ``experts``: the first so many columns of ``logits`` are the router's
     (default: all of them)."""
-    _check(weighting in ROUTER_WEIGHTINGS, f"moe_route: unknown weighting {weighting!r}")
+    if not (weighting in ROUTER_WEIGHTINGS):
+        raise KernelError(f"moe_route: unknown weighting {weighting!r}")
     _on_gpu(logits, correction)
     T, E = logits.shape
     if experts is not None:
@@ -1777,8 +1835,8 @@ def moe_route(logits: torch.Tensor, top: int, weighting: str = "softmax_top", sc
     if correction is not None:
         _f32(correction, "moe_route correction", E)
     if weighting == "sigmoid_grouped":
-        _check(groups > 0 and E % groups == 0 and 0 < keep <= groups and top <= keep * (E // groups) and groups <= 64,
-               f"moe_route: {E} experts in {groups} groups of which {keep} are kept do not give {top} choices")
+        if not (groups > 0 and E % groups == 0 and 0 < keep <= groups and top <= keep * (E // groups) and groups <= 64):
+            raise KernelError(f"moe_route: {E} experts in {groups} groups of which {keep} are kept do not give {top} choices")
         _call("tl_moe_route_grouped", _ptr(logits), ldl, _ptr(ids), _ptr(weights), T, E, int(top), int(groups), int(keep),
               _ptr(correction), _stream())
         return ids, weights
@@ -1873,11 +1931,13 @@ def causal_conv(x: torch.Tensor, taps: torch.Tensor, bias: torch.Tensor | None, 
     T, C = x.shape
     K = taps.shape[1]
     _check(x.dtype == torch.float32 and x.stride(1) == 1, "causal_conv: the input must be float32 [T, C]")
-    _check(taps.dim() == 2 and taps.shape[0] == C and 1 <= K <= CONV_MAX_TAPS, f"causal_conv: taps must be [C, up to {CONV_MAX_TAPS}]")
+    if not (taps.dim() == 2 and taps.shape[0] == C and 1 <= K <= CONV_MAX_TAPS):
+        raise KernelError(f"causal_conv: taps must be [C, up to {CONV_MAX_TAPS}]")
     _f32(taps, "causal_conv taps")
     if bias is not None:
         _f32(bias, "causal_conv bias", C)
-    _check(act in ("none", "silu"), f"causal_conv: unknown activation {act!r}")
+    if not (act in ("none", "silu")):
+        raise KernelError(f"causal_conv: unknown activation {act!r}")
     _check(offset + (K - 1) * C <= state.shape[1], "causal_conv: the kept inputs do not fit the state")
     kept, stride = _state_ptr(state, offset)
     out = torch.empty(T, C, dtype=out_dtype, device=x.device)
@@ -1900,8 +1960,8 @@ def gated_scan(gates: torch.Tensor, bias_r: torch.Tensor | None, bias_i: torch.T
     _on_gpu(gates, bias_r, bias_i, u, y, lam, state)
     T, W = u.shape
     for name, t in (("u", u), ("y", y)):
-        _check(t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, W),
-               f"gated_scan: {name} must be float32 [T, {W}]")
+        if not (t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and tuple(t.shape) == (T, W)):
+            raise KernelError(f"gated_scan: {name} must be float32 [T, {W}]")
     _check(gates.dtype == torch.float32 and gates.dim() == 3 and gates.is_contiguous() and gates.shape[0] == T
            and gates.shape[1] * gates.shape[2] == 2 * W and gates.shape[2] % 2 == 0, "gated_scan: gates must be float32 [T, blocks, 2 W / blocks]")
     bw = gates.shape[2] // 2
@@ -2019,14 +2079,16 @@ def conv_rotate_store(proj: torch.Tensor, taps: torch.Tensor, ctx, state: torch.
     K = taps.shape[0]
     _check(proj.dtype == torch.float32 and proj.dim() == 2 and proj.stride(1) == 1 and proj.shape[1] >= C,
            "conv_rotate_store: the projection must be float32 [T, >= C]")
-    _check(taps.dim() == 2 and taps.shape[1] == C and 1 <= K <= CONV_MAX_TAPS, f"conv_rotate_store: taps must be [up to {CONV_MAX_TAPS}, {C}]")
+    if not (taps.dim() == 2 and taps.shape[1] == C and 1 <= K <= CONV_MAX_TAPS):
+        raise KernelError(f"conv_rotate_store: taps must be [up to {CONV_MAX_TAPS}, {C}]")
     _f32(taps, "conv_rotate_store taps")
     _check(state.dtype == torch.float32 and offset + (K - 1) * C <= state.shape[1], "conv_rotate_store: the kept inputs do not fit the state")
     rot = 0
     if freq is not None:
         _f32(freq, "conv_rotate_store freq")
         rot = 2 * freq.numel()
-        _check(rot <= dim, f"conv_rotate_store: rotary width {rot} exceeds the head size {dim}")
+        if not (rot <= dim):
+            raise KernelError(f"conv_rotate_store: rotary width {rot} exceeds the head size {dim}")
     page = 0
     if k_heads:
         _check(v_heads > 0 and k_cache is not None and v_cache is not None and slots is not None, "conv_rotate_store: keys and values need their caches")
