@@ -601,12 +601,18 @@ __device__ __forceinline__ void at_load_to_lds(const void* g, void* lds_base) {
 // A head size of 256 (DC = 8: latent attention, whose query heads share one key/value head) has 128 KB of tiles and up to
 // 256 registers a wave: one work-group per CU.  2,048 fresh tokens of 32 heads take 98 us, where independent
 // waves, each fetching its own fragments for 16 columns, took 457 (512 behind 3,500: 130 against 357).
-template <int DC, int NT, int WAVES, int CH, int MODE>
+//
+// SPLIT: blockIdx.z is a run of `split_tiles` tiles at absolute positions and the work-group walks those of its tiles that
+// lie in it; sums, maxima and accumulators go to the workspace that attn_merge_kernel puts together, as split decode steps
+// leave them there.  For steps whose work-groups leave most CUs idle behind long contexts: 489 tokens behind 3,072 beside 24
+// decoding requests (12 query and 2 key/value heads of 128, 94 work-groups) 45 us with the merge, 62 in two chains.
+template <int DC, int NT, int WAVES, int CH, int MODE, bool SPLIT>
 __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void attn_tile_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int32_t* __restrict__ tables, int NB, const int32_t* __restrict__ q_start,
     const int32_t* __restrict__ ctx_start, bf16_t* __restrict__ out, int out_stride, int S, int nq, int nkv, int bs,
-    int bs_shift, TlMask mask, float scale, int skip_single, const float* __restrict__ sinks, float softcap, TlBias bias) {
+    int bs_shift, TlMask mask, float scale, int skip_single, const float* __restrict__ sinks, float softcap, TlBias bias,
+    float* __restrict__ ws_o, float* __restrict__ ws_ml, int split_tiles) {
     constexpr int THREADS = CH * WAVES * 64;
     constexpr int WCOLS = NT * 16;                       // columns of a wave; WAVES * WCOLS = 128 per work-group
     constexpr int D = DC * 32;
@@ -681,7 +687,7 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
     int group = ngroups - 1 - flat;
     {
         const int total = (int)(gridDim.x * gridDim.y), first = AT_CUS / (int)gridDim.x;
-        if (CH == 1 && DC < 8 && total > AT_CUS && total <= 2 * AT_CUS && flat >= first) group = flat - first;
+        if (CH == 1 && DC < 8 && !SPLIT && total > AT_CUS && total <= 2 * AT_CUS && flat >= first) group = flat - first;
     }
     const int wg_col0 = group * 128;
     const int col0 = wg_col0 + wave * WCOLS;
@@ -699,8 +705,18 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
         t_head = (mask.first + AT_KEYS - 1) / AT_KEYS;
         if (t_head > t_lo) t_head = t_lo;
     }
-    const int t_shift = t_lo - t_head, n_tiles = t_head + t_hi - t_lo + 1;
-#define AT_TILE_AT(I) ((I) < t_head ? (I) : (I) + t_shift)
+    int h_first = 0, b_first = t_lo, n_tiles = t_head + t_hi - t_lo + 1;
+    if (SPLIT) {
+        const int z0 = (int)blockIdx.z * split_tiles, z1 = z0 + split_tiles;       // this run's tiles
+        const int h_end = min(t_head, z1), b_end = min(t_hi + 1, z1);
+        h_first = min(z0, t_head);
+        b_first = max(t_lo, z0);
+        t_head = max(h_end - h_first, 0);
+        n_tiles = t_head + max(b_end - b_first, 0);
+        if (n_tiles == 0) return;             // no column of the work-group sees a key of the run; no barrier is missed
+    }
+    const int t_shift = b_first - t_head;
+#define AT_TILE_AT(I) ((I) < t_head ? (I) + h_first : (I) + t_shift)
     const int first_key = mask.first;
     int wk_lo = 1, wk_hi = 0;                 // empty for a wave without columns
     if (wave_active) {
@@ -876,6 +892,17 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
         float l_tot = l_run[j];
         l_tot += __shfl_xor(l_tot, 16, TL_WAVE);
         l_tot += __shfl_xor(l_tot, 32, TL_WAVE);
+        if (SPLIT) {
+            const size_t part = ((size_t)row_col[j] * nq + head_col[j]) * gridDim.z + blockIdx.z;
+            float* wp = ws_o + part * D + 4 * g;
+#pragma unroll
+            for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4*>(wp + db * 16) = acc[j][db];
+            if (g == 0) {
+                ws_ml[part * 2] = m_run[j];
+                ws_ml[part * 2 + 1] = l_tot;
+            }
+            continue;
+        }
         if (sinks) l_tot += exp2f(sinks[head_col[j]] * AM_LOG2E - m_run[j]);       // the head's sink: a key without a value
         const float inv = 1.0f / l_tot;
         bf16_t* op = out + (size_t)row_col[j] * out_stride + (size_t)head_col[j] * D + 4 * g;
@@ -1040,7 +1067,8 @@ static void launch_attn(int NT, dim3 grid, int wg_waves, hipStream_t stream, con
 // (the tokens' positions), ws_o holds T*nq*nsplit*d floats and ws_ml T*nq*nsplit*2.  shared != 0
 // runs unsplit steps with prompt portions on the kernel that shares keys and values through LDS
 // (when the page size and the table length allow it), shared == 2 with two chains of tiles per
-// work-group where their buffers fit; shared == 0 keeps them on independent waves.
+// work-group where their buffers fit; shared == 0 keeps them on independent waves.  With nsplit > 1 and shared
+// != 0 that kernel's walks are cut into the splits (a multiple of 64 keys each), whatever the sequences bring.
 // A step that holds prompt portions and one-token sequences with long contexts may be run as two
 // calls: one with seq_list (int32 [n_list], the indices of one-token sequences; only they are
 // computed, with split keys, and the workspace then holds n_list rows instead of T), and one
@@ -1093,15 +1121,18 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
     const bf16_t *qq = (const bf16_t*)q, *kk = (const bf16_t*)k_cache, *vv = (const bf16_t*)v_cache;
     const bool pow2 = (bs & (bs - 1)) == 0;
     // (a head size of 256 comes with NT = 1, its column tiles where the waves are independent; one chain of tiles fills LDS)
-    if ((NT == 2 || d == 256) && nsplit == 1 && shared && pow2 && !seq_list && total_groups128 > 0 &&
+    const bool tiles_split = nsplit > 1 && shared;          // a step with portions whose walks are dealt out by runs of keys
+    if ((NT == 2 || d == 256) && (nsplit == 1 || tiles_split) && shared && pow2 && !seq_list && total_groups128 > 0 &&
         at_lds_bytes(d / 32, NB, S, bias_floats) <= 160 * 1024) {
         // 128 columns per work-group, keys and values shared through LDS; shared == 2 asks for two
         // chains per work-group where their tiles fit LDS
         int bs_shift = 0;
         while ((1 << bs_shift) < bs) ++bs_shift;
         TL_CHECK_ARG(total_groups128 <= 65535, "tl_attention_mfma: %d column groups are more than a launch takes", total_groups128);
-        dim3 sgrid(nkv, (unsigned)total_groups128, 1);
-        const int chains = (shared == 2 && d != 256 && at_lds_bytes(d / 32, NB, S, bias_floats, 2) <= 160 * 1024) ? 2 : 1;
+        TL_CHECK_ARG(!tiles_split || (split_blocks % 2 == 0 && !skip_single && max_tile_groups >= 1),
+                     "tl_attention_mfma: runs of keys of the tile kernel are whole tiles of 64, and no sequence is left out");
+        dim3 sgrid(nkv, (unsigned)total_groups128, tiles_split ? nsplit : 1);
+        const int chains = (shared == 2 && d != 256 && !tiles_split && at_lds_bytes(d / 32, NB, S, bias_floats, 2) <= 160 * 1024) ? 2 : 1;
         const size_t lds = at_lds_bytes(d / 32, NB, S, bias_floats, chains);
 #define TL_TILE_CASE(DCV)                                                                                             \
     do {                                                                                                              \
@@ -1111,19 +1142,25 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
     } while (0)
 #define TL_TILE_CASE_256()                                                                                            \
     do {                                                                                                              \
-        if (bias_table) TL_TILE_GO_(8, 1, 2);                                                                         \
-        else if (softcap > 0.f) TL_TILE_GO_(8, 1, 1);                                                                 \
-        else TL_TILE_GO_(8, 1, 0);                                                                                    \
+        if (bias_table) TL_TILE_256(2);                                                                               \
+        else if (softcap > 0.f) TL_TILE_256(1);                                                                       \
+        else TL_TILE_256(0);                                                                                          \
+    } while (0)
+#define TL_TILE_256(MODEV)                                                                                            \
+    do {                                                                                                              \
+        if (tiles_split) TL_TILE_GO_(8, 1, MODEV, true);                                                              \
+        else TL_TILE_GO_(8, 1, MODEV, false);                                                                         \
     } while (0)
 #define TL_TILE_GO(DCV, MODEV)                                                                                        \
     do {                                                                                                              \
-        if (chains == 2) TL_TILE_GO_(DCV, 2, MODEV);                                                                  \
-        else TL_TILE_GO_(DCV, 1, MODEV);                                                                              \
+        if (tiles_split) TL_TILE_GO_(DCV, 1, MODEV, true);                                                            \
+        else if (chains == 2) TL_TILE_GO_(DCV, 2, MODEV, false);                                                      \
+        else TL_TILE_GO_(DCV, 1, MODEV, false);                                                                       \
     } while (0)
-#define TL_TILE_GO_(DCV, CHV, MODEV)                                                                                  \
-    hipLaunchKernelGGL((attn_tile_kernel<DCV, AT_NT, 8 / AT_NT, CHV, MODEV>), sgrid, dim3(CHV * 64 * 8 / AT_NT), lds, stream, \
+#define TL_TILE_GO_(DCV, CHV, MODEV, SPLITV)                                                                                  \
+    hipLaunchKernelGGL((attn_tile_kernel<DCV, AT_NT, 8 / AT_NT, CHV, MODEV, SPLITV>), sgrid, dim3(CHV * 64 * 8 / AT_NT), lds, stream, \
                        qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride, S, nq, nkv, bs, \
-                       bs_shift, mask, scale, skip_single, sinks, softcap, bias)
+                       bs_shift, mask, scale, skip_single, sinks, softcap, bias, ws_o, ws_ml, split_blocks / 2)
         if (d == 32) TL_TILE_CASE(1);
         else if (d == 64) TL_TILE_CASE(2);
         else if (d == 128) TL_TILE_CASE(4);
@@ -1132,9 +1169,10 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
 #undef TL_TILE_GO_
 #undef TL_TILE_GO
 #undef TL_TILE_CASE
+#undef TL_TILE_256
         TL_CHECK_LAUNCH("tl_attention_mfma tiles");
-        return 0;
-    }
+        if (!tiles_split) return 0;
+    } else
     if (d == 32)
         launch_attn<1>(NT, grid, wg_waves, stream, qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride,
                        ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias);

@@ -972,6 +972,34 @@ def _tile32_waves(q_lens, starts, num_heads: int) -> int:
     return 8 if keys >= 4096 and cols * num_heads >= 128 * 256 else 0          # at least 128 such work-groups
 
 
+def _portion_splits(plan, S: int, num_heads: int, num_kv_heads: int, head_dim: int, window: int, keep_first: int, chunk: int,
+                    total128: int) -> tuple[int, int]:
+    """(keys per run, number of runs) for a step with prompt portions; (0, 1): every work-group of 128 columns walks its keys
+    alone.  Where there is at most one work-group per two CUs, the longest walk sets the time, about 1.05 us per tile of 64 keys
+    in two chains (0.75 us at head sizes up to 64, 2.15 us at 256, in one chain); in runs at absolute positions, two work-groups
+    per CU (one at 256), a tile takes 1.5 us (1.1, 2) and the sums of every run pass through memory once.  Chosen where that is
+    estimated a quarter faster.  Measured, runs against walks, us: 64 tokens behind 3,000 (28 / 4 heads of 128) 27 / 52; 512
+    behind 8,192 107 / 136; 300 behind 3,000 (14 / 2 of 64) 28 / 40, but 1,000 behind 3,000 50 / 48; 64 behind 4,000 (16 / 1
+    of 256) 28 / 124; 1,024 behind 1,024 (12 / 2 of 128) 48 / 40, 600 behind 600 29 / 28."""
+    groups = total128 * num_kv_heads
+    sees = [min(st + n, n + window + keep_first if window else st + n, n + chunk if chunk else st + n)
+            for n, st in zip(plan.q_lens, plan.starts)]
+    longest = max(sees + [1])
+    if groups > 128 or longest < 1024:
+        return 0, 1
+    rows = sum(plan.q_lens) + max(0, S - len(plan.q_lens))
+    walk, tile, fit = (0.75, 1.1, 512) if head_dim <= 64 else (1.05, 1.5, 512) if head_dim <= 128 else (2.15, 2.0, 256)
+    best, best_us = (0, 1), 0.75 * walk * longest / 64
+    for run in (256, 512, 1024, 2048):
+        n, visited = -(-plan.max_context // run), -(-longest // run) + 1
+        if n < 2 or n > MAX_KEY_SPLITS or rows * num_heads * n * (head_dim + 2) > 1 << 26:
+            continue
+        us = tile * run / 64 * max(1, -(-groups * min(n, visited) // fit)) + 9 + rows * num_heads * min(n, visited) * head_dim * 8 / 3e6
+        if us < best_us:
+            best, best_us = (run, n), us
+    return best
+
+
 class _AttentionLaunch(NamedTuple):
     """What the host-side facts of a step say about the launches of the matrix-core attention."""
     singles: int                   # one-token sequences that could get a launch of their own
@@ -1006,14 +1034,17 @@ def _attention_launch(plan, S: int, num_heads: int, num_kv_heads: int, head_dim:
     # Splits are fixed runs of keys aligned to absolute positions, so the same keys are summed
     # together whatever the context length or the launch shape.  Pure decode steps split by the
     # batch size rounded up to a power of two (what a graph bucket pads to); steps with prompt
-    # portions have enough columns and do not split.
+    # portions only where their columns leave most of the GPU idle behind long contexts.
     split_len, nsplit = 0, 1
     if split_keys is not None:
         split_len, nsplit = _fit_key_splits(int(split_keys), plan.max_context, plan.fit_context)
     elif plan.decode_only:
         split_len, nsplit = _key_splits(S, num_kv_heads, plan.max_context, plan.fit_context)
-    waves = 8 if path == "mfma-tile32" else _tile32_waves(plan.q_lens, plan.starts, num_heads) if path in (None, "mfma") else 0
-    chains = 0 if path == "mfma-direct" or (head_dim == 256 and plan.max_query_len == 1) \
+    elif path is None and route_singles is None and not own:
+        split_len, nsplit = _portion_splits(plan, S, num_heads, num_kv_heads, head_dim, window, keep_first, chunk, total128)
+    runs = nsplit > 1 and not plan.decode_only and split_keys is None      # the tile kernel's walks in runs of keys
+    waves = 8 if path == "mfma-tile32" else _tile32_waves(plan.q_lens, plan.starts, num_heads) if path in (None, "mfma") and not runs else 0
+    chains = 0 if path == "mfma-direct" or (head_dim == 256 and plan.max_query_len == 1) or (nsplit > 1 and not runs) \
         else _tile16_chains(total128, num_kv_heads, path, plan.max_context)
     return _AttentionLaunch(len(singles), own, nt, max(groups + [1]), total128,
                             sum(-(-n * G // (32 * waves)) for n in q_lens) + pads if waves else 0, split_len, nsplit, waves, chains)
@@ -1058,7 +1089,8 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     wave, work-groups of 256, head sizes 64 and 128) or "mfma-direct" (independent waves);
     ``split_keys`` forces the number of keys per split (0: no split).
 
-    A step with prompt portions does not split keys: its one-token sequences would each be walked
+    A step with prompt portions splits keys only where its columns leave most of the GPU idle
+    (``_portion_splits``): its one-token sequences would each be walked
     by one work-group from the first key to the last.  With ``single_seqs`` (int32, the indices
     ``one_token_sequences(plan)`` on the device) they are computed by a launch of their own where that is
     estimated to be faster (``_singles_get_own_launch``), split like a decode step of that many

@@ -1146,3 +1146,26 @@ def test_batched_linear_bfloat16(T, B, N, Kd):
         # a float sum of Kd products in any order, then one rounding to bfloat16
         assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + (Kd + 8) * 2.0 ** -24 * size).all())
         assert bool((wide[:, :, [0, 1, N + 2]] == 7.0).all())
+
+
+@pytest.mark.parametrize("nq,nkv,d,bs,lens,q_lens,kw", [
+    (12, 2, 128, 16, [3200, 40, 1, 1400, 129], [70, 40, 1, 1, 129], {}),                # behind a long context, beside one-token requests
+    (14, 2, 64, 16, [4097, 300], [65, 1], dict(spike=True)),                            # one far key dominates
+    (4, 1, 32, 8, [2048, 2047], [3, 130], {}),                                          # runs' edges
+    (8, 1, 256, 16, [3000, 64], [40, 64], dict(sink=True)),
+    (8, 2, 128, 16, [4000, 900], [100, 1], dict(window=1500, keep_first=70)),           # leading runs empty, first keys in a run of their own
+    (8, 2, 64, 16, [4000, 2100], [100, 30], dict(chunk=1600, softcap=20.0)),
+    (4, 4, 32, 64, [2500, 2000], [60, 5], dict(bias=True)),
+    (6, 1, 128, 24, [3000], [40], {}),                                                  # pages of no power of two: independent waves in runs
+])
+def test_attention_portions_in_runs_of_keys(nq, nkv, d, bs, lens, q_lens, kw):
+    """Prompt portions of few columns behind long contexts, their walks cut into runs that a second kernel puts together."""
+    from tensorline_amd.engine.batch import StepFacts
+    if kw.get("bias"):
+        kw = dict(kw, bias=torch.randn(nq, 41))
+    total = sum(-(-n * (nq // nkv) // 128) for n in q_lens)
+    facts = StepFacts(max_context=max(lens), max_query_len=max(q_lens), num_seqs=len(lens), q_lens=q_lens,
+                      starts=[n - q for n, q in zip(lens, q_lens)])
+    assert K()._portion_splits(facts, len(lens), nq, nkv, d, kw.get("window", 0), kw.get("keep_first", 0), kw.get("chunk", 0), total)[1] > 1
+    got, want = _attention_case(torch.bfloat16, nq, nkv, d, bs, lens, q_lens, seed=21, **kw)
+    torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
