@@ -96,7 +96,7 @@ struct TlNormArgs {
     const float* next_weight;  // [N]
     bf16_t* a_out;             // [M, a_ld] = resid * next_weight
     int a_ld;
-    float* ss_out;             // [tiles, ss_out_ld]: row `tile` gets the tile's sums of resid^2, one per row
+    float* ss_out;             // [work-groups, ss_out_ld]: a row gets its work-group's sums of resid^2, one per row of A
     int ss_out_ld;
     // activation of a plain product's output, after the bias (the few-row kernel; no sink with it):
     // 0 none, 1 the square of relu; 2, in the gated forms of both kernels only: the tanh form of GELU passes

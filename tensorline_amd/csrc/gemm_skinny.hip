@@ -69,7 +69,11 @@ __device__ __forceinline__ void wave_lds_order() {
     asm volatile("" ::: "memory");
 }
 
-template <int MT, int MODE, typename TO>
+// SPLIT 2 (plain products): a work-group owns half a tile, eight columns, so that twice as many CUs stream a narrow matrix.  A load
+// of a wave still brings 1 KB: the half's rows of two chunks of 32 k, lanes r < 8 of the first, r >= 8 of the second.  Two
+// products per load, one with each chunk's activations, of which the rows 0..7 and the rows 8..15 are kept; the two
+// halves are added at the end.
+template <int MT, int MODE, typename TO, int SPLIT>
 __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_kernel(
     const bf16_t* __restrict__ A, const uint4* __restrict__ Ws, const float* __restrict__ bias, TO* __restrict__ C,
     int M, int n_out, int K, int K32, int lda, int ldc, int second_tile, QkvArgs qa, TlNormArgs na) {
@@ -79,24 +83,29 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
     __shared__ float sh_sq[16 * 17];                 // [row][column of the tile] squares of the new residual
     constexpr bool DUAL = MODE != MODE_PLAIN;
     constexpr int NACC = MT * (DUAL ? 2 : 1);
-    constexpr int XS_PER_WAVE = MT * SK_UNITS * SK_ROWPAD;     // in uint4
+    constexpr int COLS = 16 / SPLIT;                           // columns of a work-group
+    static_assert(SPLIT == 1 || MT == 1, "half tiles come with one tile of rows");
+    constexpr int XS_PER_WAVE = MT * SPLIT * SK_UNITS * SK_ROWPAD;     // in uint4
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
     const int r = lane & 15, g = lane >> 4;
-    int tile = blockIdx.x, tile2 = second_tile + blockIdx.x;
+    const int unit = blockIdx.x / SPLIT, col0 = (blockIdx.x - unit * SPLIT) * COLS;      // tile (pair), first column in it
+    int tile = unit, tile2 = second_tile + unit;
     if (MODE == MODE_QKV) {
         const int pph = qa.d / 32;                   // tile pairs per head
-        const int head = blockIdx.x / pph, j = blockIdx.x - head * pph;
+        const int head = unit / pph, j = unit - head * pph;
         tile = head * (qa.d / 16) + j;
         tile2 = tile + pph;
     }
-    const uint4* w1 = Ws + (size_t)tile * K32 * 64 + lane;
-    const uint4* w2 = DUAL ? Ws + (size_t)tile2 * K32 * 64 + lane : nullptr;
+    // within a chunk: this lane's 16 bytes (SPLIT 2: row col0 + r % 8 of k group g), and which of the load's chunks it reads
+    const int in_chunk = SPLIT == 1 ? lane : 16 * g + col0 + (r & 7), sub = SPLIT == 1 ? 0 : r >> 3;
+    const uint4* w1 = Ws + (size_t)tile * K32 * 64 + in_chunk;
+    const uint4* w2 = DUAL ? Ws + (size_t)tile2 * K32 * 64 + in_chunk : nullptr;
     uint4* xs = smem + (size_t)wave * XS_PER_WAVE;
     const uint4 zero = make_uint4(0, 0, 0, 0);
 
-    f32x4 acc[NACC];
+    f32x4 acc[NACC * SPLIT];                         // [s * NACC + a]: the products with chunk s of a load
 #pragma unroll
-    for (int i = 0; i < NACC; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NACC * SPLIT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // What the epilogue needs from memory is asked for now, so that it has arrived when the sums
     // are done: this thread's partial sums of squares (thread (row, part) owns every nparts-th
@@ -118,16 +127,16 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
         }
     }
     float pre_resid = 0.f, pre_weight = 0.f, pre_bias = 0.f;
-    if (sink && threadIdx.x < 256) {
-        const int l = threadIdx.x & 63, i = (threadIdx.x >> 6) & 3;
-        const int m = l & 15, n = tile * 16 + 4 * (l >> 4) + i;
+    if (sink && threadIdx.x < 256 / SPLIT) {
+        const int l = threadIdx.x & (64 / SPLIT - 1), i = threadIdx.x / (64 / SPLIT) & 3;
+        const int m = l & 15, n = tile * 16 + col0 + 4 * (l >> 4) + i;
         const int mc = m < M ? m : 0, nc = n < n_out ? n : 0;
         pre_resid = na.resid[(size_t)mc * na.resid_ld + nc];
         pre_weight = na.next_weight[nc];
         if (bias) pre_bias = bias[nc];
     }
 
-    const int nsc = (K32 + 3) / 4;                   // steps of 128 k
+    const int nsc = (K32 + 4 * SPLIT - 1) / (4 * SPLIT);     // steps of 128 k (SPLIT 2: 256)
     const int per = (nsc + nwaves - 1) / nwaves;
     const int s0 = wave * per;
     const int s1 = (s0 + per < nsc) ? s0 + per : nsc;
@@ -138,7 +147,7 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
     // unconditional: an address past the end is clamped to a valid one, and what it brings is
     // either never used (rows of A past M feed output rows that are not written; the step after
     // the last is not multiplied) or replaced by zero (k past K).
-    uint4 wf[4], uf[4], wn[4], un[4], xr[MT * 4];
+    uint4 wf[4], uf[4], wn[4], un[4], xr[SPLIT][MT * 4];
     const int xrow0 = lane >> 4, xunit = lane & 15;
     const bf16_t* xp[MT * 4];
 #pragma unroll
@@ -149,17 +158,20 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
     const int last_c = K32 - 1;
     {
         const int sc = (s0 < s1) ? s0 : 0;
-        const int kx = sc * SK_SC + xunit * 8;
-        const int kxc = (kx < K) ? kx : 0;               // past K: the row's first unit, inside the row whatever K is
 #pragma unroll
-        for (int i = 0; i < MT * 4; ++i) xr[i] = *reinterpret_cast<const uint4*>(xp[i] + kxc);
-        if (kx >= K) {
+        for (int h = 0; h < SPLIT; ++h) {
+            const int kx = (sc * SPLIT + h) * SK_SC + xunit * 8;
+            const int kxc = (kx < K) ? kx : 0;           // past K: the row's first unit, inside the row whatever K is
 #pragma unroll
-            for (int i = 0; i < MT * 4; ++i) xr[i] = zero;
+            for (int i = 0; i < MT * 4; ++i) xr[h][i] = *reinterpret_cast<const uint4*>(xp[i] + kxc);
+            if (kx >= K) {
+#pragma unroll
+                for (int i = 0; i < MT * 4; ++i) xr[h][i] = zero;
+            }
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            int c = sc * 4 + i;
+            int c = (sc * 4 + i) * SPLIT + sub;
             if (c > last_c) c = last_c;
             wf[i] = tl_load_stream(w1 + (size_t)c * 64);
             if (DUAL) uf[i] = tl_load_stream(w2 + (size_t)c * 64);
@@ -168,43 +180,56 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
     for (int sc = s0; sc < s1; ++sc) {
         // A rows of this step: registers -> LDS, lane (row = lane/16 + 4i, unit = lane%16)
 #pragma unroll
-        for (int i = 0; i < MT * 4; ++i) {
-            const int row = xrow0 + 4 * i;
-            xs[((row >> 4) * SK_UNITS + xunit) * SK_ROWPAD + (row & 15)] = xr[i];
-        }
+        for (int h = 0; h < SPLIT; ++h)
+#pragma unroll
+            for (int i = 0; i < MT * 4; ++i) {
+                const int row = xrow0 + 4 * i;
+                xs[(((row >> 4) * SPLIT + h) * SK_UNITS + xunit) * SK_ROWPAD + (row & 15)] = xr[h][i];
+            }
         wave_lds_order();
         // request the next step (clamped to the last one when there is none)
         const int sn = (sc + 1 < s1) ? sc + 1 : sc;
-        const int kxn = sn * SK_SC + xunit * 8;
-        const int kxnc = (kxn < K) ? kxn : 0;
 #pragma unroll
-        for (int i = 0; i < MT * 4; ++i) xr[i] = *reinterpret_cast<const uint4*>(xp[i] + kxnc);
+        for (int h = 0; h < SPLIT; ++h) {
+            const int kxn = (sn * SPLIT + h) * SK_SC + xunit * 8;
+            const int kxnc = (kxn < K) ? kxn : 0;
+#pragma unroll
+            for (int i = 0; i < MT * 4; ++i) xr[h][i] = *reinterpret_cast<const uint4*>(xp[i] + kxnc);
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            int c = sn * 4 + i;
+            int c = (sn * 4 + i) * SPLIT + sub;
             if (c > last_c) c = last_c;
             wn[i] = tl_load_stream(w1 + (size_t)c * 64);
             if (DUAL) un[i] = tl_load_stream(w2 + (size_t)c * 64);
         }
         // chunks past K32 of the last step read a clamped chunk: they must count as zero
-        const int cbase = sc * 4;
+        const int cbase = sc * 4 * SPLIT;
 #pragma unroll
         for (int cc = 0; cc < 4; ++cc) {
-            const bool live = cbase + cc <= last_c;
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                uint4 xf = xs[(mt * SK_UNITS + cc * 4 + g) * SK_ROWPAD + r];
-                if (!live) xf = zero;
-                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(wf[cc]), as_frag(xf), acc[mt], 0, 0, 0);
-                if (DUAL)
-                    acc[MT + mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(uf[cc]), as_frag(xf), acc[MT + mt], 0, 0, 0);
+            for (int h = 0; h < SPLIT; ++h) {
+                const bool live = cbase + cc * SPLIT + h <= last_c;
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    uint4 xf = xs[(mt * SPLIT * SK_UNITS + (cc * SPLIT + h) * 4 + g) * SK_ROWPAD + r];
+                    if (!live) xf = zero;
+                    f32x4& a = acc[h * NACC + mt];
+                    a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(wf[cc]), as_frag(xf), a, 0, 0, 0);
+                    if (DUAL) {
+                        f32x4& b = acc[h * NACC + MT + mt];
+                        b = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(uf[cc]), as_frag(xf), b, 0, 0, 0);
+                    }
+                }
             }
         }
         wave_lds_order();
-        if (kxn >= K) {
 #pragma unroll
-            for (int i = 0; i < MT * 4; ++i) xr[i] = zero;
-        }
+        for (int h = 0; h < SPLIT; ++h)
+            if ((sn * SPLIT + h) * SK_SC + xunit * 8 >= K) {
+#pragma unroll
+                for (int i = 0; i < MT * 4; ++i) xr[h][i] = zero;
+            }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             wf[i] = wn[i];
@@ -243,7 +268,8 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
 #pragma unroll
     for (int a = 0; a < NACC; ++a)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) red[((size_t)wave * NACC * 4 + a * 4 + i) * 64 + lane] = acc[a][i];
+        for (int i = 0; i < 4; ++i)          // SPLIT 2: rows 0..7 (g < 2) of the first chunks' products, 8..15 of the second's
+            red[((size_t)wave * NACC * 4 + a * 4 + i) * 64 + lane] = SPLIT == 2 && g >= 2 ? acc[(SPLIT - 1) * NACC + a][i] : acc[a][i];
     if (owed && threadIdx.x < 16) {
         const int nparts = blockDim.x >> 4;
         float ssum = 0.f;
@@ -251,16 +277,20 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
         sh_rstd[threadIdx.x] = 1.0f / sqrtf(ssum / na.dim + na.eps);
     }
     __syncthreads();
-    const int n0 = tile * 16;
-    // element e = (mt, i, l): C[m = mt*16 + l % 16][n = n0 + 4*(l / 16) + i]
-    for (int e = threadIdx.x; e < MT * 4 * 64; e += blockDim.x) {
-        const int l = e & 63, i = (e >> 6) & 3, mt = e >> 8;
+    const int n0 = tile * 16 + col0;
+    // element e = (mt, i, l): C[m = mt*16 + l % 16][n = n0 + 4*(l / 16) + i]; SPLIT 2: l < 32, its other half in lane l + 32
+    for (int e = threadIdx.x; e < MT * 4 * 64 / SPLIT; e += blockDim.x) {
+        const int l = e & (64 / SPLIT - 1), i = e / (64 / SPLIT) & 3, mt = SPLIT == 1 ? e >> 8 : 0;
         const int m = mt * 16 + (l & 15), n = n0 + 4 * (l >> 4) + i;
         if (m >= M || n >= n_out) continue;
         float v = 0.f, u = 0.f;
         for (int w = 0; w < nwaves; ++w) {
             v += red[((size_t)w * NACC * 4 + mt * 4 + i) * 64 + l];
             if (DUAL) u += red[((size_t)w * NACC * 4 + (MT + mt) * 4 + i) * 64 + l];
+            if (SPLIT == 2) {
+                v += red[((size_t)w * NACC * 4 + mt * 4 + i) * 64 + l + 32];
+                if (DUAL) u += red[((size_t)w * NACC * 4 + (MT + mt) * 4 + i) * 64 + l + 32];
+            }
         }
         if (owed) {
             const float rs = sh_rstd[m & 15];
@@ -323,40 +353,49 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
     }
     if (sink) {
         __syncthreads();
-        if ((int)threadIdx.x < M && threadIdx.x < 16) {
+        if ((int)threadIdx.x < M && threadIdx.x < 16 && n0 < n_out) {       // (the last tile's second half may have no column)
             float ssum = 0.f;
-            for (int c = 0; c < 16; ++c) ssum += sh_sq[threadIdx.x * 17 + c];
-            na.ss_out[(size_t)tile * na.ss_out_ld + threadIdx.x] = ssum;
+            for (int c = 0; c < COLS; ++c) ssum += sh_sq[threadIdx.x * 17 + c];
+            na.ss_out[(size_t)blockIdx.x * na.ss_out_ld + threadIdx.x] = ssum;
         }
     }
 }
 
-static size_t lds_per_wave(int MT, int nacc) {
-    const size_t stage = (size_t)MT * SK_UNITS * SK_ROWPAD * sizeof(uint4);
+static size_t lds_per_wave(int MT, int nacc, int split = 1) {
+    const size_t stage = (size_t)MT * split * SK_UNITS * SK_ROWPAD * sizeof(uint4);
     const size_t red = (size_t)nacc * 4 * 64 * sizeof(float);
     return stage > red ? stage : red;
 }
 
-static int pick_waves(int tiles, int nsc, int MT, int nacc, int max_waves) {
+static int pick_waves(int tiles, int nsc, int MT, int nacc, int max_waves, int split) {
     // enough waves in flight to cover HBM latency on 256 CUs; K is split among the waves of a group
     int w = 1;
     while (w < max_waves && tiles * w < 4096 && nsc >= 2 * w) w <<= 1;
-    while (w > 1 && (size_t)w * lds_per_wave(MT, nacc) > SK_MAX_LDS) w >>= 1;
+    while (w > 1 && (size_t)w * lds_per_wave(MT, nacc, split) > SK_MAX_LDS) w >>= 1;
     return w;
 }
 
-template <int MT, int MODE, typename TO>
+// Whether a plain product gives half a tile to a work-group: where whole tiles leave half of the CUs without one and are not so few
+// that nothing streams for long (8 rows, us, whole and half: 896 x 4,864 7.3 and 6.7; 1,536 x 8,960 11.4 and 9.8; 2,048 x 6,144
+// 10.6 and 9.3; 1,024 x 1,024 4.0 and 3.4; but 256 x 2,048 4.4 and 4.4, 3,584 x 3,584 7.5 and 10.2).  With a residual sink only
+// for a K that repays the next product's reading of twice as many partial sums.  By the matrix and its use, not by the rows.
+static int sk_split(int N, int K, bool sink) {
+    const int tiles = tl_ceil_div(N, 16);
+    return tiles > 48 && tiles <= 128 && K >= (sink ? 2048 : 512) ? 2 : 1;
+}
+
+template <int MT, int MODE, typename TO, int SPLIT>
 static void launch_skinny(const bf16_t* A, const uint4* Ws, const float* bias, TO* C, int M, int n_out, int K, int K32,
                           int lda, int ldc, int second_tile, hipStream_t stream, const TlNormArgs& na,
                           QkvArgs qa = QkvArgs()) {
     // the grid: one group per tile, or per pair of tiles in the two-tile modes
-    const int groups = (MODE == MODE_QKV) ? tl_ceil_div(n_out, 32) : tl_ceil_div(n_out, 16);
+    const int groups = ((MODE == MODE_QKV) ? tl_ceil_div(n_out, 32) : tl_ceil_div(n_out, 16)) * SPLIT;
     const int nacc = MT * (MODE != MODE_PLAIN ? 2 : 1);
     // at most 8 waves to a group (4 in the gate/up form): measured at the 7B shapes, 16 waves stream
     // the down projection in 30.9 us and 8 in 28.0, the fused q/k/v projection in 12.1 and 11.3
-    const int nwaves = pick_waves(groups, (K32 + 3) / 4, MT, nacc, MODE == MODE_SWIGLU ? 4 : 8);
-    const size_t smem = (size_t)nwaves * lds_per_wave(MT, nacc);
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, MODE, TO>), dim3(groups), dim3(nwaves * 64), smem, stream, A, Ws, bias, C,
+    const int nwaves = pick_waves(groups, tl_ceil_div(K32, 4 * SPLIT), MT, nacc, MODE == MODE_SWIGLU ? 4 : 8, SPLIT);
+    const size_t smem = (size_t)nwaves * lds_per_wave(MT, nacc, SPLIT);
+    hipLaunchKernelGGL((gemm_skinny_kernel<MT, MODE, TO, SPLIT>), dim3(groups), dim3(nwaves * 64), smem, stream, A, Ws, bias, C,
                        M, n_out, K, K32, lda, ldc, second_tile, qa, na);
 }
 
@@ -364,7 +403,10 @@ template <int DUAL, typename TO>
 static int dispatch_skinny(const bf16_t* A, const uint4* Ws, const float* bias, TO* C, int M, int n_out, int K, int K32,
                            int lda, int ldc, int second_tile, hipStream_t stream, const TlNormArgs& na) {
     // one 16-row MFMA tile of A; more rows go to gemm_rows64.hip
-    launch_skinny<1, DUAL, TO>(A, Ws, bias, C, M, n_out, K, K32, lda, ldc, second_tile, stream, na);
+    if (DUAL == MODE_PLAIN && sk_split(n_out, K, na.resid != nullptr) == 2)
+        launch_skinny<1, DUAL, TO, DUAL == MODE_PLAIN ? 2 : 1>(A, Ws, bias, C, M, n_out, K, K32, lda, ldc, second_tile, stream, na);
+    else
+        launch_skinny<1, DUAL, TO, 1>(A, Ws, bias, C, M, n_out, K, K32, lda, ldc, second_tile, stream, na);
     TL_CHECK_LAUNCH("tl_gemm_skinny");
     return 0;
 }
@@ -396,6 +438,9 @@ static int check_skinny(const void* A, const void* Ws, const void* C, int M, int
     TL_CHECK_ARG(lda >= K && ldc > 0, "tl_gemm_skinny: bad strides");
     return 0;
 }
+
+// Columns per partial sum of squares that a plain product with a residual sink leaves (a work-group's columns).
+extern "C" int tl_gemm_skinny_columns(int N, int K) { return 16 / sk_split(N, K, true); }
 
 // bfloat16 A [M, K] (row stride lda); Ws: the shuffled copy of W [N, K], ceil(N/16) * ceil(K/32) * 512
 // values, zero where it pads; C [M, N] float or bfloat16 (row stride ldc).
@@ -458,8 +503,8 @@ extern "C" int tl_gemm_skinny_qkv_rope(const void* A, const void* Ws, const floa
     qa.nkv = nkv;
     qa.d = d;
     qa.bs = bs;
-    launch_skinny<1, MODE_QKV, bf16_t>((const bf16_t*)A, (const uint4*)Ws, bias, (bf16_t*)nullptr, M, N, K,
-                                       tl_ceil_div(K, 32), lda, N, 0, stream, na, qa);
+    launch_skinny<1, MODE_QKV, bf16_t, 1>((const bf16_t*)A, (const uint4*)Ws, bias, (bf16_t*)nullptr, M, N, K,
+                                          tl_ceil_div(K, 32), lda, N, 0, stream, na, qa);
     TL_CHECK_LAUNCH("tl_gemm_skinny_qkv_rope");
     return 0;
 }

@@ -546,9 +546,9 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
                "linear: a deferred norm needs a streaming bfloat16 kernel (at most 64 rows, a shuffled weight copy)")
         _check_shuffled(shuffled, N, K)
         few = M <= SKINNY_MAX_ROWS and not (_few_rows_go_to_rows64(N, K) and _rows64_ok(a, shuffled, M, K, lda, few_too=True))
-        # a sink's partials: per 16-column tile where the first kernel completes the sums, per 256 columns
-        # where the mid-row product's second kernel does
-        per = 16 if few or library().tl_gemm_rows64_shares(M, N, K) == 1 else 256
+        # a sink's partials: per work-group's columns (16, or 8) where the first kernel completes the sums, per 256
+        # columns where the mid-row product's second kernel does
+        per = library().tl_gemm_skinny_columns(N, K) if few else 16 if library().tl_gemm_rows64_shares(M, N, K) == 1 else 256
         norm, produced = _norm_args(owed, sink, M, N, a.device, per)
         if produced is None:
             out = torch.empty(M, N, dtype=out_dtype, device=a.device)

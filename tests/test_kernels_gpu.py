@@ -1169,3 +1169,33 @@ def test_attention_portions_in_runs_of_keys(nq, nkv, d, bs, lens, q_lens, kw):
     assert K()._portion_splits(facts, len(lens), nq, nkv, d, kw.get("window", 0), kw.get("keep_first", 0), kw.get("chunk", 0), total)[1] > 1
     got, want = _attention_case(torch.bfloat16, nq, nkv, d, bs, lens, q_lens, seed=21, **kw)
     torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
+
+
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("N,Kd", [(784, 2048), (1000, 2056), (2048, 4864), (1030, 520), (896, 2336)])
+def test_few_rows_in_half_tiles(M, N, Kd):
+    """Few-row products whose work-groups own eight columns: an N that ends in either half of a tile, a last step with one
+    chunk, a part of one, or only the first of a load's two; a residual sink and the product that reads its partial
+    sums.  A row has the same bits whatever rows come along."""
+    torch.manual_seed(N + M)
+    a = torch.randn(M, Kd, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    b = torch.randn(N, device=DEV)
+    ws = K().shuffle_weight(w)
+    want = a.double() @ w.double().T + b.double()
+    size = a.double().abs() @ w.double().abs().T + b.double().abs()
+    got = K().linear(a, w, b, out_dtype=torch.float32, shuffled=ws)
+    assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())     # Kd float sums in any order
+    assert torch.equal(K().linear(a[M - 1:], w, b, out_dtype=torch.float32, shuffled=ws)[0], got[M - 1])
+    if N % 8:
+        return                                                   # (the rows a sink leaves are another product's input)
+    resid, gamma = torch.randn(M, N, device=DEV), 1 + 0.1 * torch.randn(N, device=DEV)
+    x = resid.clone()
+    nxt = K().linear(a, w, b, shuffled=ws, sink=K().NormSink(x, gamma, 1e-6))
+    torch.testing.assert_close(x.double(), resid.double() + want, atol=1e-5, rtol=1e-5)
+    assert nxt.sumsq.shape[0] == -(-N // (8 if Kd >= 2048 else 16))      # 1,000: the last tile's second half has no row
+    torch.testing.assert_close(nxt.sumsq.sum(0).double(), x.double().pow(2).sum(1), atol=0, rtol=1e-5)
+    w2 = (torch.randn(512, N, device=DEV) / math.sqrt(N)).to(torch.bfloat16)
+    got2 = K().linear(nxt, w2, None, out_dtype=torch.float32, shuffled=K().shuffle_weight(w2))
+    h = (x * gamma).to(torch.bfloat16).double() / torch.sqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-6)
+    torch.testing.assert_close(got2.double(), h @ w2.double().T, atol=2e-4, rtol=2e-4)
