@@ -1,5 +1,7 @@
 // The entry point of the any-shape attention (attention_generic_kernel.h) and its float instantiations;
-// the bfloat16 ones are compiled in attention_generic_bf16.hip.
+// the bfloat16 ones are compiled in attention_generic_bf16.hip.  Float steps of one token per sequence go to
+// attention_float_decode.h where it takes them.
+#include "attention_float_decode.h"
 #include "attention_generic_kernel.h"
 
 void tl_attention_generic_bf16(const AgLaunch& a);
@@ -60,7 +62,9 @@ extern "C" int tl_attention_generic(const void* q, int q_stride, const void* k_c
     a.mask = TlMask{window, chunk, keep_first}; a.nsplit = nsplit; a.split_keys = split_keys; a.scale = scale; a.keys_over_waves = keys_over_waves;
     a.grid = dim3((unsigned)groups, nkv, chunks * nsplit);
     a.smem = smem; a.stream = stream; a.sinks = sinks; a.softcap = softcap; a.bias = TlBias{bias, bias_reach};
-    if (dtype == TL_F32)
+    if (dtype == TL_F32 && afd_takes(a, max_query_len, S))
+        afd_launch(a, S);
+    else if (dtype == TL_F32)
         ag_launch_all<float>(a);
     else if (dtype == TL_BF16)
         tl_attention_generic_bf16(a);

@@ -542,6 +542,14 @@ struct AgLaunch {
     hipStream_t stream;
 };
 
+// The merge of the splits, if there are any.
+template <typename TT>
+static void ag_merge(const AgLaunch& a) {
+    if (a.nsplit > 1)
+        hipLaunchKernelGGL(attn_generic_merge_kernel<TT>, dim3(a.T, a.nq), dim3(256), 0, a.stream, a.ws_o, a.ws_ml,
+                           (TT*)a.out, a.out_stride, a.nq, a.d, a.nsplit, a.sinks);
+}
+
 // The kernel for head size 16 DB with keys over waves or not, then the merge of the splits: every
 // instantiation of one storage type.  Each storage type has a source file of its own that instantiates
 // this (attention_generic.hip: float, attention_generic_bf16.hip: bfloat16), so that the two halves of
@@ -564,7 +572,5 @@ static void ag_launch_all(const AgLaunch& a) {
     }
 #undef AG_CASE
 #undef AG_LAUNCH_KW
-    if (a.nsplit > 1)
-        hipLaunchKernelGGL(attn_generic_merge_kernel<TT>, dim3(a.T, a.nq), dim3(256), 0, a.stream, a.ws_o, a.ws_ml,
-                           (TT*)a.out, a.out_stride, a.nq, a.d, a.nsplit, a.sinks);
+    ag_merge<TT>(a);
 }

@@ -575,6 +575,7 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
 MAX_KEY_SPLITS = 1024    # key splits the attention merge kernel takes
 MFMA_HEAD_DIMS = (32, 64, 128, 256)   # head sizes of the bfloat16 matrix-core attention
 GENERIC_SPLIT_KEYS = 256  # keys per split of the any-shape attention kernel in steps of one token per sequence
+FLOAT_DECODE_SPLIT_KEYS = 128   # the same where its float form without LDS tiles runs (attention_float_decode.h; 256: 40 us for 33)
 SKINNY_MAX_ROWS = 16     # rows the few-row kernel serves (one 16-row MFMA tile)
 ROWS64_MAX_ROWS = 64     # rows the 17..64-row kernel serves; above that the library
 FLOAT_SPLIT_MAX_ROWS = 65535 * 32   # rows one launch of the float product of more than 16 rows takes
@@ -1193,13 +1194,15 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             raise KernelError(f"paged_attention: seq_of_token names sequences outside the {S} of the page table")
     if not (attention_takes_head_dim(head_dim)):
         raise KernelError(f"paged_attention: head size {head_dim} must be a multiple of 16, at most 256")
-    # Steps of one token per sequence split the keys into runs of GENERIC_SPLIT_KEYS at absolute positions
+    # Steps of one token per sequence split the keys into runs of 256 or 128 at absolute positions
     # (longer runs only where the longest context the engine ever runs would need more splits than a launch
     # takes), whatever the batch: one work-group per sequence and key/value head would walk a long context alone.
     split_len, nsplit, ws = 0, 1, None
     if plan is not None and plan.decode_only and max_query_len == 1 and split_keys != 0:
-        split_len, nsplit = _fit_key_splits(int(split_keys) if split_keys else GENERIC_SPLIT_KEYS, plan.max_context,
-                                            plan.fit_context)
+        float_form = (q.dtype == torch.float32 and head_dim in (64, 128) and page >= 4 and page & (page - 1) == 0
+                      and not softcap and bias is None)
+        split_len, nsplit = _fit_key_splits(int(split_keys) if split_keys else FLOAT_DECODE_SPLIT_KEYS if float_form
+                                            else GENERIC_SPLIT_KEYS, plan.max_context, plan.fit_context)
         _check(split_len % 64 == 0, "paged_attention: a split of the any-shape kernel is a multiple of 64 keys")
         # Whether the runs go through the merge kernel is a matter of the longest context the engine
         # runs, not of this step's: a step of short contexts and its twin in a graph captured for long

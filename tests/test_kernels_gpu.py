@@ -1199,3 +1199,15 @@ def test_few_rows_in_half_tiles(M, N, Kd):
     got2 = K().linear(nxt, w2, None, out_dtype=torch.float32, shuffled=K().shuffle_weight(w2))
     h = (x * gamma).to(torch.bfloat16).double() / torch.sqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-6)
     torch.testing.assert_close(got2.double(), h @ w2.double().T, atol=2e-4, rtol=2e-4)
+
+
+@pytest.mark.parametrize("nq,nkv,d,bs", [(3, 3, 128, 4), (6, 2, 64, 16), (28, 4, 128, 16), (18, 2, 64, 8), (17, 1, 128, 512)])
+@pytest.mark.parametrize("split", [None, 0, 64])
+@pytest.mark.parametrize("kw", [{}, dict(sink=True), dict(window=70), dict(window=44, keep_first=5), dict(chunk=96)])
+def test_float_attention_of_one_token_steps(nq, nkv, d, bs, split, kw):
+    """The float kernel of steps of one token per sequence: one, four and eight heads to a work-group and a second group of one,
+    contexts that end inside four keys, inside a wave's 32, at the end of a work-group's 128 and of a run, each mask,
+    with runs and without.  Against 64 bits: 4,096 float roundings would be 2.4e-4; sums of random sign stay under 2e-5."""
+    lens = [1, 2, 5, 31, 32, 33, 65, 127, 128, 129, 256, 257, 1030]
+    got, want = _attention_case(torch.float32, nq, nkv, d, bs, lens, None, seed=nq + d, path="generic", split_keys=split, **kw)
+    torch.testing.assert_close(got, want, **tol(torch.float32, 2e-5))
