@@ -184,6 +184,11 @@ extern "C" int tl_argmax_static(const float* logits, int ld, int R, int V, int32
 //   sp_kept   w_t is known to the bit: per chunk, the mass strictly above it and the number of ties
 //   sp_walk   the draw: target = u * kept mass; the chunk whose share of the kept mass holds the
 //             target finds the first token, in index order, whose running kept mass exceeds it
+// What bounds the chain is latency: a work-group has 16 logits per thread, so what it does before and after them counts.
+// Everything a row's chunks leave behind is read by the lanes of a wave side by side and put together by shuffles (every
+// wave for itself, no barrier), a histogram's search has three barriers, and the logits are on their way meanwhile.  48
+// rows of 152,064 (us): sp_sum 17.2 -> 12.6, sp_level 21.0 -> 14.2, sp_kept 17.9 -> 13.9, sp_walk 36.4 -> 12.2, from one loop
+// over the chunks per thread, searches by barriers (35 in a row) and, in sp_walk, a chunk's weights staged in 39 KB of LDS.
 // The rule for w_t: with P = top_p * Z, a weight is kept iff the mass of strictly larger weights is
 // < P; in a histogram, w_t lies in the lowest non-empty bucket whose mass above is < P.  Of the
 // tokens equal to w_t the first ceil((P - above) / w_t) in index order are kept, at least one.
@@ -212,6 +217,27 @@ __device__ __forceinline__ u64 sp_wave_sum(u64 v) {
     return v;
 }
 
+// inclusive sums over the lanes below (or above) and the lane itself
+__device__ __forceinline__ u64 sp_wave_scan(u64 v) {
+    const int lane = threadIdx.x & (TL_WAVE - 1);
+#pragma unroll
+    for (int off = 1; off < TL_WAVE; off <<= 1) {
+        const u64 o = __shfl_up(v, off, TL_WAVE);
+        v += lane >= off ? o : 0ull;
+    }
+    return v;
+}
+
+__device__ __forceinline__ u64 sp_wave_scan_down(u64 v) {
+    const int lane = threadIdx.x & (TL_WAVE - 1);
+#pragma unroll
+    for (int off = 1; off < TL_WAVE; off <<= 1) {
+        const u64 o = __shfl_down(v, off, TL_WAVE);
+        v += lane + off < TL_WAVE ? o : 0ull;
+    }
+    return v;
+}
+
 // sum over the block, returned to every thread; sh: room for 4 values; ends with a barrier
 __device__ __forceinline__ u64 sp_block_sum(u64 v, u64* sh) {
     v = sp_wave_sum(v);
@@ -228,17 +254,33 @@ struct SpRow {
 };
 
 // what every kernel needs of its row: greedy rows (temperature <= 0) are not touched by these kernels
-__device__ __forceinline__ SpRow sp_row(const float* temperature, const float* top_p, const float* pmax, int r, int C) {
+__device__ __forceinline__ SpRow sp_row(const float* temperature, const float* top_p, int r) {
     SpRow row;
     const float t = temperature[r];
     row.active = t > 0.f;
     row.nucleus = top_p[r] < 1.0f;
     row.inv_t = row.active ? 1.0f / t : 0.f;
-    float mx = -INFINITY;
-    if (pmax)
-        for (int c = 0; c < C; ++c) mx = fmaxf(mx, pmax[(size_t)r * C + c]);
-    row.mx = mx;
+    row.mx = -INFINITY;
     return row;
+}
+
+// the row's maximum: the largest of its chunks' (every lane of the wave takes part)
+__device__ __forceinline__ float sp_row_max(const float* pmax, int r, int C) {
+    float mx = -INFINITY;
+    for (int c = threadIdx.x & (TL_WAVE - 1); c < C; c += TL_WAVE) mx = fmaxf(mx, pmax[(size_t)r * C + c]);
+    return tl_wave_max(mx);
+}
+
+// this thread's logits of chunk c; -inf, which has no weight, past the end of the row
+__device__ __forceinline__ void sp_load(float* xv, const float* __restrict__ x, int c, int V) {
+#pragma unroll
+    for (int j = 0; j < SP_ROWS; ++j) {
+        const int i = c * SP_CHUNK + j * SP_THREADS + threadIdx.x;
+        xv[j] = x[i < V ? i : V - 1];
+    }
+#pragma unroll
+    for (int j = 0; j < SP_ROWS; ++j)
+        if (c * SP_CHUNK + j * SP_THREADS + (int)threadIdx.x >= V) xv[j] = -INFINITY;
 }
 
 __global__ __launch_bounds__(SP_THREADS) void sp_max_kernel(const float* __restrict__ logits, int ld, int V, int C,
@@ -261,28 +303,27 @@ __global__ __launch_bounds__(SP_THREADS) void sp_max_kernel(const float* __restr
 // P = top_p * Z of a row, Z the sum of its chunk masses
 __device__ __forceinline__ u64 sp_mass_wanted(const u64* psum, int C, float top_p) {
     u64 Z = 0;
-    for (int c = 0; c < C; ++c) Z += psum[c];
+    for (int c = threadIdx.x & (TL_WAVE - 1); c < C; c += TL_WAVE) Z += psum[c];
+    Z = sp_wave_sum(Z);
     return (u64)((double)Z * (double)top_p);
 }
 
 // In a histogram of SP_BUCKETS masses (buckets ordered by weight): the lowest non-empty bucket whose
 // mass above (A0 + the buckets over it) is < P, and that mass; the highest non-empty bucket if none
-// is (P == 0).  Every thread gets the answer.  sh: SP_THREADS values, shb: SP_THREADS ints.
+// is (P == 0).  Every thread gets the answer.  sh: 5 values, shb: 8 ints, nobody else's.
 __device__ void sp_find(const u64* __restrict__ hist, u64 P, u64 A0, u64* sh, int* shb, int& b_out, u64& A_out) {
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, wave = t / TL_WAVE, lane = t & (TL_WAVE - 1);
     u64 m[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) m[k] = hist[4 * t + k];
     const u64 s = m[0] + m[1] + m[2] + m[3];
-    sh[t] = s;
+    const u64 upward = sp_wave_scan_down(s);                    // of this thread's four and those of the lanes above
+    if (lane == 0) sh[wave] = upward;
     __syncthreads();
-    for (int off = 1; off < SP_THREADS; off <<= 1) {            // inclusive suffix sums over the threads
-        const u64 v = (t + off < SP_THREADS) ? sh[t + off] : 0ull;
-        __syncthreads();
-        sh[t] += v;
-        __syncthreads();
-    }
-    u64 above = A0 + sh[t] - s;                                 // mass of the buckets above this thread's four
+    u64 above = A0 + upward - s;                                // mass of the buckets above this thread's four
+#pragma unroll
+    for (int w = 1; w < SP_THREADS / TL_WAVE; ++w)
+        if (w > wave) above += sh[w];
     int best = 0x7fffffff, top = -1;
     u64 best_a = 0, top_a = 0;
 #pragma unroll
@@ -299,33 +340,24 @@ __device__ void sp_find(const u64* __restrict__ hist, u64 P, u64 A0, u64* sh, in
         }
         above += m[k];
     }
-    __syncthreads();
-    shb[t] = best;
-    __syncthreads();
-    for (int off = SP_THREADS / 2; off > 0; off >>= 1) {
-        if (t < off) shb[t] = min(shb[t], shb[t + off]);
-        __syncthreads();
+    int low = best, high = top;
+#pragma unroll
+    for (int off = TL_WAVE / 2; off > 0; off >>= 1) {
+        low = min(low, __shfl_xor(low, off, TL_WAVE));
+        high = max(high, __shfl_xor(high, off, TL_WAVE));
     }
-    int b = shb[0];
-    __syncthreads();
-    if (b == 0x7fffffff) {                                      // no bucket qualifies: the highest non-empty one
-        shb[t] = top;
-        __syncthreads();
-        for (int off = SP_THREADS / 2; off > 0; off >>= 1) {
-            if (t < off) shb[t] = max(shb[t], shb[t + off]);
-            __syncthreads();
-        }
-        b = shb[0];
-        __syncthreads();
-        if (b < 0) b = 0;                                       // an empty histogram
-        if (top == b) sh[0] = top_a;
-    } else if (best == b) {
-        sh[0] = best_a;
+    if (lane == 0) {
+        shb[wave] = low;
+        shb[4 + wave] = high;
     }
     __syncthreads();
-    b_out = b;
-    A_out = (b >= 0 && hist[b] != 0) ? sh[0] : A0;
+    low = min(min(shb[0], shb[1]), min(shb[2], shb[3]));
+    high = max(max(shb[4], shb[5]), max(shb[6], shb[7]));
+    const bool some = low != 0x7fffffff;                        // else the highest non-empty bucket, if there is one
+    if (some ? best == low : high >= 0 && top == high) sh[4] = some ? best_a : top_a;
     __syncthreads();
+    b_out = some ? low : high >= 0 ? high : 0;
+    A_out = some || high >= 0 ? sh[4] : A0;                     // (an empty histogram: bucket 0, nothing above)
 }
 
 // level 1: chunk masses and the first histogram
@@ -336,19 +368,19 @@ __global__ __launch_bounds__(SP_THREADS) void sp_sum_kernel(const float* __restr
     __shared__ u64 hist[SP_BUCKETS];
     __shared__ u64 red[4];
     const int c = blockIdx.x, r = blockIdx.y;
-    const SpRow row = sp_row(temperature, top_p, pmax, r, C);
+    SpRow row = sp_row(temperature, top_p, r);
     if (!row.active) return;
+    float xv[SP_ROWS];
+    sp_load(xv, logits + (size_t)r * ld, c, V);
+    row.mx = sp_row_max(pmax, r, C);
     u64* wr = ws + (size_t)r * (SP_ROW_WORDS + 3 * C);
     if (row.nucleus)
         for (int b = threadIdx.x; b < SP_BUCKETS; b += SP_THREADS) hist[b] = 0;
     __syncthreads();
-    const float* x = logits + (size_t)r * ld;
     u64 sum = 0;
 #pragma unroll
     for (int j = 0; j < SP_ROWS; ++j) {
-        const int i = c * SP_CHUNK + j * SP_THREADS + threadIdx.x;
-        if (i >= V) continue;
-        const float w = sp_weight(x[i], row.mx, row.inv_t);
+        const float w = sp_weight(xv[j], row.mx, row.inv_t);
         const u64 f = sp_fix(w);
         sum += f;
         if (row.nucleus && f) atomicAdd(&hist[__float_as_uint(w) >> 20], f);
@@ -367,11 +399,15 @@ __global__ __launch_bounds__(SP_THREADS) void sp_level_kernel(const float* __res
                                                               const float* __restrict__ pmax, u64* __restrict__ ws,
                                                               int level) {
     __shared__ u64 hist[SP_BUCKETS];
-    __shared__ u64 sh[SP_THREADS];
-    __shared__ int shb[SP_THREADS];
+    __shared__ u64 sh[5];
+    __shared__ int shb[8];
     const int c = blockIdx.x, r = blockIdx.y;
-    const SpRow row = sp_row(temperature, top_p, pmax, r, C);
+    SpRow row = sp_row(temperature, top_p, r);
     if (!row.active || !row.nucleus) return;
+    float xv[SP_ROWS];
+    sp_load(xv, logits + (size_t)r * ld, c, V);
+    row.mx = sp_row_max(pmax, r, C);
+    for (int b = threadIdx.x; b < SP_BUCKETS; b += SP_THREADS) hist[b] = 0;      // (sp_find's barriers come before its first use)
     u64* wr = ws + (size_t)r * (SP_ROW_WORDS + 3 * C);
     // one selection per kernel; chunk 0 leaves its result in the row's state for the kernels after it
     u64* st = wr + SP_STATE;
@@ -399,14 +435,9 @@ __global__ __launch_bounds__(SP_THREADS) void sp_level_kernel(const float* __res
         prefix = ((unsigned)st[1] << 10) | (unsigned)b2;
         shift = 0;
     }
-    for (int b = threadIdx.x; b < SP_BUCKETS; b += SP_THREADS) hist[b] = 0;
-    __syncthreads();
-    const float* x = logits + (size_t)r * ld;
 #pragma unroll
     for (int j = 0; j < SP_ROWS; ++j) {
-        const int i = c * SP_CHUNK + j * SP_THREADS + threadIdx.x;
-        if (i >= V) continue;
-        const float w = sp_weight(x[i], row.mx, row.inv_t);
+        const float w = sp_weight(xv[j], row.mx, row.inv_t);
         const u64 f = sp_fix(w);
         const unsigned bits = __float_as_uint(w);
         if (!f || (bits >> (shift + 10)) != prefix) continue;
@@ -423,12 +454,15 @@ __global__ __launch_bounds__(SP_THREADS) void sp_kept_kernel(const float* __rest
                                                              const float* __restrict__ temperature,
                                                              const float* __restrict__ top_p,
                                                              const float* __restrict__ pmax, u64* __restrict__ ws) {
-    __shared__ u64 sh[SP_THREADS];
-    __shared__ int shb[SP_THREADS];
+    __shared__ u64 sh[5];
+    __shared__ int shb[8];
     __shared__ u64 red[4];
     const int c = blockIdx.x, r = blockIdx.y;
-    const SpRow row = sp_row(temperature, top_p, pmax, r, C);
+    SpRow row = sp_row(temperature, top_p, r);
     if (!row.active || !row.nucleus) return;
+    float xv[SP_ROWS];
+    sp_load(xv, logits + (size_t)r * ld, c, V);
+    row.mx = sp_row_max(pmax, r, C);
     u64* wr = ws + (size_t)r * (SP_ROW_WORDS + 3 * C);
     u64* st = wr + SP_STATE;
     int b3;
@@ -439,13 +473,10 @@ __global__ __launch_bounds__(SP_THREADS) void sp_kept_kernel(const float* __rest
         st[5] = (u64)wt_bits;
         st[6] = above;
     }
-    const float* x = logits + (size_t)r * ld;
     u64 mass = 0, ties = 0;
 #pragma unroll
     for (int j = 0; j < SP_ROWS; ++j) {
-        const int i = c * SP_CHUNK + j * SP_THREADS + threadIdx.x;
-        if (i >= V) continue;
-        const float w = sp_weight(x[i], row.mx, row.inv_t);
+        const float w = sp_weight(xv[j], row.mx, row.inv_t);
         const u64 f = sp_fix(w);
         const unsigned bits = __float_as_uint(w);
         if (!f) continue;
@@ -460,22 +491,18 @@ __global__ __launch_bounds__(SP_THREADS) void sp_kept_kernel(const float* __rest
     }
 }
 
-// exclusive prefix sums of one value per thread, in thread order; sh: SP_THREADS values; the total
-// comes back in `total`
-__device__ u64 sp_block_scan(u64 v, u64* sh, u64& total) {
-    const int t = threadIdx.x;
-    sh[t] = v;
+// exclusive prefix sums of one value per thread, in thread order; sh: 4 values
+__device__ u64 sp_block_scan(u64 v, u64* sh) {
+    const int wave = threadIdx.x / TL_WAVE, lane = threadIdx.x & (TL_WAVE - 1);
+    const u64 incl = sp_wave_scan(v);
+    if (lane == TL_WAVE - 1) sh[wave] = incl;
     __syncthreads();
-    for (int off = 1; off < SP_THREADS; off <<= 1) {
-        const u64 add = (t >= off) ? sh[t - off] : 0ull;
-        __syncthreads();
-        sh[t] += add;
-        __syncthreads();
-    }
-    const u64 incl = sh[t];
-    total = sh[SP_THREADS - 1];
+    u64 before = incl - v;
+#pragma unroll
+    for (int w = 0; w < SP_THREADS / TL_WAVE - 1; ++w)
+        if (w < wave) before += sh[w];
     __syncthreads();
-    return incl - v;
+    return before;
 }
 
 __global__ __launch_bounds__(SP_THREADS) void sp_walk_kernel(const float* __restrict__ logits, int ld, int V, int C,
@@ -484,16 +511,15 @@ __global__ __launch_bounds__(SP_THREADS) void sp_walk_kernel(const float* __rest
                                                              const float* __restrict__ uniform,
                                                              const float* __restrict__ pmax, u64* __restrict__ ws,
                                                              int32_t* __restrict__ out) {
-    __shared__ u64 kept[SP_CHUNK];                              // kept weight of each element, in index order
-    __shared__ unsigned char is_tie[SP_CHUNK];
-    __shared__ u64 sh[SP_THREADS];
+    __shared__ u64 sh[4];
     const int c = blockIdx.x, r = blockIdx.y;
-    const SpRow row = sp_row(temperature, top_p, pmax, r, C);
+    SpRow row = sp_row(temperature, top_p, r);
     if (!row.active) return;
     const u64* wr = ws + (size_t)r * (SP_ROW_WORDS + 3 * C);
     const u64* psum = wr + SP_ROW_WORDS;
     // the kept mass of every chunk, in order: before this chunk, of this chunk, in total
     unsigned wt_bits = 0;
+    const int lane = threadIdx.x & (TL_WAVE - 1);
     u64 wt_fix = 0, keep_ties = 0, before = 0, mine = 0, total = 0, ties_before = 0;
     if (row.nucleus) {
         const u64 P = wr[SP_STATE], above = wr[SP_STATE + 6];
@@ -502,25 +528,30 @@ __global__ __launch_bounds__(SP_THREADS) void sp_walk_kernel(const float* __rest
         keep_ties = (P > above && wt_fix) ? (P - above + wt_fix - 1) / wt_fix : 1;
         if (keep_ties < 1) keep_ties = 1;
         u64 ties_seen = 0;
-        for (int k = 0; k < C; ++k) {
-            const u64 t = psum[2 * C + k];
-            const u64 room = keep_ties > ties_seen ? keep_ties - ties_seen : 0;
-            const u64 kc = psum[C + k] + (t < room ? t : room) * wt_fix;
-            if (k < c) before += kc;
-            if (k == c) {
-                mine = kc;
-                ties_before = ties_seen;
+        for (int k0 = 0; k0 < C; k0 += TL_WAVE) {               // 64 chunks at a time, one per lane
+            const int k = k0 + lane;
+            const u64 t = k < C ? psum[2 * C + k] : 0ull, m = k < C ? psum[C + k] : 0ull;
+            const u64 ties = sp_wave_scan(t), seen = ties_seen + ties - t;
+            const u64 room = keep_ties > seen ? keep_ties - seen : 0;
+            const u64 kc = m + (t < room ? t : room) * wt_fix;
+            before += sp_wave_sum(k < c ? kc : 0ull);
+            total += sp_wave_sum(kc);
+            if (c >= k0 && c < k0 + TL_WAVE) {
+                mine = __shfl(kc, c - k0, TL_WAVE);
+                ties_before = __shfl(seen, c - k0, TL_WAVE);
             }
-            total += kc;
-            ties_seen += t;
+            ties_seen += __shfl(ties, TL_WAVE - 1, TL_WAVE);
         }
     } else {
-        for (int k = 0; k < C; ++k) {
+        for (int k = lane; k < C; k += TL_WAVE) {
             const u64 kc = psum[k];
             if (k < c) before += kc;
             if (k == c) mine = kc;
             total += kc;
         }
+        before = sp_wave_sum(before);
+        mine = sp_wave_sum(mine);
+        total = sp_wave_sum(total);
     }
     if (total == 0) {                                           // a row without any weight
         if (c == 0 && threadIdx.x == 0) out[r] = 0;
@@ -530,55 +561,47 @@ __global__ __launch_bounds__(SP_THREADS) void sp_walk_kernel(const float* __rest
     if (target >= total) target = total - 1;
     if (target < before || target >= before + mine) return;    // another chunk holds the target
     target -= before;
-    // this chunk, element by element in index order
+    // this chunk in index order, a run of SP_ROWS consecutive elements per thread; one work-group of the row gets here
+    row.mx = sp_row_max(pmax, r, C);
     const float* x = logits + (size_t)r * ld;
-#pragma unroll 4
-    for (int j = 0; j < SP_ROWS; ++j) {
-        const int e = j * SP_THREADS + threadIdx.x, i = c * SP_CHUNK + e;
-        u64 f = 0;
-        bool tie = false;
-        if (i < V) {
-            const float w = sp_weight(x[i], row.mx, row.inv_t);
-            const u64 v = sp_fix(w);
-            const unsigned bits = __float_as_uint(w);
-            if (!row.nucleus || bits > wt_bits) f = v;
-            else if (v && bits == wt_bits) tie = true;
-        }
-        kept[e] = f;
-        is_tie[e] = tie ? 1 : 0;
+    const int e0 = c * SP_CHUNK + threadIdx.x * SP_ROWS;
+    float xv[SP_ROWS];
+#pragma unroll
+    for (int k = 0; k < SP_ROWS; ++k) xv[k] = x[e0 + k < V ? e0 + k : V - 1];
+    u64 kept[SP_ROWS], mine_ties = 0, sum = 0;
+    unsigned tie = 0;                                           // bit k: element k's weight is w_t
+#pragma unroll
+    for (int k = 0; k < SP_ROWS; ++k) {
+        const float w = sp_weight(e0 + k < V ? xv[k] : -INFINITY, row.mx, row.inv_t);
+        const u64 v = sp_fix(w);
+        const unsigned bits = __float_as_uint(w);
+        const bool is_tie = row.nucleus && v && bits == wt_bits;
+        kept[k] = !row.nucleus || bits > wt_bits ? v : 0ull;
+        tie |= is_tie ? 1u << k : 0u;
+        mine_ties += is_tie ? 1 : 0;
     }
-    __syncthreads();
-    const int e0 = threadIdx.x * SP_ROWS;                       // this thread's run of consecutive elements
-    u64 all;
     if (row.nucleus) {
         // of the weights equal to w_t the first keep_ties in index order are kept
-        u64 mine_ties = 0;
-#pragma unroll 1
-        for (int k = 0; k < SP_ROWS; ++k) mine_ties += is_tie[e0 + k];
-        u64 rank = ties_before + sp_block_scan(mine_ties, sh, all);
-#pragma unroll 1
+        u64 rank = ties_before + sp_block_scan(mine_ties, sh);
+#pragma unroll
         for (int k = 0; k < SP_ROWS; ++k) {
-            if (is_tie[e0 + k]) {
-                if (rank < keep_ties) kept[e0 + k] = wt_fix;
+            if (tie >> k & 1) {
+                if (rank < keep_ties) kept[k] = wt_fix;
                 ++rank;
             }
         }
-        __syncthreads();
     }
-    u64 sum = 0;
-#pragma unroll 1
-    for (int k = 0; k < SP_ROWS; ++k) sum += kept[e0 + k];
-    u64 run = sp_block_scan(sum, sh, all);
+#pragma unroll
+    for (int k = 0; k < SP_ROWS; ++k) sum += kept[k];
+    u64 run = sp_block_scan(sum, sh);
     if (target < run || target >= run + sum) return;           // another thread's run holds the target
-#pragma unroll 1
+    int found = -1;
+#pragma unroll
     for (int k = 0; k < SP_ROWS; ++k) {
-        const u64 v = kept[e0 + k];
-        if (v && target < run + v) {
-            out[r] = c * SP_CHUNK + e0 + k;
-            return;
-        }
-        run += v;
+        if (found < 0 && kept[k] && target < run + kept[k]) found = e0 + k;
+        run += kept[k];
     }
+    out[r] = found;
 }
 
 // chunks a row of V logits is cut into, and the workspace tl_sample needs: pmax holds R * chunks

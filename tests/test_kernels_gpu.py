@@ -1211,3 +1211,14 @@ def test_float_attention_of_one_token_steps(nq, nkv, d, bs, split, kw):
     lens = [1, 2, 5, 31, 32, 33, 65, 127, 128, 129, 256, 257, 1030]
     got, want = _attention_case(torch.float32, nq, nkv, d, bs, lens, None, seed=nq + d, path="generic", split_keys=split, **kw)
     torch.testing.assert_close(got, want, **tol(torch.float32, 2e-5))
+
+
+@pytest.mark.parametrize("V", [4096, 4097, 262144, 262145, 270001])
+def test_sample_ties_over_one_to_more_than_64_chunks(V):
+    """Equal logits: the kept set is the first tokens whose count stays under 0.3 V, across one chunk, at the edges of a
+    chunk and of the 64 chunks a wave adds up at a time, and beyond; u picks evenly among them.  Whole numbers, exact."""
+    us = torch.tensor([0.0, 0.25, 0.5, 0.75, 0.999999], device=DEV)
+    n, kept = us.numel(), int(0.3 * V) + 1
+    flat, one = torch.zeros(n, V, device=DEV), torch.ones(n, device=DEV)
+    assert K().sample(flat, one, one * 0.3, us).tolist() == [int(float(x) * kept) for x in us.tolist()]
+    assert K().sample(flat, one, one, us).tolist() == [int(float(x) * V) for x in us.tolist()]
