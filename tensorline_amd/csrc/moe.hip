@@ -15,9 +15,9 @@
 //
 // A pair's row is computed alone (a row of a tile does not see the other rows) and summed over k in
 // one fixed order, and a token's choices are added in one fixed order, so neither the batch nor the
-// place a pair gets inside its expert's tiles changes a bit of a result.  The products run on the
-// float matrix instruction (v_mfma_f32_16x16x4_f32), bfloat16 operands widened on the way into
-// LDS, as the any-shape product does.
+// place a pair gets inside its expert's tiles changes a bit of a result.  Float products run on the
+// float matrix instruction (v_mfma_f32_16x16x4_f32), bfloat16 ones on v_mfma_f32_16x16x32_bf16, in tiles of 16, 64 or
+// up to 256 pair rows; bfloat16 shapes those do not take are widened on the way into LDS, as the any-shape product does.
 #include "common.h"
 
 #include <math.h>
