@@ -43,7 +43,9 @@ class Sampler:
         u = [uniform_for(s, i) for s, i in zip(seeds, indices)]
         # from pinned memory: a copy from ordinary memory waits for the step in flight, and the GPU then stands idle until
         # the draw's kernels are issued (48 rows of 152,064 after 8 layers of the 7B shape: 1,677 us a step, 1,790 before)
-        params = torch.tensor([temperatures, top_ps, u], dtype=torch.float32, pin_memory=logits.is_cuda).to(self.device, non_blocking=True)
+        # (in a capture the copy stays the waiting one, which the capture refuses: a graph must not read these numbers' memory later)
+        pin = logits.is_cuda and not torch.cuda.is_current_stream_capturing()
+        params = torch.tensor([temperatures, top_ps, u], dtype=torch.float32, pin_memory=pin).to(self.device, non_blocking=pin)
         return kernels.sample(logits, params[0], params[1], params[2],
                               any_top_p=any(p < 1.0 for p in top_ps),
                               any_greedy=any(t <= 0 for t in temperatures))
