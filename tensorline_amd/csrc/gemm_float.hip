@@ -27,8 +27,10 @@
 // over the GPU by segments, whose sums a second kernel adds in the same order.
 //
 // Values that are not finite, and those so large that they round to infinity as bfloat16, make the split
-// itself infinity minus infinity: an element that comes out as NaN is computed again with plain float
-// multiply-adds, so infinities and NaN give what they give there.
+// itself infinity minus infinity, and a product of two rounded parts may pass the largest float where the product
+// itself does not: an element whose segment does not come out finite is computed again on the float instruction,
+// so infinities, NaN and sums near the largest float give what they give there.  (A wave takes its blocks of 32 x 32 in
+// turn; one lane after another along k, as it was first written, took seconds for a matrix of infinities.)
 #include "common.h"
 
 typedef __bf16 fs_bf16x8 __attribute__((ext_vector_type(8)));
@@ -103,15 +105,6 @@ __device__ __forceinline__ void fs_load_to_lds(const void* g, void* lds_base) {
 // at most N of this wave's loads are still on their way, and its LDS reads are done
 #define FS_LANDED(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory")
 
-// one element (or one segment of it) with float multiply-adds, from the values themselves
-__device__ float fs_plain(const float* __restrict__ A, const float* __restrict__ Ws, int lda, int steps, int m, int n, int k0, int k1) {
-    float sum = 0.f;
-    for (int k = k0; k < k1 && sum == sum; ++k)
-        sum = fmaf(A[(size_t)m * lda + k],
-                   Ws[(((size_t)(n >> 4) * steps + (k >> 4)) * 64 + ((k >> 2) & 3) * 16 + (n & 15)) * 4 + (k & 3)], sum);
-    return sum;
-}
-
 // MB blocks of 32 rows, FS_WAVES waves side by side with NB blocks of 32 columns each.  PARTS: blockIdx.y is a segment
 // of K and C the workspace [segments][M][N]; else the whole K, C holding the sum of the segments so far (a lane reads
 // and writes its own elements only).
@@ -170,10 +163,13 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
     float* out = PARTS ? C + (size_t)blockIdx.y * M * N : C;
     const size_t ld = PARTS ? N : ldc;
     const int row0 = b0 * 32 + 4 * (lane >> 5);
-    bool nan_seen = false;
-    auto store = [&](bool first_seg, bool last_seg) {
+    auto store = [&](int s0, int s1) {       // the sums over steps [s0, s1), a segment
+        const bool first_seg = s0 == 0, last_seg = s1 == steps;
         int row = row0, col = n0 + (lane & 31);
         asm volatile("" : "+v"(row), "+v"(col));       // addresses and bounds are made here, not kept through the loop over k
+        uint32_t again[(MB * NB + 1) / 2];             // elements to compute again: sixteen bits per block
+#pragma unroll
+        for (int u = 0; u < (MB * NB + 1) / 2; ++u) again[u] = 0;
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
             const int n = col + j * 32;
@@ -185,15 +181,53 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
                 for (int q = 0; q < 4; ++q) {          // four rows at a time: a few addresses and sums in registers
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        float v = acc[i][j][4 * q + r];
+                        const float v = acc[i][j][4 * q + r];
                         if (n < N && row + i * 32 + 8 * q + r < M) {
-                            if (!PARTS && !first_seg) v = o[r * ld] + v;
-                            nan_seen |= v != v;
-                            o[r * ld] = v + b;
+                            const bool fine = fabsf(v) < INFINITY;         // else the sum so far stays where it is
+                            again[(i * NB + j) / 2] |= fine ? 0u : 1u << (((i * NB + j) & 1) * 16 + 4 * q + r);
+                            const float so_far = !PARTS && !first_seg ? o[r * ld] : 0.f;
+                            o[r * ld] = fine ? (!PARTS && !first_seg ? so_far + v : v) + b : so_far;
                         }
                     }
                     o += 8 * ld;
                     asm volatile("" ::: "memory");
+                }
+        }
+        bool any = false;
+#pragma unroll
+        for (int u = 0; u < (MB * NB + 1) / 2; ++u) any |= again[u] != 0;
+        if (!__any(any)) return;
+        // the marked elements from the values themselves
+        for (int block = 0; block < MB * NB; ++block) {
+            uint32_t marks = 0;
+#pragma unroll
+            for (int u = 0; u < (MB * NB + 1) / 2; ++u) marks = block >> 1 == u ? again[u] : marks;
+            marks = marks >> (block & 1) * 16 & 0xffffu;
+            if (!__any(marks != 0)) continue;
+            int here = lane;
+            asm volatile("" : "+v"(here));             // nothing of this is made ahead of the loop over k
+            const int i = block / NB, n = n0 + block % NB * 32 + (here & 31), half = here >> 5;
+            const float* a = A + (size_t)min((b0 + i) * 32 + (here & 31), M - 1) * lda + half;        // rows and columns that
+            const float* w = Ws + ((size_t)min(n >> 4, (N + 15) / 16 - 1) * steps * 64 + (n & 15)) * 4 + half;   // are not there: others
+            fs_f32x16 sum;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[r] = 0.f;
+            for (int s = s0; s < s1; ++s) {
+                float av[8], wv[8];                    // k = 16 s + 2 t + half
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    av[t] = s * FS_STEP + 2 * t + half < K ? a[s * FS_STEP + 2 * t] : 0.f;
+                    wv[t] = w[(size_t)s * 256 + (t >> 1) * 64 + (t & 1) * 2];
+                }
+#pragma unroll
+                for (int t = 0; t < 8; ++t) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(av[t], wv[t], sum, 0, 0, 0);
+            }
+            const float b = !PARTS && bias && last_seg && n < N ? bias[n] : 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (marks >> r & 1) {
+                    float* o = out + (size_t)((b0 + i) * 32 + 4 * half + 8 * (r >> 2) + (r & 3)) * ld + n;
+                    *o = (!PARTS && !first_seg ? *o + sum[r] : sum[r]) + b;
                 }
         }
     };
@@ -234,22 +268,13 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
 #undef FS_MUL
         }
         if (!PARTS && (s + 1) % FS_SEG_STEPS == 0 && s + 1 < last) {
-            store(s < FS_SEG_STEPS, false);
+            store(s + 1 - FS_SEG_STEPS, s + 1);
             clear();
         }
         buf = buf == STAGES - 1 ? 0 : buf + 1;
     }
     FS_LANDED(0);                        // nothing may land in LDS that is no longer this work-group's
-    store(last <= FS_SEG_STEPS, true);
-    if (!nan_seen) return;
-    for (int j = 0; j < NB; ++j) {
-        const int n = n0 + j * 32 + (lane & 31);
-        for (int i = 0; n < N && i < MB * 16; ++i) {
-            const int m = row0 + 8 * (i >> 2) + (i & 3);
-            if (m >= M || out[(size_t)m * ld + n] == out[(size_t)m * ld + n]) continue;
-            out[(size_t)m * ld + n] = fs_plain(A, Ws, lda, steps, m, n, first * FS_STEP, min(last * FS_STEP, K)) + (!PARTS && bias ? bias[n] : 0.f);
-        }
-    }
+    store(PARTS ? first : (last - 1) / FS_SEG_STEPS * FS_SEG_STEPS, last);
 }
 
 // The segments' sums in ascending order, as the product adds them where it has the whole K.  VEC: four columns a
@@ -304,6 +329,13 @@ static int fs_choose(int M, int N, int K, bool* parts) {
         }
     }
     return best;
+}
+
+// The tile that tl_gemm_float_split takes (an index of fs_tiles), plus 4 where K is dealt out by segments.
+extern "C" int tl_gemm_float_split_tile(int M, int N, int K) {
+    bool parts = false;
+    const int tile = fs_choose(M, N, K, &parts);
+    return tile + (parts ? 4 : 0);
 }
 
 // Floats of workspace that tl_gemm_float_split needs for the segments' sums (0: none).

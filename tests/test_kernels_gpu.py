@@ -178,6 +178,50 @@ def test_linear_float_by_three_bfloat16_not_finite():
     torch.testing.assert_close(got[fine], want[fine], atol=1e-3, rtol=1e-5)
 
 
+# (tile, K dealt out by segments, M, N, K): every tile of the float product of more than 16 rows, with the whole of K (two
+# segments) and in segments, none of them filled by its rows, its columns or its last step
+FLOAT_TILES = [(0, False, 701, 66003, 2100), (0, True, 2049, 2051, 4101), (1, False, 1501, 4101, 2100), (1, True, 97, 16401, 4100),
+               (2, False, 301, 16399, 2101), (2, True, 97, 8201, 4100), (3, False, 201, 8201, 2100), (3, True, 97, 2051, 2101)]
+
+
+def _float_tile(tile, parts, M, N, Kd):
+    assert K().library().tl_gemm_float_split_tile(M, N, Kd) == tile + (4 if parts else 0)
+
+
+@pytest.mark.parametrize("tile,parts,M,N,Kd", FLOAT_TILES)
+def test_linear_float_not_finite_in_every_tile(tile, parts, M, N, Kd):
+    """Infinities, NaN, values that round to infinity as bfloat16 and a product just below the largest float whose rounded
+    parts' product is above it, in either segment: what plain float arithmetic gives; every other element as without them."""
+    _float_tile(tile, parts, M, N, Kd)
+    torch.manual_seed(tile)
+    a, w, bias = torch.randn(M, Kd, device=DEV), torch.randn(N, Kd, device=DEV), torch.randn(N, device=DEV)
+    w[:, 2] *= 1e-3                                          # 3.4e38 times that stays a float
+    a[:, 2080] *= 1e-3
+    plain_rows = K().linear(a, w, bias, shuffled=K().shuffle_weight_float(w))
+    a[3, 5], a[40, 2070], a[M - 1, 2] = float("inf"), float("nan"), 3.4e38
+    w[6, 2080], w[N - 1, 7] = 3.4e38, float("-inf")
+    big = 2.0 ** 64 - 2.0 ** 40                              # big^2 rounds to 2^128 (1 - 2^-23), finite; big rounds to 2^64 as bfloat16
+    bias[9] = 0.0
+    for row, at in ((11, 8), (M - 2, 2090)):                 # that product alone in row 9 of the matrix, in the first and the second segment
+        a[row, at], w[9, at] = big if row == 11 else -big, big
+    w[9, :8] = w[9, 9:2090] = w[9, 2091:] = 0.0
+    a[11, 2090] = a[M - 2, 8] = 0.0
+    got = K().linear(a, w, bias, shuffled=K().shuffle_weight_float(w))
+    rows, cols = [3, 11, 40, M - 2, M - 1], [6, 9, N - 1]
+    top = (2.0 ** 128 * (1.0 - 2.0 ** -23))
+    assert got[11, 9].item() == top and got[M - 2, 9].item() == -top
+    want = (a.double() @ w.double().T + bias.double()).float()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    size = (a.double().abs() @ w.double().abs().T + bias.double().abs())[fine]
+    assert bool(((got[fine].double() - want[fine].double()).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())
+    other_rows = torch.ones(M, dtype=torch.bool, device=DEV)
+    other_cols = torch.ones(N, dtype=torch.bool, device=DEV)
+    other_rows[rows], other_cols[cols] = False, False
+    assert torch.equal(got[other_rows][:, other_cols], plain_rows[other_rows][:, other_cols])
+
+
 @pytest.mark.parametrize("M", [1, 2, 8, 16, 17, 33, 48, 64])
 @pytest.mark.parametrize("N,Kd", [(1000, 1184), (4608, 3584), (136, 8), (50, 264), (3584, 18944), (5120, 1184), (2090, 72),
                                   (5120, 9728)])
