@@ -1,8 +1,10 @@
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float for more than 16 rows, on the bfloat16 matrix
 // instruction (v_mfma_f32_32x32x16_bf16): the 32-bit path's product of prompts and large batches.
 //
-// A float is exactly the sum of three bfloat16 numbers (8 + 8 + 8 significant bits; each is the rest of the
-// one before, rounded to nearest, so the rests have either sign).  Of the nine partial products of two such
+// A float times 2^24 is exactly the sum of three bfloat16 numbers (8 + 8 + 8 significant bits; each is the rest of the
+// one before, rounded to nearest, so the rests have either sign).  The factor keeps the last part of the smallest
+// float a normal bfloat16: without it floats below 2^-110 lost their rests (4.6e-4 of a value of 1e-37).  It comes out
+// again as 2^-48 of a segment's sum, and costs 1 to 3% (2,048 rows of 37,888 x 3,584: 2.79 ms against 2.75).  Of the nine partial products of two such
 // sums the six that reach 2^-18 of the largest are taken, small ones first, each exact in the instruction's
 // float sums; the three left out are below 2^-26 of the product they belong to, a quarter of the rounding
 // that a float product itself has.  Six bfloat16 products take 6 / 16 of the matrix cores' time of one on
@@ -26,10 +28,10 @@
 // order, the segments' sums added in ascending order.  Few tiles (few rows of a narrow matrix) are spread
 // over the GPU by segments, whose sums a second kernel adds in the same order.
 //
-// Values that are not finite, and those so large that they round to infinity as bfloat16, make the split
-// itself infinity minus infinity, and a product of two rounded parts may pass the largest float where the product
-// itself does not: an element whose segment does not come out finite is computed again on the float instruction,
-// so infinities, NaN and sums near the largest float give what they give there.  (A wave takes its blocks of 32 x 32 in
+// Values that are not finite, and those of 2^104 and more, which the factor takes past the largest bfloat16, make the
+// split itself infinity minus infinity, and sums of 2^80 and more pass the largest float where the sums themselves do
+// not: an element whose segment does not come out finite is computed again on the float instruction, so infinities,
+// NaN and sums of any size give what they give there.  (A wave takes its blocks of 32 x 32 in
 // turn; one lane after another along k, as it was first written, took seconds for a matrix of infinities.)
 #include "common.h"
 
@@ -43,6 +45,8 @@ typedef float fs_f32x16 __attribute__((ext_vector_type(16)));
 #define FS_SEG_STEPS (FS_SEG / FS_STEP)
 #define FS_WAVES 4
 #define FS_CUS 256
+#define FS_UP 0x1p24f                    // factor of both operands
+#define FS_DOWN 0x1p-48f
 
 // two floats as two bfloat16, rounded to nearest even, and what is left of each
 __device__ __forceinline__ uint32_t fs_take(float& a, float& b) {
@@ -52,8 +56,9 @@ __device__ __forceinline__ uint32_t fs_take(float& a, float& b) {
     b -= __uint_as_float(p & 0xffff0000u);
     return p;
 }
-// eight floats as three times eight bfloat16
+// eight floats times FS_UP as three times eight bfloat16
 __device__ __forceinline__ void fs_split8(float4 x, float4 y, uint4& hi, uint4& mid, uint4& lo) {
+    x.x *= FS_UP, x.y *= FS_UP, x.z *= FS_UP, x.w *= FS_UP, y.x *= FS_UP, y.y *= FS_UP, y.z *= FS_UP, y.w *= FS_UP;
     hi = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
     mid = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
     lo = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
@@ -181,7 +186,7 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
                 for (int q = 0; q < 4; ++q) {          // four rows at a time: a few addresses and sums in registers
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const float v = acc[i][j][4 * q + r];
+                        const float v = acc[i][j][4 * q + r] * FS_DOWN;
                         if (n < N && row + i * 32 + 8 * q + r < M) {
                             const bool fine = fabsf(v) < INFINITY;         // else the sum so far stays where it is
                             again[(i * NB + j) / 2] |= fine ? 0u : 1u << (((i * NB + j) & 1) * 16 + 4 * q + r);

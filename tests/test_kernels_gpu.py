@@ -222,6 +222,23 @@ def test_linear_float_not_finite_in_every_tile(tile, parts, M, N, Kd):
     assert torch.equal(got[other_rows][:, other_cols], plain_rows[other_rows][:, other_cols])
 
 
+@pytest.mark.parametrize("tile,parts,M,N,Kd", FLOAT_TILES)
+def test_linear_float_of_small_and_large_values_in_every_tile(tile, parts, M, N, Kd):
+    """Rows and matrix rows of every magnitude a float has, 2^-140 (subnormal, rounded by that) to 2^120, whose products come out
+    around one: the bound of K float multiply-adds, the same for all of them."""
+    _float_tile(tile, parts, M, N, Kd)
+    torch.manual_seed(tile + 10)
+    a, w = torch.randn(M, Kd, device=DEV), torch.randn(N, Kd, device=DEV)
+    up = torch.tensor([0, -100, -112, -120, -126, -140, 60, 100, 120], device=DEV)
+    at, wt = up[torch.arange(M, device=DEV) % 9], up[torch.arange(N, device=DEV) % 9]
+    a, w = torch.ldexp(a, at[:, None].float()), torch.ldexp(w, wt[:, None].float())
+    got = K().linear(a, w, shuffled=K().shuffle_weight_float(w))
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    fits = (at[:, None] + wt[None, :] >= -90) & (at[:, None] + wt[None, :] <= 100)      # products and sums that are normal floats
+    ok = (got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size
+    assert bool(ok[fits].all())
+
+
 @pytest.mark.parametrize("M", [1, 2, 8, 16, 17, 33, 48, 64])
 @pytest.mark.parametrize("N,Kd", [(1000, 1184), (4608, 3584), (136, 8), (50, 264), (3584, 18944), (5120, 1184), (2090, 72),
                                   (5120, 9728)])
