@@ -2,14 +2,24 @@
 // instruction (v_mfma_f32_32x32x16_bf16): the 32-bit path's product of prompts and large batches.
 //
 // A float times 2^24 is exactly the sum of three bfloat16 numbers (8 + 8 + 8 significant bits; each is the rest of the
-// one before, rounded to nearest, so the rests have either sign).  The factor keeps the last part of the smallest
+// one before, rounded to nearest, so the rests have either sign; splitting floats into shorter ones so that products
+// are exact is Dekker's, Numerische Mathematik 18, 1971).  The factor keeps the last part of the smallest
 // float a normal bfloat16: without it floats below 2^-110 lost their rests (4.6e-4 of a value of 1e-37).  It comes out
-// again as 2^-48 of a segment's sum, and costs 1 to 3% (2,048 rows of 37,888 x 3,584: 2.79 ms against 2.75).  Of the nine partial products of two such
-// sums the six that reach 2^-18 of the largest are taken, small ones first, each exact in the instruction's
-// float sums; the three left out are below 2^-26 of the product they belong to, a quarter of the rounding
-// that a float product itself has.  Six bfloat16 products take 6 / 16 of the matrix cores' time of one on
-// the float instruction (2.5 PFLOP/s against 157 TFLOP/s), and the sums have fewer roundings: at 2,048 rows and
-// K = 18,944 the result is 5.4e-7 off the exact one where the float instruction's was 2.5e-6 (3,584: 4.8e-7 and 1.1e-6).
+// again as 2^-48 of a segment's sum, and costs 1 to 3% (2,048 rows of 37,888 x 3,584: 2.79 ms against 2.75).
+//
+// Of the nine partial products of two such sums the six with a first part in them and the product of the two second parts
+// are taken, small ones first, each exact; the three left out come to at most 2^-24 of the product they
+// belong to (a second part is up to 2^-8 of its float, a third up to 2^-17) and 1e-8 of it on average, and a sum of K
+// products takes roundings of that size at every step whatever the instruction.  What the result is off the exact one,
+// 2-norm, 256 rows, six products here / eight of the nine / v_mfma_f32_16x16x4_f32:
+//                                    K = 16                  896                     3,584                   18,944
+//   normal numbers                   3.4e-8 3.3e-8 7.3e-8    4.6e-7 4.6e-7 5.4e-7    6.7e-7 6.7e-7 1.1e-6    7.6e-7 7.6e-7 2.5e-6
+//   positive (uniform in [0, 1))     3.3e-8 3.3e-8 6.2e-8    2.9e-7 2.9e-7 4.2e-7    2.8e-7 2.8e-7 8.4e-7    1.4e-7 1.4e-7 2.1e-6
+//   one column 3,000 times the rest  5.9e-8 5.9e-8 8.4e-8    3.9e-7 3.9e-7 6.2e-7    4.6e-7 4.6e-7 1.3e-6    6.9e-7 6.9e-7 2.9e-6
+// The two more products cost 20% (gate/up of 2,048 rows 2.74 -> 3.34 ms) and change nothing from K = 16 on; below, where a
+// result is a handful of products, the matrix instruction's own last addition is the error (K = 1: 3.4e-8 with six or eight,
+// 2.6e-8 on the float instruction), and such products go to the float instruction.  Six bfloat16 products take 6 / 16 of the
+// matrix cores' time of one on the float instruction (2.5 PFLOP/s against 157 TFLOP/s).
 //
 // What is split where: the rows of A once, by a pass of its own, into the order in which the product reads
 // them (fs_split_kernel: 4 bytes read and 6 written per value); W, which may be most of the GPU's memory,

@@ -579,6 +579,7 @@ FLOAT_DECODE_SPLIT_KEYS = 128   # the same where its float form without LDS tile
 SKINNY_MAX_ROWS = 16     # rows the few-row kernel serves (one 16-row MFMA tile)
 ROWS64_MAX_ROWS = 64     # rows the 17..64-row kernel serves; above that the library
 FLOAT_SPLIT_MAX_ROWS = 65535 * 32   # rows one launch of the float product of more than 16 rows takes
+FLOAT_SPLIT_MIN_K = 16   # below: the float instruction, whose error is smaller there (gemm_float.hip)
 
 
 def _skinny_ok(a: torch.Tensor, shuffled: torch.Tensor | None, M: int, K: int, lda: int) -> bool:
@@ -606,7 +607,7 @@ def _few_rows_go_to_rows64(N: int, K: int) -> bool:
 
 def _float_split(a, shuffled, bias, out, M, N, K, lda, ldc):
     """More than 16 float rows: every float as the sum of three bfloat16 numbers on the bfloat16 matrix instruction,
-    the weight from its matrix-core ordered copy.  Every matrix that has the copy goes here, whatever its rows beyond 16, so
+    the weight from its matrix-core ordered copy.  Every matrix with the copy and a K of 16 or more goes here, whatever its rows beyond 16, so
     that a row's bits do not depend on how many others come along: at 33 rows and more it is the faster kernel at every K
     (300 rows, N = 1,152: K = 64 8.2 us against 16, 896 29 against 89), at 17 to 32 rows it is level from K = 896 on and its
     second launch costs 2 us below (K = 128: 7.8 against 5.7)."""
@@ -627,8 +628,8 @@ def _rows64(a, shuffled, bias, out, M, N, K, lda, ldc, swiglu: bool, norm=None):
 
 
 def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None) -> torch.Tensor:
-    """bfloat16 with few rows: the streaming MFMA kernel.  float32, and shapes that kernel does not
-    take: the plain tiled kernel.  (bfloat16 with many rows went to the library before this, where
+    """bfloat16 with few rows: the streaming MFMA kernels.  float32 with the matrix-core ordered copy: the few-row kernel,
+    or (more than 16 rows, a K of 16 or more) the float product on the bfloat16 instruction.  The rest: the plain tiled kernel.  (bfloat16 with many rows went to the library before this, where
     the reference uses one too: tensorline/paged.py:179-188.)"""
     if _skinny_ok(a, shuffled, M, K, lda) and not _few_rows_go_to_rows64(N, K):
         _call("tl_gemm_skinny", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), _code(out, "linear output"),
@@ -641,7 +642,7 @@ def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None) -> 
         _call("tl_gemm_fewrows_shuffled", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), M, N, K, lda, ldc, _stream())
         return out
     if (shuffled is not None and shuffled.dtype == torch.float32 and a.dtype == torch.float32 and out.dtype == torch.float32
-            and SKINNY_MAX_ROWS < M <= FLOAT_SPLIT_MAX_ROWS):
+            and SKINNY_MAX_ROWS < M <= FLOAT_SPLIT_MAX_ROWS and K >= FLOAT_SPLIT_MIN_K):
         return _float_split(a, shuffled, bias, out, M, N, K, lda, ldc)
     _call("tl_gemm_generic", _ptr(a), _code(a, "linear input"), _ptr(weight), _code(weight, "linear weight"),
           _ptr(bias), _ptr(out), _code(out, "linear output"), M, N, K, lda, ldc, _stream())

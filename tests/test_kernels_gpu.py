@@ -178,6 +178,24 @@ def test_linear_float_by_three_bfloat16_not_finite():
     torch.testing.assert_close(got[fine], want[fine], atol=1e-3, rtol=1e-5)
 
 
+@pytest.mark.parametrize("Kd", [1, 2, 3, 7, 15, 16, 33, 128, 896, 3584])
+@pytest.mark.parametrize("values", ["normal", "positive", "one column large"])
+def test_linear_float_is_no_further_from_64_bits_than_the_float_instruction(Kd, values):
+    """More than 16 float rows, at every K: not further from the exact product, in the 2-norm, than the product on the float
+    matrix instruction (the call without the ordered copy), and a K of one is rounded once."""
+    torch.manual_seed(Kd)
+    M, N = 200, 512
+    a = torch.rand(M, Kd, device=DEV) if values == "positive" else torch.randn(M, Kd, device=DEV)
+    w = torch.rand(N, Kd, device=DEV) if values == "positive" else torch.randn(N, Kd, device=DEV)
+    if values == "one column large":
+        a[:, Kd // 3] *= 3000.0
+    want = a.double() @ w.double().T
+    got, other = K().linear(a, w, shuffled=K().shuffle_weight_float(w)), K().linear(a, w)
+    assert (got.double() - want).norm() <= (other.double() - want).norm()
+    if Kd == 1:
+        assert bool(((got.double() - want).abs() <= 2.0 ** -24 * want.abs()).all())
+
+
 # (tile, K dealt out by segments, M, N, K): every tile of the float product of more than 16 rows, with the whole of K (two
 # segments) and in segments, none of them filled by its rows, its columns or its last step
 FLOAT_TILES = [(0, False, 701, 66003, 2100), (0, True, 2049, 2051, 4101), (1, False, 1501, 4101, 2100), (1, True, 97, 16401, 4100),
