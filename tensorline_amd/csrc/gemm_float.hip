@@ -57,6 +57,7 @@ typedef float fs_f32x16 __attribute__((ext_vector_type(16)));
 #define FS_CUS 256
 #define FS_UP 0x1p24f                    // factor of both operands
 #define FS_DOWN 0x1p-48f
+#define FS_RAW_K 256                     // at most 32 aligned rows of a K below this are split where they are used
 
 // two floats as two bfloat16, rounded to nearest even, and what is left of each
 __device__ __forceinline__ uint32_t fs_take(float& a, float& b) {
@@ -125,12 +126,18 @@ __device__ __forceinline__ void fs_load_to_lds(const void* g, void* lds_base) {
 // and writes its own elements only).
 // Work-groups of one XCD (every eighth in the order of their ids) take the row tiles of one column tile in turn, so
 // that W is fetched into an L2 once and the rows are what its work-groups share at a time.
-template <int MB, int NB, int STAGES, bool PARTS>
+// RAW (one block of rows, the rows 16-byte aligned, K a multiple of four and below FS_RAW_K): the rows come as they are, 2 KB
+// a step, and every wave splits them itself, so that a product of 17 to 32 rows is one launch.  17 rows of 1,152 x K, parts
+// beforehand and RAW, us: K = 64 6.6 and 5.2, 128 8.2 and 7.1, 256 11.2 and 11.1, 512 17.3 and 19.1 (a longer chain a step).
+// A row of a step, 64 bytes, has its unit u of 16 at u ^ (row / 4) % 4: sixteen rows' reads hit all banks.  Units past K
+// are the step's before, against zeros of the weight copy.
+template <int MB, int NB, int STAGES, bool PARTS, bool RAW>
 __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_kernel(
     const uint4* __restrict__ As, const float* __restrict__ A, const float* __restrict__ Ws, const float* __restrict__ bias,
     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int steps) {
     extern __shared__ uint4 fs_lds[];
-    constexpr int CHUNKS = MB * 3, LA = (CHUNKS + FS_WAVES - 1) / FS_WAVES, LW = NB * 2, STAGE = (CHUNKS + FS_WAVES * LW) * 64;
+    static_assert(!RAW || (MB == 1 && !PARTS), "unsplit rows come in one block, with the whole of a short K");
+    constexpr int CHUNKS = RAW ? 2 : MB * 3, LA = (CHUNKS + FS_WAVES - 1) / FS_WAVES, LW = NB * 2, STAGE = (CHUNKS + FS_WAVES * LW) * 64;
     constexpr int BN = FS_WAVES * NB * 32;
     const int blocks = (M + 31) / 32, mtiles = (blocks + MB - 1) / MB, ntiles = (N + BN - 1) / BN;
     const int local = blockIdx.x >> 3;
@@ -143,10 +150,15 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
 
     const uint4* ap[LA];
     const uint4* wp[LW];
+    const int unit = (lane & 3) ^ (lane >> 4);                          // RAW: the unit that this lane fetches
+    const bool past = RAW && (steps - 1) * FS_STEP + 4 * unit >= K;     // in the last step it is not there
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
         const int c = min(wave + i * FS_WAVES, CHUNKS - 1);            // a wave without a piece of its own repeats the last one
-        ap[i] = As + ((size_t)min(b0 + c / 3, blocks - 1) * steps + first) * 192 + (c % 3) * 64 + lane;
+        if (RAW)
+            ap[i] = reinterpret_cast<const uint4*>(A + (size_t)min(16 * c + (lane >> 2), M - 1) * lda + 4 * unit);   // K >= 16
+        else
+            ap[i] = As + ((size_t)min(b0 + c / 3, blocks - 1) * steps + first) * 192 + (c % 3) * 64 + lane;
     }
 #pragma unroll
     for (int j = 0; j < LW; ++j)
@@ -160,7 +172,7 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
         for (int j = 0; j < LW; ++j) fs_load_to_lds(wp[j], stage + (CHUNKS + wave * LW + j) * 64);
         if (++ahead < last) {
 #pragma unroll
-            for (int i = 0; i < LA; ++i) ap[i] += 192;
+            for (int i = 0; i < LA; ++i) ap[i] += RAW ? (past && ahead == steps - 1 ? 0 : 4) : 192;
 #pragma unroll
             for (int j = 0; j < LW; ++j) wp[j] += 64;
         }
@@ -269,7 +281,10 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
 #pragma unroll
             for (int b = 0; b < IB; ++b)
 #pragma unroll
-                for (int p = 0; p < 3; ++p) a[b][p] = stage[((i + b) * 3 + p) * 64 + lane];
+                for (int p = 0; p < 3 && !RAW; ++p) a[b][p] = stage[((i + b) * 3 + p) * 64 + lane];
+            if (RAW)
+                fs_split8(__builtin_bit_cast(float4, stage[(lane & 31) * 4 + ((lane >> 5) * 2 ^ (lane >> 2 & 3))]),
+                          __builtin_bit_cast(float4, stage[(lane & 31) * 4 + ((lane >> 5) * 2 + 1 ^ (lane >> 2 & 3))]), a[0][0], a[0][1], a[0][2]);
 #define FS_MUL(PA, PW)                                                                                                       \
     _Pragma("unroll") for (int b = 0; b < IB; ++b) _Pragma("unroll") for (int j = 0; j < NB; ++j) acc[i + b][j] =              \
         __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fs_bf16x8, a[b][PA]), __builtin_bit_cast(fs_bf16x8, w[j][PW]), \
@@ -353,6 +368,11 @@ extern "C" int tl_gemm_float_split_tile(int M, int N, int K) {
     return tile + (parts ? 4 : 0);
 }
 
+// Whether rows that start 16-byte aligned are split where they are used and need no workspace for their parts.
+extern "C" int tl_gemm_float_split_takes_rows(int M, int K, int lda) {
+    return M <= 32 && K >= FS_STEP && K < FS_RAW_K && K % 4 == 0 && lda % 4 == 0 ? 1 : 0;
+}
+
 // Floats of workspace that tl_gemm_float_split needs for the segments' sums (0: none).
 extern "C" long long tl_gemm_float_split_workspace(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -362,7 +382,8 @@ extern "C" long long tl_gemm_float_split_workspace(int M, int N, int K) {
 }
 
 // A float [M, K] with row stride lda; Ws float [ceil(N/16), ceil(K/16), 64, 4] (the matrix-core ordered copy of W, zero
-// where it pads); split: workspace of ceil(M/32) * ceil(K/16) * 3 KB; ws: tl_gemm_float_split_workspace floats.
+// where it pads); split: workspace of ceil(M/32) * ceil(K/16) * 3 KB, or null where
+// tl_gemm_float_split_takes_rows says that the rows are split where they are used; ws: tl_gemm_float_split_workspace floats.
 extern "C" int tl_gemm_float_split(const float* A, const float* Ws, const float* bias, float* C, void* split, float* ws, int M,
                                    int N, int K, int lda, int ldc, hipStream_t stream) {
     TL_CHECK_ARG(M >= 0 && N > 0 && K > 0, "tl_gemm_float_split: bad sizes M=%d N=%d K=%d", M, N, K);
@@ -378,22 +399,27 @@ extern "C" int tl_gemm_float_split(const float* A, const float* Ws, const float*
     TL_CHECK_ARG(grid < (1ll << 31), "tl_gemm_float_split: M=%d N=%d are too many tiles for one launch", M, N);
     TL_CHECK_ARG(!parts || ws, "tl_gemm_float_split: no workspace for the segments' sums");
     const int vec = ((uintptr_t)A % 16 == 0 && lda % 4 == 0) ? 1 : 0;
-    hipLaunchKernelGGL(fs_split_kernel, dim3(tl_ceil_div(steps, 4), blocks), dim3(256), 0, stream, A, (uint4*)split, M, K, lda, steps, vec);
-#define FS_GO(MB, NB, ST, P)                                                                                                     \
-    hipLaunchKernelGGL((fs_gemm_kernel<MB, NB, ST, P>), dim3((unsigned)grid, P ? nseg : 1), dim3(FS_WAVES * 64),                 \
-                       ST * (MB * 3 + FS_WAVES * NB * 2) * 1024, stream, (const uint4*)split, A, Ws, bias, P ? ws : C, M, N, K, \
+    TL_CHECK_ARG(split || (tl_gemm_float_split_takes_rows(M, K, lda) && vec && tile == 3 && !parts),
+                 "tl_gemm_float_split: M=%d K=%d lda=%d need a workspace for the rows' parts", M, K, lda);
+    if (split)
+        hipLaunchKernelGGL(fs_split_kernel, dim3(tl_ceil_div(steps, 4), blocks), dim3(256), 0, stream, A, (uint4*)split, M, K, lda, steps, vec);
+#define FS_GO(MB, NB, ST, P, RAW)                                                                                                \
+    hipLaunchKernelGGL((fs_gemm_kernel<MB, NB, ST, P, RAW>), dim3((unsigned)grid, P ? nseg : 1), dim3(FS_WAVES * 64),            \
+                       ST * ((RAW ? 2 : MB * 3) + FS_WAVES * NB * 2) * 1024, stream, (const uint4*)split, A, Ws, bias, P ? ws : C, M, N, K, \
                        lda, ldc, steps)
-#define FS_GO_P(MB, NB, ST)             \
-    if (parts) FS_GO(MB, NB, ST, true); \
-    else FS_GO(MB, NB, ST, false)
+#define FS_GO_P(MB, NB, ST, RAW)             \
+    if (parts) FS_GO(MB, NB, ST, true, RAW); \
+    else FS_GO(MB, NB, ST, false, RAW)
     if (tile == 0) {
-        FS_GO_P(4, 2, 2);
+        FS_GO_P(4, 2, 2, false);
     } else if (tile == 1) {
-        FS_GO_P(4, 1, 3);
+        FS_GO_P(4, 1, 3, false);
     } else if (tile == 2) {
-        FS_GO_P(2, 1, 3);
+        FS_GO_P(2, 1, 3, false);
+    } else if (split) {
+        FS_GO_P(1, 1, 3, false);
     } else {
-        FS_GO_P(1, 1, 3);
+        FS_GO(1, 1, 3, false, true);
     }
 #undef FS_GO_P
 #undef FS_GO

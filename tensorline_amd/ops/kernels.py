@@ -607,11 +607,14 @@ def _few_rows_go_to_rows64(N: int, K: int) -> bool:
 
 def _float_split(a, shuffled, bias, out, M, N, K, lda, ldc):
     """More than 16 float rows: every float as the sum of three bfloat16 numbers on the bfloat16 matrix instruction,
-    the weight from its matrix-core ordered copy.  Every matrix with the copy and a K of 16 or more goes here, whatever its rows beyond 16, so
-    that a row's bits do not depend on how many others come along: at 33 rows and more it is the faster kernel at every K
-    (300 rows, N = 1,152: K = 64 8.2 us against 16, 896 29 against 89), at 17 to 32 rows it is level from K = 896 on and its
-    second launch costs 2 us below (K = 128: 7.8 against 5.7)."""
-    split = torch.empty(-(-M // 32) * -(-K // 16) * 1536, dtype=torch.int16, device=a.device)
+    the weight from its matrix-core ordered copy.  Every matrix with the copy and a K of 16 or more goes here, whatever its
+    rows beyond 16, so that a row's bits do not depend on how many others come along: at 33 rows and more it is the faster
+    kernel at every K (300 rows, N = 1,152: K = 64 8.2 us against 16, 896 29 against 92).  17 to 32 rows pay for that one order
+    of summation below K = 896, us here and on the float instruction, 17 rows of 1,152: K = 16 3.7 and 2.9, 64 5.2 and 4.1,
+    128 7.1 and 5.8, 256 11.2 and 9.1, 512 17.3 and 15.9, 896 26.3 and 25.7, 3,584 52 and 95."""
+    split = None
+    if a.data_ptr() % 16 or not library().tl_gemm_float_split_takes_rows(M, K, lda):
+        split = torch.empty(-(-M // 32) * -(-K // 16) * 1536, dtype=torch.int16, device=a.device)
     floats = library().tl_gemm_float_split_workspace(M, N, K)
     ws = torch.empty(floats, dtype=torch.float32, device=a.device) if floats else None
     _call("tl_gemm_float_split", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), _ptr(split), _ptr(ws), M, N, K, lda, ldc, _stream())

@@ -196,6 +196,25 @@ def test_linear_float_is_no_further_from_64_bits_than_the_float_instruction(Kd, 
         assert bool(((got.double() - want).abs() <= 2.0 ** -24 * want.abs()).all())
 
 
+@pytest.mark.parametrize("N,Kd", [(33, 16), (70, 20), (130, 36), (1000, 60), (257, 128), (40, 252), (1152, 256)])
+@pytest.mark.parametrize("M", [17, 30, 32])
+def test_linear_float_of_at_most_32_rows_splits_them_where_they_are_used(M, N, Kd):
+    """One launch for 17 to 32 aligned rows: the bits that the same rows get from parts made beforehand (rows that are not
+    aligned, or among more rows), the last step's missing units of k and rows' ends untouched by what lies behind them."""
+    torch.manual_seed(M + Kd)
+    behind = torch.full((40, Kd + 8), float("nan"), device=DEV)
+    behind[:, :Kd] = torch.randn(40, Kd, device=DEV)
+    a, odd = behind[:M, :Kd], torch.full((M, Kd + 5), float("nan"), device=DEV)
+    odd[:, 1:Kd + 1] = a
+    w, b = torch.randn(N, Kd, device=DEV), torch.randn(N, device=DEV)
+    ws = K().shuffle_weight_float(w)
+    got = K().linear(a, w, b, shuffled=ws)
+    want, size = a.double() @ w.double().T + b.double(), a.double().abs() @ w.double().abs().T + b.double().abs()
+    assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())
+    assert torch.equal(K().linear(odd[:, 1:Kd + 1], w, b, shuffled=ws), got)
+    assert torch.equal(K().linear(behind[:, :Kd], w, b, shuffled=ws)[:M], got)
+
+
 # (tile, K dealt out by segments, M, N, K): every tile of the float product of more than 16 rows, with the whole of K (two
 # segments) and in segments, none of them filled by its rows, its columns or its last step
 FLOAT_TILES = [(0, False, 701, 66003, 2100), (0, True, 2049, 2051, 4101), (1, False, 1501, 4101, 2100), (1, True, 97, 16401, 4100),
