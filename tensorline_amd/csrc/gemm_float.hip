@@ -55,6 +55,7 @@ typedef float fs_f32x16 __attribute__((ext_vector_type(16)));
 #define FS_SEG_STEPS (FS_SEG / FS_STEP)
 #define FS_WAVES 4
 #define FS_CUS 256
+#define FS_MOST_SUMS (512LL << 18)       // floats at most of the segments' sums (512 MB): beyond, K stays whole
 #define FS_UP 0x1p24f                    // factor of both operands
 #define FS_DOWN 0x1p-48f
 #define FS_RAW_K 256                     // at most 32 aligned rows of a K below this are split where they are used
@@ -350,7 +351,7 @@ static int fs_choose(int M, int N, int K, bool* parts) {
         const FsTile& z = fs_tiles[t];
         if (z.mb > 1 && z.mb / 2 >= blocks) continue;                  // half of it holds all the rows
         const double tiles = (double)tl_ceil_div(blocks, z.mb) * tl_ceil_div(N, FS_WAVES * 32 * z.nb);
-        for (int cut = 0; cut < (nseg > 1 && nseg <= 65535 ? 2 : 1); ++cut) {
+        for (int cut = 0; cut < (nseg > 1 && nseg <= 65535 && (long long)M * N <= FS_MOST_SUMS / nseg ? 2 : 1); ++cut) {
             const double each = tiles * (cut ? nseg : 1) / FS_CUS, whole = (double)(long long)(each + 0.999999);
             const double on_a_cu = whole < 4 ? whole : each + 0.5, turns = (double)(long long)((whole + z.fit - 1) / z.fit);
             const double step = turns * z.alone > on_a_cu * z.shared ? turns * z.alone : on_a_cu * z.shared;

@@ -579,6 +579,7 @@ FLOAT_DECODE_SPLIT_KEYS = 128   # the same where its float form without LDS tile
 SKINNY_MAX_ROWS = 16     # rows the few-row kernel serves (one 16-row MFMA tile)
 ROWS64_MAX_ROWS = 64     # rows the 17..64-row kernel serves; above that the library
 FLOAT_SPLIT_MAX_ROWS = 65535 * 32   # rows one launch of the float product of more than 16 rows takes
+FLOAT_SPLIT_BYTES = 512 << 20   # at most this much for the parts of a launch's rows: more rows go in several launches
 FLOAT_SPLIT_MIN_K = 16   # below: the float instruction, whose error is smaller there (gemm_float.hip)
 
 
@@ -612,12 +613,16 @@ def _float_split(a, shuffled, bias, out, M, N, K, lda, ldc):
     kernel at every K (300 rows, N = 1,152: K = 64 8.2 us against 16, 896 29 against 92).  17 to 32 rows pay for that one order
     of summation below K = 896, us here and on the float instruction, 17 rows of 1,152: K = 16 3.7 and 2.9, 64 5.2 and 4.1,
     128 7.1 and 5.8, 256 11.2 and 9.1, 512 17.3 and 15.9, 896 26.3 and 25.7, 3,584 52 and 95."""
-    split = None
-    if a.data_ptr() % 16 or not library().tl_gemm_float_split_takes_rows(M, K, lda):
-        split = torch.empty(-(-M // 32) * -(-K // 16) * 1536, dtype=torch.int16, device=a.device)
-    floats = library().tl_gemm_float_split_workspace(M, N, K)
-    ws = torch.empty(floats, dtype=torch.float32, device=a.device) if floats else None
-    _call("tl_gemm_float_split", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), _ptr(split), _ptr(ws), M, N, K, lda, ldc, _stream())
+    most = max(128, FLOAT_SPLIT_BYTES // (-(-K // 16) * 96) // 128 * 128)
+    split = ws = None
+    if M > 32 or a.data_ptr() % 16 or not library().tl_gemm_float_split_takes_rows(M, K, lda):
+        split = torch.empty(-(-min(M, most) // 32) * -(-K // 16) * 1536, dtype=torch.int16, device=a.device)
+    for r in range(0, M, most):
+        m = min(M - r, most)
+        floats = library().tl_gemm_float_split_workspace(m, N, K)
+        if floats and (ws is None or ws.numel() < floats):
+            ws = torch.empty(floats, dtype=torch.float32, device=a.device)
+        _call("tl_gemm_float_split", _ptr(a[r:]), _ptr(shuffled), _ptr(bias), _ptr(out[r:]), _ptr(split), _ptr(ws), m, N, K, lda, ldc, _stream())
     return out
 
 

@@ -215,6 +215,22 @@ def test_linear_float_of_at_most_32_rows_splits_them_where_they_are_used(M, N, K
     assert torch.equal(K().linear(behind[:, :Kd], w, b, shuffled=ws)[:M], got)
 
 
+@pytest.mark.parametrize("M,N,Kd", [(40003, 40, 8200), (9000, 5000, 8200)])
+def test_linear_float_of_very_many_rows_has_a_bounded_workspace(M, N, Kd):
+    """At most 512 MB for the rows' parts (here in several launches) and 512 MB for the segments' sums; rows on either side of
+    a launch's edge have the bits that they have alone."""
+    torch.manual_seed(M)
+    a, w = torch.randn(M, Kd, device=DEV), torch.randn(N, Kd, device=DEV)
+    ws, out = K().shuffle_weight_float(w), torch.empty(M, N, device=DEV)
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    K().linear(a, w, out=out, shuffled=ws)
+    assert torch.cuda.max_memory_allocated() - before <= 1 << 30
+    edge = K().FLOAT_SPLIT_BYTES // (-(-Kd // 16) * 96) // 128 * 128
+    for r in (0, min(edge - 10, M - 20), M - 20):
+        assert torch.equal(K().linear(a[r:r + 20], w, shuffled=ws), out[r:r + 20])
+
+
 # (tile, K dealt out by segments, M, N, K): every tile of the float product of more than 16 rows, with the whole of K (two
 # segments) and in segments, none of them filled by its rows, its columns or its last step
 FLOAT_TILES = [(0, False, 701, 66003, 2100), (0, True, 2049, 2051, 4101), (1, False, 1501, 4101, 2100), (1, True, 97, 16401, 4100),
