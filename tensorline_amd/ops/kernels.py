@@ -1060,6 +1060,17 @@ def _attention_launch(plan, S: int, num_heads: int, num_kv_heads: int, head_dim:
                             sum(-(-n * G // (32 * waves)) for n in q_lens) + pads if waves else 0, split_len, nsplit, waves, chains)
 
 
+def _worked_out_launch(plan, *key) -> _AttentionLaunch:
+    """``_attention_launch``, worked out once for the layers of a step that have the same heads and mask.  What it follows from
+    is kept beside it and compared: the facts are the caller's, who may write the next step's into them."""
+    memo = getattr(plan, "worked_out", {})
+    facts = (plan.max_context, plan.max_query_len, plan.num_seqs, plan.fit_context, plan.decode_only)
+    kept = memo.get(key)
+    if kept is None or kept[0] != facts or kept[1] != plan.q_lens or kept[2] != plan.starts:
+        kept = memo[key] = (facts, list(plan.q_lens), list(plan.starts), _attention_launch(plan, *key))
+    return kept[3]
+
+
 def attention_takes_head_dim(head_dim: int) -> bool:
     """The head sizes the attention kernels take: multiples of 16 up to 256 (32, 64 and 128 on the
     bfloat16 MFMA kernels, the others on the any-shape kernel)."""
@@ -1144,13 +1155,8 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         G = num_heads // num_kv_heads
         if split_keys is not None:
             _check(int(split_keys) % 32 == 0, "paged_attention: a split is a multiple of 32 keys")
-        # the choices are the same for every layer of a step that has these heads and this mask
-        key = (S, num_heads, num_kv_heads, head_dim, window, keep_first, chunk, path, split_keys, route_singles,
-               single_seqs is not None)
-        memo, memo_key = getattr(plan, "worked_out", {}), key + (plan.max_context, plan.fit_context, plan.decode_only)
-        launch = memo.get(memo_key)
-        if launch is None:
-            launch = memo[memo_key] = _attention_launch(plan, *key)
+        launch = _worked_out_launch(plan, S, num_heads, num_kv_heads, head_dim, window, keep_first, chunk, path, split_keys,
+                                    route_singles, single_seqs is not None)
         if launch.singles:
             _i32(single_seqs, "single_seqs", launch.singles)
         if launch.own_split:

@@ -66,3 +66,16 @@ def test_few_row_products_of_long_k_and_an_unfull_last_round_go_to_the_kernel_th
 
 def test_head_sizes_the_kernels_take():
     assert [d for d in range(1, 300) if K.attention_takes_head_dim(d)] == list(range(16, 257, 16))
+
+
+def test_launches_worked_out_for_a_step_follow_its_facts():
+    """A step's layers share one choice; facts that a caller writes the next step's numbers into get another."""
+    key = (2, 28, 4, 128, 0, 0, 0, None, None, None, False)
+    facts = StepFacts(max_context=900, max_query_len=300, num_seqs=2, q_lens=[300, 20], starts=[600, 40])
+    first = K._worked_out_launch(facts, *key)
+    assert K._worked_out_launch(facts, *key) is first and first == K._attention_launch(facts, *key)
+    for change in (lambda: facts.q_lens.__setitem__(1, 280), lambda: facts.starts.__setitem__(0, 0),
+                   lambda: setattr(facts, "q_lens", [1, 299]), lambda: setattr(facts, "max_query_len", 299),
+                   lambda: setattr(facts, "max_context", 8000), lambda: setattr(facts, "num_seqs", 3)):
+        change()
+        assert K._worked_out_launch(facts, *key) == K._attention_launch(facts, *key)
