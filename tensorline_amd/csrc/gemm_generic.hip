@@ -428,7 +428,8 @@ __global__ __launch_bounds__(GG_THREADS) void gemm_batched_bf16_kernel(const bf1
 
 // `batch` products of the same shape in one launch: product b reads A + b * a_bs (row stride lda),
 // W + b * w_bs ([N, K] contiguous) and writes C + b * c_bs (row stride ldc); strides in elements.
-// Each is summed as tl_gemm_generic sums it.  (A head's share of a projection that is applied per
+// Each is summed as tl_gemm_generic sums it, or (aligned bfloat16) in steps of 32 k from 0 upwards on the bfloat16
+// instruction.  (A head's share of a projection that is applied per
 // head: the operands are column blocks of wider matrices, a stride of one head apart.)
 extern "C" int tl_gemm_generic_batched(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype, int M,
                                        int N, int K, int lda, int ldc, int batch, long long a_bs, long long w_bs,
@@ -437,8 +438,11 @@ extern "C" int tl_gemm_generic_batched(const void* A, int a_dtype, const void* W
     TL_CHECK_ARG(lda >= K && ldc >= N, "tl_gemm_generic_batched: row strides lda=%d ldc=%d too small for K=%d N=%d", lda, ldc, K, N);
     if (M == 0) return 0;
     int rc;
-    // aligned bfloat16 operands; a long K stays with the tiles in LDS (a wave here has a handful of loads in flight)
-    if (a_dtype == TL_BF16 && w_dtype == TL_BF16 && c_dtype == TL_BF16 && K % 8 == 0 && K <= 1024 && lda % 8 == 0 && a_bs % 8 == 0 &&
+    // Aligned bfloat16 operands, us on the kernels below and on the one without LDS (8 products of N x K): 17 rows of 64 x 64 4.8
+    // and 3.9, 512 x 512 20.7 and 8.0, 1,024 x 1,024 44 and 17; 2,048 rows 19 and 5.8, 109 and 49, 451 and 175.  At most 16 rows
+    // go to the few-row kernel behind K = 512, whose waves share K where one wave walks it here: 8 rows of 128 x 256 7.7 and
+    // 5.4, x 448 7.3 and 7.1, x 512 7.4 and 7.7, x 640 7.6 and 8.8, 64 x 1,024 7.7 and 12.2.
+    if (a_dtype == TL_BF16 && w_dtype == TL_BF16 && c_dtype == TL_BF16 && K % 8 == 0 && K <= (M <= 16 ? 512 : 1024) && lda % 8 == 0 && a_bs % 8 == 0 &&
         w_bs % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && tl_ceil_div(M, 128) <= 65535) {
         hipLaunchKernelGGL(gemm_batched_bf16_kernel, dim3(tl_ceil_div(N, 64), tl_ceil_div(M, 128), batch), dim3(GG_THREADS), 0, stream,
                            (const bf16_t*)A, (const bf16_t*)W, (bf16_t*)C, M, N, K, lda, ldc, a_bs, w_bs, c_bs);
