@@ -115,13 +115,8 @@ __global__ __launch_bounds__(AFD_WAVES * 64, 1) void attn_float_decode_kernel(
 #pragma unroll
             for (int x = 0; x < DL; ++x) o[h][x] *= alpha;
             // lane part b hands on block b's weights
-            float w = sc[0][h];
-            w = part == 1 ? sc[1][h] : w;
-            if constexpr (KB == 4) {
-                w = part == 2 ? sc[2][h] : w;
-                w = part == 3 ? sc[3][h] : w;
-            }
-            if (KB == 4 || part < KB) ps[wave][h][16 * part + sub] = w;
+            static_assert(KB == 2, "two parts hand on two blocks");
+            if (part < KB) ps[wave][h][16 * part + sub] = part == 1 ? sc[1][h] : sc[0][h];
         }
         // written and read by this wave only; LDS operations of a wave complete in order
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -84,7 +84,7 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
     constexpr bool DUAL = MODE != MODE_PLAIN;
     constexpr int NACC = MT * (DUAL ? 2 : 1);
     constexpr int COLS = 16 / SPLIT;                           // columns of a work-group
-    static_assert(SPLIT == 1 || MT == 1, "half tiles come with one tile of rows");
+    static_assert(SPLIT == 1 || (MT == 1 && MODE == MODE_PLAIN), "half tiles come with one tile of rows and one stream of weights");
     constexpr int XS_PER_WAVE = MT * SPLIT * SK_UNITS * SK_ROWPAD;     // in uint4
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
     const int r = lane & 15, g = lane >> 4;
@@ -216,10 +216,8 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
                     if (!live) xf = zero;
                     f32x4& a = acc[h * NACC + mt];
                     a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(wf[cc]), as_frag(xf), a, 0, 0, 0);
-                    if (DUAL) {
-                        f32x4& b = acc[h * NACC + MT + mt];
-                        b = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(uf[cc]), as_frag(xf), b, 0, 0, 0);
-                    }
+                    if (DUAL)
+                        acc[MT + mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(uf[cc]), as_frag(xf), acc[MT + mt], 0, 0, 0);
                 }
             }
         }
@@ -287,10 +285,7 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
         for (int w = 0; w < nwaves; ++w) {
             v += red[((size_t)w * NACC * 4 + mt * 4 + i) * 64 + l];
             if (DUAL) u += red[((size_t)w * NACC * 4 + (MT + mt) * 4 + i) * 64 + l];
-            if (SPLIT == 2) {
-                v += red[((size_t)w * NACC * 4 + mt * 4 + i) * 64 + l + 32];
-                if (DUAL) u += red[((size_t)w * NACC * 4 + (MT + mt) * 4 + i) * 64 + l + 32];
-            }
+            if (SPLIT == 2) v += red[((size_t)w * NACC * 4 + mt * 4 + i) * 64 + l + 32];
         }
         if (owed) {
             const float rs = sh_rstd[m & 15];
