@@ -982,6 +982,17 @@ def _tile32_waves(q_lens, starts, num_heads: int) -> int:
     return 8 if keys >= 4096 and cols * num_heads >= 128 * 256 else 0          # at least 128 such work-groups
 
 
+def _walks_alone_at_256(plan, rows: int, num_heads: int, window: int, keep_first: int, chunk: int) -> bool:
+    """Whether short prompts at a head size of 256 run on independent waves and not on the kernel whose work-groups share key
+    tiles through LDS.  That one takes 9 us to begin with, 128 KB of tiles to a work-group, and about 2 us per tile of 64 keys; a
+    wave on its own begins after 5.5 us and takes 4 us for 64 keys, until there are more waves than the CUs hold.  Measured,
+    tiles / waves, us (32 / 1 heads): 17 tokens 10.5 / 6.7, 40 11.3 / 8.4, 64 11.4 / 9.0, 130 13.4 / 14.3, 400 22 / 34; 8 prompts of
+    17 11.3 / 7.7, of 40 12.4 / 11.3, of 100 15.8 / 26; 30 portions of 9 behind 60 15.6 / 14.0, behind 130 17.5 / 18.4; 17 tokens behind
+    90 13.0 / 12.2, behind 200 16.1 / 18.2."""
+    keys = min([plan.max_context] + ([window + keep_first] if window else []) + ([chunk] if chunk else []))
+    return keys < (128 if plan.max_query_len >= 64 else 160) and rows * num_heads * keys < 1 << 20
+
+
 def _portion_splits(plan, S: int, num_heads: int, num_kv_heads: int, head_dim: int, window: int, keep_first: int, chunk: int,
                     total128: int) -> tuple[int, int]:
     """(keys per run, number of runs) for a step with prompt portions; (0, 1): every work-group of 128 columns walks its keys
@@ -1054,8 +1065,10 @@ def _attention_launch(plan, S: int, num_heads: int, num_kv_heads: int, head_dim:
         split_len, nsplit = _portion_splits(plan, S, num_heads, num_kv_heads, head_dim, window, keep_first, chunk, total128)
     runs = nsplit > 1 and not plan.decode_only and split_keys is None      # the tile kernel's walks in runs of keys
     waves = 8 if path == "mfma-tile32" else _tile32_waves(plan.q_lens, plan.starts, num_heads) if path in (None, "mfma") and not runs else 0
-    chains = 0 if path == "mfma-direct" or (head_dim == 256 and plan.max_query_len == 1) or (nsplit > 1 and not runs) \
-        else _tile16_chains(total128, num_kv_heads, path, plan.max_context)
+    alone = path == "mfma-direct" or (nsplit > 1 and not runs) or (head_dim == 256 and (plan.max_query_len == 1 or (
+        path in (None, "mfma") and not runs
+        and _walks_alone_at_256(plan, sum(q_lens) + pads, num_heads, window, keep_first, chunk))))
+    chains = 0 if alone else _tile16_chains(total128, num_kv_heads, path, plan.max_context)
     return _AttentionLaunch(len(singles), own, nt, max(groups + [1]), total128,
                             sum(-(-n * G // (32 * waves)) for n in q_lens) + pads if waves else 0, split_len, nsplit, waves, chains)
 

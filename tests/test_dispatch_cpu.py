@@ -79,3 +79,17 @@ def test_launches_worked_out_for_a_step_follow_its_facts():
                    lambda: setattr(facts, "max_context", 8000), lambda: setattr(facts, "num_seqs", 3)):
         change()
         assert K._worked_out_launch(facts, *key) == K._attention_launch(facts, *key)
+
+
+def test_short_prompts_at_a_head_size_of_256_walk_on_their_own():
+    def chains(q_lens, starts=None, heads=(32, 1), path=None, **mask):
+        starts = starts or [0] * len(q_lens)
+        facts = StepFacts(max_context=max(a + b for a, b in zip(q_lens, starts)), max_query_len=max(q_lens), num_seqs=len(q_lens),
+                          q_lens=q_lens, starts=starts)
+        m = dict(window=0, keep_first=0, chunk=0) | mask
+        return K._attention_launch(facts, len(q_lens), *heads, 256, m["window"], m["keep_first"], m["chunk"], path, None, None, False).chains
+    assert chains([17]) == chains([40]) == chains([64]) == chains([17] * 8) == chains([3] * 64) == chains([17], [120]) == 0
+    assert chains([130]) and chains([400]) and chains([2048]) and chains([100] * 8) and chains([17], [200])       # long walks, or many columns
+    assert chains([17], [200], window=64) == 0                                                  # a window bounds the walk
+    assert chains([17], path="mfma-tile16") == 1 and chains([400], path="mfma-direct") == 0
+    assert chains([2], [3000]) > 0                                                              # in runs of keys
