@@ -191,10 +191,18 @@ __global__ __launch_bounds__(AFD_WAVES * 64, 1) void attn_float_decode_kernel(
     }
 }
 
+// The heads and pages the kernel above is the faster one for.  More than eight query heads to a key/value head read the
+// keys once per eight; us here and on the any-shape kernel, whose 16 rows take up to 16 heads of one read: 16 heads of 128
+// 64 sequences of 1,000 40 and 42, of 16,000 526 and 567; 10 heads of 64 64 of 300 15 and 26, but 64 of 6,000 95 and 86, 8 of
+// 16,000 50 and 40; 32 heads of 128 200 of 300 72 and 67, 8 of 16,000 122 and 81.
+static bool afd_takes_heads(int nq, int nkv, int d, int bs) {
+    return nkv > 0 && ((d == 64 && nq / nkv <= AFD_HEADS) || (d == 128 && nq / nkv <= 2 * AFD_HEADS)) && bs >= 4 && (bs & (bs - 1)) == 0;
+}
+
 // Whether a float launch runs on the kernel above.  (q rows need no alignment: they are read one number at a time.)
 static bool afd_takes(const AgLaunch& a, int max_query_len, long long sequences) {
     const int chunks = tl_ceil_div(a.nq / a.nkv, AFD_HEADS);
-    return max_query_len == 1 && (a.d == 64 || a.d == 128) && a.bs_shift >= 2 && a.softcap == 0.f && !a.bias.table &&
+    return max_query_len == 1 && afd_takes_heads(a.nq, a.nkv, a.d, a.bs) && a.softcap == 0.f && !a.bias.table &&
            (long long)chunks * a.nsplit <= 65535 && sequences <= 0x7fffffffLL && (uintptr_t)a.k_cache % 16 == 0 && (uintptr_t)a.v_cache % 16 == 0;
 }
 

@@ -6,6 +6,9 @@
 
 void tl_attention_generic_bf16(const AgLaunch& a);
 
+// Whether float steps of one token per sequence, without cap and bias, run on attention_float_decode.h, in its runs of keys.
+extern "C" int tl_attention_float_decode_takes(int nq, int nkv, int d, int bs) { return afd_takes_heads(nq, nkv, d, bs) ? 1 : 0; }
+
 // q_start: int32 [S + 1], the first row of each sequence in the flat batch (rows of a sequence are
 // consecutive); max_query_len: the most tokens one sequence brings to this step.  nsplit > 1 cuts
 // the keys into runs of split_keys (a multiple of 64) at absolute positions, one work-group each,

@@ -1227,8 +1227,8 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     # takes), whatever the batch: one work-group per sequence and key/value head would walk a long context alone.
     split_len, nsplit, ws = 0, 1, None
     if plan is not None and plan.decode_only and max_query_len == 1 and split_keys != 0:
-        float_form = (q.dtype == torch.float32 and head_dim in (64, 128) and page >= 4 and page & (page - 1) == 0
-                      and not softcap and bias is None)
+        float_form = (q.dtype == torch.float32 and not softcap and bias is None
+                      and library().tl_attention_float_decode_takes(num_heads, num_kv_heads, head_dim, page))
         split_len, nsplit = _fit_key_splits(int(split_keys) if split_keys else FLOAT_DECODE_SPLIT_KEYS if float_form
                                             else GENERIC_SPLIT_KEYS, plan.max_context, plan.fit_context)
         _check(split_len % 64 == 0, "paged_attention: a split of the any-shape kernel is a multiple of 64 keys")

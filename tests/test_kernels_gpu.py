@@ -1315,7 +1315,7 @@ def test_few_rows_in_half_tiles(M, N, Kd):
     torch.testing.assert_close(got2.double(), h @ w2.double().T, atol=2e-4, rtol=2e-4)
 
 
-@pytest.mark.parametrize("nq,nkv,d,bs", [(3, 3, 128, 4), (6, 2, 64, 16), (28, 4, 128, 16), (18, 2, 64, 8), (17, 1, 128, 512)])
+@pytest.mark.parametrize("nq,nkv,d,bs", [(3, 3, 128, 4), (6, 2, 64, 16), (28, 4, 128, 16), (18, 2, 64, 8), (17, 1, 128, 512), (18, 2, 128, 8), (16, 1, 128, 512), (16, 2, 64, 8)])
 @pytest.mark.parametrize("split", [None, 0, 64])
 @pytest.mark.parametrize("kw", [{}, dict(sink=True), dict(window=70), dict(window=44, keep_first=5), dict(chunk=96)])
 def test_float_attention_of_one_token_steps(nq, nkv, d, bs, split, kw):
