@@ -1916,14 +1916,18 @@ def moe_tile_rows(pairs: int, experts: int) -> int:
 MOE_WIDE_TILE = 256      # rows at most of a tile of the grouped bfloat16 product of many rows per expert
 
 
-def _moe_takes_wide_tiles(pairs: int, experts: int, ff: int) -> bool:
-    """Whether the experts' products run in tiles of up to 256 rows by 256 matrix rows (a work-group of one per CU) and not in
-    tiles of 64 by 128.  They fetch each matrix once and the rows half as often, which pays from few rows on where there are
+def _moe_takes_wide_tiles(pairs: int, experts: int, ff: int, width: int) -> bool:
+    """Whether the experts' products (ff x width) run in tiles of up to 256 rows by 256 matrix rows (a work-group of one per CU)
+    and not in tiles of 64 by 128.  They fetch each matrix once and the rows half as often, which pays where there are
     twice as many tiles as CUs (64 experts of 4,096 x 2,048, both products: 18 rows per expert 647 against 693 us, 90: 754
     against 932, 192: 1,066 against 1,475; of 2,048 x 1,408: 18 rows 239 against 246, 192: 433 against 616), and not where there
-    are fewer (32 experts of 1,024 x 512: 188 rows, with half a tile per CU, 101 against 75 us, 562 rows 183 against 169)."""
-    rows = -(-pairs // experts)
-    return experts * -(-rows // MOE_WIDE_TILE) * -(-ff // 128) >= 512
+    are fewer (32 experts of 1,024 x 512: 188 rows, with half a tile per CU, 101 against 75 us, 562 rows 183 against 169).
+    Small matrices for few rows stay in small tiles, whose start is cheaper: 256 experts of 1,024 x 256 17 rows 114 against 107,
+    32 130 against 121, 48 146 against 149; of 512 x 512 32 rows 132 against 119, 64 164 against 167; 512 of 512 x 256 48 rows 176
+    against 164, 64 199 against 203; 128 of 2,048 x 512 17 rows 200 against 207."""
+    rows, size = -(-pairs // experts), ff * width
+    return (experts * -(-rows // MOE_WIDE_TILE) * -(-ff // 128) >= 512
+            and (rows >= 64 or size >= 1 << 20 or (rows >= 48 and size >= 1 << 18)))
 
 
 def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
@@ -1949,7 +1953,7 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
         _f32(shared, "moe_experts shared", T * N)
     P = T * top
     BM = moe_tile_rows(P, E)
-    if (BM == 64 and _moe_takes_wide_tiles(P, E, F) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
+    if (BM == 64 and _moe_takes_wide_tiles(P, E, F, K) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
             and library().tl_moe_gemm_takes_wide(F) and (T == 1 or h.stride(0) % 8 == 0)
             and (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0):
         BM = MOE_WIDE_TILE

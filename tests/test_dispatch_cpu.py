@@ -93,3 +93,11 @@ def test_short_prompts_at_a_head_size_of_256_walk_on_their_own():
     assert chains([17], [200], window=64) == 0                                                  # a window bounds the walk
     assert chains([17], path="mfma-tile16") == 1 and chains([400], path="mfma-direct") == 0
     assert chains([2], [3000]) > 0                                                              # in runs of keys
+
+
+def test_experts_in_wide_tiles_by_tiles_rows_and_size():
+    wide = lambda rows, experts, width, ff: K._moe_takes_wide_tiles(rows * experts, experts, ff, width)
+    assert wide(18, 64, 4096, 2048) and wide(18, 64, 2048, 1408) and wide(17, 128, 2048, 768) and wide(17, 128, 2048, 512)
+    assert not wide(188, 32, 1024, 512) and not wide(100, 8, 4096, 2048)            # fewer than two tiles per CU
+    assert not wide(17, 256, 1024, 256) and not wide(32, 256, 512, 512) and not wide(48, 512, 512, 256)      # small, few rows
+    assert wide(48, 256, 1024, 256) and wide(64, 256, 512, 512) and wide(64, 512, 512, 256)
