@@ -18,7 +18,7 @@
 //   one column 3,000 times the rest  5.9e-8 5.9e-8 8.4e-8    3.9e-7 3.9e-7 6.2e-7    4.6e-7 4.6e-7 1.3e-6    6.9e-7 6.9e-7 2.9e-6
 // The two more products cost 20% (gate/up of 2,048 rows 2.74 -> 3.34 ms) and change nothing from K = 16 on; below, where a
 // result is a handful of products, the matrix instruction's own last addition is the error (K = 1: 3.4e-8 with six or eight,
-// 2.6e-8 on the float instruction), and such products go to the float instruction.  Six bfloat16 products take 6 / 16 of the
+// 2.6e-8 on the float instruction), and products of a K below 64 go to the float instruction.  Six bfloat16 products take 6 / 16 of the
 // matrix cores' time of one on the float instruction (2.5 PFLOP/s against 157 TFLOP/s).
 //
 // What is split where: the rows of A once, by a pass of its own, into the order in which the product reads

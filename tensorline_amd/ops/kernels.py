@@ -580,7 +580,7 @@ SKINNY_MAX_ROWS = 16     # rows the few-row kernel serves (one 16-row MFMA tile)
 ROWS64_MAX_ROWS = 64     # rows the 17..64-row kernel serves; above that the library
 FLOAT_SPLIT_MAX_ROWS = 65535 * 32   # rows one launch of the float product of more than 16 rows takes
 FLOAT_SPLIT_BYTES = 512 << 20   # at most this much for the parts of a launch's rows: more rows go in several launches
-FLOAT_SPLIT_MIN_K = 16   # below: the float instruction, whose error is smaller there (gemm_float.hip)
+FLOAT_SPLIT_MIN_K = 64   # below: the float instruction (_float_split)
 
 
 def _skinny_ok(a: torch.Tensor, shuffled: torch.Tensor | None, M: int, K: int, lda: int) -> bool:
@@ -608,11 +608,13 @@ def _few_rows_go_to_rows64(N: int, K: int) -> bool:
 
 def _float_split(a, shuffled, bias, out, M, N, K, lda, ldc):
     """More than 16 float rows: every float as the sum of three bfloat16 numbers on the bfloat16 matrix instruction,
-    the weight from its matrix-core ordered copy.  Every matrix with the copy and a K of 16 or more goes here, whatever its
-    rows beyond 16, so that a row's bits do not depend on how many others come along: at 33 rows and more it is the faster
-    kernel at every K (300 rows, N = 1,152: K = 64 8.2 us against 16, 896 29 against 92).  17 to 32 rows pay for that one order
-    of summation below K = 896, us here and on the float instruction, 17 rows of 1,152: K = 16 3.7 and 2.9, 64 5.2 and 4.1,
-    128 7.1 and 5.8, 256 11.2 and 9.1, 512 17.3 and 15.9, 896 26.3 and 25.7, 3,584 52 and 95."""
+    the weight from its matrix-core ordered copy.  Every matrix with the copy and a K of 64 or more goes here, whatever its
+    rows beyond 16, so that a row's bits do not depend on how many others come along.  Measured, us here and on the float
+    instruction, N = 1,152: 33 rows K = 16 7.0 and 5.8, 64 8.2 and 8.2, 128 9.8 and 11.5, 896 28 and 51; 128 rows K = 16 6.9
+    and 12.2, 64 8.3 and 16.5, 896 29 and 89; 1,000 rows of 9,728 K = 16 25 and 18, 64 31 and 30, 128 39 and 43, 896 130 and
+    204.  17 to 32 rows pay for the one order of summation from K = 64 to 896: 17 rows K = 64 5.7 and 4.8, 128 7.6 and 6.4, 256
+    12.1 and 9.7, 512 18.2 and 16.4, 896 27.2 and 26.3, 1,027 31 and 44, 4,864 54 and 147.  (Below K = 16 the float
+    instruction's error is the smaller one, too: gemm_float.hip.)"""
     most = max(128, FLOAT_SPLIT_BYTES // (-(-K // 16) * 96) // 128 * 128)
     split = ws = None
     if M > 32 or a.data_ptr() % 16 or not library().tl_gemm_float_split_takes_rows(M, K, lda):
@@ -637,8 +639,9 @@ def _rows64(a, shuffled, bias, out, M, N, K, lda, ldc, swiglu: bool, norm=None):
 
 def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None) -> torch.Tensor:
     """bfloat16 with few rows: the streaming MFMA kernels.  float32 with the matrix-core ordered copy: the few-row kernel,
-    or (more than 16 rows, a K of 16 or more) the float product on the bfloat16 instruction.  The rest: the plain tiled kernel.  (bfloat16 with many rows went to the library before this, where
-    the reference uses one too: tensorline/paged.py:179-188.)"""
+    or (more than 16 rows, a K of 64 or more) the float product on the bfloat16 instruction.  The rest: the plain tiled
+    kernel.  (bfloat16 with many rows went to the library before this, where the reference uses one too:
+    tensorline/paged.py:179-188.)"""
     if _skinny_ok(a, shuffled, M, K, lda) and not _few_rows_go_to_rows64(N, K):
         _call("tl_gemm_skinny", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), _code(out, "linear output"),
               M, N, K, lda, ldc, None, _stream())

@@ -178,7 +178,7 @@ def test_linear_float_by_three_bfloat16_not_finite():
     torch.testing.assert_close(got[fine], want[fine], atol=1e-3, rtol=1e-5)
 
 
-@pytest.mark.parametrize("Kd", [1, 2, 3, 7, 15, 16, 33, 128, 896, 3584])
+@pytest.mark.parametrize("Kd", [1, 2, 3, 7, 15, 16, 33, 64, 128, 896, 3584])
 @pytest.mark.parametrize("values", ["normal", "positive", "one column large"])
 def test_linear_float_is_no_further_from_64_bits_than_the_float_instruction(Kd, values):
     """More than 16 float rows, at every K: not further from the exact product, in the 2-norm, than the product on the float
@@ -196,7 +196,7 @@ def test_linear_float_is_no_further_from_64_bits_than_the_float_instruction(Kd, 
         assert bool(((got.double() - want).abs() <= 2.0 ** -24 * want.abs()).all())
 
 
-@pytest.mark.parametrize("N,Kd", [(33, 16), (70, 20), (130, 36), (1000, 60), (257, 128), (40, 252), (1152, 256)])
+@pytest.mark.parametrize("N,Kd", [(33, 64), (70, 68), (130, 76), (1000, 100), (257, 128), (40, 252), (1152, 256)])
 @pytest.mark.parametrize("M", [17, 30, 32])
 def test_linear_float_of_at_most_32_rows_splits_them_where_they_are_used(M, N, Kd):
     """One launch for 17 to 32 aligned rows: the bits that the same rows get from parts made beforehand (rows that are not
