@@ -242,6 +242,25 @@ def _float_tile(tile, parts, M, N, Kd):
 
 
 @pytest.mark.parametrize("tile,parts,M,N,Kd", FLOAT_TILES)
+def test_linear_float_in_every_tile(tile, parts, M, N, Kd):
+    """The bound of K float multiply-adds, ends of rows, columns and k, and a row's bits whatever rows come along: 17 rows (the
+    smallest tile) and 70 (the next) against the tile that M rows take; columns either side of the result untouched."""
+    _float_tile(tile, parts, M, N, Kd)
+    torch.manual_seed(tile + 20)
+    a, w, b = torch.randn(M, Kd, device=DEV), torch.randn(N, Kd, device=DEV), torch.randn(N, device=DEV)
+    ws = K().shuffle_weight_float(w)
+    wide = torch.full((M, N + 3), 7.0, device=DEV)
+    got = K().linear(a, w, b, out=wide[:, 1:N + 1], shuffled=ws)
+    assert bool((wide[:, [0, N + 1, N + 2]] == 7.0).all())
+    want, size = a.double() @ w.double().T + b.double(), a.double().abs() @ w.double().abs().T + b.double().abs()
+    assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())
+    for n in (17, 70):
+        assert torch.equal(K().linear(a[M - n:], w, b, shuffled=ws), got[M - n:])
+        assert torch.equal(K().linear(a[:n].contiguous(), w, b, shuffled=ws), got[:n])
+    assert K().library().tl_gemm_float_split_tile(17, N, Kd) & 3 == 3 and (tile == 3 or K().library().tl_gemm_float_split_tile(70, N, Kd) & 3 != tile)
+
+
+@pytest.mark.parametrize("tile,parts,M,N,Kd", FLOAT_TILES)
 def test_linear_float_not_finite_in_every_tile(tile, parts, M, N, Kd):
     """Infinities, NaN, values that round to infinity as bfloat16 and a product just below the largest float whose rounded
     parts' product is above it, in either segment: what plain float arithmetic gives; every other element as without them."""
@@ -524,16 +543,19 @@ def test_product_adds_into_the_residual_and_prepares_the_next_norm(M, N, Kd):
 
 def _attention_case(dtype, nq, nkv, d, bs, lens, q_lens=None, window=0, seed=0, spike=False, path=None, split_keys=None,
                     route_singles=None, pool_pages=None, spike_at=None, sink=False, spike_gain=4.0, score_shift=0.0,
-                    keep_first=0, chunk=0, softcap=0.0, bias=None):
+                    keep_first=0, chunk=0, softcap=0.0, bias=None, pads=0):
     """Sequences of context ``lens``; the last ``q_lens[i]`` positions of each are queries.
     pool_pages: the sequences' pages are the last ones of a pool of that many.  ``spike``: the key
     at position 1 (or at ``spike_at(position of the query)``, if that is a key at all) is made to
     match its query, so that it dominates the sum if it is seen.  ``score_shift``: the first dimension of
     every key and query is set so that it takes that much off every score.  ``sink``: True for a logit of 0 in every head, or
-    the heads' logits; ``softcap``: scores bent by that cap; ``bias`` [nq, reach + 1]: added by distance."""
+    the heads' logits; ``softcap``: scores bent by that cap; ``bias`` [nq, reach + 1]: added by distance.  ``pads``: so many padding
+    sequences of one token behind the others, which the step's facts do not list."""
     torch.manual_seed(seed)
+    real = len(lens)
+    q_lens = (q_lens or [1] * real) + [1] * pads
+    lens = lens + [1] * pads
     S = len(lens)
-    q_lens = q_lens or [1] * S
     nb = max(-(-n // bs) for n in lens)
     num_blocks = S * nb + 8
     kc = torch.randn(num_blocks, bs, nkv, d, device=DEV).to(dtype)
@@ -573,7 +595,7 @@ def _attention_case(dtype, nq, nkv, d, bs, lens, q_lens=None, window=0, seed=0, 
     for ql in q_lens:
         qs.append(qs[-1] + ql)
     plan = StepFacts(max_context=max(lens), max_query_len=max(q_lens), decode_only=max(q_lens) == 1,
-                     num_seqs=S, q_lens=list(q_lens), starts=[n - ql for n, ql in zip(lens, q_lens)])
+                     num_seqs=S, q_lens=list(q_lens[:real]), starts=[n - ql for n, ql in zip(lens, q_lens)][:real])
     single_seqs = None
     logits = None if sink is False else torch.zeros(nq) if sink is True else torch.as_tensor(sink, dtype=torch.float32)
     if K().one_token_sequences(plan):
@@ -581,7 +603,7 @@ def _attention_case(dtype, nq, nkv, d, bs, lens, q_lens=None, window=0, seed=0, 
     out = K().paged_attention(q, kc, vc, tables, torch.tensor(seq_of, dtype=torch.int32, device=DEV),
                               torch.tensor(pos, dtype=torch.int32, device=DEV), nq, nkv, d, d ** -0.5, window=window,
                               q_start=torch.tensor(qs, dtype=torch.int32, device=DEV),
-                              ctx_start=torch.tensor(plan.starts, dtype=torch.int32, device=DEV), plan=plan,
+                              ctx_start=torch.tensor(plan.starts + [0] * pads, dtype=torch.int32, device=DEV), plan=plan,
                               path=path, split_keys=split_keys, single_seqs=single_seqs, route_singles=route_singles,
                               sink=None if logits is None else logits.to(DEV), keep_first=keep_first, chunk=chunk, softcap=softcap,
                               bias=None if bias is None else bias.to(DEV))
@@ -1263,7 +1285,8 @@ def test_batched_linear_bfloat16(T, B, N, Kd):
 
 
 @pytest.mark.parametrize("nq,nkv,d,bs,lens,q_lens,kw", [
-    (12, 2, 128, 16, [3200, 40, 1, 1400, 129], [70, 40, 1, 1, 129], {}),                # behind a long context, beside one-token requests
+    (12, 2, 128, 16, [3200, 40, 1, 300, 129], [70, 40, 1, 1, 129], {}),                 # behind a long context, beside one-token requests
+    (12, 2, 128, 16, [3200, 40], [70, 40], dict(pads=3)),                               # beside padding sequences
     (14, 2, 64, 16, [4097, 300], [65, 1], dict(spike=True)),                            # one far key dominates
     (4, 1, 32, 8, [2048, 2047], [3, 130], {}),                                          # runs' edges
     (8, 1, 256, 16, [3000, 64], [40, 64], dict(sink=True)),
@@ -1271,17 +1294,19 @@ def test_batched_linear_bfloat16(T, B, N, Kd):
     (8, 2, 64, 16, [4000, 2100], [100, 30], dict(chunk=1600, softcap=20.0)),
     (4, 4, 32, 64, [2500, 2000], [60, 5], dict(bias=True)),
     (6, 1, 128, 24, [3000], [40], {}),                                                  # pages of no power of two: independent waves in runs
+    (4, 1, 128, 16, [3000, 1500], [4, 2], {}),                                          # one column tile of 16: independent waves in runs
 ])
-def test_attention_portions_in_runs_of_keys(nq, nkv, d, bs, lens, q_lens, kw):
-    """Prompt portions of few columns behind long contexts, their walks cut into runs that a second kernel puts together."""
-    from tensorline_amd.engine.batch import StepFacts
+def test_attention_portions_in_runs_of_keys(nq, nkv, d, bs, lens, q_lens, kw, monkeypatch):
+    """Prompt portions of few columns behind long contexts, their walks cut into runs that a second kernel puts together; the
+    one-token sequences beside them stay in the step."""
     if kw.get("bias"):
         kw = dict(kw, bias=torch.randn(nq, 41))
-    total = sum(-(-n * (nq // nkv) // 128) for n in q_lens)
-    facts = StepFacts(max_context=max(lens), max_query_len=max(q_lens), num_seqs=len(lens), q_lens=q_lens,
-                      starts=[n - q for n, q in zip(lens, q_lens)])
-    assert K()._portion_splits(facts, len(lens), nq, nkv, d, kw.get("window", 0), kw.get("keep_first", 0), kw.get("chunk", 0), total)[1] > 1
+    chosen, choose = [], K()._attention_launch
+    monkeypatch.setattr(K(), "_attention_launch", lambda *a: chosen.append(choose(*a)) or chosen[-1])
     got, want = _attention_case(torch.bfloat16, nq, nkv, d, bs, lens, q_lens, seed=21, **kw)
+    launch, = chosen
+    assert launch.nsplit > 1 and launch.chains > 0 and launch.own_split is None
+    assert launch.nt == (1 if d == 256 or max(q_lens) * nq // nkv <= 16 else 2)
     torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
 
 
@@ -1325,6 +1350,26 @@ def test_float_attention_of_one_token_steps(nq, nkv, d, bs, split, kw):
     lens = [1, 2, 5, 31, 32, 33, 65, 127, 128, 129, 256, 257, 1030]
     got, want = _attention_case(torch.float32, nq, nkv, d, bs, lens, None, seed=nq + d, path="generic", split_keys=split, **kw)
     torch.testing.assert_close(got, want, **tol(torch.float32, 2e-5))
+
+
+def test_draws_queued_one_behind_the_other_keep_their_own_numbers():
+    """Draws whose numbers come from pinned memory, none awaited before the next is issued: what the kernels give for the same
+    numbers in tensors of their own."""
+    from tensorline_amd.sampling.sampler import Sampler, uniform_for
+    torch.manual_seed(5)
+    sampler, R, V = Sampler(DEV), 6, 9000
+    logits = torch.randn(R, V, device=DEV) * 3
+    busy = torch.randn(2048, 2048, device=DEV)
+    cases = [([0.3 + 0.05 * ((i + r) % 30) if (i + r) % 5 else 0.0 for r in range(R)], [1.0 - 0.1 * ((i * r) % 7) for r in range(R)],
+              [i * 100 + r for r in range(R)], [i] * R) for i in range(200)]
+    got = []
+    for case in cases:
+        busy = torch.mm(busy, busy) * 1e-3                   # the GPU stays behind the host
+        got.append(sampler.sample_device(logits, *case))
+    for (temps, tops, seeds, at), tokens in zip(cases, got):
+        u = [uniform_for(s, i) for s, i in zip(seeds, at)]
+        t, p, x = (torch.tensor(v, dtype=torch.float32).to(DEV) for v in (temps, tops, u))
+        assert torch.equal(K().sample(logits, t, p, x, any_top_p=True, any_greedy=True), tokens)
 
 
 @pytest.mark.parametrize("V", [4096, 4097, 262144, 262145, 270001])
