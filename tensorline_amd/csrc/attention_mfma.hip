@@ -64,7 +64,13 @@ __device__ __forceinline__ float am_column_max(float v) {
 }
 
 #define AM_LOG2E 1.4426950408889634f
-#define AM_LAZY 8.0f                 // how far a block's maximum may exceed the running one before it moves
+// How far a tile's maximum may exceed the running one before it moves (base 2), by the head size 32 DC.  While it does not move the
+// largest weight is a number below 2^8 that is rounded to bfloat16 where it would be 1 exactly: 3% on the result's rounding
+// error.  At a head size of 256 it always moves, as on the independent waves that those portions ran on before: against 64 bits,
+// 600 tokens of 16 heads 1.986e-3 where 8 gave 2.037e-3 and the waves give 1.975e-3 (40 tokens behind 3,000: 2.18e-3, 2.31e-3, 2.29e-3),
+// for 3 to 4% of the time (2,048 tokens of 32 heads 92.6 us against 89.2).
+template <int DC>
+__device__ __forceinline__ constexpr float am_lazy() { return DC >= 8 ? 0.0f : 8.0f; }
 #define AM_NO_COLUMN 0x7fffffff      // position of a lane without a column: never masks, never written
 
 // One block of 32 keys for the NT column tiles of a wave: scores, online softmax, P*V.
@@ -377,10 +383,10 @@ __device__ __forceinline__ void am_block_lds(const uint4* kt, const uint4* vt, i
         }
         const float bmax = am_column_max(am_max3(am_max3(sv[0], sv[1], sv[2]), am_max3(sv[3], sv[4], sv[5]), am_max3(sv[6], sv[7], sv[7])));
         // The running maximum follows the true one lazily: it moves only when the block's maximum
-        // exceeds it by more than AM_LAZY (in the base-2 domain), so probabilities stay below
-        // 2^AM_LAZY and the accumulator is rescaled in few blocks instead of most.  Sums and
+        // exceeds it by more than am_lazy (in the base-2 domain), so probabilities stay below
+        // 2^am_lazy and the accumulator is rescaled in few blocks instead of most.  Sums and
         // accumulators stay relative to the same running maximum, so the result is the same.
-        const bool moved = bmax > m_run[j] + AM_LAZY;         // also the first keys: -inf + AM_LAZY is -inf
+        const bool moved = bmax > m_run[j] + am_lazy<DC>();   // also the first keys: -inf + 8 is -inf
         const float m_new = moved ? bmax : m_run[j];
         const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
         float pr[8], psum = 0.f;
@@ -506,7 +512,7 @@ __device__ __forceinline__ void am_tile_lds(const uint4* kt, const uint4* vt, in
                          am_max3(am_max3(sv[7], sv[8], sv[9]), am_max3(sv[10], sv[11], sv[12]), sv[13]), am_max3(sv[14], sv[15], sv[15]));
     bmax = am_column_max(bmax);
     if (!CAP) bmax *= scale2;                                // the scale is positive: the order is the same
-    const bool moved = bmax > m_run + AM_LAZY;               // also the first keys: -inf + AM_LAZY is -inf
+    const bool moved = bmax > m_run + am_lazy<DC>();         // also the first keys: -inf + 8 is -inf
     const float m_new = moved ? bmax : m_run;
     const float neg_m = (m_new == -INFINITY) ? 0.f : -m_new;
     float pr[16];
@@ -558,8 +564,8 @@ __device__ __forceinline__ void am_tile_lds(const uint4* kt, const uint4* vt, in
 // multiplied; every wave waits for its own loads before the one barrier of the iteration.  The
 // sequence's page ids are copied to LDS first, so a tile's addresses depend on no load from
 // memory.  Pages must hold a power of two of tokens (at least 8; 2^bs_shift): an 8-key run of V^T
-// then lies in one page and a page id is a shift away.  No key split: a step with prompt portions
-// has columns enough.
+// then lies in one page and a page id is a shift away.  Keys are split (SPLIT below) only where a step's
+// portions have too few columns for the GPU behind long contexts.
 #define AT_KEYS 64
 #define AT_CUS 256                   // compute units of the GPU
 #define AT_NT 1                      // column tiles per wave; 8 / AT_NT waves in a work-group
