@@ -582,22 +582,6 @@ template <int UPK>
 __device__ __forceinline__ int at_k_swizzle(int row) { return ((row & 15) * (UPK < 16 ? UPK : 16)) >> 4; }
 __device__ __forceinline__ int at_v_swizzle(int row) { return (row >> 1) & 7; }
 
-// 16 bytes per lane from memory straight into LDS at lds_base + 16 * lane (lds_base is the same for
-// the whole wave).  Written as assembly so that the compiler does not make every later LDS read wait
-// for it: a load is waited for only where AT_LANDED says so.  M0 holds the LDS base for the
-// instruction and is put back.
-__device__ __forceinline__ void at_load_to_lds_at(const void* g, uint32_t lds_base) {
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "s"(lds_base), "v"(g)
-        : "memory");
-}
-__device__ __forceinline__ void at_load_to_lds(const void* g, void* lds_base) {
-    at_load_to_lds_at(g, (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds_base);
-}
-
 // CH = 2 ("two chains"): a work-group of twice the waves, whose second half takes every other tile of
 // the same columns, with tile buffers, running maximum, sum and accumulator of its own; at the end
 // the halves are put together through LDS as two splits of the keys are.  For steps with at most one
@@ -794,11 +778,11 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
             const int w_ = wave_u + i * WAVES;                                                                \
             if (w_ < UPK) {                                                                                   \
                 if (CH > 1) {                                                                                 \
-                    at_load_to_lds_at(gk_[i], ks_lds + buf_ + w_ * 1024);                                     \
-                    at_load_to_lds_at(gv_[i], vs_lds + buf_ + w_ * 1024);                                     \
+                    tl_load_to_lds(gk_[i], ks_lds + buf_ + w_ * 1024);                                        \
+                    tl_load_to_lds(gv_[i], vs_lds + buf_ + w_ * 1024);                                        \
                 } else {                                                                                      \
-                    at_load_to_lds(gk_[i], ks + (BUF) * TILE + w_ * 64);                                      \
-                    at_load_to_lds(gv_[i], vs + (BUF) * TILE + w_ * 64);                                      \
+                    tl_load_to_lds(gk_[i], tl_lds_address(ks + (BUF) * TILE + w_ * 64));                      \
+                    tl_load_to_lds(gv_[i], tl_lds_address(vs + (BUF) * TILE + w_ * 64));                      \
                 }                                                                                             \
             }                                                                                                 \
         }                                                                                                     \

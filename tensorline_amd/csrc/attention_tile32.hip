@@ -81,22 +81,9 @@ __device__ __forceinline__ int t32_row_key(int row) {
     return 16 * (b >> 1) + 8 * h + 4 * (b & 1) + i;
 }
 
-// 16 bytes per lane from memory straight into LDS at lds_base + 16 * lane (lds_base is the same for
-// the whole wave).  Written as assembly so that the compiler does not make every later LDS read
-// wait for it: a load is waited for only where T32_LANDED says so.  M0 holds the LDS base for the
-// instruction and is put back.  Two forms: a 64-bit address per lane, and a wave-wide 64-bit base
-// in scalar registers plus a 32-bit offset per lane.
-__device__ __forceinline__ void t32_load_to_lds(const void* g, void* lds_base) {
-    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds_base;
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "s"(base), "v"(g)
-        : "memory");
-}
+// tl_load_to_lds with a wave-wide 64-bit base in scalar registers plus a 32-bit offset per lane; T32_LANDED waits for both.
 __device__ __forceinline__ void t32_load_to_lds_based(const void* wave_base, uint32_t voff, void* lds_base) {
-    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds_base;
+    const uint32_t base = tl_lds_address(lds_base);
     // the base is the same in every lane; said so explicitly, it lives in scalar registers
     const uint64_t a = (uint64_t)(uintptr_t)wave_base;
     const uint64_t sbase = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) |
@@ -403,7 +390,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_tile32_kernel(
             const uint32_t page_ = (uint32_t)__builtin_amdgcn_readfirstlane(k_page[i]);                       \
             const char* sk_ = kc_bytes + (uint64_t)((page_ << bs_shift) + (uint32_t)(k0_ & (bs - 1))) * k_stride; \
             t32_load_to_lds_based(sk_, k_voff, ks + (BUF) * TILE + L_ * 64);                                   \
-            t32_load_to_lds(gv_ + (uint64_t)L_ * v_lstep, vs + (BUF) * TILE + L_ * 64);                        \
+            tl_load_to_lds(gv_ + (uint64_t)L_ * v_lstep, tl_lds_address(vs + (BUF) * TILE + L_ * 64));         \
         }                                                                                                      \
     }
     // every load of this wave has landed (vmcnt 0; the other counters are left alone)

@@ -164,6 +164,19 @@ __device__ __forceinline__ float tl_score2(float raw, float scale2, float cap2, 
     return __builtin_fmaf(raw, scale2, add);
 }
 
+// 16 bytes per lane from memory straight into LDS at lds_base + 16 * lane (lds_base, an LDS address, is the same for the whole
+// wave).  Written as assembly so that the compiler does not make every later LDS read wait for it: a kernel waits with
+// s_waitcnt vmcnt where it needs the data.  M0 holds the LDS base for the instruction and is put back.
+__device__ __forceinline__ void tl_load_to_lds(const void* g, uint32_t lds_base) {
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "s"(lds_base), "v"(g)
+        : "memory");
+}
+__device__ __forceinline__ uint32_t tl_lds_address(void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)p; }
+
 // ---- host side -----------------------------------------------------------------------------
 // Every C entry point returns 0 on success.  On failure it returns a non-zero code and leaves a
 // message that tl_last_error() hands out; nothing is launched in that case.

@@ -108,16 +108,9 @@ __global__ __launch_bounds__(256) void fs_split_kernel(const float* __restrict__
     o[128] = lo;
 }
 
-// 16 bytes per lane from memory straight into LDS at lds_base + 16 * lane.  Written as assembly so that the
-// compiler does not make every LDS read wait for it: the loads are waited for where FS_LANDED says so.
+// tl_load_to_lds, the address made a scalar; waited for where FS_LANDED says so
 __device__ __forceinline__ void fs_load_to_lds(const void* g, void* lds_base) {
-    const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds_base);
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "s"(base), "v"(g)
-        : "memory");
+    tl_load_to_lds(g, (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(lds_base)));
 }
 // at most N of this wave's loads are still on their way, and its LDS reads are done
 #define FS_LANDED(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory")

@@ -596,18 +596,15 @@ __global__ __launch_bounds__(MG_THREADS) void moe_gemm_bf16_kernel(const bf16_t*
 #define MGW_KT 64
 #define MGW_W 2048                       // 16-byte units of 256 matrix rows in a stage
 #define MGW_LDS (144 * 1024)
-#define MGW_LOAD(NAME, POLICY)                                                                                                  \
-    __device__ __forceinline__ void NAME(const void* g, void* lds_base) {                                                       \
-        const uint32_t base =                                                                                                   \
-            (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds_base); \
-        uint32_t saved;                                                                                                         \
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off" POLICY "\n\ts_mov_b32 m0, %0" \
-                     : "=&s"(saved)                                                                                             \
-                     : "s"(base), "v"(g)                                                                                        \
-                     : "memory");                                                                                               \
-    }
-MGW_LOAD(mgw_load_to_lds, "")
-MGW_LOAD(mgw_load_to_lds_once, " nt")
+__device__ __forceinline__ uint32_t mgw_lds_address(void* p) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(p)); }
+// tl_load_to_lds for what is read once: it leaves no trace in the caches
+__device__ __forceinline__ void mgw_load_to_lds_once(const void* g, uint32_t lds_base) {
+    uint32_t saved;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off nt\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "s"(lds_base), "v"(g)
+                 : "memory");
+}
 
 template <int MW, int MODE>
 __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ We, void* __restrict__ Cv, int ldc,
@@ -639,9 +636,9 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
     auto fetch = [&](int buf) {
         uint4* stage = lds + buf * STAGE;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) mgw_load_to_lds_once(wp[i], stage + (wave * 8 + i) * 64);
+        for (int i = 0; i < 8; ++i) mgw_load_to_lds_once(wp[i], mgw_lds_address(stage + (wave * 8 + i) * 64));
 #pragma unroll
-        for (int i = 0; i < 2 * MW; ++i) mgw_load_to_lds(ap[i], stage + MGW_W + (wave * 2 * MW + i) * 64);
+        for (int i = 0; i < 2 * MW; ++i) tl_load_to_lds(ap[i], mgw_lds_address(stage + MGW_W + (wave * 2 * MW + i) * 64));
         if (++ahead < nsteps) {          // at the end the last step again, into a buffer that nobody reads
 #pragma unroll
             for (int i = 0; i < 8; ++i) wp[i] += MGW_KT;
