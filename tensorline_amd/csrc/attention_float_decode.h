@@ -1,5 +1,6 @@
 // Float attention of steps that bring one token per sequence (the 32-bit path's decode steps): head sizes 64 and 128,
-// pages of a power of two of at least four tokens, no cap and no bias.  Everything is float multiply-adds.
+// pages of a power of two of at least four tokens, up to 8 (at 64) or 16 query heads to a key/value head, no cap and no
+// bias.  Everything is float multiply-adds.
 //
 // What such a step has to do is read the cache: 75 MB a layer for 8 sequences of 2,300 keys and 4 key/value heads of 128.  The
 // any-shape kernel, whose tiles of keys go through LDS to the matrix cores between two barriers with one chain of dependent

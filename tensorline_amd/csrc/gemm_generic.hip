@@ -1,8 +1,8 @@
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]):  the any-shape matrix product.
 //
 // Float inputs, float products and sums on the matrix cores' float instruction v_mfma_f32_16x16x4_f32: the true 32-bit
-// path's product of up to 16 rows and of weights without a matrix-core ordered copy (with one, 17 rows and more go
-// to gemm_float.hip: 4.87 against 2.73 ms at 2,048 rows of 37,888 x 3,584), and the any-shape fallback for bfloat16 inputs
+// path's product of up to 16 rows, of a K below 64 and of weights without a matrix-core ordered copy (with one, 17 rows and
+// more go to gemm_float.hip: 4.84 against 2.79 ms at 2,048 rows of 37,888 x 3,584), and the any-shape fallback for bfloat16 inputs
 // (converted to float on the way into LDS, which is exact).  Any M, N and K, any row strides.
 //
 // One output element is summed over k in one fixed order: steps of 16 from k = 0 upwards, four
