@@ -58,7 +58,9 @@ typedef float fs_f32x16 __attribute__((ext_vector_type(16)));
 #define FS_MOST_SUMS (512LL << 18)       // floats at most of the segments' sums (512 MB): beyond, K stays whole
 #define FS_UP 0x1p24f                    // factor of both operands
 #define FS_DOWN 0x1p-48f
-#define FS_RAW_K 256                     // at most 32 aligned rows of a K below this are split where they are used
+#define FS_RAW_K 2048                    // at most 32 aligned rows of a K up to this are split where they are used (RAW)
+#define FS_RAW_GROUP 4                   // steps whose weights a wave asks for together
+#define FS_RAW_CHUNK 24                  // steps whose rows are in LDS at a time
 
 // two floats as two bfloat16, rounded to nearest even, and what is left of each
 __device__ __forceinline__ uint32_t fs_take(float& a, float& b) {
@@ -68,7 +70,13 @@ __device__ __forceinline__ uint32_t fs_take(float& a, float& b) {
     b -= __uint_as_float(p & 0xffff0000u);
     return p;
 }
-// eight floats times FS_UP as three times eight bfloat16
+// floats times FS_UP as three times as many bfloat16
+__device__ __forceinline__ void fs_split4(float4 x, uint2& hi, uint2& mid, uint2& lo) {
+    x.x *= FS_UP, x.y *= FS_UP, x.z *= FS_UP, x.w *= FS_UP;
+    hi = make_uint2(fs_take(x.x, x.y), fs_take(x.z, x.w));
+    mid = make_uint2(fs_take(x.x, x.y), fs_take(x.z, x.w));
+    lo = make_uint2(fs_take(x.x, x.y), fs_take(x.z, x.w));
+}
 __device__ __forceinline__ void fs_split8(float4 x, float4 y, uint4& hi, uint4& mid, uint4& lo) {
     x.x *= FS_UP, x.y *= FS_UP, x.z *= FS_UP, x.w *= FS_UP, y.x *= FS_UP, y.y *= FS_UP, y.z *= FS_UP, y.w *= FS_UP;
     hi = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
@@ -115,23 +123,31 @@ __device__ __forceinline__ void fs_load_to_lds(const void* g, void* lds_base) {
 // at most N of this wave's loads are still on their way, and its LDS reads are done
 #define FS_LANDED(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory")
 
+#define FS_MUL_ONE(ACC, A_, W_)                                                                                              \
+    ACC = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fs_bf16x8, A_), __builtin_bit_cast(fs_bf16x8, W_), ACC, 0, 0, 0);
+
 // MB blocks of 32 rows, FS_WAVES waves side by side with NB blocks of 32 columns each.  PARTS: blockIdx.y is a segment
 // of K and C the workspace [segments][M][N]; else the whole K, C holding the sum of the segments so far (a lane reads
 // and writes its own elements only).
 // Work-groups of one XCD (every eighth in the order of their ids) take the row tiles of one column tile in turn, so
 // that W is fetched into an L2 once and the rows are what its work-groups share at a time.
-// RAW (one block of rows, the rows 16-byte aligned, K a multiple of four and below FS_RAW_K): the rows come as they are, 2 KB
-// a step, and every wave splits them itself, so that a product of 17 to 32 rows is one launch.  17 rows of 1,152 x K, parts
-// beforehand and RAW, us: K = 64 6.6 and 5.2, 128 8.2 and 7.1, 256 11.2 and 11.1, 512 17.3 and 19.1 (a longer chain a step).
-// A row of a step, 64 bytes, has its unit u of 16 at u ^ (row / 4) % 4: sixteen rows' reads hit all banks.  Units past K
-// are the step's before, against zeros of the weight copy.
+// RAW (17 to 32 rows, 16-byte aligned, K a multiple of four and one segment): one launch, the rows split by the work-group that
+// uses them.  What bounds such a product is the chain of one element's products, six a step that wait for each other (0.25 us a
+// step with what lies between), and ahead of it a launch and two waits for memory.  So a wave's eight rows come by whole lines
+// of 128 bytes, a chunk of 24 steps at a time with the next one on its way, and go to LDS as parts once; the weights go from memory to
+// registers, three groups of four steps ahead, and the next step's are split between a step's products, where nothing else would
+// run; a barrier per chunk.  17 and 32 rows of 1,152 x K, us: parts beforehand / here / the float instruction: K = 64 7.2, 7.9 /
+// 5.3, 5.9 / 4.8, 5.1; 128 8.6, 9.4 / 6.2, 6.8 / 6.4, 6.7; 256 11.7, 12.4 / 8.1, 8.7 / 9.7, 10.1; 896 26, 27 / 18, 19 / 26, 27;
+// 2,048 52, 53 / 35, 36 / 56, 56.  (Waves that fetched and split 16 k at a time between barriers: 64 5.2, 128 7.1, 256 11.1; left to
+// the compiler, the splitting ran ahead of the products: 2,048 40.)
 template <int MB, int NB, int STAGES, bool PARTS, bool RAW>
 __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_kernel(
     const uint4* __restrict__ As, const float* __restrict__ A, const float* __restrict__ Ws, const float* __restrict__ bias,
     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int steps) {
     extern __shared__ uint4 fs_lds[];
-    static_assert(!RAW || (MB == 1 && !PARTS), "unsplit rows come in one block, with the whole of a short K");
-    constexpr int CHUNKS = RAW ? 2 : MB * 3, LA = (CHUNKS + FS_WAVES - 1) / FS_WAVES, LW = NB * 2, STAGE = (CHUNKS + FS_WAVES * LW) * 64;
+    static_assert(!RAW || (MB == 1 && NB == 1 && !PARTS), "unsplit rows come in one block, with the whole of a short K");
+    static_assert(FS_RAW_K <= FS_SEG && FS_RAW_CHUNK % (3 * FS_RAW_GROUP) == 0 && FS_RAW_CHUNK % 2 == 0, "RAW: one segment, whole turns of three groups");
+    constexpr int CHUNKS = MB * 3, LA = (CHUNKS + FS_WAVES - 1) / FS_WAVES, LW = NB * 2, STAGE = (CHUNKS + FS_WAVES * LW) * 64;
     constexpr int BN = FS_WAVES * NB * 32;
     const int blocks = (M + 31) / 32, mtiles = (blocks + MB - 1) / MB, ntiles = (N + BN - 1) / BN;
     const int local = blockIdx.x >> 3;
@@ -144,15 +160,10 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
 
     const uint4* ap[LA];
     const uint4* wp[LW];
-    const int unit = (lane & 3) ^ (lane >> 4);                          // RAW: the unit that this lane fetches
-    const bool past = RAW && (steps - 1) * FS_STEP + 4 * unit >= K;     // in the last step it is not there
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
         const int c = min(wave + i * FS_WAVES, CHUNKS - 1);            // a wave without a piece of its own repeats the last one
-        if (RAW)
-            ap[i] = reinterpret_cast<const uint4*>(A + (size_t)min(16 * c + (lane >> 2), M - 1) * lda + 4 * unit);   // K >= 16
-        else
-            ap[i] = As + ((size_t)min(b0 + c / 3, blocks - 1) * steps + first) * 192 + (c % 3) * 64 + lane;
+        ap[i] = As + ((size_t)min(b0 + c / 3, blocks - 1) * steps + first) * 192 + (c % 3) * 64 + lane;
     }
 #pragma unroll
     for (int j = 0; j < LW; ++j)
@@ -166,7 +177,7 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
         for (int j = 0; j < LW; ++j) fs_load_to_lds(wp[j], stage + (CHUNKS + wave * LW + j) * 64);
         if (++ahead < last) {
 #pragma unroll
-            for (int i = 0; i < LA; ++i) ap[i] += RAW ? (past && ahead == steps - 1 ? 0 : 4) : 192;
+            for (int i = 0; i < LA; ++i) ap[i] += 192;
 #pragma unroll
             for (int j = 0; j < LW; ++j) wp[j] += 64;
         }
@@ -186,6 +197,7 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
     const int row0 = b0 * 32 + 4 * (lane >> 5);
     auto store = [&](int s0, int s1) {       // the sums over steps [s0, s1), a segment
         const bool first_seg = s0 == 0, last_seg = s1 == steps;
+        const bool inside = RAW && M == MB * 32 && n0 + NB * 32 <= N;      // no element's place is looked at
         int row = row0, col = n0 + (lane & 31);
         asm volatile("" : "+v"(row), "+v"(col));       // addresses and bounds are made here, not kept through the loop over k
         uint32_t again[(MB * NB + 1) / 2];             // elements to compute again: sixteen bits per block
@@ -203,7 +215,7 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const float v = acc[i][j][4 * q + r] * FS_DOWN;
-                        if (n < N && row + i * 32 + 8 * q + r < M) {
+                        if (inside || (n < N && row + i * 32 + 8 * q + r < M)) {
                             const bool fine = fabsf(v) < INFINITY;         // else the sum so far stays where it is
                             again[(i * NB + j) / 2] |= fine ? 0u : 1u << (((i * NB + j) & 1) * 16 + 4 * q + r);
                             const float so_far = !PARTS && !first_seg ? o[r * ld] : 0.f;
@@ -253,6 +265,95 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
         }
     };
     clear();
+    if constexpr (RAW) {
+        const float4* wl = reinterpret_cast<const float4*>(Ws) + (size_t)min(n0 / 16 + (lane >> 4 & 1), (N + 15) / 16 - 1) * steps * 64 +
+                           (lane >> 5) * 32 + (lane & 15);
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 w[3][FS_RAW_GROUP][2];                                // three groups of steps on their way
+        auto ask = [&](float4 (&to)[FS_RAW_GROUP][2], int s) {       // a step past the last one: the last one again, not used
+            if (s >= steps) return;
+#pragma unroll
+            for (int u = 0; u < FS_RAW_GROUP; ++u) {
+                const size_t at = (size_t)min(s + u, steps - 1) * 64;
+                to[u][0] = wl[at];
+                to[u][1] = wl[at + 16];
+            }
+        };
+        // One step's products, each of which waits for the one before, and between them the splitting of the next step's weights.
+        uint4 x[3];
+        auto step = [&](const uint4* rows_of, const float4 (&next)[2]) {
+            uint4 a[3];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) a[p] = rows_of[p * 64];
+            float f[8] = {next[0].x, next[0].y, next[0].z, next[0].w, next[1].x, next[1].y, next[1].z, next[1].w};
+            uint32_t y[12];
+            auto take = [&](int t) { y[t] = fs_take(f[2 * (t & 3)], f[2 * (t & 3) + 1]); };
+#define FS_AMONG(PA, PW, ...)                   \
+    FS_MUL_ONE(acc[0][0], a[PA], x[PW])         \
+    __VA_ARGS__;                                \
+    __builtin_amdgcn_sched_barrier(0);
+            FS_AMONG(0, 2, _Pragma("unroll") for (int i = 0; i < 8; ++i) f[i] *= FS_UP; take(0))
+            FS_AMONG(2, 0, take(1); take(2))
+            FS_AMONG(1, 1, take(3); take(4))
+            FS_AMONG(0, 1, take(5); take(6))
+            FS_AMONG(1, 0, take(7); take(8))
+            FS_AMONG(0, 0, take(9); take(10); take(11))
+#undef FS_AMONG
+#pragma unroll
+            for (int p = 0; p < 3; ++p) x[p] = make_uint4(y[4 * p], y[4 * p + 1], y[4 * p + 2], y[4 * p + 3]);
+        };
+        auto multiply = [&](float4 (&from)[FS_RAW_GROUP][2], const float4 (&then)[FS_RAW_GROUP][2], int s, int c0) {
+            const uint4* rows_of = fs_lds + (s - c0) * 192 + lane;
+#pragma unroll
+            for (int u = 0; u < FS_RAW_GROUP; ++u)
+                if (s + u < steps) step(rows_of + u * 192, u + 1 < FS_RAW_GROUP ? from[u + 1 < FS_RAW_GROUP ? u + 1 : 0] : then[0]);
+            ask(from, s + 3 * FS_RAW_GROUP);
+        };
+        // Rows: a wave has eight of them, a lane 16 bytes of one in a line of 128 (two steps), so that no line is asked for twice.
+        constexpr int LINES = FS_RAW_CHUNK / 2;
+        const int row = wave * 8 + (lane >> 3), unit = 4 * (lane & 7);
+        const float* al = A + (size_t)min(row, M - 1) * lda;
+        uint2* part = reinterpret_cast<uint2*>(fs_lds) + ((lane >> 2 & 1) * 192 + (lane >> 1 & 1) * 32 + row) * 2 + (lane & 1);
+        float4 rows[LINES];
+        auto ask_rows = [&](int c0) {
+#pragma unroll
+            for (int i = 0; i < LINES; ++i)
+                if (c0 + 2 * i < steps) rows[i] = *reinterpret_cast<const float4*>(al + min((c0 + 2 * i) * FS_STEP + unit, K - 4));
+        };
+#pragma unroll
+        for (int i = 0; i < LINES; ++i) rows[i] = zero;
+        ask_rows(0);
+#pragma unroll
+        for (int g = 0; g < 3; ++g) {
+#pragma unroll
+            for (int u = 0; u < FS_RAW_GROUP; ++u) w[g][u][0] = w[g][u][1] = zero;
+            ask(w[g], g * FS_RAW_GROUP);
+        }
+        for (int c0 = 0; c0 < steps; c0 += FS_RAW_CHUNK) {
+            const int here = min(steps - c0, FS_RAW_CHUNK);
+            if (c0) __syncthreads();                     // every wave has read the rows before
+#pragma unroll
+            for (int i = 0; i < LINES; ++i)
+                if (2 * i < here) {
+                    uint2 hi, mid, lo;
+                    fs_split4((c0 + 2 * i) * FS_STEP + unit < K ? rows[i] : zero, hi, mid, lo);
+                    uint2* to = part + i * 768;
+                    to[0] = hi;
+                    to[128] = mid;
+                    to[256] = lo;
+                }
+            if (c0 + FS_RAW_CHUNK < steps) ask_rows(c0 + FS_RAW_CHUNK);
+            if (c0 == 0) fs_split8(w[0][0][0], w[0][0][1], x[0], x[1], x[2]);
+            __syncthreads();
+            for (int s = c0; s < c0 + here; s += 3 * FS_RAW_GROUP) {
+                multiply(w[0], w[1], s, c0);
+                if (s + FS_RAW_GROUP < c0 + here) multiply(w[1], w[2], s + FS_RAW_GROUP, c0);
+                if (s + 2 * FS_RAW_GROUP < c0 + here) multiply(w[2], w[0], s + 2 * FS_RAW_GROUP, c0);
+            }
+        }
+        store(0, steps);
+        return;
+    }
     for (int i = 0; i < STAGES - 1; ++i) fetch(i);
     int buf = 0;
     const int wfrag = (CHUNKS + wave * LW) * 64 + ((lane >> 4) & 1) * 64 + (lane >> 5) * 32 + (lane & 15);
@@ -275,14 +376,9 @@ __global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_ke
 #pragma unroll
             for (int b = 0; b < IB; ++b)
 #pragma unroll
-                for (int p = 0; p < 3 && !RAW; ++p) a[b][p] = stage[((i + b) * 3 + p) * 64 + lane];
-            if (RAW)
-                fs_split8(__builtin_bit_cast(float4, stage[(lane & 31) * 4 + ((lane >> 5) * 2 ^ (lane >> 2 & 3))]),
-                          __builtin_bit_cast(float4, stage[(lane & 31) * 4 + ((lane >> 5) * 2 + 1 ^ (lane >> 2 & 3))]), a[0][0], a[0][1], a[0][2]);
+                for (int p = 0; p < 3; ++p) a[b][p] = stage[((i + b) * 3 + p) * 64 + lane];
 #define FS_MUL(PA, PW)                                                                                                       \
-    _Pragma("unroll") for (int b = 0; b < IB; ++b) _Pragma("unroll") for (int j = 0; j < NB; ++j) acc[i + b][j] =              \
-        __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fs_bf16x8, a[b][PA]), __builtin_bit_cast(fs_bf16x8, w[j][PW]), \
-                                                acc[i + b][j], 0, 0, 0);
+    _Pragma("unroll") for (int b = 0; b < IB; ++b) _Pragma("unroll") for (int j = 0; j < NB; ++j) FS_MUL_ONE(acc[i + b][j], a[b][PA], w[j][PW])
             FS_MUL(0, 2)
             FS_MUL(2, 0)
             FS_MUL(1, 1)
@@ -362,9 +458,14 @@ extern "C" int tl_gemm_float_split_tile(int M, int N, int K) {
     return tile + (parts ? 4 : 0);
 }
 
-// Whether rows that start 16-byte aligned are split where they are used and need no workspace for their parts.
-extern "C" int tl_gemm_float_split_takes_rows(int M, int K, int lda) {
-    return M <= 32 && K >= FS_STEP && K < FS_RAW_K && K % 4 == 0 && lda % 4 == 0 ? 1 : 0;
+// Whether rows that start 16-byte aligned are split where they are used and need no workspace for their parts: where every
+// work-group of 128 columns has a CU of its own, and, for a K that leaves little else to do, where two share one (32 rows, us,
+// parts beforehand and not: 32,768 x 512 20.1 and 20.3, x 2,048 67 and 65; 37,888 x 128 10.6 and 9.9, x 160 11.7 and 11.9, x 512 21.6
+// and 22.3, where more columns' work-groups split the rows again than there are CUs).
+extern "C" int tl_gemm_float_split_takes_rows(int M, int N, int K, int lda) {
+    const int groups = tl_ceil_div(N, FS_WAVES * 32);
+    return M <= 32 && K >= FS_STEP && K <= FS_RAW_K && K % 4 == 0 && lda % 4 == 0 &&
+                   (groups <= FS_CUS || (K < 160 && groups <= 2 * FS_CUS)) ? 1 : 0;
 }
 
 // Floats of workspace that tl_gemm_float_split needs for the segments' sums (0: none).
@@ -393,27 +494,26 @@ extern "C" int tl_gemm_float_split(const float* A, const float* Ws, const float*
     TL_CHECK_ARG(grid < (1ll << 31), "tl_gemm_float_split: M=%d N=%d are too many tiles for one launch", M, N);
     TL_CHECK_ARG(!parts || ws, "tl_gemm_float_split: no workspace for the segments' sums");
     const int vec = ((uintptr_t)A % 16 == 0 && lda % 4 == 0) ? 1 : 0;
-    TL_CHECK_ARG(split || (tl_gemm_float_split_takes_rows(M, K, lda) && vec && tile == 3 && !parts),
+    TL_CHECK_ARG(split || (tl_gemm_float_split_takes_rows(M, N, K, lda) && vec && tile == 3 && !parts),
                  "tl_gemm_float_split: M=%d K=%d lda=%d need a workspace for the rows' parts", M, K, lda);
     if (split)
         hipLaunchKernelGGL(fs_split_kernel, dim3(tl_ceil_div(steps, 4), blocks), dim3(256), 0, stream, A, (uint4*)split, M, K, lda, steps, vec);
-#define FS_GO(MB, NB, ST, P, RAW)                                                                                                \
-    hipLaunchKernelGGL((fs_gemm_kernel<MB, NB, ST, P, RAW>), dim3((unsigned)grid, P ? nseg : 1), dim3(FS_WAVES * 64),            \
-                       ST * ((RAW ? 2 : MB * 3) + FS_WAVES * NB * 2) * 1024, stream, (const uint4*)split, A, Ws, bias, P ? ws : C, M, N, K, \
-                       lda, ldc, steps)
-#define FS_GO_P(MB, NB, ST, RAW)             \
-    if (parts) FS_GO(MB, NB, ST, true, RAW); \
-    else FS_GO(MB, NB, ST, false, RAW)
+#define FS_GO(MB, NB, ST, P, RAW, LDS)                                                                                           \
+    hipLaunchKernelGGL((fs_gemm_kernel<MB, NB, ST, P, RAW>), dim3((unsigned)grid, P ? nseg : 1), dim3(FS_WAVES * 64), LDS, stream, \
+                       (const uint4*)split, A, Ws, bias, P ? ws : C, M, N, K, lda, ldc, steps)
+#define FS_GO_P(MB, NB, ST)                                                               \
+    if (parts) FS_GO(MB, NB, ST, true, false, ST * (MB * 3 + FS_WAVES * NB * 2) * 1024); \
+    else FS_GO(MB, NB, ST, false, false, ST * (MB * 3 + FS_WAVES * NB * 2) * 1024)
     if (tile == 0) {
-        FS_GO_P(4, 2, 2, false);
+        FS_GO_P(4, 2, 2);
     } else if (tile == 1) {
-        FS_GO_P(4, 1, 3, false);
+        FS_GO_P(4, 1, 3);
     } else if (tile == 2) {
-        FS_GO_P(2, 1, 3, false);
+        FS_GO_P(2, 1, 3);
     } else if (split) {
-        FS_GO_P(1, 1, 3, false);
+        FS_GO_P(1, 1, 3);
     } else {
-        FS_GO(1, 1, 3, false, true);
+        FS_GO(1, 1, 1, false, true, (steps < FS_RAW_CHUNK ? (steps + 1) / 2 * 2 : FS_RAW_CHUNK) * 3072);
     }
 #undef FS_GO_P
 #undef FS_GO

@@ -612,12 +612,13 @@ def _float_split(a, shuffled, bias, out, M, N, K, lda, ldc):
     rows beyond 16, so that a row's bits do not depend on how many others come along.  Measured, us here and on the float
     instruction, N = 1,152: 33 rows K = 16 7.0 and 5.8, 64 8.2 and 8.2, 128 9.8 and 11.5, 896 28 and 51; 128 rows K = 16 6.9
     and 12.2, 64 8.3 and 16.5, 896 29 and 89; 1,000 rows of 9,728 K = 16 25 and 18, 64 31 and 30, 128 39 and 43, 896 130 and
-    204.  17 to 32 rows pay for the one order of summation from K = 64 to 896: 17 rows K = 64 5.7 and 4.8, 128 7.6 and 6.4, 256
-    12.1 and 9.7, 512 18.2 and 16.4, 896 27.2 and 26.3, 1,027 31 and 44, 4,864 54 and 147.  (Below K = 16 the float
+    204.  17 and 32 rows: K = 64 5.3, 5.9 and 4.8, 5.1, 100 6.1, 6.7 and 6.0, 6.3, 128 6.2, 6.8 and 6.4, 6.7, 256 8.1, 8.7 and 9.7,
+    10.1, 896 18, 19 and 26, 27, 2,048 35, 36 and 56, 56, 4,864 54 and 147: below K = 100 they pay up to a fifth for the one order of
+    summation.  (Below K = 16 the float
     instruction's error is the smaller one, too: gemm_float.hip.)"""
     most = max(128, FLOAT_SPLIT_BYTES // (-(-K // 16) * 96) // 128 * 128)
     split = ws = None
-    if M > 32 or a.data_ptr() % 16 or not library().tl_gemm_float_split_takes_rows(M, K, lda):
+    if M > 32 or a.data_ptr() % 16 or not library().tl_gemm_float_split_takes_rows(M, N, K, lda):
         split = torch.empty(-(-min(M, most) // 32) * -(-K // 16) * 1536, dtype=torch.int16, device=a.device)
     for r in range(0, M, most):
         m = min(M - r, most)

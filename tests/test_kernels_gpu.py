@@ -196,7 +196,8 @@ def test_linear_float_is_no_further_from_64_bits_than_the_float_instruction(Kd, 
         assert bool(((got.double() - want).abs() <= 2.0 ** -24 * want.abs()).all())
 
 
-@pytest.mark.parametrize("N,Kd", [(33, 64), (70, 68), (130, 76), (1000, 100), (257, 128), (40, 252), (1152, 256)])
+@pytest.mark.parametrize("N,Kd", [(33, 64), (70, 68), (130, 76), (1000, 100), (257, 128), (40, 252), (1152, 256),
+                                  (129, 384), (70, 388), (40, 772), (33, 1000), (300, 2044), (128, 2048), (32769, 64), (33000, 156)])
 @pytest.mark.parametrize("M", [17, 30, 32])
 def test_linear_float_of_at_most_32_rows_splits_them_where_they_are_used(M, N, Kd):
     """One launch for 17 to 32 aligned rows: the bits that the same rows get from parts made beforehand (rows that are not
@@ -213,6 +214,11 @@ def test_linear_float_of_at_most_32_rows_splits_them_where_they_are_used(M, N, K
     assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())
     assert torch.equal(K().linear(odd[:, 1:Kd + 1], w, b, shuffled=ws), got)
     assert torch.equal(K().linear(behind[:, :Kd], w, b, shuffled=ws)[:M], got)
+    # infinities, NaN and values past the split's range, in the rows and in the matrix
+    behind[3, Kd - 1], behind[16, 5], behind[9, Kd // 2], w[7, 2], w[N - 1, Kd - 2] = float("inf"), float("nan"), 2.0 ** 110, 2.0 ** 120, float("-inf")
+    odd[:, 1:Kd + 1] = a
+    ws = K().shuffle_weight_float(w)
+    torch.testing.assert_close(K().linear(a, w, b, shuffled=ws), K().linear(odd[:, 1:Kd + 1], w, b, shuffled=ws), rtol=0, atol=0, equal_nan=True)
 
 
 @pytest.mark.parametrize("M,N,Kd", [(40003, 40, 8200), (9000, 5000, 8200)])
