@@ -1328,7 +1328,7 @@ def test_attention_portions_in_runs_of_keys(nq, nkv, d, bs, lens, q_lens, kw, mo
 
 
 @pytest.mark.parametrize("M", [1, 5, 16])
-@pytest.mark.parametrize("N,Kd", [(784, 2048), (1000, 2056), (2048, 4864), (1030, 520), (896, 2336), (1030, 776)])
+@pytest.mark.parametrize("N,Kd", [(784, 2048), (1000, 2056), (2048, 4864), (1030, 520), (896, 2336), (1030, 776), (1030, 904)])
 def test_few_rows_in_half_tiles(M, N, Kd):
     """Few-row products whose work-groups own eight columns: an N that ends in either half of a tile, a last step with one
     chunk, a part of one, or only the first of a load's two; a residual sink and the product that reads its partial
