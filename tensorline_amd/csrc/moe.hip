@@ -778,9 +778,11 @@ extern "C" int tl_moe_gemm(const void* A, int a_dtype, int lda, const void* W, i
         return 0;
     }
     if (bf && K % 8 == 0 && lda % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0) {
-        // With tiles of 16 rows a matrix is read once a step: one that no cache holds until the next step streams 10% faster
-        // with loads that leave no trace there (64 experts of 4,096 x 2,048, 8 tokens: 326 against 363 us for both products), one
-        // that a cache does hold slower (8 experts of 512 x 96: gate and up 11 against 9 us).
+        // With tiles of 16 rows a matrix is read once a step: one that no cache holds until the next step streams faster with
+        // loads that leave no trace there (other experts with every call, both products, us: 64 of 4,096 x 2,048, 4 tokens of
+        // eight choices 278 -> 249, one of two 76 -> 72; 64 of 2,048 x 1,408 108 -> 97 and 48 -> 44; 16 of 2,048 x 1,024 54 -> 53 and
+        // 42 -> 41), one that a cache does hold slower (8 experts of 512 x 96: gate and up 9 -> 11).  From 96 MB on two layers' stacks
+        // are more than the last-level cache; a single layer called over and over pays (16 of 2,048 x 1,024, 16 tokens 40 -> 49).
         const bool once = BM == 16 && (double)experts * (glu == 1 ? 2 : 1) * N * K * 2.0 >= 96e6;
 #define GO_BF(MB, GLU)                                                                                                   \
     do {                                                                                                                 \
