@@ -374,11 +374,14 @@ static int pick_waves(int tiles, int nsc, int MT, int nacc, int max_waves, int s
 // and 16 rows, time of half tiles over whole ones: 49 to 128 tiles K = 640 1.07 to 0.96, 776 1.10 to 0.97 and 864 1.11 to 0.99 (two
 // waves with an uneven share), 896 0.95 to 0.88, 1,024 0.93 to 0.83, 1,056 1.04 to 0.97, 2,048 1.02 to 0.95, 4,096 1.02 to 0.94, 8,192 0.93 to 0.85; from 136 tiles on
 // (more than a half-tile group per CU) 1.04 to 1.46; 16 to 40 tiles 0.9 at K = 1,024 and 8,192 but up to 1.06 at 2,048, and left
-// whole.  With a residual sink only for a K that repays the next product's reading of twice as many partial sums.  By the matrix
-// and its use, not by the rows.
+// whole.  With a residual sink the next product reads twice as many partial sums, in every work-group: only for a K of more than
+// twice the columns, which ends a feed-forward and goes before a narrow q/k/v product, and not one that goes before a wide gate/up.  The two
+// products together, half over whole: 1,152 columns next, 96 tiles K = 2,304 0.96 to 0.93, 4,864 0.95 to 0.93, 56 tiles 1.00 to 0.98
+// and 0.96 (2,048 1.02 to 1.00); 9,728 columns next, 72 to 128 tiles K = 2,048 1.01 to 1.10, 4,864 1.00 to 1.07.  By the matrix and
+// its use, not by the rows.
 static int sk_split(int N, int K, bool sink) {
     const int tiles = tl_ceil_div(N, 16);
-    return tiles > 48 && tiles <= 128 && K >= (sink ? 2048 : 896) ? 2 : 1;
+    return tiles > 48 && tiles <= 128 && (sink ? K >= 2048 && K > 2 * N : K >= 896) ? 2 : 1;
 }
 
 template <int MT, int MODE, typename TO, int SPLIT>
