@@ -597,7 +597,8 @@ __global__ __launch_bounds__(MG_THREADS) void moe_gemm_bf16_kernel(const bf16_t*
 #define MGW_THREADS 256
 #define MGW_KT 64
 #define MGW_W 2048                       // 16-byte units of 256 matrix rows in a stage
-#define MGW_LDS (144 * 1024)
+#define MGW_W_STAGES 3
+#define MGW_LDS (160 * 1024)
 __device__ __forceinline__ uint32_t mgw_lds_address(void* p) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(p)); }
 // tl_load_to_lds for what is read once: it leaves no trace in the caches
 __device__ __forceinline__ void mgw_load_to_lds_once(const void* g, uint32_t lds_base) {
@@ -613,9 +614,9 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
                                          const int32_t* __restrict__ order, int place0, int rows, int n0, int top, int N, int K,
                                          float limit, float alpha, float shift, uint4* lds) {
     constexpr bool GLU = MODE == 1, BY_TOKEN = MODE != 0;
-    constexpr int LOADS = 2 * MW + 8;    // per wave and step: 8 rows each
-    constexpr int STAGES = MW <= 2 ? 3 : 2, STAGE = MGW_W + MW * 512;
-    static_assert(STAGES * STAGE * 16 <= MGW_LDS, "the stages do not fit");
+    constexpr int A_LOADS = 2 * MW, W_LOADS = 8;    // per wave and step: 8 rows each
+    constexpr int A_STAGES = MW <= 2 ? 3 : 2, STAGE_A = MW * 512;
+    static_assert((MGW_W_STAGES * MGW_W + A_STAGES * STAGE_A) * 16 <= MGW_LDS, "the stages do not fit");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1, c = lane & 15, g = lane >> 4;
 
@@ -634,18 +635,24 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
         wp[i] = We + ((size_t)(GLU && r >= 128 ? N : 0) + col) * K + 8 * ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4)));
     }
     const int nsteps = K / MGW_KT;
-    int ahead = 0;
-    auto fetch = [&](int buf) {
-        uint4* stage = lds + buf * STAGE;
+    uint4* lds_a = lds + MGW_W_STAGES * MGW_W;
+    int ahead_w = 0, ahead_a = 0;        // at the end the last step again, into a buffer that nobody reads
+    auto fetch_w = [&](int buf) {
+        uint4* stage = lds + buf * MGW_W;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) mgw_load_to_lds_once(wp[i], mgw_lds_address(stage + (wave * 8 + i) * 64));
+        for (int i = 0; i < W_LOADS; ++i) mgw_load_to_lds_once(wp[i], mgw_lds_address(stage + (wave * 8 + i) * 64));
+        if (++ahead_w < nsteps) {
 #pragma unroll
-        for (int i = 0; i < 2 * MW; ++i) tl_load_to_lds(ap[i], mgw_lds_address(stage + MGW_W + (wave * 2 * MW + i) * 64));
-        if (++ahead < nsteps) {          // at the end the last step again, into a buffer that nobody reads
+            for (int i = 0; i < W_LOADS; ++i) wp[i] += MGW_KT;
+        }
+    };
+    auto fetch_a = [&](int buf) {
+        uint4* stage = lds_a + buf * STAGE_A;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) wp[i] += MGW_KT;
+        for (int i = 0; i < A_LOADS; ++i) tl_load_to_lds(ap[i], mgw_lds_address(stage + (wave * 2 * MW + i) * 64));
+        if (++ahead_a < nsteps) {
 #pragma unroll
-            for (int i = 0; i < 2 * MW; ++i) ap[i] += MGW_KT;
+            for (int i = 0; i < A_LOADS; ++i) ap[i] += MGW_KT;
         }
     };
 
@@ -657,15 +664,20 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
 
     // blocks of sixteen columns: GLU the gate rows 64 wn + 16 j (j < 4) and the up rows behind 128; else 128 wn + 16 j
     const int frag = c * 8 + (g ^ (c >> 1));
-    const int wbase = (GLU ? wn * 64 : wn * 128) * 8 + frag, abase = MGW_W + wm * MW * 256 + frag;
-    for (int i = 0; i < STAGES - 1; ++i) fetch(i);
-    int buf = 0;
+    const int wbase = (GLU ? wn * 64 : wn * 128) * 8 + frag, abase = wm * MW * 256 + frag;
+    for (int i = 0; i < MGW_W_STAGES - 1; ++i) {     // rows before matrix rows, as in the loop: what may be on its way at a wait is the newest
+        if (i < A_STAGES - 1) fetch_a(i);
+        fetch_w(i);
+    }
+    int buf = 0, buf_a = 0;
     for (int s = 0; s < nsteps; ++s) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * LOADS) : "memory");    // step s is here, its reads of s - 1 done
+        // step s is here (on their way: the matrix rows of step s + 1, and its rows where they have three buffers), the reads of s - 1 are done
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(W_LOADS + (A_STAGES - 2) * A_LOADS) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        fetch(buf == 0 ? STAGES - 1 : buf - 1);      // the buffer of step s - 1
-        const uint4* stage = lds + buf * STAGE;
+        fetch_a(buf_a == 0 ? A_STAGES - 1 : buf_a - 1);          // the buffers of step s - 1
+        fetch_w(buf == 0 ? MGW_W_STAGES - 1 : buf - 1);
+        const uint4 *stage = lds + buf * MGW_W, *stage_a = lds_a + buf_a * STAGE_A;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {                // 32 k each: the other half of a row's units
             mg_bf16x8 w[8];
@@ -673,12 +685,13 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
             for (int j = 0; j < 8; ++j) w[j] = __builtin_bit_cast(mg_bf16x8, stage[(wbase ^ (4 * h)) + (GLU && j >= 4 ? 1024 + (j - 4) * 128 : j * 128)]);
 #pragma unroll
             for (int i = 0; i < 2 * MW; ++i) {
-                const mg_bf16x8 a = __builtin_bit_cast(mg_bf16x8, stage[(abase ^ (4 * h)) + i * 128]);
+                const mg_bf16x8 a = __builtin_bit_cast(mg_bf16x8, stage_a[(abase ^ (4 * h)) + i * 128]);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[j], acc[i][j], 0, 0, 0);
             }
         }
-        buf = buf == STAGES - 1 ? 0 : buf + 1;
+        buf = buf == MGW_W_STAGES - 1 ? 0 : buf + 1;
+        buf_a = buf_a == A_STAGES - 1 ? 0 : buf_a + 1;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may land in LDS that is no longer this work-group's
 
