@@ -671,6 +671,12 @@ def _library_linear(a, weight, bias, out_dtype, keep_shares: bool = False):
     M, K = a.shape
     N = weight.shape[0]
     tiles = -(-M // 256) * -(-N // 256)
+    if out_dtype == torch.float32 and _MM_OUT_DTYPE_OK is None:
+        try:
+            torch.mm(a[:1], wt[:, :16], out_dtype=torch.float32)
+            _MM_OUT_DTYPE_OK = True
+        except Exception:
+            _MM_OUT_DTYPE_OK = False
     if out_dtype == torch.float32 and _MM_OUT_DTYPE_OK and K >= 8192 and tiles < 200:
         # A long K with few output tiles leaves most of the 256 CUs idle in the library's product:
         # K is cut into 2, 4 or 8 shares run as one batched product, and the shares are added in order.
@@ -686,12 +692,6 @@ def _library_linear(a, weight, bias, out_dtype, keep_shares: bool = False):
                 y.add_(bias)
             return y
     if out_dtype == torch.float32:
-        if _MM_OUT_DTYPE_OK is None:
-            try:
-                torch.mm(a[:1], wt[:, :16], out_dtype=torch.float32)
-                _MM_OUT_DTYPE_OK = True
-            except Exception:
-                _MM_OUT_DTYPE_OK = False
         y = torch.mm(a, wt, out_dtype=torch.float32) if _MM_OUT_DTYPE_OK else torch.mm(a, wt).to(torch.float32)
         if bias is not None:
             y.add_(bias)
