@@ -1,0 +1,340 @@
+// bfloat16 products of more than 64 rows (prompts, portions, large decode batches): C = A W^T, W from its matrix-core ordered
+// copy (1 KB pieces: 16 columns x 32 k, lane 16 g + r holding column r at k = 8 g .. + 8), sums in float on
+// v_mfma_f32_16x16x32_bf16.
+//
+// What bounds it: at 2,048 rows the matrix cores at the clock this load runs at (products alone 1.5 to 1.7 PFLOP/s, with the
+// fragment reads 1.4 to 1.6, with the loads 1.2 to 1.4), at a few hundred rows the start and end of a work-group's walk and
+// how evenly the tiles fill the CUs.  A CU gets 100 to 130 bytes a ns from L2 or the last-level cache where loads never drain,
+// and 36 where each step's loads are waited for one step after they were asked for: so the next steps' tiles are on their way
+// across every barrier (two stages of LDS for A and three for W, or three each), and a barrier waits for the older ones only.
+//
+// WM x WN waves, each MB x NB blocks of 16 x 16, k in steps of 64 in two halves of 32.  The fragments of a half are read while
+// the other half is multiplied, a few in front of each row of products; the barrier lies in the middle of a step, between
+// the reads of its second half and those of the next step's first, and the loads of a later step follow it, spread over the
+// products too.  Eight waves hold 128 accumulators each at 256 x 256; four waves with 256 each took 1.6 times as long (the
+// compiler moves accumulators back and forth).  The rows of A (128 bytes a step) have their eight 16-byte units at
+// unit ^ (row / 2) % 8, so that the sixteen lanes that are served together hit all banks; W's pieces are read as they lie.
+// The operands are swapped (W's fragment first), so that a lane ends with four neighbouring columns of one row.
+//
+// Tiles are dealt to the XCDs in runs (work-group id modulo 8), rows fastest within panels of 2,048 rows: an XCD walks a few
+// tiles of W against all rows and its L2 holds both.
+//
+// K may be cut into shares (whole steps); the partial products go to a float workspace and are added in order, by whoever
+// takes them or by gt_add_kernel.
+//
+// us, here and in the library with its own choice of kernel (gate/up with the SiLU pass it needs; other weights at every call):
+// 2,048 rows of 37,888 x 3,584 gate/up 457 and 609, of 3,584 x 18,944 205 in two shares and 357, of 4,608 x 3,584 68 and 59;
+// 801 rows of 17,920 x 1,536 gate/up 55 and 66, of 1,536 x 8,960 28 and 44, of 2,048 x 1,536 11 and 19;
+// 200 rows of the same 24 and 32, 17 and 24, 8 and 22 to 53.
+#include "common.h"
+
+#include <math.h>
+
+typedef float gt_f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 gt_bf16x8 __attribute__((ext_vector_type(8)));
+#define GT_KT 64
+
+// 16 bytes a lane from sbase + voff into LDS at lds_base + 16 * lane
+__device__ __forceinline__ void gt_load(uint32_t voff, const void* sbase, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sbase) : "memory", "m0");
+}
+
+struct GtOut {
+    void* C;                   // [M, ldc], or shares x [M, N] float
+    int ldc;
+    const float* bias;         // [N] or null
+    int act;                   // plain: 1 the square of relu; gated: 0 SiLU, 2 the tanh form of GELU passes the gate
+};
+
+__device__ __forceinline__ float gt_gate(float v, int act) {
+    if (act == 2) return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
+    return v / (1.0f + expf(-v));
+}
+__device__ __forceinline__ void gt_store4(float* p, gt_f32x4 o) { *reinterpret_cast<gt_f32x4*>(p) = o; }
+__device__ __forceinline__ void gt_store4(bf16_t* p, gt_f32x4 o) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(tl_f2bf_bits(o[0]) | (uint32_t)tl_f2bf_bits(o[1]) << 16, tl_f2bf_bits(o[2]) | (uint32_t)tl_f2bf_bits(o[3]) << 16);
+}
+
+// GLU: W has the N / 2 gate rows, then the N / 2 up rows, and C = act(gate) * up [M, N / 2]; a wave's first NB / 2 blocks are gate
+// columns, the others the up columns of the same places.
+template <int WM, int WN, int MB, int NB, int AST, int BST, bool GLU, typename TO>
+__global__ __launch_bounds__(64 * WM * WN, MB * NB >= 16 ? 2 : 4) void gemm_tiles_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
+                                                                                  GtOut out, int M, int N, int K, int mtiles, int ntiles, int shares) {
+    constexpr int WAVES = WM * WN, BM = 16 * WM * MB, BN = 16 * WN * NB;
+    constexpr int A_UNITS = BM * 8, B_UNITS = BN * 8;                  // 16-byte units of a stage
+    constexpr int LA = BM / 8 / WAVES, LB = BN / 8 / WAVES;            // loads per wave and step
+    static_assert(LA * 8 * WAVES == BM && LB * 8 * WAVES == BN, "the loads of a step do not divide among the waves");
+    static_assert(AST == BST || (AST == 2 && BST == 3), "the waits know these stages");
+    constexpr int PANEL = 2048 / BM;
+    extern __shared__ uint4 gt_lds[];
+    uint4 *lds_a = gt_lds, *lds_b = gt_lds + AST * A_UNITS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave / WN, wn = wave % WN, c = lane & 15, g = lane >> 4;
+
+    const int plane = mtiles * ntiles, total = plane * shares, per = (total + 7) >> 3;
+    const int id = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (id >= total) return;                                           // (the grid is 8 * per)
+    const int share = id / plane, in = id - share * plane;
+    const int panel = in / (PANEL * ntiles), rows_of = min(PANEL, mtiles - panel * PANEL), q = in - panel * PANEL * ntiles;
+    const int nt = q / rows_of, m0 = (panel * PANEL + q % rows_of) * BM;
+    const int steps = K / GT_KT, s0 = (int)((long)steps * share / shares), nsteps = (int)((long)steps * (share + 1) / shares) - s0;
+    const int ctiles = (N + 15) >> 4, chunks = K >> 5, half = ctiles >> 1;
+    const int tile0 = nt * (GLU ? WN * NB / 2 : WN * NB);              // of 16 columns
+
+    // where this lane reads: rows and column tiles that the matrix does not have are its last one again
+    uint32_t aoff[LA], boff[LB];
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+        const int x = wave * LA + i, r = min(m0 + x * 8 + (lane >> 3), M - 1) - m0;
+        aoff[i] = (uint32_t)r * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ ((x & 1) * 4 + (lane >> 4)));
+    }
+#pragma unroll
+    for (int i = 0; i < LB; ++i) {
+        const int f = wave * LB + i, t = f >> 1, w = t / NB, j = t % NB;
+        const int tile = GLU ? min(tile0 + w * (NB / 2) + j % (NB / 2), half - 1) + (j >= NB / 2 ? half : 0) : min(tile0 + t, ctiles - 1);
+        boff[i] = ((uint32_t)(tile - tile0) * (uint32_t)chunks + (f & 1)) * 1024u + lane * 16u;
+    }
+    const char* ab = (const char*)(A + (size_t)m0 * lda + (size_t)s0 * GT_KT);
+    const char* bb = (const char*)W + ((size_t)tile0 * chunks + 2 * s0) * 1024;
+    const uint32_t la = (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(lds_a)) + wave * LA * 1024;
+    const uint32_t lb = (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(lds_b)) + wave * LB * 1024;
+    int na = 0, nb = 0;                                                // at the end the last step again, into a buffer that nobody reads
+    auto next_a = [&]() { if (++na < nsteps) ab += GT_KT * 2; };
+    auto next_b = [&]() { if (++nb < nsteps) bb += 2048; };
+    auto load_a = [&](int buf, int i) { gt_load(aoff[i], ab, la + buf * (A_UNITS * 16) + i * 1024); };
+    auto load_b = [&](int buf, int i) { gt_load(boff[i], bb, lb + buf * (B_UNITS * 16) + i * 1024); };
+    auto stage_a = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LA; ++i) load_a(buf, i);
+        next_a();
+    };
+    auto stage_b = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LB; ++i) load_b(buf, i);
+        next_b();
+    };
+
+    gt_f32x4 acc[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = (gt_f32x4){0.f, 0.f, 0.f, 0.f};
+    const int afrag = (wm * MB * 16 + c) * 8 + (g ^ (c >> 1)), bfrag = wn * NB * 128 + lane;
+    gt_bf16x8 a[2][MB], b[2][NB];
+    auto read_a = [&](int buf, int h, int i) { a[h][i] = __builtin_bit_cast(gt_bf16x8, lds_a[buf * A_UNITS + ((afrag + i * 128) ^ (4 * h))]); };
+    auto read_b = [&](int buf, int h, int j) { b[h][j] = __builtin_bit_cast(gt_bf16x8, lds_b[buf * B_UNITS + bfrag + j * 128 + h * 64]); };
+
+    if (AST == BST) {
+#pragma unroll
+        for (int i = 0; i < AST; ++i) { stage_a(i); stage_b(i); }
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AST - 1) * (LA + LB)) : "memory");
+    } else {
+        stage_a(0), stage_b(0), stage_b(1), stage_a(1), stage_b(2);    // in the order the waits below count in
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + 2 * LB) : "memory");
+    }
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < NB; ++j) read_b(0, 0, j);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) read_a(0, 0, i);
+    constexpr int RP = (2 * MB + NB - 1) / MB, LP = (LA + LB + MB - 1) / MB;      // reads and loads in front of a row of products
+    int bufa = 0, bufb = 0;
+    for (int s = 0; s < nsteps; ++s) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+            for (int x = i * RP; x < (i + 1) * RP; ++x) {
+                if (x < NB) read_b(bufb, 1, x);
+                else if (x < MB + NB) read_a(bufa, 1, x - NB);
+            }
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0][j], a[0][i], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const int nexta = bufa == AST - 1 ? 0 : bufa + 1, nextb = bufb == BST - 1 ? 0 : bufb + 1;
+        // step s + 1 is here (on their way: W of step s + 2, or all of the steps after s + 1); this wave's reads of step s are done
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AST == BST ? (AST - 2) * (LA + LB) : LB) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+            for (int x = i * RP; x < (i + 1) * RP; ++x) {
+                if (x < NB) read_b(nextb, 0, x);
+                else if (x < MB + NB) read_a(nexta, 0, x - NB);
+            }
+#pragma unroll
+            for (int x = i * LP; x < (i + 1) * LP; ++x) {              // into the buffers of step s
+                if (x < LA) load_a(bufa, x);
+                else if (x < LA + LB) load_b(bufb, x - LA);
+            }
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[1][j], a[1][i], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        next_a();
+        next_b();
+        bufa = nexta, bufb = nextb;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may land in LDS that is no longer this work-group's
+
+    // this lane holds row c and the columns 4 g .. 4 g + 3 of each block (N, or N / 2, is a multiple of 4 or of 16: whole quads)
+    TO* C = reinterpret_cast<TO*>(out.C);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+        const int m = m0 + (wm * MB + i) * 16 + c;
+        if (m >= M) continue;
+        TO* row = C + ((size_t)share * M + m) * out.ldc;
+        if (GLU) {
+#pragma unroll
+            for (int j = 0; j < NB / 2; ++j) {
+                const int n = (tile0 + wn * (NB / 2) + j) * 16 + 4 * g;
+                if (2 * n >= N) continue;
+                gt_f32x4 o;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[v] = gt_gate(acc[i][j][v], out.act) * acc[i][NB / 2 + j][v];
+                gt_store4(row + n, o);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                const int n = (tile0 + wn * NB + j) * 16 + 4 * g;
+                if (n >= N) continue;
+                gt_f32x4 o = acc[i][j];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    if (out.bias) o[v] += out.bias[n + v];
+                    if (out.act == 1) o[v] = fmaxf(o[v], 0.f) * fmaxf(o[v], 0.f);
+                }
+                gt_store4(row + n, o);
+            }
+        }
+    }
+}
+
+// The shares' sum in order, with what the product itself does to its result.  Bound by memory; four columns a thread.
+template <typename TO>
+__global__ __launch_bounds__(256) void gt_add_kernel(const float* __restrict__ parts, int shares, GtOut out, int M, int N) {
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, plane = (size_t)M * N;
+    if (i >= plane) return;
+    const int m = (int)(i / N), n = (int)(i - (size_t)m * N);
+    gt_f32x4 o = *reinterpret_cast<const gt_f32x4*>(parts + i);
+    for (int s = 1; s < shares; ++s) {
+        const gt_f32x4 p = *reinterpret_cast<const gt_f32x4*>(parts + s * plane + i);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[v] += p[v];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        if (out.bias) o[v] += out.bias[n + v];
+        if (out.act == 1) o[v] = fmaxf(o[v], 0.f) * fmaxf(o[v], 0.f);
+    }
+    gt_store4(reinterpret_cast<TO*>(out.C) + (size_t)m * out.ldc + n, o);
+}
+
+// ---- which tile ------------------------------------------------------------------------------------------------
+// The tiles, and what a step of 64 k takes a work-group: alone on its CU, beside a second one, and its start and end (us).  The
+// figures, and those of gt_time, are a fit to 24 matrices (896 x 896 to 37,888 x 3,584) at 65 to 2,048 rows in every tile and
+// 1 to 12 shares: half of the 3,600 times are within 5%, and the choice by them takes 1.4% longer than the best one in the mean
+// (0.79 of the library's time; at worst, 65 rows of 3,584 x 18,944, 41 us where the best takes 28 and the library 32).
+//    id  waves  blocks stages a CU holds  step alone, beside a second; start and end
+#define GT_TILES(X)                                  \
+    X(0, 2, 4, 8, 4, 2, 3, 1, 1.126, 1.126, 4.82)    \
+    X(1, 2, 4, 8, 3, 2, 3, 1, 0.842, 0.842, 4.70)    \
+    X(2, 2, 4, 4, 4, 3, 3, 1, 0.694, 0.694, 3.53)    \
+    X(3, 2, 4, 4, 2, 2, 3, 2, 0.489, 0.706, 1.89)    \
+    X(4, 2, 4, 2, 2, 3, 3, 2, 0.263, 0.487, 1.70)    \
+    X(5, 4, 2, 1, 2, 5, 5, 2, 0.187, 0.311, 1.50)    \
+    X(6, 2, 4, 6, 4, 2, 3, 1, 0.946, 0.946, 4.30)
+struct GtTile {
+    int bm, bn, lds, per_cu;
+    bool pairs;                // the gated form: whole blocks of gate and of up columns in a wave
+    double step1, step2, ends;
+};
+#define X(ID, WM, WN, MB, NB, AST, BST, CU, T1, T2, ENDS) \
+    {16 * WM * MB, 16 * WN * NB, (16 * WM * MB * AST + 16 * WN * NB * BST) * 128, CU, NB % 2 == 0, T1, T2, ENDS},
+static const GtTile gt_tiles[] = {GT_TILES(X)};
+#undef X
+#define GT_TILE_COUNT 7
+#define GT_MAX_SHARES 12
+
+static int gt_ntiles(const GtTile& t, int N, bool gated) { return gated ? tl_ceil_div(N / 2, t.bn / 2) : tl_ceil_div(N, t.bn); }
+
+// us of a product in tiles of t and `shares`: whole rounds of work-groups over the 256 CUs, or W from memory, or what the CUs
+// load, whichever is more; then the result's bytes, and the shares' second reading (by whoever takes them, or by a kernel)
+static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shares, bool takes_shares) {
+    const int mtiles = tl_ceil_div(M, t.bm);
+    const double groups = (double)mtiles * gt_ntiles(t, N, gated) * shares, slots = 256.0 * t.per_cu;
+    const double steps = tl_ceil_div(K / GT_KT, shares), full = floor(groups / slots), rest = groups - full * slots;
+    const double step1 = t.step1 * (1.0 + 0.074 / mtiles), step2 = t.per_cu == 1 ? step1 : t.step2 * (1.0 + 0.526 / mtiles);
+    double busy = full * (steps * step2 + t.ends);
+    if (rest > 0) busy += steps * (rest <= 256 ? step1 : step2) + t.ends;
+    const double weights = 0.213e-6 * 2.0 * N * K, loads = 0.053e-6 * groups * steps * (t.bm + t.bn) * 128.0;
+    const double plane = 4e-6 * (double)M * N;           // MB of float
+    double us = 2.3 + fmax(busy, fmax(weights, loads)) + 0.168 * (gated ? 0.25 : shares) * plane;
+    if (shares > 1) us += takes_shares ? 0.2 * (shares - 1) * plane : 2.7 + 0.13 * (shares + 1) * plane;
+    return us;
+}
+
+// The tile and the number of shares for a product (shares * 256 + tile), or -1: not one this file takes.
+extern "C" int tl_gemm_tiles_plan(int M, int N, int K, int gated, int takes_shares) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % GT_KT || N % (gated ? 32 : 4) || (double)N * K * 2.0 >= 4e9) return -1;
+    int best = -1;
+    double least = 0.0;
+    for (int i = 0; i < GT_TILE_COUNT; ++i) {
+        const GtTile& t = gt_tiles[i];
+        if (gated && !t.pairs) continue;
+        const double plane = (double)tl_ceil_div(M, t.bm) * gt_ntiles(t, N, gated);
+        for (int shares = 1; shares <= (gated ? 1 : GT_MAX_SHARES); ++shares) {
+            if (shares > 1 && (K / GT_KT / shares < 4 || plane * shares > 1.35 * 256 * t.per_cu)) break;
+            if (plane * shares >= 2e9) break;
+            const double us = gt_time(t, M, N, K, gated, shares, takes_shares);
+            if (best < 0 || us < least) best = shares * 256 + i, least = us;
+        }
+    }
+    return best;
+}
+
+// A [M, K] (row stride lda), W the matrix-core ordered copy of [N, K].  gated 0: C [M, N] (float or bfloat16) = act(A W^T + bias);
+// 1: C [M, N / 2] bfloat16 = act(gate) * up without bias.  shares > 1 (not gated): partial products into ws [shares, M, N] float,
+// added into C unless C is null.
+extern "C" int tl_gemm_tiles(const void* A, const void* W, const float* bias, void* C, int c_dtype, float* ws, int M, int N, int K, int lda, int ldc,
+                             int tile, int shares, int gated, int act, hipStream_t stream) {
+    TL_CHECK_ARG(M > 0 && N > 0 && K > 0 && K % GT_KT == 0 && N % (gated ? 32 : 4) == 0 && lda >= K && lda % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0,
+                 "tl_gemm_tiles: not sizes or an alignment this product takes: M=%d N=%d K=%d lda=%d", M, N, K, lda);
+    TL_CHECK_ARG(tile >= 0 && tile < GT_TILE_COUNT && shares >= 1 && shares <= GT_MAX_SHARES && shares <= K / GT_KT && (shares == 1 || (!gated && ws && (uintptr_t)ws % 16 == 0)) &&
+                     (C || shares > 1),
+                 "tl_gemm_tiles: tile %d in %d shares", tile, shares);
+    TL_CHECK_ARG((double)N * K * 2.0 < 4e9 && (double)lda * 512.0 < 4e9, "tl_gemm_tiles: N=%d K=%d lda=%d are beyond 32-bit offsets", N, K, lda);
+    TL_CHECK_ARG(!gated || (c_dtype == TL_BF16 && !bias && gt_tiles[tile].pairs), "tl_gemm_tiles: the gated form stores bfloat16, without bias, in tiles of whole pairs");
+    TL_CHECK_ARG((gated && (act == 0 || act == 2)) || (!gated && (act == 0 || act == 1)), "tl_gemm_tiles: activation %d is not one this product applies", act);
+    TL_CHECK_ARG(!C || (ldc >= (gated ? N / 2 : N) && ldc % 4 == 0 && (uintptr_t)C % (c_dtype == TL_F32 ? 16 : 8) == 0 && (c_dtype == TL_F32 || c_dtype == TL_BF16)),
+                 "tl_gemm_tiles: bad output");
+    const GtTile& t = gt_tiles[tile];
+    const int mtiles = tl_ceil_div(M, t.bm), ntiles = gt_ntiles(t, N, gated);
+    TL_CHECK_ARG((double)mtiles * ntiles * shares < 2e9, "tl_gemm_tiles: too many tiles");
+    const dim3 grid((unsigned)tl_ceil_div(mtiles * ntiles * shares, 8) * 8);
+    const GtOut direct = {C, ldc, bias, act}, partial = {ws, N, nullptr, 0};
+    const GtOut& o = shares > 1 ? partial : direct;
+#define GO(WM, WN, MB, NB, AST, BST, GLU, TO)                                                                                             \
+    hipLaunchKernelGGL((gemm_tiles_kernel<WM, WN, MB, NB, AST, BST, GLU, TO>), grid, dim3(64 * WM * WN), (size_t)t.lds, stream, (const bf16_t*)A, lda, \
+                       (const bf16_t*)W, o, M, N, K, mtiles, ntiles, shares)
+#define X(ID, WM, WN, MB, NB, AST, BST, CU, T1, T2, ENDS)                      \
+    case ID:                                                                   \
+        if (gated) GO(WM, WN, MB, (NB % 2 ? NB + 1 : NB), AST, BST, true, bf16_t); \
+        else if (shares > 1 || c_dtype == TL_F32) GO(WM, WN, MB, NB, AST, BST, false, float); \
+        else GO(WM, WN, MB, NB, AST, BST, false, bf16_t);                      \
+        break;
+    switch (tile) { GT_TILES(X) }
+#undef X
+#undef GO
+    TL_CHECK_LAUNCH("tl_gemm_tiles");
+    if (shares > 1 && C) {
+        const dim3 blocks((unsigned)(((size_t)M * N / 4 + 255) / 256));
+        if (c_dtype == TL_F32) hipLaunchKernelGGL(gt_add_kernel<float>, blocks, dim3(256), 0, stream, ws, shares, direct, M, N);
+        else hipLaunchKernelGGL(gt_add_kernel<bf16_t>, blocks, dim3(256), 0, stream, ws, shares, direct, M, N);
+        TL_CHECK_LAUNCH("tl_gemm_tiles (shares)");
+    }
+    return 0;
+}

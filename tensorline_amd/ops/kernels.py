@@ -525,6 +525,11 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
             _call("tl_gemm_skinny", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(res), _code(res, "linear output"), M, N, K, lda, N,
                   ctypes.byref(na), _stream())
             return res
+        if weight.dtype == torch.bfloat16 and a.dim() == 2 and a.stride(1) == 1 and weight.shape[1] == K:
+            plan = _tiles_plan(a, shuffled, M, weight.shape[0], K, lda)
+            if plan:
+                _on_gpu(a, weight, bias, shuffled)
+                return _tiles(a, shuffled, bias, out_dtype or a.dtype, M, weight.shape[0], K, lda, plan, act=1)
         return relu_squared(linear(a, weight, bias, out_dtype=torch.float32, shuffled=shuffled), out_dtype or a.dtype)
     owed = a if isinstance(a, NormedRows) else None
     if owed is not None:
@@ -561,6 +566,10 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
     if out is None:
         if a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and (
                 M > ROWS64_MAX_ROWS or (M > SKINNY_MAX_ROWS and shuffled is None)):
+            lda = a.stride(0) if M > 1 else K
+            plan = _tiles_plan(a, shuffled, M, N, K, lda, takes_shares=keep_shares and bias is None and out_dtype == torch.float32)
+            if plan:
+                return _tiles(a, shuffled, bias, out_dtype, M, N, K, lda, plan, keep_shares=keep_shares)
             return _library_linear(a, weight, bias, out_dtype, keep_shares)
         out = torch.empty(M, N, dtype=out_dtype, device=a.device)
     _check(out.dim() == 2 and tuple(out.shape) == (M, N) and out.stride(1) == 1 and out.dtype == out_dtype,
@@ -636,6 +645,27 @@ def _rows64(a, shuffled, bias, out, M, N, K, lda, ldc, swiglu: bool, norm=None):
     _call("tl_gemm_rows64", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), F32 if out is None else _code(out, "linear output"),
           _ptr(ws), M, N, K, lda, ldc, shares, 1 if swiglu else 0, norm, _stream())
     return out
+
+
+def _tiles_plan(a, shuffled, M, N, K, lda, gated: bool = False, takes_shares: bool = False) -> int:
+    """How a bfloat16 product of more than 64 rows is cut (tile and shares of K: gemm_tiles.hip), 0 where that kernel does not
+    take it (no matrix-core ordered copy, a K that is not a multiple of 64, unaligned rows)."""
+    if (shuffled is None or shuffled.dtype != torch.bfloat16 or a.dtype != torch.bfloat16 or M <= ROWS64_MAX_ROWS
+            or lda % 8 or lda < K or lda >= 1 << 22 or a.data_ptr() % 16):
+        return 0
+    return max(0, library().tl_gemm_tiles_plan(M, N, K, 1 if gated else 0, 1 if takes_shares else 0))
+
+
+def _tiles(a, shuffled, bias, out_dtype, M, N, K, lda, plan: int, keep_shares: bool = False, gated: bool = False, act: int = 0):
+    """The product as :func:`_tiles_plan` cut it; a :class:`ShareSum` where the caller keeps shares and there are any."""
+    _check_shuffled(shuffled, N, K)
+    tile, shares = plan & 255, plan >> 8
+    ws = torch.empty(shares, M, N, dtype=torch.float32, device=a.device) if shares > 1 else None
+    kept = shares > 1 and keep_shares and bias is None and out_dtype == torch.float32
+    out = None if kept else torch.empty(M, N // 2 if gated else N, dtype=out_dtype, device=a.device)
+    _call("tl_gemm_tiles", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), F32 if out is None else _code(out, "linear output"), _ptr(ws),
+          M, N, K, lda, N // 2 if gated else N, tile, shares, 1 if gated else 0, act, _stream())
+    return ShareSum(ws) if kept else out
 
 
 def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None) -> torch.Tensor:
@@ -785,6 +815,11 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
             na = _NormArgs()
             na.act = 2
             return _rows64(h, shuffled, None, out, M, 2 * I, K, lda, I, swiglu=True, norm=ctypes.byref(na))
+        if h.dim() == 2 and h.stride(1) == 1 and gate_up_weight.shape[1] == K:
+            plan = _tiles_plan(h, shuffled, M, 2 * I, K, lda, gated=True)
+            if plan:
+                _on_gpu(h, gate_up_weight, shuffled)
+                return _tiles(h, shuffled, None, h.dtype, M, 2 * I, K, lda, plan, gated=True, act=2)
         return glu(linear(h, gate_up_weight, shuffled=shuffled), activation, h.dtype)
     owed = h if isinstance(h, NormedRows) else None
     if owed is not None:
@@ -806,6 +841,10 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
         out = torch.empty(M, I, dtype=h.dtype, device=h.device)
         norm, _ = _norm_args(owed, None, M, 2 * I, h.device)
         return _rows64(h, shuffled, None, out, M, 2 * I, K, lda, I, swiglu=True, norm=norm)
+    if owed is None:
+        plan = _tiles_plan(h, shuffled, M, 2 * I, K, lda, gated=True)
+        if plan:
+            return _tiles(h, shuffled, None, h.dtype, M, 2 * I, K, lda, plan, gated=True)
     return silu_mul(linear(owed if owed is not None else h, gate_up_weight, shuffled=shuffled))
 
 

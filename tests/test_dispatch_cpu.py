@@ -101,3 +101,14 @@ def test_experts_in_wide_tiles_by_tiles_rows_and_size():
     assert not wide(188, 32, 1024, 512) and not wide(100, 8, 4096, 2048)            # fewer than two tiles per CU
     assert not wide(17, 256, 1024, 256) and not wide(32, 256, 512, 512) and not wide(48, 512, 512, 256)      # small, few rows
     assert wide(48, 256, 1024, 256) and wide(64, 256, 512, 512) and wide(64, 512, 512, 256)
+
+
+def test_many_row_products_are_cut_within_the_tiles_limits():
+    plan = K.library().tl_gemm_tiles_plan
+    for M, N, Kd in ((65, 64, 64), (2048, 37888, 3584), (801, 1536, 8960), (100000, 896, 896), (70, 512, 1 << 16)):
+        for gated, takes in ((0, 0), (0, 1), (1, 0)):
+            p = plan(M, N, Kd, gated, takes)
+            tile, shares = p & 255, p >> 8
+            assert 0 <= tile < 7 and 1 <= shares <= 12 and shares <= max(1, Kd // 256) and not (gated and (shares > 1 or tile == 1))
+    for M, N, Kd, gated in ((70, 64, 96, 0), (70, 66, 64, 0), (70, 48, 64, 1), (70, 1 << 17, 1 << 15, 0), (0, 64, 64, 0)):
+        assert plan(M, N, Kd, gated, 0) == -1

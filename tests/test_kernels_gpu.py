@@ -116,6 +116,56 @@ def test_linear_many_rows_keeps_its_shares_on_request():
     assert isinstance(small, torch.Tensor)
 
 
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("M,N,Kd,shares", [(65, 36, 64, 1), (257, 272, 128, 2), (129, 516, 320, 1), (200, 96, 832, 3), (1, 4, 192, 1), (193, 260, 1024, 4)])
+def test_many_row_product_in_every_tile(tile, M, N, Kd, shares):
+    """Every tile of the many-row product at the edges of tiles and panels, with one step of K and fewer steps than stages, in shares,
+    rows with a stride, columns that are no whole block; bias and activation behind the sum.  The products of bfloat16 numbers are
+    exact in float, so a sum of K of them is off by at most K 2^-24 of the sum of their sizes."""
+    torch.manual_seed(tile)
+    a = torch.randn(M, Kd + 24, device=DEV).to(torch.bfloat16)[:, :Kd]
+    w = (torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    bias = torch.randn(N, device=DEV)
+    sh = K().shuffle_weight(w)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    run = lambda b, dt, **kw: K()._tiles(a, sh, b, dt, M, N, Kd, a.stride(0), shares * 256 + tile, **kw)
+    err = (Kd + shares) * 2.0 ** -24 * size
+    assert bool(((run(None, torch.float32).double() - want).abs() <= err).all())
+    with_bias = want + bias.double()
+    assert bool(((run(bias, torch.float32).double() - with_bias).abs() <= err + 2.0 ** -24 * with_bias.abs()).all())
+    got, relu2 = run(bias, torch.bfloat16, act=1).double(), with_bias.clamp_min(0) ** 2      # (the square doubles what its argument is off by)
+    assert bool(((got - relu2).abs() <= 2.0 ** -8 * relu2 + 2.1 * with_bias.abs() * err + 1e-6).all())
+    kept = run(None, torch.float32, keep_shares=True)
+    if shares > 1:
+        assert isinstance(kept, K().ShareSum) and kept.parts.shape == (shares, M, N)
+        torch.testing.assert_close(kept.sum(), run(None, torch.float32), atol=0, rtol=0)
+    if tile == 1 or shares > 1:                                       # (a wave of that tile has three blocks of columns: no pairs)
+        return
+    for I in (16, 80):
+        w = (torch.randn(2 * I, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+        both = a.double() @ w.double().T
+        for act, fn in ((0, torch.nn.functional.silu), (2, lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+            got = K()._tiles(a, K().shuffle_weight(w), None, torch.bfloat16, M, 2 * I, Kd, a.stride(0), 256 + tile, gated=True, act=act)
+            want_g = fn(both[:, :I]) * both[:, I:]
+            torch.testing.assert_close(got.double(), want_g, rtol=2.0 ** -8, atol=1e-4)
+
+
+def test_many_row_product_by_its_rule():
+    """linear and swiglu_gate_up take the tiles the rule picks, for the library's own results: a product with its K in shares, one
+    without, and a K the tiles do not take."""
+    torch.manual_seed(5)
+    for M, N, Kd in ((2100, 256, 512), (70, 512, 9216), (130, 320, 96)):
+        a = torch.randn(M, Kd, device=DEV).to(torch.bfloat16)
+        w = (torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+        sh = K().shuffle_weight(w)
+        assert bool(K()._tiles_plan(a, sh, M, N, Kd, Kd)) == (Kd % 64 == 0)
+        want = a.double() @ w.double().T
+        torch.testing.assert_close(K().linear(a, w, None, out_dtype=torch.float32, shuffled=sh).double(), want, atol=1e-4, rtol=1e-4)
+        torch.testing.assert_close(K().linear(a, w, None, shuffled=sh).double(), want, atol=1e-4, rtol=2.0 ** -8)
+        silu = torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:]
+        torch.testing.assert_close(K().swiglu_gate_up(a, w, shuffled=sh).double(), silu, atol=2e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("M", [1, 7, 16])
 @pytest.mark.parametrize("N,Kd", [(1000, 1184), (3584, 18944), (50, 1030), (70, 513), (130, 7), (16, 512), (37, 40000)])
 def test_linear_few_rows_float32(M, N, Kd):
