@@ -236,17 +236,18 @@ __global__ __launch_bounds__(256) void gt_add_kernel(const float* __restrict__ p
 // ---- which tile ------------------------------------------------------------------------------------------------
 // The tiles, and what a step of 64 k takes a work-group: alone on its CU, beside a second one, and its start and end (us).  The
 // figures, and those of gt_time, are a fit to 24 matrices (896 x 896 to 37,888 x 3,584) at 65 to 2,048 rows in every tile and
-// 1 to 12 shares: half of the 3,600 times are within 5%, and the choice by them takes 1.4% longer than the best one in the mean
-// (0.79 of the library's time; at worst, 65 rows of 3,584 x 18,944, 41 us where the best takes 28 and the library 32).
+// 1 to 12 shares, with weights from memory (those that the last-level cache holds give other times and other choices): half of the
+// 3,600 times are within 5%, and the choice by them takes 0.8% longer than the best one in the mean (0.75 of the library's time; at
+// worst, 192 rows of 4,096 x 12,288, 38 us where the best takes 34 and the library 32).
 //    id  waves  blocks stages a CU holds  step alone, beside a second; start and end
 #define GT_TILES(X)                                  \
-    X(0, 2, 4, 8, 4, 2, 3, 1, 1.126, 1.126, 4.82)    \
-    X(1, 2, 4, 8, 3, 2, 3, 1, 0.842, 0.842, 4.70)    \
-    X(2, 2, 4, 4, 4, 3, 3, 1, 0.694, 0.694, 3.53)    \
-    X(3, 2, 4, 4, 2, 2, 3, 2, 0.489, 0.706, 1.89)    \
-    X(4, 2, 4, 2, 2, 3, 3, 2, 0.263, 0.487, 1.70)    \
-    X(5, 4, 2, 1, 2, 5, 5, 2, 0.187, 0.311, 1.50)    \
-    X(6, 2, 4, 6, 4, 2, 3, 1, 0.946, 0.946, 4.30)
+    X(0, 2, 4, 8, 4, 2, 3, 1, 1.072, 1.072, 4.22)    \
+    X(1, 2, 4, 8, 3, 2, 3, 1, 0.854, 0.854, 3.94)    \
+    X(2, 2, 4, 4, 4, 3, 3, 1, 0.735, 0.735, 3.29)    \
+    X(3, 2, 4, 4, 2, 2, 3, 2, 0.584, 0.785, 1.46)    \
+    X(4, 2, 4, 2, 2, 3, 3, 2, 0.407, 0.649, 0.95)    \
+    X(5, 4, 2, 1, 2, 5, 5, 2, 0.224, 0.406, 0.99)    \
+    X(6, 2, 4, 6, 4, 2, 3, 1, 0.931, 0.931, 3.72)
 struct GtTile {
     int bm, bn, lds, per_cu;
     bool pairs;                // the gated form: whole blocks of gate and of up columns in a wave
@@ -267,12 +268,12 @@ static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shar
     const int mtiles = tl_ceil_div(M, t.bm);
     const double groups = (double)mtiles * gt_ntiles(t, N, gated) * shares, slots = 256.0 * t.per_cu;
     const double steps = tl_ceil_div(K / GT_KT, shares), full = floor(groups / slots), rest = groups - full * slots;
-    const double step1 = t.step1 * (1.0 + 0.074 / mtiles), step2 = t.per_cu == 1 ? step1 : t.step2 * (1.0 + 0.526 / mtiles);
+    const double step1 = t.step1 * (1.0 + 0.243 / mtiles), step2 = t.per_cu == 1 ? step1 : t.step2 * (1.0 + 0.760 / mtiles);
     double busy = full * (steps * step2 + t.ends);
     if (rest > 0) busy += steps * (rest <= 256 ? step1 : step2) + t.ends;
-    const double weights = 0.213e-6 * 2.0 * N * K, loads = 0.053e-6 * groups * steps * (t.bm + t.bn) * 128.0;
+    const double weights = 0.233e-6 * 2.0 * N * K, loads = 0.060e-6 * groups * steps * (t.bm + t.bn) * 128.0;
     const double plane = 4e-6 * (double)M * N;           // MB of float
-    double us = 2.3 + fmax(busy, fmax(weights, loads)) + 0.168 * (gated ? 0.25 : shares) * plane;
+    double us = 3.4 + fmax(busy, fmax(weights, loads)) + 0.211 * (gated ? 0.25 : shares) * plane;
     if (shares > 1) us += takes_shares ? 0.2 * (shares - 1) * plane : 2.7 + 0.13 * (shares + 1) * plane;
     return us;
 }
