@@ -448,6 +448,12 @@ typedef __bf16 mg_bf16x8 __attribute__((ext_vector_type(8)));
 #define MGB_KT 64
 #define MGB_LD 72
 
+// Where the walk over k begins, in steps of 64: at another place for every expert and every 512 columns, and round.  Rows whose
+// stride is a power of two put the same k of all rows on few of the memory's channels, and work-groups that all begin at k = 0
+// read just those at any time (streaming 256 rows of 8 KB a work-group: 5.0 TB/s, begun at different places 6.9; rows of
+// 7 KB 6.9 either way).  The order of an element's sum depends on its expert and column and on K, and on nothing else.
+__device__ __forceinline__ int moe_first_step(int expert, int column, int nsteps) { return (4 * expert + (column >> 9)) % nsteps; }
+
 // ONCE: the matrices are read with non-temporal loads.
 template <int MB, int MODE, bool ONCE>
 __global__ __launch_bounds__(MG_THREADS) void moe_gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda,
@@ -524,23 +530,24 @@ __global__ __launch_bounds__(MG_THREADS) void moe_gemm_bf16_kernel(const bf16_t*
         }
     };
 
-    const int nsteps = (K + MGB_KT - 1) / MGB_KT;
-    fetch(0, areg[0], wreg[0]);
+    const int nsteps = (K + MGB_KT - 1) / MGB_KT, first = moe_first_step(e, n0, nsteps);
+    auto k_of = [&](int s) { return (s + first < nsteps ? s + first : s + first - nsteps) * MGB_KT; };
+    fetch(k_of(0), areg[0], wreg[0]);
     to_lds(0, areg[0], wreg[0]);
-    if (nsteps > 1) fetch(MGB_KT, areg[0], wreg[0]);
-    if (nsteps > 2) fetch(2 * MGB_KT, areg[1], wreg[1]);
+    if (nsteps > 1) fetch(k_of(1), areg[0], wreg[0]);
+    if (nsteps > 2) fetch(k_of(2), areg[1], wreg[1]);
     __syncthreads();
     // step s is in LDS buffer s % 2; set s % 2 holds step s + 1, the other set step s + 2
     for (int s = 0; s < nsteps; s += 2) {
         multiply(0);
         if (s + 1 < nsteps) {
             to_lds(1, areg[0], wreg[0]);
-            if (s + 3 < nsteps) fetch((s + 3) * MGB_KT, areg[0], wreg[0]);
+            if (s + 3 < nsteps) fetch(k_of(s + 3), areg[0], wreg[0]);
             __syncthreads();
             multiply(1);
             if (s + 2 < nsteps) {
                 to_lds(0, areg[1], wreg[1]);
-                if (s + 4 < nsteps) fetch((s + 4) * MGB_KT, areg[1], wreg[1]);
+                if (s + 4 < nsteps) fetch(k_of(s + 4), areg[1], wreg[1]);
                 __syncthreads();
             }
         }
@@ -611,7 +618,7 @@ __device__ __forceinline__ void mgw_load_to_lds_once(const void* g, uint32_t lds
 
 template <int MW, int MODE>
 __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ We, void* __restrict__ Cv, int ldc,
-                                         const int32_t* __restrict__ order, int place0, int rows, int n0, int top, int N, int K,
+                                         const int32_t* __restrict__ order, int place0, int rows, int expert, int n0, int top, int N, int K,
                                          float limit, float alpha, float shift, uint4* lds) {
     constexpr bool GLU = MODE == 1, BY_TOKEN = MODE != 0;
     constexpr int A_LOADS = 2 * MW, W_LOADS = 8;    // per wave and step: 8 rows each
@@ -620,21 +627,21 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1, c = lane & 15, g = lane >> 4;
 
+    const int nsteps = K / MGW_KT, first = moe_first_step(expert, n0, nsteps), k0 = first * MGW_KT;
     // where this lane reads its 16 bytes: row lane / 8 of the eight, unit (lane % 8) ^ (row / 2) % 8
     const bf16_t* ap[2 * MW];
     const bf16_t* wp[8];
 #pragma unroll
     for (int i = 0; i < 2 * MW; ++i) {
         const int r = min((wave * 2 * MW + i) * 8 + (lane >> 3), rows - 1);    // rows the tile does not have: its last one again
-        ap[i] = A + (size_t)(BY_TOKEN ? order[place0 + r] / top : place0 + r) * lda + 8 * ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4)));
+        ap[i] = A + k0 + (size_t)(BY_TOKEN ? order[place0 + r] / top : place0 + r) * lda + 8 * ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4)));
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int r = (wave * 8 + i) * 8 + (lane >> 3);
         const int col = min(GLU ? n0 + (r & 127) : n0 + r, N - 1);
-        wp[i] = We + ((size_t)(GLU && r >= 128 ? N : 0) + col) * K + 8 * ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4)));
+        wp[i] = We + k0 + ((size_t)(GLU && r >= 128 ? N : 0) + col) * K + 8 * ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4)));
     }
-    const int nsteps = K / MGW_KT;
     uint4* lds_a = lds + MGW_W_STAGES * MGW_W;
     int ahead_w = 0, ahead_a = 0;        // at the end the last step again, into a buffer that nobody reads
     auto fetch_w = [&](int buf) {
@@ -642,8 +649,9 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
 #pragma unroll
         for (int i = 0; i < W_LOADS; ++i) mgw_load_to_lds_once(wp[i], mgw_lds_address(stage + (wave * 8 + i) * 64));
         if (++ahead_w < nsteps) {
+            const int by = first + ahead_w == nsteps ? MGW_KT - K : MGW_KT;
 #pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) wp[i] += MGW_KT;
+            for (int i = 0; i < W_LOADS; ++i) wp[i] += by;
         }
     };
     auto fetch_a = [&](int buf) {
@@ -651,8 +659,9 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i) tl_load_to_lds(ap[i], mgw_lds_address(stage + (wave * 2 * MW + i) * 64));
         if (++ahead_a < nsteps) {
+            const int by = first + ahead_a == nsteps ? MGW_KT - K : MGW_KT;
 #pragma unroll
-            for (int i = 0; i < A_LOADS; ++i) ap[i] += MGW_KT;
+            for (int i = 0; i < A_LOADS; ++i) ap[i] += by;
         }
     };
 
@@ -741,7 +750,7 @@ __global__ __launch_bounds__(MGW_THREADS, 1) void moe_gemm_wide_kernel(const bf1
     const int e = tiles[1 + 3 * mt], place0 = tiles[2 + 3 * mt], rows = tiles[3 + 3 * mt];
     const bf16_t* We = W + (size_t)e * (MODE == 1 ? 2 : 1) * N * K;
     const int n0 = nt * (MODE == 1 ? 128 : 256);
-#define GO(MW) mgw_tile<MW, MODE>(A, lda, We, C, ldc, order, place0, rows, n0, top, N, K, limit, alpha, shift, mgw_lds)
+#define GO(MW) mgw_tile<MW, MODE>(A, lda, We, C, ldc, order, place0, rows, e, n0, top, N, K, limit, alpha, shift, mgw_lds)
     if (rows <= 64) GO(1);
     else if (rows <= 128) GO(2);
     else if (rows <= 192) GO(3);
