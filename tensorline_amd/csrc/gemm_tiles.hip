@@ -4,17 +4,11 @@
 //
 // What bounds it: at 2,048 rows the matrix cores at the clock this load runs at (products alone 1.5 to 1.7 PFLOP/s, with the
 // fragment reads 1.4 to 1.6, with the loads 1.2 to 1.4), at a few hundred rows the start and end of a work-group's walk and
-// how evenly the tiles fill the CUs.  A CU gets 100 to 130 bytes a ns from L2 or the last-level cache where loads never drain,
-// and 36 where each step's loads are waited for one step after they were asked for: so the next steps' tiles are on their way
-// across every barrier (two stages of LDS for A and three for W, or three each), and a barrier waits for the older ones only.
+// how evenly the tiles fill the CUs.  tile_walk.h has the walk over k and why its loads never drain.
 //
-// WM x WN waves, each MB x NB blocks of 16 x 16, k in steps of 64 in two halves of 32.  The fragments of a half are read while
-// the other half is multiplied, a few in front of each row of products; the barrier lies in the middle of a step, between
-// the reads of its second half and those of the next step's first, and the loads of a later step follow it, spread over the
-// products too.  Eight waves hold 128 accumulators each at 256 x 256; four waves with 256 each took 1.6 times as long (the
+// WM x WN waves.  Eight waves hold 128 accumulators each at 256 x 256; four waves with 256 each took 1.6 times as long (the
 // compiler moves accumulators back and forth).  The rows of A (128 bytes a step) have their eight 16-byte units at
 // unit ^ (row / 2) % 8, so that the sixteen lanes that are served together hit all banks; W's pieces are read as they lie.
-// The operands are swapped (W's fragment first), so that a lane ends with four neighbouring columns of one row.
 //
 // Tiles are dealt to the XCDs in runs (work-group id modulo 8), rows fastest within panels of 2,048 rows: an XCD walks a few
 // tiles of W against all rows and its L2 holds both.
@@ -26,18 +20,11 @@
 // 2,048 rows of 37,888 x 3,584 gate/up 457 and 609, of 3,584 x 18,944 205 in two shares and 357, of 4,608 x 3,584 68 and 59;
 // 801 rows of 17,920 x 1,536 gate/up 55 and 66, of 1,536 x 8,960 28 and 44, of 2,048 x 1,536 11 and 19;
 // 200 rows of the same 24 and 32, 17 and 24, 8 and 22 to 53.
-#include "common.h"
+#include "tile_walk.h"
 
 #include <math.h>
 
-typedef float gt_f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 gt_bf16x8 __attribute__((ext_vector_type(8)));
 #define GT_KT 64
-
-// 16 bytes a lane from sbase + voff into LDS at lds_base + 16 * lane
-__device__ __forceinline__ void gt_load(uint32_t voff, const void* sbase, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sbase) : "memory", "m0");
-}
 
 struct GtOut {
     void* C;                   // [M, ldc], or shares x [M, N] float
@@ -50,11 +37,6 @@ __device__ __forceinline__ float gt_gate(float v, int act) {
     if (act == 2) return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
     return v / (1.0f + expf(-v));
 }
-__device__ __forceinline__ void gt_store4(float* p, gt_f32x4 o) { *reinterpret_cast<gt_f32x4*>(p) = o; }
-__device__ __forceinline__ void gt_store4(bf16_t* p, gt_f32x4 o) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(tl_f2bf_bits(o[0]) | (uint32_t)tl_f2bf_bits(o[1]) << 16, tl_f2bf_bits(o[2]) | (uint32_t)tl_f2bf_bits(o[3]) << 16);
-}
-
 // GLU: W has the N / 2 gate rows, then the N / 2 up rows, and C = act(gate) * up [M, N / 2]; a wave's first NB / 2 blocks are gate
 // columns, the others the up columns of the same places.
 template <int WM, int WN, int MB, int NB, int AST, int BST, bool GLU, typename TO>
@@ -64,7 +46,6 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB >= 16 ? 2 : 4) void gemm_tile
     constexpr int A_UNITS = BM * 8, B_UNITS = BN * 8;                  // 16-byte units of a stage
     constexpr int LA = BM / 8 / WAVES, LB = BN / 8 / WAVES;            // loads per wave and step
     static_assert(LA * 8 * WAVES == BM && LB * 8 * WAVES == BN, "the loads of a step do not divide among the waves");
-    static_assert(AST == BST || (AST == 2 && BST == 3), "the waits know these stages");
     constexpr int PANEL = 2048 / BM;
     extern __shared__ uint4 gt_lds[];
     uint4 *lds_a = gt_lds, *lds_b = gt_lds + AST * A_UNITS;
@@ -98,86 +79,15 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB >= 16 ? 2 : 4) void gemm_tile
     const char* bb = (const char*)W + ((size_t)tile0 * chunks + 2 * s0) * 1024;
     const uint32_t la = (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(lds_a)) + wave * LA * 1024;
     const uint32_t lb = (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(lds_b)) + wave * LB * 1024;
-    int na = 0, nb = 0;                                                // at the end the last step again, into a buffer that nobody reads
-    auto next_a = [&]() { if (++na < nsteps) ab += GT_KT * 2; };
-    auto next_b = [&]() { if (++nb < nsteps) bb += 2048; };
-    auto load_a = [&](int buf, int i) { gt_load(aoff[i], ab, la + buf * (A_UNITS * 16) + i * 1024); };
-    auto load_b = [&](int buf, int i) { gt_load(boff[i], bb, lb + buf * (B_UNITS * 16) + i * 1024); };
-    auto stage_a = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < LA; ++i) load_a(buf, i);
-        next_a();
-    };
-    auto stage_b = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < LB; ++i) load_b(buf, i);
-        next_b();
-    };
-
-    gt_f32x4 acc[MB][NB];
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) acc[i][j] = (gt_f32x4){0.f, 0.f, 0.f, 0.f};
     const int afrag = (wm * MB * 16 + c) * 8 + (g ^ (c >> 1)), bfrag = wn * NB * 128 + lane;
-    gt_bf16x8 a[2][MB], b[2][NB];
-    auto read_a = [&](int buf, int h, int i) { a[h][i] = __builtin_bit_cast(gt_bf16x8, lds_a[buf * A_UNITS + ((afrag + i * 128) ^ (4 * h))]); };
-    auto read_b = [&](int buf, int h, int j) { b[h][j] = __builtin_bit_cast(gt_bf16x8, lds_b[buf * B_UNITS + bfrag + j * 128 + h * 64]); };
-
-    if (AST == BST) {
-#pragma unroll
-        for (int i = 0; i < AST; ++i) { stage_a(i); stage_b(i); }
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AST - 1) * (LA + LB)) : "memory");
-    } else {
-        stage_a(0), stage_b(0), stage_b(1), stage_a(1), stage_b(2);    // in the order the waits below count in
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + 2 * LB) : "memory");
-    }
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int j = 0; j < NB; ++j) read_b(0, 0, j);
-#pragma unroll
-    for (int i = 0; i < MB; ++i) read_a(0, 0, i);
-    constexpr int RP = (2 * MB + NB - 1) / MB, LP = (LA + LB + MB - 1) / MB;      // reads and loads in front of a row of products
-    int bufa = 0, bufb = 0;
-    for (int s = 0; s < nsteps; ++s) {
-#pragma unroll
-        for (int i = 0; i < MB; ++i) {
-#pragma unroll
-            for (int x = i * RP; x < (i + 1) * RP; ++x) {
-                if (x < NB) read_b(bufb, 1, x);
-                else if (x < MB + NB) read_a(bufa, 1, x - NB);
-            }
-#pragma unroll
-            for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0][j], a[0][i], acc[i][j], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        const int nexta = bufa == AST - 1 ? 0 : bufa + 1, nextb = bufb == BST - 1 ? 0 : bufb + 1;
-        // step s + 1 is here (on their way: W of step s + 2, or all of the steps after s + 1); this wave's reads of step s are done
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AST == BST ? (AST - 2) * (LA + LB) : LB) : "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int i = 0; i < MB; ++i) {
-#pragma unroll
-            for (int x = i * RP; x < (i + 1) * RP; ++x) {
-                if (x < NB) read_b(nextb, 0, x);
-                else if (x < MB + NB) read_a(nexta, 0, x - NB);
-            }
-#pragma unroll
-            for (int x = i * LP; x < (i + 1) * LP; ++x) {              // into the buffers of step s
-                if (x < LA) load_a(bufa, x);
-                else if (x < LA + LB) load_b(bufb, x - LA);
-            }
-#pragma unroll
-            for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[1][j], a[1][i], acc[i][j], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        next_a();
-        next_b();
-        bufa = nexta, bufb = nextb;
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may land in LDS that is no longer this work-group's
+    int na = 0, nb = 0;
+    tw_f32x4 acc[MB][NB];
+    tile_walk<MB, NB, AST, BST, LA, LB>(
+        nsteps, acc, [&](int buf, int i) { tw_load(aoff[i], ab, la + buf * (A_UNITS * 16) + i * 1024); },
+        [&](int buf, int i) { tw_load(boff[i], bb, lb + buf * (B_UNITS * 16) + i * 1024); }, [&]() { if (++na < nsteps) ab += GT_KT * 2; },
+        [&]() { if (++nb < nsteps) bb += 2048; },
+        [&](int buf, int h, int i) { return __builtin_bit_cast(tw_bf16x8, lds_a[buf * A_UNITS + ((afrag + i * 128) ^ (4 * h))]); },
+        [&](int buf, int h, int j) { return __builtin_bit_cast(tw_bf16x8, lds_b[buf * B_UNITS + bfrag + j * 128 + h * 64]); });
 
     // this lane holds row c and the columns 4 g .. 4 g + 3 of each block (N, or N / 2, is a multiple of 4 or of 16: whole quads)
     TO* C = reinterpret_cast<TO*>(out.C);
@@ -191,23 +101,23 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB >= 16 ? 2 : 4) void gemm_tile
             for (int j = 0; j < NB / 2; ++j) {
                 const int n = (tile0 + wn * (NB / 2) + j) * 16 + 4 * g;
                 if (2 * n >= N) continue;
-                gt_f32x4 o;
+                tw_f32x4 o;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) o[v] = gt_gate(acc[i][j][v], out.act) * acc[i][NB / 2 + j][v];
-                gt_store4(row + n, o);
+                tw_store4(row + n, o);
             }
         } else {
 #pragma unroll
             for (int j = 0; j < NB; ++j) {
                 const int n = (tile0 + wn * NB + j) * 16 + 4 * g;
                 if (n >= N) continue;
-                gt_f32x4 o = acc[i][j];
+                tw_f32x4 o = acc[i][j];
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     if (out.bias) o[v] += out.bias[n + v];
                     if (out.act == 1) o[v] = fmaxf(o[v], 0.f) * fmaxf(o[v], 0.f);
                 }
-                gt_store4(row + n, o);
+                tw_store4(row + n, o);
             }
         }
     }
@@ -219,9 +129,9 @@ __global__ __launch_bounds__(256) void gt_add_kernel(const float* __restrict__ p
     const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, plane = (size_t)M * N;
     if (i >= plane) return;
     const int m = (int)(i / N), n = (int)(i - (size_t)m * N);
-    gt_f32x4 o = *reinterpret_cast<const gt_f32x4*>(parts + i);
+    tw_f32x4 o = *reinterpret_cast<const tw_f32x4*>(parts + i);
     for (int s = 1; s < shares; ++s) {
-        const gt_f32x4 p = *reinterpret_cast<const gt_f32x4*>(parts + s * plane + i);
+        const tw_f32x4 p = *reinterpret_cast<const tw_f32x4*>(parts + s * plane + i);
 #pragma unroll
         for (int v = 0; v < 4; ++v) o[v] += p[v];
     }
@@ -230,7 +140,7 @@ __global__ __launch_bounds__(256) void gt_add_kernel(const float* __restrict__ p
         if (out.bias) o[v] += out.bias[n + v];
         if (out.act == 1) o[v] = fmaxf(o[v], 0.f) * fmaxf(o[v], 0.f);
     }
-    gt_store4(reinterpret_cast<TO*>(out.C) + (size_t)m * out.ldc + n, o);
+    tw_store4(reinterpret_cast<TO*>(out.C) + (size_t)m * out.ldc + n, o);
 }
 
 // ---- which tile ------------------------------------------------------------------------------------------------

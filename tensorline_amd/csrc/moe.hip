@@ -19,6 +19,7 @@
 // float matrix instruction (v_mfma_f32_16x16x4_f32), bfloat16 ones on v_mfma_f32_16x16x32_bf16, in tiles of 16, 64 or
 // up to 256 pair rows; bfloat16 shapes those do not take are widened on the way into LDS, as the any-shape product does.
 #include "common.h"
+#include "tile_walk.h"
 
 #include <math.h>
 
@@ -456,7 +457,7 @@ __device__ __forceinline__ int moe_first_step(int expert, int column, int nsteps
 
 // ONCE: the matrices are read with non-temporal loads.
 template <int MB, int MODE, bool ONCE>
-__global__ __launch_bounds__(MG_THREADS) void moe_gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda,
+__global__ __launch_bounds__(MG_THREADS, 2) void moe_gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda,
                                                                   const bf16_t* __restrict__ W, void* __restrict__ Cv, int ldc,
                                                                   const int32_t* __restrict__ order,
                                                                   const int32_t* __restrict__ tiles, int top, int N, int K,
@@ -590,157 +591,104 @@ __global__ __launch_bounds__(MG_THREADS) void moe_gemm_bf16_kernel(const bf16_t*
 // rows of its matrix (GLU: 128 gate rows and the 128 up rows of the same columns).  What bounds this product is what its
 // work-groups fetch: an expert's matrices are read from memory once whatever its rows (3.2 GB for 64 experts of 4,096 x
 // 2,048, 0.6 ms at a large copy's rate), and with tiles of 64 x 128 every byte of LDS filled serves 43 products where a
-// tile of 192 x 256 gets 110 out of it.  By the counters (requests of 128 bytes from L2, gate and up of 192 rows an expert) the
-// smaller tiles fetch 10.7 GB in 1.01 to 1.17 ms, 36 to 41 bytes a ns and CU, which is what L2 gives one; these 3.8 GB in 0.72,
-// 21 bytes a ns, behind one barrier a step.
+// tile of 192 x 256 gets 110 out of it: by the counters (requests of 128 bytes from L2, gate and up of 192 rows an expert) the
+// smaller tiles fetch 10.7 GB in 1.01 to 1.17 ms, these 3.8 GB in 0.43, of which 2.1 are the matrices from memory at 5.0 TB/s.
 //
-// Four waves, two by two: a wave has half of the tile's rows (32 MW of 64 MW) and 128 of its columns, so a fragment read
-// from LDS (1 KB) feeds 8 or 2 MW products.  k in steps of 64, whole lines of 128 bytes per row (steps of 32 fetched every line
-// twice), through two or three LDS stages filled by global_load_lds with no registers in between; one barrier a step.  The
-// eight units of 16 bytes of a row lie at unit ^ (row / 2) % 8, so that the sixteen lanes that are served at a time (rows
-// r .. r + 15, one unit) hit all banks.
+// Eight waves, two by four: a wave has half of the tile's rows (32 MW of 64 MW) and 64 of its columns; tile_walk.h has the walk
+// over k, in steps of 64: whole lines of 128 bytes per row (steps of 32 fetched every line twice).  The matrix rows have three
+// stages of LDS, the rows two or three.  The eight units of 16 bytes of a row lie at unit ^ (row / 2) % 8, so that the sixteen
+// lanes that are served at a time (rows r .. r + 15, one unit) hit all banks.  Four waves with whole steps of fragments ahead of
+// their products took 543 and 304 us for gate and up and for down of 192 rows an expert (64 of 4,096 x 2,048) where this takes 427
+// and 270 (5.0 and 4.0 TB/s of matrices).
 // MW is the tile's rows in sixties-fours, chosen by the work-group, so that a tile of 70 rows does the products of 128.
 // The tiles of one expert, all its column tiles, go to one XCD (every eighth work-group id), whose L2 then holds the rows.
-#define MGW_THREADS 256
+#define MGW_THREADS 512
 #define MGW_KT 64
 #define MGW_W 2048                       // 16-byte units of 256 matrix rows in a stage
 #define MGW_W_STAGES 3
 #define MGW_LDS (160 * 1024)
-__device__ __forceinline__ uint32_t mgw_lds_address(void* p) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(p)); }
-// tl_load_to_lds for what is read once: it leaves no trace in the caches
-__device__ __forceinline__ void mgw_load_to_lds_once(const void* g, uint32_t lds_base) {
-    uint32_t saved;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off nt\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved)
-                 : "s"(lds_base), "v"(g)
-                 : "memory");
-}
 
 template <int MW, int MODE>
 __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ We, void* __restrict__ Cv, int ldc,
                                          const int32_t* __restrict__ order, int place0, int rows, int expert, int n0, int top, int N, int K,
                                          float limit, float alpha, float shift, uint4* lds) {
     constexpr bool GLU = MODE == 1, BY_TOKEN = MODE != 0;
-    constexpr int A_LOADS = 2 * MW, W_LOADS = 8;    // per wave and step: 8 rows each
+    constexpr int MB = 2 * MW, NB = 4, LA = MW, LB = 4;                          // blocks of a wave; loads per wave and step, 8 rows each
     constexpr int A_STAGES = MW <= 2 ? 3 : 2, STAGE_A = MW * 512;
     static_assert((MGW_W_STAGES * MGW_W + A_STAGES * STAGE_A) * 16 <= MGW_LDS, "the stages do not fit");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave >> 1, wn = wave & 1, c = lane & 15, g = lane >> 4;
+    const int wm = wave >> 2, wn = wave & 3, c = lane & 15, g = lane >> 4;
 
-    const int nsteps = K / MGW_KT, first = moe_first_step(expert, n0, nsteps), k0 = first * MGW_KT;
-    // where this lane reads its 16 bytes: row lane / 8 of the eight, unit (lane % 8) ^ (row / 2) % 8
-    const bf16_t* ap[2 * MW];
-    const bf16_t* wp[8];
+    const int nsteps = K / MGW_KT, first = moe_first_step(expert, n0, nsteps);
+    // where this lane reads its 16 bytes, from A and from the expert's matrix on: row lane / 8 of the eight, unit (lane % 8) ^ (row / 2) % 8
+    uint32_t aoff[LA], woff[LB];
 #pragma unroll
-    for (int i = 0; i < 2 * MW; ++i) {
-        const int r = min((wave * 2 * MW + i) * 8 + (lane >> 3), rows - 1);    // rows the tile does not have: its last one again
-        ap[i] = A + k0 + (size_t)(BY_TOKEN ? order[place0 + r] / top : place0 + r) * lda + 8 * ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4)));
+    for (int i = 0; i < LA; ++i) {
+        const int x = wave * LA + i, r = min(x * 8 + (lane >> 3), rows - 1);     // rows the tile does not have: its last one again
+        aoff[i] = (uint32_t)(BY_TOKEN ? order[place0 + r] / top : place0 + r) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ ((x & 1) * 4 + (lane >> 4)));
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int r = (wave * 8 + i) * 8 + (lane >> 3);
-        const int col = min(GLU ? n0 + (r & 127) : n0 + r, N - 1);
-        wp[i] = We + k0 + ((size_t)(GLU && r >= 128 ? N : 0) + col) * K + 8 * ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4)));
+    for (int i = 0; i < LB; ++i) {
+        const int x = wave * LB + i, r = x * 8 + (lane >> 3), col = min(GLU ? n0 + (r & 127) : n0 + r, N - 1);
+        woff[i] = ((GLU && r >= 128 ? (uint32_t)N : 0u) + (uint32_t)col) * (uint32_t)K * 2u + 16u * ((lane & 7) ^ ((x & 1) * 4 + (lane >> 4)));
     }
     uint4* lds_a = lds + MGW_W_STAGES * MGW_W;
-    int ahead_w = 0, ahead_a = 0;        // at the end the last step again, into a buffer that nobody reads
-    auto fetch_w = [&](int buf) {
-        uint4* stage = lds + buf * MGW_W;
-#pragma unroll
-        for (int i = 0; i < W_LOADS; ++i) mgw_load_to_lds_once(wp[i], mgw_lds_address(stage + (wave * 8 + i) * 64));
-        if (++ahead_w < nsteps) {
-            const int by = first + ahead_w == nsteps ? MGW_KT - K : MGW_KT;
-#pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) wp[i] += by;
-        }
-    };
-    auto fetch_a = [&](int buf) {
-        uint4* stage = lds_a + buf * STAGE_A;
-#pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) tl_load_to_lds(ap[i], mgw_lds_address(stage + (wave * 2 * MW + i) * 64));
-        if (++ahead_a < nsteps) {
-            const int by = first + ahead_a == nsteps ? MGW_KT - K : MGW_KT;
-#pragma unroll
-            for (int i = 0; i < A_LOADS; ++i) ap[i] += by;
-        }
-    };
+    const uint32_t la = (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(lds_a)) + wave * LA * 1024;
+    const uint32_t lw = (uint32_t)__builtin_amdgcn_readfirstlane((int)tl_lds_address(lds)) + wave * LB * 1024;
+    const bf16_t *ap = A + first * MGW_KT, *wp = We + first * MGW_KT;
+    int na = 0, nw = 0;
+    auto by = [&](int n) { return first + n == nsteps ? MGW_KT - K : MGW_KT; };
+    // blocks of sixteen columns: GLU the gate rows 32 wn + 16 j (j < 2) and the up rows behind 128; else 64 wn + 16 j
+    const int frag = c * 8 + (g ^ (c >> 1)), wbase = (GLU ? wn * 32 : wn * 64) * 8 + frag, abase = wm * MB * 128 + frag;
+    tw_f32x4 acc[MB][NB];
+    tile_walk<MB, NB, A_STAGES, MGW_W_STAGES, LA, LB>(
+        nsteps, acc, [&](int buf, int i) { tw_load(aoff[i], ap, la + buf * (STAGE_A * 16) + i * 1024); },
+        [&](int buf, int i) { tw_load_once(woff[i], wp, lw + buf * (MGW_W * 16) + i * 1024); }, [&]() { if (++na < nsteps) ap += by(na); },
+        [&]() { if (++nw < nsteps) wp += by(nw); },
+        [&](int buf, int h, int i) { return __builtin_bit_cast(tw_bf16x8, lds_a[buf * STAGE_A + ((abase + i * 128) ^ (4 * h))]); },
+        [&](int buf, int h, int j) { return __builtin_bit_cast(tw_bf16x8, lds[buf * MGW_W + ((wbase + (GLU && j >= 2 ? 1024 + (j - 2) * 128 : j * 128)) ^ (4 * h))]); });
 
-    mg_f32x4 acc[2 * MW][8];
+    // this lane holds row c and the columns 4 g .. 4 g + 3 of each block (N is a multiple of 4)
 #pragma unroll
-    for (int i = 0; i < 2 * MW; ++i)
+    for (int i = 0; i < MB; ++i) {
+        const int r = (wm * MB + i) * 16 + c;
+        if (r >= rows) continue;
+        if (GLU) {
+            bf16_t* crow = reinterpret_cast<bf16_t*>(Cv) + (size_t)(place0 + r) * ldc;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = (mg_f32x4){0.f, 0.f, 0.f, 0.f};
-
-    // blocks of sixteen columns: GLU the gate rows 64 wn + 16 j (j < 4) and the up rows behind 128; else 128 wn + 16 j
-    const int frag = c * 8 + (g ^ (c >> 1));
-    const int wbase = (GLU ? wn * 64 : wn * 128) * 8 + frag, abase = wm * MW * 256 + frag;
-    for (int i = 0; i < MGW_W_STAGES - 1; ++i) {     // rows before matrix rows, as in the loop: what may be on its way at a wait is the newest
-        if (i < A_STAGES - 1) fetch_a(i);
-        fetch_w(i);
-    }
-    int buf = 0, buf_a = 0;
-    for (int s = 0; s < nsteps; ++s) {
-        // step s is here (on their way: the matrix rows of step s + 1, and its rows where they have three buffers), the reads of s - 1 are done
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(W_LOADS + (A_STAGES - 2) * A_LOADS) : "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        fetch_a(buf_a == 0 ? A_STAGES - 1 : buf_a - 1);          // the buffers of step s - 1
-        fetch_w(buf == 0 ? MGW_W_STAGES - 1 : buf - 1);
-        const uint4 *stage = lds + buf * MGW_W, *stage_a = lds_a + buf_a * STAGE_A;
+            for (int j = 0; j < 2; ++j) {
+                const int n = n0 + wn * 32 + j * 16 + 4 * g;
+                if (n >= N) continue;
+                tw_f32x4 o;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {                // 32 k each: the other half of a row's units
-            mg_bf16x8 w[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] = __builtin_bit_cast(mg_bf16x8, stage[(wbase ^ (4 * h)) + (GLU && j >= 4 ? 1024 + (j - 4) * 128 : j * 128)]);
-#pragma unroll
-            for (int i = 0; i < 2 * MW; ++i) {
-                const mg_bf16x8 a = __builtin_bit_cast(mg_bf16x8, stage_a[(abase ^ (4 * h)) + i * 128]);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[j], acc[i][j], 0, 0, 0);
-            }
-        }
-        buf = buf == MGW_W_STAGES - 1 ? 0 : buf + 1;
-        buf_a = buf_a == A_STAGES - 1 ? 0 : buf_a + 1;
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may land in LDS that is no longer this work-group's
-
-    // this lane holds rows 4 g + v and column c of each block
-#pragma unroll
-    for (int i = 0; i < 2 * MW; ++i)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r = wm * 32 * MW + i * 16 + 4 * g + v;
-            if (r >= rows) continue;
-            if (GLU) {
-                bf16_t* crow = reinterpret_cast<bf16_t*>(Cv) + (size_t)(place0 + r) * ldc;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int n = n0 + wn * 64 + j * 16 + c;
+                for (int v = 0; v < 4; ++v) {
                     const float gt = fminf(acc[i][j][v], limit);
-                    const float up = fminf(fmaxf(acc[i][4 + j][v], -limit), limit);
-                    if (n < N) crow[n] = tl_from_float<bf16_t>(gt * (1.0f / (1.0f + expf(-alpha * gt))) * (up + shift));
+                    const float up = fminf(fmaxf(acc[i][2 + j][v], -limit), limit);
+                    o[v] = gt * (1.0f / (1.0f + expf(-alpha * gt))) * (up + shift);
                 }
-            } else if (MODE == 2) {
-                bf16_t* crow = reinterpret_cast<bf16_t*>(Cv) + (size_t)(place0 + r) * ldc;
+                tw_store4(crow + n, o);
+            }
+        } else {
+            const size_t at = (size_t)(MODE == 2 ? place0 + r : order[place0 + r]) * ldc;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int n = n0 + wn * 128 + j * 16 + c;
-                    const float u = fmaxf(acc[i][j][v], 0.f);
-                    if (n < N) crow[n] = tl_from_float<bf16_t>(u * u);
-                }
-            } else {
-                float* crow = reinterpret_cast<float*>(Cv) + (size_t)order[place0 + r] * ldc;
+            for (int j = 0; j < 4; ++j) {
+                const int n = n0 + wn * 64 + j * 16 + 4 * g;
+                if (n >= N) continue;
+                if (MODE == 2) {
+                    tw_f32x4 o;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int n = n0 + wn * 128 + j * 16 + c;
-                    if (n < N) crow[n] = acc[i][j][v];
+                    for (int v = 0; v < 4; ++v) o[v] = fmaxf(acc[i][j][v], 0.f) * fmaxf(acc[i][j][v], 0.f);
+                    tw_store4(reinterpret_cast<bf16_t*>(Cv) + at + n, o);
+                } else {
+                    tw_store4(reinterpret_cast<float*>(Cv) + at + n, acc[i][j]);
                 }
             }
         }
+    }
 }
 
 template <int MODE>
-__global__ __launch_bounds__(MGW_THREADS, 1) void moe_gemm_wide_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
+__global__ __launch_bounds__(MGW_THREADS, 2) void moe_gemm_wide_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
                                                                        void* __restrict__ C, int ldc, const int32_t* __restrict__ order,
                                                                        const int32_t* __restrict__ tiles, int top, int N, int K,
                                                                        int ntiles, float limit, float alpha, float shift) {
@@ -786,8 +734,10 @@ extern "C" int tl_moe_gemm(const void* A, int a_dtype, int lda, const void* W, i
     } while (0)
     const bool bf = a_dtype == TL_BF16 && w_dtype == TL_BF16 && c_dtype == (glu ? TL_BF16 : TL_F32);
     if (BM == 256) {
-        TL_CHECK_ARG(bf && tl_moe_gemm_takes_wide(K) && lda % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0,
+        TL_CHECK_ARG(bf && tl_moe_gemm_takes_wide(K) && lda % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0,
                      "tl_moe_gemm: tiles of 256 rows are for aligned bfloat16 operands with K a multiple of %d, not K=%d", MGW_KT, K);
+        TL_CHECK_ARG(((double)max_tiles * 256.0 + 256.0) * lda * 2.0 < 4e9 && (glu == 1 ? 2.0 : 1.0) * N * K * 2.0 < 4e9,
+                     "tl_moe_gemm: tiles of 256 rows reach 4 GB of rows and of an expert's matrix");
         const int ntiles = tl_ceil_div(N, glu == 1 ? 128 : 256);
 #define GO_WIDE(MODE)                                                                                                      \
     hipLaunchKernelGGL(moe_gemm_wide_kernel<MODE>, dim3((unsigned)(tl_ceil_div(max_tiles, 8) * 8 * ntiles)), dim3(MGW_THREADS), \

@@ -1,0 +1,106 @@
+// The walk over k of a product whose operands' tiles go from memory straight into LDS (gemm_tiles.hip, moe.hip): bfloat16,
+// v_mfma_f32_16x16x32_bf16, k in steps of 64 in two halves of 32, for a work-group of waves that each hold MB x NB blocks of 16 x 16.
+//
+// AST and BST stages of LDS for the rows of A and of W (equal, or 2 and 3); a wave asks for LA and LB pieces of a step.  The
+// fragments of a half are read while the other half is multiplied, a few in front of each row of products.  The barrier lies in the
+// middle of a step, between the reads of its second half and those of the next step's first; the loads of a later step follow it
+// into the buffers of this one, spread over the products too.  A barrier waits for the next step's pieces only, the newer ones
+// stay on their way: a CU gets 100 to 130 bytes a ns from L2 or the last-level cache where loads never drain, and 36 where each
+// step's loads are waited for one step after they were asked for.
+//
+// load_a(buffer, i), load_b(buffer, i): ask for the i-th piece; next_a(), next_b(): go on to the next step (at the end the last step
+// again, into a buffer that nobody reads); read_a(buffer, half, i), read_b(buffer, half, j): a block's fragment.  W's fragment is the
+// first operand, so that lane 16 g + c ends with row c and the columns 4 g .. 4 g + 3 of each block.
+#pragma once
+#include "common.h"
+
+typedef float tw_f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 tw_bf16x8 __attribute__((ext_vector_type(8)));
+
+template <int MB, int NB, int AST, int BST, int LA, int LB, typename LoadA, typename LoadB, typename NextA, typename NextB, typename ReadA, typename ReadB>
+__device__ __forceinline__ void tile_walk(int nsteps, tw_f32x4 (&acc)[MB][NB], LoadA load_a, LoadB load_b, NextA next_a, NextB next_b,
+                                          ReadA read_a, ReadB read_b) {
+    static_assert(AST == BST || (AST == 2 && BST == 3), "the waits know these stages");
+    auto stage_a = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LA; ++i) load_a(buf, i);
+        next_a();
+    };
+    auto stage_b = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LB; ++i) load_b(buf, i);
+        next_b();
+    };
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = (tw_f32x4){0.f, 0.f, 0.f, 0.f};
+    tw_bf16x8 a[2][MB], b[2][NB];
+    if (AST == BST) {
+#pragma unroll
+        for (int i = 0; i < AST; ++i) { stage_a(i); stage_b(i); }
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AST - 1) * (LA + LB)) : "memory");
+    } else {
+        stage_a(0), stage_b(0), stage_b(1), stage_a(1), stage_b(2);    // in the order the waits below count in
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + 2 * LB) : "memory");
+    }
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < NB; ++j) b[0][j] = read_b(0, 0, j);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) a[0][i] = read_a(0, 0, i);
+    constexpr int RP = (2 * MB + NB - 1) / MB, LP = (LA + LB + MB - 1) / MB;      // reads and loads in front of a row of products
+    int bufa = 0, bufb = 0;
+    for (int s = 0; s < nsteps; ++s) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+            for (int x = i * RP; x < (i + 1) * RP; ++x) {
+                if (x < NB) b[1][x] = read_b(bufb, 1, x);
+                else if (x < MB + NB) a[1][x - NB] = read_a(bufa, 1, x - NB);
+            }
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0][j], a[0][i], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const int nexta = bufa == AST - 1 ? 0 : bufa + 1, nextb = bufb == BST - 1 ? 0 : bufb + 1;
+        // step s + 1 is here (on their way: W of step s + 2, or all of the steps after s + 1); this wave's reads of step s are done
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AST == BST ? (AST - 2) * (LA + LB) : LB) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+            for (int x = i * RP; x < (i + 1) * RP; ++x) {
+                if (x < NB) b[0][x] = read_b(nextb, 0, x);
+                else if (x < MB + NB) a[0][x - NB] = read_a(nexta, 0, x - NB);
+            }
+#pragma unroll
+            for (int x = i * LP; x < (i + 1) * LP; ++x) {              // into the buffers of step s
+                if (x < LA) load_a(bufa, x);
+                else if (x < LA + LB) load_b(bufb, x - LA);
+            }
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[1][j], a[1][i], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        next_a();
+        next_b();
+        bufa = nexta, bufb = nextb;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may land in LDS that is no longer this work-group's
+}
+
+// 16 bytes a lane from sbase + voff into LDS at lds_base + 16 * lane (lds_base is the same for the whole wave); tw_load_once: read
+// once, leaving no trace in the caches
+__device__ __forceinline__ void tw_load(uint32_t voff, const void* sbase, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sbase) : "memory", "m0");
+}
+__device__ __forceinline__ void tw_load_once(uint32_t voff, const void* sbase, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(voff), "s"(sbase) : "memory", "m0");
+}
+__device__ __forceinline__ void tw_store4(float* p, tw_f32x4 o) { *reinterpret_cast<tw_f32x4*>(p) = o; }
+__device__ __forceinline__ void tw_store4(bf16_t* p, tw_f32x4 o) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(tl_f2bf_bits(o[0]) | (uint32_t)tl_f2bf_bits(o[1]) << 16, tl_f2bf_bits(o[2]) | (uint32_t)tl_f2bf_bits(o[3]) << 16);
+}
