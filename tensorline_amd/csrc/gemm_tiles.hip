@@ -189,8 +189,15 @@ static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shar
 }
 
 // The tile and the number of shares for a product (shares * 256 + tile), or -1: not one this file takes.
+// More than 512 rows of a matrix that is large both ways stay in the library.  There it is level (us, library and here: 513 rows of
+// 4,608 x 3,584 29 and 30, 37,888 x 3,584 with SiLU 161 and 164; 2,048 rows 65 and 67, of 3,584 x 3,584 53 and 51, 3,584 x 18,944
+// 212 and 216, 4,096 x 12,288 153 and 152) but for gate and up of many rows (801 rows of 37,888 x 3,584 277 and 249, 2,048 549 and
+// 438), and another order of summation in a long prompt changes the tokens that are drawn after it: of 48 draws at top-p 0.9
+// behind 150 to 2,300 tokens 15 to 31% came out differently, with logits as far from 64 bits as before.  Fewer rows and smaller
+// matrices gain more: 128 rows of 4,608 x 3,584 20 and 12; 2,048 rows of 1,536 x 8,960 86 and 49, of gate and up 9,728 x 896 66 and 48.
 extern "C" int tl_gemm_tiles_plan(int M, int N, int K, int gated, int takes_shares) {
     if (M <= 0 || N <= 0 || K <= 0 || K % GT_KT || N % (gated ? 32 : 4) || (double)N * K * 2.0 >= 4e9) return -1;
+    if (M > 512 && N > 2048 && K > 2048) return -1;
     int best = -1;
     double least = 0.0;
     for (int i = 0; i < GT_TILE_COUNT; ++i) {

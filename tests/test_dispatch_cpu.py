@@ -105,10 +105,10 @@ def test_experts_in_wide_tiles_by_tiles_rows_and_size():
 
 def test_many_row_products_are_cut_within_the_tiles_limits():
     plan = K.library().tl_gemm_tiles_plan
-    for M, N, Kd in ((65, 64, 64), (2048, 37888, 3584), (801, 1536, 8960), (100000, 896, 896), (70, 512, 1 << 16)):
+    for M, N, Kd in ((65, 64, 64), (512, 37888, 3584), (801, 1536, 8960), (100000, 896, 896), (70, 512, 1 << 16), (2048, 2048, 6144)):
         for gated, takes in ((0, 0), (0, 1), (1, 0)):
             p = plan(M, N, Kd, gated, takes)
             tile, shares = p & 255, p >> 8
             assert 0 <= tile < 7 and 1 <= shares <= 12 and shares <= max(1, Kd // 256) and not (gated and (shares > 1 or tile == 1))
-    for M, N, Kd, gated in ((70, 64, 96, 0), (70, 66, 64, 0), (70, 48, 64, 1), (70, 1 << 17, 1 << 15, 0), (0, 64, 64, 0)):
+    for M, N, Kd, gated in ((70, 64, 96, 0), (70, 66, 64, 0), (70, 48, 64, 1), (70, 1 << 17, 1 << 15, 0), (0, 64, 64, 0), (513, 3584, 3584, 0)):
         assert plan(M, N, Kd, gated, 0) == -1
