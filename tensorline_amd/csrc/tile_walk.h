@@ -8,11 +8,13 @@
 // stay on their way: a CU gets 100 to 130 bytes a ns from L2 or the last-level cache where loads never drain, and 36 where each
 // step's loads are waited for one step after they were asked for.
 //
-// load_a(buffer, i), load_b(buffer, i): ask for the i-th piece; next_a(), next_b(): go on to the next step (at the end the last step
-// again, into a buffer that nobody reads); read_a(buffer, half, i), read_b(buffer, half, j): a block's fragment.  W's fragment is the
+// load_a(buffer, i), load_b(buffer, i): ask for the i-th piece; next_a(), next_b(): go on to the next step (where there are fewer
+// steps than stages, the last step stays); read_a(buffer, half, i), read_b(buffer, half, j): a block's fragment.  W's fragment is the
 // first operand, so that lane 16 g + c ends with row c and the columns 4 g .. 4 g + 3 of each block.
 #pragma once
 #include "common.h"
+
+#include <type_traits>
 
 typedef float tw_f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 tw_bf16x8 __attribute__((ext_vector_type(8)));
@@ -52,7 +54,8 @@ __device__ __forceinline__ void tile_walk(int nsteps, tw_f32x4 (&acc)[MB][NB], L
     for (int i = 0; i < MB; ++i) a[0][i] = read_a(0, 0, i);
     constexpr int RP = (2 * MB + NB - 1) / MB, LP = (LA + LB + MB - 1) / MB;      // reads and loads in front of a row of products
     int bufa = 0, bufb = 0;
-    for (int s = 0; s < nsteps; ++s) {
+    auto step = [&](int s, auto loads) {
+        constexpr bool LOADS = decltype(loads)::value;
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
 #pragma unroll
@@ -66,9 +69,11 @@ __device__ __forceinline__ void tile_walk(int nsteps, tw_f32x4 (&acc)[MB][NB], L
         }
         const int nexta = bufa == AST - 1 ? 0 : bufa + 1, nextb = bufb == BST - 1 ? 0 : bufb + 1;
         // step s + 1 is here (on their way: W of step s + 2, or all of the steps after s + 1); this wave's reads of step s are done
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AST == BST ? (AST - 2) * (LA + LB) : LB) : "memory");
+        if (LOADS || s + BST <= nsteps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AST == BST ? (AST - 2) * (LA + LB) : LB) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+        if (!LOADS && AST < BST && s + AST < nsteps) stage_a(bufa);    // the rows of the last step, where they have fewer stages
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
 #pragma unroll
@@ -76,19 +81,23 @@ __device__ __forceinline__ void tile_walk(int nsteps, tw_f32x4 (&acc)[MB][NB], L
                 if (x < NB) b[0][x] = read_b(nextb, 0, x);
                 else if (x < MB + NB) a[0][x - NB] = read_a(nexta, 0, x - NB);
             }
+            if (LOADS) {
 #pragma unroll
-            for (int x = i * LP; x < (i + 1) * LP; ++x) {              // into the buffers of step s
-                if (x < LA) load_a(bufa, x);
-                else if (x < LA + LB) load_b(bufb, x - LA);
+                for (int x = i * LP; x < (i + 1) * LP; ++x) {          // into the buffers of step s
+                    if (x < LA) load_a(bufa, x);
+                    else if (x < LA + LB) load_b(bufb, x - LA);
+                }
             }
 #pragma unroll
             for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[1][j], a[1][i], acc[i][j], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
-        next_a();
-        next_b();
+        if (LOADS) next_a(), next_b();
         bufa = nexta, bufb = nextb;
-    }
+    };
+    int s = 0;
+    for (; s + BST < nsteps; ++s) step(s, std::integral_constant<bool, true>());
+    for (; s < nsteps; ++s) step(s, std::integral_constant<bool, false>());       // all of W is on its way or here
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may land in LDS that is no longer this work-group's
 }
 
