@@ -243,8 +243,7 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
     const bool pages_in_lanes = npages <= 64;
     const int my_page = pages_in_lanes ? table[page_lo + (lane < npages ? lane : npages - 1)] : 0;
     const int krow_in_block0 = 8 * (c >> 2) + (c & 3);         // key of row c in tile 0; tile 1: + 4
-    // One block ahead: while block b is multiplied, the fragments of block b + 1 are in flight
-    // (past the last block the same block is requested again and not used).
+    // One block ahead: while block b is multiplied, the fragments of block b + 1 are in flight.
     uint4 kf0[DC], kf1[DC], vf[DB], kn0[DC], kn1[DC], vn[DB];
 #define AM_LOAD_BLOCK(B, K0, K1, V)                                                                          \
     {                                                                                                        \
@@ -272,14 +271,10 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
             V[db] = *reinterpret_cast<const uint4*>(vp_ + (size_t)db * 16 * bs);                             \
     }
     AM_LOAD_BLOCK(b_first, kf0, kf1, vf)
-    for (int i = 0; i < n_blocks; ++i) {
-        const int b = i < n_head ? ha + i : bb + (i - n_head);
-        const int kb = b << 5;
-        const int i_next = (i + 1 < n_blocks) ? i + 1 : i;
-        const int b_next = i_next < n_head ? ha + i_next : bb + (i_next - n_head);
-        // what the bias adds to this block's scores is asked for ahead of the next block's keys and values, so that
-        // waiting for it does not wait for those (nearly all of it comes from the nearest cache: a few rows of numbers)
-        float add[NT][8];
+    float add[NT][8];
+    // what the bias adds to a block's scores is asked for ahead of the next block's keys and values, so that
+    // waiting for it does not wait for those (nearly all of it comes from the nearest cache: a few rows of numbers)
+    auto load_bias = [&](int kb) {
         if (MODE == 2) {
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
@@ -288,6 +283,12 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
                 for (int x = 0; x < 8; ++x) add[j][x] = brow[tl_bias_at(p_col[j] - (kb + 8 * g + x), bias.reach)];
             }
         }
+    };
+    for (int i = 0; i + 1 < n_blocks; ++i) {
+        const int b = i < n_head ? ha + i : bb + (i - n_head);
+        const int kb = b << 5;
+        const int b_next = i + 1 < n_head ? ha + i + 1 : bb + (i + 1 - n_head);
+        load_bias(kb);
         AM_LOAD_BLOCK(b_next, kn0, kn1, vn)
 
         am_block<DC, NT, MODE>(kf0, kf1, vf, qf, p_col, lo_col, mask.first, kb, g, scale2, cap2, add, m_run, l_run, acc);
@@ -299,6 +300,9 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
 #pragma unroll
         for (int db = 0; db < DB; ++db) vf[db] = vn[db];
     }
+    // the last block asks for nothing: a split of a decode step has two to sixteen, and one asked for again is waited for
+    load_bias(b_last << 5);
+    am_block<DC, NT, MODE>(kf0, kf1, vf, qf, p_col, lo_col, mask.first, b_last << 5, g, scale2, cap2, add, m_run, l_run, acc);
 
 #undef AM_LOAD_BLOCK
     // ---- write: accumulator register i of lane (c, g) is (dim db*16 + 4g + i, column c) ----
