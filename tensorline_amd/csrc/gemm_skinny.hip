@@ -187,7 +187,7 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
             }
         wave_lds_order();
     };
-    auto multiply = [&](int sc) {
+    auto multiply = [&](int sc, const uint4 (&w)[4], const uint4 (&u)[4]) {
         // chunks past K32 of the last step read a clamped chunk: they must count as zero
         const int cbase = sc * 4 * SPLIT;
 #pragma unroll
@@ -200,17 +200,16 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
                     uint4 xf = xs[(mt * SPLIT * SK_UNITS + (cc * SPLIT + h) * 4 + g) * SK_ROWPAD + r];
                     if (!live) xf = zero;
                     f32x4& a = acc[h * NACC + mt];
-                    a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(wf[cc]), as_frag(xf), a, 0, 0, 0);
+                    a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(w[cc]), as_frag(xf), a, 0, 0, 0);
                     if (DUAL)
-                        acc[MT + mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(uf[cc]), as_frag(xf), acc[MT + mt], 0, 0, 0);
+                        acc[MT + mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(u[cc]), as_frag(xf), acc[MT + mt], 0, 0, 0);
                 }
             }
         }
         wave_lds_order();
     };
-    for (int sc = s0; sc + 1 < s1; ++sc) {
-        stage();
-        const int sn = sc + 1;                           // request the next step
+    // step sn's A rows (k past K zero when they are stored) and W fragments
+    auto request = [&](int sn, uint4 (&w)[4], uint4 (&u)[4]) {
 #pragma unroll
         for (int h = 0; h < SPLIT; ++h) {
             const int kxn = (sn * SPLIT + h) * SK_SC + xunit * 8;
@@ -222,27 +221,42 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
         for (int i = 0; i < 4; ++i) {
             int c = (sn * 4 + i) * SPLIT + sub;
             if (c > last_c) c = last_c;
-            wn[i] = tl_load_stream(w1 + (size_t)c * 64);
-            if (DUAL) un[i] = tl_load_stream(w2 + (size_t)c * 64);
+            w[i] = tl_load_stream(w1 + (size_t)c * 64);
+            if (DUAL) u[i] = tl_load_stream(w2 + (size_t)c * 64);
         }
-        multiply(sc);
+    };
+    auto clear_past = [&](int sn) {
 #pragma unroll
         for (int h = 0; h < SPLIT; ++h)
             if ((sn * SPLIT + h) * SK_SC + xunit * 8 >= K) {
 #pragma unroll
                 for (int i = 0; i < MT * 4; ++i) xr[h][i] = zero;
             }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            wf[i] = wn[i];
-            if (DUAL) uf[i] = un[i];
-        }
+    };
+    // two sets of W fragments in turn, so that nothing is moved between registers
+    int sc = s0;
+    for (; sc + 2 < s1; sc += 2) {
+        stage();
+        request(sc + 1, wn, un);
+        multiply(sc, wf, uf);
+        clear_past(sc + 1);
+        stage();
+        request(sc + 2, wf, uf);
+        multiply(sc + 1, wn, un);
+        clear_past(sc + 2);
     }
     // The last step asks for nothing: a wave of a narrow matrix has one to four steps, and a step asked for once more (to
     // keep the loop one body) was waited for at its end: a decode step of 28 layers of 3,584 at 8 rows 3,390 -> 3,242 us, of 24 layers of 896 at one 904 -> 877.
-    if (s0 < s1) {
+    if (sc + 1 < s1) {
         stage();
-        multiply(s1 - 1);
+        request(sc + 1, wn, un);
+        multiply(sc, wf, uf);
+        clear_past(sc + 1);
+        stage();
+        multiply(sc + 1, wn, un);
+    } else if (sc < s1) {
+        stage();
+        multiply(sc, wf, uf);
     }
 
     // Owed normalisation: thread (row, part) adds its partials in ascending order, then one thread
