@@ -189,9 +189,10 @@ __global__ __launch_bounds__(GG_THREADS) void gemm_generic_kernel(const TA* __re
 // of a 7B model: 224) has one work-group per CU, and what streams its weights is the loads that
 // group keeps in flight (eight waves: 2.5 TB/s for the float down projection, sixteen: 3.4), and how
 // evenly the segments deal out over the waves (74 segments of 256 over 16 waves: 5 at most, 4.6 on
-// average; 37 of 512: 3 against 2.3).  A deeper ring gains nothing (8 steps ahead: slower).
+// average; 37 of 512: 3 against 2.3).  A deeper ring pays only where nothing stands between its loads (GF_AHEAD).
 #define GF_SEG 256
 #define GF_RING 4
+#define GF_AHEAD 8
 #define GF_WAVES 16
 #define GF_MAX_SEGMENTS 128   // 128 KB of LDS for the segments' sums: K up to 32,768 (beyond: the kernel above)
 
@@ -252,30 +253,70 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_fewrows_kernel(const TA* _
     const int my_segs = (nseg - wave + nwaves - 1) / nwaves;   // 0 for a wave beyond the segments
     const int nsteps = my_segs * SPS;
     auto k_of = [&](int j) { return (wave + (j / SPS) * nwaves) * GF_SEG + (j % SPS) * GG_KS; };
-    float4 wreg[GF_RING], areg[GF_RING];
-#pragma unroll
-    for (int r = 0; r < GF_RING - 1; ++r) {
-        if (r < nsteps) load_step(k_of(r), wreg[r], areg[r]);
-    }
+    // as in the kernel above: the lane gives row li of A and row li of the W tile at k = k0 + 4 lg + v to the v-th product
+    // and holds C[4 lg + v][n0 + li]
     gg_f32x4 acc = (gg_f32x4){0.f, 0.f, 0.f, 0.f};
-    for (int jb = 0; jb < nsteps; jb += GF_RING) {
+    auto multiply = [&](const float4& av, const float4& wv) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, wv.x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, wv.y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av.z, wv.z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av.w, wv.w, acc, 0, 0, 0);
+    };
+    auto end_segment = [&](int j) {                               // step j was the segment's last one
+        const int seg = wave + (j / SPS) * nwaves;
 #pragma unroll
-        for (int r = 0; r < GF_RING; ++r) {
-            const int j = jb + r;
-            if (j < nsteps) {                                 // the same for the whole wave
-                const int ahead = j + GF_RING - 1;
-                if (ahead < nsteps) load_step(k_of(ahead), wreg[(r + GF_RING - 1) % GF_RING], areg[(r + GF_RING - 1) % GF_RING]);
-                // as in the kernel above: the lane gives row li of A and row li of the W tile at k = k0 + 4 lg + v
-                // to the v-th product and holds C[4 lg + v][n0 + li]
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(areg[r].x, wreg[r].x, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(areg[r].y, wreg[r].y, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(areg[r].z, wreg[r].z, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(areg[r].w, wreg[r].w, acc, 0, 0, 0);
-                if (j % SPS == SPS - 1) {                     // the segment is complete
-                    const int seg = wave + (j / SPS) * nwaves;
+        for (int v = 0; v < 4; ++v) gf_part[(seg * 4 + v) * 64 + lane] = acc[v];
+        acc = (gg_f32x4){0.f, 0.f, 0.f, 0.f};
+    };
+    if (SHUF && a_vec != 0 && K % GG_KS == 0) {
+        // Whole steps only, and of those that lie in K alone (a wave's first ones): the loop asks without a condition, so that
+        // the loads of GF_AHEAD steps stay on their way.  With conditions around them a product waited for nearly all that
+        // was on its way (8 rows, us: 37,888 x 3,584 108 -> 95, 152,064 x 3,584 387 -> 355, 3,584 x 18,944 68 -> 53).
+        static_assert(SPS % GF_AHEAD == 0, "segments end with a round of the ring");
+        const bool ends = (nseg - 1 - wave) % nwaves == 0;        // this wave has the last segment
+        const int mine = ends ? nsteps - SPS + (K - (nseg - 1) * GF_SEG) / GG_KS : nsteps;
+        float4 wr[GF_AHEAD], ar[GF_AHEAD];
+        auto ask = [&](int j, int r) {
+            const int k0 = k_of(j);
+            wr[r] = __builtin_bit_cast(float4, tl_load_stream(reinterpret_cast<const uint4*>(wtile + (size_t)(k0 / GG_KS) * 64)));
+            ar[r] = gg_load4_whole<TA>(arow_any + k0 + 4 * lg);
+        };
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) gf_part[(seg * 4 + v) * 64 + lane] = acc[v];
-                    acc = (gg_f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int r = 0; r < GF_AHEAD; ++r) ask(r < mine ? r : mine - 1, r);
+        int j = 0;
+        for (; j + 2 * GF_AHEAD <= mine; j += GF_AHEAD) {
+#pragma unroll
+            for (int r = 0; r < GF_AHEAD; ++r) {
+                multiply(ar[r], wr[r]);
+                __builtin_amdgcn_sched_barrier(0);
+                ask(j + r + GF_AHEAD, r);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if ((j + GF_AHEAD) % SPS == 0) end_segment(j + GF_AHEAD - 1);
+        }
+#pragma unroll
+        for (int r = 0; r < 2 * GF_AHEAD; ++r) {
+            const int t = j + r;
+            if (t >= mine) break;
+            multiply(ar[r % GF_AHEAD], wr[r % GF_AHEAD]);
+            if (t + GF_AHEAD < mine) ask(t + GF_AHEAD, r % GF_AHEAD);
+            if ((t + 1) % SPS == 0 || t + 1 == mine) end_segment(t);
+        }
+    } else {
+        float4 wreg[GF_RING], areg[GF_RING];
+#pragma unroll
+        for (int r = 0; r < GF_RING - 1; ++r) {
+            if (r < nsteps) load_step(k_of(r), wreg[r], areg[r]);
+        }
+        for (int jb = 0; jb < nsteps; jb += GF_RING) {
+#pragma unroll
+            for (int r = 0; r < GF_RING; ++r) {
+                const int j = jb + r;
+                if (j < nsteps) {                                 // the same for the whole wave
+                    const int ahead = j + GF_RING - 1;
+                    if (ahead < nsteps) load_step(k_of(ahead), wreg[(r + GF_RING - 1) % GF_RING], areg[(r + GF_RING - 1) % GF_RING]);
+                    multiply(areg[r], wreg[r]);
+                    if (j % SPS == SPS - 1) end_segment(j);
                 }
             }
         }
