@@ -671,7 +671,7 @@ def _tiles(a, shuffled, bias, out_dtype, M, N, K, lda, plan: int, keep_shares: b
 def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None) -> torch.Tensor:
     """bfloat16 with few rows: the streaming MFMA kernels.  float32 with the matrix-core ordered copy: the few-row kernel,
     or (more than 16 rows, a K of 64 or more) the float product on the bfloat16 instruction.  The rest: the plain tiled
-    kernel.  (bfloat16 with many rows went to the library before this, where the reference uses one too:
+    kernel.  (bfloat16 with many rows went to gemm_tiles.hip or the library before this; the reference uses a library:
     tensorline/paged.py:179-188.)"""
     if _skinny_ok(a, shuffled, M, K, lda) and not _few_rows_go_to_rows64(N, K):
         _call("tl_gemm_skinny", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), _code(out, "linear output"),
