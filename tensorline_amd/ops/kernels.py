@@ -1961,16 +1961,23 @@ MOE_WIDE_TILE = 256      # rows at most of a tile of the grouped bfloat16 produc
 
 def _moe_takes_wide_tiles(pairs: int, experts: int, ff: int, width: int) -> bool:
     """Whether the experts' products (ff x width) run in tiles of up to 256 rows by 256 matrix rows (a work-group of one per CU)
-    and not in tiles of 64 by 128.  They fetch each matrix once and the rows half as often, which pays where there are
-    twice as many tiles as CUs (64 experts of 4,096 x 2,048, both products: 18 rows per expert 647 against 693 us, 90: 754
-    against 932, 192: 1,066 against 1,475; of 2,048 x 1,408: 18 rows 239 against 246, 192: 433 against 616), and not where there
-    are fewer (32 experts of 1,024 x 512: 188 rows, with half a tile per CU, 101 against 75 us, 562 rows 183 against 169).
-    Small matrices for few rows stay in small tiles, whose start is cheaper: 256 experts of 1,024 x 256 17 rows 114 against 107,
-    32 130 against 121, 48 146 against 149; of 512 x 512 32 rows 132 against 119, 64 164 against 167; 512 of 512 x 256 48 rows 176
-    against 164, 64 199 against 203; 128 of 2,048 x 512 17 rows 200 against 207."""
+    and not in tiles of 64 by 128: where there are twice as many tiles as CUs and the matrices or the rows are not small.  They
+    fetch each matrix once and the rows half as often (64 experts of 4,096 x 2,048, both products and what goes ahead of them, us,
+    small and wide tiles: 18 rows per expert 592 and 530, 90: 909 and 588, 192: 1,449 and 739; of 2,048 x 1,408: 18 rows 217 and
+    191, 192: 615 and 303; 256 of 512 x 512 64 rows 153 and 120).  :func:`_moe_takes_wide_stack` adds what large stacks gain with
+    fewer tiles."""
     rows, size = -(-pairs // experts), ff * width
     return (experts * -(-rows // MOE_WIDE_TILE) * -(-ff // 128) >= 512
             and (rows >= 64 or size >= 1 << 20 or (rows >= 48 and size >= 1 << 18)))
+
+
+def _moe_takes_wide_stack(experts: int, ff: int, width: int) -> bool:
+    """The same for any number of tiles: where the stacked matrices are large, streaming them is what takes the time, and the wide
+    tiles do that faster even where they leave CUs without one (us, small and wide: 32 experts of 1,024 x 512 17 rows 39 and 36,
+    188: 80 and 63, 562: 182 and 132; 8 of 4,096 x 2,048 100 rows 134 and 114; 8 of 2,048 x 1,024 17 rows 52 and 45; 256 of
+    1,024 x 256 17 rows 107 and 96).  Below, their start costs more: 16 of 1,024 x 512 17 rows 32 and 30 but 100 38 and 40, 8 of
+    1,024 x 512 200 rows 35 and 54, 32 of 512 x 128 48 rows 23 and 25."""
+    return experts * ff * width >= 1 << 24
 
 
 def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
@@ -1996,7 +2003,7 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
         _f32(shared, "moe_experts shared", T * N)
     P = T * top
     BM = moe_tile_rows(P, E)
-    if (BM == 64 and _moe_takes_wide_tiles(P, E, F, K) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
+    if (BM == 64 and (_moe_takes_wide_tiles(P, E, F, K) or _moe_takes_wide_stack(E, F, K)) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
             and library().tl_moe_gemm_takes_wide(F) and (T == 1 or h.stride(0) % 8 == 0)
             and (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0
             and (P + 256 * (E + 2)) * max(h.stride(0), K, F) < 2e9 and F2 * K < 2e9 and N * F < 2e9):      # 32-bit offsets

@@ -112,3 +112,8 @@ def test_many_row_products_are_cut_within_the_tiles_limits():
             assert 0 <= tile < 7 and 1 <= shares <= 12 and shares <= max(1, Kd // 256) and not (gated and (shares > 1 or tile == 1))
     for M, N, Kd, gated in ((70, 64, 96, 0), (70, 66, 64, 0), (70, 48, 64, 1), (70, 1 << 17, 1 << 15, 0), (0, 64, 64, 0), (513, 3584, 3584, 0)):
         assert plan(M, N, Kd, gated, 0) == -1
+
+
+def test_large_stacks_of_experts_take_wide_tiles_whatever_their_number():
+    assert K._moe_takes_wide_stack(32, 512, 1024) and K._moe_takes_wide_stack(4, 1024, 4096) and K._moe_takes_wide_stack(256, 512, 512)
+    assert not K._moe_takes_wide_stack(16, 512, 1024) and not K._moe_takes_wide_stack(64, 128, 256)

@@ -1289,6 +1289,20 @@ def test_experts_in_wide_tiles(gated, Kd, F, N, monkeypatch):
         assert bool(((got[True][rows].double() - want[rows]).abs() <= slack).all()), e
 
 
+def test_a_large_stack_of_few_experts_takes_wide_tiles(monkeypatch):
+    """Four experts of 4,096 x 1,024 have 32 wide tiles for 256 CUs and take them for their size: bit for bit what small tiles give."""
+    torch.manual_seed(4)
+    T, E, Kd, F, top = 70, 4, 4096, 1024, 2
+    ids = torch.rand(T, E, device=DEV).topk(top, 1).indices.int().contiguous()
+    h, weights = torch.randn(T, Kd, device=DEV).to(torch.bfloat16), torch.rand(T, top, device=DEV)
+    up = (torch.randn(E, 2 * F, Kd, device=DEV) / 64).to(torch.bfloat16)
+    down = (torch.randn(E, Kd, F, device=DEV) / 32).to(torch.bfloat16)
+    assert K()._moe_takes_wide_stack(E, F, Kd) and not K()._moe_takes_wide_tiles(T * top, E, F, Kd)
+    wide = K().moe_experts(h, up, down, ids, weights, 7.0, 1.0)
+    monkeypatch.setattr(K(), "_moe_takes_wide_stack", lambda *a: False)
+    assert torch.equal(wide, K().moe_experts(h, up, down, ids, weights, 7.0, 1.0))
+
+
 @pytest.mark.parametrize("P,E,BM", [(1, 1, 16), (7, 3, 256), (1000, 70, 16), (5000, 64, 256), (12288, 64, 64), (9000, 200, 256), (3000, 1024, 16)])
 def test_pairs_in_tiles_by_expert(P, E, BM):
     """The order of the pairs and the tiles made of it: every pair once, in a tile of its expert, tiles within BM rows."""
