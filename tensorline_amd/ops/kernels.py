@@ -659,6 +659,9 @@ def _tiles_plan(a, shuffled, M, N, K, lda, gated: bool = False, takes_shares: bo
 def _tiles(a, shuffled, bias, out_dtype, M, N, K, lda, plan: int, keep_shares: bool = False, gated: bool = False, act: int = 0):
     """The product as :func:`_tiles_plan` cut it; a :class:`ShareSum` where the caller keeps shares and there are any."""
     _check_shuffled(shuffled, N, K)
+    if bias is not None:
+        if not (bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == N):
+            raise KernelError(f"linear: bias must be float32 of {N} entries")
     tile, shares = plan & 255, plan >> 8
     ws = torch.empty(shares, M, N, dtype=torch.float32, device=a.device) if shares > 1 else None
     kept = shares > 1 and keep_shares and bias is None and out_dtype == torch.float32

@@ -1,8 +1,21 @@
 """The host-side choices of kernels and launch shapes (tensorline_amd/ops/kernels.py): pure functions of
 the step's facts and the matrices' shapes, checked here without a GPU.  They decide speed, never a
 result beyond rounding; what they must keep is stated per test."""
+import pytest
+import torch
+
 from tensorline_amd.engine.batch import StepFacts
 from tensorline_amd.ops import kernels as K
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    """Every launch as (entry point, arguments) instead of on a GPU: operands may be CPU or meta tensors."""
+    calls = []
+    monkeypatch.setattr(K, "_on_gpu", lambda *t: None)
+    monkeypatch.setattr(K, "_stream", lambda: None)
+    monkeypatch.setattr(K, "_call", lambda name, *args: calls.append((name, args)))
+    return calls
 
 
 def test_key_splits_follow_the_batch_and_the_context_and_never_exceed_what_the_merge_takes():
@@ -117,3 +130,16 @@ def test_many_row_products_are_cut_within_the_tiles_limits():
 def test_large_stacks_of_experts_take_wide_tiles_whatever_their_number():
     assert K._moe_takes_wide_stack(32, 512, 1024) and K._moe_takes_wide_stack(4, 1024, 4096) and K._moe_takes_wide_stack(256, 512, 512)
     assert not K._moe_takes_wide_stack(16, 512, 1024) and not K._moe_takes_wide_stack(64, 128, 256)
+
+
+def test_a_many_row_product_with_an_activation_refuses_a_wrong_bias(launches):
+    """The product with relu squared in its epilogue takes the biases that the one without takes: float32, contiguous, N entries."""
+    a, w = torch.zeros(100, 256, dtype=torch.bfloat16), torch.zeros(512, 256, dtype=torch.bfloat16)
+    sh = K.shuffle_weight(w)
+    for bias in (torch.zeros(3), torch.zeros(512, dtype=torch.bfloat16), torch.zeros(1024)[::2], torch.zeros(513)):
+        for act in ("relu2", None):
+            with pytest.raises(K.KernelError, match="bias must be float32 of 512"):
+                K.linear(a, w, bias, shuffled=sh, act=act)
+    assert not launches
+    K.linear(a, w, torch.zeros(512), shuffled=sh, act="relu2")
+    assert [name for name, _ in launches] == ["tl_gemm_tiles"]
