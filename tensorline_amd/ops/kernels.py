@@ -525,7 +525,7 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
             _call("tl_gemm_skinny", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(res), _code(res, "linear output"), M, N, K, lda, N,
                   ctypes.byref(na), _stream())
             return res
-        if weight.dtype == torch.bfloat16 and a.dim() == 2 and a.stride(1) == 1 and weight.shape[1] == K:
+        if a.dim() == 2 and a.stride(1) == 1 and _bfloat16_matrix(weight, weight.shape[0], K):
             plan = _tiles_plan(a, shuffled, M, weight.shape[0], K, lda)
             if plan:
                 _on_gpu(a, weight, bias, shuffled)
@@ -568,7 +568,7 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
                 M > ROWS64_MAX_ROWS or (M > SKINNY_MAX_ROWS and shuffled is None)):
             lda = a.stride(0) if M > 1 else K
             plan = _tiles_plan(a, shuffled, M, N, K, lda, takes_shares=keep_shares and bias is None and out_dtype == torch.float32)
-            if plan:
+            if plan and out_dtype in _DTYPE_CODE:
                 return _tiles(a, shuffled, bias, out_dtype, M, N, K, lda, plan, keep_shares=keep_shares)
             return _library_linear(a, weight, bias, out_dtype, keep_shares)
         out = torch.empty(M, N, dtype=out_dtype, device=a.device)
@@ -647,11 +647,17 @@ def _rows64(a, shuffled, bias, out, M, N, K, lda, ldc, swiglu: bool, norm=None):
     return out
 
 
+def _bfloat16_matrix(weight: torch.Tensor, N: int, K: int) -> bool:
+    return weight.dtype == torch.bfloat16 and tuple(weight.shape) == (N, K) and weight.is_contiguous()
+
+
 def _tiles_plan(a, shuffled, M, N, K, lda, gated: bool = False, takes_shares: bool = False) -> int:
     """How a bfloat16 product of more than 64 rows is cut (tile and shares of K: gemm_tiles.hip), 0 where that kernel does not
-    take it (no matrix-core ordered copy, a K that is not a multiple of 64, unaligned rows)."""
+    take it (no matrix-core ordered copy of an [N, K] matrix, a K that is not a multiple of 64, unaligned rows).  The callers ask
+    for matrices that the other ways take too (:func:`_bfloat16_matrix`): what those refuse is left to them."""
     if (shuffled is None or shuffled.dtype != torch.bfloat16 or a.dtype != torch.bfloat16 or M <= ROWS64_MAX_ROWS
-            or lda % 8 or lda < K or lda >= 1 << 22 or a.data_ptr() % 16):
+            or lda % 8 or lda < K or lda >= 1 << 22 or a.data_ptr() % 16
+            or tuple(shuffled.shape) != (-(-N // 16), -(-K // 32), 4, 16, 8) or not shuffled.is_contiguous()):
         return 0
     return max(0, library().tl_gemm_tiles_plan(M, N, K, 1 if gated else 0, 1 if takes_shares else 0))
 
@@ -818,7 +824,7 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
             na = _NormArgs()
             na.act = 2
             return _rows64(h, shuffled, None, out, M, 2 * I, K, lda, I, swiglu=True, norm=ctypes.byref(na))
-        if h.dim() == 2 and h.stride(1) == 1 and gate_up_weight.shape[1] == K:
+        if h.dim() == 2 and h.stride(1) == 1 and _bfloat16_matrix(gate_up_weight, 2 * I, K):
             plan = _tiles_plan(h, shuffled, M, 2 * I, K, lda, gated=True)
             if plan:
                 _on_gpu(h, gate_up_weight, shuffled)
@@ -844,7 +850,7 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
         out = torch.empty(M, I, dtype=h.dtype, device=h.device)
         norm, _ = _norm_args(owed, None, M, 2 * I, h.device)
         return _rows64(h, shuffled, None, out, M, 2 * I, K, lda, I, swiglu=True, norm=norm)
-    if owed is None:
+    if owed is None and _bfloat16_matrix(gate_up_weight, 2 * I, K):
         plan = _tiles_plan(h, shuffled, M, 2 * I, K, lda, gated=True)
         if plan:
             return _tiles(h, shuffled, None, h.dtype, M, 2 * I, K, lda, plan, gated=True)

@@ -143,3 +143,31 @@ def test_a_many_row_product_with_an_activation_refuses_a_wrong_bias(launches):
     assert not launches
     K.linear(a, w, torch.zeros(512), shuffled=sh, act="relu2")
     assert [name for name, _ in launches] == ["tl_gemm_tiles"]
+
+
+def test_many_row_products_take_and_refuse_the_matrices_that_the_other_ways_do(launches, monkeypatch):
+    """More than 64 rows: a weight of another type, shape or layout is no business of the tiles whatever its copy says, and a copy
+    of another matrix, or a result in another type, goes the way that does not look at the copy."""
+    monkeypatch.setattr(K, "_library_linear", lambda a, weight, bias, out_dtype, keep_shares=False: launches.append(("library", ()))
+                        or torch.empty(a.shape[0], weight.shape[0], dtype=out_dtype))
+    a, w = torch.zeros(100, 256, dtype=torch.bfloat16), torch.zeros(512, 256, dtype=torch.bfloat16)
+    sh, other = K.shuffle_weight(w), K.shuffle_weight(w[:256])
+    names = lambda: [name for name, _ in launches]
+
+    def run(weight, copy):
+        for call in (lambda: K.linear(a, weight, None, shuffled=copy), lambda: K.linear(a, weight, None, shuffled=copy, act="relu2"),
+                     lambda: K.swiglu_gate_up(a, weight, copy), lambda: K.swiglu_gate_up(a, weight, copy, activation="gelu_tanh")):
+            launches.clear()
+            try:
+                call()
+            except K.KernelError:
+                yield "refused"
+                continue
+            yield names()[0]
+    assert list(run(w, sh)) == ["tl_gemm_tiles"] * 4
+    assert list(run(w, other)) == ["library", "library", "refused", "library"]
+    assert list(run(w.float(), sh)) == ["tl_gemm_generic"] * 4                       # (which refuses the pair of types)
+    assert list(run(torch.zeros(512, 512, dtype=torch.bfloat16)[:, ::2], sh)) == ["refused"] * 4
+    assert list(run(torch.zeros(512, 1, 256, dtype=torch.bfloat16), sh)) == ["refused"] * 4
+    launches.clear()
+    assert K.linear(a, w, None, out_dtype=torch.float16, shuffled=sh).dtype == torch.float16 and names() == ["library"]
