@@ -735,7 +735,7 @@ extern "C" int tl_moe_gemm(const void* A, int a_dtype, int lda, const void* W, i
     const bool bf = a_dtype == TL_BF16 && w_dtype == TL_BF16 && c_dtype == (glu ? TL_BF16 : TL_F32);
     if (BM == 256) {
         TL_CHECK_ARG(bf && tl_moe_gemm_takes_wide(K) && lda % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0,
-                     "tl_moe_gemm: tiles of 256 rows are for aligned bfloat16 operands with K a multiple of %d, not K=%d", MGW_KT, K);
+                     "tl_moe_gemm: tiles of 256 rows are for aligned bfloat16 operands with K a multiple of %d and N and ldc of 4, not K=%d N=%d ldc=%d", MGW_KT, K, N, ldc);
         TL_CHECK_ARG(((double)max_tiles * 256.0 + 256.0) * lda * 2.0 < 4e9 && (glu == 1 ? 2.0 : 1.0) * N * K * 2.0 < 4e9,
                      "tl_moe_gemm: tiles of 256 rows reach 4 GB of rows and of an expert's matrix");
         const int ntiles = tl_ceil_div(N, glu == 1 ? 128 : 256);

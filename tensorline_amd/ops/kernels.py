@@ -2014,7 +2014,7 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
     BM = moe_tile_rows(P, E)
     if (BM == 64 and (_moe_takes_wide_tiles(P, E, F, K) or _moe_takes_wide_stack(E, F, K)) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
             and library().tl_moe_gemm_takes_wide(F) and (T == 1 or h.stride(0) % 8 == 0)
-            and (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0
+            and (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0 and N % 4 == 0       # (results are stored four columns at a time)
             and (P + 256 * (E + 2)) * max(h.stride(0), K, F) < 2e9 and F2 * K < 2e9 and N * F < 2e9):      # 32-bit offsets
         BM = MOE_WIDE_TILE
     max_tiles = P // BM + E

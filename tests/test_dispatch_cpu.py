@@ -171,3 +171,16 @@ def test_many_row_products_take_and_refuse_the_matrices_that_the_other_ways_do(l
     assert list(run(torch.zeros(512, 1, 256, dtype=torch.bfloat16), sh)) == ["refused"] * 4
     launches.clear()
     assert K.linear(a, w, None, out_dtype=torch.float16, shuffled=sh).dtype == torch.float16 and names() == ["library"]
+
+
+def _expert_launches(launches, T, E, top, Kd, F, N):
+    """The rows of a tile that each product of an experts' call is launched with; operands without memory."""
+    at = lambda *shape, dtype=torch.bfloat16: torch.empty(*shape, dtype=dtype, device="meta")
+    launches.clear()
+    K.moe_experts(at(T, Kd), at(E, 2 * F, Kd), at(E, N, F), at(T, top, dtype=torch.int32), at(T, top, dtype=torch.float32), 7.0, 1.0)
+    return [args[12] for name, args in launches if name == "tl_moe_gemm"]
+
+
+def test_experts_whose_result_is_no_whole_quads_stay_in_tiles_of_64_rows(launches):
+    assert _expert_launches(launches, 600, 16, 2, 1024, 1024, 1024) == _expert_launches(launches, 600, 16, 2, 1024, 1024, 68) == [256, 256]
+    assert all(_expert_launches(launches, 600, 16, 2, 1024, 1024, n) == [64, 64] for n in (66, 1023, 1, 1025))

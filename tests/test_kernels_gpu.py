@@ -1303,6 +1303,29 @@ def test_a_large_stack_of_few_experts_takes_wide_tiles(monkeypatch):
     assert torch.equal(wide, K().moe_experts(h, up, down, ids, weights, 7.0, 1.0))
 
 
+@pytest.mark.parametrize("N", [66, 68, 3])
+def test_a_large_stack_of_experts_with_few_columns_of_result(N):
+    """Stacks that take wide tiles by their size, with a result of so many columns, whole quads (which wide tiles store) or not:
+    against the sums in float64."""
+    torch.manual_seed(N)
+    T, E, Kd, F, top = 600, 16, 1024, 1024, 2
+    ids = torch.rand(T, E, device=DEV).topk(top, 1).indices.int().contiguous()
+    h, weights = torch.randn(T, Kd, device=DEV).to(torch.bfloat16), torch.rand(T, top, device=DEV)
+    up = (torch.randn(E, 2 * F, Kd, device=DEV) / 32).to(torch.bfloat16)
+    down = (torch.randn(E, N, F, device=DEV) / 32).to(torch.bfloat16)
+    got = K().moe_experts(h, up, down, ids, weights, 7.0, 1.0)
+    want, slack = torch.zeros(T, N, dtype=torch.float64, device=DEV), torch.full((T, N), 1e-4, dtype=torch.float64, device=DEV)
+    for e in range(E):
+        rows, place = (ids == e).nonzero(as_tuple=True)
+        z = h[rows].double() @ up[e].double().T
+        g = z[:, :F].clamp(max=7.0)
+        act, w = g * torch.sigmoid(g) * (z[:, F:].clamp(-7.0, 7.0) + 1.0), weights[rows, place].double()[:, None]
+        want[rows] += w * (act @ down[e].double().T)
+        # the activations are kept as bfloat16 (2^-9 of each at most): what that can move in a sum of F products
+        slack[rows] += w * ((act.abs() * 2.0 ** -8 + 1e-4) @ down[e].double().abs().T)
+    assert bool(((got.double() - want).abs() <= slack).all())
+
+
 @pytest.mark.parametrize("P,E,BM", [(1, 1, 16), (7, 3, 256), (1000, 70, 16), (5000, 64, 256), (12288, 64, 64), (9000, 200, 256), (3000, 1024, 16)])
 def test_pairs_in_tiles_by_expert(P, E, BM):
     """The order of the pairs and the tiles made of it: every pair once, in a tile of its expert, tiles within BM rows."""
