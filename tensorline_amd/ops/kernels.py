@@ -1966,6 +1966,7 @@ def moe_tile_rows(pairs: int, experts: int) -> int:
 
 
 MOE_WIDE_TILE = 256      # rows at most of a tile of the grouped bfloat16 product of many rows per expert
+MOE_WIDE_REACH = 2_000_000_000   # entries of the rows and of an expert's matrix that its 32-bit byte offsets reach: more rows go in several passes
 
 
 def _moe_takes_wide_tiles(pairs: int, experts: int, ff: int, width: int) -> bool:
@@ -2010,36 +2011,54 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
     _f32(weights, "moe_experts weights", T * top)
     if shared is not None:
         _f32(shared, "moe_experts shared", T * N)
-    P = T * top
-    BM = moe_tile_rows(P, E)
-    if (BM == 64 and (_moe_takes_wide_tiles(P, E, F, K) or _moe_takes_wide_stack(E, F, K)) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
-            and library().tl_moe_gemm_takes_wide(F) and (T == 1 or h.stride(0) % 8 == 0)
-            and (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0 and N % 4 == 0       # (results are stored four columns at a time)
-            and (P + 256 * (E + 2)) * max(h.stride(0), K, F) < 2e9 and F2 * K < 2e9 and N * F < 2e9):      # 32-bit offsets
-        BM = MOE_WIDE_TILE
-    max_tiles = P // BM + E
-    order = torch.empty(P, dtype=torch.int32, device=h.device)
-    tiles = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=h.device)
-    _call("tl_moe_sort", _ptr(ids), _ptr(order), _ptr(tiles), P, E, BM, _stream())
-    act = torch.empty(P, F, dtype=h.dtype, device=h.device)
-    _call("tl_moe_gemm", _ptr(h), _code(h, "moe_experts input"), h.stride(0) if T > 1 else K, _ptr(gate_up),
-          _code(gate_up, "moe_experts weights"), _ptr(act), _code(act, "moe_experts"), F, _ptr(order), _ptr(tiles), max_tiles, E, BM,
-          top, F, K, 1 if gated else 2, ctypes.c_float(limit), ctypes.c_float(alpha), ctypes.c_float(shift), _stream())
-    y = torch.empty(P, N, dtype=torch.float32, device=h.device)
-    _call("tl_moe_gemm", _ptr(act), _code(act, "moe_experts"), F, _ptr(down), _code(down, "moe_experts weights"), _ptr(y), F32, N,
-          _ptr(order), _ptr(tiles), max_tiles, E, BM, top, N, F, 0, ctypes.c_float(0.0), ctypes.c_float(0.0), ctypes.c_float(0.0),
-          _stream())
     if keep_rows:
         _check(shared is None, "moe_experts: the experts' rows are handed on without a shared expert only")
-        return ExpertRows(y, weights)
-    out = torch.empty(T, N, dtype=torch.float32, device=h.device)
     ldg = 0
     if shared_gate is not None:
         _check(shared is not None and shared_gate.dtype == torch.float32 and tuple(shared_gate.shape) == (T, 1),
                "moe_experts: the shared expert's gate is float32 [T, 1]")
         ldg = shared_gate.stride(0) if T > 1 else 1
-    _call("tl_moe_combine", _ptr(y), _ptr(weights), _ptr(shared), _ptr(shared_gate), ldg, _ptr(out), T, N, top, _stream())
-    return out
+    BM, at_once = moe_tile_rows(T * top, E), T
+    if (BM == 64 and (_moe_takes_wide_tiles(T * top, E, F, K) or _moe_takes_wide_stack(E, F, K)) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
+            and library().tl_moe_gemm_takes_wide(F) and (T == 1 or h.stride(0) % 8 == 0)
+            and (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0 and N % 4 == 0       # (results are stored four columns at a time)
+            and max(F2 * K, N * F) < MOE_WIDE_REACH):
+        most = (MOE_WIDE_REACH // max(h.stride(0), K, F) - 256 * (E + 2)) // top
+        if most > 0:
+            BM, at_once = MOE_WIDE_TILE, min(T, most)
+    rows = torch.empty(T * top, N, dtype=torch.float32, device=h.device) if keep_rows else None
+    out = None if keep_rows else torch.empty(T, N, dtype=torch.float32, device=h.device)
+    ldh, call = h.stride(0) if T > 1 else K, (gate_up, down, F, N, BM, limit, alpha, shift, gated, ldg)
+    if at_once == T:
+        _experts_pass(h, ldh, ids, weights, shared, shared_gate, rows, out, *call)
+    else:                                                  # (a token's bits do not depend on the others)
+        weights, shared = weights.view(T, top), shared if shared is None else shared.view(T, N)
+        for t in range(0, T, at_once):
+            s = slice(t, min(T, t + at_once))
+            _experts_pass(h[s], ldh, ids[s], weights[s], shared if shared is None else shared[s], shared_gate if shared_gate is None else shared_gate[s],
+                          rows[s.start * top:s.stop * top] if keep_rows else None, None if keep_rows else out[s], *call)
+    return ExpertRows(rows, weights) if keep_rows else out
+
+
+def _experts_pass(h, ldh, ids, weights, shared, shared_gate, rows, out, gate_up, down, F, N, BM, limit, alpha, shift, gated, ldg) -> None:
+    """:func:`moe_experts` for the tokens given: pairs sorted into tiles of ``BM`` rows, both products, and the sum into ``out``, or
+    the experts' rows into ``rows``."""
+    (T, K), E, top = h.shape, gate_up.shape[0], ids.shape[1]
+    P = T * top
+    max_tiles = P // BM + E
+    order = torch.empty(P, dtype=torch.int32, device=h.device)
+    tiles = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=h.device)
+    _call("tl_moe_sort", _ptr(ids), _ptr(order), _ptr(tiles), P, E, BM, _stream())
+    act = torch.empty(P, F, dtype=h.dtype, device=h.device)
+    _call("tl_moe_gemm", _ptr(h), _code(h, "moe_experts input"), ldh, _ptr(gate_up),
+          _code(gate_up, "moe_experts weights"), _ptr(act), _code(act, "moe_experts"), F, _ptr(order), _ptr(tiles), max_tiles, E, BM,
+          top, F, K, 1 if gated else 2, ctypes.c_float(limit), ctypes.c_float(alpha), ctypes.c_float(shift), _stream())
+    y = torch.empty(P, N, dtype=torch.float32, device=h.device) if rows is None else rows
+    _call("tl_moe_gemm", _ptr(act), _code(act, "moe_experts"), F, _ptr(down), _code(down, "moe_experts weights"), _ptr(y), F32, N,
+          _ptr(order), _ptr(tiles), max_tiles, E, BM, top, N, F, 0, ctypes.c_float(0.0), ctypes.c_float(0.0), ctypes.c_float(0.0),
+          _stream())
+    if rows is None:
+        _call("tl_moe_combine", _ptr(y), _ptr(weights), _ptr(shared), _ptr(shared_gate), ldg, _ptr(out), T, N, top, _stream())
 
 
 # ---------------------------------------------------------------------------------------------

@@ -184,3 +184,15 @@ def _expert_launches(launches, T, E, top, Kd, F, N):
 def test_experts_whose_result_is_no_whole_quads_stay_in_tiles_of_64_rows(launches):
     assert _expert_launches(launches, 600, 16, 2, 1024, 1024, 1024) == _expert_launches(launches, 600, 16, 2, 1024, 1024, 68) == [256, 256]
     assert all(_expert_launches(launches, 600, 16, 2, 1024, 1024, n) == [64, 64] for n in (66, 1023, 1, 1025))
+
+
+def test_rows_beyond_the_wide_tiles_reach_go_in_passes(launches):
+    """Wide tiles whatever the number of pairs: in passes over the tokens whose rows 32-bit offsets reach, and whose tiles one launch
+    takes (tiles of 64 rows would be too many of them)."""
+    E, top, Kd, F = 64, 8, 1024, 512
+    for T in (240_000, 600_000):
+        assert set(_expert_launches(launches, T, E, top, Kd, F, 1024)) == {256}
+        sorts, products = [a for n, a in launches if n == "tl_moe_sort"], [a for n, a in launches if n == "tl_moe_gemm"]
+        assert sum(a[3] for a in sorts) == T * top and len(products) == 2 * len(sorts) and len(sorts) == (1 if T < 250_000 else 3)
+        assert all((a[10] * 256 + 256) * a[2] * 2 < 4e9 and a[10] <= 65535 for a in products)       # what tl_moe_gemm asks for
+        assert sum(a[6] for n, a in launches if n == "tl_moe_combine") == T

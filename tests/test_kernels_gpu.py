@@ -1326,6 +1326,27 @@ def test_a_large_stack_of_experts_with_few_columns_of_result(N):
     assert bool(((got.double() - want).abs() <= slack).all())
 
 
+@pytest.mark.parametrize("keep_rows", [False, True])
+def test_experts_in_passes_over_the_tokens(keep_rows, monkeypatch):
+    """Where the wide tiles' offsets do not reach all rows, passes over the tokens: bit for bit what one pass gives, with input
+    rows wider than K, a shared expert and its gate."""
+    torch.manual_seed(8)
+    T, E, Kd, F, top = 700, 16, 1024, 1024, 2
+    ids = torch.rand(T, E, device=DEV).topk(top, 1).indices.int().contiguous()
+    h, weights = torch.randn(T, Kd + 8, device=DEV).to(torch.bfloat16)[:, :Kd], torch.rand(T, top, device=DEV)
+    up = (torch.randn(E, 2 * F, Kd, device=DEV) / 32).to(torch.bfloat16)
+    down = (torch.randn(E, Kd, F, device=DEV) / 32).to(torch.bfloat16)
+    extra = dict(keep_rows=True) if keep_rows else dict(shared=torch.randn(T, Kd, device=DEV), shared_gate=torch.randn(T, 3, device=DEV)[:, 1:2])
+    passes = []
+    run_pass = K()._experts_pass
+    monkeypatch.setattr(K(), "_experts_pass", lambda *a: passes.append(a[0].shape[0]) or run_pass(*a))
+    once = K().moe_experts(h, up, down, ids, weights, 7.0, 1.0, **extra)
+    monkeypatch.setattr(K(), "MOE_WIDE_REACH", (256 * (E + 2) + 2 * 300) * (Kd + 8))
+    parts = K().moe_experts(h, up, down, ids, weights, 7.0, 1.0, **extra)
+    assert passes == [700, 300, 300, 100]
+    assert torch.equal(once.rows, parts.rows) and torch.equal(parts.weights, weights) if keep_rows else torch.equal(once, parts)
+
+
 @pytest.mark.parametrize("P,E,BM", [(1, 1, 16), (7, 3, 256), (1000, 70, 16), (5000, 64, 256), (12288, 64, 64), (9000, 200, 256), (3000, 1024, 16)])
 def test_pairs_in_tiles_by_expert(P, E, BM):
     """The order of the pairs and the tiles made of it: every pair once, in a tile of its expert, tiles within BM rows."""
