@@ -69,7 +69,7 @@ class LLM:
             runner = GraphRunner(self.model, self.cache, max_batch=ec.max_num_seqs,
                                  max_blocks_per_seq=-(-ec.max_model_len // ec.block_size))
             if ec.tune_library and self.model.dtype == torch.bfloat16:
-                # decode steps of more rows than the engine's own kernels take are library products too,
+                # decode steps of more than 64 rows have library products too (those that gemm_tiles.hip does not take),
                 # of exactly the graphs' row counts
                 for rows in runner.batch_buckets:
                     if rows > kernels.ROWS64_MAX_ROWS and rows != ec.max_batched_tokens:

@@ -111,15 +111,15 @@ class DecoderModel:
     # ---- one step ------------------------------------------------------------------------
     def tune_library(self, rows: int) -> int:
         """Let the library choose its kernels by measurement for steps of ``rows`` tokens (a full
-        prompt portion): one search per distinct product shape.  Returns how many were searched."""
+        prompt portion): one search per distinct product shape that is the library's.  Returns how many were searched."""
         seen, done = set(), 0
         for part in self._all_parts():
-            for weight, out_dtype in getattr(part, "library_products", lambda: [])():
-                key = (tuple(weight.shape), weight.dtype, out_dtype)
+            for weight, out_dtype, *how in getattr(part, "library_products", lambda: [])():
+                key = (tuple(weight.shape), weight.dtype, out_dtype, *(tuple(h.shape) if isinstance(h, torch.Tensor) else h for h in how))
                 if key in seen:
                     continue
                 seen.add(key)
-                done += bool(kernels.tune_library_linear(rows, weight, out_dtype))
+                done += bool(kernels.tune_library_linear(rows, weight, out_dtype, 2.0, *how))
         return done
 
     def _tail_intake(self) -> Intake:

@@ -586,7 +586,7 @@ MFMA_HEAD_DIMS = (32, 64, 128, 256)   # head sizes of the bfloat16 matrix-core a
 GENERIC_SPLIT_KEYS = 256  # keys per split of the any-shape attention kernel in steps of one token per sequence
 FLOAT_DECODE_SPLIT_KEYS = 128   # the same where its float form without LDS tiles runs (attention_float_decode.h; 256: 40 us for 33)
 SKINNY_MAX_ROWS = 16     # rows the few-row kernel serves (one 16-row MFMA tile)
-ROWS64_MAX_ROWS = 64     # rows the 17..64-row kernel serves; above that the library
+ROWS64_MAX_ROWS = 64     # rows the 17..64-row kernel serves; above that gemm_tiles.hip or the library
 FLOAT_SPLIT_MAX_ROWS = 65535 * 32   # rows one launch of the float product of more than 16 rows takes
 FLOAT_SPLIT_BYTES = 512 << 20   # at most this much for the parts of a launch's rows: more rows go in several launches
 FLOAT_SPLIT_MIN_K = 64   # below: the float instruction (_float_split)
@@ -765,23 +765,30 @@ def _keep_tuning_records_out_of_the_way(tn) -> None:
     atexit.register(remove)
 
 
-def tune_library_linear(rows: int, weight: torch.Tensor, out_dtype: torch.dtype, seconds: float = 2.0) -> bool:
+def tune_library_linear(rows: int, weight: torch.Tensor, out_dtype: torch.dtype, seconds: float = 2.0,
+                        shuffled: torch.Tensor | None = None, form: str = "plain") -> bool:
     """Have the library pick its kernel for the ``[rows, K] x [N, K]^T`` product by measurement
     (torch's TunableOp searches the hipBLASLt and rocBLAS solutions once and keeps the fastest for
     later calls of that shape) instead of by its heuristic: at 2,048 rows and the widths of a 7B
     model the heuristic's choice reaches about 1.0 PFLOP/s, the measured one 1.25.  Only the shape
     given is searched, here and now; other shapes keep the heuristic and are never searched at a
     request's cost.  Returns False when this torch has no TunableOp or the product does not go to
-    the library."""
+    the library: ``shuffled`` is the matrix-core ordered copy that the program calls it with, if any, and ``form`` "gated"
+    where it does so by :func:`swiglu_gate_up`, "relu2" by :func:`linear` with that activation."""
+    if not (form in ("plain", "gated", "relu2")):
+        raise KernelError(f"tune_library_linear: unknown form {form!r}")
     tn = getattr(torch.cuda, "tunable", None)
     if tn is None or weight.dtype != torch.bfloat16 or rows <= ROWS64_MAX_ROWS:
         return False
-    _on_gpu(weight)
+    _on_gpu(weight, shuffled)
+    N, K = weight.shape
+    a = torch.randn(rows, K, device=weight.device).to(torch.bfloat16)
+    if _tiles_plan(a, shuffled, rows, N, K, K, gated=form == "gated"):
+        return False
     tn.enable(True)
     _keep_tuning_records_out_of_the_way(tn)
     tn.set_max_tuning_duration(int(seconds * 1000))
     tn.set_max_tuning_iterations(50)
-    a = torch.randn(rows, weight.shape[1], device=weight.device).to(torch.bfloat16)
     tn.tuning_enable(True)
     try:
         _library_linear(a, weight, None, out_dtype)

@@ -100,7 +100,7 @@ class PagedAttention(Part):
 
     # ---- one step ------------------------------------------------------------------------
     def library_products(self):
-        return [(self.qkv.weight, self.dtype), (self.o_proj.weight, torch.float32)]
+        return [self.qkv.in_library(self.dtype), self.o_proj.in_library(torch.float32)]
 
     @property
     def defers_norm(self) -> bool:
@@ -216,7 +216,7 @@ class NormedAttention(Part):
         return self.qkv.tensors_kept() + self.o_proj.tensors_kept() + [t for t in (self.q_norm, self.k_norm) if t is not None]
 
     def library_products(self):
-        return [(lin.weight, torch.float32) for lin in (self.qkv, self.o_proj) if lin.weight is not None]
+        return [lin.in_library(torch.float32) for lin in (self.qkv, self.o_proj) if lin.weight is not None]
 
     def cache_need(self) -> CacheNeed | None:
         return keys_and_values(self.kv_heads, self.kernel_dim, self.window)

@@ -34,8 +34,9 @@ class Part:
         """Device tensors this part keeps (for byte accounting)."""
         return []
 
-    def library_products(self) -> list[tuple[torch.Tensor, torch.dtype]]:
-        """(weight, output dtype) of the products this part hands to the library in many-row steps."""
+    def library_products(self) -> list[tuple]:
+        """(weight, output dtype) of the products this part may hand to the library in many-row steps, and the further arguments
+        of :func:`tensorline_amd.ops.kernels.tune_library_linear` that tell which of them it does (:meth:`Linear.in_library`)."""
         return []
 
     # Optional hand-off of the norms to the products around them (few-row bfloat16 steps).  A mixer
@@ -90,6 +91,10 @@ class Linear:
 
     def tensors_kept(self) -> list[torch.Tensor]:
         return [t for t in (self.weight, self.bias, self.shuffled, self.shuffled_float) if t is not None]
+
+    def in_library(self, out_dtype: torch.dtype, form: str = "plain") -> tuple:
+        """This matrix for :meth:`Part.library_products`; ``form``: what its product's kernel does with the sums."""
+        return self.weight, out_dtype, self.streamed, form
 
     @property
     def streamed(self) -> torch.Tensor | None:

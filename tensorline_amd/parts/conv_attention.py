@@ -132,7 +132,7 @@ class _ConvAttention(Part):
         return self.qkv.tensors_kept() + self.o_proj.tensors_kept() + [self.taps] + ([self.freq] if self.freq is not None else [])
 
     def library_products(self):
-        return [(lin.weight, torch.float32) for lin in (self.qkv, self.o_proj) if lin is not None and lin.weight is not None]
+        return [lin.in_library(torch.float32) for lin in (self.qkv, self.o_proj) if lin is not None and lin.weight is not None]
 
     # ---- what it keeps -------------------------------------------------------------------
     def cache_need(self) -> CacheNeed:

@@ -139,7 +139,7 @@ class RoutedExperts(Part):
     def library_products(self):
         if self.shared_down is None:
             return []
-        return [(self.shared_gate_up.weight, self.dtype), (self.shared_down.weight, torch.float32)]
+        return [self.shared_gate_up.in_library(self.dtype, "gated" if self.activation == "swiglu" else "plain"), self.shared_down.in_library(torch.float32)]
 
     @property
     def keeps_expert_rows(self) -> bool:

@@ -47,7 +47,7 @@ class SwiGLU(Part):
         return self.gate_up.tensors_kept() + self.down.tensors_kept()
 
     def library_products(self):
-        return [(self.gate_up.weight, self.dtype), (self.down.weight, torch.float32)]
+        return [self.gate_up.in_library(self.dtype, "gated"), self.down.in_library(torch.float32)]
 
     @property
     def defers_norm(self) -> bool:
@@ -92,7 +92,7 @@ class UpDown(Part):
         return self.up.tensors_kept() + self.down.tensors_kept()
 
     def library_products(self):
-        return [(self.up.weight, torch.float32), (self.down.weight, torch.float32)]
+        return [self.up.in_library(torch.float32, self.activation), self.down.in_library(torch.float32)]
 
     def forward(self, h, ctx):
         act = self.up(h, out_dtype=self.dtype, act=self.activation)       # the activation rides on few-row products

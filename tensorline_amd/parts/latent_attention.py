@@ -131,7 +131,7 @@ class LatentAttention(Part):
         return self.proj.tensors_kept() + self.o_proj.tensors_kept() + [self.norm_w, self.uk_t, self.uv] + own
 
     def library_products(self):
-        return [(lin.weight, torch.float32) for lin in (self.proj, self._q if self.q_rank else None, self.o_proj) if lin is not None]
+        return [lin.in_library(torch.float32) for lin in (self.proj, self._q if self.q_rank else None, self.o_proj) if lin is not None]
 
     def cache_need(self) -> CacheNeed | None:
         return keys_and_values(1, self.cache_dim, self.window)

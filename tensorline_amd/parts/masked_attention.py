@@ -198,7 +198,7 @@ class MaskedAttention(Part):
         return self.qkv.tensors_kept() + self.o_proj.tensors_kept() + [t for t in (self.q_norm, self.k_norm, self.freq, self.sink, self.distance_bias) if t is not None]
 
     def library_products(self):
-        return [(lin.weight, torch.float32) for lin in (self.qkv, self.o_proj) if lin.weight is not None]
+        return [lin.in_library(torch.float32) for lin in (self.qkv, self.o_proj) if lin.weight is not None]
 
     # ---- what it keeps -------------------------------------------------------------------
     def cache_need(self) -> CacheNeed:

@@ -66,7 +66,7 @@ class ParallelMixers(Part):
         return (self.fused.tensors_kept() if self.fused is not None else []) + [t for m in self.sides for t in m.weight_tensors()]
 
     def library_products(self):
-        own = [(self.fused.weight, torch.float32)] if self.fused is not None else []
+        own = [self.fused.in_library(torch.float32)] if self.fused is not None else []
         return own + [p for m in self.sides for p in m.library_products()]
 
     def cache_need(self):

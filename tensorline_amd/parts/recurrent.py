@@ -73,7 +73,7 @@ class LightningAttention(Part):
         return self.proj.tensors_kept() + self.o_proj.tensors_kept() + [self.norm_w]
 
     def library_products(self):
-        return [(self.proj.weight, torch.float32), (self.o_proj.weight, torch.float32)]
+        return [self.proj.in_library(torch.float32), self.o_proj.in_library(torch.float32)]
 
     def cache_need(self):
         return None
@@ -139,7 +139,7 @@ class WKV(Part):
         return out
 
     def library_products(self):
-        return [(p.weight, torch.float32) for p in (self.r, self.g, self.o_proj)]
+        return [p.in_library(torch.float32) for p in (self.r, self.g, self.o_proj)]
 
     def cache_need(self):
         return None
@@ -215,7 +215,7 @@ class StateSpaceDuality(Part):
             self.conv_w, self.conv_b, self.dt_bias, self.rate_log, self.skip, self.norm_w]
 
     def library_products(self):
-        return [(lin.weight, torch.float32) for lin in (self.proj, self.o_proj) if lin.weight is not None]
+        return [lin.in_library(torch.float32) for lin in (self.proj, self.o_proj) if lin.weight is not None]
 
     def cache_need(self):
         return None
@@ -304,7 +304,7 @@ class RealGatedLRU(Part):
             self.conv_w, self.conv_b, self.gates, self.bias_r, self.bias_i, self.lam]
 
     def library_products(self):
-        return [(self.proj.weight, torch.float32), (self.o_proj.weight, torch.float32)]
+        return [self.proj.in_library(torch.float32), self.o_proj.in_library(torch.float32)]
 
     def cache_need(self):
         return None
@@ -396,7 +396,7 @@ class GatedDeltaRule(Part):
         return self.proj.tensors_kept() + self.o_proj.tensors_kept() + [self.conv_w, self.rate_log, self.dt_bias, self.norm_w]
 
     def library_products(self):
-        return [(lin.weight, torch.float32) for lin in (self.proj, self.o_proj) if lin is not None and lin.weight is not None]
+        return [lin.in_library(torch.float32) for lin in (self.proj, self.o_proj) if lin is not None and lin.weight is not None]
 
     def cache_need(self):
         return None
@@ -484,7 +484,7 @@ class SelectiveScan(Part):
         return [t for lin in self._linears() for t in lin.tensors_kept()] + [self.conv_w, self.conv_b, self.dt_bias, self.a2, self.skip]
 
     def library_products(self):
-        return [(lin.weight, torch.float32) for lin in self._linears() if lin.weight is not None]
+        return [lin.in_library(torch.float32) for lin in self._linears() if lin.weight is not None]
 
     def cache_need(self):
         return None
@@ -577,7 +577,7 @@ class MatrixLSTM(Part):
         return self.proj.tensors_kept() + self.o_proj.tensors_kept() + [self.bias_in, self.bias_forget, self.norm_w]
 
     def library_products(self):
-        return [(lin.weight, torch.float32) for lin in (self.proj, self.o_proj) if lin is not None and lin.weight is not None]
+        return [lin.in_library(torch.float32) for lin in (self.proj, self.o_proj) if lin is not None and lin.weight is not None]
 
     def cache_need(self):
         return None

@@ -196,3 +196,24 @@ def test_rows_beyond_the_wide_tiles_reach_go_in_passes(launches):
         assert sum(a[3] for a in sorts) == T * top and len(products) == 2 * len(sorts) and len(sorts) == (1 if T < 250_000 else 3)
         assert all((a[10] * 256 + 256) * a[2] * 2 < 4e9 and a[10] <= 65535 for a in products)       # what tl_moe_gemm asks for
         assert sum(a[6] for n, a in launches if n == "tl_moe_combine") == T
+
+
+def test_the_library_is_searched_for_its_own_products_only(launches, monkeypatch):
+    """What runs on the many-row tiles is not searched: with the copy that the program calls it with, in the form it has."""
+    class Tunable:
+        def __getattr__(self, name):
+            return lambda *a: None
+    searched = []
+    monkeypatch.setattr(torch.cuda, "tunable", Tunable())
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    monkeypatch.setattr(K, "_keep_tuning_records_out_of_the_way", lambda tn: None)
+    monkeypatch.setattr(K, "_library_linear", lambda a, weight, bias, out_dtype: searched.append((a.shape[0], *weight.shape)))
+    matrix = lambda N, Kd: torch.zeros(N, Kd, dtype=torch.bfloat16)
+    w, odd, narrow = matrix(512, 256), matrix(512, 120), matrix(80, 256)
+    for rows, weight, copy, form, is_searched in ((100, w, True, "plain", False), (100, w, True, "gated", False), (100, w, True, "relu2", False),
+                                                  (100, w, False, "plain", True), (100, odd, True, "plain", True), (64, w, True, "plain", False),
+                                                  (100, narrow, True, "plain", False), (100, narrow, True, "gated", True)):      # 40 pairs: no whole blocks
+        searched.clear()
+        got = K.tune_library_linear(rows, weight, torch.float32, 2.0, K.shuffle_weight(weight) if copy else None, form)
+        assert got is is_searched and searched == ([(rows, *weight.shape)] if is_searched else []), (rows, tuple(weight.shape), copy, form)
+    assert K.tune_library_linear(100, w, torch.float32) and not launches            # without a copy, as ever

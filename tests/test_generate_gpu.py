@@ -658,12 +658,14 @@ def test_command_line_generate(case):
     assert counters["tokens_generated"] == 2 * case.max_tokens and counters["ttft_s"]["count"] == 2
 
 
-def test_library_tuning_keeps_results(folder_b):
+@pytest.mark.parametrize("config,own", [("B", True), ("C", False)])
+def test_library_tuning_keeps_results(folder_b, tmp_path_factory, config, own):
     """Letting the library choose its kernels by measurement changes which kernel runs, not what a
-    prompt portion computes."""
+    prompt portion computes.  ``own``: the many-row products of this model are the engine's own, and nothing is searched;
+    the other one's rows are no multiple of 64 long, and its products are the library's."""
     from tensorline_amd import LLM, SamplingParams
-    d, w, cfg = folder_b
-    prompt = helpers.prompts_for("B", [150], seed=9)
+    d = folder_b[0] if config == "B" else helpers.make_model_dir(tmp_path_factory, config, seed=21)
+    prompt = helpers.prompts_for(config, [150], seed=9)
     sp = SamplingParams(max_tokens=6, stop_token_ids=NO_STOP)
     plainly = LLM(d, dtype="bfloat16", device=DEV, num_blocks=64, block_size=8, max_batched_tokens=128)
     want = plainly.generate(prompt, sp)[0].token_ids
@@ -671,7 +673,8 @@ def test_library_tuning_keeps_results(folder_b):
     tuned = LLM(d, dtype="bfloat16", device=DEV, num_blocks=64, block_size=8, max_batched_tokens=128, tune_library=True,
                 max_num_seqs=96)
     try:
-        assert tuned.engine.runner.batch_buckets[-1] == 96 and tuned.model.tune_library(128) >= 1
+        assert tuned.engine.runner.batch_buckets[-1] == 96
+        assert tuned.model.tune_library(128) == 0 if own else tuned.model.tune_library(128) >= 1
         assert tuned.generate(prompt, sp)[0].token_ids == want
     finally:
         torch.cuda.tunable.enable(False)
