@@ -173,7 +173,10 @@ static const GtTile gt_tiles[] = {GT_TILES(X)};
 static int gt_ntiles(const GtTile& t, int N, bool gated) { return gated ? tl_ceil_div(N / 2, t.bn / 2) : tl_ceil_div(N, t.bn); }
 
 // us of a product in tiles of t and `shares`: whole rounds of work-groups over the 256 CUs, or W from memory, or what the CUs
-// load, whichever is more; then the result's bytes, and the shares' second reading (by whoever takes them, or by a kernel)
+// load, whichever is more, and of tiles that the same bound holds for those that keep the CUs least busy: where W from memory is
+// the bound tiles of 256 rows are slower than those of 128 (us, 256 and 128 rows and the library: a head of 152,064 x 3,584 for
+// 65 rows 283, 234, 244, for 128 289, 252, 252; of 151,936 x 1,536 for 65 128, 109, 124); then the result's bytes, and the shares'
+// second reading (by whoever takes them, or by a kernel)
 static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shares, bool takes_shares) {
     const int mtiles = tl_ceil_div(M, t.bm);
     const double groups = (double)mtiles * gt_ntiles(t, N, gated) * shares, slots = 256.0 * t.per_cu;
@@ -183,7 +186,7 @@ static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shar
     if (rest > 0) busy += steps * (rest <= 256 ? step1 : step2) + t.ends;
     const double weights = 0.233e-6 * 2.0 * N * K, loads = 0.060e-6 * groups * steps * (t.bm + t.bn) * 128.0;
     const double plane = 4e-6 * (double)M * N;           // MB of float
-    double us = 3.4 + fmax(busy, fmax(weights, loads)) + 0.211 * (gated ? 0.25 : shares) * plane;
+    double us = 3.4 + fmax(busy, fmax(weights, loads)) + 1e-4 * busy + 0.211 * (gated ? 0.25 : shares) * plane;
     if (shares > 1) us += takes_shares ? 0.2 * (shares - 1) * plane : 2.7 + 0.13 * (shares + 1) * plane;
     return us;
 }

@@ -217,3 +217,10 @@ def test_the_library_is_searched_for_its_own_products_only(launches, monkeypatch
         got = K.tune_library_linear(rows, weight, torch.float32, 2.0, K.shuffle_weight(weight) if copy else None, form)
         assert got is is_searched and searched == ([(rows, *weight.shape)] if is_searched else []), (rows, tuple(weight.shape), copy, form)
     assert K.tune_library_linear(100, w, torch.float32) and not launches            # without a copy, as ever
+
+
+def test_products_bound_by_their_weights_take_the_tiles_that_keep_the_cus_least_busy():
+    """A head's matrix is read from memory once whatever the tile: no more rows in a tile than there are."""
+    plan = K.library().tl_gemm_tiles_plan
+    for N, Kd in ((152064, 3584), (151936, 1536), (131072, 5120)):
+        assert all(plan(M, N, Kd, 0, 0) == 256 + 2 for M in (65, 96, 128)) and plan(192, N, Kd, 0, 0) == 256 + 6      # of 128 and 192 rows
