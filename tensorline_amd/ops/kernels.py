@@ -1978,23 +1978,16 @@ MOE_WIDE_REACH = 2_000_000_000   # entries of the rows and of an expert's matrix
 
 def _moe_takes_wide_tiles(pairs: int, experts: int, ff: int, width: int) -> bool:
     """Whether the experts' products (ff x width) run in tiles of up to 256 rows by 256 matrix rows (a work-group of one per CU)
-    and not in tiles of 64 by 128: where there are twice as many tiles as CUs and the matrices or the rows are not small.  They
-    fetch each matrix once and the rows half as often (64 experts of 4,096 x 2,048, both products and what goes ahead of them, us,
-    small and wide tiles: 18 rows per expert 592 and 530, 90: 909 and 588, 192: 1,449 and 739; of 2,048 x 1,408: 18 rows 217 and
-    191, 192: 615 and 303; 256 of 512 x 512 64 rows 153 and 120).  :func:`_moe_takes_wide_stack` adds what large stacks gain with
-    fewer tiles."""
-    rows, size = -(-pairs // experts), ff * width
-    return (experts * -(-rows // MOE_WIDE_TILE) * -(-ff // 128) >= 512
-            and (rows >= 64 or size >= 1 << 20 or (rows >= 48 and size >= 1 << 18)))
-
-
-def _moe_takes_wide_stack(experts: int, ff: int, width: int) -> bool:
-    """The same for any number of tiles: where the stacked matrices are large, streaming them is what takes the time, and the wide
-    tiles do that faster even where they leave CUs without one (us, small and wide: 32 experts of 1,024 x 512 17 rows 39 and 36,
-    188: 80 and 63, 562: 182 and 132; 8 of 4,096 x 2,048 100 rows 134 and 114; 8 of 2,048 x 1,024 17 rows 52 and 45; 256 of
-    1,024 x 256 17 rows 107 and 96).  Below, their start costs more: 16 of 1,024 x 512 17 rows 32 and 30 but 100 38 and 40, 8 of
-    1,024 x 512 200 rows 35 and 54, 32 of 512 x 128 48 rows 23 and 25."""
-    return experts * ff * width >= 1 << 24
+    and not in tiles of 64 by 128.  They fetch each matrix once and the rows half as often.  Where the stacked matrices are large,
+    streaming them is what takes the time, and the wide tiles do that faster from 17 rows an expert on, even where they leave CUs
+    without one (us, both products and what goes ahead of them, small and wide: 64 experts of 4,096 x 2,048 18 rows 592 and 530, 90
+    909 and 588, 192 1,449 and 739; of 2,048 x 1,408 18 rows 217 and 191, 192 615 and 303; 32 of 1,024 x 512 17 rows 39 and 36, 188 80
+    and 63, 562 182 and 132; 8 of 4,096 x 2,048 100 rows 134 and 114; 8 of 2,048 x 1,024 17 rows 52 and 45; 256 of 1,024 x 256 17
+    rows 107 and 96).  Small stacks take them for many rows where there are twice as many tiles as CUs; else their start costs more
+    (16 of 1,024 x 512 17 rows 32 and 30 but 100 38 and 40, 8 of 1,024 x 512 200 rows 35 and 54, 32 of 512 x 128 48 rows 23 and 25)."""
+    rows = -(-pairs // experts)
+    return (experts * ff * width >= 1 << 24
+            or (rows >= 64 and experts * -(-rows // MOE_WIDE_TILE) * -(-ff // 128) >= 512))
 
 
 def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
@@ -2026,8 +2019,8 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
                "moe_experts: the shared expert's gate is float32 [T, 1]")
         ldg = shared_gate.stride(0) if T > 1 else 1
     BM, at_once = moe_tile_rows(T * top, E), T
-    if (BM == 64 and (_moe_takes_wide_tiles(T * top, E, F, K) or _moe_takes_wide_stack(E, F, K)) and h.dtype == torch.bfloat16 and library().tl_moe_gemm_takes_wide(K)
-            and library().tl_moe_gemm_takes_wide(F) and (T == 1 or h.stride(0) % 8 == 0)
+    if (BM == 64 and _moe_takes_wide_tiles(T * top, E, F, K) and h.dtype == torch.bfloat16
+            and library().tl_moe_gemm_takes_wide(K) and library().tl_moe_gemm_takes_wide(F) and (T == 1 or h.stride(0) % 8 == 0)
             and (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0 and N % 4 == 0       # (results are stored four columns at a time)
             and max(F2 * K, N * F) < MOE_WIDE_REACH):
         most = (MOE_WIDE_REACH // max(h.stride(0), K, F) - 256 * (E + 2)) // top

@@ -18,6 +18,14 @@ def launches(monkeypatch):
     return calls
 
 
+def _expert_launches(launches, T, E, top, Kd, F, N):
+    """The rows of a tile that each product of an experts' call is launched with; operands without memory."""
+    at = lambda *shape, dtype=torch.bfloat16: torch.empty(*shape, dtype=dtype, device="meta")
+    launches.clear()
+    K.moe_experts(at(T, Kd), at(E, 2 * F, Kd), at(E, N, F), at(T, top, dtype=torch.int32), at(T, top, dtype=torch.float32), 7.0, 1.0)
+    return [args[12] for name, args in launches if name == "tl_moe_gemm"]
+
+
 def test_key_splits_follow_the_batch_and_the_context_and_never_exceed_what_the_merge_takes():
     for seqs in (1, 2, 8, 9, 64, 65, 300):
         for kv in (1, 4, 8):
@@ -108,12 +116,19 @@ def test_short_prompts_at_a_head_size_of_256_walk_on_their_own():
     assert chains([2], [3000]) > 0                                                              # in runs of keys
 
 
-def test_experts_in_wide_tiles_by_tiles_rows_and_size():
-    wide = lambda rows, experts, width, ff: K._moe_takes_wide_tiles(rows * experts, experts, ff, width)
-    assert wide(18, 64, 4096, 2048) and wide(18, 64, 2048, 1408) and wide(17, 128, 2048, 768) and wide(17, 128, 2048, 512)
-    assert not wide(188, 32, 1024, 512) and not wide(100, 8, 4096, 2048)            # fewer than two tiles per CU
-    assert not wide(17, 256, 1024, 256) and not wide(32, 256, 512, 512) and not wide(48, 512, 512, 256)      # small, few rows
-    assert wide(48, 256, 1024, 256) and wide(64, 256, 512, 512) and wide(64, 512, 512, 256)
+def test_experts_in_wide_tiles_by_tiles_rows_and_size(launches):
+    """The tiles that the products are launched with, by rows an expert, experts, width and the experts' width."""
+    def wide(rows, experts, width, ff):
+        tiles = set(_expert_launches(launches, rows * experts // 4, experts, 4, width, ff, width))
+        assert tiles in ({64}, {256})
+        return tiles == {256}
+    # large stacks, with tiles for every CU or not
+    assert wide(20, 64, 4096, 2048) and wide(20, 64, 2048, 1408) and wide(20, 128, 2048, 768) and wide(20, 128, 2048, 512)
+    assert wide(188, 32, 1024, 512) and wide(100, 8, 4096, 2048) and wide(20, 256, 1024, 256) and wide(32, 256, 512, 512) and wide(48, 512, 512, 256)
+    # small ones, with twice as many tiles as CUs and many rows, with fewer tiles, with few rows
+    assert wide(64, 512, 128, 128) and wide(1100, 16, 512, 1024) and wide(600, 64, 512, 384)
+    assert not wide(20, 16, 1024, 512) and not wide(100, 16, 1024, 512) and not wide(200, 8, 1024, 512) and not wide(48, 32, 512, 128)
+    assert not wide(60, 512, 128, 128)
 
 
 def test_many_row_products_are_cut_within_the_tiles_limits():
@@ -125,11 +140,6 @@ def test_many_row_products_are_cut_within_the_tiles_limits():
             assert 0 <= tile < 7 and 1 <= shares <= 12 and shares <= max(1, Kd // 256) and not (gated and (shares > 1 or tile == 1))
     for M, N, Kd, gated in ((70, 64, 96, 0), (70, 66, 64, 0), (70, 48, 64, 1), (70, 1 << 17, 1 << 15, 0), (0, 64, 64, 0), (513, 3584, 3584, 0)):
         assert plan(M, N, Kd, gated, 0) == -1
-
-
-def test_large_stacks_of_experts_take_wide_tiles_whatever_their_number():
-    assert K._moe_takes_wide_stack(32, 512, 1024) and K._moe_takes_wide_stack(4, 1024, 4096) and K._moe_takes_wide_stack(256, 512, 512)
-    assert not K._moe_takes_wide_stack(16, 512, 1024) and not K._moe_takes_wide_stack(64, 128, 256)
 
 
 def test_a_many_row_product_with_an_activation_refuses_a_wrong_bias(launches):
@@ -171,14 +181,6 @@ def test_many_row_products_take_and_refuse_the_matrices_that_the_other_ways_do(l
     assert list(run(torch.zeros(512, 1, 256, dtype=torch.bfloat16), sh)) == ["refused"] * 4
     launches.clear()
     assert K.linear(a, w, None, out_dtype=torch.float16, shuffled=sh).dtype == torch.float16 and names() == ["library"]
-
-
-def _expert_launches(launches, T, E, top, Kd, F, N):
-    """The rows of a tile that each product of an experts' call is launched with; operands without memory."""
-    at = lambda *shape, dtype=torch.bfloat16: torch.empty(*shape, dtype=dtype, device="meta")
-    launches.clear()
-    K.moe_experts(at(T, Kd), at(E, 2 * F, Kd), at(E, N, F), at(T, top, dtype=torch.int32), at(T, top, dtype=torch.float32), 7.0, 1.0)
-    return [args[12] for name, args in launches if name == "tl_moe_gemm"]
 
 
 def test_experts_whose_result_is_no_whole_quads_stay_in_tiles_of_64_rows(launches):

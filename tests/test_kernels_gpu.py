@@ -1297,9 +1297,9 @@ def test_a_large_stack_of_few_experts_takes_wide_tiles(monkeypatch):
     h, weights = torch.randn(T, Kd, device=DEV).to(torch.bfloat16), torch.rand(T, top, device=DEV)
     up = (torch.randn(E, 2 * F, Kd, device=DEV) / 64).to(torch.bfloat16)
     down = (torch.randn(E, Kd, F, device=DEV) / 32).to(torch.bfloat16)
-    assert K()._moe_takes_wide_stack(E, F, Kd) and not K()._moe_takes_wide_tiles(T * top, E, F, Kd)
+    assert K()._moe_takes_wide_tiles(T * top, E, F, Kd)
     wide = K().moe_experts(h, up, down, ids, weights, 7.0, 1.0)
-    monkeypatch.setattr(K(), "_moe_takes_wide_stack", lambda *a: False)
+    monkeypatch.setattr(K(), "_moe_takes_wide_tiles", lambda *a: False)
     assert torch.equal(wide, K().moe_experts(h, up, down, ids, weights, 7.0, 1.0))
 
 
