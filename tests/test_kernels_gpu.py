@@ -119,7 +119,7 @@ def test_linear_many_rows_keeps_its_shares_on_request():
 @pytest.mark.parametrize("tile", range(7))
 @pytest.mark.parametrize("M,N,Kd,shares", [(65, 36, 64, 1), (257, 272, 128, 2), (129, 516, 320, 1), (200, 96, 832, 3), (1, 4, 192, 1), (193, 260, 1024, 4)])
 def test_many_row_product_in_every_tile(tile, M, N, Kd, shares):
-    """Every tile of the many-row product at the edges of tiles and panels, with one step of K and fewer steps than stages, in shares,
+    """Every tile of the many-row product at the edges of tiles, with one step of K and fewer steps than stages, in shares,
     rows with a stride, columns that are no whole block; bias and activation behind the sum.  The products of bfloat16 numbers are
     exact in float, so a sum of K of them is off by at most K 2^-24 of the sum of their sizes."""
     torch.manual_seed(tile)
@@ -148,6 +148,71 @@ def test_many_row_product_in_every_tile(tile, M, N, Kd, shares):
             got = K()._tiles(a, K().shuffle_weight(w), None, torch.bfloat16, M, 2 * I, Kd, a.stride(0), 256 + tile, gated=True, act=act)
             want_g = fn(both[:, :I]) * both[:, I:]
             torch.testing.assert_close(got.double(), want_g, rtol=2.0 ** -8, atol=1e-4)
+
+
+TILE_SIZES = [(256, 256), (256, 192), (128, 256), (128, 128), (64, 128), (64, 64), (192, 256)]      # rows and columns, as gemm_tiles.hip numbers them
+
+
+def _gate_error(gate, up, err_gate, err_up, act):
+    """What errors of a float gate and up leave of ``act(gate) * up`` in bfloat16: neither activation is steeper than 1.13."""
+    return 1.13 * err_gate * (up.abs() + err_up) + act(gate).abs() * err_up + (2.0 ** -8 * (act(gate) * up).abs()) + 1e-6
+
+
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("Kd", [128, 384, 448, 832])
+def test_many_row_product_beyond_one_panel(tile, Kd):
+    """More rows than a panel (2,048) and three tiles of columns, the last one partial, over 2, 6, 7 and 13 steps (fewer than the
+    stages, and several rounds of them); gated: three tiles of pairs, the last one partial.  Bounds as in the test above."""
+    bm, bn = TILE_SIZES[tile]
+    torch.manual_seed(tile)
+    M, N = 2048 + bm + 9, 2 * bn + 20
+    a = torch.randn(M, Kd, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    want, err = a.double() @ w.double().T, Kd * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+    got = K()._tiles(a, K().shuffle_weight(w), None, torch.float32, M, N, Kd, Kd, 256 + tile)
+    assert bool(((got.double() - want).abs() <= err).all())
+    if tile == 1:
+        return
+    M, I = 2048 + bm + 9 if Kd == 448 else bm + 9, bn + 48
+    a, w = a[:M], (torch.randn(2 * I, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    both, err = a.double() @ w.double().T, Kd * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+    for act, fn in ((0, torch.nn.functional.silu), (2, lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+        got = K()._tiles(a, K().shuffle_weight(w), None, torch.bfloat16, M, 2 * I, Kd, Kd, 256 + tile, gated=True, act=act)
+        gate, up = both[:, :I], both[:, I:]
+        assert bool(((got.double() - fn(gate) * up).abs() <= _gate_error(gate, up, err[:, :I], err[:, I:], fn)).all())
+
+
+@pytest.mark.parametrize("M,N,Kd,gated,tile,shares", [(2049, 17920, 1536, True, 0, 1), (801, 17920, 1536, True, 2, 1), (513, 17920, 1536, True, 6, 1),
+                                                      (700, 9728, 896, True, 3, 1), (65, 9728, 896, True, 4, 1), (1300, 1536, 8960, False, 1, 5),
+                                                      (801, 1536, 8960, False, 2, 6), (1025, 1536, 8960, False, 6, 7), (2049, 6144, 1024, False, 0, 1),
+                                                      (801, 2048, 1536, False, 4, 1), (2049, 2048, 1536, False, 3, 1), (65, 2048, 1536, False, 5, 4)])
+def test_many_row_calls_in_the_tiles_of_real_steps(M, N, Kd, gated, tile, shares):
+    """linear and swiglu_gate_up at sizes that the rule gives each of the tiles, with bias, activation and in every result type."""
+    torch.manual_seed(M)
+    a = torch.randn(M, Kd, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    bias, sh = torch.randn(N, device=DEV), K().shuffle_weight(w)
+    assert K()._tiles_plan(a, sh, M, N, Kd, Kd, gated=gated) == 256 * shares + tile
+    want, err = a.double() @ w.double().T, (Kd + shares) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+    if gated:
+        gate, up, eg, eu = want[:, :N // 2], want[:, N // 2:], err[:, :N // 2], err[:, N // 2:]
+        for activation, fn in (("silu", torch.nn.functional.silu), ("gelu_tanh", lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+            got = K().swiglu_gate_up(a, w, shuffled=sh, activation=activation)
+            assert got.dtype == torch.bfloat16 and bool(((got.double() - fn(gate) * up).abs() <= _gate_error(gate, up, eg, eu, fn)).all())
+        return
+    want = want + bias.double()
+    err = err + 2.0 ** -24 * want.abs()
+    got = K().linear(a, w, bias, out_dtype=torch.float32, shuffled=sh)
+    assert bool(((got.double() - want).abs() <= err).all())
+    got = K().linear(a, w, bias, shuffled=sh)
+    assert got.dtype == torch.bfloat16 and bool(((got.double() - want).abs() <= err + 2.0 ** -8 * want.abs()).all())
+    relu2 = want.clamp_min(0) ** 2                                    # (the square doubles what its argument is off by)
+    for dt, rel in ((torch.float32, 2.0 ** -23), (torch.bfloat16, 2.0 ** -8)):
+        got = K().linear(a, w, bias, out_dtype=dt, shuffled=sh, act="relu2")
+        assert got.dtype == dt and bool(((got.double() - relu2).abs() <= rel * relu2 + 2 * want.abs() * err + err ** 2 + 1e-6).all())
+    if shares > 1:
+        kept = K().linear(a, w, None, out_dtype=torch.float32, shuffled=sh, keep_shares=True)
+        assert isinstance(kept, K().ShareSum) and bool(((kept.sum().double() + bias.double() - want).abs() <= err + 2.0 ** -24 * want.abs()).all())
 
 
 def test_many_row_product_by_its_rule():
