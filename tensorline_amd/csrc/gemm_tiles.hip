@@ -16,10 +16,13 @@
 // K may be cut into shares (whole steps); the partial products go to a float workspace and are added in order, by whoever
 // takes them or by gt_add_kernel.
 //
-// us, here and in the library with its own choice of kernel (gate/up with the SiLU pass it needs; other weights at every call):
-// 2,048 rows of 37,888 x 3,584 gate/up 457 and 609, of 3,584 x 18,944 205 in two shares and 357, of 4,608 x 3,584 68 and 59;
-// 801 rows of 17,920 x 1,536 gate/up 55 and 66, of 1,536 x 8,960 28 and 44, of 2,048 x 1,536 11 and 19;
-// 200 rows of the same 24 and 32, 17 and 24, 8 and 22 to 53.
+// us, here and in the library with its own choice of kernel (gate/up with the SiLU pass it needs; weights from memory), of sizes that
+// are taken (tl_gemm_tiles_plan): 2,048 rows of 17,920 x 1,536 gate/up 131 and 141, of 9,728 x 896 52 and 66, of 1,536 x 8,960 52 and 90;
+// 801 rows of 17,920 x 1,536 gate/up 57 and 69, of 1,536 x 8,960 30 and 44, of 2,048 x 1,536 15 and 18; 192 rows of the same 27
+// and 33, 16 and 38, 11 and 11; 128 rows of 37,888 x 3,584 gate/up 70 and 74, of 3,584 x 18,944 37 and 54, of 3,584 x 3,584 17 and 25.
+// Alone, plain products of 2^20 to 2^23 results and a K of 2,048 to 4,096 are 4% slower here in the mean, 20% at most (640 rows of
+// 2,048 x 2,816 23 and 20; 1,521 of 1,024 x 3,072 25 and 21); in whole steps the library is level there, and slower where the host
+// queues the step (1,500 tokens of four layers of 1,024 769 us here, 889 with these products in the library).
 #include "tile_walk.h"
 
 #include <math.h>
@@ -192,12 +195,14 @@ static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shar
 }
 
 // The tile and the number of shares for a product (shares * 256 + tile), or -1: not one this file takes.
-// More than 512 rows of a matrix that is large both ways stay in the library.  There it is level (us, library and here: 513 rows of
-// 4,608 x 3,584 29 and 30, 37,888 x 3,584 with SiLU 161 and 164; 2,048 rows 65 and 67, of 3,584 x 3,584 53 and 51, 3,584 x 18,944
-// 212 and 216, 4,096 x 12,288 153 and 152) but for gate and up of many rows (801 rows of 37,888 x 3,584 277 and 249, 2,048 549 and
-// 438), and another order of summation in a long prompt changes the tokens that are drawn after it: of 48 draws at top-p 0.9
-// behind 150 to 2,300 tokens 15 to 31% came out differently, with logits as far from 64 bits as before.  Fewer rows and smaller
-// matrices gain more: 128 rows of 4,608 x 3,584 20 and 12; 2,048 rows of 1,536 x 8,960 86 and 49, of gate and up 9,728 x 896 66 and 48.
+// More than 512 rows of a matrix that is large both ways stay in the library (us, library and here in the best tile):
+// - plain products are level in sum: 513, 801 and 2,048 rows of 4,608 x 3,584 31, 39, 62 and 36, 40, 66; of 3,584 x 3,584 28, 34, 55 and
+//   29, 38, 54; of 3,584 x 18,944 89, 116, 224 and 77, 127, 224; of 4,096 x 12,288 91, 98, 185 and 66, 88, 167;
+// - gated ones would be faster here (of 37,888 x 3,584 with SiLU 175, 286, 553 and 143, 226, 444; 2,048 rows of 24,576 x 4,096 325 and
+//   313) and stay for their results, not for speed: with another order of summation, and gate and up not rounded to bfloat16 ahead of
+//   the SiLU, 15 to 31% of 48 draws at top-p 0.9 behind prompts of 150 to 2,300 tokens of the 7B shape came out differently, with
+//   logits as far from 64 bits as before.  No
+//   limit of the kernel lies here.
 extern "C" int tl_gemm_tiles_plan(int M, int N, int K, int gated, int takes_shares) {
     if (M <= 0 || N <= 0 || K <= 0 || K % GT_KT || N % (gated ? 32 : 4) || (double)N * K * 2.0 >= 4e9) return -1;
     if (M > 512 && N > 2048 && K > 2048) return -1;

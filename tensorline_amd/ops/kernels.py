@@ -502,8 +502,8 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
     :class:`NormSink` (then the result is the next norm's :class:`NormedRows`); both need the few-row
     kernel (:func:`can_defer_norm` rows, a shuffled copy).  ``keep_shares``: the caller takes a
     :class:`ShareSum` where the product is computed in shares of K (many rows, a long K).  ``act`` "relu2":
-    the result is ``max(y, 0)^2`` in ``out_dtype``, computed in float32: in the few-row bfloat16 kernel's
-    epilogue where that kernel runs the product, by a pass of its own otherwise."""
+    the result is ``max(y, 0)^2`` in ``out_dtype``, computed in float32: in the few-row bfloat16 kernel's or the many-row tiles'
+    epilogue where one of them runs the product, by a pass of its own otherwise."""
     if act is not None:
         _check(act == "relu2" and not isinstance(a, NormedRows) and sink is None and out is None and not keep_shares,
                "linear: the activation is 'relu2', on a plain product")
@@ -804,7 +804,7 @@ def tune_library_linear(rows: int, weight: torch.Tensor, out_dtype: torch.dtype,
 def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
                    shuffled: torch.Tensor | None = None, activation: str = "silu") -> torch.Tensor:
     """``silu(h Wg^T) * (h Wu^T)`` for a fused [2I, K] weight (gate rows first): one kernel for
-    few-row bfloat16 batches (it streams the ``shuffled`` copy), product then SiLU-multiply otherwise.
+    bfloat16 rows where it reads the ``shuffled`` copy (few rows, or what gemm_tiles.hip takes), product then SiLU-multiply otherwise.
     ``h`` may be :class:`NormedRows` (few-row kernel only).  ``activation`` "gelu_tanh": the tanh form of GELU
     passes the gate instead of SiLU (in the streaming kernels' epilogues, or by a pass over the product)."""
     if not (activation in GLU_ACTIVATIONS):

@@ -82,9 +82,9 @@ class Linear:
         self.bias = get(self.bias_name) if self.has_bias else None
 
     def prepare(self) -> "Linear":
-        """Make the second, matrix-core ordered copy of a bfloat16 weight.  Decode steps stream
-        that copy, many-row steps hand the row-major one to the library: twice the bytes, for
-        which 288 GB of HBM has room."""
+        """Make the second, matrix-core ordered copy of a bfloat16 weight.  Decode steps and most
+        many-row products read that copy, the others hand the row-major one to the library: twice the
+        bytes, for which 288 GB of HBM has room."""
         self.shuffled = kernels.shuffle_weight(self.weight)
         self.shuffled_float = kernels.shuffle_weight_float(self.weight)
         return self
