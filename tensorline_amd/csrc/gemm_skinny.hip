@@ -35,6 +35,8 @@
 // added in a fixed order that depends on the shapes only.
 #include "common.h"
 
+#include <type_traits>
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -380,6 +382,320 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
     }
 }
 
+// ---- few steps a wave -------------------------------------------------------------------------------------------
+// The same product where a wave's share of K is at most four steps, which is the products of narrow and of small models: every wave asks for all it
+// reads before it waits for anything.  What bounds such a product is not memory but the instructions in a row: a vector
+// instruction takes a wave 5 cycles and one that needs the result before it 8 (3.4 ns; measured), so the nine hundred instructions a
+// wave of the kernel above goes through are 2 to 3 us beside 1.6 us that an empty kernel takes.  Hence: addresses in scalar registers
+// (buffer loads: a lane's offset once, the steps in the scalar offset), whole steps only, so that nothing is clamped or
+// cleared, sums of squares and rotations worked out while the weights are on their way, and an epilogue of one wave whose
+// lanes hold four columns in a row.  Waves, shares of K and the order of every sum are those of the kernel above: the
+// same bits.
+//
+// us before and now, weights from memory, M = 1 / 8 / 16: with a sink 896 x 896 3.9, 2.9 / 4.0, 3.2 / 4.1, 3.3; 896 x 4,864 7.0, 4.8 / 7.2, 5.8 / 8.1,
+// 6.6; 2,048 x 6,144 9.1, 6.5 / 9.3, 7.5 / 9.9, 9.3; 3,584 x 3,584 7.7, 6.4 / 8.0, 7.0 / 8.8, 7.7; plain 1,024 x 1,024 3.6, 2.5 / 3.6, 2.6 / 3.6, 3.0; gate/up
+// 9,728 x 896 7.2, 5.9 / 7.1, 6.3 / 7.5, 6.6; 12,288 x 2,048 12.2, 10.4 / 12.7, 12.6 / 13.6, 13.6; q/k/v 1,152 x 896 5.0, 3.6 / 4.7, 3.9 / 5.0, 4.2; 3,072 x 2,048 7.2,
+// 5.3 / 7.2, 5.8 / 7.3, 6.3.  A decode step of 24 layers of 896 at one row 845 -> 676.  Above 640 work-groups the rate of the
+// stream counts and not the latency, and the kernel above has more waves to a CU: 32,000 x 2,048 in this form 26.7 for 23.7.
+typedef int sk_i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ sk_i32x4 sk_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(sk_i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
+}
+__device__ __forceinline__ sk_i32x4 sk_load_stream(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(sk_i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 2));
+}
+__device__ __forceinline__ sk_i32x4 sk_swap8(sk_i32x4 v) {     // lanes 0..7 and 8..15 of every row of 16 change places
+    sk_i32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_update_dpp(0, v[i], 0x128, 0xf, 0xf, true);      // row_ror:8
+    return r;
+}
+// a barrier of the work-group that waits for LDS only: loads stay on their way
+__device__ __forceinline__ void sk_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void sk_store4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
+__device__ __forceinline__ void sk_store4(bf16_t* p, f32x4 v) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(tl_f2bf_bits(v[0]) | (uint32_t)tl_f2bf_bits(v[1]) << 16, tl_f2bf_bits(v[2]) | (uint32_t)tl_f2bf_bits(v[3]) << 16);
+}
+
+// NW waves with shares of STEPS steps (the last ones of fewer or none) and one more that puts their sums together: it has nothing of the matrix to wait
+// for, so the owed norm's factor, the angles and the residual are ready when the sums are.  K a whole number of steps, N of
+// tiles, up to 4 RG rows.  The grid: plain tiles * SPLIT, gated pairs of tiles, q/k/v (pairs of a head, heads).
+template <int MODE, typename TO, int SPLIT, bool NARROW, int STEPS, int NW, int RG>
+__global__ __launch_bounds__(64 * (NW + (MODE == MODE_QKV ? 2 : 1))) void gemm_few_kernel(const uint4* __restrict__ Ws, const bf16_t* __restrict__ A, int K32, int lda, int M,
+                                                                 int second_tile, const float* __restrict__ bias, TO* __restrict__ C, int ldc,
+                                                                 QkvArgs qa, TlNormArgs na) {
+    constexpr bool DUAL = MODE != MODE_PLAIN;
+    constexpr int NACC = DUAL ? 2 : 1, NPARTS = 4 * NW;
+    static_assert(SPLIT == 1 || (MODE == MODE_PLAIN && !NARROW), "half tiles come with one stream of weights");
+    constexpr bool HALF = SPLIT == 2 || NARROW;                // eight columns of a tile
+    constexpr int XS = SPLIT * SK_UNITS * SK_ROWPAD;           // a wave's region of LDS, in units of 16 bytes: its rows, then its sums
+    __shared__ uint4 lds[NW * XS];
+    __shared__ float sh_part[NPARTS * 16];                     // [part][row] partial sums of squares
+    __shared__ float2 sh_rot[MODE == MODE_QKV ? 256 : 1];      // sine and cosine for column i of lane l at 64 i + l
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int unit = HALF ? blockIdx.x >> 1 : blockIdx.x, col0 = HALF ? (blockIdx.x & 1) * 8 : 0;
+    int tile = unit, tile2 = second_tile + unit;
+    if (MODE == MODE_QKV) {
+        const int pph = HALF ? gridDim.x >> 1 : gridDim.x;     // tile pairs per head
+        tile = blockIdx.y * 2 * pph + unit, tile2 = tile + pph;
+    }
+    if (wave < NW) {
+        const int s0 = wave * STEPS, mine = (K32 / (4 * SPLIT)) - s0;      // steps of this wave: min(mine, STEPS)
+        f32x4 acc[NACC * SPLIT];                               // [h * NACC + a]: the products with chunk h of a load
+#pragma unroll
+        for (int i = 0; i < NACC * SPLIT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        uint4* xs = lds + wave * XS;
+        if (mine > 0) {
+            const uint32_t tile_bytes = (uint32_t)K32 * 1024u;
+            const __amdgpu_buffer_rsrc_t w1 = sk_rsrc((const char*)Ws + (size_t)tile * tile_bytes, tile_bytes);
+            const __amdgpu_buffer_rsrc_t w2 = sk_rsrc((const char*)Ws + (size_t)tile2 * tile_bytes, tile_bytes);
+            // rows past M lie past the end of the buffer: they come as zeros and feed rows that are not written
+            const __amdgpu_buffer_rsrc_t rows = sk_rsrc(A, ((uint32_t)(M - 1) * lda + (uint32_t)K32 * 32u) * 2u);
+            const uint32_t in_chunk = !HALF ? lane * 16u : (16 * g + col0 + (c & 7)) * 16u + (c >> 3) * 1024u;
+            uint32_t xoff[RG];
+#pragma unroll
+            for (int i = 0; i < RG; ++i) xoff[i] = (uint32_t)(g + 4 * i) * lda * 2u + c * 16u;
+            auto share = [&](auto n) {                         // a share of N steps (in one block: no branch that a load could be moved behind)
+                constexpr int N = decltype(n)::value;
+                constexpr int NL = NARROW ? 2 : 4;             // loads of a step and tile (NARROW, SPLIT 2: two chunks each)
+                sk_i32x4 wv[N][NL], uv[N][NL], xr[N][SPLIT][RG];
+#pragma unroll
+                for (int st = 0; st < N; ++st) {
+                    const uint32_t s = s0 + st;
+#pragma unroll
+                    for (int h = 0; h < SPLIT; ++h)
+#pragma unroll
+                        for (int i = 0; i < RG; ++i) xr[st][h][i] = sk_load(rows, xoff[i] + 256 * h, s * 256 * SPLIT);
+#pragma unroll
+                    for (int i = 0; i < NL; ++i) {
+                        const int at = i * (HALF ? 2048 : 1024);
+                        wv[st][i] = sk_load_stream(w1, in_chunk + (at & 4095), s * 4096 * SPLIT + (at & ~4095));
+                        if (DUAL) uv[st][i] = sk_load_stream(w2, in_chunk + at, s * 4096);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);             // (the compiler would move the loads down to their uses)
+#pragma unroll
+                for (int st = 0; st < N; ++st) {
+                    // rows to LDS, 16 bytes a lane (row g + 4 i, unit c), and back as the product's second operand
+#pragma unroll
+                    for (int h = 0; h < SPLIT; ++h)
+#pragma unroll
+                        for (int i = 0; i < RG; ++i) xs[(h * SK_UNITS + c) * SK_ROWPAD + g + 4 * i] = __builtin_bit_cast(uint4, xr[st][h][i]);
+                    wave_lds_order();
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc)
+#pragma unroll
+                        for (int h = 0; h < SPLIT; ++h) {
+                            const bf16x8 xf = as_frag(xs[((cc * SPLIT + h) * 4 + g) * SK_ROWPAD + c]);
+                            f32x4& a = acc[h * NACC];
+                            // NARROW: the odd chunk's columns lie in the lanes of the upper eight and are brought down; what the upper eight
+                            // rows of the result add up belongs to no column
+                            const sk_i32x4 w = !NARROW ? wv[st][cc] : cc & 1 ? sk_swap8(wv[st][cc >> 1]) : wv[st][cc >> 1];
+                            a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), xf, a, 0, 0, 0);
+                            if (DUAL) {
+                                const sk_i32x4 u = !NARROW ? uv[st][cc] : cc & 1 ? sk_swap8(uv[st][cc >> 1]) : uv[st][cc >> 1];
+                                acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, u), xf, acc[1], 0, 0, 0);
+                            }
+                        }
+                    wave_lds_order();
+                }
+            };
+            if (mine >= STEPS) share(std::integral_constant<int, STEPS>());
+            else if (STEPS > 3 && mine == 3) share(std::integral_constant<int, 3>());
+            else if (STEPS > 2 && mine == 2) share(std::integral_constant<int, 2>());
+            else share(std::integral_constant<int, 1>());
+        }
+        // SPLIT 2: rows 0..7 (g < 2) of the first chunks' products, 8..15 of the second's
+        f32x4* red = reinterpret_cast<f32x4*>(xs);
+#pragma unroll
+        for (int a = 0; a < NACC; ++a) {
+            f32x4 r = acc[a];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[i] = SPLIT == 2 && g >= 2 ? acc[SPLIT - 1][i] : r[i];
+            red[a * 64 + lane] = r;
+        }
+        sk_barrier();
+        return;
+    }
+
+    if (MODE == MODE_QKV && wave == NW + 1) {                  // this one works out the angles
+        if ((int)blockIdx.y < qa.nq + qa.nkv) {
+            const float at = (float)qa.pos[c < M ? c : 0];
+            const float* freq = qa.inv_freq + unit * 16 + col0 + 4 * (HALF ? g & 1 : g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float sn, cs;
+                sincosf(at * freq[i], &sn, &cs);
+                sh_rot[i * 64 + lane] = make_float2(sn, cs);
+            }
+        }
+        sk_barrier();
+        return;
+    }
+
+    // the wave that puts the sums together: a lane has row c and the columns n0 .. n0 + 3
+    const int n0 = tile * 16 + col0 + 4 * g;
+    const bool writes = c < M && (!HALF || g < 2);
+    const bool owed = na.ss_in != nullptr, sink = MODE == MODE_PLAIN && na.resid != nullptr;
+    f32x4 pre_resid = {0.f, 0.f, 0.f, 0.f}, pre_weight = pre_resid, pre_bias = pre_resid, pre_bias2 = pre_resid;
+    int head = 0, idx = 0, slot = 0;
+    float rstd = 1.f;
+    if (owed) {
+        // sums of squares: NPARTS running sums of every NPARTS-th partial of the row, NS of them in a lane; past the last one come
+        // zeros.  A load brings 64 / R partials of R rows.
+        constexpr int R = 4 * RG, LANES = 64 / R, NS = NPARTS / LANES;
+        const int row = lane & (R - 1), q = lane / R;
+        const __amdgpu_buffer_rsrc_t ss = sk_rsrc(na.ss_in, (uint32_t)na.ss_n * na.ss_ld * 4u);
+        float sum[NS];
+#pragma unroll
+        for (int p = 0; p < NS; ++p) sum[p] = 0.f;
+        const uint32_t hop = (uint32_t)LANES * na.ss_ld * 4u;
+        uint32_t off = ((uint32_t)q * na.ss_ld + row) * 4u;
+        for (int t = 0; t < na.ss_n; t += 4 * NPARTS) {
+            float more[4][NS];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int p = 0; p < NS; ++p, off += hop) {
+                    more[k][p] = 0.f;
+                    if (t + k * NPARTS < na.ss_n) more[k][p] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ss, (int)off, 0, 0));
+                }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int p = 0; p < NS; ++p) sum[p] += more[k][p];
+        }
+#pragma unroll
+        for (int p = 0; p < NS; ++p) sh_part[(LANES * p + q) * 16 + row] = sum[p];
+    }
+    if (writes) {
+        if (sink) {
+            pre_resid = *reinterpret_cast<const f32x4*>(na.resid + (size_t)c * na.resid_ld + n0);
+            pre_weight = *reinterpret_cast<const f32x4*>(na.next_weight + n0);
+        }
+        if (MODE != MODE_SWIGLU && bias) {
+            pre_bias = *reinterpret_cast<const f32x4*>(bias + n0);
+            if (MODE == MODE_QKV) pre_bias2 = *reinterpret_cast<const f32x4*>(bias + n0 + qa.d / 2);
+        }
+        if (MODE == MODE_QKV) slot = qa.slots[c];
+    }
+    if (MODE == MODE_QKV) head = blockIdx.y, idx = unit * 16 + col0 + 4 * g;
+    if (owed) {
+        wave_lds_order();
+        float parts[NPARTS], ssum = 0.f;
+#pragma unroll
+        for (int p = 0; p < NPARTS; ++p) parts[p] = sh_part[p * 16 + (c & (4 * RG - 1))];
+#pragma unroll
+        for (int p = 0; p < NPARTS; ++p) ssum += parts[p];
+        rstd = 1.0f / sqrtf(ssum / na.dim + na.eps);
+    }
+    sk_barrier();
+    f32x4 part[NW][NACC * SPLIT];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const f32x4* from = reinterpret_cast<const f32x4*>(lds + w * XS);
+#pragma unroll
+        for (int a = 0; a < NACC; ++a) part[w][a] = from[a * 64 + lane];
+        if (SPLIT == 2) part[w][1] = from[(lane + 32) & 63];
+    }
+    f32x4 v = {0.f, 0.f, 0.f, 0.f}, u = v;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] += part[w][0][i];
+            if (DUAL) u[i] += part[w][1][i];
+            if (SPLIT == 2) v[i] += part[w][1][i];
+        }
+    if (owed) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] *= rstd;
+            if (DUAL) u[i] *= rstd;
+        }
+    }
+    if (MODE == MODE_QKV) {
+        // v, u: dims idx .. idx + 3 and the same + d / 2 of head `head` for token c
+        if (!writes) return;
+        const int d = qa.d, half = d / 2;
+        if (bias) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] += pre_bias[i], u[i] += pre_bias2[i];
+        }
+        if (head < qa.nq + qa.nkv) {
+            f32x4 o1, o2;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float2 r = sh_rot[i * 64 + lane];
+                o1[i] = v[i] * r.y - u[i] * r.x, o2[i] = u[i] * r.y + v[i] * r.x;
+            }
+            bf16_t* p = head < qa.nq ? qa.q_out + ((size_t)c * qa.nq + head) * d + idx : qa.k_cache + ((size_t)slot * qa.nkv + (head - qa.nq)) * d + idx;
+            if (head < qa.nq || slot >= 0) sk_store4(p, o1), sk_store4(p + half, o2);
+        } else if (slot >= 0) {
+            const int page = slot / qa.bs, off = slot - page * qa.bs;
+            bf16_t* vp = qa.v_cache + (((size_t)page * qa.nkv + (head - qa.nq - qa.nkv)) * d + idx) * qa.bs + off;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                vp[(size_t)i * qa.bs] = tl_from_float<bf16_t>(v[i]);
+                vp[(size_t)(i + half) * qa.bs] = tl_from_float<bf16_t>(u[i]);
+            }
+        }
+        return;
+    }
+    if (MODE == MODE_SWIGLU) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (na.act == 2)                                   // the tanh form of GELU passes the gate instead of SiLU
+                v[i] = 0.5f * v[i] * (1.0f + tanhf(0.7978845608028654f * (v[i] + 0.044715f * v[i] * v[i] * v[i]))) * u[i];
+            else
+                v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
+        }
+    } else if (bias) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += pre_bias[i];
+    }
+    if (sink) {
+        float sq[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = pre_resid[i] + v[i];
+            sq[i] = v[i] * v[i];
+            pre_weight[i] = v[i] * pre_weight[i];
+        }
+        if (writes) {
+            sk_store4(na.resid + (size_t)c * na.resid_ld + n0, v);
+            sk_store4(na.a_out + (size_t)c * na.a_ld + n0, pre_weight);
+        }
+        // the columns' squares in ascending order: on from the four columns of the lanes before
+        float ssum = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4 / SPLIT; ++q) {
+            float t = q == 0 ? 0.f : __shfl_up(ssum, 16, 64);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t += sq[i];
+            ssum = t;
+        }
+        if (writes && g == 4 / SPLIT - 1) na.ss_out[(size_t)blockIdx.x * na.ss_out_ld + c] = ssum;
+        return;
+    }
+    if (MODE == MODE_PLAIN && na.act == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float p = fmaxf(v[i], 0.f);
+            v[i] = p * p;
+        }
+    }
+    if (writes) sk_store4(C + (size_t)c * ldc + n0, v);
+}
+
 static size_t lds_per_wave(int MT, int nacc, int split = 1) {
     const size_t stage = (size_t)MT * split * SK_UNITS * SK_ROWPAD * sizeof(uint4);
     const size_t red = (size_t)nacc * 4 * 64 * sizeof(float);
@@ -408,6 +724,54 @@ static int sk_split(int N, int K, bool sink) {
     return tiles > 48 && tiles <= 128 && (sink ? K >= 2048 && K > 2 * N : K >= 896) ? 2 : 1;
 }
 
+// Whether the kernel of few steps takes a product (of these waves and steps a wave), and its launch.  Whole steps and tiles, rows of the
+// epilogue's operands on whole quads of columns.
+// Pairs of tiles in halves (the same bits): where whole pairs leave half of the CUs without one, or, of up to four rows, where there are
+// more pairs than CUs.  us, whole and halves, M = 1 / 8 / 16: q/k/v 1,152 x 896 (36 pairs) 4.5, 3.6 / 4.9, 3.9 / 5.1, 4.2; 3,072 x 2,048 (96) 7.0,
+// 5.3 / 7.5, 5.8 / 7.5, 6.3; 4,608 x 3,584 (144) 10.8, 10.8 / 11.2, 12.2 / 11.8, 14.9; gate/up 2,816 x 2,048 (88) 6.9, 4.8 / 7.0, 5.5 / 7.3,
+// 6.1; 4,096 x 1,024 (128) 4.2, 4.0 / 4.4, 4.0 / 4.7, 4.5; 6,144 x 1,024 (192) 4.6, 4.9 / 4.8, 5.3 / 5.1, 6.1; 9,728 x 896 (304) 5.9, 5.7 / 6.1, 6.2 /
+// 6.7, 6.9; 12,288 x 2,048 (384) 12.1, 10.4 / 12.5, 12.1 / 13.6, 14.7; 17,920 x 1,536 (560) 12.1, 11.4 / 12.7, 13.1 / 15.0, 16.4.
+static bool few_narrow(int pairs, int M) { return pairs <= 128 || (M <= 4 && pairs > 256); }
+static bool few_aligned(const void* p, int bytes, int ld) { return (uintptr_t)p % bytes == 0 && ld % 4 == 0; }
+template <int MODE, typename TO, int SPLIT, bool NARROW>
+static bool launch_few(const bf16_t* A, const uint4* Ws, const float* bias, TO* C, int M, int N, int K, int lda, int ldc, int second_tile,
+                       hipStream_t stream, const TlNormArgs& na, const QkvArgs& qa, int nwaves, int steps) {
+    if (steps > 4 || nwaves < 4 || N > 16 * 640 * (MODE == MODE_QKV ? 2 : 1) || K % (SK_SC * SPLIT) || N % 16 || K >= 1 << 26 || (double)M * lda * 2 >= 2e9) return false;
+    if (SPLIT == 2 ? steps == 4 : MODE != MODE_PLAIN && !NARROW && steps == 4) return false;       // (more registers than such a group has)
+    if (bias && (uintptr_t)bias % 16) return false;
+    if (na.ss_in && (double)na.ss_n * na.ss_ld * 4 >= 2e9) return false;
+    if (na.resid && !(few_aligned(na.resid, 16, na.resid_ld) && few_aligned(na.a_out, 8, na.a_ld) && (uintptr_t)na.next_weight % 16 == 0)) return false;
+    if (MODE == MODE_QKV ? !(few_aligned(qa.q_out, 8, 0) && few_aligned(qa.k_cache, 8, 0)) : !na.resid && !few_aligned(C, 4 * sizeof(TO), ldc)) return false;
+    constexpr int H = NARROW || SPLIT == 2 ? 2 : 1, EXTRA = MODE == MODE_QKV ? 128 : 64;
+    const dim3 grid = MODE == MODE_QKV ? dim3(qa.d / 32 * H, qa.nq + 2 * qa.nkv) : dim3(N / 16 * H);
+#define GO(STEPS, NW, RG)                                                                                                                      \
+    hipLaunchKernelGGL((gemm_few_kernel<MODE, TO, SPLIT, NARROW, STEPS, NW, RG>), grid, dim3(64 * NW + EXTRA), 0, stream, Ws, A, K / 32, lda, M,       \
+                       second_tile, bias, C, ldc, qa, na)
+#define ROWS(STEPS, NW)               \
+    if (M <= 4) GO(STEPS, NW, 1);     \
+    else if (M <= 8) GO(STEPS, NW, 2); \
+    else GO(STEPS, NW, 4)
+#define STEP(STEPS)                                             \
+    case STEPS:                                                 \
+        if (MODE == MODE_SWIGLU || nwaves == 4) {               \
+            ROWS(STEPS, 4);                                     \
+        } else {                                                \
+            ROWS(STEPS, (MODE == MODE_SWIGLU ? 4 : 8));         \
+        }                                                       \
+        return true
+    switch (steps) {
+        STEP(1);
+        STEP(2);
+        STEP(3);
+        default:
+            if constexpr (SPLIT == 1 && (MODE == MODE_PLAIN || NARROW)) switch (steps) { STEP(4); }
+    }
+#undef STEP
+#undef ROWS
+#undef GO
+    return false;
+}
+
 template <int MT, int MODE, typename TO, int SPLIT>
 static void launch_skinny(const bf16_t* A, const uint4* Ws, const float* bias, TO* C, int M, int n_out, int K, int K32,
                           int lda, int ldc, int second_tile, hipStream_t stream, const TlNormArgs& na,
@@ -417,7 +781,13 @@ static void launch_skinny(const bf16_t* A, const uint4* Ws, const float* bias, T
     const int nacc = MT * (MODE != MODE_PLAIN ? 2 : 1);
     // at most 8 waves to a group (4 in the gate/up form): measured at the 7B shapes, 16 waves stream
     // the down projection in 30.9 us and 8 in 28.0, the fused q/k/v projection in 12.1 and 11.3
-    const int nwaves = pick_waves(groups, tl_ceil_div(K32, 4 * SPLIT), MT, nacc, MODE == MODE_SWIGLU ? 4 : 8, SPLIT);
+    const int nsc = tl_ceil_div(K32, 4 * SPLIT), nwaves = pick_waves(groups, nsc, MT, nacc, MODE == MODE_SWIGLU ? 4 : 8, SPLIT);
+    const int steps = tl_ceil_div(nsc, nwaves);
+    if (MODE != MODE_PLAIN && few_narrow(groups, M)) {
+        if (launch_few<MODE, TO, SPLIT, MODE != MODE_PLAIN>(A, Ws, bias, C, M, n_out, K, lda, ldc, second_tile, stream, na, qa, nwaves, steps)) return;
+    } else if (launch_few<MODE, TO, SPLIT, false>(A, Ws, bias, C, M, n_out, K, lda, ldc, second_tile, stream, na, qa, nwaves, steps)) {
+        return;
+    }
     const size_t smem = (size_t)nwaves * lds_per_wave(MT, nacc, SPLIT);
     hipLaunchKernelGGL((gemm_skinny_kernel<MT, MODE, TO, SPLIT>), dim3(groups), dim3(nwaves * 64), smem, stream, A, Ws, bias, C,
                        M, n_out, K, K32, lda, ldc, second_tile, qa, na);

@@ -1571,3 +1571,73 @@ def test_sample_ties_over_one_to_more_than_64_chunks(V):
     flat, one = torch.zeros(n, V, device=DEV), torch.ones(n, device=DEV)
     assert K().sample(flat, one, one * 0.3, us).tolist() == [int(float(x) * kept) for x in us.tolist()]
     assert K().sample(flat, one, one, us).tolist() == [int(float(x) * V) for x in us.tolist()]
+
+
+def _off_by_one_float(t):
+    """The same values at an address that is a multiple of 4 bytes and not of 16."""
+    return torch.cat([t.new_zeros(1), t])[1:]
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,Kd", [(160, 512), (896, 896), (1024, 2304), (512, 2688), (512, 3456), (800, 4864), (8192, 1024)])
+def test_few_rows_asked_for_whole(M, N, Kd):
+    """Few-row products whose waves ask for their whole share of K at once: one to four steps a wave, last waves with fewer or
+    none, whole and half tiles, an owed norm with as many partial sums as there are columns / 16.  Operands at an address that the
+    kernel does not take send the product to the general one, which adds in the same order: the same bits."""
+    torch.manual_seed(N + M)
+    a = torch.randn(M, Kd, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    b, ws = torch.randn(N, device=DEV), K().shuffle_weight(w)
+    owed = K().NormedRows(a, torch.rand(Kd // 16, M, device=DEV) + 0.5, Kd, 1e-6)
+    for rows in (a, owed):
+        for kw in (dict(out_dtype=torch.float32), dict(out_dtype=torch.bfloat16)):
+            got, general = (K().linear(rows, w, bias, shuffled=ws, **kw) for bias in (b, _off_by_one_float(b)))
+            assert torch.equal(got, general)
+    want, size = a.double() @ w.double().T + b.double(), a.double().abs() @ w.double().abs().T + b.double().abs()
+    got = K().linear(a, w, b, out_dtype=torch.float32, shuffled=ws)
+    assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())     # Kd float sums in any order
+    resid, gamma = torch.randn(M, N, device=DEV), 1 + 0.1 * torch.randn(N, device=DEV)
+    left = []
+    for g in (gamma, _off_by_one_float(gamma)):
+        x = resid.clone()
+        nxt = K().linear(a, w, b, shuffled=ws, sink=K().NormSink(x, g, 1e-6))
+        left.append((x, nxt.rows, nxt.sumsq))
+    assert all(torch.equal(x, y) for x, y in zip(*left))
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 9, 16])
+@pytest.mark.parametrize("I,Kd", [(2048, 1024), (3072, 1024), (4864, 896), (6144, 2048), (688, 1408)])
+def test_few_rows_gated_asked_for_whole(M, I, Kd):
+    """The gated form of the above in pairs of tiles and of half tiles, behind an owed norm and without, against 64 bits: gate and up are float sums of
+    Kd products; then one rounding to bfloat16."""
+    torch.manual_seed(I + M)
+    a = torch.randn(M, Kd, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(2 * I, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    ss = torch.rand(Kd // 16, M, device=DEV) + 0.5
+    for rows, factor in ((a, torch.ones(M, 1, device=DEV).double()), (K().NormedRows(a, ss, Kd, 1e-6), 1 / (ss.double().sum(0)[:, None] / Kd + 1e-6).sqrt())):
+        got = K().swiglu_gate_up(rows, w, K().shuffle_weight(w))
+        gate, up = ((a.double() @ w.double().T) * factor).chunk(2, 1)
+        torch.testing.assert_close(got.double(), torch.nn.functional.silu(gate) * up, atol=1e-4, rtol=2.0 ** -8 + 1e-4)
+
+
+@pytest.mark.parametrize("M", [1, 4, 8, 13])
+@pytest.mark.parametrize("nq,nkv,d,Kd", [(14, 2, 64, 896), (3, 1, 96, 512), (12, 4, 128, 2688), (28, 4, 128, 1024), (40, 8, 128, 1024)])
+def test_few_rows_qkv_asked_for_whole(M, nq, nkv, d, Kd):
+    """The fused q/k/v projection of the above: whole pairs (more than 128) and halves, a head of three pairs, a row without a slot: the
+    general kernel's bits, queries and both caches."""
+    torch.manual_seed(d + M)
+    h = torch.randn(M, Kd, device=DEV).to(torch.bfloat16)
+    N = (nq + 2 * nkv) * d
+    ws = K().shuffle_weight((torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16))
+    b, pos = torch.randn(N, device=DEV), torch.randint(0, 5000, (M,), dtype=torch.int32, device=DEV)
+    freq = (10000.0 ** (-torch.arange(d // 2, device=DEV).float() * 2 / d)).contiguous()
+    slots = (torch.randperm(64, device=DEV)[:M]).to(torch.int32)
+    slots[M // 2] = -1 if M > 1 else slots[0]
+    owed = K().NormedRows(h, torch.rand(Kd // 16, M, device=DEV) + 0.5, Kd, 1e-6)
+    for rows in (h, owed):
+        left = []
+        for bias in (b, _off_by_one_float(b)):
+            kc, vc = torch.zeros(4, 16, nkv, d, dtype=torch.bfloat16, device=DEV), torch.zeros(4, nkv, d, 16, dtype=torch.bfloat16, device=DEV)
+            left.append((K().qkv_rope_store(rows, ws, bias, pos, freq, nq, nkv, d, kc, vc, slots), kc, vc))
+        assert all(torch.equal(x, y) for x, y in zip(*left))
+        assert bool(left[0][1].any()) and bool(left[0][2].any())
