@@ -337,6 +337,122 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
     }
 }
 
+// Split keys of sequences whose columns fit one tile of 16 (a decoded token and its query heads): a work-group is one wave with one
+// split of one sequence and key/value head.  The sums and their order are those of attn_mfma_kernel, and so are the bits.
+// What bounds a split is memory latency: ST blocks of 32 keys are on their way while one is multiplied, and nothing that can be
+// scalar is worked out per lane: the split, the pages (one or two to a block; the split's page ids are asked for before the
+// sequence's length is known, and are at most 64, one a lane), the block's range.  Pages of 16 tokens (ONE 0), or of 32 and more (ONE 1).
+// Two blocks at a head size of 128 are 128 registers; three spill at two waves per SIMD, and at one wave the compiler keeps
+// them in accumulation registers, behind moves that wait (7B shape, 48 sequences, the kernel before, two and three blocks: 44, 36, 59 us).
+// The heads come first in the grid, then the sequences, the splits last: consecutive work-groups go to different XCDs, and eight splits a sequence in
+// front would put every first split on the same one (59 us again).
+//
+// us with the merge kernel, attn_mfma_kernel and here (splits of both, the merge as it was): 14 / 2 heads of 64, one sequence of 300 keys 8.2 and 7.2, 64 of 100
+// to 1,000 20.1 and 13.9; 28 / 4 of 128, eight of 4,000 20.7 and 20.3, 48 of 150 to 2,300 44.5 and 36.5, 64 of 4,000 107 and 103; 16 / 4 of 128,
+// 16 of 700 to 1,500 23.6 and 16.8, one of 30,000 beside one of 17 35.8 and 25.3.
+template <int DC, int MODE, int ST, bool ONE>
+__global__ __launch_bounds__(64, 2) void attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
+                                                         const int32_t* __restrict__ tables, const int32_t* __restrict__ q_start,
+                                                         const int32_t* __restrict__ ctx_start, int NB, int q_stride, float* __restrict__ ws_o,
+                                                         float* __restrict__ ws_ml, int nq, int nkv, int bs, int bs_shift, TlMask mask, float scale,
+                                                         int split_blocks, const int32_t* __restrict__ seq_list, int skip_single, float softcap) {
+    constexpr int D = DC * 32, DB = D / 16;
+    const int lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+    const int sp = blockIdx.z, nsplit = gridDim.z, kvh = blockIdx.x;
+    const int s = seq_list ? seq_list[blockIdx.y] : (int)blockIdx.y;
+    const int page_lo = (sp * split_blocks << 5) >> bs_shift;
+    const int my_page = tables[(size_t)s * NB + min(page_lo + lane, NB - 1)];
+    const int r0 = q_start[s], n = q_start[s + 1] - r0, start = ctx_start[s];
+    const int G = nq / nkv, ncols = n * G;
+    if (ncols <= 0 || (seq_list ? n != 1 : (skip_single && n == 1))) return;       // another launch of the step owns it
+    const float scale2 = (MODE != 0 && softcap > 0.f) ? 2.0f * AM_LOG2E * scale / softcap : scale * AM_LOG2E;   // see tl_score2
+    const float cap2 = softcap * AM_LOG2E;
+    const int ws_shift = seq_list ? (int)blockIdx.y - r0 : 0;
+
+    // this split's blocks: [ha, hb) of the kept first keys, [bb, be) from the first key in sight on
+    const int khi = start + n - 1, b_lo = tl_mask_lo(mask, start) >> 5, split0 = sp * split_blocks;
+    int ha = 0, hb = 0, bb = max(b_lo, split0);
+    const int be = min((khi >> 5) + 1, split0 + split_blocks);
+    if (mask.first > 0 && b_lo > 0) ha = split0, hb = min(min((mask.first + 31) >> 5, b_lo), split0 + split_blocks);
+    const int n_head = max(hb - ha, 0), n_blocks = n_head + max(be - bb, 0);
+    if (n_blocks == 0) return;
+    bb -= n_head;                                              // block i of the walk: i + (i < n_head ? ha : bb)
+
+    const bool valid = c < ncols;
+    const int tok = n == 1 || !valid ? 0 : c / G, head = kvh * G + (valid ? c - tok * G : 0), row = r0 + tok;
+    const int p_col[1] = {valid ? start + tok : AM_NO_COLUMN}, lo_col[1] = {valid ? tl_mask_lo(mask, start + tok) : 0};
+    uint4 qf[1][DC];
+    const bf16_t* qp = q + (size_t)row * q_stride + head * D + g * 8;
+#pragma unroll
+    for (int dc = 0; dc < DC; ++dc) qf[0][dc] = valid ? *reinterpret_cast<const uint4*>(qp + dc * 32) : make_uint4(0, 0, 0, 0);
+
+    uint4 kf0[ST][DC], kf1[ST][DC], vf[ST][DB];
+    const int krow = 8 * (c >> 2) + (c & 3);                   // key of row c in score tile 0; tile 1: + 4
+    const bf16_t *kbase = kc + (size_t)kvh * D + g * 8, *vbase = vc + ((size_t)kvh * D + c) * bs;
+    const int krow_stride = nkv * D;
+    auto load = [&](int i, uint4 (&k0)[DC], uint4 (&k1)[DC], uint4 (&v)[DB]) {
+        const int kb = (i + (i < n_head ? ha : bb)) << 5;
+        // keys past khi are masked for every column; their addresses are clamped to stay on pages the sequence owns
+        const int last = khi - kb, r_0 = min(krow, last), r_1 = min(krow + 4, last), r_v = min(8 * g, last & ~7);
+        const int at = (kb >> bs_shift) - page_lo, p0 = __builtin_amdgcn_readlane(my_page, at);
+        const bf16_t *kp0, *kp1, *vp;
+        if (ONE) {
+            const int in = kb & (bs - 1);
+            const bf16_t* kp = kbase + (size_t)p0 * bs * krow_stride;
+            kp0 = kp + (in + r_0) * krow_stride, kp1 = kp + (in + r_1) * krow_stride;
+            vp = vbase + (size_t)p0 * bs * krow_stride + in + r_v;
+        } else {
+            const int p1 = __builtin_amdgcn_readlane(my_page, last >= 16 ? at + 1 : at);
+            const bf16_t *ka = kbase + (size_t)p0 * 16 * krow_stride, *kz = kbase + (size_t)p1 * 16 * krow_stride;
+            kp0 = (r_0 < 16 ? ka : kz) + (r_0 & 15) * krow_stride, kp1 = (r_1 < 16 ? ka : kz) + (r_1 & 15) * krow_stride;
+            vp = vbase + (size_t)(r_v < 16 ? p0 : p1) * 16 * krow_stride + (r_v & 15);
+        }
+#pragma unroll
+        for (int dc = 0; dc < DC; ++dc) {
+            k0[dc] = *reinterpret_cast<const uint4*>(kp0 + dc * 32);
+            k1[dc] = *reinterpret_cast<const uint4*>(kp1 + dc * 32);
+        }
+#pragma unroll
+        for (int db = 0; db < DB; ++db) v[db] = *reinterpret_cast<const uint4*>(vp + db * 16 * bs);
+    };
+    float m_run[1] = {-INFINITY}, l_run[1] = {0.f}, add[1][8];
+    f32x4 acc[1][DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) acc[0][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](int i, const uint4 (&k0)[DC], const uint4 (&k1)[DC], const uint4 (&v)[DB]) {
+        am_block<DC, 1, MODE>(k0, k1, v, qf, p_col, lo_col, mask.first, (i + (i < n_head ? ha : bb)) << 5, g, scale2, cap2, add, m_run, l_run, acc);
+    };
+#pragma unroll
+    for (int j = 0; j < ST; ++j)
+        if (j < n_blocks) load(j, kf0[j], kf1[j], vf[j]);
+    int i = 0;
+    for (; i + 2 * ST <= n_blocks; i += ST)                    // (no condition around a load here: a wait would count without it)
+#pragma unroll
+        for (int j = 0; j < ST; ++j) {
+            multiply(i + j, kf0[j], kf1[j], vf[j]);
+            load(i + j + ST, kf0[j], kf1[j], vf[j]);
+        }
+#pragma unroll
+    for (int j = 0; j < ST; ++j)
+        if (i + j < n_blocks) {
+            multiply(i + j, kf0[j], kf1[j], vf[j]);
+            if (i + j + ST < n_blocks) load(i + j + ST, kf0[j], kf1[j], vf[j]);
+        }
+#pragma unroll
+    for (int j = 0; j < ST - 1; ++j)
+        if (i + j + ST < n_blocks) multiply(i + j + ST, kf0[j], kf1[j], vf[j]);
+
+    if (!valid) return;
+    float l_tot = l_run[0];
+    l_tot += __shfl_xor(l_tot, 16, TL_WAVE);
+    l_tot += __shfl_xor(l_tot, 32, TL_WAVE);
+    const size_t part = ((size_t)(row + ws_shift) * nq + head) * nsplit + sp;
+    float* wp = ws_o + part * D + 4 * g;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4*>(wp + db * 16) = acc[0][db];
+    if (g == 0) *reinterpret_cast<float2*>(ws_ml + part * 2) = make_float2(m_run[0], l_tot);
+}
+
 // The same block of 32 keys (half `half` of a 64-key tile) with the fragments taken from LDS where
 // they are used.  kt is the tile's 64 key rows of 4 DC units in matrix-core order (row c of score
 // tile r, which is key 32 (r / 2) + 8 (c / 4) + 4 (r % 2) + c % 4 of the tile, in LDS row 16 r + c), vt
@@ -1033,10 +1149,22 @@ static void launch_attn(int NT, dim3 grid, int wg_waves, hipStream_t stream, con
                         const bf16_t* vc, const int32_t* tables, int NB, const int32_t* q_start,
                         const int32_t* ctx_start, bf16_t* out, int out_stride, float* ws_o, float* ws_ml, int nq, int nkv,
                         int bs, TlMask mask, float scale, int nsplit, int split_blocks, const int32_t* seq_list,
-                        int skip_single, const float* sinks, float softcap, TlBias bias) {
+                        int skip_single, const float* sinks, float softcap, TlBias bias, bool one_tile) {
     int bs_shift = -1;                               // pages of a power of two of tokens: a shift finds the page
     if ((bs & (bs - 1)) == 0)
         for (bs_shift = 0; (1 << bs_shift) < bs;) ++bs_shift;
+    // one tile of columns in splits of at most 64 pages
+    if constexpr (DC <= 4) if (nsplit > 1 && NT == 1 && one_tile && !bias.table && bs_shift >= 4 && split_blocks <= 2 << bs_shift && grid.x <= 65535) {
+#define AM_DECODE(MODEV, ONE)                                                                                                               \
+    hipLaunchKernelGGL((attn_decode_kernel<DC, MODEV, 2, ONE>), dim3(nkv, grid.x, nsplit), dim3(64), 0, stream, q, kc, vc, tables, q_start, \
+                       ctx_start, NB, q_stride, ws_o, ws_ml, nq, nkv, bs, bs_shift, mask, scale, split_blocks, seq_list, skip_single, softcap)
+        if (softcap > 0.f && bs_shift > 4) AM_DECODE(1, true);
+        else if (softcap > 0.f) AM_DECODE(1, false);
+        else if (bs_shift > 4) AM_DECODE(0, true);
+        else AM_DECODE(0, false);
+#undef AM_DECODE
+        return;
+    }
 #define AM_GO(NTV, MODEV)                                                                                                        \
     hipLaunchKernelGGL((attn_mfma_kernel<DC, NTV, MODEV>), grid, dim3(64 * wg_waves), 0, stream, q, q_stride, kc, vc, tables, NB, \
                        q_start, ctx_start, out, out_stride, ws_o, ws_ml, nq, nkv, bs, bs_shift, mask, scale, nsplit,           \
@@ -1169,16 +1297,16 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
     } else
     if (d == 32)
         launch_attn<1>(NT, grid, wg_waves, stream, qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride,
-                       ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias);
+                       ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias, max_tile_groups == 1);
     else if (d == 64)
         launch_attn<2>(NT, grid, wg_waves, stream, qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride,
-                       ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias);
+                       ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias, max_tile_groups == 1);
     else if (d == 128)
         launch_attn<4>(NT, grid, wg_waves, stream, qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride,
-                       ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias);
+                       ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias, max_tile_groups == 1);
     else
         launch_attn<8>(NT, grid, wg_waves, stream, qq, q_stride, kk, vv, tables, NB, q_start, ctx_start, (bf16_t*)out, out_stride,
-                       ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias);
+                       ws_o, ws_ml, nq, nkv, bs, mask, scale, nsplit, split_blocks, seq_list, skip_single, sinks, softcap, bias, max_tile_groups == 1);
     TL_CHECK_LAUNCH("tl_attention_mfma");
     if (nsplit > 1) {
         const int merge_rows = seq_list ? n_list : T;

@@ -1641,3 +1641,29 @@ def test_few_rows_qkv_asked_for_whole(M, nq, nkv, d, Kd):
             left.append((K().qkv_rope_store(rows, ws, bias, pos, freq, nq, nkv, d, kc, vc, slots), kc, vc))
         assert all(torch.equal(x, y) for x, y in zip(*left))
         assert bool(left[0][1].any()) and bool(left[0][2].any())
+
+
+@pytest.mark.parametrize("nq,nkv,d,bs", [(14, 2, 64, 16), (12, 2, 128, 16), (16, 1, 128, 64), (6, 2, 32, 32), (4, 1, 128, 8), (16, 1, 256, 16)])
+@pytest.mark.parametrize("split", [32, 64, 160, 512])
+@pytest.mark.parametrize("kw", [{}, dict(window=70, keep_first=5), dict(chunk=96, softcap=20.0, sink=True)])
+def test_decode_attention_in_splits_of_one_wave(nq, nkv, d, bs, split, kw):
+    """One-token sequences in splits of one to sixteen blocks of 32 keys (the ring of two, its remainder of none to three), contexts at the edges of a
+    block, a page and a split, first keys in splits of their own, more than 64 splits (32) and few, pages of one, two and four to a block."""
+    lens = [1, 2, 16, 31, 32, 33, 63, 65, 160, 161, 511, 512, 513, 700, 2049]
+    got, want = _attention_case(torch.bfloat16, nq, nkv, d, bs, lens, None, seed=nq + split, split_keys=split, path="mfma", **kw)
+    torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
+
+
+@pytest.mark.parametrize("split", [64, 512])
+def test_few_tokens_in_splits_of_one_wave(split):
+    """Several tokens of a sequence whose columns fit one tile of 16."""
+    got, want = _attention_case(torch.bfloat16, 8, 2, 64, 16, [700, 3, 40, 1030], [4, 3, 1, 2], seed=5, split_keys=split, path="mfma")
+    torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
+
+
+@pytest.mark.parametrize("n", [64, 256, 1000, 4096])
+def test_block_sums_take_every_lane_once(n):
+    """The norm of rows with one entry each, at every place: an entry that a sum left out or took twice would not come out as sqrt(n)."""
+    x = torch.diag(torch.linspace(1.0, 2.0, n, device=DEV))
+    got = K().norm_rows(x, torch.ones(n, device=DEV), 0.0, torch.float32)
+    torch.testing.assert_close(got, math.sqrt(n) * torch.eye(n, device=DEV), atol=0, rtol=5e-7)
