@@ -1047,14 +1047,74 @@ template <int AM_MERGE_THREADS>
 __global__ __launch_bounds__(AM_MERGE_THREADS) void attn_merge_kernel(
     const float* __restrict__ ws_o, const float* __restrict__ ws_ml, const int32_t* __restrict__ pos,
     bf16_t* __restrict__ out, int out_stride, int nq, int D, int nsplit, int split_blocks, TlMask mask,
-    const int32_t* __restrict__ seq_list, const int32_t* __restrict__ q_start, const float* __restrict__ sinks) {
+    const int32_t* __restrict__ seq_list, const int32_t* __restrict__ q_start, const float* __restrict__ sinks, bool ahead) {
     __shared__ float wgt[AM_MAX_SPLITS];
     __shared__ float red_m[AM_MERGE_THREADS / 64], red_l[AM_MERGE_THREADS / 64];
     __shared__ float4 part[AM_MERGE_THREADS];
     const int wrow = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
     const int t = seq_list ? q_start[seq_list[wrow]] : wrow;   // listed one-token sequences: their row of the step
     const int p = pos[t];
-    const int lo = tl_mask_lo(mask, p);
+    const size_t base = ((size_t)wrow * nq + h) * nsplit;
+    const int D4 = D >> 2, SG = AM_MERGE_THREADS / D4;      // D is 32, 64, 128 or 256
+    const int d4 = tid & (D4 - 1), sg = tid / D4;
+    const float4* acc4 = reinterpret_cast<const float4*>(ws_o) + base * D4 + d4;
+    const float2* ml2 = reinterpret_cast<const float2*>(ws_ml) + base;
+    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 a[AM_MERGE_AHEAD];
+    const int lo = mask.window || mask.chunk ? tl_mask_lo(mask, p) : 0;
+    if (nsplit <= 64 && lo < 32 * split_blocks) {
+        // At most 64 splits, all from the first one on: every wave finds the weights for itself (lane s that of split s), and there is one barrier.
+        // Where the splits are few bytes they are asked for whether the token has them or not, so that nothing waits for its position.
+        // us of decode attention with the three-barrier walk below and here: 14 / 2 heads of 64, one sequence of 300 keys 7.2 and 6.4, 28 / 4 of 128, eight of
+        // 4,000 20.3 and 19.2, 48 of 150 to 2,300 36.5 and 34.8.
+        const int lane = tid & 63, split_len = 32 * split_blocks;
+        float2 ml = make_float2(-INFINITY, 0.f);
+        if (ahead) {
+            if (lane < nsplit) ml = ml2[lane];
+#pragma unroll
+            for (int k = 0; k < AM_MERGE_AHEAD; ++k)
+                if (k * SG < nsplit) a[k] = acc4[(size_t)min(sg + k * SG, nsplit - 1) * D4];
+        } else {
+            if (lane * split_len <= p) ml = ml2[lane];
+#pragma unroll
+            for (int k = 0; k < AM_MERGE_AHEAD; ++k)
+                if ((sg + k * SG) * split_len <= p) a[k] = acc4[(size_t)(sg + k * SG) * D4];
+        }
+        const bool live = lane * split_len <= p;
+        const float M = tl_wave_max(live ? ml.x : -INFINITY);
+        const float w = live && ml.x > -INFINITY ? exp2f(ml.x - M) : 0.f;
+        float L = tl_wave_sum(live ? ml.y * w : 0.f);
+        if (sinks) L += exp2f(sinks[h] * AM_LOG2E - M);      // the head's sink: a key without a value
+        float4 o4 = zero4;
+#pragma unroll
+        for (int k = 0; k < AM_MERGE_AHEAD; ++k) {
+            const int s = sg + k * SG;
+            const float ws = __shfl(w, s & 63, 64);
+            if (s * split_len <= p) o4.x += a[k].x * ws, o4.y += a[k].y * ws, o4.z += a[k].z * ws, o4.w += a[k].w * ws;
+        }
+        for (int s0 = AM_MERGE_AHEAD * SG; s0 * split_len <= p; s0 += SG) {      // (the same for all threads: lanes of all splits answer)
+            const int s = s0 + sg;
+            const float ws = __shfl(w, s & 63, 64);
+            if (s * split_len <= p) {
+                const float4 v = acc4[(size_t)s * D4];
+                o4.x += v.x * ws, o4.y += v.y * ws, o4.z += v.z * ws, o4.w += v.w * ws;
+            }
+        }
+        part[tid] = o4;
+        __syncthreads();
+        if (tid < D4) {
+            float4 r = part[tid];
+#pragma unroll 4
+            for (int g = 1; g < SG; ++g) {
+                const float4 v = part[g * D4 + tid];
+                r.x += v.x, r.y += v.y, r.z += v.z, r.w += v.w;
+            }
+            const float inv_l = 1.0f / L;
+            *reinterpret_cast<uint2*>(out + (size_t)t * out_stride + (size_t)h * D + tid * 4) =
+                make_uint2(am_pack2(r.x * inv_l, r.y * inv_l), am_pack2(r.z * inv_l, r.w * inv_l));
+        }
+        return;
+    }
     const int s_lo = (lo >> 5) / split_blocks, s_hi = (p >> 5) / split_blocks;
     // the splits that hold kept first keys, [0, s_head), are visited ahead of those from s_lo on where the
     // two do not touch: place s of the walk is split s below s_head and split s + s_shift from there on
@@ -1066,13 +1126,6 @@ __global__ __launch_bounds__(AM_MERGE_THREADS) void attn_merge_kernel(
     const int s_shift = s_lo - s_head;
     const int ns = s_head + s_hi - s_lo + 1;
 #define AM_SPLIT_AT(S) ((S) < s_head ? (S) : (S) + s_shift)
-    const size_t base = ((size_t)wrow * nq + h) * nsplit;
-    const int D4 = D >> 2, SG = AM_MERGE_THREADS / D4;      // D is 32, 64, 128 or 256
-    const int d4 = tid % D4, sg = tid / D4;
-    const float4* acc4 = reinterpret_cast<const float4*>(ws_o) + base * D4 + d4;
-    const float2* ml2 = reinterpret_cast<const float2*>(ws_ml) + base;
-    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 a[AM_MERGE_AHEAD];
 #pragma unroll
     for (int k = 0; k < AM_MERGE_AHEAD; ++k) {
         const int s = sg + k * SG;
@@ -1310,12 +1363,13 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
     TL_CHECK_LAUNCH("tl_attention_mfma");
     if (nsplit > 1) {
         const int merge_rows = seq_list ? n_list : T;
+        const bool ahead = (double)merge_rows * nq * nsplit * d <= 1 << 19;      // 2 MB: within a launch's latency
         if (nsplit > 32)
             hipLaunchKernelGGL(attn_merge_kernel<256>, dim3(merge_rows, nq), dim3(256), 0, stream, ws_o, ws_ml, pos,
-                               (bf16_t*)out, out_stride, nq, d, nsplit, split_blocks, mask, seq_list, q_start, sinks);
+                               (bf16_t*)out, out_stride, nq, d, nsplit, split_blocks, mask, seq_list, q_start, sinks, ahead);
         else
             hipLaunchKernelGGL(attn_merge_kernel<128>, dim3(merge_rows, nq), dim3(128), 0, stream, ws_o, ws_ml, pos,
-                               (bf16_t*)out, out_stride, nq, d, nsplit, split_blocks, mask, seq_list, q_start, sinks);
+                               (bf16_t*)out, out_stride, nq, d, nsplit, split_blocks, mask, seq_list, q_start, sinks, ahead);
         TL_CHECK_LAUNCH("tl_attention_mfma merge");
     }
     return 0;
