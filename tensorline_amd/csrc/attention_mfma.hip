@@ -39,12 +39,6 @@ __device__ __forceinline__ bf16x8 am_frag(uint4 v) { return __builtin_bit_cast(b
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// two floats -> two bfloat16 (round to nearest even) in one register: v_cvt_pk_bf16_f32
-__device__ __forceinline__ uint32_t am_pack2(float a, float b) {
-    const f32x2 v = {a, b};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-}
-
 // max(a, b, c) of numbers that are not NaN as the one instruction it is (fmaxf first quiets each
 // operand with an instruction of its own)
 __device__ __forceinline__ float am_max3(float a, float b, float c) {
@@ -118,10 +112,10 @@ __device__ __forceinline__ void am_block(const uint4* kf0, const uint4* kf1, con
             psum += pr[i];
         }
         uint4 pf;
-        pf.x = am_pack2(pr[0], pr[1]);
-        pf.y = am_pack2(pr[2], pr[3]);
-        pf.z = am_pack2(pr[4], pr[5]);
-        pf.w = am_pack2(pr[6], pr[7]);
+        pf.x = tl_pack_bf16(pr[0], pr[1]);
+        pf.y = tl_pack_bf16(pr[2], pr[3]);
+        pf.z = tl_pack_bf16(pr[4], pr[5]);
+        pf.w = tl_pack_bf16(pr[6], pr[7]);
         if (__any(moved)) {
             const float alpha = __builtin_amdgcn_exp2f(m_run[j] - m_safe);
             l_run[j] = l_run[j] * alpha + psum;
@@ -319,8 +313,8 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
                 uint2 w;
-                w.x = am_pack2(acc[j][db][0] * inv, acc[j][db][1] * inv);
-                w.y = am_pack2(acc[j][db][2] * inv, acc[j][db][3] * inv);
+                w.x = tl_pack_bf16(acc[j][db][0] * inv, acc[j][db][1] * inv);
+                w.y = tl_pack_bf16(acc[j][db][2] * inv, acc[j][db][3] * inv);
                 *reinterpret_cast<uint2*>(op + db * 16) = w;
             }
         } else {
@@ -515,10 +509,10 @@ __device__ __forceinline__ void am_block_lds(const uint4* kt, const uint4* vt, i
             pr[i] = __builtin_amdgcn_exp2f(sv[i] - m_safe);
             psum += pr[i];
         }
-        pf[j].x = am_pack2(pr[0], pr[1]);
-        pf[j].y = am_pack2(pr[2], pr[3]);
-        pf[j].z = am_pack2(pr[4], pr[5]);
-        pf[j].w = am_pack2(pr[6], pr[7]);
+        pf[j].x = tl_pack_bf16(pr[0], pr[1]);
+        pf[j].y = tl_pack_bf16(pr[2], pr[3]);
+        pf[j].z = tl_pack_bf16(pr[4], pr[5]);
+        pf[j].w = tl_pack_bf16(pr[6], pr[7]);
         if (__any(moved)) {
             const float alpha = __builtin_amdgcn_exp2f(m_run[j] - m_safe);
             l_run[j] = l_run[j] * alpha + psum;
@@ -643,10 +637,10 @@ __device__ __forceinline__ void am_tile_lds(const uint4* kt, const uint4* vt, in
     uint4 pf[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        pf[h].x = am_pack2(pr[8 * h + 0], pr[8 * h + 1]);
-        pf[h].y = am_pack2(pr[8 * h + 2], pr[8 * h + 3]);
-        pf[h].z = am_pack2(pr[8 * h + 4], pr[8 * h + 5]);
-        pf[h].w = am_pack2(pr[8 * h + 6], pr[8 * h + 7]);
+        pf[h].x = tl_pack_bf16(pr[8 * h + 0], pr[8 * h + 1]);
+        pf[h].y = tl_pack_bf16(pr[8 * h + 2], pr[8 * h + 3]);
+        pf[h].z = tl_pack_bf16(pr[8 * h + 4], pr[8 * h + 5]);
+        pf[h].w = tl_pack_bf16(pr[8 * h + 6], pr[8 * h + 7]);
     }
     if (__any(moved)) {
         const float alpha = __builtin_amdgcn_exp2f(m_run + neg_m);
@@ -1019,8 +1013,8 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
             uint2 w;
-            w.x = am_pack2(acc[j][db][0] * inv, acc[j][db][1] * inv);
-            w.y = am_pack2(acc[j][db][2] * inv, acc[j][db][3] * inv);
+            w.x = tl_pack_bf16(acc[j][db][0] * inv, acc[j][db][1] * inv);
+            w.y = tl_pack_bf16(acc[j][db][2] * inv, acc[j][db][3] * inv);
             *reinterpret_cast<uint2*>(op + db * 16) = w;
         }
     }
@@ -1111,7 +1105,7 @@ __global__ __launch_bounds__(AM_MERGE_THREADS) void attn_merge_kernel(
             }
             const float inv_l = 1.0f / L;
             *reinterpret_cast<uint2*>(out + (size_t)t * out_stride + (size_t)h * D + tid * 4) =
-                make_uint2(am_pack2(r.x * inv_l, r.y * inv_l), am_pack2(r.z * inv_l, r.w * inv_l));
+                make_uint2(tl_pack_bf16(r.x * inv_l, r.y * inv_l), tl_pack_bf16(r.z * inv_l, r.w * inv_l));
         }
         return;
     }

@@ -23,8 +23,8 @@ __device__ __forceinline__ float4 bn_load4(const float* p) { return *reinterpret
 __device__ __forceinline__ void bn_store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void bn_store4(bf16_t* p, float4 v) {
     uint2 u;
-    u.x = (uint32_t)tl_f2bf_bits(v.x) | ((uint32_t)tl_f2bf_bits(v.y) << 16);
-    u.y = (uint32_t)tl_f2bf_bits(v.z) | ((uint32_t)tl_f2bf_bits(v.w) << 16);
+    u.x = tl_pack_bf16(v.x, v.y);
+    u.y = tl_pack_bf16(v.z, v.w);
     *reinterpret_cast<uint2*>(p) = u;
 }
 

@@ -17,11 +17,13 @@ struct bf16_t {
 __device__ __forceinline__ float tl_to_float(float v) { return v; }
 __device__ __forceinline__ float tl_to_float(bf16_t v) { return __uint_as_float(((uint32_t)v.bits) << 16); }
 
-__device__ __forceinline__ uint16_t tl_f2bf_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x0040u);  // quiet NaN
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
+// round to nearest even by the conversion instruction: for every one of the 2^32 floats, NaN included, the bits that adding 0x7fff and
+// the last kept bit gives, in one instruction for two of them where that takes a dozen
+__device__ __forceinline__ uint16_t tl_f2bf_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+__device__ __forceinline__ uint32_t tl_pack_bf16(float lo, float hi) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
 
 // 16 bytes that are read once and not again soon (the weights of a decode step's products): a

@@ -171,8 +171,8 @@ __device__ __forceinline__ float4 tl_load4(const bf16_t* p) {
 __device__ __forceinline__ void tl_store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void tl_store4(bf16_t* p, float4 v) {
     uint2 u;
-    u.x = (uint32_t)tl_f2bf_bits(v.x) | ((uint32_t)tl_f2bf_bits(v.y) << 16);
-    u.y = (uint32_t)tl_f2bf_bits(v.z) | ((uint32_t)tl_f2bf_bits(v.w) << 16);
+    u.x = tl_pack_bf16(v.x, v.y);
+    u.y = tl_pack_bf16(v.z, v.w);
     *reinterpret_cast<uint2*>(p) = u;
 }
 
@@ -475,8 +475,8 @@ __global__ void rope_store_kernel(T* __restrict__ qkv, const int32_t* __restrict
                     }
                     const float c0 = cs_s[i + 2 * k], c1 = cs_s[i + 2 * k + 1];
                     const float s0 = sn_s[i + 2 * k], s1 = sn_s[i + 2 * k + 1];
-                    o1[k] = (uint32_t)tl_f2bf_bits(a0 * c0 - b0 * s0) | ((uint32_t)tl_f2bf_bits(a1 * c1 - b1 * s1) << 16);
-                    o2[k] = (uint32_t)tl_f2bf_bits(b0 * c0 + a0 * s0) | ((uint32_t)tl_f2bf_bits(b1 * c1 + a1 * s1) << 16);
+                    o1[k] = tl_pack_bf16(a0 * c0 - b0 * s0, a1 * c1 - b1 * s1);
+                    o2[k] = tl_pack_bf16(b0 * c0 + a0 * s0, b1 * c1 + a1 * s1);
                 }
                 bf16_t* dst = hp;
                 if (h >= nq) {
@@ -582,7 +582,7 @@ __global__ void silu_mul_bf16x8_kernel(const bf16_t* __restrict__ gu, bf16_t* __
         const float g0 = __uint_as_float(gw[k] << 16), g1 = __uint_as_float(gw[k] & 0xffff0000u);
         const float u0 = __uint_as_float(uw[k] << 16), u1 = __uint_as_float(uw[k] & 0xffff0000u);
         const float o0 = g0 / (1.0f + expf(-g0)) * u0, o1 = g1 / (1.0f + expf(-g1)) * u1;
-        ow[k] = (uint32_t)tl_f2bf_bits(o0) | ((uint32_t)tl_f2bf_bits(o1) << 16);
+        ow[k] = tl_pack_bf16(o0, o1);
     }
     *reinterpret_cast<uint4*>(out + (size_t)t * I + i8 * 8) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
 }

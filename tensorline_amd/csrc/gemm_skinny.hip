@@ -421,7 +421,7 @@ __device__ __forceinline__ void sk_barrier() {
 }
 __device__ __forceinline__ void sk_store4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 __device__ __forceinline__ void sk_store4(bf16_t* p, f32x4 v) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(tl_f2bf_bits(v[0]) | (uint32_t)tl_f2bf_bits(v[1]) << 16, tl_f2bf_bits(v[2]) | (uint32_t)tl_f2bf_bits(v[3]) << 16);
+    *reinterpret_cast<uint2*>(p) = make_uint2(tl_pack_bf16(v[0], v[1]), tl_pack_bf16(v[2], v[3]));
 }
 
 // NW waves with shares of STEPS steps (the last ones of fewer or none) and one more that puts their sums together: it has nothing of the matrix to wait

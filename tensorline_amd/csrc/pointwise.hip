@@ -723,7 +723,7 @@ __global__ __launch_bounds__(256) void glu_bf16x8_kernel(const bf16_t* __restric
     for (int k = 0; k < 4; ++k) {
         const float o0 = gate(__uint_as_float(gw[k] << 16)) * __uint_as_float(uw[k] << 16);
         const float o1 = gate(__uint_as_float(gw[k] & 0xffff0000u)) * __uint_as_float(uw[k] & 0xffff0000u);
-        ow[k] = (uint32_t)tl_f2bf_bits(o0) | ((uint32_t)tl_f2bf_bits(o1) << 16);
+        ow[k] = tl_pack_bf16(o0, o1);
     }
     *reinterpret_cast<uint4*>(out + (size_t)blockIdx.x * F + i8 * 8) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
 }

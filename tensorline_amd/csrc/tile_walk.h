@@ -111,5 +111,5 @@ __device__ __forceinline__ void tw_load_once(uint32_t voff, const void* sbase, u
 }
 __device__ __forceinline__ void tw_store4(float* p, tw_f32x4 o) { *reinterpret_cast<tw_f32x4*>(p) = o; }
 __device__ __forceinline__ void tw_store4(bf16_t* p, tw_f32x4 o) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(tl_f2bf_bits(o[0]) | (uint32_t)tl_f2bf_bits(o[1]) << 16, tl_f2bf_bits(o[2]) | (uint32_t)tl_f2bf_bits(o[3]) << 16);
+    *reinterpret_cast<uint2*>(p) = make_uint2(tl_pack_bf16(o[0], o[1]), tl_pack_bf16(o[2], o[3]));
 }
