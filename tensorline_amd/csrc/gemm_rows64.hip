@@ -35,10 +35,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define R64_SC 128
 #define R64_UNITS (R64_SC / 8)
 #define R64_ROWPAD 17
-#define R64_MT 4
-#define R64_DEPTH 2                          // steps of loads in flight per wave
+#define R64_DEPTH 2                          // steps of loads in flight per wave (straight through shares of up to eight steps with four: 55 registers spilled, 0.65 to 0.9)
 #define R64_A_WEIGHT 1                       // a group's loads of A, in units of one wave's loads of W (cost model)
-#define R64_PIECES (64 * R64_UNITS)          // 16-byte pieces of A per step
+#define R64_AHEAD 8                          // shares that the second kernels ask for at once
 #define R64_MIN_WAVES 4
 #define R64_MAX_WAVES 16
 #define R64_CUS 256
@@ -65,18 +64,18 @@ __device__ __forceinline__ void r64_issue(const bf16_t* const (&xp)[P], const ui
     }
 }
 
-// P: pieces of A a thread loads per step; the group has at least 1024 / P threads (a multiple of
+// MT tiles of 16 rows: 2, 3 or 4, those that M has.  P: pieces of A a thread loads per step; the group has at least 256 MT / P threads (a multiple of
 // 16, so that a thread's pieces all lie in one 16-byte column of the step).  Wave w of group x owns
 // tile w * gridDim.x + x: groups differ by at most one live wave.  PAIR: W is a fused gate/up
 // matrix of ntiles + ntiles tiles, a wave owns gate tile t and up tile ntiles + t and writes
 // silu(gate) * up to C [M, N / 2] (one share only: the sums must be complete).
-template <typename TO, int P, int THREADS, bool PAIR>
+template <typename TO, int MT, int P, int THREADS, bool PAIR>
 __global__ __launch_bounds__(THREADS) void gemm_rows64_kernel(
     const bf16_t* __restrict__ A, const uint4* __restrict__ Ws, const float* __restrict__ bias, TO* __restrict__ C,
     float* __restrict__ partial, int M, int N, int K, int K32, int lda, int ldc, int steps_per_share, int ntiles,
     TlNormArgs na) {
-    constexpr int DEPTH = R64_DEPTH;
-    __shared__ uint4 xs[2][R64_MT * R64_UNITS * R64_ROWPAD];
+    constexpr int DEPTH = R64_DEPTH, PIECES = 16 * MT * R64_UNITS;       // 16-byte pieces of A per step
+    __shared__ uint4 xs[2][MT * R64_UNITS * R64_ROWPAD];
     __shared__ float sh_rstd[64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nthreads = blockDim.x;
@@ -92,20 +91,20 @@ __global__ __launch_bounds__(THREADS) void gemm_rows64_kernel(
     const uint4 zero = make_uint4(0, 0, 0, 0);
     const int last_c = K32 - 1;
 
-    f32x4 acc[R64_MT], acc2[PAIR ? R64_MT : 1];
+    f32x4 acc[MT], acc2[PAIR ? MT : 1];
 #pragma unroll
-    for (int i = 0; i < R64_MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < (PAIR ? R64_MT : 1); ++i) acc2[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < (PAIR ? MT : 1); ++i) acc2[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // loader of A: 64 rows x 16 units = 1024 16-byte pieces, up to P per thread
+    // loader of A: 16 MT rows x 16 units, up to P pieces per thread
     const bf16_t* xp[P];
     int xslot[P];
     bool xmine[P];
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         const int idx = tid + nthreads * i;
-        xmine[i] = idx < R64_PIECES;
+        xmine[i] = idx < PIECES;
         const int row = xmine[i] ? idx >> 4 : 0, unit = idx & 15;
         xp[i] = A + (size_t)(row < M ? row : 0) * lda;       // the row's start: the unit (this thread's xunit) is part of the k offset
         xslot[i] = ((row >> 4) * R64_UNITS + unit) * R64_ROWPAD + (row & 15);
@@ -135,7 +134,7 @@ __global__ __launch_bounds__(THREADS) void gemm_rows64_kernel(
 #pragma unroll
         for (int cc = 0; cc < 4; ++cc) {
 #pragma unroll
-            for (int mt = 0; mt < R64_MT; ++mt) {
+            for (int mt = 0; mt < MT; ++mt) {
                 const uint4 xf = xs[cur][(mt * R64_UNITS + cc * 4 + g) * R64_ROWPAD + r];
                 acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r64_frag(wr[j][cc]), r64_frag(xf), acc[mt], 0, 0, 0);
                 if (PAIR)
@@ -155,7 +154,6 @@ __global__ __launch_bounds__(THREADS) void gemm_rows64_kernel(
     // The loop runs without a branch, as long as every slot is refilled; at most three steps are left, and ask for what
     // there is.  (Steps asked for past a share's end, and zeros multiplied where its steps are odd, were up to three of seven:
     // with the same in the attention of these steps, 48 sequences of eight 7B layers 1,655 -> 1,615 us.)
-    static_assert(DEPTH == 2, "the remainder is written out for two slots");
     const std::integral_constant<int, 0> slot0;
     const std::integral_constant<int, 1> slot1;
     int base = 0;
@@ -195,8 +193,14 @@ __global__ __launch_bounds__(THREADS) void gemm_rows64_kernel(
     // accumulator register i of lane l: C[m = mt*16 + l % 16][n = tile*16 + 4*(l / 16) + i]
     const int n0 = tile * 16 + 4 * g;
     const bool sink = na.resid != nullptr && partial == nullptr;
+    if (partial && N % 4 == 0 && (uintptr_t)partial % 16 == 0) {     // whole quads of columns
 #pragma unroll
-    for (int mt = 0; mt < R64_MT; ++mt) {
+        for (int mt = 0; mt < MT; ++mt)
+            if (mt * 16 + r < M && n0 < N) *reinterpret_cast<f32x4*>(partial + ((size_t)blockIdx.y * M + mt * 16 + r) * N + n0) = acc[mt];
+        return;
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
         const int m = mt * 16 + r;
         float sq = 0.f;
 #pragma unroll
@@ -246,19 +250,35 @@ __global__ __launch_bounds__(256) void gemm_rows64_reduce_kernel(const float* __
     __shared__ float red[16];
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     const int m = blockIdx.y;
+    const bool live = n < n_out;
+    // the first shares, and what a residual sink reads, are asked for ahead of the row's sum of squares
+    const int at = live ? n : 0;
+    const float* p0 = partial + (size_t)m * N;
+    float pv[R64_AHEAD], pu[R64_AHEAD], pre_resid = 0.f, pre_weight = 0.f;
+#pragma unroll
+    for (int s = 0; s < R64_AHEAD; ++s)
+        if (s < shares) {
+            pv[s] = p0[(size_t)s * M * N + at];
+            if (swiglu) pu[s] = p0[(size_t)s * M * N + n_out + at];
+        }
+    if (na.resid) pre_resid = na.resid[(size_t)m * na.resid_ld + at], pre_weight = na.next_weight[at];
     float rs = 1.f;
     if (na.ss_in) {
         float ssum = 0.f;
         for (int t = threadIdx.x; t < na.ss_n; t += blockDim.x) ssum += na.ss_in[(size_t)t * na.ss_ld + m];
         rs = 1.0f / sqrtf(tl_block_sum(ssum, red) / na.dim + na.eps);
     }
-    const bool live = n < n_out;
     float v = 0.f, u = 0.f;
     if (live) {
-        for (int s = 0; s < shares; ++s) {
-            const float* p = partial + ((size_t)s * M + m) * N;
-            v += p[n];
-            if (swiglu) u += p[n_out + n];
+#pragma unroll
+        for (int s = 0; s < R64_AHEAD; ++s)
+            if (s < shares) {
+                v += pv[s];
+                if (swiglu) u += pu[s];
+            }
+        for (int s = R64_AHEAD; s < shares; ++s) {
+            v += p0[(size_t)s * M * N + n];
+            if (swiglu) u += p0[(size_t)s * M * N + n_out + n];
         }
         v *= rs;
         if (swiglu) v = r64_gate(v, na.act) * (u * rs);
@@ -267,10 +287,9 @@ __global__ __launch_bounds__(256) void gemm_rows64_reduce_kernel(const float* __
     if (na.resid) {
         float sq = 0.f;
         if (live) {
-            float* rp = na.resid + (size_t)m * na.resid_ld + n;
-            const float h = *rp + v;
-            *rp = h;
-            na.a_out[(size_t)m * na.a_ld + n] = tl_from_float<bf16_t>(h * na.next_weight[n]);
+            const float h = pre_resid + v;
+            na.resid[(size_t)m * na.resid_ld + n] = h;
+            na.a_out[(size_t)m * na.a_ld + n] = tl_from_float<bf16_t>(h * pre_weight);
             sq = h * h;
         }
         const float tot = tl_block_sum(sq, red);
@@ -294,32 +313,41 @@ __global__ __launch_bounds__(256) void gemm_rows64_reduce_qkv_kernel(
     __shared__ float red[16];
     const int pi = blockIdx.x * blockDim.x + threadIdx.x;
     const int m = blockIdx.y;
+    const int half = d / 2, pair = pi < N / 2 ? pi : 0;
+    const int head = pair / half, idx = pair - head * half;
+    const int n1 = head * d + idx, n2 = n1 + half;
+    // the first shares and the angle ahead of the row's sum of squares
+    const float* p0 = partial + (size_t)m * N;
+    float pv[R64_AHEAD], pu[R64_AHEAD];
+#pragma unroll
+    for (int s = 0; s < R64_AHEAD; ++s)
+        if (s < shares) pv[s] = p0[(size_t)s * M * N + n1], pu[s] = p0[(size_t)s * M * N + n2];
+    const int slot = slots[m];
+    const float b1 = bias ? bias[n1] : 0.f, b2 = bias ? bias[n2] : 0.f;
+    float sn = 0.f, cs = 1.f;
+    if (head < nq + nkv) sincosf((float)pos[m] * inv_freq[idx], &sn, &cs);
     float rs = 1.f;
     if (na.ss_in) {
         float ssum = 0.f;
         for (int t = threadIdx.x; t < na.ss_n; t += blockDim.x) ssum += na.ss_in[(size_t)t * na.ss_ld + m];
         rs = 1.0f / sqrtf(tl_block_sum(ssum, red) / na.dim + na.eps);
     }
-    const int half = d / 2;
     if (pi >= N / 2) return;
-    const int head = pi / half, idx = pi - head * half;
-    const int n1 = head * d + idx, n2 = n1 + half;
     float v = 0.f, u = 0.f;
-    for (int s = 0; s < shares; ++s) {
-        const float* p = partial + ((size_t)s * M + m) * N;
-        v += p[n1];
-        u += p[n2];
+#pragma unroll
+    for (int s = 0; s < R64_AHEAD; ++s)
+        if (s < shares) v += pv[s], u += pu[s];
+    for (int s = R64_AHEAD; s < shares; ++s) {
+        v += p0[(size_t)s * M * N + n1];
+        u += p0[(size_t)s * M * N + n2];
     }
     v *= rs;
     u *= rs;
     if (bias) {
-        v += bias[n1];
-        u += bias[n2];
+        v += b1;
+        u += b2;
     }
-    const int slot = slots[m];
     if (head < nq + nkv) {
-        float sn, cs;
-        sincosf((float)pos[m] * inv_freq[idx], &sn, &cs);
         const float o1 = v * cs - u * sn, o2 = u * cs + v * sn;
         if (head < nq) {
             bf16_t* qp = q_out + (size_t)m * nq * d + (size_t)head * d + idx;
@@ -337,6 +365,9 @@ __global__ __launch_bounds__(256) void gemm_rows64_reduce_qkv_kernel(
         vp[(size_t)half * bs] = tl_from_float<bf16_t>(u);
     }
 }
+
+// (The second kernels ask for the shares, the residual and the angle's operands ahead of the row's sum of squares, and shares are written by whole
+// quads of columns: 17 / 64 rows of 2,048 x 2,048 with a sink 9.3 -> 7.3 / 11.8 -> 9.0 us, of 3,584 x 18,944 30.0 -> 26.9 / 34.5 -> 30.4.)
 
 // The cut of a [N, K] product with M rows: waves per group and shares of K.  The cost of a cut is
 // the work of the busiest CU in units of one wave's step (4 KB of W): whole rounds of groups over
@@ -393,19 +424,34 @@ static R64Plan r64_plan_pairs(int M, int npairs, int K) {
 // Number of shares K is cut into for a [N, K] matrix and M rows (the caller sizes the workspace by it).
 extern "C" int tl_gemm_rows64_shares(int M, int N, int K) { return r64_plan(M, N, K).shares; }
 
-template <typename TO>
+// Two, three or four tiles of 16 rows: what is read, staged and multiplied per step follows from the rows that are there.  us with four for all / as
+// here (second kernel included): 17 rows of 4,608 x 3,584 q/k/v 12.8, 11.8, 3,584 x 3,584 11.3, 10.0, 896 x 4,864 10.6, 10.0, 9,728 x 896
+// gate/up 12.0, 10.9, 37,888 x 3,584 46.6, 45.7; 33 and 48 rows of 4,608 x 3,584 14.4 and 13.2, of 152,064 x 3,584 200 and 204 (four tiles: 208).
+template <typename TO, bool PAIR>
 static void r64_launch(const R64Plan& p, hipStream_t stream, const bf16_t* A, const uint4* Ws, const float* bias, TO* C,
                        float* part, int M, int N, int K, int K32, int lda, int ldc, int ntiles, const TlNormArgs& na) {
     dim3 grid(p.groups_x, p.shares), block(p.waves * 64);
-    if (p.waves >= 16)
-        hipLaunchKernelGGL((gemm_rows64_kernel<TO, 1, 1024, false>), grid, block, 0, stream, A, Ws, bias, C, part, M, N, K,
-                           K32, lda, ldc, p.steps, ntiles, na);
-    else if (p.waves >= 8)
-        hipLaunchKernelGGL((gemm_rows64_kernel<TO, 2, 1024, false>), grid, block, 0, stream, A, Ws, bias, C, part, M, N, K,
-                           K32, lda, ldc, p.steps, ntiles, na);
-    else
-        hipLaunchKernelGGL((gemm_rows64_kernel<TO, 4, 512, false>), grid, block, 0, stream, A, Ws, bias, C, part, M, N, K,
-                           K32, lda, ldc, p.steps, ntiles, na);
+#define GO(MT, P, THREADS)                                                                                                            \
+    hipLaunchKernelGGL((gemm_rows64_kernel<TO, MT, P, THREADS, PAIR>), grid, block, 0, stream, A, Ws, bias, C, part, M, N, K, K32, lda, ldc, \
+                       p.steps, ntiles, na)
+    if constexpr (!PAIR) {
+        if (p.waves >= 16) {
+            if (M <= 32) GO(2, 1, 1024);
+            else if (M <= 48) GO(3, 1, 1024);
+            else GO(4, 1, 1024);
+            return;
+        }
+        if (p.waves >= 8) {
+            if (M <= 32) GO(2, 1, 1024);
+            else if (M <= 48) GO(3, 2, 1024);
+            else GO(4, 2, 1024);
+            return;
+        }
+    }
+    if (M <= 32) GO(2, 2, 512);
+    else if (M <= 48) GO(3, 3, 512);
+    else GO(4, 4, 512);
+#undef GO
 }
 
 // A: bfloat16 [M, K], 16 < M <= 64 is what it is for (any M from 1 to 64 works); Ws: shuffled copy of
@@ -449,16 +495,14 @@ extern "C" int tl_gemm_rows64(const void* A, const void* Ws, const float* bias, 
         TL_CHECK_ARG(c_dtype == TL_BF16, "tl_gemm_rows64: the paired SwiGLU form writes bfloat16");
         const int npairs = N / 32;
         const R64Plan pp = r64_plan_pairs(M, npairs, K);
-        hipLaunchKernelGGL((gemm_rows64_kernel<bf16_t, 4, 512, true>), dim3(pp.groups_x, 1), dim3(pp.waves * 64), 0, stream,
-                           (const bf16_t*)A, (const uint4*)Ws, nullptr, (bf16_t*)C, nullptr, M, N, K, K32, lda, ldc,
-                           pp.steps, npairs, na);
+        r64_launch<bf16_t, true>(pp, stream, (const bf16_t*)A, (const uint4*)Ws, nullptr, (bf16_t*)C, nullptr, M, N, K, K32, lda, ldc, npairs, na);
         TL_CHECK_LAUNCH("tl_gemm_rows64 pairs");
         return 0;
     }
     if (c_dtype == TL_F32)
-        r64_launch<float>(plan, stream, (const bf16_t*)A, (const uint4*)Ws, bias, (float*)C, part, M, N, K, K32, lda, ldc, ntiles, na);
+        r64_launch<float, false>(plan, stream, (const bf16_t*)A, (const uint4*)Ws, bias, (float*)C, part, M, N, K, K32, lda, ldc, ntiles, na);
     else
-        r64_launch<bf16_t>(plan, stream, (const bf16_t*)A, (const uint4*)Ws, bias, (bf16_t*)C, part, M, N, K, K32, lda, ldc, ntiles, na);
+        r64_launch<bf16_t, false>(plan, stream, (const bf16_t*)A, (const uint4*)Ws, bias, (bf16_t*)C, part, M, N, K, K32, lda, ldc, ntiles, na);
     TL_CHECK_LAUNCH("tl_gemm_rows64");
     if (shares > 1) {
         dim3 rgrid(tl_ceil_div(n_out, 256), M), rblock(256);
@@ -497,7 +541,7 @@ extern "C" int tl_gemm_rows64_qkv_rope(const void* A, const void* Ws, const floa
                      "tl_gemm_rows64_qkv_rope: bad owed-norm arguments (partials %d, stride %d)", na.ss_n, na.ss_ld);
     if (M == 0) return 0;
     const int K32 = tl_ceil_div(K, 32), ntiles = tl_ceil_div(N, 16);
-    r64_launch<bf16_t>(plan, stream, (const bf16_t*)A, (const uint4*)Ws, nullptr, (bf16_t*)nullptr, partial, M, N, K, K32,
+    r64_launch<bf16_t, false>(plan, stream, (const bf16_t*)A, (const uint4*)Ws, nullptr, (bf16_t*)nullptr, partial, M, N, K, K32,
                        lda, N, ntiles, TlNormArgs());
     TL_CHECK_LAUNCH("tl_gemm_rows64_qkv_rope");
     dim3 rgrid(tl_ceil_div(N / 2, 256), M), rblock(256);

@@ -1667,3 +1667,27 @@ def test_block_sums_take_every_lane_once(n):
     x = torch.diag(torch.linspace(1.0, 2.0, n, device=DEV))
     got = K().norm_rows(x, torch.ones(n, device=DEV), 0.0, torch.float32)
     torch.testing.assert_close(got, math.sqrt(n) * torch.eye(n, device=DEV), atol=0, rtol=5e-7)
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,Kd", [(896, 896), (1026, 1032), (2048, 2048), (896, 4864), (8192, 512)])
+def test_17_to_64_rows_in_tiles_of_what_is_there(M, N, Kd):
+    """Two, three and four tiles of rows, with K whole and in shares, rows that end a tile and begin one, an N of no whole quads: plain, with a residual
+    sink, and gate/up pairs, against 64 bits."""
+    torch.manual_seed(N + M)
+    a = torch.randn(M, Kd, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    b, ws = torch.randn(N, device=DEV), K().shuffle_weight(w)
+    want, size = a.double() @ w.double().T + b.double(), a.double().abs() @ w.double().abs().T + b.double().abs()
+    got = K().linear(a, w, b, out_dtype=torch.float32, shuffled=ws)
+    assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())     # Kd float sums in any order
+    resid, gamma = torch.randn(M, N, device=DEV), 1 + 0.1 * torch.randn(N, device=DEV)
+    x = resid.clone()
+    nxt = K().linear(a, w, b, shuffled=ws, sink=K().NormSink(x, gamma, 1e-6))
+    torch.testing.assert_close(x.double(), resid.double() + want, atol=1e-5, rtol=1e-5)
+    assert torch.equal(nxt.rows, (x * gamma).to(torch.bfloat16))
+    torch.testing.assert_close(nxt.sumsq.sum(0).double(), x.double().pow(2).sum(1), atol=0, rtol=1e-5)
+    if N % 32 == 0:
+        got = K().swiglu_gate_up(K().NormedRows(a, nxt.sumsq, N, 1e-6), w, ws)
+        gate, up = (a.double() @ w.double().T / (x.double().pow(2).mean(1, keepdim=True) + 1e-6).sqrt()).chunk(2, 1)
+        torch.testing.assert_close(got.double(), torch.nn.functional.silu(gate) * up, atol=1e-4, rtol=2.0 ** -8 + 1e-4)
