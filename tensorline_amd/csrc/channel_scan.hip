@@ -547,7 +547,7 @@ __global__ __launch_bounds__(256) void conv_unit_kernel(
         if (n_unit > 0) {
             // channels that do not exist are zero (those units have no bias); every lane forms the sum of its unit
             float ss = (y.x * y.x + y.y * y.y) + (y.z * y.z + y.w * y.w);
-            for (int off = 1; off < (1 << lpu); off <<= 1) ss += __shfl_xor(ss, off, TL_WAVE);
+            ss = tl_group_sum(ss, lpu);
             if (u < n_unit) {
                 float f = 1.0f / sqrtf(ss + eps);
                 if (u < n_scaled) f *= scale;

@@ -71,6 +71,26 @@ __device__ __forceinline__ float tl_wave_max(float v) {
     return tl_wave_all(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
+// The sum over aligned groups of 2^log2 lanes, lane i with i ^ 1, then ^ 2, ^ 4, ..: within a row of 16 by permutations of quads and mirrors (after
+// the step of 2 a quad holds one value, so the mirror within eight lanes brings what lane ^ 4 holds, and so on).
+__device__ __forceinline__ float tl_group_sum(float v, int log2) {
+#define TL_MOVED(CTRL) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true))
+    if (log2 > 0) v += TL_MOVED(0xB1);                   // quad_perm 1, 0, 3, 2
+    if (log2 > 1) v += TL_MOVED(0x4E);                   // quad_perm 2, 3, 0, 1
+    if (log2 > 2) v += TL_MOVED(0x141);                  // row_half_mirror
+    if (log2 > 3) v += TL_MOVED(0x140);                  // row_mirror
+#undef TL_MOVED
+    if (log2 > 4) {
+        const tl_u32x2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    }
+    if (log2 > 5) {
+        const tl_u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    }
+    return v;
+}
+
 // Block-wide reductions for blocks of up to 1024 threads (16 waves).  `scratch` is LDS with room
 // for 16 floats.  The value is returned to every thread; the combination order is fixed, so the
 // result does not depend on timing.  Both end with a barrier, so `scratch` can be reused at once.
@@ -81,7 +101,15 @@ __device__ __forceinline__ float tl_block_sum(float v, float* scratch) {
     if (lane == 0) scratch[wave] = v;
     __syncthreads();
     float r = 0.f;
-    for (int w = 0; w < nwaves; ++w) r += scratch[w];
+#pragma unroll
+    for (int w0 = 0; w0 < 16; w0 += 4) {                 // four at a time are read before they are added
+        if (w0 >= nwaves) break;
+        const float s0 = scratch[w0], s1 = scratch[w0 + 1], s2 = scratch[w0 + 2], s3 = scratch[w0 + 3];
+        r += s0;
+        if (w0 + 1 < nwaves) r += s1;
+        if (w0 + 2 < nwaves) r += s2;
+        if (w0 + 3 < nwaves) r += s3;
+    }
     __syncthreads();
     return r;
 }

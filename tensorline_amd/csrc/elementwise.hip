@@ -38,6 +38,18 @@ __global__ void embed_kernel(const int32_t* __restrict__ ids, const T* __restric
         return;
     }
     const T* row = table + (size_t)id * H;
+    constexpr int V4 = 16 / sizeof(T);                       // a row is scattered memory: 16 bytes a thread, all of it on its way at once
+    if (H % V4 == 0 && (uintptr_t)table % 16 == 0 && (uintptr_t)x % 16 == 0) {
+        for (int c = threadIdx.x * V4; c < H; c += blockDim.x * V4) {
+            const uint4 raw = *reinterpret_cast<const uint4*>(row + c);
+            const T* e = reinterpret_cast<const T*>(&raw);
+#pragma unroll
+            for (int i = 0; i < V4; i += 4)
+                *reinterpret_cast<float4*>(xr + c + i) = make_float4(tl_to_float(e[i]) * scale, tl_to_float(e[i + 1]) * scale,
+                                                                     tl_to_float(e[i + 2]) * scale, tl_to_float(e[i + 3]) * scale);
+        }
+        return;
+    }
     for (int c = threadIdx.x; c < H; c += blockDim.x) xr[c] = tl_to_float(row[c]) * scale;
 }
 
@@ -45,7 +57,7 @@ extern "C" int tl_embed(const int32_t* ids, const void* table, int table_dtype, 
                         float scale, hipStream_t stream) {
     TL_CHECK_ARG(T >= 0 && H > 0 && V > 0, "tl_embed: bad sizes T=%d H=%d V=%d", T, H, V);
     if (T == 0) return 0;
-    dim3 grid(T), block(256);
+    dim3 grid(T), block(H > 2048 ? 512 : 256);
     if (table_dtype == TL_F32)
         hipLaunchKernelGGL(embed_kernel<float>, grid, block, 0, stream, ids, (const float*)table, x, H, V, scale);
     else if (table_dtype == TL_BF16)
@@ -189,21 +201,24 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict
     const R* rr = HAS_RES ? res + src * H : nullptr;
     O* orow = out + (size_t)r * H;
     const int n4 = H >> 2;
-    float4 v[NORM_VPT];
+    float4 v[NORM_VPT], gw[NORM_VPT];
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < NORM_VPT; ++i) {
         const int c4 = threadIdx.x + i * blockDim.x;
         if (c4 < n4) {
             float4 a = tl_load4(xr + 4 * c4);
+            gw[i] = tl_load4(w + 4 * c4);                    // used at the end
             if (HAS_RES) {
                 float4 b = tl_load4(rr + 4 * c4);
-                for (int p = 1; p < parts; ++p) {
-                    const float4 e = tl_load4(rr + 4 * c4 + p * pstride);
-                    b.x += e.x;
-                    b.y += e.y;
-                    b.z += e.z;
-                    b.w += e.w;
+                for (int p = 1; p < parts; p += 4) {         // four shares are asked for before they are added
+                    float4 e[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (p + k < parts) e[k] = tl_load4(rr + 4 * c4 + (p + k) * pstride);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (p + k < parts) b.x += e[k].x, b.y += e[k].y, b.z += e[k].z, b.w += e[k].w;
                 }
                 a.x += b.x;
                 a.y += b.y;
@@ -224,12 +239,11 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict
     for (int i = 0; i < NORM_VPT; ++i) {
         const int c4 = threadIdx.x + i * blockDim.x;
         if (c4 < n4) {
-            const float4 g = tl_load4(w + 4 * c4);
             float4 o;
-            o.x = v[i].x * rstd * g.x;
-            o.y = v[i].y * rstd * g.y;
-            o.z = v[i].z * rstd * g.z;
-            o.w = v[i].w * rstd * g.w;
+            o.x = v[i].x * rstd * gw[i].x;
+            o.y = v[i].y * rstd * gw[i].y;
+            o.z = v[i].z * rstd * gw[i].z;
+            o.w = v[i].w * rstd * gw[i].w;
             tl_store4(orow + 4 * c4, o);
         }
     }

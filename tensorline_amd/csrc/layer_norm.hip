@@ -32,9 +32,14 @@ __device__ __forceinline__ float ln_branch(const LnBranch& b, size_t i) {
 }
 __device__ __forceinline__ float4 ln_branch4(const LnBranch& b, size_t i) {
     float4 v = ln_load4(b.y + i);
-    for (int p = 1; p < b.parts; ++p) {
-        const float4 e = ln_load4(b.y + i + p * b.stride);
-        v.x += e.x, v.y += e.y, v.z += e.z, v.w += e.w;
+    for (int p = 1; p < b.parts; p += 4) {                   // four shares are asked for before they are added
+        float4 e[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (p + k < b.parts) e[k] = ln_load4(b.y + i + (p + k) * b.stride);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (p + k < b.parts) v.x += e[k].x, v.y += e[k].y, v.z += e[k].z, v.w += e[k].w;
     }
     return v;
 }
@@ -82,13 +87,14 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     const size_t src = rows ? (size_t)rows[r] : (size_t)r;
     float* xr = x + src * H;
     const int n4 = H >> 2;
-    float4 v[LN_VPT];
+    float4 v[LN_VPT], g[LN_VPT], s[LN_VPT];
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < LN_VPT; ++i) {
         const int c4 = threadIdx.x + i * blockDim.x;
         if (c4 < n4) {
             float4 a = ln_load4(xr + 4 * c4);
+            if (w) g[i] = ln_load4(w + 4 * c4), s[i] = ln_load4(b + 4 * c4);       // used at the end
             if (b1.y) {
                 float4 p = ln_branch4(b1, src * H + 4 * c4);
                 if (b2.y) {
@@ -121,12 +127,11 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     for (int i = 0; i < LN_VPT; ++i) {
         const int c4 = threadIdx.x + i * blockDim.x;
         if (c4 < n4) {
-            const float4 g = ln_load4(w + 4 * c4), s = ln_load4(b + 4 * c4);
             float4 o;
-            o.x = v[i].x * rstd * g.x + s.x;
-            o.y = v[i].y * rstd * g.y + s.y;
-            o.z = v[i].z * rstd * g.z + s.z;
-            o.w = v[i].w * rstd * g.w + s.w;
+            o.x = v[i].x * rstd * g[i].x + s[i].x;
+            o.y = v[i].y * rstd * g[i].y + s[i].y;
+            o.z = v[i].z * rstd * g[i].z + s[i].z;
+            o.w = v[i].w * rstd * g[i].w + s[i].w;
             ln_store4(orow + 4 * c4, o);
         }
     }

@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(const float* 
     const bool live = g < groups;
     const float* row = o + (size_t)t * ldo + (size_t)(live ? g : 0) * group;
     const float* grow = gate + (size_t)t * ldg + (size_t)(live ? g : 0) * group;
-    float4 v[4], z[4];
+    float4 v[4], z[4], weights[4];
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -193,6 +193,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(const float* 
         if (c < group) {
             v[i] = *reinterpret_cast<const float4*>(row + c);
             z[i] = *reinterpret_cast<const float4*>(grow + c);
+            weights[i] = *reinterpret_cast<const float4*>(weight + (size_t)(live ? g : 0) * group + c);
         }
     }
 #pragma unroll
@@ -202,13 +203,13 @@ __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(const float* 
         }
         ss += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
     }
-    for (int off = 1; off < (1 << lpg); off <<= 1) ss += __shfl_xor(ss, off, TL_WAVE);
+    ss = tl_group_sum(ss, lpg);
     const float rstd = 1.0f / sqrtf(ss / (float)group + eps);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int c = 4 * l + i * step;
         if (!live || c >= group) continue;
-        const float4 w = *reinterpret_cast<const float4*>(weight + (size_t)g * group + c);
+        const float4 w = weights[i];
         float r[4] = {v[i].x * rstd * w.x, v[i].y * rstd * w.y, v[i].z * rstd * w.z, v[i].w * rstd * w.w};
         const float zz[4] = {z[i].x, z[i].y, z[i].z, z[i].w};
         O* dst = out + (size_t)t * N + (size_t)g * group + c;
