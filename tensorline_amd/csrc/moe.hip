@@ -601,16 +601,33 @@ __global__ __launch_bounds__(MG_THREADS, 2) void moe_gemm_bf16_kernel(const bf16
 // their products took 543 and 304 us for gate and up and for down of 192 rows an expert (64 of 4,096 x 2,048) where this takes 427
 // and 270 (5.0 and 4.0 TB/s of matrices).
 // MW is the tile's rows in sixties-fours, chosen by the work-group, so that a tile of 70 rows does the products of 128.
-// The tiles of one expert, all its column tiles, go to one XCD (every eighth work-group id), whose L2 then holds the rows.
+// The tiles of one expert, all its column tiles, go to one XCD (every eighth work-group id), whose L2 then holds the rows; of the last tiles, that are
+// fewer than there are XCDs, every XCD takes its share of the column tiles: whole ones gave the XCDs that had one a round of work-groups
+// more (64 experts of 2,048 x 1,408, 64 to 67 tiles, 188 -> 169 us).
+// The matrix rows are asked for ahead of the tokens' rows, whose places have to be looked up.
 #define MGW_THREADS 512
 #define MGW_KT 64
 #define MGW_W 2048                       // 16-byte units of 256 matrix rows in a stage
 #define MGW_W_STAGES 3
 #define MGW_LDS (160 * 1024)
 
+// the token of a pair, pair / top, by the reciprocal ceil(2^32 / top) (0: top is 1): exact for fewer than 2^27 pairs
+__device__ __forceinline__ int moe_token(int pair, uint32_t per_top) { return per_top ? (int)__umulhi((uint32_t)pair, per_top) : pair; }
+// which row tile and column tile a work-group has; `whole` of the `have` row tiles are dealt out whole
+__device__ __forceinline__ bool moe_wide_tile(int id, int have, int whole, int ntiles, int* mt, int* nt) {
+    int local = id >> 3;
+    if (local < (whole >> 3) * ntiles) {
+        *mt = (local / ntiles) * 8 + (id & 7), *nt = local % ntiles;
+        return true;
+    }
+    local = (local - (whole >> 3) * ntiles) * 8 + (id & 7);
+    *mt = whole + local / ntiles, *nt = local % ntiles;
+    return *mt < have;
+}
+
 template <int MW, int MODE>
 __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ We, void* __restrict__ Cv, int ldc,
-                                         const int32_t* __restrict__ order, int place0, int rows, int expert, int n0, int top, int N, int K,
+                                         const int32_t* __restrict__ order, int place0, int rows, int expert, int n0, uint32_t per_top, int N, int K,
                                          float limit, float alpha, float shift, uint4* lds) {
     constexpr bool GLU = MODE == 1, BY_TOKEN = MODE != 0;
     constexpr int MB = 2 * MW, NB = 4, LA = MW, LB = 4;                          // blocks of a wave; loads per wave and step, 8 rows each
@@ -625,7 +642,7 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
         const int x = wave * LA + i, r = min(x * 8 + (lane >> 3), rows - 1);     // rows the tile does not have: its last one again
-        aoff[i] = (uint32_t)(BY_TOKEN ? order[place0 + r] / top : place0 + r) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ ((x & 1) * 4 + (lane >> 4)));
+        aoff[i] = (uint32_t)(BY_TOKEN ? moe_token(order[place0 + r], per_top) : place0 + r) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ ((x & 1) * 4 + (lane >> 4)));
     }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
@@ -690,15 +707,16 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
 template <int MODE>
 __global__ __launch_bounds__(MGW_THREADS, 2) void moe_gemm_wide_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
                                                                        void* __restrict__ C, int ldc, const int32_t* __restrict__ order,
-                                                                       const int32_t* __restrict__ tiles, int top, int N, int K,
+                                                                       const int32_t* __restrict__ tiles, uint32_t per_top, int N, int K,
                                                                        int ntiles, float limit, float alpha, float shift) {
     extern __shared__ uint4 mgw_lds[];
-    const int local = blockIdx.x >> 3, mt = (local / ntiles) * 8 + (blockIdx.x & 7), nt = local % ntiles;
-    if (mt >= tiles[0]) return;
+    const int have = tiles[0], whole = have & ~7;
+    int mt, nt;
+    if (!moe_wide_tile(blockIdx.x, have, whole, ntiles, &mt, &nt)) return;
     const int e = tiles[1 + 3 * mt], place0 = tiles[2 + 3 * mt], rows = tiles[3 + 3 * mt];
     const bf16_t* We = W + (size_t)e * (MODE == 1 ? 2 : 1) * N * K;
     const int n0 = nt * (MODE == 1 ? 128 : 256);
-#define GO(MW) mgw_tile<MW, MODE>(A, lda, We, C, ldc, order, place0, rows, e, n0, top, N, K, limit, alpha, shift, mgw_lds)
+#define GO(MW) mgw_tile<MW, MODE>(A, lda, We, C, ldc, order, place0, rows, e, n0, per_top, N, K, limit, alpha, shift, mgw_lds)
     if (rows <= 64) GO(1);
     else if (rows <= 128) GO(2);
     else if (rows <= 192) GO(3);
@@ -741,7 +759,7 @@ extern "C" int tl_moe_gemm(const void* A, int a_dtype, int lda, const void* W, i
         const int ntiles = tl_ceil_div(N, glu == 1 ? 128 : 256);
 #define GO_WIDE(MODE)                                                                                                      \
     hipLaunchKernelGGL(moe_gemm_wide_kernel<MODE>, dim3((unsigned)(tl_ceil_div(max_tiles, 8) * 8 * ntiles)), dim3(MGW_THREADS), \
-                       MGW_LDS, stream, (const bf16_t*)A, lda, (const bf16_t*)W, C, ldc, order, tiles, top, N, K, ntiles, limit, alpha, shift)
+                       MGW_LDS, stream, (const bf16_t*)A, lda, (const bf16_t*)W, C, ldc, order, tiles, (uint32_t)(((1ull << 32) + top - 1) / top), N, K, ntiles, limit, alpha, shift)
         if (glu == 1) GO_WIDE(1);
         else if (glu == 2) GO_WIDE(2);
         else GO_WIDE(0);

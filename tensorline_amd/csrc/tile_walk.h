@@ -40,11 +40,11 @@ __device__ __forceinline__ void tile_walk(int nsteps, tw_f32x4 (&acc)[MB][NB], L
     tw_bf16x8 a[2][MB], b[2][NB];
     if (AST == BST) {
 #pragma unroll
-        for (int i = 0; i < AST; ++i) { stage_a(i); stage_b(i); }
+        for (int i = 0; i < AST; ++i) { stage_b(i); stage_a(i); }
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AST - 1) * (LA + LB)) : "memory");
     } else {
-        stage_a(0), stage_b(0), stage_b(1), stage_a(1), stage_b(2);    // in the order the waits below count in
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + 2 * LB) : "memory");
+        stage_b(0), stage_b(1), stage_a(0), stage_a(1), stage_b(2);    // in the order the waits below count in
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + LB) : "memory");
     }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
