@@ -611,8 +611,11 @@ __global__ __launch_bounds__(MG_THREADS, 2) void moe_gemm_bf16_kernel(const bf16
 #define MGW_W_STAGES 3
 #define MGW_LDS (160 * 1024)
 
-// the token of a pair, pair / top, by the reciprocal ceil(2^32 / top) (0: top is 1): exact for fewer than 2^27 pairs
-__device__ __forceinline__ int moe_token(int pair, uint32_t per_top) { return per_top ? (int)__umulhi((uint32_t)pair, per_top) : pair; }
+// the token of a pair, pair / top, by the reciprocal ceil(2^32 / top) (0: top is 1), which is one too many at most
+__host__ __device__ __forceinline__ int moe_token(int pair, int top, uint32_t per_top) {
+    const uint32_t q = per_top ? (uint32_t)(((uint64_t)(uint32_t)pair * per_top) >> 32) : (uint32_t)pair;
+    return (int)(q - (q * (uint32_t)top > (uint32_t)pair));
+}
 // which row tile and column tile a work-group has; `whole` of the `have` row tiles are dealt out whole
 __device__ __forceinline__ bool moe_wide_tile(int id, int have, int whole, int ntiles, int* mt, int* nt) {
     int local = id >> 3;
@@ -627,7 +630,7 @@ __device__ __forceinline__ bool moe_wide_tile(int id, int have, int whole, int n
 
 template <int MW, int MODE>
 __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ We, void* __restrict__ Cv, int ldc,
-                                         const int32_t* __restrict__ order, int place0, int rows, int expert, int n0, uint32_t per_top, int N, int K,
+                                         const int32_t* __restrict__ order, int place0, int rows, int expert, int n0, int top, uint32_t per_top, int N, int K,
                                          float limit, float alpha, float shift, uint4* lds) {
     constexpr bool GLU = MODE == 1, BY_TOKEN = MODE != 0;
     constexpr int MB = 2 * MW, NB = 4, LA = MW, LB = 4;                          // blocks of a wave; loads per wave and step, 8 rows each
@@ -642,7 +645,7 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
         const int x = wave * LA + i, r = min(x * 8 + (lane >> 3), rows - 1);     // rows the tile does not have: its last one again
-        aoff[i] = (uint32_t)(BY_TOKEN ? moe_token(order[place0 + r], per_top) : place0 + r) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ ((x & 1) * 4 + (lane >> 4)));
+        aoff[i] = (uint32_t)(BY_TOKEN ? moe_token(order[place0 + r], top, per_top) : place0 + r) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ ((x & 1) * 4 + (lane >> 4)));
     }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
@@ -707,7 +710,7 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
 template <int MODE>
 __global__ __launch_bounds__(MGW_THREADS, 2) void moe_gemm_wide_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
                                                                        void* __restrict__ C, int ldc, const int32_t* __restrict__ order,
-                                                                       const int32_t* __restrict__ tiles, uint32_t per_top, int N, int K,
+                                                                       const int32_t* __restrict__ tiles, int top, uint32_t per_top, int N, int K,
                                                                        int ntiles, float limit, float alpha, float shift) {
     extern __shared__ uint4 mgw_lds[];
     const int have = tiles[0], whole = have & ~7;
@@ -716,7 +719,7 @@ __global__ __launch_bounds__(MGW_THREADS, 2) void moe_gemm_wide_kernel(const bf1
     const int e = tiles[1 + 3 * mt], place0 = tiles[2 + 3 * mt], rows = tiles[3 + 3 * mt];
     const bf16_t* We = W + (size_t)e * (MODE == 1 ? 2 : 1) * N * K;
     const int n0 = nt * (MODE == 1 ? 128 : 256);
-#define GO(MW) mgw_tile<MW, MODE>(A, lda, We, C, ldc, order, place0, rows, e, n0, per_top, N, K, limit, alpha, shift, mgw_lds)
+#define GO(MW) mgw_tile<MW, MODE>(A, lda, We, C, ldc, order, place0, rows, e, n0, top, per_top, N, K, limit, alpha, shift, mgw_lds)
     if (rows <= 64) GO(1);
     else if (rows <= 128) GO(2);
     else if (rows <= 192) GO(3);
@@ -759,7 +762,7 @@ extern "C" int tl_moe_gemm(const void* A, int a_dtype, int lda, const void* W, i
         const int ntiles = tl_ceil_div(N, glu == 1 ? 128 : 256);
 #define GO_WIDE(MODE)                                                                                                      \
     hipLaunchKernelGGL(moe_gemm_wide_kernel<MODE>, dim3((unsigned)(tl_ceil_div(max_tiles, 8) * 8 * ntiles)), dim3(MGW_THREADS), \
-                       MGW_LDS, stream, (const bf16_t*)A, lda, (const bf16_t*)W, C, ldc, order, tiles, (uint32_t)(((1ull << 32) + top - 1) / top), N, K, ntiles, limit, alpha, shift)
+                       MGW_LDS, stream, (const bf16_t*)A, lda, (const bf16_t*)W, C, ldc, order, tiles, top, (uint32_t)(((1ull << 32) + top - 1) / top), N, K, ntiles, limit, alpha, shift)
         if (glu == 1) GO_WIDE(1);
         else if (glu == 2) GO_WIDE(2);
         else GO_WIDE(0);

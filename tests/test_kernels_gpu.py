@@ -1354,6 +1354,23 @@ def test_experts_in_wide_tiles(gated, Kd, F, N, monkeypatch):
         assert bool(((got[True][rows].double() - want[rows]).abs() <= slack).all()), e
 
 
+@pytest.mark.parametrize("E,top,F,N", [(7, 1, 64, 260), (9, 3, 320, 768), (13, 2, 640, 516), (37, 33, 192, 1280)])
+def test_wide_tiles_that_are_no_multiple_of_the_xcds(E, top, F, N, monkeypatch):
+    """Row tiles of which fewer than eight are left over, alone or behind whole eights, with one to five column tiles and choices
+    of one to many: every tile once, bit for bit what tiles of 64 rows give."""
+    torch.manual_seed(E)
+    T, Kd = 190, 128
+    ids = torch.rand(T, E, device=DEV).topk(top, 1).indices.int().contiguous()
+    h, weights = torch.randn(T, Kd, device=DEV).to(torch.bfloat16), torch.rand(T, top, device=DEV)
+    up = (torch.randn(E, 2 * F, Kd, device=DEV) / 11).to(torch.bfloat16)
+    down = (torch.randn(E, N, F, device=DEV) / 16).to(torch.bfloat16)
+    got = {}
+    for wide in (True, False):
+        monkeypatch.setattr(K(), "_moe_takes_wide_tiles", lambda *a: wide)
+        got[wide] = K().moe_experts(h, up, down, ids, weights, 7.0, 1.0)
+    assert torch.equal(got[True], got[False])
+
+
 def test_a_large_stack_of_few_experts_takes_wide_tiles(monkeypatch):
     """Four experts of 4,096 x 1,024 have 32 wide tiles for 256 CUs and take them for their size: bit for bit what small tiles give."""
     torch.manual_seed(4)
