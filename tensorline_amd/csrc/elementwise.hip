@@ -454,56 +454,98 @@ extern "C" int tl_add_rmsnorm(float* x, const void* residual, int res_dtype, int
 //   out[i + rot/2] = b*cos(theta_i) + a*sin(theta_i)       theta_i = pos * inv_freq[i]
 // The angle, sine and cosine are float.  A negative slot skips the cache write of that token.
 // k_cache is [pages, page, nkv, d] (addressed as [slot, nkv, d]); v_cache is [pages, nkv, d, page].
+// One work-group a token.  In a step of a few hundred tokens it is a chain of waits (801 tokens of 12 + 2 + 2 heads of 128
+// are 6.6 MB): a thread asks for its first pairs and their bias ahead of the angles, the waves that have no angle copy the values
+// meanwhile, and a head's number is a multiplication by the reciprocal ceil(2^32 / pairs a head).
+// bfloat16, 12 + 2 + 2 heads of 128, us: 160 tokens 4.0 -> 3.0, 801 tokens 5.5 -> 4.3; 28 + 4 + 4 heads, 2,048 tokens 12.5 -> 10.4 (3.6 TB/s);
+// float32 8 tokens 5.0 -> 2.8.  A thread has one group of pairs wherever 1,024 threads are enough: with two the second was asked for
+// behind the angles (float32, 2,048 tokens of 28 + 4 + 4 heads 20.8 against 19.4).
 template <typename T>
-__global__ void rope_store_kernel(T* __restrict__ qkv, const int32_t* __restrict__ pos,
-                                  const float* __restrict__ inv_freq, T* __restrict__ k_cache, T* __restrict__ v_cache,
-                                  const int32_t* __restrict__ slots, int nq, int nkv, int d, int rot, int write_kv,
-                                  int bs, const float* __restrict__ bias, int vec8) {
-    __shared__ float cs_s[256], sn_s[256];          // one sine and cosine per rotated pair of the token
-    const int t = blockIdx.x;
-    const int half = rot / 2;
-    const float p = (float)pos[t];
-    const int slot = write_kv ? slots[t] : -1;
+__global__ __launch_bounds__(1024) void rope_store_kernel(T* __restrict__ qkv, const int32_t* __restrict__ pos,
+                                                         const float* __restrict__ inv_freq, T* __restrict__ k_cache, T* __restrict__ v_cache,
+                                                         const int32_t* __restrict__ slots, int nq, int nkv, int d, int rot, int write_kv,
+                                                         int bs, const float* __restrict__ bias, int vec, uint32_t per_head_rcp) {
+    constexpr int V = 16 / sizeof(T);               // pairs to a thread where the sizes allow 16-byte accesses (vec)
+    struct __attribute__((aligned(4))) Quad { float v[4]; };
+    __shared__ __attribute__((aligned(16))) float cs_s[256], sn_s[256];          // one sine and cosine per rotated pair of the token
+    const int t = blockIdx.x, half = rot / 2;
     T* row = qkv + (size_t)t * (nq + 2 * nkv) * d;
     const int nrot = nq + nkv;  // heads that are rotated: q then k
-    for (int i = threadIdx.x; i < half; i += blockDim.x) sincosf(p * inv_freq[i], &sn_s[i], &cs_s[i]);
-    __syncthreads();
-    // rotated pairs; bfloat16 with eight pairs to a thread where the sizes allow 16-byte accesses
-    if (vec8) {
-        if constexpr (sizeof(T) == 2) {
-            const int per_head = half >> 3;
-            for (int idx = threadIdx.x; idx < nrot * per_head; idx += blockDim.x) {
-                const int h = idx / per_head, i = (idx - h * per_head) * 8;
-                bf16_t* hp = reinterpret_cast<bf16_t*>(row) + (size_t)h * d;
-                const uint4 lo = *reinterpret_cast<const uint4*>(hp + i);
-                const uint4 hi = *reinterpret_cast<const uint4*>(hp + i + half);
-                const uint32_t lw[4] = {lo.x, lo.y, lo.z, lo.w}, hw[4] = {hi.x, hi.y, hi.z, hi.w};
-                uint32_t o1[4], o2[4];
+    const int per_head = vec ? half / V : half, items = nrot * per_head;
+    const auto head_of = [&](int idx) {             // (the product with the rounded reciprocal is one too many at most)
+        const uint32_t q = per_head_rcp ? __umulhi((uint32_t)idx, per_head_rcp) : (uint32_t)idx;
+        return (int)(q - (q * (uint32_t)per_head > (uint32_t)idx));
+    };
+    uint4 lo, hi;
+    Quad blo[V / 4], bhi[V / 4];
+    const auto ask = [&](int h, int i) {
+        const T* hp = row + (size_t)h * d + i;
+        lo = *reinterpret_cast<const uint4*>(hp), hi = *reinterpret_cast<const uint4*>(hp + half);
+        if (bias) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    float a0 = __uint_as_float(lw[k] << 16), a1 = __uint_as_float(lw[k] & 0xffff0000u);
-                    float b0 = __uint_as_float(hw[k] << 16), b1 = __uint_as_float(hw[k] & 0xffff0000u);
-                    if (bias) {
-                        a0 += bias[h * d + i + 2 * k], a1 += bias[h * d + i + 2 * k + 1];
-                        b0 += bias[h * d + i + half + 2 * k], b1 += bias[h * d + i + half + 2 * k + 1];
-                    }
-                    const float c0 = cs_s[i + 2 * k], c1 = cs_s[i + 2 * k + 1];
-                    const float s0 = sn_s[i + 2 * k], s1 = sn_s[i + 2 * k + 1];
-                    o1[k] = tl_pack_bf16(a0 * c0 - b0 * s0, a1 * c1 - b1 * s1);
-                    o2[k] = tl_pack_bf16(b0 * c0 + a0 * s0, b1 * c1 + a1 * s1);
+            for (int k = 0; k < V / 4; ++k) {
+                blo[k] = *reinterpret_cast<const Quad*>(bias + (size_t)h * d + i + 4 * k);
+                bhi[k] = *reinterpret_cast<const Quad*>(bias + (size_t)h * d + i + half + 4 * k);
+            }
+        }
+    };
+    int h = 0, i = 0;
+    if (vec) {
+        const int idx = min((int)threadIdx.x, items - 1);
+        h = head_of(idx), i = (idx - h * per_head) * V;
+        ask(h, i);
+    }
+    const int slot = write_kv ? slots[t] : -1;
+    const float p = (float)pos[t];
+    const int busy = (half + 63) & ~63, spare = busy < (int)blockDim.x ? busy : 0;   // threads in waves with angles
+    for (int k = threadIdx.x; k < half; k += blockDim.x) sincosf(p * inv_freq[k], &sn_s[k], &cs_s[k]);
+    if (slot >= 0 && (int)threadIdx.x >= spare) {
+        const T* vrow = row + (size_t)nrot * d;
+        const float* vbias = bias ? bias + (size_t)nrot * d : nullptr;
+        const int page = slot / bs, off = slot - page * bs;
+        T* vdst = v_cache + (size_t)page * nkv * d * bs + off;
+        for (int idx = threadIdx.x - spare; idx < nkv * d; idx += blockDim.x - spare)
+            vdst[(size_t)idx * bs] = vbias ? tl_from_float<T>(tl_to_float(vrow[idx]) + vbias[idx]) : vrow[idx];
+    }
+    __syncthreads();
+    if (vec) {
+        for (int idx = threadIdx.x; idx < items; idx += blockDim.x) {
+            if (idx != (int)threadIdx.x) h = head_of(idx), i = (idx - h * per_head) * V, ask(h, i);
+            T* dst = h < nq ? row + (size_t)h * d : k_cache + ((size_t)slot * nkv + (h - nq)) * d;
+            if (h >= nq && slot < 0) continue;
+            float cs[V], sn[V], o1[V], o2[V];
+#pragma unroll
+            for (int k = 0; k < V; k += 4) {
+                *reinterpret_cast<float4*>(cs + k) = *reinterpret_cast<const float4*>(cs_s + i + k);
+                *reinterpret_cast<float4*>(sn + k) = *reinterpret_cast<const float4*>(sn_s + i + k);
+            }
+            const uint32_t lw[4] = {lo.x, lo.y, lo.z, lo.w}, hw[4] = {hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+            for (int k = 0; k < V; ++k) {
+                float a, b;
+                if constexpr (sizeof(T) == 2) {
+                    a = __uint_as_float(k & 1 ? lw[k / 2] & 0xffff0000u : lw[k / 2] << 16);
+                    b = __uint_as_float(k & 1 ? hw[k / 2] & 0xffff0000u : hw[k / 2] << 16);
+                } else {
+                    a = __uint_as_float(lw[k]), b = __uint_as_float(hw[k]);
                 }
-                bf16_t* dst = hp;
-                if (h >= nq) {
-                    if (slot < 0) continue;
-                    dst = reinterpret_cast<bf16_t*>(k_cache) + ((size_t)slot * nkv + (h - nq)) * d;
-                }
-                *reinterpret_cast<uint4*>(dst + i) = make_uint4(o1[0], o1[1], o1[2], o1[3]);
-                *reinterpret_cast<uint4*>(dst + i + half) = make_uint4(o2[0], o2[1], o2[2], o2[3]);
+                if (bias) a += blo[k / 4].v[k % 4], b += bhi[k / 4].v[k % 4];
+                o1[k] = a * cs[k] - b * sn[k];
+                o2[k] = b * cs[k] + a * sn[k];
+            }
+            if constexpr (sizeof(T) == 2) {
+                *reinterpret_cast<uint4*>(dst + i) =
+                    make_uint4(tl_pack_bf16(o1[0], o1[1]), tl_pack_bf16(o1[2], o1[3]), tl_pack_bf16(o1[4], o1[5]), tl_pack_bf16(o1[6], o1[7]));
+                *reinterpret_cast<uint4*>(dst + i + half) =
+                    make_uint4(tl_pack_bf16(o2[0], o2[1]), tl_pack_bf16(o2[2], o2[3]), tl_pack_bf16(o2[4], o2[5]), tl_pack_bf16(o2[6], o2[7]));
+            } else {
+                *reinterpret_cast<float4*>(dst + i) = make_float4(o1[0], o1[1], o1[2], o1[3]);
+                *reinterpret_cast<float4*>(dst + i + half) = make_float4(o2[0], o2[1], o2[2], o2[3]);
             }
         }
     } else
-    for (int idx = threadIdx.x; idx < nrot * half; idx += blockDim.x) {
-        const int h = idx / half, i = idx - h * half;
+    for (int idx = threadIdx.x; idx < items; idx += blockDim.x) {
+        const int h = head_of(idx), i = idx - h * half;
         const float sn = sn_s[i], cs = cs_s[i];
         T* hp = row + (size_t)h * d;
         float a = tl_to_float(hp[i]), b = tl_to_float(hp[i + half]);
@@ -524,6 +566,7 @@ __global__ void rope_store_kernel(T* __restrict__ qkv, const int32_t* __restrict
     }
     // dims beyond the rotated part pass through: query dims only change when a bias is owed
     const int tail = d - rot;
+    if (!tail) return;
     if (bias) {
         for (int idx = threadIdx.x; idx < nq * tail; idx += blockDim.x) {
             const int h = idx / tail, i = rot + (idx - h * tail);
@@ -536,13 +579,6 @@ __global__ void rope_store_kernel(T* __restrict__ qkv, const int32_t* __restrict
         const T v = row[(size_t)(nq + h) * d + i];
         k_cache[((size_t)slot * nkv + h) * d + i] = bias ? tl_from_float<T>(tl_to_float(v) + bias[(nq + h) * d + i]) : v;
     }
-    // values
-    const T* vrow = row + (size_t)(nq + nkv) * d;
-    const float* vbias = bias ? bias + (size_t)(nq + nkv) * d : nullptr;
-    const int page = slot / bs, off = slot - page * bs;
-    T* vdst = v_cache + (size_t)page * nkv * d * bs + off;
-    for (int idx = threadIdx.x; idx < nkv * d; idx += blockDim.x)
-        vdst[(size_t)idx * bs] = vbias ? tl_from_float<T>(tl_to_float(vrow[idx]) + vbias[idx]) : vrow[idx];
 }
 
 extern "C" int tl_rope_store(void* qkv, int dtype, const int32_t* pos, const float* inv_freq, void* k_cache,
@@ -553,16 +589,21 @@ extern "C" int tl_rope_store(void* qkv, int dtype, const int32_t* pos, const flo
     TL_CHECK_ARG(rot <= 512, "tl_rope_store: rotary width %d is above the supported 512", rot);
     TL_CHECK_ARG(!write_kv || (k_cache && v_cache && slots && bs > 0), "tl_rope_store: cache write asked for without a cache");
     if (T == 0) return 0;
-    dim3 grid(T), block(256);
-    // 16-byte accesses: every head and both halves of the rotated part start at a multiple of 8 values
-    const int vec8 = dtype == TL_BF16 && d % 8 == 0 && rot % 16 == 0 && rot > 0 && ((uintptr_t)qkv % 16) == 0 &&
-                     (!write_kv || ((uintptr_t)k_cache % 16) == 0);
+    dim3 grid(T);
+    // 16-byte accesses: every head and both halves of the rotated part start at a multiple of 8 (float: 4) values
+    const int V = dtype == TL_BF16 ? 8 : 4;
+    const int vec = d % V == 0 && rot % (2 * V) == 0 && rot > 0 && ((uintptr_t)qkv % 16) == 0 &&
+                    (!write_kv || ((uintptr_t)k_cache % 16) == 0);
+    const int per_head = rot ? (vec ? rot / 2 / V : rot / 2) : 1;
+    const uint32_t rcp = (uint32_t)(((1ull << 32) + per_head - 1) / per_head);      // 0: one a head
+    const int items = (nq + nkv) * per_head;
+    const dim3 block(items <= 256 ? 256 : items <= 512 ? 512 : 1024);               // one item a thread: the first is asked for ahead
     if (dtype == TL_F32)
         hipLaunchKernelGGL(rope_store_kernel<float>, grid, block, 0, stream, (float*)qkv, pos, inv_freq,
-                           (float*)k_cache, (float*)v_cache, slots, nq, nkv, d, rot, write_kv, bs, bias, 0);
+                           (float*)k_cache, (float*)v_cache, slots, nq, nkv, d, rot, write_kv, bs, bias, vec, rcp);
     else if (dtype == TL_BF16)
         hipLaunchKernelGGL(rope_store_kernel<bf16_t>, grid, block, 0, stream, (bf16_t*)qkv, pos, inv_freq,
-                           (bf16_t*)k_cache, (bf16_t*)v_cache, slots, nq, nkv, d, rot, write_kv, bs, bias, vec8);
+                           (bf16_t*)k_cache, (bf16_t*)v_cache, slots, nq, nkv, d, rot, write_kv, bs, bias, vec, rcp);
     else
         return tl_fail("tl_rope_store: unknown dtype %d", dtype);
     TL_CHECK_LAUNCH("tl_rope_store");

@@ -530,6 +530,38 @@ def test_rope_store(dtype, nq, nkv, d, rot):
             torch.testing.assert_close(a.float(), b.float(), atol=3e-2, rtol=3e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nq,nkv,d,rot,shift", [
+    (7, 1, 16, 16, 0), (3, 1, 8, 8, 0), (30, 2, 128, 128, 0),      # one pair group a head; as many as 256 threads and their half
+    (31, 2, 128, 128, 1), (60, 8, 120, 120, 0),                    # one head more, a bias at 4 bytes; groups that no power of two counts
+    (33, 2, 512, 512, 0), (3, 1, 512, 512, 3),                     # more groups than a work-group has threads; every wave has an angle
+    (5, 2, 40, 12, 0), (9, 3, 37, 2, 1),                           # single pairs with dims that pass through
+])
+def test_rope_store_in_groups_of_pairs(dtype, nq, nkv, d, rot, shift):
+    """Pairs by the 16 bytes and one by one, at the numbers of threads a token gets: against the rotation in float64."""
+    torch.manual_seed(d)
+    T, bs, width = 5, 8, (nq + 2 * nkv) * d
+    qkv, bias = torch.randn(T, width, device=DEV).to(dtype), torch.randn(width + shift, device=DEV)[shift:]
+    pos, slots = torch.tensor([0, 1, 77, 900, 1500], dtype=torch.int32, device=DEV), torch.tensor([3, 15, -1, 0, 9], dtype=torch.int32, device=DEV)
+    inv = (10000.0 ** (-torch.arange(0, rot, 2, dtype=torch.float64) / rot)).float().to(DEV)
+    x = (qkv.double() + bias.double()).view(T, nq + 2 * nkv, d)
+    theta = (pos.float()[:, None] * inv).double()[:, None]         # (the angle is a float32 product)
+    a, b, heads = x[:, :nq + nkv, :rot // 2], x[:, :nq + nkv, rot // 2:rot], x.clone()
+    heads[:, :nq + nkv, :rot // 2], heads[:, :nq + nkv, rot // 2:rot] = a * theta.cos() - b * theta.sin(), b * theta.cos() + a * theta.sin()
+    kc, vc = torch.full((2, bs, nkv, d), 7.0, device=DEV).to(dtype), torch.full((2, nkv, d, bs), 7.0, device=DEV).to(dtype)
+    K().rope_store(qkv, pos, inv, nq, nkv, d, kc, vc, slots, bias)
+    keys, values = kc.double().view(-1, nkv, d), vc.double().permute(0, 3, 1, 2).reshape(-1, nkv, d)
+    # of values up to 12: a sum with the bias, two products, their sum and a sine rounded in float32, and one rounding of the result
+    t = dict(atol=12 * 8 * 2.0 ** -24, rtol=2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22)
+    torch.testing.assert_close(qkv.double().view(T, -1, d)[:, :nq], heads[:, :nq], **t)
+    for t_, s in enumerate(slots.tolist()):
+        if s >= 0:
+            torch.testing.assert_close(keys[s], heads[t_, nq:nq + nkv], **t)
+            torch.testing.assert_close(values[s], heads[t_, nq + nkv:], **t)
+    left = [s for s in range(2 * bs) if s not in slots.tolist()]
+    assert bool((keys[left] == 7).all()) and bool((values[left] == 7).all())
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 17, 40, 64])
 @pytest.mark.parametrize("nq,nkv,d,Kd", [(6, 2, 32, 192), (28, 4, 128, 3584), (4, 4, 64, 264), (5, 1, 96, 120)])
 def test_fused_projection_rotation_and_cache_write(M, nq, nkv, d, Kd):
