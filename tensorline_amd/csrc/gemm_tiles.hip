@@ -10,6 +10,10 @@
 // compiler moves accumulators back and forth).  The rows of A (128 bytes a step) have their eight 16-byte units at
 // unit ^ (row / 2) % 8, so that the sixteen lanes that are served together hit all banks; W's pieces are read as they lie.
 //
+// Tile 7 has W's fragments go from memory into registers (four waves of 128 x 64, 232 registers, two work-groups to a CU): only the rows pass
+// through LDS, 96 KB of a step's traffic there for the 176 KB of tile 2, and one work-group's start and end pass beside the other's
+// products.  It is the gated form's, whose results of some thousand columns are many tiles.
+//
 // Tiles are dealt to the XCDs in runs (work-group id modulo 8), rows fastest within panels of 2,048 rows: an XCD walks a few
 // tiles of W against all rows and its L2 holds both.
 //
@@ -17,8 +21,8 @@
 // takes them or by gt_add_kernel.
 //
 // us, here and in the library with its own choice of kernel (gate/up with the SiLU pass it needs; weights from memory), of sizes that
-// are taken (tl_gemm_tiles_plan): 2,048 rows of 17,920 x 1,536 gate/up 131 and 141, of 9,728 x 896 52 and 66, of 1,536 x 8,960 52 and 90;
-// 801 rows of 17,920 x 1,536 gate/up 57 and 69, of 1,536 x 8,960 30 and 44, of 2,048 x 1,536 15 and 18; 192 rows of the same 27
+// are taken (tl_gemm_tiles_plan): 2,048 rows of 17,920 x 1,536 gate/up 111 and 141, of 9,728 x 896 52 and 66, of 1,536 x 8,960 52 and 90;
+// 801 rows of 17,920 x 1,536 gate/up 51 and 69, of 1,536 x 8,960 30 and 44, of 2,048 x 1,536 15 and 18; 192 rows of the same 27
 // and 33, 16 and 38, 11 and 11; 128 rows of 37,888 x 3,584 gate/up 70 and 74, of 3,584 x 18,944 37 and 54, of 3,584 x 3,584 17 and 25.
 // Alone, plain products of 2^20 to 2^23 results and a K of 2,048 to 4,096 are 4% slower here in the mean, 20% at most (640 rows of
 // 2,048 x 2,816 23 and 20; 1,521 of 1,024 x 3,072 25 and 21); in whole steps the library is level there, and slower where the host
@@ -43,7 +47,7 @@ __device__ __forceinline__ float gt_gate(float v, int act) {
 // GLU: W has the N / 2 gate rows, then the N / 2 up rows, and C = act(gate) * up [M, N / 2]; a wave's first NB / 2 blocks are gate
 // columns, the others the up columns of the same places.
 template <int WM, int WN, int MB, int NB, int AST, int BST, bool GLU, typename TO>
-__global__ __launch_bounds__(64 * WM * WN, MB * NB >= 16 ? 2 : 4) void gemm_tiles_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
+__global__ __launch_bounds__(64 * WM * WN, MB * NB >= 16 || !BST ? 2 : 4) void gemm_tiles_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
                                                                                   GtOut out, int M, int N, int K, int mtiles, int ntiles, int shares) {
     constexpr int WAVES = WM * WN, BM = 16 * WM * MB, BN = 16 * WN * NB;
     constexpr int A_UNITS = BM * 8, B_UNITS = BN * 8;                  // 16-byte units of a stage
@@ -85,6 +89,29 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB >= 16 ? 2 : 4) void gemm_tile
     const int afrag = (wm * MB * 16 + c) * 8 + (g ^ (c >> 1)), bfrag = wn * NB * 128 + lane;
     int na = 0, nb = 0;
     tw_f32x4 acc[MB][NB];
+    if constexpr (BST == 0) {
+        static_assert(WM == 1 && AST == 4, "W from memory into registers");
+        // (voff is the lane's place in a piece; the scalar offsets are those of the wave's column tiles)
+        const __amdgpu_buffer_rsrc_t w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(W), 0, (int)((uint32_t)ctiles * (uint32_t)chunks * 1024u), 0x00027000);
+        uint32_t toff[NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            const int tile = GLU ? min(tile0 + wn * (NB / 2) + j % (NB / 2), half - 1) + (j >= NB / 2 ? half : 0) : min(tile0 + wn * NB + j, ctiles - 1);
+            toff[j] = ((uint32_t)tile * (uint32_t)chunks + 2 * s0) * 1024u;
+        }
+        tile_walk_direct<MB, NB, LA>(
+            nsteps, acc, lane * 16u, [&](int buf, int i, uint32_t& token) { tw_load_token(aoff[i], ab, la + buf * (A_UNITS * 16) + i * 1024, token); },
+            [&](int x, uint32_t token) {
+                return __builtin_bit_cast(tw_bf16x8, __builtin_amdgcn_raw_buffer_load_b128(w, (int)(token + x / NB * 1024), (int)toff[x % NB], 0));
+            },
+            [&]() { if (++na < nsteps) ab += GT_KT * 2; },
+            [&]() {
+                const uint32_t on = ++nb < nsteps ? 2048u : 0u;
+#pragma unroll
+                for (int j = 0; j < NB; ++j) toff[j] += on;
+            },
+            [&](int buf, int h, int i) { return __builtin_bit_cast(tw_bf16x8, lds_a[buf * A_UNITS + (afrag ^ (4 * h)) + i * 128]); });
+    } else
     tile_walk<MB, NB, AST, BST, LA, LB>(
         nsteps, acc, [&](int buf, int i) { tw_load(aoff[i], ab, la + buf * (A_UNITS * 16) + i * 1024); },
         [&](int buf, int i) { tw_load(boff[i], bb, lb + buf * (B_UNITS * 16) + i * 1024); }, [&]() { if (++na < nsteps) ab += GT_KT * 2; },
@@ -152,7 +179,7 @@ __global__ __launch_bounds__(256) void gt_add_kernel(const float* __restrict__ p
 // 1 to 12 shares, with weights from memory (those that the last-level cache holds give other times and other choices): half of the
 // 3,600 times are within 5%, and the choice by them takes 0.8% longer than the best one in the mean (0.75 of the library's time; at
 // worst, 192 rows of 4,096 x 12,288, 38 us where the best takes 34 and the library 32).
-//    id  waves  blocks stages a CU holds  step alone, beside a second; start and end
+//    id  waves  blocks stages (0: registers) a CU holds  step alone, beside a second; start and end
 #define GT_TILES(X)                                  \
     X(0, 2, 4, 8, 4, 2, 3, 1, 1.072, 1.072, 4.22)    \
     X(1, 2, 4, 8, 3, 2, 3, 1, 0.854, 0.854, 3.94)    \
@@ -160,17 +187,19 @@ __global__ __launch_bounds__(256) void gt_add_kernel(const float* __restrict__ p
     X(3, 2, 4, 4, 2, 2, 3, 2, 0.584, 0.785, 1.46)    \
     X(4, 2, 4, 2, 2, 3, 3, 2, 0.407, 0.649, 0.95)    \
     X(5, 4, 2, 1, 2, 5, 5, 2, 0.224, 0.406, 0.99)    \
-    X(6, 2, 4, 6, 4, 2, 3, 1, 0.931, 0.931, 3.72)
+    X(6, 2, 4, 6, 4, 2, 3, 1, 0.931, 0.931, 3.72)    \
+    X(7, 1, 4, 8, 4, 4, 0, 2, 0.670, 1.153, 3.72)
 struct GtTile {
     int bm, bn, lds, per_cu;
-    bool pairs;                // the gated form: whole blocks of gate and of up columns in a wave
+    bool pairs, direct;        // the gated form: whole blocks of gate and of up columns in a wave; W straight into registers
     double step1, step2, ends;
 };
 #define X(ID, WM, WN, MB, NB, AST, BST, CU, T1, T2, ENDS) \
-    {16 * WM * MB, 16 * WN * NB, (16 * WM * MB * AST + 16 * WN * NB * BST) * 128, CU, NB % 2 == 0, T1, T2, ENDS},
+    {16 * WM * MB, 16 * WN * NB, (16 * WM * MB * AST + 16 * WN * NB * BST) * 128, CU, NB % 2 == 0, BST == 0, T1, T2, ENDS},
 static const GtTile gt_tiles[] = {GT_TILES(X)};
 #undef X
-#define GT_TILE_COUNT 7
+#define GT_TILE_COUNT 8
+#define GT_DIRECT 7
 #define GT_MAX_SHARES 12
 
 static int gt_ntiles(const GtTile& t, int N, bool gated) { return gated ? tl_ceil_div(N / 2, t.bn / 2) : tl_ceil_div(N, t.bn); }
@@ -194,6 +223,18 @@ static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shar
     return us;
 }
 
+// Whether the gated form of a product cut into tiles of t runs in tiles of 128 x 256 with W straight into registers, two to a CU: where
+// there are more of them than CUs and the formula has them ahead.  Their figures are a fit to gated products of such sizes, 7% under
+// their times as the formula is under those of several rounds in the other tiles.  46 sizes that take them (of 9,728 x 896 to
+// 37,888 x 3,584, weights from memory) are 1.00 to 1.16 times as fast as in the plan's tile, 1.06 in the mean: us, 801 rows of 17,920 x
+// 1,536 55 and 51, 2,048 127 and 111, 380 rows of 37,888 x 3,584 115 and 107, 1,600 of 11,008 x 2,048 85 and 80; sizes that do not:
+// 1,300 rows of 17,920 x 1,536 69 and 79, 513 34 and 44, 1,521 of 9,728 x 896 30 and 32.  Plain products of up to 3,000 rows with a
+// choice of shares were level at best (256 tiles) or slower (384 tiles 28 and 36), and have no such form.
+static bool gt_goes_direct(const GtTile& t, const GtTile& direct, int M, int N, int K) {
+    return !t.direct && (double)tl_ceil_div(M, direct.bm) * gt_ntiles(direct, N, true) > 256 &&
+           gt_time(direct, M, N, K, true, 1, false) < gt_time(t, M, N, K, true, 1, false);
+}
+
 // The tile and the number of shares for a product (shares * 256 + tile), or -1: not one this file takes.
 // More than 512 rows of a matrix that is large both ways stay in the library (us, library and here in the best tile):
 // - plain products are level in sum: 513, 801 and 2,048 rows of 4,608 x 3,584 31, 39, 62 and 36, 40, 66; of 3,584 x 3,584 28, 34, 55 and
@@ -210,7 +251,7 @@ extern "C" int tl_gemm_tiles_plan(int M, int N, int K, int gated, int takes_shar
     double least = 0.0;
     for (int i = 0; i < GT_TILE_COUNT; ++i) {
         const GtTile& t = gt_tiles[i];
-        if (gated && !t.pairs) continue;
+        if (t.direct || (gated && !t.pairs)) continue;
         const double plane = (double)tl_ceil_div(M, t.bm) * gt_ntiles(t, N, gated);
         for (int shares = 1; shares <= (gated ? 1 : GT_MAX_SHARES); ++shares) {
             if (shares > 1 && (K / GT_KT / shares < 4 || plane * shares > 1.35 * 256 * t.per_cu)) break;
@@ -233,10 +274,12 @@ extern "C" int tl_gemm_tiles(const void* A, const void* W, const float* bias, vo
                      (C || shares > 1),
                  "tl_gemm_tiles: tile %d in %d shares", tile, shares);
     TL_CHECK_ARG((double)N * K * 2.0 < 4e9 && (double)lda * 512.0 < 4e9, "tl_gemm_tiles: N=%d K=%d lda=%d are beyond 32-bit offsets", N, K, lda);
+    TL_CHECK_ARG(gated || !gt_tiles[tile].direct, "tl_gemm_tiles: tile %d serves the gated form", tile);
     TL_CHECK_ARG(!gated || (c_dtype == TL_BF16 && !bias && gt_tiles[tile].pairs), "tl_gemm_tiles: the gated form stores bfloat16, without bias, in tiles of whole pairs");
     TL_CHECK_ARG((gated && (act == 0 || act == 2)) || (!gated && (act == 0 || act == 1)), "tl_gemm_tiles: activation %d is not one this product applies", act);
     TL_CHECK_ARG(!C || (ldc >= (gated ? N / 2 : N) && ldc % 4 == 0 && (uintptr_t)C % (c_dtype == TL_F32 ? 16 : 8) == 0 && (c_dtype == TL_F32 || c_dtype == TL_BF16)),
                  "tl_gemm_tiles: bad output");
+    if (gated && gt_goes_direct(gt_tiles[tile], gt_tiles[GT_DIRECT], M, N, K)) tile = GT_DIRECT;
     const GtTile& t = gt_tiles[tile];
     const int mtiles = tl_ceil_div(M, t.bm), ntiles = gt_ntiles(t, N, gated);
     TL_CHECK_ARG((double)mtiles * ntiles * shares < 2e9, "tl_gemm_tiles: too many tiles");
@@ -249,8 +292,10 @@ extern "C" int tl_gemm_tiles(const void* A, const void* W, const float* bias, vo
 #define X(ID, WM, WN, MB, NB, AST, BST, CU, T1, T2, ENDS)                      \
     case ID:                                                                   \
         if (gated) GO(WM, WN, MB, (NB % 2 ? NB + 1 : NB), AST, BST, true, bf16_t); \
-        else if (shares > 1 || c_dtype == TL_F32) GO(WM, WN, MB, NB, AST, BST, false, float); \
-        else GO(WM, WN, MB, NB, AST, BST, false, bf16_t);                      \
+        else if constexpr (BST != 0) {                                         \
+            if (shares > 1 || c_dtype == TL_F32) GO(WM, WN, MB, NB, AST, BST, false, float); \
+            else GO(WM, WN, MB, NB, AST, BST, false, bf16_t);                  \
+        }                                                                      \
         break;
     switch (tile) { GT_TILES(X) }
 #undef X

@@ -101,10 +101,84 @@ __device__ __forceinline__ void tile_walk(int nsteps, tw_f32x4 (&acc)[MB][NB], L
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may land in LDS that is no longer this work-group's
 }
 
+// The same walk with W's fragments straight from memory into the registers they are multiplied from: only the rows go through LDS,
+// which four waves of 128 x 64 side by side then read 64 KB of a step.  A's stages are four, W's are two steps of registers; a half's
+// registers are asked for again, two steps ahead, behind the products that used them.
+// load_b(piece, token): W's fragment j of half h of the step that next_b counts (piece = 4 h + j), asked for behind all loads of A that gave `token`.
+// How a stage of A is waited for: loads return in order, and W's fragments of half 1 of step s are asked for behind A's pieces of
+// step s + 1, which the token that goes from those loads into these addresses makes sure of.  To have the one is to have the other,
+// so a wave that has its fragments in registers (the empty asm reads them) may go to the barrier.
+template <int MB, int NB, int LA, typename LoadA, typename LoadB, typename NextA, typename NextB, typename ReadA>
+__device__ __forceinline__ void tile_walk_direct(int nsteps, tw_f32x4 (&acc)[MB][NB], uint32_t token, LoadA load_a, LoadB load_b, NextA next_a, NextB next_b,
+                                                 ReadA read_a) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = (tw_f32x4){0.f, 0.f, 0.f, 0.f};
+    constexpr int AHEAD = MB / 2;            // fragments of A read ahead
+    tw_bf16x8 a[AHEAD], b[2][2][NB];
+    auto ask_a = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LA; ++i) load_a(buf, i, token);
+        next_a();
+    };
+    auto ask_b = [&](auto set, auto half) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) b[decltype(set)::value][decltype(half)::value][j] = load_b(decltype(half)::value * NB + j, token);
+    };
+    auto here = [&](auto set, auto half) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) asm volatile("" ::"v"(b[decltype(set)::value][decltype(half)::value][j]) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    constexpr std::integral_constant<int, 0> _0;
+    constexpr std::integral_constant<int, 1> _1;
+    ask_a(0), ask_b(_0, _0), ask_a(1), ask_b(_0, _1), next_b(), ask_b(_1, _0), ask_a(2), ask_b(_1, _1), next_b();
+    here(_0, _0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) a[i] = read_a(0, 0, i);
+    int buf = 0;
+    auto step = [&](auto set) {
+        constexpr int S = decltype(set)::value;
+        const int next = (buf + 1) & 3;
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[S][0][j], a[i % AHEAD], acc[i][j], 0, 0, 0);
+            a[i % AHEAD] = i < MB - AHEAD ? read_a(buf, 0, i + AHEAD) : read_a(buf, 1, i + AHEAD - MB);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        ask_b(set, _0);
+        __builtin_amdgcn_sched_barrier(0);
+        here(set, _1);                       // and so are the rows of the next step; nobody reads those of the step before this one
+        ask_a((buf + 3) & 3);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[S][1][j], a[i % AHEAD], acc[i][j], 0, 0, 0);
+            a[i % AHEAD] = i < MB - AHEAD ? read_a(buf, 1, i + AHEAD) : read_a(next, 0, i + AHEAD - MB);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        ask_b(set, _1);
+        next_b();
+        __builtin_amdgcn_sched_barrier(0);
+        buf = next;
+    };
+    int s = 0;
+    for (; s + 2 <= nsteps; s += 2) step(_0), step(_1);
+    if (s < nsteps) step(_0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // nothing may land in LDS that is no longer this work-group's
+}
+
 // 16 bytes a lane from sbase + voff into LDS at lds_base + 16 * lane (lds_base is the same for the whole wave); tw_load_once: read
 // once, leaving no trace in the caches
 __device__ __forceinline__ void tw_load(uint32_t voff, const void* sbase, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sbase) : "memory", "m0");
+}
+// the same, with a token that goes through the load: what is computed from it comes behind
+__device__ __forceinline__ void tw_load_token(uint32_t voff, const void* sbase, uint32_t lds_base, uint32_t& token) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" : "+v"(token) : "s"(lds_base), "v"(voff), "s"(sbase) : "memory", "m0");
 }
 __device__ __forceinline__ void tw_load_once(uint32_t voff, const void* sbase, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(voff), "s"(sbase) : "memory", "m0");

@@ -182,6 +182,19 @@ def test_many_row_product_beyond_one_panel(tile, Kd):
         assert bool(((got.double() - fn(gate) * up).abs() <= _gate_error(gate, up, err[:, :I], err[:, I:], fn)).all())
 
 
+@pytest.mark.parametrize("M,I,Kd", [(1, 16, 64), (65, 144, 128), (127, 128, 192), (128, 272, 256), (129, 112, 320), (257, 400, 832), (2200, 48, 448)])
+def test_gated_product_with_the_matrix_in_registers(M, I, Kd):
+    """Tiles whose matrix goes straight into registers, from one step of K to fewer and more than are under way, at the edges of rows
+    and of columns, rows with a stride: bit for bit what tiles of the same rows with the matrix in LDS give (every sum is
+    of the same order)."""
+    torch.manual_seed(Kd)
+    a = torch.randn(M, Kd + 8, device=DEV).to(torch.bfloat16)[:, :Kd]
+    sh = K().shuffle_weight((torch.randn(2 * I, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16))
+    for act in (0, 2):
+        got, want = (K()._tiles(a, sh, None, torch.bfloat16, M, 2 * I, Kd, a.stride(0), 256 + tile, gated=True, act=act) for tile in (7, 2))
+        assert bool(torch.isfinite(got).all()) and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("M,N,Kd,gated,tile,shares", [(2049, 17920, 1536, True, 0, 1), (801, 17920, 1536, True, 2, 1), (513, 17920, 1536, True, 6, 1),
                                                       (700, 9728, 896, True, 3, 1), (65, 9728, 896, True, 4, 1), (1300, 1536, 8960, False, 1, 5),
                                                       (801, 1536, 8960, False, 2, 6), (1025, 1536, 8960, False, 6, 7), (2049, 6144, 1024, False, 0, 1),
