@@ -98,7 +98,8 @@ __device__ __forceinline__ void am_block(const uint4* kf0, const uint4* kf1, con
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int key = key_base + i;
-                if (key > p_col[j] || (key < lo_col[j] && key >= first)) sv[i] = -INFINITY;
+                const bool hidden = (key > p_col[j]) | ((key < lo_col[j]) & (key >= first));
+                sv[i] = hidden ? -INFINITY : sv[i];
             }
         }
         const float bmax = am_column_max(am_max3(am_max3(sv[0], sv[1], sv[2]), am_max3(sv[3], sv[4], sv[5]), am_max3(sv[6], sv[7], sv[7])));
@@ -492,7 +493,8 @@ __device__ __forceinline__ void am_block_lds(const uint4* kt, const uint4* vt, i
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int key = key_base + i;
-                if (key > p_col[j] || (key < lo_col[j] && key >= first)) sv[i] = -INFINITY;
+                const bool hidden = (key > p_col[j]) | ((key < lo_col[j]) & (key >= first));
+                sv[i] = hidden ? -INFINITY : sv[i];
             }
         }
         const float bmax = am_column_max(am_max3(am_max3(sv[0], sv[1], sv[2]), am_max3(sv[3], sv[4], sv[5]), am_max3(sv[6], sv[7], sv[7])));
@@ -612,15 +614,20 @@ __device__ __forceinline__ void am_tile_lds(const uint4* kt, const uint4* vt, in
 #pragma unroll
         for (int i = 0; i < 4; ++i) vf[i] = AM_VFRAG(i);     // only now: their registers are in use until here
     }
-    const bool edge = (kb + 63 > p_col) || (kb < lo_col);
-    if (__any(edge)) {
+    // (in lanes, not in branches: two instructions a key of a tile that reaches beyond a column, four of one ahead of what it sees)
+    if (__any(kb + 63 > p_col)) {
+        const int last = p_col - kb - 8 * g;                 // of the lane's keys, counted from its first
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int i = 0; i < 16; ++i) sv[i] = 32 * (i >> 3) + (i & 7) > last ? -INFINITY : sv[i];
+    }
+    if (__any(kb < lo_col)) {
+        const int from = lo_col - kb - 8 * g, kept = first - kb - 8 * g;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int key = kb + 32 * h + 8 * g + i;
-                if (key > p_col || (key < lo_col && key >= first)) sv[8 * h + i] = -INFINITY;
-            }
+        for (int i = 0; i < 16; ++i) {
+            const int key = 32 * (i >> 3) + (i & 7);
+            const bool hidden = (key < from) & (key >= kept);
+            sv[i] = hidden ? -INFINITY : sv[i];
+        }
     }
     float bmax = am_max3(am_max3(am_max3(sv[0], sv[1], sv[2]), am_max3(sv[3], sv[4], sv[5]), sv[6]),
                          am_max3(am_max3(sv[7], sv[8], sv[9]), am_max3(sv[10], sv[11], sv[12]), sv[13]), am_max3(sv[14], sv[15], sv[15]));
@@ -709,7 +716,9 @@ __device__ __forceinline__ int at_v_swizzle(int row) { return (row >> 1) & 7; }
 // SPLIT: blockIdx.z is a run of `split_tiles` tiles at absolute positions and the work-group walks those of its tiles that
 // lie in it; sums, maxima and accumulators go to the workspace that attn_merge_kernel puts together, as split decode steps
 // leave them there.  For steps whose work-groups leave most CUs idle behind long contexts: 489 tokens behind 3,072 beside 24
-// decoding requests (12 query and 2 key/value heads of 128, 94 work-groups) 45 us with the merge, 62 in two chains.
+// decoding requests (12 query and 2 key/value heads of 128, 94 work-groups) 36 us with the merge, 62 in two chains.
+// A third buffer, loads two tiles ahead, gives nothing (36 and 36 us; 512 behind 8,192 94 and 115).  A tile's addresses are a page id and
+// one product for K and one for V^T; in the last tile, which may reach beyond the keys, they are made key by key.
 template <int DC, int NT, int WAVES, int CH, int MODE, bool SPLIT>
 __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void attn_tile_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
@@ -735,8 +744,7 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
         (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ks) : 0u;
     const uint32_t vs_lds = ks_lds + 2 * TILE * 16;
     int* tab = reinterpret_cast<int*>(at_smem + CH * 4 * TILE);   // page ids of the sequence, as far as needed (NB ints)
-    int* qst = tab + NB;                                   // q_start of the step (S + 1 ints)
-    float* bias_lds = reinterpret_cast<float*>(qst + S + 1);   // mode 2: the group's rows of the bias table, times log2 e
+    float* bias_lds = reinterpret_cast<float*>(tab + NB);  // mode 2: the group's rows of the bias table, times log2 e
     const int c = lane & 15, g = lane >> 4;
     const int kvh = blockIdx.x;                            // fastest: the heads of a group start together
     const int G = nq / nkv;
@@ -746,42 +754,68 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
     // group that exists (a step mixes a long prompt portion with many one-token sequences, and a
     // grid of sequences x most groups would be nearly all empty work-groups).  Within a sequence
     // the groups with the most keys (the last columns) come first.
-    for (int i = tid; i <= S; i += THREADS) qst[i] = q_start[i];
-    __syncthreads();
-    int s = 0, flat = blockIdx.y, ngroups = 0;
-    for (; s < S; ++s) {
-        const int nn = qst[s + 1] - qst[s];
-        ngroups = (skip_single && nn == 1) ? 0 : (nn * G + 127) / 128;   // one-token sequences: another launch's
-        if (flat < ngroups) break;
-        flat -= ngroups;
+    // A lane looks at a sequence, and what the work-group needs of its own comes from that lane: with the offsets in LDS and a search
+    // one by one it took a second trip to memory, a barrier and 50 ns a sequence (150 prompts of 40 tokens, 12 + 2 heads of 128, 34 -> 18 us,
+    // nine of 21 to 157 9.9 -> 9.5).
+    int q0, nn, st;
+    auto look = [&](int base) {
+        const int seq = min(base + lane, S - 1);
+        q0 = q_start[seq], nn = base + lane < S ? q_start[seq + 1] - q0 : 0, st = ctx_start[seq];
+    };
+    look(0);
+    int flat = blockIdx.y, run = blockIdx.z;
+    bool portions = true;
+    if (SPLIT) {
+        // The runs of portions ahead of those of one-token sequences, whose work-groups have one wave with columns: the heavy ones get
+        // a CU each while there are CUs (with the merge and what else changed here, us: 489 tokens
+        // behind 3,072 beside 24 decoding requests, 12 + 2 heads of 128, 51 -> 36; 300 behind 3,000 of 14 + 2 heads of 64 30 -> 22; 512
+        // behind 8,192 of 28 + 4 heads 110 -> 94).
+        int many = 0;
+        for (int base = 0; base < S; base += 64) {
+            if (base) look(base);
+            many += __builtin_amdgcn_readlane(tl_wave_scan(nn > 1 ? (nn * G + 127) / 128 : 0), 63);
+        }
+        if (S > 64) look(0);
+        const int z = (int)gridDim.z, groups = (int)gridDim.y;
+        int id = run * groups + flat;
+        portions = id < many * z;
+        if (!portions) id -= many * z;
+        const int of = portions ? many : groups - many;
+        run = id / of, flat = id - run * of;
     }
-    if (s >= S) return;                       // the whole work-group leaves: no barrier is missed
-    const int r0 = qst[s];
-    const int n = qst[s + 1] - r0;
-    const int start = ctx_start[s];
+    int s = -1, ngroups = 0, r0 = 0, n = 0, start = 0;
+    for (int base = 0; base < S && s < 0; base += 64) {
+        if (base) look(base);
+        const bool mine = SPLIT ? (nn > 1) == portions : !(skip_single && nn == 1);   // skip_single: one-token sequences are another launch's
+        const int groups = mine ? (nn * G + 127) / 128 : 0, upto = tl_wave_scan(groups), total = __builtin_amdgcn_readlane(upto, 63);
+        if (flat < total) {
+            const int l = (int)__builtin_ctzll(__ballot(upto > flat));
+            s = base + l, ngroups = __builtin_amdgcn_readlane(groups, l), flat -= __builtin_amdgcn_readlane(upto, l) - ngroups;
+            r0 = __builtin_amdgcn_readlane(q0, l), n = __builtin_amdgcn_readlane(nn, l), start = __builtin_amdgcn_readlane(st, l);
+        } else {
+            flat -= total;
+        }
+    }
+    if (s < 0) return;                        // the whole work-group leaves: no barrier is missed
     const int ncols = n * G;
     // Loader.  A K tile is 64 rows x UPK units of 16 bytes, a V^T tile D rows x 8 units (8 keys
     // each): UPK wave-loads of 64 consecutive units each, dealt round-robin to the waves.  For its
-    // load number i a lane knows which key and unit (K) and which dim and first key (V^T) the LDS
-    // place it fills holds.
-    constexpr int NI = (UPK + WAVES - 1) / WAVES;
+    // first load a lane knows which key and unit (K) and which dim and first key (V^T) the LDS
+    // place it fills holds; the load i later rows of K (a multiple of 16: the same swizzle) on has a key that is more by the
+    // same for all lanes, in bits that the first one's does not have, and 64 dims of V^T on has the same keys.
+    constexpr int NI = (UPK + WAVES - 1) / WAVES, K_ROWS = WAVES * 64 / UPK;
+    static_assert(NI == 1 || K_ROWS % 16 == 0, "loads of a lane whose rows are swizzled alike");
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    int k_key[NI], v_key[NI];                  // K: the lane's key of the tile; V^T: the first key of its unit
-    const char *k_base[NI], *v_base[NI];       // where that unit lies in slot 0 (K), in page 0 at offset 0 (V^T)
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        int w = wave_u + i * WAVES;
-        if (w >= UPK) w = UPK - 1;                           // not issued
-        const int idx = w * 64 + lane;
-        const int krow = idx / UPK, kpu = idx % UPK;
-        k_key[i] = at_lds_key(krow);
-        k_base[i] = reinterpret_cast<const char*>(kc + (size_t)kvh * D + (kpu ^ at_k_swizzle<UPK>(krow)) * 8);
-        const int vrow = idx >> 3, vpu = idx & 7;
-        v_key[i] = (vpu ^ at_v_swizzle(vrow)) * 8;
-        v_base[i] = reinterpret_cast<const char*>(vc + ((size_t)kvh * D + vrow) * bs);
-    }
     const uint32_t k_stride = (uint32_t)nkv * D * 2;         // bytes from a slot to the next
     const uint32_t v_stride = (uint32_t)nkv * D * bs * 2;    // bytes from a page to the next
+    const int k_unit = (wave_u < UPK ? wave_u : UPK - 1) * 64 + lane;          // (waves beyond have no load)
+#define AT_K_KEY at_lds_key(k_unit / UPK)
+#define AT_V_KEY (((k_unit & 7) ^ at_v_swizzle(k_unit >> 3)) * 8)
+    // where the unit lies in page 0, and 4 x the page of a tile that holds it (an offset into tab)
+    const char* k_base = reinterpret_cast<const char*>(kc + (size_t)kvh * D + ((k_unit % UPK) ^ at_k_swizzle<UPK>(k_unit / UPK)) * 8) +
+                         (uint64_t)(uint32_t)(AT_K_KEY & (bs - 1)) * k_stride;
+    const char* v_base = reinterpret_cast<const char*>(vc + ((size_t)kvh * D + (k_unit >> 3)) * bs + (AT_V_KEY & (bs - 1)));
+    const int k_page = (AT_K_KEY >> bs_shift) * 4, v_page = (AT_V_KEY >> bs_shift) * 4;
     const int kx = at_k_swizzle<UPK>(c), vx = at_v_swizzle(c);
     // Which of its sequence's groups: the one with the most keys first.  The hardware places
     // work-group i + 256 on the CU of work-group i (256 CUs, two work-groups each), so when the
@@ -811,7 +845,7 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
     }
     int h_first = 0, b_first = t_lo, n_tiles = t_head + t_hi - t_lo + 1;
     if (SPLIT) {
-        const int z0 = (int)blockIdx.z * split_tiles, z1 = z0 + split_tiles;       // this run's tiles
+        const int z0 = run * split_tiles, z1 = z0 + split_tiles;       // this run's tiles
         const int h_end = min(t_head, z1), b_end = min(t_hi + 1, z1);
         h_first = min(z0, t_head);
         b_first = max(t_lo, z0);
@@ -877,15 +911,24 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
 #define AT_FETCH(T, BUF)                                                                                       \
     {                                                                                                         \
         const int kb_ = (T) * AT_KEYS;                                                                        \
-        const char *gk_[NI], *gv_[NI];                                                                        \
-        _Pragma("unroll") for (int i = 0; i < NI; ++i) {                                                      \
-            int key_ = kb_ + k_key[i];                                                                        \
-            if (key_ > khi) key_ = khi;                                                                       \
-            const uint32_t slot_ = ((uint32_t)tab[key_ >> bs_shift] << bs_shift) + (key_ & (bs - 1));         \
-            gk_[i] = k_base[i] + (uint64_t)slot_ * k_stride;                                                  \
-            int vk_ = kb_ + v_key[i];                                                                         \
-            if (vk_ > khi) vk_ = khi & ~7;                                                                    \
-            gv_[i] = v_base[i] + (uint64_t)(uint32_t)tab[vk_ >> bs_shift] * v_stride + (vk_ & (bs - 1)) * 2;  \
+        const int in_ = kb_ & (bs - 1);                          /* (pages of more than a tile) */            \
+        const char *gk_[NI], *gv_;                                                                            \
+        if (kb_ + AT_KEYS - 1 <= khi) {                                                                       \
+            const char* tab_ = reinterpret_cast<const char*>(tab + (kb_ >> bs_shift));                        \
+            _Pragma("unroll") for (int i = 0; i < NI; ++i) {                                                  \
+                const int on_ = at_lds_key(i * K_ROWS);                                                       \
+                const uint32_t page_ = *reinterpret_cast<const uint32_t*>(tab_ + 4 * (on_ >> bs_shift) + k_page); \
+                gk_[i] = k_base + (uint64_t)((page_ << bs_shift) + in_ + (on_ & (bs - 1))) * k_stride;        \
+            }                                                                                                 \
+            gv_ = v_base + ((uint64_t)*reinterpret_cast<const uint32_t*>(tab_ + v_page) * v_stride + in_ * 2); \
+        } else {                                                                                              \
+            _Pragma("unroll") for (int i = 0; i < NI; ++i) {                                                  \
+                const int key_ = min(kb_ + AT_K_KEY + at_lds_key(i * K_ROWS), khi);                           \
+                const uint32_t slot_ = ((uint32_t)tab[key_ >> bs_shift] << bs_shift) + (key_ & (bs - 1));     \
+                gk_[i] = k_base + ((int64_t)slot_ - (AT_K_KEY & (bs - 1))) * k_stride;                        \
+            }                                                                                                 \
+            const int vk_ = kb_ + AT_V_KEY > khi ? khi & ~7 : kb_ + AT_V_KEY;                                 \
+            gv_ = v_base + (uint64_t)(uint32_t)tab[vk_ >> bs_shift] * v_stride + ((vk_ & (bs - 1)) - (AT_V_KEY & (bs - 1))) * 2; \
         }                                                                                                     \
         const uint32_t buf_ = CH > 1 ? (uint32_t)__builtin_amdgcn_readfirstlane((BUF) * TILE * 16) : 0u;      \
         _Pragma("unroll") for (int i = 0; i < NI; ++i) {                                                      \
@@ -893,10 +936,10 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
             if (w_ < UPK) {                                                                                   \
                 if (CH > 1) {                                                                                 \
                     tl_load_to_lds(gk_[i], ks_lds + buf_ + w_ * 1024);                                        \
-                    tl_load_to_lds(gv_[i], vs_lds + buf_ + w_ * 1024);                                        \
+                    tl_load_to_lds(gv_ + (size_t)i * (WAVES * 8) * bs * 2, vs_lds + buf_ + w_ * 1024);        \
                 } else {                                                                                      \
                     tl_load_to_lds(gk_[i], tl_lds_address(ks + (BUF) * TILE + w_ * 64));                      \
-                    tl_load_to_lds(gv_[i], tl_lds_address(vs + (BUF) * TILE + w_ * 64));                      \
+                    tl_load_to_lds(gv_ + (size_t)i * (WAVES * 8) * bs * 2, tl_lds_address(vs + (BUF) * TILE + w_ * 64)); \
                 }                                                                                             \
             }                                                                                                 \
         }                                                                                                     \
@@ -997,7 +1040,7 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
         l_tot += __shfl_xor(l_tot, 16, TL_WAVE);
         l_tot += __shfl_xor(l_tot, 32, TL_WAVE);
         if (SPLIT) {
-            const size_t part = ((size_t)row_col[j] * nq + head_col[j]) * gridDim.z + blockIdx.z;
+            const size_t part = ((size_t)row_col[j] * nq + head_col[j]) * gridDim.z + run;
             float* wp = ws_o + part * D + 4 * g;
 #pragma unroll
             for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4*>(wp + db * 16) = acc[j][db];
@@ -1027,6 +1070,8 @@ __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void att
 // head size 128, so two work-groups share a CU's 160 KB up to some 8,000 pages per sequence and one
 // work-group has it alone beyond that
 // (bias_floats: the rows of the bias table of a group of query heads)
+// (what the kernel takes with S = -1; the choice counts S + 1 ints more, as it did when it held the step's offsets too: which
+// sums a step's rows are made of does not change)
 static size_t at_lds_bytes(int DC, int pages, int S, size_t bias_floats, int chains = 1) {
     return (size_t)chains * (4 * AT_KEYS * DC * 4) * sizeof(uint4) + (size_t)(pages + S + 1) * sizeof(int) + bias_floats * sizeof(float);
 }
@@ -1302,7 +1347,7 @@ extern "C" int tl_attention_mfma(const void* q, int q_stride, const void* k_cach
                      "tl_attention_mfma: runs of keys of the tile kernel are whole tiles of 64, and no sequence is left out");
         dim3 sgrid(nkv, (unsigned)total_groups128, tiles_split ? nsplit : 1);
         const int chains = (shared == 2 && d != 256 && !tiles_split && at_lds_bytes(d / 32, NB, S, bias_floats, 2) <= 160 * 1024) ? 2 : 1;
-        const size_t lds = at_lds_bytes(d / 32, NB, S, bias_floats, chains);
+        const size_t lds = at_lds_bytes(d / 32, NB, -1, bias_floats, chains);
 #define TL_TILE_CASE(DCV)                                                                                             \
     do {                                                                                                              \
         if (bias_table) TL_TILE_GO(DCV, 2);                                                                           \

@@ -44,6 +44,17 @@ template <> __device__ __forceinline__ bf16_t tl_from_float<bf16_t>(float v) {
     return r;
 }
 
+// the sum over the lanes up to and with the lane's own
+__device__ __forceinline__ int tl_wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);       // within rows of 16: from 1, 2, 4, 8 lanes below
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // rows 1 and 3: the last lane of the row below
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);      // the upper half: lane 31
+    return v;
+}
+
 // ---- reductions ----------------------------------------------------------------------------
 // Over a wave with all its lanes active, lane i with lane i ^ 32, then ^ 16, ^ 8, ^ 4, ^ 2, ^ 1, without trips through LDS: the halves of 32 and 16
 // lanes by register swaps, the rest by rotations within a row of 16 (after the step of 8 the values repeat every 8 lanes, so the

@@ -1562,6 +1562,20 @@ def test_attention_portions_in_runs_of_keys(nq, nkv, d, bs, lens, q_lens, kw, mo
     torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
 
 
+@pytest.mark.parametrize("runs,bs,first", [(True, 16, 3), (True, 128, 66), (False, 32, 63), (False, 128, 0)])
+def test_attention_of_portions_among_many_sequences(runs, bs, first, monkeypatch):
+    """Steps of more sequences than a wave has lanes, portions ahead of, between and behind one-token requests, in runs of keys
+    (where the portions' work-groups come first) and in whole walks; pages smaller and larger than a tile of keys."""
+    lens, q_lens = [5 + 3 * i for i in range(70)], [1] * 70
+    for at, n, ql in ((first, 2100 if runs else 150, 43), (first + 1, 200, 130), (len(lens), 77, 70)):
+        lens.insert(at, n), q_lens.insert(at, ql)
+    chosen, choose = [], K()._attention_launch
+    monkeypatch.setattr(K(), "_attention_launch", lambda *a: chosen.append(choose(*a)) or chosen[-1])
+    got, want = _attention_case(torch.bfloat16, 6, 1, 128, bs, lens, q_lens, seed=bs, route_singles=None if runs else False)
+    assert (chosen[0].nsplit > 1) == runs and chosen[0].chains > 0 and chosen[0].own_split is None
+    torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
+
+
 @pytest.mark.parametrize("M", [1, 5, 16])
 @pytest.mark.parametrize("N,Kd", [(784, 2048), (1000, 2056), (2048, 4864), (1030, 520), (896, 2336), (1030, 776), (1030, 904)])
 def test_few_rows_in_half_tiles(M, N, Kd):
