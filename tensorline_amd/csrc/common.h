@@ -183,6 +183,35 @@ __host__ __device__ __forceinline__ int tl_mask_lo(const TlMask& k, int p) {
 // a key below lo is hidden unless it is one of the kept first keys
 __device__ __forceinline__ bool tl_mask_hides(const TlMask& k, int key, int lo) { return key < lo && key >= k.first; }
 
+// ---- v / (1 + e^-v) and 1 / (1 + e^-x) of numbers of middling size ---------------------------------
+// expf and the division spend half their instructions on ends of the range that a product's results seldom reach (26 for the gate of SiLU where
+// these take 14, and a tile's end has 64 of them a lane).  For |x| <= TL_MID (and a v of 2^-60 and more) they give the same bits: all
+// floats of that range were compared.  Callers ask tl_mid_* for a wave's values first.
+#define TL_MID 40.0f
+__device__ __forceinline__ float tl_exp_mid(float x) {
+    const float ph = x * 0x1.715476p+0f, e = __builtin_rintf(ph);           // x log2 e in two parts, as expf has it
+    const float pl = __builtin_fmaf(x, 0x1.4ae0bep-26f, __builtin_fmaf(x, 0x1.715476p+0f, -ph));
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((ph - e) + pl), (int)e);
+}
+__device__ __forceinline__ float tl_silu_mid(float v) {
+    const float d = 1.0f + tl_exp_mid(-v), r = __builtin_amdgcn_rcpf(d), q = v * r;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, v), r, q);
+}
+__device__ __forceinline__ float tl_sigmoid_mid(float x) {
+    const float d = 1.0f + tl_exp_mid(-x), r = __builtin_amdgcn_rcpf(d);
+    return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+}
+// the least and largest magnitudes of a wave's values (as bits without the sign)
+struct TlMagnitudes {
+    uint32_t least = 0xffffffffu, most = 0;
+    __device__ __forceinline__ void take(float v) {
+        const uint32_t u = __float_as_uint(v) << 1;
+        least = min(least, u), most = max(most, u);
+    }
+    __device__ __forceinline__ bool mid_silu() const { return !__any(most > __float_as_uint(TL_MID) << 1 || least < __float_as_uint(0x1p-60f) << 1); }
+    __device__ __forceinline__ bool mid_sigmoid() const { return !__any(most > __float_as_uint(TL_MID) << 1); }
+};
+
 // ---- scores bent by a cap ------------------------------------------------------------------------
 // cap * tanh(score / cap), in the units the caller keeps scores in: raw is the bare product of query and
 // key, to_exp = 2 log2(e) * scale / cap turns it into the exponent of e^(2 score / cap) = 2^(raw to_exp), and

@@ -40,10 +40,6 @@ struct GtOut {
     int act;                   // plain: 1 the square of relu; gated: 0 SiLU, 2 the tanh form of GELU passes the gate
 };
 
-__device__ __forceinline__ float gt_gate(float v, int act) {
-    if (act == 2) return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
-    return v / (1.0f + expf(-v));
-}
 // GLU: W has the N / 2 gate rows, then the N / 2 up rows, and C = act(gate) * up [M, N / 2]; a wave's first NB / 2 blocks are gate
 // columns, the others the up columns of the same places.
 template <int WM, int WN, int MB, int NB, int AST, int BST, bool GLU, typename TO>
@@ -121,22 +117,42 @@ __global__ __launch_bounds__(64 * WM * WN, MB * NB >= 16 || !BST ? 2 : 4) void g
 
     // this lane holds row c and the columns 4 g .. 4 g + 3 of each block (N, or N / 2, is a multiple of 4 or of 16: whole quads)
     TO* C = reinterpret_cast<TO*>(out.C);
+    if constexpr (GLU) {
+        const auto store = [&](auto gate) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                const int m = m0 + (wm * MB + i) * 16 + c;
+                if (m >= M) continue;
+                TO* row = C + (size_t)m * out.ldc;
+#pragma unroll
+                for (int j = 0; j < NB / 2; ++j) {
+                    const int n = (tile0 + wn * (NB / 2) + j) * 16 + 4 * g;
+                    if (2 * n >= N) continue;
+                    tw_f32x4 o;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) o[v] = gate(acc[i][j][v]) * acc[i][NB / 2 + j][v];
+                    tw_store4(row + n, o);
+                }
+            }
+        };
+        TlMagnitudes size;
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB / 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) size.take(acc[i][j][v]);
+        if (out.act == 2) store([](float v) { return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v))); });
+        else if (size.mid_silu()) store([](float v) { return tl_silu_mid(v); });
+        else store([](float v) { return v / (1.0f + expf(-v)); });
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
         const int m = m0 + (wm * MB + i) * 16 + c;
         if (m >= M) continue;
         TO* row = C + ((size_t)share * M + m) * out.ldc;
-        if (GLU) {
-#pragma unroll
-            for (int j = 0; j < NB / 2; ++j) {
-                const int n = (tile0 + wn * (NB / 2) + j) * 16 + 4 * g;
-                if (2 * n >= N) continue;
-                tw_f32x4 o;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) o[v] = gt_gate(acc[i][j][v], out.act) * acc[i][NB / 2 + j][v];
-                tw_store4(row + n, o);
-            }
-        } else {
+        {
 #pragma unroll
             for (int j = 0; j < NB; ++j) {
                 const int n = (tile0 + wn * NB + j) * 16 + 4 * g;

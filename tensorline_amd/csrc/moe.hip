@@ -669,26 +669,44 @@ __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, 
         [&](int buf, int h, int j) { return __builtin_bit_cast(tw_bf16x8, lds[buf * MGW_W + ((wbase + (GLU && j >= 2 ? 1024 + (j - 2) * 128 : j * 128)) ^ (4 * h))]); });
 
     // this lane holds row c and the columns 4 g .. 4 g + 3 of each block (N is a multiple of 4)
+    if constexpr (GLU) {
+        const auto store = [&](auto sigmoid) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                const int r = (wm * MB + i) * 16 + c;
+                if (r >= rows) continue;
+                bf16_t* crow = reinterpret_cast<bf16_t*>(Cv) + (size_t)(place0 + r) * ldc;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int n = n0 + wn * 32 + j * 16 + 4 * g;
+                    if (n >= N) continue;
+                    tw_f32x4 o;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float gt = fminf(acc[i][j][v], limit);
+                        const float up = fminf(fmaxf(acc[i][2 + j][v], -limit), limit);
+                        o[v] = gt * sigmoid(alpha * gt) * (up + shift);
+                    }
+                    tw_store4(crow + n, o);
+                }
+            }
+        };
+        TlMagnitudes size;
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) size.take(alpha * fminf(acc[i][j][v], limit));
+        if (size.mid_sigmoid()) store([](float x) { return tl_sigmoid_mid(x); });
+        else store([](float x) { return 1.0f / (1.0f + expf(-x)); });
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
         const int r = (wm * MB + i) * 16 + c;
         if (r >= rows) continue;
-        if (GLU) {
-            bf16_t* crow = reinterpret_cast<bf16_t*>(Cv) + (size_t)(place0 + r) * ldc;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int n = n0 + wn * 32 + j * 16 + 4 * g;
-                if (n >= N) continue;
-                tw_f32x4 o;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const float gt = fminf(acc[i][j][v], limit);
-                    const float up = fminf(fmaxf(acc[i][2 + j][v], -limit), limit);
-                    o[v] = gt * (1.0f / (1.0f + expf(-alpha * gt))) * (up + shift);
-                }
-                tw_store4(crow + n, o);
-            }
-        } else {
+        {
             const size_t at = (size_t)(MODE == 2 ? place0 + r : order[place0 + r]) * ldc;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {

@@ -195,6 +195,30 @@ def test_gated_product_with_the_matrix_in_registers(M, I, Kd):
         assert bool(torch.isfinite(got).all()) and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("tile", [0, 3, 5, 6, 7])
+def test_gate_of_every_size(tile):
+    """SiLU behind the product for every finite bfloat16 number as the gate: sorted, so that waves have middling numbers only, and in
+    disorder, so that they have some beyond.  The same bits both ways (a number's steps do not depend on its wave's others), and within
+    the rounding of the float steps (2^-21) and of the result; where e^-v passes the largest float, 2^128, the result is 0 for at
+    most 89 / 2^128 < 2^-121."""
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    v = v[torch.isfinite(v)].to(DEV)
+    v = v[v.float().abs().sort().indices]
+    M, I, Kd = v.numel(), 16, 64
+    w = torch.zeros(2 * I, Kd, device=DEV, dtype=torch.bfloat16)
+    w[:I, 0], w[I:, 1] = 1, 0.75
+    sh = K().shuffle_weight(w)
+
+    def run(values):
+        a = torch.zeros(M, Kd, device=DEV, dtype=torch.bfloat16)
+        a[:, 0], a[:, 1] = values, 1
+        return K()._tiles(a, sh, None, torch.bfloat16, M, 2 * I, Kd, Kd, 256 + tile, gated=True)[:, 3]
+    got, mixed = run(v), torch.randperm(M, device=DEV)
+    assert torch.equal(run(v[mixed]).view(torch.int16), got[mixed].view(torch.int16))
+    want = v.double() / (1 + (-v.double()).exp()) * 0.75
+    assert bool(((got.double() - want).abs() <= (2.0 ** -8 + 2.0 ** -21) * want.abs() + 2.0 ** -121).all())
+
+
 @pytest.mark.parametrize("M,N,Kd,gated,tile,shares", [(2049, 17920, 1536, True, 0, 1), (801, 17920, 1536, True, 2, 1), (513, 17920, 1536, True, 6, 1),
                                                       (700, 9728, 896, True, 3, 1), (65, 9728, 896, True, 4, 1), (1300, 1536, 8960, False, 1, 5),
                                                       (801, 1536, 8960, False, 2, 6), (1025, 1536, 8960, False, 6, 7), (2049, 6144, 1024, False, 0, 1),
