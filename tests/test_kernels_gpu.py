@@ -1123,6 +1123,24 @@ def test_silu_mul(dtype):
     torch.testing.assert_close(got.double(), torch.nn.functional.silu(g) * u, **tol(dtype, 1e-5, 2e-2))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("I", [8, 1032, 2044, 2047])
+def test_silu_mul_of_gates_beyond_middling_ones(dtype, I):
+    """By 16 bytes, with a last thread of the row alone, and one by one; rows of middling gates beside rows with zeros, gates past where
+    the exponent leaves the range, and infinities: what a row alone gives, and the float64 gate."""
+    torch.manual_seed(I)
+    gu = (torch.randn(5, 2 * I, device=DEV) * torch.tensor([3.0, 30.0, 90.0, 1e-20, 1.0], device=DEV)[:, None]).to(dtype)
+    gu[4, :I:3], gu[4, 1:I:3], gu[4, 2] = 0.0, float("-inf"), float("inf")
+    got, g, u = K().silu_mul(gu), gu[:, :I].double(), gu[:, I:].double()
+    assert all(torch.equal(got[t:t + 1].isnan(), K().silu_mul(gu[t:t + 1]).isnan()) for t in range(5))
+    want = g / (1 + (-g).exp()) * u
+    assert torch.equal(got.isnan(), want.isnan())
+    # e^-v has no float beyond 2^128: there the result is 0, for 89 / 2^128 < 2^-121 times |u| at most (|u| is up to some hundreds here)
+    t = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -21
+    ok = ~want.isnan() & ~want.isinf()
+    assert bool(((got.double() - want).abs() <= t * want.abs() + 2.0 ** -121 * u.abs() + 2.0 ** -126)[ok].all()) and bool((got.double() == want)[want.isinf()].all())
+
+
 def test_argmax_and_ties():
     torch.manual_seed(0)
     lg = torch.randn(6, 1000, device=DEV)
