@@ -194,7 +194,6 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict
                                                                const float* __restrict__ w, O* __restrict__ out,
                                                                const int32_t* __restrict__ rows, int H, float eps,
                                                                int parts, size_t pstride) {
-    constexpr int AHEAD = 8;
     __shared__ float red[16];
     const int r = blockIdx.x;
     const size_t src = HAS_ROWS ? (size_t)rows[r] : (size_t)r;
@@ -212,13 +211,13 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict
             gw[i] = tl_load4(w + 4 * c4);                    // used at the end
             if (HAS_RES) {
                 float4 b = tl_load4(rr + 4 * c4);
-                for (int p = 1; p < parts; p += AHEAD) {     // shares are asked for before they are added
-                    float4 e[AHEAD];
+                for (int p = 1; p < parts; p += 4) {         // four shares are asked for before they are added
+                    float4 e[4];
 #pragma unroll
-                    for (int k = 0; k < AHEAD; ++k)
+                    for (int k = 0; k < 4; ++k)
                         if (p + k < parts) e[k] = tl_load4(rr + 4 * c4 + (p + k) * pstride);
 #pragma unroll
-                    for (int k = 0; k < AHEAD; ++k)
+                    for (int k = 0; k < 4; ++k)
                         if (p + k < parts) b.x += e[k].x, b.y += e[k].y, b.z += e[k].z, b.w += e[k].w;
                 }
                 a.x += b.x;
