@@ -1236,6 +1236,15 @@ __global__ __launch_bounds__(AM_MERGE_THREADS) void attn_merge_kernel(
 
 #undef AM_SPLIT_AT
 
+// Whether attn_decode_kernel takes splits of so many blocks on pages of bs tokens: it holds a split's page ids one a lane, so a split may touch
+// 64 pages.  Splits that are not whole pages begin inside pages, as far in as bs - gcd(split, bs) tokens, and can touch one page more than
+// their length says (pages of 128: splits of 255 blocks, 63.75 pages, touch 65).
+extern "C" int tl_attention_decode_takes(int bs, int split_blocks) {
+    if (bs < 16 || (bs & (bs - 1)) || split_blocks < 1) return 0;
+    const long long split = 32ll * split_blocks, step = split & -split;
+    return bs - (step < bs ? step : bs) + split <= 64ll * bs;
+}
+
 template <int DC>
 static void launch_attn(int NT, dim3 grid, int wg_waves, hipStream_t stream, const bf16_t* q, int q_stride, const bf16_t* kc,
                         const bf16_t* vc, const int32_t* tables, int NB, const int32_t* q_start,
@@ -1245,8 +1254,8 @@ static void launch_attn(int NT, dim3 grid, int wg_waves, hipStream_t stream, con
     int bs_shift = -1;                               // pages of a power of two of tokens: a shift finds the page
     if ((bs & (bs - 1)) == 0)
         for (bs_shift = 0; (1 << bs_shift) < bs;) ++bs_shift;
-    // one tile of columns in splits of at most 64 pages
-    if constexpr (DC <= 4) if (nsplit > 1 && NT == 1 && one_tile && !bias.table && bs_shift >= 4 && split_blocks <= 2 << bs_shift && grid.x <= 65535) {
+    // one tile of columns in splits on at most 64 pages
+    if constexpr (DC <= 4) if (nsplit > 1 && NT == 1 && one_tile && !bias.table && tl_attention_decode_takes(bs, split_blocks) && grid.x <= 65535) {
 #define AM_DECODE(MODEV, ONE)                                                                                                               \
     hipLaunchKernelGGL((attn_decode_kernel<DC, MODEV, 2, ONE>), dim3(nkv, grid.x, nsplit), dim3(64), 0, stream, q, kc, vc, tables, q_start, \
                        ctx_start, NB, q_stride, ws_o, ws_ml, nq, nkv, bs, bs_shift, mask, scale, split_blocks, seq_list, skip_single, softcap)

@@ -45,6 +45,20 @@ def test_key_splits_follow_the_batch_and_the_context_and_never_exceed_what_the_m
     assert K._fit_key_splits(64, 100, fit_context=1 << 20)[0] == K._fit_key_splits(64, 1 << 20)[0]
 
 
+def test_splits_of_one_wave_never_touch_more_pages_than_lanes():
+    """The decode kernel has a split's page ids one a lane: it takes the splits that touch at most 64 pages wherever they begin."""
+    takes = K.library().tl_attention_decode_takes
+    for page in (16, 32, 64, 128, 256, 1024):
+        for blocks in [*range(1, 40), *range(2 * page - 40, 2 * page + 40)]:
+            if blocks < 1:
+                continue
+            length = 32 * blocks
+            touched = max(((i + 1) * length - 1) // page - i * length // page + 1 for i in range(page))
+            assert bool(takes(page, blocks)) == (touched <= 64), (page, blocks, touched)
+    assert not takes(128, 255) and not takes(256, 511) and takes(128, 256) and takes(128, 254) and takes(64, 127) and takes(16, 32)
+    assert not any(takes(page, 4) for page in (8, 24, 48, 0)) and not takes(16, 0)
+
+
 def test_one_token_sequences_of_a_step():
     mixed = StepFacts(max_context=900, max_query_len=300, decode_only=False, num_seqs=5, q_lens=[300, 1, 1, 7], starts=[600, 40, 0, 3])
     assert K.one_token_sequences(mixed) == [1, 2, 4]                # the padding sequence too

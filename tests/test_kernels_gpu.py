@@ -1772,6 +1772,17 @@ def test_decode_attention_in_splits_of_one_wave(nq, nkv, d, bs, split, kw):
     torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
 
 
+@pytest.mark.parametrize("bs,blocks", [(128, 255), (256, 510), (256, 511), (128, 254), (128, 256), (64, 127)])
+def test_decode_attention_in_splits_of_some_64_pages(bs, blocks):
+    """Splits that begin inside a page and touch 64 pages or 65: more than a wave has lanes for their ids.  The spiked key is in the last page
+    that the second split touches; chunks keep the sums to its keys."""
+    split = 32 * blocks
+    page = (2 * split - 1) // bs * bs
+    for kw in (dict(spike=True, spike_at=lambda p: p - 3), dict(chunk=page)):
+        got, want = _attention_case(torch.bfloat16, 4, 2, 64, bs, [page + 40, 2 * split, 77], None, seed=blocks, split_keys=split, path="mfma", **kw)
+        torch.testing.assert_close(got, want, **tol(torch.bfloat16, 3e-5, 2e-2))
+
+
 @pytest.mark.parametrize("split", [64, 512])
 def test_few_tokens_in_splits_of_one_wave(split):
     """Several tokens of a sequence whose columns fit one tile of 16."""
