@@ -247,7 +247,7 @@ static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shar
 // 1,300 rows of 17,920 x 1,536 69 and 79, 513 34 and 44, 1,521 of 9,728 x 896 30 and 32.  Plain products of up to 3,000 rows with a
 // choice of shares were level at best (256 tiles) or slower (384 tiles 28 and 36), and have no such form.
 static bool gt_goes_direct(const GtTile& t, const GtTile& direct, int M, int N, int K) {
-    return !t.direct && (double)tl_ceil_div(M, direct.bm) * gt_ntiles(direct, N, true) > 256 &&
+    return (double)tl_ceil_div(M, direct.bm) * gt_ntiles(direct, N, true) > 256 &&
            gt_time(direct, M, N, K, true, 1, false) < gt_time(t, M, N, K, true, 1, false);
 }
 
@@ -276,6 +276,7 @@ extern "C" int tl_gemm_tiles_plan(int M, int N, int K, int gated, int takes_shar
             if (best < 0 || us < least) best = shares * 256 + i, least = us;
         }
     }
+    if (gated && best >= 0 && gt_goes_direct(gt_tiles[best & 255], gt_tiles[GT_DIRECT], M, N, K)) best = 256 + GT_DIRECT;
     return best;
 }
 
@@ -295,7 +296,6 @@ extern "C" int tl_gemm_tiles(const void* A, const void* W, const float* bias, vo
     TL_CHECK_ARG((gated && (act == 0 || act == 2)) || (!gated && (act == 0 || act == 1)), "tl_gemm_tiles: activation %d is not one this product applies", act);
     TL_CHECK_ARG(!C || (ldc >= (gated ? N / 2 : N) && ldc % 4 == 0 && (uintptr_t)C % (c_dtype == TL_F32 ? 16 : 8) == 0 && (c_dtype == TL_F32 || c_dtype == TL_BF16)),
                  "tl_gemm_tiles: bad output");
-    if (gated && gt_goes_direct(gt_tiles[tile], gt_tiles[GT_DIRECT], M, N, K)) tile = GT_DIRECT;
     const GtTile& t = gt_tiles[tile];
     const int mtiles = tl_ceil_div(M, t.bm), ntiles = gt_ntiles(t, N, gated);
     TL_CHECK_ARG((double)mtiles * ntiles * shares < 2e9, "tl_gemm_tiles: too many tiles");

@@ -151,9 +151,14 @@ def test_many_row_products_are_cut_within_the_tiles_limits():
         for gated, takes in ((0, 0), (0, 1), (1, 0)):
             p = plan(M, N, Kd, gated, takes)
             tile, shares = p & 255, p >> 8
-            assert 0 <= tile < 7 and 1 <= shares <= 12 and shares <= max(1, Kd // 256) and not (gated and (shares > 1 or tile == 1))
+            assert 0 <= tile < 8 and 1 <= shares <= 12 and shares <= max(1, Kd // 256) and not (gated and (shares > 1 or tile == 1))
+            assert gated or tile != 7
     for M, N, Kd, gated in ((70, 64, 96, 0), (70, 66, 64, 0), (70, 48, 64, 1), (70, 1 << 17, 1 << 15, 0), (0, 64, 64, 0), (513, 3584, 3584, 0)):
         assert plan(M, N, Kd, gated, 0) == -1
+    # what is launched is what the plan says: gated products of more such tiles than CUs with their matrix in registers where that is ahead
+    for M, N, Kd, tile in ((801, 17920, 1536, 7), (2048, 17920, 1536, 7), (380, 37888, 3584, 7), (1521, 9728, 896, 0), (1300, 17920, 1536, 6),
+                           (513, 17920, 1536, 6), (300, 17920, 1536, 2), (65280, 32, 64, 3)):
+        assert plan(M, N, Kd, 1, 0) == 256 + tile, (M, N, Kd)
 
 
 def test_a_many_row_product_with_an_activation_refuses_a_wrong_bias(launches):

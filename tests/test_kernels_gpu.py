@@ -219,8 +219,8 @@ def test_gate_of_every_size(tile):
     assert bool(((got.double() - want).abs() <= (2.0 ** -8 + 2.0 ** -21) * want.abs() + 2.0 ** -121).all())
 
 
-@pytest.mark.parametrize("M,N,Kd,gated,tile,shares", [(2049, 17920, 1536, True, 0, 1), (801, 17920, 1536, True, 2, 1), (513, 17920, 1536, True, 6, 1),
-                                                      (700, 9728, 896, True, 3, 1), (65, 9728, 896, True, 4, 1), (1300, 1536, 8960, False, 1, 5),
+@pytest.mark.parametrize("M,N,Kd,gated,tile,shares", [(2049, 17920, 1536, True, 7, 1), (801, 17920, 1536, True, 7, 1), (513, 17920, 1536, True, 6, 1),
+                                                      (1521, 9728, 896, True, 0, 1), (300, 17920, 1536, True, 2, 1), (700, 9728, 896, True, 3, 1), (65, 9728, 896, True, 4, 1), (1300, 1536, 8960, False, 1, 5),
                                                       (801, 1536, 8960, False, 2, 6), (1025, 1536, 8960, False, 6, 7), (2049, 6144, 1024, False, 0, 1),
                                                       (801, 2048, 1536, False, 4, 1), (2049, 2048, 1536, False, 3, 1), (65, 2048, 1536, False, 5, 4)])
 def test_many_row_calls_in_the_tiles_of_real_steps(M, N, Kd, gated, tile, shares):
