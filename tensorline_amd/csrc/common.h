@@ -185,11 +185,15 @@ __device__ __forceinline__ bool tl_mask_hides(const TlMask& k, int key, int lo) 
 
 // ---- v / (1 + e^-v) and 1 / (1 + e^-x) of numbers of middling size ---------------------------------
 // expf and the division spend half their instructions on ends of the range that a product's results seldom reach (26 for the gate of SiLU where
-// these take 14, and a tile's end has 64 of them a lane).  For |x| <= TL_MID (and a v of 2^-60 and more) they give the same bits: all
-// floats of that range were compared.  Callers ask tl_mid_* for a wave's values first.
+// these take 14, and a tile's end has 64 of them a lane).  A wave asks TlMagnitudes for its values and takes these steps or expf and the
+// division, so for |x| <= TL_MID (and a v of 2^-60 and more) both must give the same bits, or a row's would depend on its neighbours':
+// tl_gate_forms_differ counts the floats of the range where they do not (none).  Hence the exponent's steps are those that expf has in
+// ROCm's device library (ocml, open source) between its checks: x log2 e in two floats, the second by fused multiply-adds, the nearest
+// whole number of it as an exponent, the rest by the instruction.  The quotient is that of the rounded reciprocal, corrected once by its
+// remainder (P. Markstein, IBM Journal of Research and Development 34, 1990).
 #define TL_MID 40.0f
 __device__ __forceinline__ float tl_exp_mid(float x) {
-    const float ph = x * 0x1.715476p+0f, e = __builtin_rintf(ph);           // x log2 e in two parts, as expf has it
+    const float ph = x * 0x1.715476p+0f, e = __builtin_rintf(ph);
     const float pl = __builtin_fmaf(x, 0x1.4ae0bep-26f, __builtin_fmaf(x, 0x1.715476p+0f, -ph));
     return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((ph - e) + pl), (int)e);
 }
@@ -201,15 +205,17 @@ __device__ __forceinline__ float tl_sigmoid_mid(float x) {
     const float d = 1.0f + tl_exp_mid(-x), r = __builtin_amdgcn_rcpf(d);
     return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
 }
-// the least and largest magnitudes of a wave's values (as bits without the sign)
+// the least and largest magnitudes of a lane's values (as bits without the sign), and whether all of a wave's are of middling size
 struct TlMagnitudes {
     uint32_t least = 0xffffffffu, most = 0;
     __device__ __forceinline__ void take(float v) {
         const uint32_t u = __float_as_uint(v) << 1;
         least = min(least, u), most = max(most, u);
     }
-    __device__ __forceinline__ bool mid_silu() const { return !__any(most > __float_as_uint(TL_MID) << 1 || least < __float_as_uint(0x1p-60f) << 1); }
-    __device__ __forceinline__ bool mid_sigmoid() const { return !__any(most > __float_as_uint(TL_MID) << 1); }
+    __device__ __forceinline__ bool beyond_silu() const { return most > __float_as_uint(TL_MID) << 1 || least < __float_as_uint(0x1p-60f) << 1; }
+    __device__ __forceinline__ bool beyond_sigmoid() const { return most > __float_as_uint(TL_MID) << 1; }
+    __device__ __forceinline__ bool mid_silu() const { return !__any(beyond_silu()); }
+    __device__ __forceinline__ bool mid_sigmoid() const { return !__any(beyond_sigmoid()); }
 };
 
 // ---- scores bent by a cap ------------------------------------------------------------------------

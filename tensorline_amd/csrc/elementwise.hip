@@ -659,6 +659,31 @@ __global__ void silu_mul_vec_kernel(const T* __restrict__ gu, T* __restrict__ ou
         *reinterpret_cast<float4*>(dst) = make_float4(g[0], g[1], g[2], g[3]);
 }
 
+// The two forms of the gates (common.h) over the floats whose bits are first, first + 1, ..: counts[0] and [1] take how many have another SiLU
+// and another 1 / (1 + e^-x), [2] and [3] how many were of middling size for each.  For tests.
+__global__ __launch_bounds__(256) void gate_forms_kernel(uint32_t first, uint64_t n, uint32_t* __restrict__ counts) {
+    uint32_t silu = 0, sigmoid = 0, mid_silu = 0, mid_sigmoid = 0;
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
+        const float v = __uint_as_float(first + (uint32_t)i);
+        TlMagnitudes size;
+        size.take(v);
+        if (!size.beyond_silu()) ++mid_silu, silu += __float_as_uint(tl_silu_mid(v)) != __float_as_uint(v / (1.0f + expf(-v)));
+        if (!size.beyond_sigmoid()) ++mid_sigmoid, sigmoid += __float_as_uint(tl_sigmoid_mid(v)) != __float_as_uint(1.0f / (1.0f + expf(-v)));
+    }
+    if (silu) atomicAdd(counts, silu);
+    if (sigmoid) atomicAdd(counts + 1, sigmoid);
+    if (mid_silu) atomicAdd(counts + 2, mid_silu);
+    if (mid_sigmoid) atomicAdd(counts + 3, mid_sigmoid);
+}
+
+extern "C" int tl_gate_forms_differ(uint32_t first, long long n, uint32_t* counts, hipStream_t stream) {
+    TL_CHECK_ARG(n > 0 && n <= 1ll << 32 && counts, "tl_gate_forms_differ: bad range of %lld floats", n);
+    const long long blocks = (n + 255) / 256;
+    hipLaunchKernelGGL(gate_forms_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(256), 0, stream, first, (uint64_t)n, counts);
+    TL_CHECK_LAUNCH("tl_gate_forms_differ");
+    return 0;
+}
+
 extern "C" int tl_silu_mul(const void* gu, void* out, int dtype, int T, int I, hipStream_t stream) {
     TL_CHECK_ARG(T >= 0 && I > 0, "tl_silu_mul: bad sizes T=%d I=%d", T, I);
     TL_CHECK_ARG(T <= 65535 * 64, "tl_silu_mul: too many rows %d", T);

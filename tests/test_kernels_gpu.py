@@ -1132,13 +1132,30 @@ def test_silu_mul_of_gates_beyond_middling_ones(dtype, I):
     gu = (torch.randn(5, 2 * I, device=DEV) * torch.tensor([3.0, 30.0, 90.0, 1e-20, 1.0], device=DEV)[:, None]).to(dtype)
     gu[4, :I:3], gu[4, 1:I:3], gu[4, 2] = 0.0, float("-inf"), float("inf")
     got, g, u = K().silu_mul(gu), gu[:, :I].double(), gu[:, I:].double()
-    assert all(torch.equal(got[t:t + 1].isnan(), K().silu_mul(gu[t:t + 1]).isnan()) for t in range(5))
+    bits = torch.int16 if dtype == torch.bfloat16 else torch.int32
+    assert all(torch.equal(got[t:t + 1].view(bits), K().silu_mul(gu[t:t + 1]).view(bits)) for t in range(5))
+    beside = gu.clone()
+    beside[:, 3:I:7] = 100.0                                          # a column's bits do not depend on the columns beside it
+    kept = torch.arange(I, device=DEV) % 7 != 3
+    assert torch.equal(K().silu_mul(beside)[:, kept].view(bits), got[:, kept].view(bits))
     want = g / (1 + (-g).exp()) * u
     assert torch.equal(got.isnan(), want.isnan())
     # e^-v has no float beyond 2^128: there the result is 0, for 89 / 2^128 < 2^-121 times |u| at most (|u| is up to some hundreds here)
     t = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -21
     ok = ~want.isnan() & ~want.isinf()
     assert bool(((got.double() - want).abs() <= t * want.abs() + 2.0 ** -121 * u.abs() + 2.0 ** -126)[ok].all()) and bool((got.double() == want)[want.isinf()].all())
+
+
+def test_gates_of_middling_numbers_have_the_bits_of_the_general_form():
+    """All 2^32 floats: of those that a wave may take the short steps for, |v| <= 40 and for SiLU 2^-60 and more, none comes out with other bits
+    than by expf and the division."""
+    import ctypes
+    counts = torch.zeros(4, dtype=torch.int32, device=DEV)
+    K()._call("tl_gate_forms_differ", ctypes.c_uint32(0), ctypes.c_longlong(1 << 32), ctypes.c_void_p(counts.data_ptr()), K()._stream())
+    bits = lambda x: int(torch.tensor(x).view(torch.int32))
+    silu, sigmoid, mid_silu, mid_sigmoid = (c & 0xffffffff for c in counts.tolist())
+    assert (silu, sigmoid) == (0, 0)
+    assert mid_silu == 2 * (bits(40.0) - bits(2.0 ** -60) + 1) and mid_sigmoid == 2 * (bits(40.0) + 1)
 
 
 def test_argmax_and_ties():
@@ -1439,6 +1456,35 @@ def test_experts_in_wide_tiles(gated, Kd, F, N, monkeypatch):
         want[rows] = weights[rows].double() * (act @ down[e].double().T)
         slack = weights[rows].double() * ((act.abs() * 2.0 ** -8 + 1e-4) @ down[e].double().abs().T) + 1e-4
         assert bool(((got[True][rows].double() - want[rows]).abs() <= slack).all()), e
+
+
+@pytest.mark.parametrize("limit,alpha,shift", [(float("inf"), 1.0, 0.0), (float("inf"), 1.702, 0.0), (7.0, 1.702, 1.0)])
+def test_experts_gates_of_every_size(limit, alpha, shift, monkeypatch):
+    """The experts' gate for every finite bfloat16 number: sorted, so that waves of wide tiles have middling numbers only, and in disorder, so that they
+    have some beyond; and in tiles of 64 rows, which know one form.  The same bits each way, and within the rounding of the result (2^-9) and
+    of the float steps (of the exponent's argument, 89 at most: 2^-17; the others 2^-21); where e^-x passes the largest float the
+    result is 0 for at most 89 / 2^128 < 2^-121."""
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    v = v[torch.isfinite(v)].to(DEV)
+    v = v[v.float().abs().sort().indices]
+    T, E, Kd, F = v.numel(), 3, 64, 64
+    up, down = torch.zeros(E, 2 * F, Kd, device=DEV, dtype=torch.bfloat16), torch.eye(F, device=DEV, dtype=torch.bfloat16).repeat(E, 1, 1)
+    up[:, :F, 0], up[:, F:, 1] = 1, 0.75
+    ids, one = (torch.arange(T, dtype=torch.int32, device=DEV) * E // T)[:, None].contiguous(), torch.ones(T, 1, device=DEV)
+
+    def run(values, wide):
+        monkeypatch.setattr(K(), "_moe_takes_wide_tiles", lambda *a: wide)
+        h = torch.zeros(T, Kd, device=DEV, dtype=torch.bfloat16)
+        h[:, 0], h[:, 1] = values, 1
+        out = K().moe_experts(h, up, down, ids, one, limit, alpha, shift=shift)
+        assert torch.equal(out[:, :1].expand_as(out), out)
+        return out[:, 0].contiguous()
+    got, mixed = run(v, True), torch.randperm(T, device=DEV)
+    assert torch.equal(run(v[mixed], True).view(torch.int32), got[mixed].view(torch.int32))
+    assert torch.equal(run(v, False).view(torch.int32), got.view(torch.int32))
+    g = v.double().clamp(max=limit)
+    want = g / (1 + (-alpha * g).exp()) * (0.75 + shift)
+    assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -121).all())
 
 
 @pytest.mark.parametrize("E,top,F,N", [(7, 1, 64, 260), (9, 3, 320, 768), (13, 2, 640, 516), (37, 33, 192, 1280)])
