@@ -601,9 +601,10 @@ __global__ __launch_bounds__(MG_THREADS, 2) void moe_gemm_bf16_kernel(const bf16
 // their products took 543 and 304 us for gate and up and for down of 192 rows an expert (64 of 4,096 x 2,048) where this takes 427
 // and 270 (5.0 and 4.0 TB/s of matrices).
 // MW is the tile's rows in sixties-fours, chosen by the work-group, so that a tile of 70 rows does the products of 128.
-// The tiles of one expert, all its column tiles, go to one XCD (every eighth work-group id), whose L2 then holds the rows; of the last tiles, that are
-// fewer than there are XCDs, every XCD takes its share of the column tiles: whole ones gave the XCDs that had one a round of work-groups
-// more (64 experts of 2,048 x 1,408, 64 to 67 tiles, 188 -> 169 us).
+// The tiles of one expert, all its column tiles, go to one XCD (every eighth work-group id), whose L2 then holds the rows.  Of the last tiles, that are
+// fewer than there are XCDs, every XCD takes its share of the column tiles where the XCDs that had a whole one would have a round of work-groups
+// more (64 experts of 2,048 x 1,408, 67 tiles in 11 columns, 188 -> 169 us); elsewhere they would only fetch the rows once each (8 experts of 1,024 x
+// 1,024, 66 tiles in 4 columns 54 us whole and 71 dealt out, 67 in 8 97 and 104).
 // The matrix rows are asked for ahead of the tokens' rows, whose places have to be looked up.
 #define MGW_THREADS 512
 #define MGW_KT 64
@@ -616,15 +617,17 @@ __host__ __device__ __forceinline__ int moe_token(int pair, int top, uint32_t pe
     const uint32_t q = per_top ? (uint32_t)(((uint64_t)(uint32_t)pair * per_top) >> 32) : (uint32_t)pair;
     return (int)(q - (q * (uint32_t)top > (uint32_t)pair));
 }
-// which row tile and column tile a work-group has; `whole` of the `have` row tiles are dealt out whole
-__device__ __forceinline__ bool moe_wide_tile(int id, int have, int whole, int ntiles, int* mt, int* nt) {
+// which row tile and column tile a work-group has: 32 CUs to an XCD have one work-group each at a time
+__device__ __forceinline__ bool moe_wide_tile(int id, int have, int ntiles, int* mt, int* nt) {
+    const bool dealt = (((have + 7) >> 3) * ntiles + 31) >> 5 > (have * ntiles + 255) >> 8;
+    const int whole = dealt ? have >> 3 : (have + 7) >> 3;                       // row tiles of an XCD
     int local = id >> 3;
-    if (local < (whole >> 3) * ntiles) {
+    if (local < whole * ntiles) {
         *mt = (local / ntiles) * 8 + (id & 7), *nt = local % ntiles;
-        return true;
+    } else {
+        local = (local - whole * ntiles) * 8 + (id & 7);
+        *mt = whole * 8 + local / ntiles, *nt = local % ntiles;
     }
-    local = (local - (whole >> 3) * ntiles) * 8 + (id & 7);
-    *mt = whole + local / ntiles, *nt = local % ntiles;
     return *mt < have;
 }
 
@@ -731,9 +734,8 @@ __global__ __launch_bounds__(MGW_THREADS, 2) void moe_gemm_wide_kernel(const bf1
                                                                        const int32_t* __restrict__ tiles, int top, uint32_t per_top, int N, int K,
                                                                        int ntiles, float limit, float alpha, float shift) {
     extern __shared__ uint4 mgw_lds[];
-    const int have = tiles[0], whole = have & ~7;
     int mt, nt;
-    if (!moe_wide_tile(blockIdx.x, have, whole, ntiles, &mt, &nt)) return;
+    if (!moe_wide_tile(blockIdx.x, tiles[0], ntiles, &mt, &nt)) return;
     const int e = tiles[1 + 3 * mt], place0 = tiles[2 + 3 * mt], rows = tiles[3 + 3 * mt];
     const bf16_t* We = W + (size_t)e * (MODE == 1 ? 2 : 1) * N * K;
     const int n0 = nt * (MODE == 1 ? 128 : 256);

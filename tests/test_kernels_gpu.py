@@ -1487,10 +1487,10 @@ def test_experts_gates_of_every_size(limit, alpha, shift, monkeypatch):
     assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -121).all())
 
 
-@pytest.mark.parametrize("E,top,F,N", [(7, 1, 64, 260), (9, 3, 320, 768), (13, 2, 640, 516), (37, 33, 192, 1280)])
+@pytest.mark.parametrize("E,top,F,N", [(7, 1, 64, 260), (9, 3, 320, 768), (13, 2, 640, 516), (37, 33, 192, 1280), (9, 2, 2176, 4352), (15, 3, 2112, 4100)])
 def test_wide_tiles_that_are_no_multiple_of_the_xcds(E, top, F, N, monkeypatch):
-    """Row tiles of which fewer than eight are left over, alone or behind whole eights, with one to five column tiles and choices
-    of one to many: every tile once, bit for bit what tiles of 64 rows give."""
+    """Row tiles of which fewer than eight are left over, alone or behind whole eights, whole (one to five column tiles) or dealt out over the XCDs
+    (seventeen), and choices of one to many: every tile once, bit for bit what tiles of 64 rows give."""
     torch.manual_seed(E)
     T, Kd = 190, 128
     ids = torch.rand(T, E, device=DEV).topk(top, 1).indices.int().contiguous()
