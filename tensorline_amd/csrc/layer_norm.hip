@@ -78,7 +78,8 @@ __global__ __launch_bounds__(1024) void add_layernorm_kernel(float* __restrict__
 }
 
 // H a multiple of 4 and at most 16384: one pass over memory, 16-byte accesses, the row in registers meanwhile.
-template <typename O>
+// AHEAD: weight and bias are asked for with the row, which takes 79 registers for 54, so that a CU has one work-group of 1,024 threads for two.
+template <typename O, bool AHEAD>
 __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restrict__ x, LnBranch b1, LnBranch b2, float mult,
                                                                  const float* __restrict__ w, const float* __restrict__ b, float eps,
                                                                  O* __restrict__ out, const int32_t* __restrict__ rows, int H) {
@@ -87,14 +88,14 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     const size_t src = rows ? (size_t)rows[r] : (size_t)r;
     float* xr = x + src * H;
     const int n4 = H >> 2;
-    float4 v[LN_VPT], g[LN_VPT], s[LN_VPT];
+    float4 v[LN_VPT], g[AHEAD ? LN_VPT : 1], s[AHEAD ? LN_VPT : 1];
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < LN_VPT; ++i) {
         const int c4 = threadIdx.x + i * blockDim.x;
         if (c4 < n4) {
             float4 a = ln_load4(xr + 4 * c4);
-            if (w) g[i] = ln_load4(w + 4 * c4), s[i] = ln_load4(b + 4 * c4);       // used at the end
+            if (AHEAD && w) g[i] = ln_load4(w + 4 * c4), s[i] = ln_load4(b + 4 * c4);       // used at the end
             if (b1.y) {
                 float4 p = ln_branch4(b1, src * H + 4 * c4);
                 if (b2.y) {
@@ -127,11 +128,12 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     for (int i = 0; i < LN_VPT; ++i) {
         const int c4 = threadIdx.x + i * blockDim.x;
         if (c4 < n4) {
+            const float4 gw = AHEAD ? g[AHEAD ? i : 0] : ln_load4(w + 4 * c4), sb = AHEAD ? s[AHEAD ? i : 0] : ln_load4(b + 4 * c4);
             float4 o;
-            o.x = v[i].x * rstd * g[i].x + s[i].x;
-            o.y = v[i].y * rstd * g[i].y + s[i].y;
-            o.z = v[i].z * rstd * g[i].z + s[i].z;
-            o.w = v[i].w * rstd * g[i].w + s[i].w;
+            o.x = v[i].x * rstd * gw.x + sb.x;
+            o.y = v[i].y * rstd * gw.y + sb.y;
+            o.z = v[i].z * rstd * gw.z + sb.z;
+            o.w = v[i].w * rstd * gw.w + sb.w;
             ln_store4(orow + 4 * c4, o);
         }
     }
@@ -155,15 +157,29 @@ extern "C" int tl_add_layernorm(float* x, const float* y1, int parts1, long long
     int threads = (((vec ? H / 4 : H) + 63) / 64) * 64;
     if (threads > 1024) threads = 1024;
     if (vec && threads > 256 && n_rows >= 512) threads = H / 4 <= 256 * LN_VPT ? 256 : threads;   // many rows: several float4 per thread
+    // Weight and bias with the row where there is a work-group a CU at most, or where groups of 256 hold rows of 2,049 to 4,096; elsewhere what the
+    // registers cost is more than the wait.  us, two branches, with and at the end: 200 rows of 4,096 5.3 and 5.2, of 8,192 6.6 and 6.7; 300 of 3,584
+    // 8.0 and 6.3, of 8,192 13.1 and 11.4; 846 of 1,280 5.3 and 5.2, of 4,096 13.9 and 14.3, of 5,120 22.5 and 19.4; 2,048 of 1,280 11.4 and 10.1, of
+    // 3,584 24.9 and 25.6, of 8,192 69.1 and 58.6.
+    const bool ahead = n_rows <= 256 || (n_rows >= 512 && H > 2048 && H <= 4096);
     dim3 grid(n_rows), block(threads);
-#define TL_LN(KERNEL, OT) hipLaunchKernelGGL(KERNEL<OT>, grid, block, 0, stream, x, b1, b2, mult, w, b, eps, (OT*)out, rows, H)
+#define TL_LN(KERNEL, ...) hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, block, 0, stream, x, b1, b2, mult, w, b, eps, (TL_LN_OUT*)out, rows, H)
+#define TL_LN_ANY()                                                       \
+    do {                                                                  \
+        if (vec && ahead) TL_LN(add_layernorm_vec_kernel, TL_LN_OUT, true); \
+        else if (vec) TL_LN(add_layernorm_vec_kernel, TL_LN_OUT, false);    \
+        else TL_LN(add_layernorm_kernel, TL_LN_OUT);                        \
+    } while (0)
     if (out_dtype == TL_BF16) {
-        if (vec) TL_LN(add_layernorm_vec_kernel, bf16_t);
-        else TL_LN(add_layernorm_kernel, bf16_t);
+#define TL_LN_OUT bf16_t
+        TL_LN_ANY();
+#undef TL_LN_OUT
     } else if (out_dtype == TL_F32) {
-        if (vec) TL_LN(add_layernorm_vec_kernel, float);
-        else TL_LN(add_layernorm_kernel, float);
+#define TL_LN_OUT float
+        TL_LN_ANY();
+#undef TL_LN_OUT
     } else return tl_fail("tl_add_layernorm: unknown dtype %d", out_dtype);
+#undef TL_LN_ANY
 #undef TL_LN
     TL_CHECK_LAUNCH("tl_add_layernorm");
     return 0;

@@ -116,6 +116,23 @@ def test_branches_join_the_stream_and_the_layer_norm_reads_it(H, dtype):
     torch.testing.assert_close(got_x.double().cpu(), x.double() + 0.35 * (y1.double() + y2.double()), atol=1e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("T,H", [(257, 3584), (300, 16384), (511, 1280), (512, 2048), (520, 4100)])
+def test_layer_norms_of_many_rows(T, H):
+    """Rows enough for more than a work-group a CU, at the edges of where weight and bias come with the row and at the end."""
+    from tensorline_amd.ops import kernels
+    torch.manual_seed(H)
+    x, y, w, b = torch.randn(T, H, device=DEV) + 3.0, torch.randn(T, H, device=DEV), torch.randn(H, device=DEV), torch.randn(H, device=DEV)
+    total = x.double() + 0.5 * y.double()
+    want = P.layer_norm(total, w.double(), b.double(), 1e-5)
+    for dtype, tol in ((torch.float32, dict(atol=2e-5, rtol=2e-5)), (torch.bfloat16, dict(atol=3e-2, rtol=1e-2))):
+        got_x = x.clone()
+        torch.testing.assert_close(kernels.add_layernorm(got_x, kernels.ScaledBranches(y, None, 0.5), w, b, 1e-5, dtype).double(), want, **tol)
+        torch.testing.assert_close(got_x.double(), total, atol=1e-5, rtol=1e-5)
+    got_x = x.clone()
+    kernels.add_scaled_branches(got_x, kernels.ScaledBranches(y, None, 0.5))
+    torch.testing.assert_close(got_x.double(), total, atol=1e-5, rtol=1e-5)
+
+
 def test_layer_norm_keeps_its_digits_behind_a_large_mean():
     from tensorline_amd.ops import kernels
     torch.manual_seed(0)
