@@ -464,7 +464,7 @@ template <typename T>
 __global__ __launch_bounds__(1024) void rope_store_kernel(T* __restrict__ qkv, const int32_t* __restrict__ pos,
                                                          const float* __restrict__ inv_freq, T* __restrict__ k_cache, T* __restrict__ v_cache,
                                                          const int32_t* __restrict__ slots, int nq, int nkv, int d, int rot, int write_kv,
-                                                         int bs, const float* __restrict__ bias, int vec, uint32_t per_head_rcp) {
+                                                         int bs, const float* __restrict__ bias, int vec, uint32_t per_head_rcp, int values_last) {
     constexpr int V = 16 / sizeof(T);               // pairs to a thread where the sizes allow 16-byte accesses (vec)
     struct __attribute__((aligned(4))) Quad { float v[4]; };
     __shared__ __attribute__((aligned(16))) float cs_s[256], sn_s[256];          // one sine and cosine per rotated pair of the token
@@ -499,14 +499,15 @@ __global__ __launch_bounds__(1024) void rope_store_kernel(T* __restrict__ qkv, c
     const float p = (float)pos[t];
     const int busy = (half + 63) & ~63, spare = busy < (int)blockDim.x ? busy : 0;   // threads in waves with angles
     for (int k = threadIdx.x; k < half; k += blockDim.x) sincosf(p * inv_freq[k], &sn_s[k], &cs_s[k]);
-    if (slot >= 0 && (int)threadIdx.x >= spare) {
+    const auto values = [&](int from) {             // by the threads from `from` on
         const T* vrow = row + (size_t)nrot * d;
         const float* vbias = bias ? bias + (size_t)nrot * d : nullptr;
         const int page = slot / bs, off = slot - page * bs;
         T* vdst = v_cache + (size_t)page * nkv * d * bs + off;
-        for (int idx = threadIdx.x - spare; idx < nkv * d; idx += blockDim.x - spare)
+        for (int idx = threadIdx.x - from; idx < nkv * d; idx += blockDim.x - from)
             vdst[(size_t)idx * bs] = vbias ? tl_from_float<T>(tl_to_float(vrow[idx]) + vbias[idx]) : vrow[idx];
-    }
+    };
+    if (!values_last && slot >= 0 && (int)threadIdx.x >= spare) values(spare);
     __syncthreads();
     if (vec) {
         for (int idx = threadIdx.x; idx < items; idx += blockDim.x) {
@@ -566,8 +567,7 @@ __global__ __launch_bounds__(1024) void rope_store_kernel(T* __restrict__ qkv, c
     }
     // dims beyond the rotated part pass through: query dims only change when a bias is owed
     const int tail = d - rot;
-    if (!tail) return;
-    if (bias) {
+    if (tail && bias) {
         for (int idx = threadIdx.x; idx < nq * tail; idx += blockDim.x) {
             const int h = idx / tail, i = rot + (idx - h * tail);
             row[(size_t)h * d + i] = tl_from_float<T>(tl_to_float(row[(size_t)h * d + i]) + bias[h * d + i]);
@@ -579,6 +579,7 @@ __global__ __launch_bounds__(1024) void rope_store_kernel(T* __restrict__ qkv, c
         const T v = row[(size_t)(nq + h) * d + i];
         k_cache[((size_t)slot * nkv + h) * d + i] = bias ? tl_from_float<T>(tl_to_float(v) + bias[(nq + h) * d + i]) : v;
     }
+    if (values_last) values(0);
 }
 
 extern "C" int tl_rope_store(void* qkv, int dtype, const int32_t* pos, const float* inv_freq, void* k_cache,
@@ -597,13 +598,20 @@ extern "C" int tl_rope_store(void* qkv, int dtype, const int32_t* pos, const flo
     const int per_head = rot ? (vec ? rot / 2 / V : rot / 2) : 1;
     const uint32_t rcp = (uint32_t)(((1ull << 32) + per_head - 1) / per_head);      // 0: one a head
     const int items = (nq + nkv) * per_head;
-    const dim3 block(items <= 256 ? 256 : items <= 512 ? 512 : 1024);               // one item a thread: the first is asked for ahead
+    // One item a thread: the first is asked for ahead.  Steps of many tokens hide a work-group's waits behind the others and are bound by
+    // memory, where small work-groups, or values behind the keys, are better (us, as for few tokens and as here):
+    // - bfloat16 pairs one by one: 32 + 32 + 32 heads of 24, 700, 2,048, 4,000 tokens 7.1, 13.9, 23.7 and 6.6, 11.6, 18.8 (but 500 5.6 and 6.1);
+    // - values last, float32 28 + 4 + 4 heads of 128, 2,048 tokens 20.2 and 18.8 (4,000 36.1 and 35.4), without rotation 8 + 8 + 8 20.9 and 20.0;
+    //   bfloat16 with half of 128 rotated, 32 + 8 + 8 heads 15.3 and 14.8; fully rotated bfloat16 loses (12 + 2 + 2, 4,000 tokens 9.7 and 10.7).
+    const int values_last = T >= 2048 && (vec || !rot) && (dtype == TL_F32 || rot < d);
+    const bool small = vec ? values_last && dtype == TL_F32 && items % 256 == 0 && items <= 512 : dtype == TL_BF16 && T > 512;
+    const dim3 block(small || items <= 256 ? 256 : items <= 512 ? 512 : 1024);
     if (dtype == TL_F32)
         hipLaunchKernelGGL(rope_store_kernel<float>, grid, block, 0, stream, (float*)qkv, pos, inv_freq,
-                           (float*)k_cache, (float*)v_cache, slots, nq, nkv, d, rot, write_kv, bs, bias, vec, rcp);
+                           (float*)k_cache, (float*)v_cache, slots, nq, nkv, d, rot, write_kv, bs, bias, vec, rcp, values_last);
     else if (dtype == TL_BF16)
         hipLaunchKernelGGL(rope_store_kernel<bf16_t>, grid, block, 0, stream, (bf16_t*)qkv, pos, inv_freq,
-                           (bf16_t*)k_cache, (bf16_t*)v_cache, slots, nq, nkv, d, rot, write_kv, bs, bias, vec, rcp);
+                           (bf16_t*)k_cache, (bf16_t*)v_cache, slots, nq, nkv, d, rot, write_kv, bs, bias, vec, rcp, values_last);
     else
         return tl_fail("tl_rope_store: unknown dtype %d", dtype);
     TL_CHECK_LAUNCH("tl_rope_store");

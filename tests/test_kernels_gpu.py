@@ -599,6 +599,25 @@ def test_rope_store_in_groups_of_pairs(dtype, nq, nkv, d, rot, shift):
     assert bool((keys[left] == 7).all()) and bool((values[left] == 7).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,nq,nkv,d,rot", [(2048, 6, 2, 64, 64), (2060, 5, 1, 128, 32), (2051, 3, 3, 32, 0), (513, 4, 4, 24, 24), (2049, 33, 1, 128, 128)])
+def test_rope_store_of_many_tokens(dtype, T, nq, nkv, d, rot):
+    """Steps of many tokens, whose work-groups are smaller and whose values come last, leave what the same tokens in small steps do."""
+    torch.manual_seed(T)
+    pages, bs, width = T // 16 + 2, 16, (nq + 2 * nkv) * d
+    rows, bias = torch.randn(T, width, device=DEV).to(dtype), torch.randn(width, device=DEV)
+    pos, slots = torch.randint(0, 5000, (T,), dtype=torch.int32, device=DEV), torch.randperm(pages * bs, device=DEV)[:T].int()
+    slots[::7] = -1
+    inv = (10000.0 ** (-torch.arange(0, rot, 2, dtype=torch.float64) / rot)).float().to(DEV) if rot else None
+    left = []
+    for step in (T, 100):
+        x, kc, vc = rows.clone(), torch.full((pages, bs, nkv, d), 7.0, device=DEV).to(dtype), torch.full((pages, nkv, d, bs), 7.0, device=DEV).to(dtype)
+        for t in range(0, T, step):
+            K().rope_store(x[t:t + step], pos[t:t + step], inv, nq, nkv, d, kc, vc, slots[t:t + step], bias)
+        left.append((x, kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*left)) and not torch.equal(left[0][0], rows)
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 17, 40, 64])
 @pytest.mark.parametrize("nq,nkv,d,Kd", [(6, 2, 32, 192), (28, 4, 128, 3584), (4, 4, 64, 264), (5, 1, 96, 120)])
 def test_fused_projection_rotation_and_cache_write(M, nq, nkv, d, Kd):
