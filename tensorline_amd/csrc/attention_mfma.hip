@@ -598,18 +598,28 @@ __device__ __forceinline__ void am_tile_lds(const uint4* kt, const uint4* vt, in
 #pragma unroll
         for (int i = 0; i < 4; ++i) sv[4 * r + i] = MODE == 1 ? tl_capped(st[r][i], scale2, cap2) : st[r][i];
     if (MODE == 2) {
+        // The cap is asked for once and all biases are read first: key by key the compiler branches for the cap and waits for its bias sixteen
+        // times (us so and as here: 2,048 tokens of 32 / 2 heads of 32 48.9 and 39.4, 28 / 4 of 128 61 and 52, 512 behind 8,192 of 32 / 32 208 and 145;
+        // registers spill for it at a head size of 128: 100 tokens beside 40 decoding requests of 32 / 32 heads 103 and 108).
+        const auto bend = [&](auto add) {
+            if (cap2 > 0.f) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sv[i] = tl_score2<2>(sv[i], scale2, cap2, add(i));
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sv[i] = __builtin_fmaf(sv[i], scale2, add(i));
+            }
+        };
         if (__any(p_col - (kb + 63) < reach)) {
             int away = p_col - kb - 8 * g;                   // the column's distance from the lane's first key
             asm volatile("" : "+v"(away));                   // made here: sixteen distances kept across tiles would spill
+            float near[16];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    sv[4 * r + i] = tl_score2<2>(sv[4 * r + i], scale2, cap2, brow[tl_bias_at(away - 32 * (r >> 1) - 4 * (r & 1) - i, reach)]);
+            for (int i = 0; i < 16; ++i) near[i] = brow[tl_bias_at(away - 32 * (i >> 3) - (i & 7), reach)];
+            bend([&](int i) { return near[i]; });
         } else {
             const float far = brow[reach];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) sv[i] = tl_score2<2>(sv[i], scale2, cap2, far);
+            bend([&](int) { return far; });
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) vf[i] = AM_VFRAG(i);     // only now: their registers are in use until here
