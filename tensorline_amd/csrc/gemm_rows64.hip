@@ -35,7 +35,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define R64_SC 128
 #define R64_UNITS (R64_SC / 8)
 #define R64_ROWPAD 17
-#define R64_DEPTH 2                          // steps of loads in flight per wave (straight through shares of up to eight steps with four: 55 registers spilled, 0.65 to 0.9)
+#define R64_DEPTH 2                          // steps of loads in flight per wave (a form with four, straight through shares of up to eight steps: 55 registers spilled, 0.65 to 0.9)
 #define R64_A_WEIGHT 1                       // a group's loads of A, in units of one wave's loads of W (cost model)
 #define R64_AHEAD 8                          // shares that the second kernels ask for at once
 #define R64_MIN_WAVES 4
@@ -154,6 +154,7 @@ __global__ __launch_bounds__(THREADS) void gemm_rows64_kernel(
     // The loop runs without a branch, as long as every slot is refilled; at most three steps are left, and ask for what
     // there is.  (Steps asked for past a share's end, and zeros multiplied where its steps are odd, were up to three of seven:
     // with the same in the attention of these steps, 48 sequences of eight 7B layers 1,655 -> 1,615 us.)
+    static_assert(DEPTH == 2, "the loop and the remainder are written out for two slots");
     const std::integral_constant<int, 0> slot0;
     const std::integral_constant<int, 1> slot1;
     int base = 0;
