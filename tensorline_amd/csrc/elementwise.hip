@@ -601,9 +601,11 @@ extern "C" int tl_rope_store(void* qkv, int dtype, const int32_t* pos, const flo
     // One item a thread: the first is asked for ahead.  Steps of many tokens hide a work-group's waits behind the others and are bound by
     // memory, where small work-groups, or values behind the keys, are better (us, as for few tokens and as here):
     // - bfloat16 pairs one by one: 32 + 32 + 32 heads of 24, 700, 2,048, 4,000 tokens 7.1, 13.9, 23.7 and 6.6, 11.6, 18.8 (but 500 5.6 and 6.1);
-    // - values last, float32 28 + 4 + 4 heads of 128, 2,048 tokens 20.2 and 18.8 (4,000 36.1 and 35.4), without rotation 8 + 8 + 8 20.9 and 20.0;
-    //   bfloat16 with half of 128 rotated, 32 + 8 + 8 heads 15.3 and 14.8; fully rotated bfloat16 loses (12 + 2 + 2, 4,000 tokens 9.7 and 10.7).
-    const int values_last = T >= 2048 && (vec || !rot) && (dtype == TL_F32 || rot < d);
+    // - values last, float32 28 + 4 + 4 heads of 128, 2,048 tokens 20.2 and 18.8 (12 + 2 + 2, 17 MB, 9.2 and 9.7), bfloat16 with half of 128 rotated,
+    //   32 + 8 + 8 heads 15.3 and 14.8; fully rotated bfloat16 loses (12 + 2 + 2, 4,000 tokens 9.7 and 10.7);
+    // - without rotation there is less to hide: float32, 14 + 2 + 2 heads of 256, 631 tokens 11.0 and 9.8, 8 + 8 + 8 of 64, 1,500 tokens (9 MB) 9.9 and 10.1.
+    const double bytes = (double)T * (nq + 2 * nkv) * d * (dtype == TL_F32 ? 4 : 2);
+    const int values_last = bytes >= (rot ? 24e6 : 10e6) && (vec || !rot) && (dtype == TL_F32 || rot < d);
     const bool small = vec ? values_last && dtype == TL_F32 && items % 256 == 0 && items <= 512 : dtype == TL_BF16 && T > 512;
     const dim3 block(small || items <= 256 ? 256 : items <= 512 ? 512 : 1024);
     if (dtype == TL_F32)

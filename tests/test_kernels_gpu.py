@@ -600,7 +600,8 @@ def test_rope_store_in_groups_of_pairs(dtype, nq, nkv, d, rot, shift):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("T,nq,nkv,d,rot", [(2048, 6, 2, 64, 64), (2060, 5, 1, 128, 32), (2051, 3, 3, 32, 0), (513, 4, 4, 24, 24), (2049, 33, 1, 128, 128)])
+@pytest.mark.parametrize("T,nq,nkv,d,rot", [(2051, 20, 2, 128, 128), (4100, 20, 2, 128, 32), (3000, 3, 3, 192, 0), (513, 4, 4, 24, 24), (2049, 33, 1, 128, 128),
+                                             (2048, 28, 2, 128, 128)])
 def test_rope_store_of_many_tokens(dtype, T, nq, nkv, d, rot):
     """Steps of many tokens, whose work-groups are smaller and whose values come last, leave what the same tokens in small steps do."""
     torch.manual_seed(T)
