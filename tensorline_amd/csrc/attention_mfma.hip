@@ -728,7 +728,8 @@ __device__ __forceinline__ int at_v_swizzle(int row) { return (row >> 1) & 7; }
 // leave them there.  For steps whose work-groups leave most CUs idle behind long contexts: 489 tokens behind 3,072 beside 24
 // decoding requests (12 query and 2 key/value heads of 128, 94 work-groups) 36 us with the merge, 62 in two chains.
 // A third buffer, loads two tiles ahead, gives nothing (36 and 36 us; 512 behind 8,192 94 and 115).  A tile's addresses are a page id and
-// one product for K and one for V^T; in the last tile, which may reach beyond the keys, they are made key by key.
+// one product for K and one for V^T; in the last tile, which may reach beyond the keys, they are made key by key.  Of the forms at a head size of 128,
+// which have 128 registers, two chains with a cap spill 2 and those with a bias 3 (runs 5, two chains 11); no other form spills.
 template <int DC, int NT, int WAVES, int CH, int MODE, bool SPLIT>
 __global__ __launch_bounds__(CH * WAVES * 64, DC >= 8 ? 2 : 32 / WAVES) void attn_tile_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,

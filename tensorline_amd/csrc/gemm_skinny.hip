@@ -395,8 +395,9 @@ __global__ __launch_bounds__(MODE == MODE_SWIGLU ? 256 : 512) void gemm_skinny_k
 // us before and now, weights from memory, M = 1 / 8 / 16: with a sink 896 x 896 3.9, 2.9 / 4.0, 3.2 / 4.1, 3.3; 896 x 4,864 7.0, 4.8 / 7.2, 5.8 / 8.1,
 // 6.6; 2,048 x 6,144 9.1, 6.5 / 9.3, 7.5 / 9.9, 9.3; 3,584 x 3,584 7.7, 6.4 / 8.0, 7.0 / 8.8, 7.7; plain 1,024 x 1,024 3.6, 2.5 / 3.6, 2.6 / 3.6, 3.0; gate/up
 // 9,728 x 896 7.2, 5.9 / 7.1, 6.3 / 7.5, 6.6; 12,288 x 2,048 12.2, 10.4 / 12.7, 12.6 / 13.6, 13.6; q/k/v 1,152 x 896 5.0, 3.6 / 4.7, 3.9 / 5.0, 4.2; 3,072 x 2,048 7.2,
-// 5.3 / 7.2, 5.8 / 7.3, 6.3.  A decode step of 24 layers of 896 at one row 845 -> 676.  Above 640 work-groups the rate of the
-// stream counts and not the latency, and the kernel above has more waves to a CU: 32,000 x 2,048 in this form 26.7 for 23.7.
+// 5.3 / 7.2, 5.8 / 7.3, 6.3.  A decode step of 24 layers of 896 at one row 845 -> 676.  Above 640 tiles, or pairs of tiles
+// (1,280 work-groups in halves), the rate of the stream counts and not the latency, and the kernel above has more waves to a CU: 32,000 x 2,048
+// in this form 26.7 for 23.7.
 typedef int sk_i32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_rsrc(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);

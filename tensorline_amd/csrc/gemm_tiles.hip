@@ -21,8 +21,8 @@
 // takes them or by gt_add_kernel.
 //
 // us, here and in the library with its own choice of kernel (gate/up with the SiLU pass it needs; weights from memory), of sizes that
-// are taken (tl_gemm_tiles_plan): 2,048 rows of 17,920 x 1,536 gate/up 111 and 141, of 9,728 x 896 52 and 66, of 1,536 x 8,960 52 and 90;
-// 801 rows of 17,920 x 1,536 gate/up 51 and 69, of 1,536 x 8,960 30 and 44, of 2,048 x 1,536 15 and 18; 192 rows of the same 27
+// are taken (tl_gemm_tiles_plan): 2,048 rows of 17,920 x 1,536 gate/up 106 and 141, of 9,728 x 896 43 and 66, of 1,536 x 8,960 52 and 90;
+// 801 rows of 17,920 x 1,536 gate/up 47 and 69, of 1,536 x 8,960 30 and 44, of 2,048 x 1,536 15 and 18; 192 rows of the same 27
 // and 33, 16 and 38, 11 and 11; 128 rows of 37,888 x 3,584 gate/up 70 and 74, of 3,584 x 18,944 37 and 54, of 3,584 x 3,584 17 and 25.
 // Alone, plain products of 2^20 to 2^23 results and a K of 2,048 to 4,096 are 4% slower here in the mean, 20% at most (640 rows of
 // 2,048 x 2,816 23 and 20; 1,521 of 1,024 x 3,072 25 and 21); in whole steps the library is level there, and slower where the host
@@ -239,13 +239,13 @@ static double gt_time(const GtTile& t, int M, int N, int K, bool gated, int shar
     return us;
 }
 
-// Whether the gated form of a product cut into tiles of t runs in tiles of 128 x 256 with W straight into registers, two to a CU: where
-// there are more of them than CUs and the formula has them ahead.  Their figures are a fit to gated products of such sizes, 7% under
-// their times as the formula is under those of several rounds in the other tiles.  46 sizes that take them (of 9,728 x 896 to
-// 37,888 x 3,584, weights from memory) are 1.00 to 1.16 times as fast as in the plan's tile, 1.06 in the mean: us, 801 rows of 17,920 x
-// 1,536 55 and 51, 2,048 127 and 111, 380 rows of 37,888 x 3,584 115 and 107, 1,600 of 11,008 x 2,048 85 and 80; sizes that do not:
-// 1,300 rows of 17,920 x 1,536 69 and 79, 513 34 and 44, 1,521 of 9,728 x 896 30 and 32.  Plain products of up to 3,000 rows with a
-// choice of shares were level at best (256 tiles) or slower (384 tiles 28 and 36), and have no such form.
+// Whether the gated form of a product that the formula cuts into tiles of t runs in tiles of 128 x 256 with W straight into registers, two to a
+// CU: where there are more of them than CUs and the formula has them ahead.  It is 8% under their times in the mean of 33 sizes (of 9,728
+// x 896 to 37,888 x 3,584, 200 to 6,000 rows, weights from memory; 2 to 13%), 10% under those of the other tiles.  The ten of these sizes that take them are 1.05 to 1.17
+// times as fast as in the other tile, 1.09 in the mean: us, 801 rows of 17,920 x 1,536 53 and 47, 2,048 121 and 106, 380 of 37,888 x 3,584
+// 112 and 104, 1,600 of 11,008 x 2,048 83 and 78.  The others take 5% longer in them in the mean (1,300 rows of 17,920 x 1,536 73 and 82, 513
+// 36 and 43, 1,521 of 9,728 x 896 31 and 32), but for three that would take 3 to 8% less (1,000 of 17,920 x 1,536 68 and 63).  Plain products
+// of up to 3,000 rows with a choice of shares were level at best (256 tiles) or slower (384 tiles 28 and 36), and have no such form.
 static bool gt_goes_direct(const GtTile& t, const GtTile& direct, int M, int N, int K) {
     return (double)tl_ceil_div(M, direct.bm) * gt_ntiles(direct, N, true) > 256 &&
            gt_time(direct, M, N, K, true, 1, false) < gt_time(t, M, N, K, true, 1, false);

@@ -1056,11 +1056,14 @@ def _portion_splits(plan, S: int, num_heads: int, num_kv_heads: int, head_dim: i
                     total128: int) -> tuple[int, int]:
     """(keys per run, number of runs) for a step with prompt portions; (0, 1): every work-group of 128 columns walks its keys
     alone.  Where there is at most one work-group per two CUs, the longest walk sets the time, about 1.05 us per tile of 64 keys
-    in two chains (0.75 us at head sizes up to 64, 2.15 us at 256, in one chain); in runs at absolute positions, two work-groups
-    per CU (one at 256), a tile takes 1.5 us (1.1, 2) and the sums of every run pass through memory once.  Chosen where that is
-    estimated a quarter faster.  Measured, runs against walks, us: 64 tokens behind 3,000 (28 / 4 heads of 128) 27 / 52; 512
-    behind 8,192 107 / 136; 300 behind 3,000 (14 / 2 of 64) 28 / 40, but 1,000 behind 3,000 50 / 48; 64 behind 4,000 (16 / 1
-    of 256) 28 / 124; 1,024 behind 1,024 (12 / 2 of 128) 48 / 40, 600 behind 600 29 / 28."""
+    in two chains (0.75 us at head sizes up to 64, 2.15 us at 256, in one chain); runs lie at absolute positions, two work-groups
+    per CU (one at 256), and the sums of every run pass through memory once.  Chosen where that is estimated a quarter faster.  The
+    estimate (1.5 us a tile of a run, 1.1 and 2 at the other head sizes, and 9 us) is a fit to an earlier form of the kernel; now a tile
+    takes 1.05 us where the runs are few, and 16 us go ahead of them.  Measured, us, the runs chosen and walks: 64 tokens behind 3,000 (28 / 4 heads
+    of 128) 20 / 48; 512 behind 8,192 99 / 129; 489 behind 3,072 beside 24 decoding requests (12 / 2 of 128) 35 / 57; 300 behind 3,000 (14 / 2 of
+    64) 23 / 37; 64 behind 4,000 (16 / 1 of 256) 26 / 126; walks chosen, the best runs and walks: 1,000 behind 3,000 (14 / 2 of 64) 42 / 45, 1,024 behind
+    1,024 (12 / 2 of 128) 39 / 37, 600 behind 600 24 / 25.  Over nineteen such steps the choice takes 6% longer than the best one in the mean; at worst
+    500 behind 2,000 beside 40 requests (14 / 2 of 64) 31 for 25, 40 behind 1,000 (28 / 4 of 128) 22 for 15."""
     groups = total128 * num_kv_heads
     sees = [min(st + n, n + window + keep_first if window else st + n, n + chunk if chunk else st + n)
             for n, st in zip(plan.q_lens, plan.starts)]
