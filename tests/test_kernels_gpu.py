@@ -1886,3 +1886,33 @@ def test_17_to_64_rows_in_tiles_of_what_is_there(M, N, Kd):
         got = K().swiglu_gate_up(K().NormedRows(a, nxt.sumsq, N, 1e-6), w, ws)
         gate, up = (a.double() @ w.double().T / (x.double().pow(2).mean(1, keepdim=True) + 1e-6).sqrt()).chunk(2, 1)
         torch.testing.assert_close(got.double(), torch.nn.functional.silu(gate) * up, atol=1e-4, rtol=2.0 ** -8 + 1e-4)
+
+
+@pytest.mark.parametrize("M,N,Kd", [(17, 130, 64), (32, 300, 2048), (33, 129, 2064), (97, 2051, 4112), (300, 1000, 896), (700, 5000, 2050)])
+def test_linear_float_where_halves_lose_the_smallest_values(M, N, Kd):
+    """Rows whose large values meet zeros in the matrix, and the other way round, so that a result is made of values 2^-30 of their
+    segment's largest, which a half no longer holds: the bound of K float multiply-adds all the same.  Rows and columns of zeros give zeros,
+    and a row has the same bits whatever rows come along and whether the matrix' ranges are given or made."""
+    torch.manual_seed(M + Kd)
+    a, w, b = torch.randn(M, Kd, device=DEV), torch.randn(N, Kd, device=DEV), torch.randn(N, device=DEV)
+    a[1, ::2] *= 2.0 ** 30                                   # meets columns that are zero there
+    w[3, ::2] = 0.0
+    w[5, 1::2] *= 2.0 ** 40                                  # meets a row that is zero there
+    a[2, 1::2] = 0.0
+    a[4], w[7] = 0.0, 0.0
+    w[8] = 0.0
+    w[8, Kd - 1] = 1.0                                       # picks one value out of every row, the smallest too
+    a[6, Kd - 1], a[9, Kd - 1] = 2.0 ** -30, 2.0 ** -100
+    ws = K().shuffle_weight_float(w)
+    ranges = K().weight_ranges(ws, N, Kd)
+    got = K().linear(a, w, b, shuffled=ws)
+    want, size = a.double() @ w.double().T + b.double(), a.double().abs() @ w.double().abs().T + b.double().abs()
+    assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())
+    plain_sums = K().linear(a, w, shuffled=ws, ranges=ranges)
+    assert bool((plain_sums[4] == 0).all()) and bool((plain_sums[:, 7] == 0).all())
+    small = plain_sums[:, 8].double() - a[:, Kd - 1].double()        # of one product each, within the float's last place
+    assert bool((small.abs() <= 2.0 ** -22 * a[:, Kd - 1].double().abs()).all())
+    assert torch.equal(K().linear(a, w, b, shuffled=ws, ranges=ranges), got)
+    assert torch.equal(K().linear(a[:17], w, b, shuffled=ws, ranges=ranges), got[:17])
+    with pytest.raises(K().KernelError):
+        K().linear(a, w, b, shuffled=ws, ranges=ranges[1:])
