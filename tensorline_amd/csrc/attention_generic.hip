@@ -1,7 +1,8 @@
 // The entry point of the any-shape attention (attention_generic_kernel.h) and its float instantiations;
 // the bfloat16 ones are compiled in attention_generic_bf16.hip.  Float steps of one token per sequence go to
-// attention_float_decode.h where it takes them.
+// attention_float_decode.h, others to attention_float_tile.h, where those take them.
 #include "attention_float_decode.h"
+#include "attention_float_tile.h"
 #include "attention_generic_kernel.h"
 
 void tl_attention_generic_bf16(const AgLaunch& a);
@@ -67,6 +68,8 @@ extern "C" int tl_attention_generic(const void* q, int q_stride, const void* k_c
     a.smem = smem; a.stream = stream; a.sinks = sinks; a.softcap = softcap; a.bias = TlBias{bias, bias_reach};
     if (dtype == TL_F32 && afd_takes(a, max_query_len, S))
         afd_launch(a, S);
+    else if (dtype == TL_F32 && aft_takes(a))
+        aft_launch(a, S, max_query_len);
     else if (dtype == TL_F32)
         ag_launch_all<float>(a);
     else if (dtype == TL_BF16)

@@ -1,8 +1,8 @@
 // Causal attention of the step's tokens over the paged cache, for any head size that is a multiple
 // of 16 up to 256, any group size, any page size and both storage types; all arithmetic in float.
 // Products run on the matrix cores' float instruction (v_mfma_f32_16x16x4_f32: float in, float
-// out, no reduced precision anywhere): this is the attention of the true 32-bit path (one-token steps at head
-// sizes 64 and 128: attention_float_decode.h), and of bfloat16 shapes the bfloat16 matrix-core kernel does not take.
+// out, no reduced precision anywhere): this is the attention of the true 32-bit path (at head sizes 64 and 128 one-token steps
+// go to attention_float_decode.h and portions to attention_float_tile.h), and of bfloat16 shapes the bfloat16 matrix-core kernel does not take.
 //
 // A token at position p of sequence s attends to keys [lo, p] of that sequence, lo = 0, p - window + 1
 // for a windowed layer or the start of p's chunk for a chunked one, and to the first keys a layer keeps

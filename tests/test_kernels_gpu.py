@@ -1916,3 +1916,71 @@ def test_linear_float_where_halves_lose_the_smallest_values(M, N, Kd):
     assert torch.equal(K().linear(a[:17], w, b, shuffled=ws, ranges=ranges), got[:17])
     with pytest.raises(K().KernelError):
         K().linear(a, w, b, shuffled=ws, ranges=ranges[1:])
+
+
+@pytest.mark.parametrize("nq,nkv,d,bs", [(4, 4, 64, 4), (14, 2, 64, 16), (28, 4, 128, 16), (3, 1, 128, 8), (40, 2, 64, 128), (130, 1, 128, 16)])
+@pytest.mark.parametrize("kw", [{}, dict(sink=True), dict(window=70), dict(window=44, keep_first=5), dict(window=9, keep_first=40), dict(chunk=96)])
+def test_float_attention_of_prompt_portions(nq, nkv, d, bs, kw):
+    """The float kernel of portions: columns that end within a wave's 32 and a work-group's 128, one token beside portions, keys that end
+    within a page, four keys and a tile of 32, every mask.  Against 64 bits, as the one-token steps."""
+    lens, q_lens = [33, 1, 32, 300, 257, 129, 70], [33, 1, 31, 65, 1, 128, 17]
+    got, want = _attention_case(torch.float32, nq, nkv, d, bs, lens, q_lens, seed=nq + d, **kw)
+    torch.testing.assert_close(got, want, **tol(torch.float32, 2e-5))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("what", ["cut", "strided", "not finite", "tiny", "huge"])
+def test_float_attention_of_prompt_portions_at_their_limits(d, what):
+    """A position's bits do not depend on how its sequence is cut, nor on rows' strides.  Infinities and NaN in a key, a value or a query give
+    what plain float arithmetic gives, in the tiles and columns that see them, and every other column stays as it is; values of
+    2^-70 and 2^70 are as close to 64 bits as others."""
+    torch.manual_seed(d)
+    nq, nkv, bs, n = 6, 2, 16, 200
+    kc, vc = torch.randn(16, bs, nkv, d, device=DEV), torch.randn(16, nkv, d, bs, device=DEV)
+    table = torch.randperm(16, device=DEV)[:13].to(torch.int32)[None].contiguous()
+    q = torch.randn(n, nq * d, device=DEV)
+    if what in ("tiny", "huge"):
+        by = 2.0 ** -70 if what == "tiny" else 2.0 ** 70
+        kc, q, vc = kc * by, q / by, vc * by
+
+    def run(lo, hi, rows=None):
+        from tensorline_amd.engine.batch import StepFacts
+        facts = StepFacts(max_context=hi, max_query_len=hi - lo, decode_only=False, num_seqs=1, q_lens=[hi - lo], starts=[lo])
+        i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+        return K().paged_attention(q[lo:hi] if rows is None else rows, kc, vc, table, i32(*[0] * (hi - lo)), i32(*range(lo, hi)), nq, nkv, d, d ** -0.5,
+                                   q_start=i32(0, hi - lo), ctx_start=i32(lo), plan=facts)
+    rows = table[0].long()
+    def want():
+        kf = kc[rows].view(-1, nkv, d)[:n].double().cpu()
+        vf = vc[rows].permute(0, 3, 1, 2).reshape(-1, nkv, d)[:n].double().cpu()
+        return plain.causal_attention(q.double().cpu().view(n, nq, d), kf, vf, d ** -0.5).reshape(n, nq * d).to(DEV)
+    got = run(0, n)
+    scale = vc.abs().max().item()
+    torch.testing.assert_close(got.double() / scale, want() / scale, atol=2e-5, rtol=2e-5)
+    if what == "cut":
+        for cut in (10, 33, 100, 160):
+            assert torch.equal(torch.cat((run(0, cut), run(cut, n))), got)
+    if what == "strided":
+        wide = torch.full((n, nq * d + 3), float("nan"), device=DEV)
+        wide[:, 1:nq * d + 1] = q
+        assert torch.equal(run(0, n, wide[:, 1:nq * d + 1]), got)
+    if what == "not finite":
+        key = 70                                             # of key/value head 1: heads 3 to 5
+        page, at = int(table[0, key // bs]), key % bs
+        vc[page, 1, 5, at] = float("inf")
+        after = run(0, n).view(n, nq, d)
+        assert bool((after[key:, 3:, 5] == float("inf")).all())
+        near = key // 32 * 32                                # (what a masked weight of zero makes of an infinity in its tile is left open)
+        same = torch.ones(n, nq, d, dtype=torch.bool, device=DEV)
+        same[near:, 3:, 5] = False
+        assert torch.equal(after[same].isfinite(), torch.ones_like(after[same], dtype=torch.bool))
+        torch.testing.assert_close(after[same], got.view(n, nq, d)[same], atol=1e-5, rtol=1e-5)
+        vc[page, 1, 5, at] = 1.0
+        kc[page, at, 1, 7] = float("-inf")                   # a score of -inf hides the key, +inf makes the row NaN
+        after, sign = run(0, n).view(n, nq, d), q.view(n, nq, d)[key:, 3:, 7] > 0
+        assert bool(after[key:, 3:][sign].isfinite().all()) and bool(after[key:, 3:][~sign].isnan().all())
+        assert torch.equal(after[:near], got.view(n, nq, d)[:near]) and torch.equal(after[:, :3], got.view(n, nq, d)[:, :3])
+        kc[page, at, 1, 7] = 0.5
+        q[40, 2 * d + 3] = float("nan")
+        after, before = run(0, n).view(n, nq, d), None
+        assert bool(after[40, 2].isnan().all()) and int(after.isnan().sum()) == d
