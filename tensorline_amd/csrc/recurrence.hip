@@ -24,12 +24,21 @@
 // template size); queries, keys, decays and values of 16 tokens at a time go through LDS, the next
 // chunk's on their way in registers meanwhile; a column's sixteen shares of an output are left in
 // LDS and added in ascending order of the rows once per chunk.
+//
+// Steps that bring portions of more than a chunk (HELP) have a second four waves to a work-group, one to a SIMD, that bring the chunks to LDS
+// (SiLU and decays among it), and add up and write the outputs of the chunk before, while the first four do nothing but walk: what a token
+// costs is then the walk's instructions and reads alone.  Sequences of 803, 211 and 507 tokens, us: 16 heads of 128 x 128 with one decay 219 -> 138,
+// 32 of 64 x 64 with a decay per channel 127 -> 87; one of 2,048 547 -> 291 and 317 -> 187.  Where more work-groups come than CUs hold two of, the
+// second four waves are in the way (40 sequences of 33 tokens 104 and 118, eight of 100 61 and 59 or 84 and 96), and one chunk leaves them nothing to do.
 #include "common.h"
 
 #include <math.h>
 
 #define REC_MAX_DK 256
 #define REC_COLS 16
+#define REC_HELP_DK 128        // (beyond, LDS does not hold two chunks)
+#define REC_HELP_TOKENS 16
+#define REC_HELP_GROUPS 512
 
 __device__ __forceinline__ float rec_silu(float z) { return z / (1.0f + expf(-z)); }
 
@@ -39,8 +48,8 @@ __device__ __forceinline__ float rec_softplus(float z) { return fmaxf(z, 0.f) + 
 // MODE 0: a decay per head; 1: per token and key channel; 2: a step size per token and head.  In mode 2
 // wlog is the step [T, >= H] (row stride ldw), decay is rate_log [H], bonus is step_bias [H], skip [H] or
 // null, and head h reads queries and keys of group h / share.
-template <int R, int MODE>
-__global__ __launch_bounds__(256) void linear_recurrence_kernel(
+template <int R, int MODE, bool HELP>
+__global__ __launch_bounds__(HELP ? 512 : 256) void linear_recurrence_kernel(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v, int ldv,
     const float* __restrict__ wlog, int ldw, const float* __restrict__ decay, const float* __restrict__ bonus,
     const float* __restrict__ skip, int share,
@@ -51,11 +60,13 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(
     constexpr int DKP = 16 * R;                       // rows the tile holds; those beyond dk stay zero
     constexpr int REC_TB = R == 16 ? 8 : 16;          // tokens per chunk (fewer for the largest tile: LDS)
     constexpr int PER = REC_TB * DKP / 256;           // elements of a [REC_TB][DKP] tile per thread
-    __shared__ __attribute__((aligned(16))) float qs[REC_TB][DKP], ks[REC_TB][DKP], ws[PER_TOKEN ? REC_TB : 1][DKP];
-    __shared__ float vs[REC_TB][REC_COLS];
-    __shared__ float dts[REC_TB], decs[REC_TB];       // mode 2: a token's step size and its decay
-    __shared__ float part[16][REC_TB][REC_COLS];      // a row group's share of every output of the chunk
-    const int tid = threadIdx.x, lane = tid & 63, g = tid >> 6;
+    constexpr int BUFS = HELP ? 2 : 1, VBUFS = HELP ? 3 : 1;     // (values are read again with the outputs, a chunk later)
+    __shared__ __attribute__((aligned(16))) float qs_of[BUFS][REC_TB][DKP], ks_of[BUFS][REC_TB][DKP], ws_of[BUFS][PER_TOKEN ? REC_TB : 1][DKP];
+    __shared__ float vs_of[VBUFS][REC_TB][REC_COLS];
+    __shared__ float dts_of[BUFS][REC_TB], decs_of[BUFS][REC_TB];        // mode 2: a token's step size and its decay
+    __shared__ float part_of[BUFS][16][REC_TB][REC_COLS];                // a row group's share of every output of the chunk
+    const bool helper = HELP && threadIdx.x >= 256;
+    const int tid = threadIdx.x & 255, lane = tid & 63, g = tid >> 6;
     const int col = lane & 15, rg = 4 * g + (lane >> 4);
     const int j0 = blockIdx.x * REC_COLS, h = blockIdx.y, s = blockIdx.z;
     const int r0 = q_start[s], r1 = q_start[s + 1];
@@ -68,7 +79,7 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(
 #pragma unroll
     for (int rr = 0; rr < R; ++rr) {
         const int i = rg * R + rr;
-        S[rr] = (i < dk && col_ok) ? st[(size_t)i * dv + j] : 0.f;
+        S[rr] = (i < dk && col_ok && !helper) ? st[(size_t)i * dv + j] : 0.f;
         ur[rr] = (PER_TOKEN && bonus && i < dk) ? bonus[h * dk + i] : 1.f;
     }
     const float dec = MODE == 0 ? decay[h] : 1.f;
@@ -93,30 +104,46 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(
         vreg = (tt < n && j0 + jj < dv) ? v[(size_t)(t0 + tt) * ldv + h * dv + j0 + jj] : 0.f;
         if (STEPS) dtreg = tid < n ? wlog[(size_t)(t0 + tid) * ldw + h] : 0.f;
     };
-    auto stash = [&](int n) {
+    auto stash = [&](int n, int buf, int vbuf) {
+        float *qs = &qs_of[buf][0][0], *ks = &ks_of[buf][0][0], *ws = &ws_of[buf][0][0], *vs = &vs_of[vbuf][0][0];
+        if (silu_inputs) {
+            TlMagnitudes size;                        // numbers of middling size: the same bits in half the instructions
+#pragma unroll
+            for (int it = 0; it < PER; ++it) {
+                size.take(qreg[it] == 0.f ? 1.f : qreg[it]);           // zeros stay as they are
+                size.take(kreg[it] == 0.f ? 1.f : kreg[it]);
+            }
+            size.take(vreg == 0.f ? 1.f : vreg);
+            auto silu = [](float z) { return z == 0.f ? z : tl_silu_mid(z); };
+            if (size.mid_silu()) {
+#pragma unroll
+                for (int it = 0; it < PER; ++it) qreg[it] = silu(qreg[it]), kreg[it] = silu(kreg[it]);
+                vreg = silu(vreg);
+            } else {
+#pragma unroll
+                for (int it = 0; it < PER; ++it) qreg[it] = rec_silu(qreg[it]), kreg[it] = rec_silu(kreg[it]);
+                vreg = rec_silu(vreg);
+            }
+        }
 #pragma unroll
         for (int it = 0; it < PER; ++it) {
             const int idx = tid + it * 256, tt = idx / DKP, i = idx - tt * DKP;
             const bool ok = tt < n && i < dk;
-            (&qs[0][0])[idx] = silu_inputs ? rec_silu(qreg[it]) : qreg[it];
-            (&ks[0][0])[idx] = silu_inputs ? rec_silu(kreg[it]) : kreg[it];
-            if (PER_TOKEN) (&ws[0][0])[idx] = ok ? expf(-expf(wreg[it])) : 0.f;
+            qs[idx] = qreg[it];
+            ks[idx] = kreg[it];
+            if (PER_TOKEN) ws[idx] = ok ? expf(-expf(wreg[it])) : 0.f;
         }
-        if (tid < REC_TB * REC_COLS) (&vs[0][0])[tid] = silu_inputs ? rec_silu(vreg) : vreg;
+        if (tid < REC_TB * REC_COLS) vs[tid] = vreg;
         if (STEPS && tid < REC_TB) {
             const float dt = rec_softplus(dtreg + step_bias);
-            dts[tid] = dt;
-            decs[tid] = expf(-rate * dt);
+            dts_of[buf][tid] = dt;
+            decs_of[buf][tid] = expf(-rate * dt);
         }
     };
-
-    fetch(r0, min(REC_TB, r1 - r0));
-    stash(min(REC_TB, r1 - r0));
-    __syncthreads();
-    for (int t0 = r0; t0 < r1; t0 += REC_TB) {
-        const int n = min(REC_TB, r1 - t0);
-        const bool more = t0 + REC_TB < r1;
-        if (more) fetch(t0 + REC_TB, min(REC_TB, r1 - t0 - REC_TB));
+    auto walk = [&](int n, int buf, int vbuf) {
+        float (&qs)[REC_TB][DKP] = qs_of[buf], (&ks)[REC_TB][DKP] = ks_of[buf], (&ws)[PER_TOKEN ? REC_TB : 1][DKP] = ws_of[buf];
+        float (&vs)[REC_TB][REC_COLS] = vs_of[vbuf], (&part)[16][REC_TB][REC_COLS] = part_of[buf];
+        float *dts = dts_of[buf], *decs = decs_of[buf];
 #pragma unroll 4
         for (int tt = 0; tt < n; ++tt) {
             const float vj = STEPS ? dts[tt] * vs[tt][col] : vs[tt][col];
@@ -136,19 +163,59 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(
             }
             part[rg][tt][col] = acc;
         }
-        __syncthreads();
-        {
-            const int tt = tid / REC_COLS, jj = tid % REC_COLS;
-            if (tt < n && j0 + jj < dv) {
-                float sum = part[0][tt][jj];
+    };
+    auto write = [&](int t0, int n, int buf, int vbuf) {
+        const int tt = tid / REC_COLS, jj = tid % REC_COLS;
+        if (tt < n && j0 + jj < dv) {
+            float (&part)[16][REC_TB][REC_COLS] = part_of[buf];
+            float sum = part[0][tt][jj];
 #pragma unroll
-                for (int r = 1; r < 16; ++r) sum += part[r][tt][jj];       // the row groups in ascending order
-                if (STEPS) sum += skip_h * vs[tt][jj];
-                out[(size_t)(t0 + tt) * ldo + h * dv + j0 + jj] = sum;
-            }
+            for (int r = 1; r < 16; ++r) sum += part[r][tt][jj];       // the row groups in ascending order
+            if (STEPS) sum += skip_h * vs_of[vbuf][tt][jj];
+            out[(size_t)(t0 + tt) * ldo + h * dv + j0 + jj] = sum;
         }
-        if (more) stash(min(REC_TB, r1 - t0 - REC_TB));
+    };
+    auto length = [&](int t0) { return min(REC_TB, r1 - t0); };
+
+    if constexpr (HELP) {
+        if (helper) {
+            fetch(r0, length(r0));
+            stash(length(r0), 0, 0);
+            if (r0 + REC_TB < r1) fetch(r0 + REC_TB, length(r0 + REC_TB));
+        }
         __syncthreads();
+        int buf = 0, vbuf = 0;
+        for (int t0 = r0; t0 < r1; t0 += REC_TB) {
+            const int before = vbuf == 0 ? 2 : vbuf - 1, after = vbuf == 2 ? 0 : vbuf + 1;
+            if (helper) {                             // (a chunk before the last one has all its tokens)
+                if (t0 > r0) write(t0 - REC_TB, REC_TB, buf ^ 1, before);
+                if (t0 + REC_TB < r1) {
+                    stash(length(t0 + REC_TB), buf ^ 1, after);
+                    if (t0 + 2 * REC_TB < r1) fetch(t0 + 2 * REC_TB, length(t0 + 2 * REC_TB));
+                }
+            } else
+                walk(length(t0), buf, vbuf);
+            __syncthreads();
+            buf ^= 1, vbuf = after;
+        }
+        if (helper) {
+            const int t0 = r0 + (r1 - r0 - 1) / REC_TB * REC_TB;
+            write(t0, r1 - t0, buf ^ 1, vbuf == 0 ? 2 : vbuf - 1);
+            return;
+        }
+    } else {
+        fetch(r0, length(r0));
+        stash(length(r0), 0, 0);
+        __syncthreads();
+        for (int t0 = r0; t0 < r1; t0 += REC_TB) {
+            const bool more = t0 + REC_TB < r1;
+            if (more) fetch(t0 + REC_TB, length(t0 + REC_TB));
+            walk(length(t0), 0, 0);
+            __syncthreads();
+            write(t0, length(t0), 0, 0);
+            if (more) stash(length(t0 + REC_TB), 0, 0);
+            __syncthreads();
+        }
     }
 #pragma unroll
     for (int rr = 0; rr < R; ++rr) {
@@ -163,13 +230,13 @@ extern "C" int tl_linear_recurrence_takes(int dk) { return dk > 0 && dk <= REC_M
 // [T, >= H*dk] with row stride ldw, bonus [H, dk] or null; per_token 2: q, k [T, >= (H/share)*dk], wlog the
 // steps [T, >= H], decay rate_log [H], bonus step_bias [H] or null, skip [H] or null.  state: float, a
 // request's [H, dk, dv] at state + slot * state_stride.  out float [T, >= H*dv].  S sequences, rows
-// q_start[s] .. q_start[s+1].
+// q_start[s] .. q_start[s+1]; longest: the most tokens that one of them brings, 0 where the caller does not know.
 extern "C" int tl_linear_recurrence(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
                                     const float* wlog, int ldw, const float* decay, const float* bonus, int per_token,
                                     const float* skip, int share,
                                     float* state, long long state_stride, const int32_t* state_slots,
                                     const int32_t* q_start, float* out, int ldo, int S, int H, int dk, int dv,
-                                    int silu_inputs, hipStream_t stream) {
+                                    int silu_inputs, int longest, hipStream_t stream) {
     TL_CHECK_ARG(S >= 0 && H > 0 && dv > 0, "tl_linear_recurrence: bad sizes S=%d H=%d dv=%d", S, H, dv);
     TL_CHECK_ARG(tl_linear_recurrence_takes(dk), "tl_linear_recurrence: a key size of %d is not served (at most %d)", dk, REC_MAX_DK);
     TL_CHECK_ARG(per_token >= 0 && per_token <= 2, "tl_linear_recurrence: unknown form %d", per_token);
@@ -183,25 +250,31 @@ extern "C" int tl_linear_recurrence(const float* q, int ldq, const float* k, int
                  "tl_linear_recurrence: decays are missing");
     TL_CHECK_ARG(H <= 65535 && S <= 65535, "tl_linear_recurrence: too many heads or sequences for one launch");
     if (S == 0) return 0;
-    dim3 grid(tl_ceil_div(dv, REC_COLS), H, S), block(256);
-#define GO(R)                                                                                                            \
-    do {                                                                                                                 \
-        if (per_token == 1)                                                                                              \
-            hipLaunchKernelGGL((linear_recurrence_kernel<R, 1>), grid, block, 0, stream, q, ldq, k, ldk, v, ldv, wlog, ldw, \
-                               decay, bonus, skip, share, state, state_stride, state_slots, q_start, out, ldo, H, dk, dv, silu_inputs); \
-        else if (per_token == 2)                                                                                         \
-            hipLaunchKernelGGL((linear_recurrence_kernel<R, 2>), grid, block, 0, stream, q, ldq, k, ldk, v, ldv, wlog, ldw, \
-                               decay, bonus, skip, share, state, state_stride, state_slots, q_start, out, ldo, H, dk, dv, silu_inputs); \
-        else                                                                                                             \
-            hipLaunchKernelGGL((linear_recurrence_kernel<R, 0>), grid, block, 0, stream, q, ldq, k, ldk, v, ldv, wlog, ldw, \
-                               decay, bonus, skip, share, state, state_stride, state_slots, q_start, out, ldo, H, dk, dv, silu_inputs); \
+    const dim3 grid(tl_ceil_div(dv, REC_COLS), H, S);
+    const bool help = longest > REC_HELP_TOKENS && dk <= REC_HELP_DK && (long long)grid.x * H * S <= REC_HELP_GROUPS;
+    const dim3 block(help ? 512 : 256);
+#define GO_MODE(R, MODE, HELP)                                                                                          \
+    hipLaunchKernelGGL((linear_recurrence_kernel<R, MODE, HELP>), grid, block, 0, stream, q, ldq, k, ldk, v, ldv, wlog, ldw, \
+                       decay, bonus, skip, share, state, state_stride, state_slots, q_start, out, ldo, H, dk, dv, silu_inputs)
+#define GO_HELP(R, HELP)                         \
+    do {                                         \
+        if (per_token == 1) GO_MODE(R, 1, HELP); \
+        else if (per_token == 2) GO_MODE(R, 2, HELP); \
+        else GO_MODE(R, 0, HELP);                \
+    } while (0)
+#define GO(R)                       \
+    do {                            \
+        if (help) GO_HELP(R, true); \
+        else GO_HELP(R, false);     \
     } while (0)
     if (dk <= 16) GO(1);
     else if (dk <= 32) GO(2);
     else if (dk <= 64) GO(4);
     else if (dk <= 128) GO(8);
-    else GO(16);
+    else GO_HELP(16, false);
 #undef GO
+#undef GO_HELP
+#undef GO_MODE
     TL_CHECK_LAUNCH("tl_linear_recurrence");
     return 0;
 }

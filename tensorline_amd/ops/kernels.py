@@ -1718,7 +1718,8 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ctx, st
     _call("tl_linear_recurrence", _ptr(q), ld(q), _ptr(k), ld(k), _ptr(v), ld(v), _ptr(wlog), ld(wlog) if per_token else 0,
           _ptr(decay), _ptr(bonus), per_token, _ptr(skip if per_token == 2 else None), share,
           st, ctypes.c_longlong(stride), _ptr(ctx.state_slots),
-          _ptr(ctx.q_start), _ptr(out), heads * dv, ctx.num_seqs, heads, dk, dv, 1 if silu_inputs else 0, _stream())
+          _ptr(ctx.q_start), _ptr(out), heads * dv, ctx.num_seqs, heads, dk, dv, 1 if silu_inputs else 0,
+          int(facts.max_query_len) if facts is not None else 0, _stream())
     return out
 
 

@@ -1984,3 +1984,32 @@ def test_float_attention_of_prompt_portions_at_their_limits(d, what):
         q[40, 2 * d + 3] = float("nan")
         after, before = run(0, n).view(n, nq, d), None
         assert bool(after[40, 2].isnan().all()) and int(after.isnan().sum()) == d
+
+
+@pytest.mark.parametrize("form", ["decay", "channels", "steps"])
+@pytest.mark.parametrize("dk,dv", [(16, 16), (24, 40), (64, 64), (128, 17)])
+def test_recurrences_of_portions_with_helping_waves(form, dk, dv):
+    """Sequences that end at a chunk of 16 tokens, one behind it and far behind it, zeros and numbers past 40 among the inputs: the waves
+    that bring the chunks and write the outputs change no bit of them nor of the states (a caller that does not say how many
+    tokens come gets none), whatever the cutting."""
+    from types import SimpleNamespace
+    torch.manual_seed(dk + dv)
+    heads, lens = 3, [1, 16, 17, 32, 33, 100]
+    T, S = sum(lens), len(lens)
+    q, k, v = torch.randn(T, heads * dk, device=DEV), 0.1 * torch.randn(T, heads * dk, device=DEV), torch.randn(T, heads * dv, device=DEV)
+    q[5], k[7, ::2], v[20, 0], q[30, 1], q[31, 2] = 0.0, -0.0, 70.0, -70.0, 1e-30
+    kw = {"decay": dict(decay=torch.rand(heads, device=DEV), silu_inputs=True),
+          "channels": dict(wlog=torch.randn(T, heads * dk, device=DEV), bonus=torch.randn(heads, dk, device=DEV)),
+          "steps": dict(steps=torch.randn(T, heads, device=DEV), rate_log=torch.randn(heads, device=DEV), step_bias=torch.randn(heads, device=DEV),
+                        skip=torch.randn(heads, device=DEV))}[form]
+    starts = [0]
+    for n in lens:
+        starts.append(starts[-1] + n)
+    def run(longest):
+        state = torch.linspace(-1, 1, S * heads * dk * dv, device=DEV).view(S, -1).contiguous()
+        facts = None if longest is None else SimpleNamespace(max_query_len=longest, decode_only=True)     # (decode_only: no chunked form of steps)
+        ctx = SimpleNamespace(num_seqs=S, state_slots=torch.arange(S, dtype=torch.int32, device=DEV), facts=facts,
+                              q_start=torch.tensor(starts, dtype=torch.int32, device=DEV))
+        return K().linear_recurrence(q, k, v, ctx, state, heads, dk, dv, **kw), state
+    (out, state), (want, want_state) = run(max(lens)), run(None)
+    assert torch.equal(out.view(torch.int32), want.view(torch.int32)) and torch.equal(state.view(torch.int32), want_state.view(torch.int32))
