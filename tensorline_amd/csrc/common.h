@@ -61,11 +61,7 @@ __device__ __forceinline__ int tl_wave_scan(int v) {
 // lane 4 further holds what lane ^ 4 holds, and so on).  Six shuffles in a row take a wave 0.3 us, these 0.05.
 typedef unsigned int tl_u32x2 __attribute__((ext_vector_type(2)));
 template <typename Op>
-__device__ __forceinline__ float tl_wave_all(float v, Op op) {
-    tl_u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = op(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = op(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+__device__ __forceinline__ float tl_row_all(float v, Op op) {
 #define TL_ROTATED(N) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true))
     v = op(v, TL_ROTATED(8));
     v = op(v, TL_ROTATED(4));
@@ -74,8 +70,20 @@ __device__ __forceinline__ float tl_wave_all(float v, Op op) {
 #undef TL_ROTATED
     return v;
 }
+template <typename Op>
+__device__ __forceinline__ float tl_wave_all(float v, Op op) {
+    tl_u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    return tl_row_all(v, op);
+}
 __device__ __forceinline__ float tl_wave_sum(float v) {
     return tl_wave_all(v, [](float a, float b) { return a + b; });
+}
+
+__device__ __forceinline__ float tl_row_sum(float v) {       // of 16 lanes
+    return tl_row_all(v, [](float a, float b) { return a + b; });
 }
 
 __device__ __forceinline__ float tl_wave_max(float v) {

@@ -228,41 +228,52 @@ __device__ __forceinline__ int moe_rows_of_a_tile(int n, int BM) {
     const int tiles = (n + BM - 1) / BM;
     return ((n + tiles - 1) / tiles + 63) / 64 * 64;
 }
+// A thread keeps the experts of its first KEEP pairs and the places that counting them gave, all asked for at once, where both passes read the
+// pairs one trip to memory after another: 12,288 pairs of 64 experts 9.5 -> 8.2 us with 16 pairs, 96 pairs 2.4 -> 1.9 with one.
+template <int KEEP>
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restrict__ ids, int32_t* __restrict__ order,
                                                          int32_t* __restrict__ tiles, int P, int E, int BM) {
-    __shared__ int count[MOE_MAX_EXPERTS], first[MOE_MAX_EXPERTS], tile0[MOE_MAX_EXPERTS];
-    for (int e = threadIdx.x; e < E; e += blockDim.x) count[e] = 0;
-    __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) {
-        const int e = ids[p];
-        if (e >= 0 && e < E) atomicAdd(&count[e], 1);
+    __shared__ int count[MOE_MAX_EXPERTS], kept[MOE_MAX_EXPERTS], first[MOE_MAX_EXPERTS], tile0[MOE_MAX_EXPERTS];
+    const int tid = threadIdx.x, step = blockDim.x;
+    int expert[KEEP], place[KEEP];
+#pragma unroll
+    for (int j = 0; j < KEEP; ++j) {
+        expert[j] = -1;
+        if (j * step < P && tid + j * step < P) expert[j] = ids[tid + j * step];
     }
+    for (int e = tid; e < E; e += step) count[e] = 0;
     __syncthreads();
+#pragma unroll
+    for (int j = 0; j < KEEP; ++j)
+        if (j * step < P && expert[j] >= 0 && expert[j] < E) place[j] = atomicAdd(&count[expert[j]], 1);
+    __syncthreads();
+    if (P > KEEP * step) {                                    // the rest: counted now, placed behind the kept ones at the end
+        for (int e = tid; e < E; e += step) kept[e] = count[e];
+        __syncthreads();
+        for (int p = tid + KEEP * step; p < P; p += step) {
+            const int e = ids[p];
+            if (e >= 0 && e < E) atomicAdd(&count[e], 1);
+        }
+        __syncthreads();
+    }
     // places and tiles before each expert's: the first wave, 64 experts at a time
-    if (threadIdx.x < 64) {
+    if (tid < 64) {
         int at = 0, nt = 0;
         for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + (int)threadIdx.x, n = e < E ? count[e] : 0, per = moe_rows_of_a_tile(n, BM);
+            const int e = e0 + tid, n = e < E ? count[e] : 0, per = moe_rows_of_a_tile(n, BM);
             const int t = per ? (n + per - 1) / per : 0;
-            int n_to = n, t_to = t;                                    // sums up to and with this lane
-            for (int d = 1; d < 64; d <<= 1) {
-                const int pn = __shfl_up(n_to, d), pt = __shfl_up(t_to, d);
-                if ((int)threadIdx.x >= d) {
-                    n_to += pn;
-                    t_to += pt;
-                }
-            }
+            const int n_to = tl_wave_scan(n), t_to = tl_wave_scan(t);    // sums up to and with this lane
             if (e < E) {
                 first[e] = at + n_to - n;
                 tile0[e] = nt + t_to - t;
             }
-            at += __shfl(n_to, 63);
-            nt += __shfl(t_to, 63);
+            at += __builtin_amdgcn_readlane(n_to, 63);
+            nt += __builtin_amdgcn_readlane(t_to, 63);
         }
-        if (threadIdx.x == 0) tiles[0] = nt;
+        if (tid == 0) tiles[0] = nt;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
+    for (int e = tid; e < E; e += step) {
         const int n = count[e], per = moe_rows_of_a_tile(n, BM);
         for (int i = 0, tl = tile0[e]; i < n; i += per, ++tl) {
             tiles[1 + 3 * tl] = e;
@@ -270,18 +281,19 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restric
             tiles[3 + 3 * tl] = min(per, n - i);
         }
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < E; e += blockDim.x) count[e] = 0;      // now the cursor within the expert
-    __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) {
+#pragma unroll
+    for (int j = 0; j < KEEP; ++j)
+        if (j * step < P && expert[j] >= 0 && expert[j] < E) order[first[expert[j]] + place[j]] = tid + j * step;
+    for (int p = tid + KEEP * step; p < P; p += step) {
         const int e = ids[p];
-        if (e >= 0 && e < E) order[first[e] + atomicAdd(&count[e], 1)] = p;
+        if (e >= 0 && e < E) order[first[e] + atomicAdd(&kept[e], 1)] = p;
     }
 }
 
 extern "C" int tl_moe_sort(const int32_t* ids, int32_t* order, int32_t* tiles, int P, int E, int BM, hipStream_t stream) {
     TL_CHECK_ARG(P >= 0 && E > 0 && E <= MOE_MAX_EXPERTS && (BM == 16 || BM == 64 || BM == 256), "tl_moe_sort: bad sizes P=%d E=%d BM=%d", P, E, BM);
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(P >= 1024 ? 1024 : 256), 0, stream, ids, order, tiles, P, E, BM);
+    // (16 kept are no gain below four rounds: 1,200 pairs 3.5 against 3.0 us)
+    hipLaunchKernelGGL((P >= 4096 ? moe_sort_kernel<16> : moe_sort_kernel<1>), dim3(1), dim3(P >= 1024 ? 1024 : 256), 0, stream, ids, order, tiles, P, E, BM);
     TL_CHECK_LAUNCH("tl_moe_sort");
     return 0;
 }

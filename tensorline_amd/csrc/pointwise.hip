@@ -15,6 +15,24 @@ __device__ __forceinline__ float pw_gelu_tanh(float z) {
     return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
 
+// Four values in a row: 16 bytes of floats or 8 of bfloat16.  The element-wise kernels below come in that form and a number at a time, for rows that
+// are not whole aligned quads; the arithmetic of a value is the same.
+template <typename T> struct pw_quad;
+template <> struct pw_quad<float> {
+    static __device__ __forceinline__ float4 load(const float* p) { return *reinterpret_cast<const float4*>(p); }
+    static __device__ __forceinline__ void store(float* p, float a, float b, float c, float d) { *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d); }
+};
+template <> struct pw_quad<bf16_t> {
+    static __device__ __forceinline__ float4 load(const bf16_t* p) {
+        const uint2 v = *reinterpret_cast<const uint2*>(p);
+        return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
+    }
+    static __device__ __forceinline__ void store(bf16_t* p, float a, float b, float c, float d) {
+        *reinterpret_cast<uint2*>(p) = make_uint2(tl_pack_bf16(a, b), tl_pack_bf16(c, d));
+    }
+};
+static bool pw_quads(const void* p, int dtype) { return (uintptr_t)p % (dtype == TL_F32 ? 16 : 8) == 0; }
+
 // ---- residual add + Dynamic Tanh ---------------------------------------------------------------
 // Without `rows`: x[r] += residual[r] (float, written back); out[r] = tanh(alpha x[r]) * w + b.
 // With `rows`: the same for x[rows[r]] + residual[rows[r]], x untouched.  No statistic of the row
@@ -36,16 +54,39 @@ __global__ void add_dyt_kernel(float* __restrict__ x, const R* __restrict__ res,
     }
 }
 
+// 1,521 rows of 2,048, float residual, bfloat16 out: 9.0 -> 6.3 us (4 rows 5.1 -> 2.3).
+template <typename R, typename O>
+__global__ void add_dyt_quad_kernel(float* __restrict__ x, const R* __restrict__ res, const float* __restrict__ w, const float* __restrict__ b,
+                                    const float* __restrict__ alpha, O* __restrict__ out, const int32_t* __restrict__ rows, int H) {
+    const int r = blockIdx.x;
+    const size_t src = rows ? (size_t)rows[r] : (size_t)r;
+    const float a = alpha[0];
+    for (int c = 4 * threadIdx.x; c < H; c += 4 * blockDim.x) {
+        float4 v = *reinterpret_cast<const float4*>(x + src * H + c);
+        const float4 ww = *reinterpret_cast<const float4*>(w + c), bb = *reinterpret_cast<const float4*>(b + c);
+        if (res) {
+            const float4 y = pw_quad<R>::load(res + src * H + c);
+            v.x += y.x, v.y += y.y, v.z += y.z, v.w += y.w;
+            if (!rows) *reinterpret_cast<float4*>(x + src * H + c) = v;
+        }
+        pw_quad<O>::store(out + (size_t)r * H + c, tanhf(a * v.x) * ww.x + bb.x, tanhf(a * v.y) * ww.y + bb.y, tanhf(a * v.z) * ww.z + bb.z,
+                          tanhf(a * v.w) * ww.w + bb.w);
+    }
+}
+
 extern "C" int tl_add_dyt(float* x, const void* res, int res_dtype, const float* w, const float* b, const float* alpha,
                           void* out, int out_dtype, const int32_t* rows, int n, int H, hipStream_t stream) {
     TL_CHECK_ARG(n >= 0 && H > 0, "tl_add_dyt: bad sizes n=%d H=%d", n, H);
     if (n == 0) return 0;
-    dim3 grid(n), block(H >= 1024 ? 256 : 128);
-#define GO(R, O) hipLaunchKernelGGL((add_dyt_kernel<R, O>), grid, block, 0, stream, x, (const R*)res, w, b, alpha, (O*)out, rows, H)
-    if (res_dtype == TL_F32 && out_dtype == TL_F32) GO(float, float);
-    else if (res_dtype == TL_F32 && out_dtype == TL_BF16) GO(float, bf16_t);
-    else if (res_dtype == TL_BF16 && out_dtype == TL_F32) GO(bf16_t, float);
-    else if (res_dtype == TL_BF16 && out_dtype == TL_BF16) GO(bf16_t, bf16_t);
+    const bool quads = H % 4 == 0 && pw_quads(x, TL_F32) && pw_quads(res, res_dtype) && pw_quads(w, TL_F32) && pw_quads(b, TL_F32) && pw_quads(out, out_dtype);
+    const dim3 grid(n), block(quads ? (H >= 2048 ? 512 : H >= 1024 ? 256 : 128) : H >= 1024 ? 256 : 128);
+#define GO(R, O)                                                                                                                             \
+    if (quads) hipLaunchKernelGGL((add_dyt_quad_kernel<R, O>), grid, block, 0, stream, x, (const R*)res, w, b, alpha, (O*)out, rows, H);       \
+    else hipLaunchKernelGGL((add_dyt_kernel<R, O>), grid, block, 0, stream, x, (const R*)res, w, b, alpha, (O*)out, rows, H)
+    if (res_dtype == TL_F32 && out_dtype == TL_F32) { GO(float, float); }
+    else if (res_dtype == TL_F32 && out_dtype == TL_BF16) { GO(float, bf16_t); }
+    else if (res_dtype == TL_BF16 && out_dtype == TL_F32) { GO(bf16_t, float); }
+    else if (res_dtype == TL_BF16 && out_dtype == TL_BF16) { GO(bf16_t, bf16_t); }
     else return tl_fail("tl_add_dyt: unknown dtypes %d %d", res_dtype, out_dtype);
 #undef GO
     TL_CHECK_LAUNCH("tl_add_dyt");
@@ -65,11 +106,28 @@ __global__ void add_cast_kernel(float* __restrict__ x, const float* __restrict__
     out[i] = tl_from_float<O>(v);
 }
 
+// 1,521 rows of 2,048, bfloat16 out: 6.2 -> 5.1 us.
+template <typename O>
+__global__ __launch_bounds__(256) void add_cast_quad_kernel(float* __restrict__ x, const float* __restrict__ res, O* __restrict__ out, size_t n) {
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= n) return;
+    float4 v = *reinterpret_cast<const float4*>(x + i);
+    if (res) {
+        const float4 y = *reinterpret_cast<const float4*>(res + i);
+        v.x += y.x, v.y += y.y, v.z += y.z, v.w += y.w;
+        *reinterpret_cast<float4*>(x + i) = v;
+    }
+    pw_quad<O>::store(out + i, v.x, v.y, v.z, v.w);
+}
+
 extern "C" int tl_add_cast(float* x, const float* res, void* out, int out_dtype, long long n, hipStream_t stream) {
     TL_CHECK_ARG(n >= 0, "tl_add_cast: bad size");
     if (n == 0) return 0;
-    dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    if (out_dtype == TL_F32) hipLaunchKernelGGL(add_cast_kernel<float>, grid, block, 0, stream, x, res, (float*)out, (size_t)n);
+    const bool quads = n % 4 == 0 && pw_quads(x, TL_F32) && pw_quads(res, TL_F32) && pw_quads(out, out_dtype);
+    const dim3 grid((unsigned)(((quads ? n / 4 : n) + 255) / 256)), block(256);
+    if (quads && out_dtype == TL_F32) hipLaunchKernelGGL(add_cast_quad_kernel<float>, grid, block, 0, stream, x, res, (float*)out, (size_t)n);
+    else if (quads && out_dtype == TL_BF16) hipLaunchKernelGGL(add_cast_quad_kernel<bf16_t>, grid, block, 0, stream, x, res, (bf16_t*)out, (size_t)n);
+    else if (out_dtype == TL_F32) hipLaunchKernelGGL(add_cast_kernel<float>, grid, block, 0, stream, x, res, (float*)out, (size_t)n);
     else if (out_dtype == TL_BF16) hipLaunchKernelGGL(add_cast_kernel<bf16_t>, grid, block, 0, stream, x, res, (bf16_t*)out, (size_t)n);
     else return tl_fail("tl_add_cast: unknown dtype %d", out_dtype);
     TL_CHECK_LAUNCH("tl_add_cast");
@@ -121,15 +179,48 @@ __global__ void clamp_glu_kernel(const I* __restrict__ gu, O* __restrict__ out, 
     out[i] = tl_from_float<O>(pw_clamp_glu(tl_to_float(gu[t * 2 * F + c]), tl_to_float(gu[t * 2 * F + F + c]), limit, alpha));
 }
 
+// Four columns a thread, and the sigmoid of middling numbers in its short form (the same bits): 1,521 rows of 2,048, floats to
+// bfloat16 7.2 -> 4.2 us.
+template <typename I, typename O>
+__global__ __launch_bounds__(256) void clamp_glu_quad_kernel(const I* __restrict__ gu, O* __restrict__ out, int F, float limit, float alpha) {
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4;
+    const size_t t = blockIdx.x;
+    const bool here = c < F;
+    float4 g = make_float4(0.f, 0.f, 0.f, 0.f), u = g;
+    if (here) g = pw_quad<I>::load(gu + t * 2 * F + c), u = pw_quad<I>::load(gu + t * 2 * F + F + c);
+    float gv[4] = {g.x, g.y, g.z, g.w}, uv[4] = {u.x, u.y, u.z, u.w};
+    TlMagnitudes size;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        gv[i] = fminf(gv[i], limit);
+        uv[i] = fminf(fmaxf(uv[i], -limit), limit);
+        size.take(alpha * gv[i]);
+    }
+    float s[4];
+    if (size.mid_sigmoid()) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] = tl_sigmoid_mid(alpha * gv[i]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] = pw_sigmoid(alpha * gv[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = gv[i] * s[i] * (uv[i] + 1.0f);
+    if (here) pw_quad<O>::store(out + t * F + c, s[0], s[1], s[2], s[3]);
+}
+
 extern "C" int tl_clamp_glu(const void* gu, int in_dtype, void* out, int out_dtype, int T, int F, float limit, float alpha,
                             hipStream_t stream) {
     TL_CHECK_ARG(T >= 0 && F > 0, "tl_clamp_glu: bad sizes");
     if (T == 0) return 0;
-    dim3 grid((unsigned)(((size_t)T * F + 255) / 256)), block(256);
-#define GO(I, O) hipLaunchKernelGGL((clamp_glu_kernel<I, O>), grid, block, 0, stream, (const I*)gu, (O*)out, T, F, limit, alpha)
-    if (in_dtype == TL_F32 && out_dtype == TL_F32) GO(float, float);
-    else if (in_dtype == TL_F32 && out_dtype == TL_BF16) GO(float, bf16_t);
-    else if (in_dtype == TL_BF16 && out_dtype == TL_BF16) GO(bf16_t, bf16_t);
+    const bool quads = F % 4 == 0 && tl_ceil_div(F, 1024) <= 65535 && pw_quads(gu, in_dtype) && pw_quads(out, out_dtype);
+    const dim3 grid = quads ? dim3(T, tl_ceil_div(F, 1024)) : dim3((unsigned)(((size_t)T * F + 255) / 256)), block(256);
+#define GO(I, O)                                                                                                                  \
+    if (quads) hipLaunchKernelGGL((clamp_glu_quad_kernel<I, O>), grid, block, 0, stream, (const I*)gu, (O*)out, F, limit, alpha);   \
+    else hipLaunchKernelGGL((clamp_glu_kernel<I, O>), grid, block, 0, stream, (const I*)gu, (O*)out, T, F, limit, alpha)
+    if (in_dtype == TL_F32 && out_dtype == TL_F32) { GO(float, float); }
+    else if (in_dtype == TL_F32 && out_dtype == TL_BF16) { GO(float, bf16_t); }
+    else if (in_dtype == TL_BF16 && out_dtype == TL_BF16) { GO(bf16_t, bf16_t); }
     else return tl_fail("tl_clamp_glu: unsupported dtypes %d %d", in_dtype, out_dtype);
 #undef GO
     TL_CHECK_LAUNCH("tl_clamp_glu");
@@ -343,32 +434,54 @@ extern "C" int tl_gelu_token_gate(const float* z, const void* table, int dtype, 
 //     (the first `rank` columns are written by the product with the key expansion);
 //   * the row [c | rotated key part | zeros] of D columns goes into the cache at `slot`, once token-major
 //     ([pages, page, 1, D]) and once with a page's tokens innermost ([pages, 1, D, page]).
+// (A token's cosines and sines are worked out once, plain queries go by 16 bytes: 1,521 tokens of 16 heads 17.0 -> 13.6 us,
+// 16 tokens 7.4 -> 5.8.)
+#define LATENT_ANGLES 128
 template <typename T>
 __global__ void latent_prepare_kernel(const float* __restrict__ q, int ldq, const float* __restrict__ down, int ldd,
                                       const int32_t* __restrict__ pos,
                                       const float* __restrict__ freq, float mag, const float* __restrict__ norm_w, float eps,
                                       const int32_t* __restrict__ slots, T* __restrict__ q_plain, T* __restrict__ q_lat,
                                       T* __restrict__ k_cache, T* __restrict__ v_cache, int H, int d, int r, int rank, int D,
-                                      int page) {
+                                      int page, int quads) {
     __shared__ float red[16];
+    __shared__ float cs_of[LATENT_ANGLES], sn_of[LATENT_ANGLES];
     const int t = blockIdx.x;
     const float* row = q + (size_t)t * ldq;
     const float p = (float)pos[t];
     const int half = r / 2;
+    for (int i = threadIdx.x; i < min(half, LATENT_ANGLES); i += blockDim.x) {
+        const float a = p * freq[i];
+        cs_of[i] = cosf(a) * mag;
+        sn_of[i] = sinf(a) * mag;
+    }
+    __syncthreads();
+    auto angle = [&](int i) {
+        if (i < LATENT_ANGLES) return make_float2(cs_of[i], sn_of[i]);
+        const float a = p * freq[i];
+        return make_float2(cosf(a) * mag, sinf(a) * mag);
+    };
     // queries
-    for (int idx = threadIdx.x; idx < H * d; idx += blockDim.x) {
-        const int h = idx / d, c = idx - h * d;
-        q_plain[(size_t)t * H * d + idx] = tl_from_float<T>(row[h * (d + r) + c]);
+    if (quads) {
+        for (int idx = 4 * threadIdx.x; idx < H * d; idx += 4 * blockDim.x) {
+            const int h = idx / d, c = idx - h * d;
+            const float4 v = *reinterpret_cast<const float4*>(row + h * (d + r) + c);
+            pw_quad<T>::store(q_plain + (size_t)t * H * d + idx, v.x, v.y, v.z, v.w);
+        }
+    } else {
+        for (int idx = threadIdx.x; idx < H * d; idx += blockDim.x) {
+            const int h = idx / d, c = idx - h * d;
+            q_plain[(size_t)t * H * d + idx] = tl_from_float<T>(row[h * (d + r) + c]);
+        }
     }
     for (int idx = threadIdx.x; idx < H * (D - rank); idx += blockDim.x) {
         const int h = idx / (D - rank), c = idx - h * (D - rank);
         float v = 0.f;
         if (c < r) {
             const int i = c < half ? c : c - half;
-            const float a = p * freq[i];
-            const float cs = cosf(a) * mag, sn = sinf(a) * mag;
+            const float2 turn = angle(i);
             const float* qr = row + h * (d + r) + d;
-            v = c < half ? qr[i] * cs - qr[i + half] * sn : qr[i + half] * cs + qr[i] * sn;
+            v = c < half ? qr[i] * turn.x - qr[i + half] * turn.y : qr[i + half] * turn.x + qr[i] * turn.y;
         }
         q_lat[((size_t)t * H + h) * D + rank + c] = tl_from_float<T>(v);
     }
@@ -388,10 +501,9 @@ __global__ void latent_prepare_kernel(const float* __restrict__ q, int ldq, cons
         } else if (c < rank + r) {
             const int cc = c - rank;
             const int i = cc < half ? cc : cc - half;
-            const float a = p * freq[i];
-            const float cs = cosf(a) * mag, sn = sinf(a) * mag;
+            const float2 turn = angle(i);
             const float* kr = kv + rank;
-            v = cc < half ? kr[i] * cs - kr[i + half] * sn : kr[i + half] * cs + kr[i] * sn;
+            v = cc < half ? kr[i] * turn.x - kr[i + half] * turn.y : kr[i + half] * turn.x + kr[i] * turn.y;
         }
         const T o = tl_from_float<T>(v);
         k_cache[(size_t)slot * D + c] = o;
@@ -408,12 +520,13 @@ extern "C" int tl_latent_prepare(const float* q, int ldq, const float* down, int
     TL_CHECK_ARG(ldq >= H * (d + r) && ldd >= rank + r, "tl_latent_prepare: the projections' rows are too short");
     if (T == 0) return 0;
     dim3 grid(T), block(256);
+    const int quads = d % 4 == 0 && (d + r) % 4 == 0 && ldq % 4 == 0 && pw_quads(q, TL_F32) && pw_quads(q_plain, dtype);
     if (dtype == TL_F32)
         hipLaunchKernelGGL(latent_prepare_kernel<float>, grid, block, 0, stream, q, ldq, down, ldd, pos, freq, mag, norm_w, eps, slots,
-                           (float*)q_plain, (float*)q_lat, (float*)k_cache, (float*)v_cache, H, d, r, rank, D, page);
+                           (float*)q_plain, (float*)q_lat, (float*)k_cache, (float*)v_cache, H, d, r, rank, D, page, quads);
     else if (dtype == TL_BF16)
         hipLaunchKernelGGL(latent_prepare_kernel<bf16_t>, grid, block, 0, stream, q, ldq, down, ldd, pos, freq, mag, norm_w, eps, slots,
-                           (bf16_t*)q_plain, (bf16_t*)q_lat, (bf16_t*)k_cache, (bf16_t*)v_cache, H, d, r, rank, D, page);
+                           (bf16_t*)q_plain, (bf16_t*)q_lat, (bf16_t*)k_cache, (bf16_t*)v_cache, H, d, r, rank, D, page, quads);
     else return tl_fail("tl_latent_prepare: unknown dtype %d", dtype);
     TL_CHECK_LAUNCH("tl_latent_prepare");
     return 0;
@@ -431,11 +544,28 @@ __global__ void head_gate_kernel(T* __restrict__ o, const float* __restrict__ ga
     }
 }
 
+// Four numbers of a head at a time, its gate worked out once for them: 2,048 tokens of 32 heads of 128
+// 14.2 -> 7.3 us, 16 tokens 5.2 -> 1.9.
+template <typename T>
+__global__ __launch_bounds__(256) void head_gate_quad_kernel(T* __restrict__ o, const float* __restrict__ gate, int ldg, int H, int dv) {
+    const int t = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (c >= H * dv) return;
+    const float s = pw_sigmoid(gate[(size_t)t * ldg + c / dv]);
+    T* at = o + (size_t)t * H * dv + c;
+    const float4 v = pw_quad<T>::load(at);
+    pw_quad<T>::store(at, v.x * s, v.y * s, v.z * s, v.w * s);
+}
+
 extern "C" int tl_head_gate(void* o, int dtype, const float* gate, int ldg, int T, int H, int dv, hipStream_t stream) {
     TL_CHECK_ARG(T >= 0 && H > 0 && dv > 0 && ldg >= H, "tl_head_gate: bad sizes");
     if (T == 0) return 0;
-    dim3 grid(T), block(256);
-    if (dtype == TL_F32) hipLaunchKernelGGL(head_gate_kernel<float>, grid, block, 0, stream, (float*)o, gate, ldg, H, dv);
+    const dim3 grid(T), block(256);
+    if (dv % 4 == 0 && T <= 65535 && pw_quads(o, dtype) && (dtype == TL_F32 || dtype == TL_BF16)) {
+        const dim3 quads(tl_ceil_div(H * dv, 1024), T);
+        if (dtype == TL_F32) hipLaunchKernelGGL(head_gate_quad_kernel<float>, quads, block, 0, stream, (float*)o, gate, ldg, H, dv);
+        else hipLaunchKernelGGL(head_gate_quad_kernel<bf16_t>, quads, block, 0, stream, (bf16_t*)o, gate, ldg, H, dv);
+    }
+    else if (dtype == TL_F32) hipLaunchKernelGGL(head_gate_kernel<float>, grid, block, 0, stream, (float*)o, gate, ldg, H, dv);
     else if (dtype == TL_BF16) hipLaunchKernelGGL(head_gate_kernel<bf16_t>, grid, block, 0, stream, (bf16_t*)o, gate, ldg, H, dv);
     else return tl_fail("tl_head_gate: unknown dtype %d", dtype);
     TL_CHECK_LAUNCH("tl_head_gate");
@@ -763,90 +893,120 @@ extern "C" int tl_glu(const void* gu, int in_dtype, void* out, int out_dtype, in
 //     ([pages, page, G, D], zeros from d to D); v with a page's tokens innermost ([pages, G, D, page], zeros
 //     from dv to D).  With v_from_k the values are the keys as projected: before norm and rotation.  With `first` (float
 //     [T, >= G*dv], row stride ldf) the values are (1 - lam) v + lam first.
-// A work-group per token and a share of the heads (of queries, keys or values, in that order); a wave takes one head at a
-// time, a lane the pairs lane and lane + 64 of it (d <= 256).  A work-group computes the token's cosines and sines once, into
-// LDS.  Steps of many tokens leave the values to a kernel of their own (n_units then ends with the keys): written a token at
+// A work-group per token and a share of the heads (of queries, keys or values, in that order); LANES lanes take a head, a lane the
+// pairs LANES apart of it.  What bounds large steps is the instructions of a head, most of them the same for all its lanes (the sum, the
+// root and quotient of the norm, addresses): sixteen lanes to a head give them to four heads of a wave at once, 2,048 tokens of 32 query,
+// 8 key and 8 value heads of 128 35 -> 26 us with a norm, 27 -> 23 without, where a wave took one head at a time.  Small steps are bound by a wave's chain, and
+// 64 lanes to a head make it short: 16 tokens 3.4 against 4.1 us; 128 tokens 7.3 us either way.  The sum of squares adds pairs 64 apart, then 32, 16 .. 1
+// apart in both.  A work-group computes the token's cosines and sines once, into LDS.  Steps of many tokens leave the values to a kernel of their own (n_units then ends with the keys): written a token at
 // a time they are single numbers a page apart, written for sixteen neighbouring tokens at a time they are runs.
-template <typename T>
+template <typename T, int D_MAX, int LANES>
 __global__ __launch_bounds__(256) void head_norm_rotate_store_kernel(
     const float* __restrict__ proj, int ldp, const int32_t* __restrict__ pos, const float* __restrict__ wq,
     const float* __restrict__ wk, float eps, const float* __restrict__ freq, float mag, int rot,
     const int32_t* __restrict__ slots, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache, int H, int G,
-    int d, int dv, int D, int page, int v_from_k, int norm, int halves, int n_units, const float* __restrict__ first, int ldf, float lam) {
+    int d, int dv, int D, int page, int v_from_k, int norm, int halves, int n_units, const float* __restrict__ first, int ldf, float lam, int pairs) {
+    constexpr int NQ = D_MAX / 2 / LANES;                          // pairs of a lane
     __shared__ float cs[128], sn[128];
-    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t = blockIdx.x, m = threadIdx.x % LANES;
     const float* row = proj + (size_t)t * ldp;
-    const float p = (float)pos[t];
-    for (int i = threadIdx.x; i < rot / 2; i += blockDim.x) {
+    const float p = freq ? (float)pos[t] : 0.f;
+    for (int i = threadIdx.x; 2 * i < rot; i += 256) {
         const float a = p * freq[i];
         cs[i] = cosf(a) * mag;
         sn[i] = sinf(a) * mag;
     }
     __syncthreads();
     const int slot = slots ? slots[t] : -1;
-    const size_t pg = slot >= 0 ? (size_t)slot / page : 0, within = slot >= 0 ? (size_t)slot % page : 0;
-    for (int u = blockIdx.y * 4 + wave; u < n_units; u += 4 * gridDim.y) {
+    const unsigned pg = slot >= 0 ? (unsigned)slot / (unsigned)page : 0, within = slot >= 0 ? (unsigned)slot - pg * page : 0;
+    for (int u0 = blockIdx.y * (256 / LANES); u0 < n_units; u0 += 256 / LANES * gridDim.y) {
+        const int u = u0 + (threadIdx.x / LANES);
         const bool is_q = u < H, is_k = !is_q && u < H + G;
         const int head = is_q ? u : is_k ? u - H : u - H - G;
-        const int n = (is_q || is_k) ? d : dv;                   // the values the head has
+        const int n = u >= n_units ? 0 : (is_q || is_k) ? d : dv;                  // the values the head has
+        const bool keep = u < n_units && (is_q || slot >= 0);
         const float* x = row + (is_q ? head * d : is_k ? H * d + head * d : (H + G) * d + head * dv);
-        float raw[4], y[4];
-        // the dimensions of the lane's two pairs: neighbours, or with `halves` those rot / 2 apart among the turned ones
-        int ca[2], cb[2];
+        const float* y0 = first && !is_q && !is_k ? first + (size_t)t * ldf + head * dv : nullptr;
+        float raw[2 * NQ];
+        // the dimensions of a pair: neighbours, or with `halves` those rot / 2 apart among the turned ones
+        int ca[NQ], cb[NQ];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int i = lane + 64 * j;
+        for (int j = 0; j < NQ; ++j) {
+            const int i = m + LANES * j;
             const bool apart = halves && (is_q || is_k) && 2 * i < rot;
             ca[j] = apart ? i : 2 * i;
             cb[j] = apart ? i + (rot >> 1) : 2 * i + 1;
-            raw[2 * j] = ca[j] < n ? x[ca[j]] : 0.f;
-            raw[2 * j + 1] = cb[j] < n ? x[cb[j]] : 0.f;
+            if (pairs && !apart) {
+                const float2 v = ca[j] < n ? *reinterpret_cast<const float2*>(x + ca[j]) : make_float2(0.f, 0.f);
+                raw[2 * j] = v.x, raw[2 * j + 1] = v.y;
+            } else {
+                raw[2 * j] = ca[j] < n ? x[ca[j]] : 0.f;
+                raw[2 * j + 1] = cb[j] < n ? x[cb[j]] : 0.f;
+            }
         }
-        if (first && !is_q && !is_k) {
-            const float* y0 = first + (size_t)t * ldf + head * dv;
+        const float* w = norm == 1 ? (is_q ? wq : is_k ? wk : nullptr) : nullptr;
+        float by[2 * NQ];                                         // asked for with the values, ahead of the sum
+        if (norm == 1) {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int j = 0; j < NQ; ++j) {
+                by[2 * j] = w && ca[j] < n ? w[ca[j]] : 0.f;
+                by[2 * j + 1] = w && cb[j] < n ? w[cb[j]] : 0.f;
+            }
+        }
+        if (y0) {
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) {
                 raw[2 * j] = (1.0f - lam) * raw[2 * j] + (ca[j] < n ? lam * y0[ca[j]] : 0.f);
                 raw[2 * j + 1] = (1.0f - lam) * raw[2 * j + 1] + (cb[j] < n ? lam * y0[cb[j]] : 0.f);
             }
         }
-        if (!is_q && slot < 0) continue;                         // nothing to write for this token (the same for the wave)
-        const float* w = norm == 1 ? (is_q ? wq : is_k ? wk : nullptr) : nullptr;
         float rstd = 1.0f;
-        if (norm && (is_q || is_k)) {
-            const float ss = tl_wave_sum(raw[0] * raw[0] + raw[1] * raw[1] + raw[2] * raw[2] + raw[3] * raw[3]);
-            rstd = 1.0f / sqrtf(ss / (float)n + eps);
-        }
+        if (norm) {
+            constexpr int N = 64 / LANES;
+            float sq[N];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int i = lane + 64 * j;
-            float a = raw[2 * j] * rstd, b = raw[2 * j + 1] * rstd;
-            if (w) {
-                a = ca[j] < n ? a * w[ca[j]] : 0.f;
-                b = cb[j] < n ? b * w[cb[j]] : 0.f;
+            for (int j = 0; j < N; ++j) {
+                sq[j] = raw[2 * j] * raw[2 * j] + raw[2 * j + 1] * raw[2 * j + 1];
+                if constexpr (D_MAX == 256) sq[j] = sq[j] + raw[2 * (j + N)] * raw[2 * (j + N)] + raw[2 * (j + N) + 1] * raw[2 * (j + N) + 1];
             }
-            if ((is_q || is_k) && 2 * i + 1 < rot) {
-                const float ra = a * cs[i] - b * sn[i], rb = b * cs[i] + a * sn[i];
-                a = ra;
-                b = rb;
-            }
-            y[2 * j] = a;
-            y[2 * j + 1] = b;
+            float ss = sq[0];
+            if constexpr (LANES == 64) ss = tl_wave_sum(ss);
+            else ss = tl_row_sum((sq[0] + sq[2]) + (sq[1] + sq[3]));
+            if (is_q || is_k) rstd = 1.0f / sqrtf(ss / (float)n + eps);
         }
+        T* at = is_q ? q_out + ((size_t)t * H + head) * D : k_cache + ((size_t)slot * G + head) * D;
+        T* vat = v_cache + ((size_t)pg * G + head) * D * page + within;
+        if (keep) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int c = e ? cb[j] : ca[j];
-                if (c >= D) continue;
-                const T o = tl_from_float<T>(y[2 * j + e]);       // zeros beyond the head's values
-                if (is_q) {
-                    q_out[((size_t)t * H + head) * D + c] = o;
-                } else if (is_k) {
-                    k_cache[((size_t)slot * G + head) * D + c] = o;
-                    if (v_from_k) v_cache[((pg * G + head) * D + c) * page + within] = tl_from_float<T>(raw[2 * j + e]);
+            for (int j = 0; j < NQ; ++j) {
+                const int i = m + LANES * j;
+                float a = raw[2 * j] * rstd, b = raw[2 * j + 1] * rstd;
+                if (w) {
+                    a = ca[j] < n ? a * by[2 * j] : 0.f;
+                    b = cb[j] < n ? b * by[2 * j + 1] : 0.f;
+                }
+                if ((is_q || is_k) && 2 * i + 1 < rot) {
+                    const float ra = a * cs[i] - b * sn[i], rb = b * cs[i] + a * sn[i];
+                    a = ra;
+                    b = rb;
+                }
+                if (is_q || is_k) {                               // zeros beyond the head's values
+                    if (pairs && cb[j] == ca[j] + 1) {            // neighbours: one store (D is even)
+                        if (ca[j] < D) {
+                            if constexpr (sizeof(T) == 4) *reinterpret_cast<float2*>(at + ca[j]) = make_float2(a, b);
+                            else *reinterpret_cast<uint32_t*>(at + ca[j]) = tl_pack_bf16(a, b);
+                        }
+                    } else {
+                        if (ca[j] < D) at[ca[j]] = tl_from_float<T>(a);
+                        if (cb[j] < D) at[cb[j]] = tl_from_float<T>(b);
+                    }
+                    if (is_k && v_from_k) {
+                        if (ca[j] < D) vat[(size_t)ca[j] * page] = tl_from_float<T>(raw[2 * j]);
+                        if (cb[j] < D) vat[(size_t)cb[j] * page] = tl_from_float<T>(raw[2 * j + 1]);
+                    }
                 } else {
-                    v_cache[((pg * G + head) * D + c) * page + within] = o;
+                    if (ca[j] < D) vat[(size_t)ca[j] * page] = tl_from_float<T>(a);
+                    if (cb[j] < D) vat[(size_t)cb[j] * page] = tl_from_float<T>(b);
                 }
             }
         }
@@ -891,11 +1051,17 @@ extern "C" int tl_head_norm_rotate_store(const float* proj, int ldp, const int32
     if (T == 0) return 0;
     const bool values_apart = !v_from_k && G > 0 && G <= 65535 && T >= 64;
     const int units = H + G + (v_from_k || values_apart ? 0 : G);
-    dim3 grid(T, tl_ceil_div(units, T >= 512 ? 16 : 4)), block(256);
+    const bool few = T < 128;
+    dim3 grid(T, tl_ceil_div(units, few ? 4 : 16)), block(256);
     TL_CHECK_ARG(grid.y <= 65535, "tl_head_norm_rotate_store: too many heads");
+    const size_t two = 2 * (dtype == TL_F32 ? sizeof(float) : sizeof(bf16_t));
+    // neighbours go by one access
+    const int pairs = D % 2 == 0 && d % 2 == 0 && dv % 2 == 0 && ldp % 2 == 0 && (uintptr_t)proj % 8 == 0 && (uintptr_t)q_out % two == 0 &&
+                      (uintptr_t)k_cache % two == 0;
 #define GO(TT)                                                                                                         \
-    hipLaunchKernelGGL(head_norm_rotate_store_kernel<TT>, grid, block, 0, stream, proj, ldp, pos, wq, wk, eps, freq, mag, \
-                       rot, slots, (TT*)q_out, (TT*)k_cache, (TT*)v_cache, H, G, d, dv, D, page, v_from_k, norm, halves, units, first, ldf, lam)
+    hipLaunchKernelGGL((few ? D <= 128 ? head_norm_rotate_store_kernel<TT, 128, 64> : head_norm_rotate_store_kernel<TT, 256, 64>                \
+                            : D <= 128 ? head_norm_rotate_store_kernel<TT, 128, 16> : head_norm_rotate_store_kernel<TT, 256, 16>), grid, block, 0, stream, proj, ldp, pos, wq, wk, eps, freq, mag, \
+                       rot, slots, (TT*)q_out, (TT*)k_cache, (TT*)v_cache, H, G, d, dv, D, page, v_from_k, norm, halves, units, first, ldf, lam, pairs)
     if (dtype == TL_F32) GO(float);
     else if (dtype == TL_BF16) GO(bf16_t);
     else return tl_fail("tl_head_norm_rotate_store: unknown dtype %d", dtype);

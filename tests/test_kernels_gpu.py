@@ -2013,3 +2013,111 @@ def test_recurrences_of_portions_with_helping_waves(form, dk, dv):
         return K().linear_recurrence(q, k, v, ctx, state, heads, dk, dv, **kw), state
     (out, state), (want, want_state) = run(max(lens)), run(None)
     assert torch.equal(out.view(torch.int32), want.view(torch.int32)) and torch.equal(state.view(torch.int32), want_state.view(torch.int32))
+
+
+@pytest.mark.parametrize("what", ["dyt", "cast", "clamp", "gate", "latent"])
+@pytest.mark.parametrize("rows,width", [(1, 4), (3, 1020), (5, 2052)])
+def test_four_values_at_a_time_and_one(what, rows, width):
+    """Rows of aligned quads, and the same numbers where an access of four would be misaligned: the same bits, and within a rounding to
+    bfloat16 (2^-8 of the value) of the expression in 64 bits."""
+    k, bf = K(), torch.bfloat16
+    torch.manual_seed(rows)
+    def placed(t, off):                                      # contiguous, `off` numbers behind an aligned address
+        room = torch.empty(t.numel() + off, dtype=t.dtype, device=DEV)
+        room[off:] = t.flatten()
+        return room[off:].view(t.shape)
+    x, y, w, b = torch.randn(rows, width, device=DEV), torch.randn(rows, width, device=DEV), torch.randn(width, device=DEV), torch.randn(width, device=DEV)
+    gu = 4.0 * torch.randn(rows, 2 * width, device=DEV)
+    gu[0, 0], gu[0, 1], gu[0, 2], gu[0, 3] = float("inf"), -300.0, 0.0, float("nan")
+    gate = torch.randn(rows, 4, device=DEV)
+    proj, alpha = torch.randn(rows, 2 * 48 + 24 + 16, device=DEV), torch.tensor([0.6], device=DEV)
+    def run(off):
+        if what == "dyt":
+            a = placed(x, off)
+            return k.add_dyt(a, placed(y, off), w, b, alpha, bf), a
+        if what == "cast":
+            a = placed(x, off)
+            return k.add_cast(a, placed(y, off), bf), a
+        if what == "clamp":
+            return k.clamp_glu(placed(gu, off), 7.0, 1.702, bf), placed(gu.to(bf), off)
+        if what == "gate":
+            return k.head_gate(placed(x.to(bf), off), gate, 4), gate
+        kc, vc = torch.zeros(1, 16, 1, 48, dtype=bf, device=DEV), torch.zeros(1, 1, 48, 16, dtype=bf, device=DEV)
+        n = torch.arange(rows, dtype=torch.int32, device=DEV)
+        plain, lat = k.latent_prepare(placed(proj, off), 7 * n, torch.linspace(0.01, 1, 8, device=DEV), 1.25, w[:1].expand(24).contiguous(), 1e-5, n, kc, vc, 2, 32, 16, 24)
+        return plain, torch.cat([lat.view(rows, -1, 48)[:, :, 24:].flatten(), kc.flatten()])
+    got, one = run(0), run(1)
+    assert all(torch.equal(g.view(torch.int16) if g.dtype == bf else g.view(torch.int32), o.view(torch.int16) if o.dtype == bf else o.view(torch.int32))
+               for g, o in zip(got, one))
+    s = (x + y).double()
+    if what == "dyt":
+        want = torch.tanh(0.6 * s) * w.double() + b.double()
+    elif what == "cast":
+        want = s
+    elif what == "clamp":
+        g, u = gu[:, :width].double(), gu[:, width:].double()
+        g = torch.where(g.isnan(), 7.0, g.clamp(max=7.0))    # (the smaller of NaN and the limit is the limit)
+        want = g * torch.sigmoid(1.702 * g) * (u.clamp(-7.0, 7.0) + 1.0)
+    elif what == "gate":
+        want = (x.to(bf).double().view(rows, 4, -1) * torch.sigmoid(gate.double()).unsqueeze(2)).view(rows, width)
+    else:
+        want = proj[:, :96].reshape(rows, 2, 48)[:, :, :32].reshape(rows, 64).double()
+    torch.testing.assert_close(got[0].double(), want, rtol=2 ** -8, atol=2e-6)
+
+
+@pytest.mark.parametrize("halves", [False, True])
+@pytest.mark.parametrize("d,dv,D,turned", [(128, 128, 128, 64), (50, 40, 64, 20), (63, 63, 63, 30), (200, 256, 256, 200)])
+def test_heads_of_small_and_large_steps_alike(d, dv, D, turned, halves):
+    """A head has 64 lanes in steps of up to 127 tokens and 16 in larger ones, accesses of two numbers where sizes and addresses are even:
+    the same bits of queries, keys and values."""
+    H, G, T, page = 5, 2, 128, 16
+    torch.manual_seed(d)
+    cols = (H + G) * d + G * dv
+    proj, wide = torch.randn(T, cols + cols % 2, device=DEV), torch.empty(T, cols + 3 - cols % 2, device=DEV)
+    wide[:, 1:cols + 1] = proj[:, :cols]
+    n = torch.arange(T, dtype=torch.int32, device=DEV)
+    slots, freq = n.flip(0).contiguous(), torch.linspace(0.01, 1.0, turned // 2, device=DEV)
+    slots[3] = -1
+    w = torch.randn(2, d, device=DEV)
+    def run(x):
+        t = x.shape[0]
+        kc, vc = torch.zeros(T // page, page, G, D, dtype=torch.bfloat16, device=DEV), torch.zeros(T // page, G, D, page, dtype=torch.bfloat16, device=DEV)
+        q = K().head_norm_rotate_store(x, n[:t], w[0].contiguous(), w[1].contiguous(), 1e-5, freq, 1.1, kc, vc, slots[:t], H, G, d, dv, False, torch.bfloat16, halves=halves)
+        return q, kc.view(-1, G, D)[1:], vc.permute(0, 3, 1, 2).reshape(-1, G, D)[1:]      # (slot 0 is the last token's)
+    (q, kc, vc), (q1, kc1, vc1), (q2, kc2, vc2) = run(proj), run(wide[:, 1:cols + 1]), run(proj[:T - 1])
+    assert torch.equal(q, q1) and torch.equal(kc, kc1) and torch.equal(vc, vc1)
+    assert torch.equal(q[:T - 1], q2) and torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    x = proj[:, :H * d].double().view(T, H, d)
+    x = x / torch.sqrt(x.square().mean(2, keepdim=True) + 1e-5) * w[0].double()
+    angle = (n.unsqueeze(1).float() * freq).double()
+    cs, sn = 1.1 * angle.cos().unsqueeze(1), 1.1 * angle.sin().unsqueeze(1)
+    a, b = (x[:, :, :turned // 2], x[:, :, turned // 2:turned]) if halves else (x[:, :, :turned:2], x[:, :, 1:turned:2])
+    ra, rb = a * cs - b * sn, b * cs + a * sn
+    rot = torch.cat([ra, rb], 2) if halves else torch.stack([ra, rb], 3).flatten(2)
+    want = torch.nn.functional.pad(torch.cat([rot, x[:, :, turned:]], 2), (0, D - d))
+    torch.testing.assert_close(q.view(T, H, D).double(), want, rtol=2 ** -8, atol=2e-5)
+
+
+@pytest.mark.parametrize("pairs,experts,tile", [(1, 1, 16), (257, 8, 16), (1023, 64, 64), (1024, 3, 64), (4095, 64, 64), (4096, 64, 256), (16385, 256, 256), (40000, 64, 256)])
+def test_pairs_sorted_by_expert(pairs, experts, tile):
+    """Numbers of pairs on both sides of what the sort's threads keep: every pair once, among its expert's, the tiles cover them in order;
+    experts out of range are left out."""
+    k = K()
+    ids = torch.randint(0, experts, (pairs,), generator=torch.Generator().manual_seed(pairs)).to(torch.int32)
+    if pairs > 300:
+        ids[::97], ids[5] = -1, experts
+    order, tiles = torch.full((pairs,), -1, dtype=torch.int32, device=DEV), torch.zeros(1 + 3 * (pairs // tile + experts), dtype=torch.int32, device=DEV)
+    dev = ids.to(DEV)
+    k._call("tl_moe_sort", k._ptr(dev), k._ptr(order), k._ptr(tiles), pairs, experts, tile, k._stream())
+    order, tiles = order.cpu().long(), tiles.cpu()
+    at = covered = 0
+    for e in range(experts):
+        mine = (ids == e).nonzero().flatten()
+        assert torch.equal(order[at:at + mine.numel()].sort().values, mine)
+        rows = [r for r in tiles[1:1 + 3 * int(tiles[0])].view(-1, 3).tolist() if r[0] == e]
+        assert sum(r[2] for r in rows) == mine.numel() and all(0 < r[2] <= tile for r in rows)
+        for _, first, n in rows:
+            assert first == at
+            at += n
+        covered += len(rows)
+    assert covered == int(tiles[0]) and bool((order[at:] == -1).all())
