@@ -606,13 +606,15 @@ __global__ __launch_bounds__(MG_THREADS, 2) void moe_gemm_bf16_kernel(const bf16
 // tile of 192 x 256 gets 110 out of it: by the counters (requests of 128 bytes from L2, gate and up of 192 rows an expert) the
 // smaller tiles fetch 10.7 GB in 1.01 to 1.17 ms, these 3.8 GB in 0.43, of which 2.1 are the matrices from memory at 5.0 TB/s.
 //
-// Eight waves, two by four: a wave has half of the tile's rows (32 MW of 64 MW) and 64 of its columns; tile_walk.h has the walk
+// Eight waves, two by four: a wave has half of the tile's rows (16 MB of 32 MB) and 64 of its columns; tile_walk.h has the walk
 // over k, in steps of 64: whole lines of 128 bytes per row (steps of 32 fetched every line twice).  The matrix rows have three
 // stages of LDS, the rows two or three.  The eight units of 16 bytes of a row lie at unit ^ (row / 2) % 8, so that the sixteen
 // lanes that are served at a time (rows r .. r + 15, one unit) hit all banks.  Four waves with whole steps of fragments ahead of
 // their products took 543 and 304 us for gate and up and for down of 192 rows an expert (64 of 4,096 x 2,048) where this takes 427
 // and 270 (5.0 and 4.0 TB/s of matrices).
-// MW is the tile's rows in sixties-fours, chosen by the work-group, so that a tile of 70 rows does the products of 128.
+// MB is the tile's rows in thirties-twos, chosen by the work-group, so that a tile of 195 rows does the products of 224 (160 to 219 rows an expert,
+// 64 of 4,096 x 2,048, gate and up 491 -> 480 us and down 268 -> 263 against rows in sixties-fours; without any products the loads alone
+// take 381 and 243, at 5.6 and 4.4 TB/s of matrices).  Loads and stages go by 64 rows, the last row again where there is none.
 // The tiles of one expert, all its column tiles, go to one XCD (every eighth work-group id), whose L2 then holds the rows.  Of the last tiles, that are
 // fewer than there are XCDs, every XCD takes its share of the column tiles where the XCDs that had a whole one would have a round of work-groups
 // more (64 experts of 2,048 x 1,408, 67 tiles in 11 columns, 188 -> 169 us); elsewhere they would only fetch the rows once each (8 experts of 1,024 x
@@ -643,12 +645,12 @@ __device__ __forceinline__ bool moe_wide_tile(int id, int have, int ntiles, int*
     return *mt < have;
 }
 
-template <int MW, int MODE>
+template <int MB, int MODE>
 __device__ __forceinline__ void mgw_tile(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ We, void* __restrict__ Cv, int ldc,
                                          const int32_t* __restrict__ order, int place0, int rows, int expert, int n0, int top, uint32_t per_top, int N, int K,
                                          float limit, float alpha, float shift, uint4* lds) {
     constexpr bool GLU = MODE == 1, BY_TOKEN = MODE != 0;
-    constexpr int MB = 2 * MW, NB = 4, LA = MW, LB = 4;                          // blocks of a wave; loads per wave and step, 8 rows each
+    constexpr int MW = (MB + 1) / 2, NB = 4, LA = MW, LB = 4;                          // blocks of a wave; loads per wave and step, 8 rows each
     constexpr int A_STAGES = MW <= 2 ? 3 : 2, STAGE_A = MW * 512;
     static_assert((MGW_W_STAGES * MGW_W + A_STAGES * STAGE_A) * 16 <= MGW_LDS, "the stages do not fit");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -751,11 +753,14 @@ __global__ __launch_bounds__(MGW_THREADS, 2) void moe_gemm_wide_kernel(const bf1
     const int e = tiles[1 + 3 * mt], place0 = tiles[2 + 3 * mt], rows = tiles[3 + 3 * mt];
     const bf16_t* We = W + (size_t)e * (MODE == 1 ? 2 : 1) * N * K;
     const int n0 = nt * (MODE == 1 ? 128 : 256);
-#define GO(MW) mgw_tile<MW, MODE>(A, lda, We, C, ldc, order, place0, rows, e, n0, top, per_top, N, K, limit, alpha, shift, mgw_lds)
-    if (rows <= 64) GO(1);
-    else if (rows <= 128) GO(2);
-    else if (rows <= 192) GO(3);
-    else GO(4);
+#define GO(MB) mgw_tile<MB, MODE>(A, lda, We, C, ldc, order, place0, rows, e, n0, top, per_top, N, K, limit, alpha, shift, mgw_lds)
+    if (rows <= 64) GO(2);
+    else if (rows <= 96) GO(3);
+    else if (rows <= 128) GO(4);
+    else if (rows <= 160) GO(5);
+    else if (rows <= 192) GO(6);
+    else if (rows <= 224) GO(7);
+    else GO(8);
 #undef GO
 }
 

@@ -1,4 +1,5 @@
 """Each HIP kernel alone against its plain reference, at sizes other than the engine's."""
+import ctypes
 import math
 
 import pytest
@@ -2121,3 +2122,28 @@ def test_pairs_sorted_by_expert(pairs, experts, tile):
             at += n
         covered += len(rows)
     assert covered == int(tiles[0]) and bool((order[at:] == -1).all())
+
+
+@pytest.mark.parametrize("glu", [0, 1, 2])
+def test_wide_expert_tiles_of_every_height(glu):
+    """Experts whose rows end at each height a wide tile is multiplied in and one beyond it: the bits of the tiles of 64 rows, which take the
+    same sums in the same order."""
+    k, (N, W) = K(), (260, 192)
+    rows = [1, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256, 257]
+    E, P = len(rows), sum(rows)
+    torch.manual_seed(glu)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).to(torch.int32).to(DEV)
+    a = torch.randn(P, W, device=DEV).to(torch.bfloat16)
+    w = (0.1 * torch.randn(E, (2 if glu == 1 else 1) * N, W, device=DEV)).to(torch.bfloat16)
+    f = ctypes.c_float
+    def run(tile):
+        most = P // tile + E
+        order, tiles = torch.empty(P, dtype=torch.int32, device=DEV), torch.empty(1 + 3 * most, dtype=torch.int32, device=DEV)
+        k._call("tl_moe_sort", k._ptr(ids), k._ptr(order), k._ptr(tiles), P, E, tile, k._stream())
+        order.copy_(torch.arange(P))                         # (the sort leaves open where in its expert's places a pair goes)
+        out = torch.zeros(P, N, dtype=torch.bfloat16 if glu else torch.float32, device=DEV)
+        k._call("tl_moe_gemm", k._ptr(a), k.BF16, W, k._ptr(w), k.BF16, k._ptr(out), k.BF16 if glu else k.F32, N, k._ptr(order), k._ptr(tiles),
+                most, E, tile, 1, N, W, glu, f(7.0), f(1.702), f(1.0), k._stream())
+        return out
+    got, want = run(256), run(64)
+    assert torch.equal(got.float(), want.float()) and bool(got.isfinite().all()) and bool((got != 0).any(1).all())
