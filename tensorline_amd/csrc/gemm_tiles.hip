@@ -32,6 +32,7 @@
 #include <math.h>
 
 #define GT_KT 64
+#define GT_CUS 256
 
 struct GtOut {
     void* C;                   // [M, ldc], or shares x [M, N] float
@@ -195,23 +196,31 @@ __global__ __launch_bounds__(256) void gt_add_kernel(const float* __restrict__ p
 // 1 to 12 shares, with weights from memory (those that the last-level cache holds give other times and other choices): half of the
 // 3,600 times are within 5%, and the choice by them takes 0.8% longer than the best one in the mean (0.75 of the library's time; at
 // worst, 192 rows of 4,096 x 12,288, 38 us where the best takes 34 and the library 32).
-//    id  waves  blocks stages (0: registers) a CU holds  step alone, beside a second; start and end
-#define GT_TILES(X)                                  \
-    X(0, 2, 4, 8, 4, 2, 3, 1, 1.072, 1.072, 4.22)    \
-    X(1, 2, 4, 8, 3, 2, 3, 1, 0.854, 0.854, 3.94)    \
-    X(2, 2, 4, 4, 4, 3, 3, 1, 0.735, 0.735, 3.29)    \
-    X(3, 2, 4, 4, 2, 2, 3, 2, 0.584, 0.785, 1.46)    \
-    X(4, 2, 4, 2, 2, 3, 3, 2, 0.407, 0.649, 0.95)    \
-    X(5, 4, 2, 1, 2, 5, 5, 2, 0.224, 0.406, 0.99)    \
-    X(6, 2, 4, 6, 4, 2, 3, 1, 0.931, 0.931, 3.72)    \
-    X(7, 1, 4, 8, 4, 4, 0, 2, 0.670, 1.153, 3.72)
+//    id  waves  blocks stages (0: registers); where each has a CU of its own, from so many steps on; a CU holds  step alone, beside a second; start and end
+// A grid that leaves every work-group a CU of its own has room for more stages: what bounds a 128 x 128 or 64 x 128 tile there is how much is
+// on its way (32 or 24 KB a step, 40 to 50 KB ahead: 55 to 60 bytes a ns and CU), and 64 or 72 KB ahead bring a step in 0.42 us
+// where it took 0.58.  The same products in the same order.  us before and after, weights from memory, 801 rows of 3,072 x 2,048 24.3 and
+// 19.0; 1,521 of 2,048 x 2,048 24.6 and 21.5; 200 of 12,288 x 2,048 gate/up 25.4 and 21.9; 200 of 4,608 x
+// 3,584 22.9 and 20.6; 801 of 2,048 x 2,048 (64 x 128) 17.1 and 16.3.  45 such products in tile 3: 1.13 times as fast in the mean, 1.02 to
+// 1.29.  Tile 4 gains 1.02 to 1.11 from some 20 steps on and loses up to 4% below, where filling the stages is a part of the walk; tile 5's
+// five stages are enough (nine: 0.97).
+#define GT_TILES(X)                                         \
+    X(0, 2, 4, 8, 4, 2, 3, 0, 0, 1, 1.072, 1.072, 4.22)     \
+    X(1, 2, 4, 8, 3, 2, 3, 0, 0, 1, 0.854, 0.854, 3.94)     \
+    X(2, 2, 4, 4, 4, 3, 3, 0, 0, 1, 0.735, 0.735, 3.29)     \
+    X(3, 2, 4, 4, 2, 2, 3, 4, 1, 2, 0.584, 0.785, 1.46)     \
+    X(4, 2, 4, 2, 2, 3, 3, 5, 20, 2, 0.407, 0.649, 0.95)    \
+    X(5, 4, 2, 1, 2, 5, 5, 0, 0, 2, 0.224, 0.406, 0.99)     \
+    X(6, 2, 4, 6, 4, 2, 3, 0, 0, 1, 0.931, 0.931, 3.72)     \
+    X(7, 1, 4, 8, 4, 4, 0, 0, 0, 2, 0.670, 1.153, 3.72)
 struct GtTile {
     int bm, bn, lds, per_cu;
+    int alone_lds, alone_from;           // of the form for work-groups with a CU of their own (0: none)
     bool pairs, direct;        // the gated form: whole blocks of gate and of up columns in a wave; W straight into registers
     double step1, step2, ends;
 };
-#define X(ID, WM, WN, MB, NB, AST, BST, CU, T1, T2, ENDS) \
-    {16 * WM * MB, 16 * WN * NB, (16 * WM * MB * AST + 16 * WN * NB * BST) * 128, CU, NB % 2 == 0, BST == 0, T1, T2, ENDS},
+#define X(ID, WM, WN, MB, NB, AST, BST, DEEP, FROM, CU, T1, T2, ENDS) \
+    {16 * WM * MB, 16 * WN * NB, (16 * WM * MB * AST + 16 * WN * NB * BST) * 128, CU, (16 * WM * MB + 16 * WN * NB) * DEEP * 128, FROM, NB % 2 == 0, BST == 0, T1, T2, ENDS},
 static const GtTile gt_tiles[] = {GT_TILES(X)};
 #undef X
 #define GT_TILE_COUNT 8
@@ -302,20 +311,29 @@ extern "C" int tl_gemm_tiles(const void* A, const void* W, const float* bias, vo
     const dim3 grid((unsigned)tl_ceil_div(mtiles * ntiles * shares, 8) * 8);
     const GtOut direct = {C, ldc, bias, act}, partial = {ws, N, nullptr, 0};
     const GtOut& o = shares > 1 ? partial : direct;
-#define GO(WM, WN, MB, NB, AST, BST, GLU, TO)                                                                                             \
-    hipLaunchKernelGGL((gemm_tiles_kernel<WM, WN, MB, NB, AST, BST, GLU, TO>), grid, dim3(64 * WM * WN), (size_t)t.lds, stream, (const bf16_t*)A, lda, \
+    const bool alone = t.alone_lds && K / GT_KT / shares >= t.alone_from && (long long)mtiles * ntiles * shares <= GT_CUS;
+#define GO_OF(WM, WN, MB, NB, AST, BST, LDS, GLU, TO)                                                                                              \
+    hipLaunchKernelGGL((gemm_tiles_kernel<WM, WN, MB, NB, AST, BST, GLU, TO>), grid, dim3(64 * WM * WN), (size_t)LDS, stream, (const bf16_t*)A, lda, \
                        (const bf16_t*)W, o, M, N, K, mtiles, ntiles, shares)
-#define X(ID, WM, WN, MB, NB, AST, BST, CU, T1, T2, ENDS)                      \
+#define GO(WM, WN, MB, NB, AST, BST, DEEP, GLU, TO)                                                            \
+    do {                                                                                                       \
+        if constexpr (DEEP != 0) {                                                                             \
+            if (alone) { GO_OF(WM, WN, MB, NB, DEEP, DEEP, t.alone_lds, GLU, TO); break; }                     \
+        }                                                                                                      \
+        GO_OF(WM, WN, MB, NB, AST, BST, t.lds, GLU, TO);                                                       \
+    } while (0)
+#define X(ID, WM, WN, MB, NB, AST, BST, DEEP, FROM, CU, T1, T2, ENDS)          \
     case ID:                                                                   \
-        if (gated) GO(WM, WN, MB, (NB % 2 ? NB + 1 : NB), AST, BST, true, bf16_t); \
+        if (gated) GO(WM, WN, MB, (NB % 2 ? NB + 1 : NB), AST, BST, DEEP, true, bf16_t); \
         else if constexpr (BST != 0) {                                         \
-            if (shares > 1 || c_dtype == TL_F32) GO(WM, WN, MB, NB, AST, BST, false, float); \
-            else GO(WM, WN, MB, NB, AST, BST, false, bf16_t);                  \
+            if (shares > 1 || c_dtype == TL_F32) GO(WM, WN, MB, NB, AST, BST, DEEP, false, float); \
+            else GO(WM, WN, MB, NB, AST, BST, DEEP, false, bf16_t);            \
         }                                                                      \
         break;
     switch (tile) { GT_TILES(X) }
 #undef X
 #undef GO
+#undef GO_OF
     TL_CHECK_LAUNCH("tl_gemm_tiles");
     if (shares > 1 && C) {
         const dim3 blocks((unsigned)(((size_t)M * N / 4 + 255) / 256));

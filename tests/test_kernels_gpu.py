@@ -183,6 +183,25 @@ def test_many_row_product_beyond_one_panel(tile, Kd):
         assert bool(((got.double() - fn(gate) * up).abs() <= _gate_error(gate, up, err[:, :I], err[:, I:], fn)).all())
 
 
+@pytest.mark.parametrize("tile,M,Kd,shares", [(3, 1, 64, 1), (3, 129, 192, 1), (3, 300, 256, 1), (3, 257, 320, 1), (3, 129, 832, 2), (3, 2048, 576, 1),
+                                              (4, 65, 1216, 1), (4, 65, 1280, 1), (4, 130, 1344, 1), (4, 63, 2624, 2), (4, 512, 1600, 1)])
+def test_tiles_with_a_cu_of_their_own(tile, M, Kd, shares):
+    """A grid of at most one work-group to a CU (tile 4: of 20 steps or more) has more stages, from fewer steps than stages on: bit for bit
+    the rows of a call of more tiles than CUs, which has the other form (every sum is of the same order)."""
+    bm, N = TILE_SIZES[tile][0], 2048
+    many = 2048 // shares // 2 if tile == 4 else 2048 // shares       # rows that fill the CUs
+    assert M <= many
+    torch.manual_seed(Kd)
+    a = torch.randn(many + bm, Kd, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, Kd, device=DEV) / math.sqrt(Kd)).to(torch.bfloat16)
+    sh = K().shuffle_weight(w)
+    run = lambda rows, dt, **kw: K()._tiles(a[:rows], sh, None, dt, rows, N, Kd, Kd, shares * 256 + tile, **kw)
+    for dt in (torch.float32, torch.bfloat16):
+        torch.testing.assert_close(run(M, dt), run(many + bm, dt)[:M], atol=0, rtol=0)
+    if shares == 1:
+        torch.testing.assert_close(run(M, torch.bfloat16, gated=True), run(many + bm, torch.bfloat16, gated=True)[:M], atol=0, rtol=0)
+
+
 @pytest.mark.parametrize("M,I,Kd", [(1, 16, 64), (65, 144, 128), (127, 128, 192), (128, 272, 256), (129, 112, 320), (257, 400, 832), (2200, 48, 448)])
 def test_gated_product_with_the_matrix_in_registers(M, I, Kd):
     """Tiles whose matrix goes straight into registers, from one step of K to fewer and more than are under way, at the edges of rows
