@@ -103,10 +103,17 @@ class Linear:
         """The matrix-core ordered copy few-row products stream, of whichever type the weight has."""
         return self.shuffled if self.shuffled is not None else self.shuffled_float
 
+    @property
+    def copies(self) -> dict[str, torch.Tensor]:
+        """What a product may read in the matrix's place, by the names that :func:`kernels.linear` gives it."""
+        if self.ranges is None:
+            return {"shuffled": self.streamed}
+        return {"shuffled": self.shuffled_float, "ranges": self.ranges}
+
     def __call__(self, x, out_dtype: torch.dtype | None = None, sink=None, with_bias: bool = True,
                  keep_shares: bool = False, act: str | None = None):
         return kernels.linear(x, self.weight, self.bias if with_bias else None, out_dtype=out_dtype,
-                              shuffled=self.streamed, sink=sink, keep_shares=keep_shares, act=act, ranges=self.ranges)
+                              sink=sink, keep_shares=keep_shares, act=act, **self.copies)
 
 
 def fuse_linears(name: str, parts: list[Linear]) -> Linear:
