@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import time
 from concurrent.futures import ThreadPoolExecutor
@@ -45,6 +46,7 @@ def _headers() -> list[str]:
 def source_hash() -> str:
     h = hashlib.sha256()
     h.update(" ".join(HIPCC_FLAGS).encode())
+    h.update((sysconfig.get_config_var("SOABI") or "").encode())      # host_call.hip is Python's as well
     for path in sources() + _headers():
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as f:
@@ -120,7 +122,7 @@ def build(verbose: bool = True, jobs: int | None = None) -> str:
 
     def compile_one(src: str) -> str:
         obj = os.path.join(obj_dir, os.path.basename(src)[:-4] + ".o")
-        cmd = [hipcc, *HIPCC_FLAGS, "-I", CSRC, "-c", src, "-o", obj]
+        cmd = [hipcc, *HIPCC_FLAGS, "-I", CSRC, "-I", sysconfig.get_paths()["include"], "-c", src, "-o", obj]
         proc = subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, env=env, text=True)
         last = time.time()
         while True:

@@ -8,7 +8,10 @@ from __future__ import annotations
 
 import atexit
 import ctypes
+import functools
 import glob
+import importlib.machinery
+import importlib.util
 import os
 import tempfile
 import threading
@@ -65,23 +68,34 @@ def require_gpu(device) -> torch.device:
     return dev
 
 
-_entry_points: dict[str, object] = {}
+_entry_points: dict[str, int] = {}      # addresses, by name
+_enter = None
+
+
+def _entry_point(name: str) -> int:
+    """The address of a C entry point, for ``_enter``: ``enter(address, *arguments)`` of the library as a Python module (host_call.hip)."""
+    global _enter
+    lib = library()
+    if _enter is None:
+        loader = importlib.machinery.ExtensionFileLoader("libtensorline_hip", lib._name)
+        _enter = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader)).enter
+    address = _entry_points[name] = ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+    return address
 
 
 def _call(name: str, *args) -> None:
-    fn = _entry_points.get(name)
-    if fn is None:
-        fn = _entry_points[name] = getattr(library(), name)
-    if fn(*args) != 0:
+    """An entry point with tensors (their addresses), None, integers, floats (32 bits) and ctypes objects as its arguments."""
+    address = _entry_points.get(name) or _entry_point(name)
+    if _enter(address, *args) != 0:
         raise KernelError(library().tl_last_error().decode("utf-8", "replace"))
 
 
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+def _stream() -> int:
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
-def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: torch.Tensor | None) -> int:
+    return 0 if t is None else t.data_ptr()
 
 
 def _code(t: torch.Tensor, what: str) -> int:
@@ -129,7 +143,7 @@ def embed(ids: torch.Tensor, table: torch.Tensor, out: torch.Tensor | None = Non
     if out is None:
         out = torch.empty(T, H, dtype=torch.float32, device=table.device)
     _check(out.dtype == torch.float32 and out.is_contiguous() and tuple(out.shape) == (T, H), "embed: bad output")
-    _call("tl_embed", _ptr(ids), _ptr(table), _code(table, "embed"), _ptr(out), T, H, V, ctypes.c_float(scale), _stream())
+    _call("tl_embed", ids, table, _code(table, "embed"), out, T, H, V, float(scale), _stream())
     return out
 
 
@@ -149,10 +163,10 @@ def embed_bigram(ids: torch.Tensor, ctx, table: torch.Tensor, bigram: torch.Tens
     _i32(ctx.pos, "pos", T)
     _i32(ctx.seq_of_token, "seq_of_token", T)
     out = torch.empty(T, H, dtype=torch.float32, device=table.device)
-    _call("tl_embed_bigram", _ptr(ids), _ptr(ctx.pos), _ptr(ctx.seq_of_token), _ptr(ctx.q_start), _ptr(ctx.state_slots),
-          _ptr(kept), ctypes.c_longlong(kept.stride(0)), _ptr(table), _ptr(bigram), _code(table, "embed_bigram"), _ptr(out), T,
-          ctx.num_seqs, H, V, ctypes.c_longlong(bigram.shape[0] - 1), ctypes.c_longlong(int(mul_prev)),
-          ctypes.c_longlong(int(mul_cur)), _stream())
+    _call("tl_embed_bigram", ids, ctx.pos, ctx.seq_of_token, ctx.q_start, ctx.state_slots,
+          kept, kept.stride(0), table, bigram, _code(table, "embed_bigram"), out, T,
+          ctx.num_seqs, H, V, bigram.shape[0] - 1, int(mul_prev),
+          int(mul_cur), _stream())
     return out
 
 
@@ -186,8 +200,8 @@ def _branch_norm_add(x, branch: NormedBranch, weight, eps, out_dtype, rows):
             _i32(rows, "rows")
             n = rows.numel()
         out = torch.empty(n, H, dtype=out_dtype, device=x.device)
-    _call("tl_branch_norm_add", _ptr(x), _ptr(y), _ptr(wb), ctypes.c_float(branch.mult), ctypes.c_float(branch.eps), _ptr(weight),
-          ctypes.c_float(eps), _ptr(out), _code(out, "normed branch out") if out is not None else F32, _ptr(rows), n, H, _stream())
+    _call("tl_branch_norm_add", x, y, wb, float(branch.mult), float(branch.eps), weight,
+          float(eps), out, _code(out, "normed branch out") if out is not None else F32, rows, n, H, _stream())
     return out
 
 
@@ -228,7 +242,7 @@ class JoinedBranches:
 def _branch_args(y, scale, T: int, H: int):
     """(tensors to check, ctypes arguments) of one branch of :func:`join_norms`."""
     if y is None:
-        return [], (_ptr(None), 1, ctypes.c_longlong(0), ctypes.c_longlong(0), _ptr(None), _ptr(None))
+        return [], (None, 1, 0, 0, None, None)
     weights, pieces, piece, token = None, 1, 0, H
     if isinstance(y, ShareSum):
         t, pieces, piece = y.parts, y.parts.shape[0], T * H
@@ -244,7 +258,7 @@ def _branch_args(y, scale, T: int, H: int):
     _f32(t, "join_norms branch")
     if scale is not None:
         _f32(scale, "join_norms scale", H)
-    return [t, weights, scale], (_ptr(t), pieces, ctypes.c_longlong(piece), ctypes.c_longlong(token), _ptr(weights), _ptr(scale))
+    return [t, weights, scale], (t, pieces, piece, token, weights, scale)
 
 
 def join_norms(x: torch.Tensor, residual: "torch.Tensor | ShareSum | JoinedBranches | None", weight1: torch.Tensor | None,
@@ -269,8 +283,8 @@ def join_norms(x: torch.Tensor, residual: "torch.Tensor | ShareSum | JoinedBranc
         if w is not None:
             _f32(w, "join_norms weight", H)
         outs.append(torch.empty(n, H, dtype=out_dtype, device=x.device) if w is not None else None)
-    _call("tl_join_norms", _ptr(x), *a1, *a2, _ptr(weight1), _ptr(weight2), ctypes.c_float(eps), _ptr(outs[0]), _ptr(outs[1]),
-          _code(outs[0], "join_norms out") if outs[0] is not None else F32, _ptr(rows), n, H, _stream())
+    _call("tl_join_norms", x, *a1, *a2, weight1, weight2, float(eps), outs[0], outs[1],
+          _code(outs[0], "join_norms out") if outs[0] is not None else F32, rows, n, H, _stream())
     return outs[0], outs[1]
 
 
@@ -281,7 +295,7 @@ def norm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torc
     T, n = x.shape
     _f32(weight, "norm_rows weight", n)
     out = torch.empty(T, n, dtype=out_dtype, device=x.device)
-    _call("tl_norm_rows", _ptr(x), x.stride(0) if T > 1 else max(n, x.stride(0)), _ptr(weight), ctypes.c_float(eps), _ptr(out),
+    _call("tl_norm_rows", x, x.stride(0) if T > 1 else max(n, x.stride(0)), weight, float(eps), out,
           _code(out, "norm_rows out"), T, n, _stream())
     return out
 
@@ -290,7 +304,7 @@ def scale_cap(z: torch.Tensor, scale: float, cap: float = 0.0) -> torch.Tensor:
     """``cap * tanh(scale * z / cap)`` of a float32 tensor, written over it; ``cap`` 0: ``scale * z``."""
     _on_gpu(z)
     _f32(z, "scale_cap input")
-    _call("tl_scale_cap", _ptr(z), ctypes.c_longlong(z.numel()), ctypes.c_float(scale), ctypes.c_float(cap), _stream())
+    _call("tl_scale_cap", z, z.numel(), float(scale), float(cap), _stream())
     return z
 
 
@@ -323,8 +337,8 @@ def add_layernorm(x: torch.Tensor, residual: "torch.Tensor | ScaledBranches | No
             _i32(rows, "rows")
             n = rows.numel()
         out = torch.empty(n, H, dtype=out_dtype, device=x.device)
-    _call("tl_add_layernorm", _ptr(x), _ptr(y1), n1, ctypes.c_longlong(st1), _ptr(y2), n2, ctypes.c_longlong(st2), ctypes.c_float(mult), _ptr(weight), _ptr(bias), ctypes.c_float(eps),
-          _ptr(out), _code(out, "add_layernorm out") if out is not None else F32, _ptr(rows), n, H, _stream())
+    _call("tl_add_layernorm", x, y1, n1, st1, y2, n2, st2, float(mult), weight, bias, float(eps),
+          out, _code(out, "add_layernorm out") if out is not None else F32, rows, n, H, _stream())
     return out
 
 
@@ -363,9 +377,9 @@ def add_rmsnorm(x: torch.Tensor, residual: "torch.Tensor | ShareSum | None", wei
     if out is None:
         out = torch.empty(n, H, dtype=out_dtype, device=x.device)
     _check(out.dtype == out_dtype and out.is_contiguous() and tuple(out.shape) == (n, H), "add_rmsnorm: bad output")
-    _call("tl_add_rmsnorm", _ptr(x), _ptr(residual), res_code, parts, ctypes.c_longlong(part_stride), _ptr(weight),
-          _ptr(out), _code(out, "add_rmsnorm out"),
-          _ptr(rows), n, H, ctypes.c_float(eps), _stream())
+    _call("tl_add_rmsnorm", x, residual, res_code, parts, part_stride, weight,
+          out, _code(out, "add_rmsnorm out"),
+          rows, n, H, float(eps), _stream())
     return out
 
 
@@ -411,7 +425,7 @@ def weight_ranges(shuffled: torch.Tensor | None, N: int, K: int) -> torch.Tensor
     _check_shuffled(shuffled, N, K)
     _on_gpu(shuffled)
     out = torch.empty(library().tl_gemm_float_ranges_size(N, K), dtype=torch.int32, device=shuffled.device)
-    _call("tl_gemm_float_ranges", _ptr(shuffled), _ptr(out), N, K, _stream())
+    _call("tl_gemm_float_ranges", shuffled, out, N, K, _stream())
     return out
 
 
@@ -503,7 +517,7 @@ def _norm_args(owed: NormedRows | None, sink: NormSink | None, M: int, N: int, d
         na.resid, na.resid_ld, na.next_weight = r.data_ptr(), r.stride(0), w.data_ptr()
         na.a_out, na.a_ld = produced.rows.data_ptr(), N
         na.ss_out, na.ss_out_ld = produced.sumsq.data_ptr(), M
-    return ctypes.byref(na), produced
+    return na, produced
 
 
 def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tensor | None = None,
@@ -538,8 +552,8 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
             na = _NormArgs()
             na.act = 1
             res = torch.empty(M, N, dtype=out_dtype or a.dtype, device=a.device)
-            _call("tl_gemm_skinny", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(res), _code(res, "linear output"), M, N, K, lda, N,
-                  ctypes.byref(na), _stream())
+            _call("tl_gemm_skinny", a, shuffled, bias, res, _code(res, "linear output"), M, N, K, lda, N,
+                  na, _stream())
             return res
         if a.dim() == 2 and a.stride(1) == 1 and _bfloat16_matrix(weight, weight.shape[0], K):
             plan = _tiles_plan(a, shuffled, M, weight.shape[0], K, lda)
@@ -574,7 +588,7 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
         if produced is None:
             out = torch.empty(M, N, dtype=out_dtype, device=a.device)
         if few:
-            _call("tl_gemm_skinny", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out),
+            _call("tl_gemm_skinny", a, shuffled, bias, out,
                   F32 if out is None else _code(out, "linear output"), M, N, K, lda, N, norm, _stream())
         else:
             _rows64(a, shuffled, bias, out, M, N, K, lda, N, swiglu=False, norm=norm)
@@ -653,7 +667,7 @@ def _float_split(a, shuffled, ranges, bias, out, M, N, K, lda, ldc):
         floats = library().tl_gemm_float_split_workspace(m, N, K)
         if floats and (ws is None or ws.numel() < floats):
             ws = torch.empty(floats, dtype=torch.float32, device=a.device)
-        _call("tl_gemm_float_split", _ptr(a[r:]), _ptr(shuffled), _ptr(ranges), _ptr(bias), _ptr(out[r:]), _ptr(split), _ptr(ws), m, N, K, lda, ldc, _stream())
+        _call("tl_gemm_float_split", a[r:], shuffled, ranges, bias, out[r:], split, ws, m, N, K, lda, ldc, _stream())
     return out
 
 
@@ -661,13 +675,18 @@ def _rows64(a, shuffled, bias, out, M, N, K, lda, ldc, swiglu: bool, norm=None):
     """17 to 64 rows: a 16-column tile per wave, rows shared through LDS, K split over the grid."""
     shares = library().tl_gemm_rows64_shares(M, N, K)
     ws = torch.empty(shares * M * N, dtype=torch.float32, device=a.device) if shares > 1 else None
-    _call("tl_gemm_rows64", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), F32 if out is None else _code(out, "linear output"),
-          _ptr(ws), M, N, K, lda, ldc, shares, 1 if swiglu else 0, norm, _stream())
+    _call("tl_gemm_rows64", a, shuffled, bias, out, F32 if out is None else _code(out, "linear output"),
+          ws, M, N, K, lda, ldc, shares, 1 if swiglu else 0, norm, _stream())
     return out
 
 
 def _bfloat16_matrix(weight: torch.Tensor, N: int, K: int) -> bool:
     return weight.dtype == torch.bfloat16 and tuple(weight.shape) == (N, K) and weight.is_contiguous()
+
+
+@functools.lru_cache(maxsize=4096)
+def _tiles_cut(M: int, N: int, K: int, gated: bool, takes_shares: bool) -> int:
+    return max(0, library().tl_gemm_tiles_plan(M, N, K, 1 if gated else 0, 1 if takes_shares else 0))
 
 
 def _tiles_plan(a, shuffled, M, N, K, lda, gated: bool = False, takes_shares: bool = False) -> int:
@@ -678,7 +697,7 @@ def _tiles_plan(a, shuffled, M, N, K, lda, gated: bool = False, takes_shares: bo
             or lda % 8 or lda < K or lda >= 1 << 22 or a.data_ptr() % 16
             or tuple(shuffled.shape) != (-(-N // 16), -(-K // 32), 4, 16, 8) or not shuffled.is_contiguous()):
         return 0
-    return max(0, library().tl_gemm_tiles_plan(M, N, K, 1 if gated else 0, 1 if takes_shares else 0))
+    return _tiles_cut(M, N, K, gated, takes_shares)
 
 
 def _tiles(a, shuffled, bias, out_dtype, M, N, K, lda, plan: int, keep_shares: bool = False, gated: bool = False, act: int = 0):
@@ -691,7 +710,7 @@ def _tiles(a, shuffled, bias, out_dtype, M, N, K, lda, plan: int, keep_shares: b
     ws = torch.empty(shares, M, N, dtype=torch.float32, device=a.device) if shares > 1 else None
     kept = shares > 1 and keep_shares and bias is None and out_dtype == torch.float32
     out = None if kept else torch.empty(M, N // 2 if gated else N, dtype=out_dtype, device=a.device)
-    _call("tl_gemm_tiles", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), F32 if out is None else _code(out, "linear output"), _ptr(ws),
+    _call("tl_gemm_tiles", a, shuffled, bias, out, F32 if out is None else _code(out, "linear output"), ws,
           M, N, K, lda, N // 2 if gated else N, tile, shares, 1 if gated else 0, act, _stream())
     return ShareSum(ws) if kept else out
 
@@ -702,20 +721,20 @@ def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None, ran
     kernel.  (bfloat16 with many rows went to gemm_tiles.hip or the library before this; the reference uses a library:
     tensorline/paged.py:179-188.)"""
     if _skinny_ok(a, shuffled, M, K, lda) and not _few_rows_go_to_rows64(N, K):
-        _call("tl_gemm_skinny", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), _code(out, "linear output"),
+        _call("tl_gemm_skinny", a, shuffled, bias, out, _code(out, "linear output"),
               M, N, K, lda, ldc, None, _stream())
         return out
     if _rows64_ok(a, shuffled, M, K, lda, few_too=True):
         return _rows64(a, shuffled, bias, out, M, N, K, lda, ldc, swiglu=False)
     if (shuffled is not None and shuffled.dtype == torch.float32 and a.dtype == torch.float32 and out.dtype == torch.float32
             and M <= SKINNY_MAX_ROWS and library().tl_gemm_fewrows_takes(K)):
-        _call("tl_gemm_fewrows_shuffled", _ptr(a), _ptr(shuffled), _ptr(bias), _ptr(out), M, N, K, lda, ldc, _stream())
+        _call("tl_gemm_fewrows_shuffled", a, shuffled, bias, out, M, N, K, lda, ldc, _stream())
         return out
     if (shuffled is not None and shuffled.dtype == torch.float32 and a.dtype == torch.float32 and out.dtype == torch.float32
             and SKINNY_MAX_ROWS < M <= FLOAT_SPLIT_MAX_ROWS and K >= FLOAT_SPLIT_MIN_K):
         return _float_split(a, shuffled, ranges, bias, out, M, N, K, lda, ldc)
-    _call("tl_gemm_generic", _ptr(a), _code(a, "linear input"), _ptr(weight), _code(weight, "linear weight"),
-          _ptr(bias), _ptr(out), _code(out, "linear output"), M, N, K, lda, ldc, _stream())
+    _call("tl_gemm_generic", a, _code(a, "linear input"), weight, _code(weight, "linear weight"),
+          bias, out, _code(out, "linear output"), M, N, K, lda, ldc, _stream())
     return out
 
 
@@ -840,7 +859,7 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
             out = torch.empty(M, I, dtype=h.dtype, device=h.device)
             na = _NormArgs()
             na.act = 2
-            _call("tl_gemm_skinny_swiglu", _ptr(h), _ptr(shuffled), _ptr(out), M, I, K, lda, I, ctypes.byref(na), _stream())
+            _call("tl_gemm_skinny_swiglu", h, shuffled, out, M, I, K, lda, I, na, _stream())
             return out
         if _rows64_ok(h, shuffled, M, K, lda) and (I % 16 == 0 or library().tl_gemm_rows64_shares(M, 2 * I, K) > 1):
             _on_gpu(h, gate_up_weight, shuffled)
@@ -849,7 +868,7 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
             out = torch.empty(M, I, dtype=h.dtype, device=h.device)
             na = _NormArgs()
             na.act = 2
-            return _rows64(h, shuffled, None, out, M, 2 * I, K, lda, I, swiglu=True, norm=ctypes.byref(na))
+            return _rows64(h, shuffled, None, out, M, 2 * I, K, lda, I, swiglu=True, norm=na)
         if h.dim() == 2 and h.stride(1) == 1 and _bfloat16_matrix(gate_up_weight, 2 * I, K):
             plan = _tiles_plan(h, shuffled, M, 2 * I, K, lda, gated=True)
             if plan:
@@ -870,7 +889,7 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
     if _skinny_ok(h, shuffled, M, K, lda) and I % 16 == 0:
         out = torch.empty(M, I, dtype=h.dtype, device=h.device)
         norm, _ = _norm_args(owed, None, M, 2 * I, h.device)
-        _call("tl_gemm_skinny_swiglu", _ptr(h), _ptr(shuffled), _ptr(out), M, I, K, lda, I, norm, _stream())
+        _call("tl_gemm_skinny_swiglu", h, shuffled, out, M, I, K, lda, I, norm, _stream())
         return out
     if _rows64_ok(h, shuffled, M, K, lda) and (I % 16 == 0 or library().tl_gemm_rows64_shares(M, 2 * I, K) > 1):
         out = torch.empty(M, I, dtype=h.dtype, device=h.device)
@@ -928,12 +947,12 @@ def qkv_rope_store(h: torch.Tensor | NormedRows, shuffled: torch.Tensor, bias: t
     norm, _ = _norm_args(owed, None, M, N, h.device)
     if M > SKINNY_MAX_ROWS:
         ws = torch.empty(shares * M * N, dtype=torch.float32, device=h.device)
-        _call("tl_gemm_rows64_qkv_rope", _ptr(h), _ptr(shuffled), _ptr(bias), _ptr(pos), _ptr(inv_freq), _ptr(slots),
-              _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(ws), M, K, h.stride(0), num_heads, num_kv_heads, head_dim,
+        _call("tl_gemm_rows64_qkv_rope", h, shuffled, bias, pos, inv_freq, slots,
+              q, k_cache, v_cache, ws, M, K, h.stride(0), num_heads, num_kv_heads, head_dim,
               k_cache.shape[1], shares, norm, _stream())
         return q
-    _call("tl_gemm_skinny_qkv_rope", _ptr(h), _ptr(shuffled), _ptr(bias), _ptr(pos), _ptr(inv_freq), _ptr(slots),
-          _ptr(q), _ptr(k_cache), _ptr(v_cache), M, K, h.stride(0) if M > 1 else K, num_heads, num_kv_heads,
+    _call("tl_gemm_skinny_qkv_rope", h, shuffled, bias, pos, inv_freq, slots,
+          q, k_cache, v_cache, M, K, h.stride(0) if M > 1 else K, num_heads, num_kv_heads,
           head_dim, k_cache.shape[1], norm, _stream())
     return q
 
@@ -964,9 +983,9 @@ def rope_store(qkv: torch.Tensor, pos: torch.Tensor, inv_freq: torch.Tensor | No
         _check(v_cache is not None and slots is not None, "rope_store: cache write needs k_cache, v_cache and slots")
         _check_caches(k_cache, v_cache, qkv.dtype, num_kv_heads, head_dim, "rope_store")
         _i32(slots, "slots", T)
-    _call("tl_rope_store", _ptr(qkv), _code(qkv, "rope_store"), _ptr(pos), _ptr(inv_freq), _ptr(k_cache), _ptr(v_cache),
-          _ptr(slots), T, num_heads, num_kv_heads, head_dim, rot, 1 if write else 0,
-          k_cache.shape[1] if write else 0, _ptr(bias), _stream())
+    _call("tl_rope_store", qkv, _code(qkv, "rope_store"), pos, inv_freq, k_cache, v_cache,
+          slots, T, num_heads, num_kv_heads, head_dim, rot, 1 if write else 0,
+          k_cache.shape[1] if write else 0, bias, _stream())
 
 
 def one_token_sequences(facts) -> list[int]:
@@ -1214,7 +1233,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     _on_gpu(q, k_cache, v_cache, tables, seq_of_token, pos, out, q_start, ctx_start, sink)
     if sink is not None:
         _f32(sink, "paged_attention sink", num_heads)
-    cap = ctypes.c_float(softcap)
+    cap = float(softcap)
     reach = 0
     if bias is not None:
         _on_gpu(q, bias)
@@ -1258,11 +1277,11 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             nt1 = 1 if G <= 16 or head_dim == 256 else 2      # a head size of 256: one column tile per wave (registers)
             ws = torch.empty(launch.singles * num_heads * nsplit * (head_dim + 2), dtype=torch.float32, device=q.device)
             n_o = launch.singles * num_heads * nsplit * head_dim
-            _call("tl_attention_mfma", _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(tables), tables.shape[1],
-                  _ptr(q_start), _ptr(ctx_start), _ptr(pos), _ptr(out), o_stride, _ptr(ws[:n_o]), _ptr(ws[n_o:]), T, S,
-                  num_heads, num_kv_heads, head_dim, page, int(window), ctypes.c_float(scale), nt1,
-                  -(-G // (16 * nt1)), nsplit, max(split_len // 32, 1), 0, 0, _ptr(single_seqs), launch.singles, 0,
-                  _ptr(sink), cap, keep_first, chunk, _ptr(bias), reach, _stream())
+            _call("tl_attention_mfma", q, q_stride, k_cache, v_cache, tables, tables.shape[1],
+                  q_start, ctx_start, pos, out, o_stride, ws[:n_o], ws[n_o:], T, S,
+                  num_heads, num_kv_heads, head_dim, page, int(window), float(scale), nt1,
+                  -(-G // (16 * nt1)), nsplit, max(split_len // 32, 1), 0, 0, ctypes.c_void_p(_ptr(single_seqs)), launch.singles, 0,
+                  sink, cap, keep_first, chunk, bias, reach, _stream())
         skip_single, nt, max_groups, total128 = 1 if launch.own_split else 0, launch.nt, launch.max_groups, launch.total128
         split_len, nsplit = launch.split_len, launch.nsplit
         split_blocks = max(split_len // 32, 1)
@@ -1275,17 +1294,17 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                 and library().tl_attention_tile32_takes(head_dim, page, tables.shape[1], S, waves, G * (reach + 1) if bias is not None else 0)):
             # prompt portions behind many keys, head size 64 or 128: 32 columns per wave on the 32x32
             # matrix-core instruction, work-groups of 256 columns
-            _call("tl_attention_tile32", _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(tables), tables.shape[1],
-                  _ptr(q_start), _ptr(ctx_start), _ptr(out), o_stride, T, S, num_heads, num_kv_heads, head_dim, page,
-                  int(window), ctypes.c_float(scale), waves, launch.total32, skip_single, _ptr(sink), cap, keep_first, chunk,
-                  _ptr(bias), reach, _stream())
+            _call("tl_attention_tile32", q, q_stride, k_cache, v_cache, tables, tables.shape[1],
+                  q_start, ctx_start, out, o_stride, T, S, num_heads, num_kv_heads, head_dim, page,
+                  int(window), float(scale), waves, launch.total32, skip_single, sink, cap, keep_first, chunk,
+                  bias, reach, _stream())
             return out
-        _call("tl_attention_mfma", _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(tables), tables.shape[1],
-              _ptr(q_start), _ptr(ctx_start), _ptr(pos), _ptr(out), o_stride, _ptr(ws_o), _ptr(ws_ml), T, S, num_heads,
-              num_kv_heads, head_dim, page, int(window), ctypes.c_float(scale), nt, max_groups, nsplit, split_blocks,
+        _call("tl_attention_mfma", q, q_stride, k_cache, v_cache, tables, tables.shape[1],
+              q_start, ctx_start, pos, out, o_stride, ws_o, ws_ml, T, S, num_heads,
+              num_kv_heads, head_dim, page, int(window), float(scale), nt, max_groups, nsplit, split_blocks,
               launch.chains, total128,
-              _ptr(None), 0,
-              skip_single, _ptr(sink), cap, keep_first, chunk, _ptr(bias), reach, _stream())
+              ctypes.c_void_p(0), 0,
+              skip_single, sink, cap, keep_first, chunk, bias, reach, _stream())
         return out
     # The any-shape kernel tiles each sequence's tokens: it needs the first row of every sequence and the
     # most tokens one of them brings.  The engine has both; a bare call derives them from seq_of_token.
@@ -1320,10 +1339,10 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             nsplit = 2
         if nsplit > 1:
             ws = torch.empty(T * num_heads * nsplit * (head_dim + 2), dtype=torch.float32, device=q.device)
-    _call("tl_attention_generic", _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(tables), tables.shape[1],
-          _ptr(q_start), _ptr(pos), _ptr(out), o_stride, _code(q, "paged_attention"), T, S, max(max_query_len, 1), num_heads,
-          num_kv_heads, head_dim, page, int(window), ctypes.c_float(scale), nsplit, split_len, _ptr(ws), _ptr(sink), cap,
-          keep_first, chunk, _ptr(bias), reach, _stream())
+    _call("tl_attention_generic", q, q_stride, k_cache, v_cache, tables, tables.shape[1],
+          q_start, pos, out, o_stride, _code(q, "paged_attention"), T, S, max(max_query_len, 1), num_heads,
+          num_kv_heads, head_dim, page, int(window), float(scale), nsplit, split_len, ws, sink, cap,
+          keep_first, chunk, bias, reach, _stream())
     return out
 
 
@@ -1336,7 +1355,7 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Te
     if out is None:
         out = torch.empty(T, I2 // 2, dtype=gate_up.dtype, device=gate_up.device)
     _check(out.dtype == gate_up.dtype and out.is_contiguous() and tuple(out.shape) == (T, I2 // 2), "silu_mul: bad output")
-    _call("tl_silu_mul", _ptr(gate_up), _ptr(out), _code(gate_up, "silu_mul"), T, I2 // 2, _stream())
+    _call("tl_silu_mul", gate_up, out, _code(gate_up, "silu_mul"), T, I2 // 2, _stream())
     return out
 
 
@@ -1352,7 +1371,7 @@ def argmax(logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tenso
     if V > 8192:            # wide rows: per-chunk bests, then the row's best among them
         sv = torch.empty(R * 64, dtype=torch.float32, device=logits.device)
         si = torch.empty(R * 64, dtype=torch.int32, device=logits.device)
-    _call("tl_argmax", _ptr(logits), logits.stride(0) if R > 1 else V, R, V, _ptr(out), _ptr(sv), _ptr(si), _stream())
+    _call("tl_argmax", logits, logits.stride(0) if R > 1 else V, R, V, out, sv, si, _stream())
     return out
 
 
@@ -1377,8 +1396,8 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.Tensor,
     chunks = library().tl_sample_chunks(V)
     pmax = torch.empty(R * chunks, dtype=torch.float32, device=logits.device)
     ws = torch.zeros(R * (3080 + 3 * chunks), dtype=torch.int64, device=logits.device)
-    _call("tl_sample", _ptr(logits), logits.stride(0) if R > 1 else V, R, V, _ptr(temperature), _ptr(top_p),
-          _ptr(uniform), _ptr(out), _ptr(pmax), _ptr(ws), 1 if any_greedy else 0, 1 if any_top_p else 0, _stream())
+    _call("tl_sample", logits, logits.stride(0) if R > 1 else V, R, V, temperature, top_p,
+          uniform, out, pmax, ws, 1 if any_greedy else 0, 1 if any_top_p else 0, _stream())
     return out
 
 
@@ -1412,8 +1431,8 @@ def add_dyt(x: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor
         _i32(rows, "rows")
         n = rows.numel()
     out = torch.empty(n, H, dtype=out_dtype, device=x.device)
-    _call("tl_add_dyt", _ptr(x), _ptr(residual), res_code, _ptr(weight), _ptr(bias), _ptr(alpha), _ptr(out),
-          _code(out, "add_dyt out"), _ptr(rows), n, H, _stream())
+    _call("tl_add_dyt", x, residual, res_code, weight, bias, alpha, out,
+          _code(out, "add_dyt out"), rows, n, H, _stream())
     return out
 
 
@@ -1425,7 +1444,7 @@ def add_cast(x: torch.Tensor, residual: torch.Tensor | None, out_dtype: torch.dt
         _check(residual.dtype == torch.float32 and residual.is_contiguous() and residual.shape == x.shape,
                "add_cast: the residual must be float32 of x's shape")
     out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    _call("tl_add_cast", _ptr(x), _ptr(residual), _ptr(out), _code(out, "add_cast out"), ctypes.c_longlong(x.numel()), _stream())
+    _call("tl_add_cast", x, residual, out, _code(out, "add_cast out"), x.numel(), _stream())
     return out
 
 
@@ -1435,7 +1454,7 @@ def cast_rows(x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     _check(x.dtype == torch.float32 and x.dim() == 2 and x.stride(1) == 1, "cast_rows: the input must be float32 [T, n]")
     T, n = x.shape
     out = torch.empty(T, n, dtype=out_dtype, device=x.device)
-    _call("tl_cast_rows", _ptr(x), x.stride(0) if T > 1 else max(n, x.stride(0)), _ptr(out), _code(out, "cast_rows out"), T, n, _stream())
+    _call("tl_cast_rows", x, x.stride(0) if T > 1 else max(n, x.stride(0)), out, _code(out, "cast_rows out"), T, n, _stream())
     return out
 
 
@@ -1444,7 +1463,7 @@ def tanh_rows(z: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     _on_gpu(z)
     _check(z.dtype == torch.float32 and z.is_contiguous(), "tanh_rows: input must be contiguous float32")
     out = torch.empty(z.shape, dtype=out_dtype, device=z.device)
-    _call("tl_unary", _ptr(z), _ptr(out), _code(out, "tanh_rows out"), ctypes.c_longlong(z.numel()), 0, _stream())
+    _call("tl_unary", z, out, _code(out, "tanh_rows out"), z.numel(), 0, _stream())
     return out
 
 
@@ -1453,7 +1472,7 @@ def relu_squared(z: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     _on_gpu(z)
     _check(z.dtype == torch.float32 and z.is_contiguous(), "relu_squared: input must be contiguous float32")
     out = torch.empty(z.shape, dtype=out_dtype, device=z.device)
-    _call("tl_unary", _ptr(z), _ptr(out), _code(out, "relu_squared out"), ctypes.c_longlong(z.numel()), 1, _stream())
+    _call("tl_unary", z, out, _code(out, "relu_squared out"), z.numel(), 1, _stream())
     return out
 
 
@@ -1462,7 +1481,7 @@ def scaled_sum(x: torch.Tensor, y: torch.Tensor, a: float, b: float) -> torch.Te
     _on_gpu(x, y)
     _check(x.dtype == y.dtype == torch.float32 and x.is_contiguous() and y.is_contiguous() and x.shape == y.shape,
            "scaled_sum: two contiguous float32 tensors of one shape are needed")
-    _call("tl_scaled_sum", _ptr(x), _ptr(y), _ptr(x), ctypes.c_float(a), ctypes.c_float(b), ctypes.c_longlong(x.numel()), _stream())
+    _call("tl_scaled_sum", x, y, x, float(a), float(b), x.numel(), _stream())
     return x
 
 
@@ -1473,8 +1492,8 @@ def clamp_glu(gate_up: torch.Tensor, limit: float, alpha: float, out_dtype: torc
     _check(gate_up.dim() == 2 and gate_up.is_contiguous() and gate_up.shape[1] % 2 == 0, "clamp_glu: input must be contiguous [T, 2F]")
     T, F2 = gate_up.shape
     out = torch.empty(T, F2 // 2, dtype=out_dtype or gate_up.dtype, device=gate_up.device)
-    _call("tl_clamp_glu", _ptr(gate_up), _code(gate_up, "clamp_glu in"), _ptr(out), _code(out, "clamp_glu out"), T, F2 // 2,
-          ctypes.c_float(limit), ctypes.c_float(alpha), _stream())
+    _call("tl_clamp_glu", gate_up, _code(gate_up, "clamp_glu in"), out, _code(out, "clamp_glu out"), T, F2 // 2,
+          float(limit), float(alpha), _stream())
     return out
 
 
@@ -1490,7 +1509,7 @@ def glu(gate_up: torch.Tensor, activation: str, out_dtype: torch.dtype | None = 
     _check(gate_up.dim() == 2 and gate_up.is_contiguous() and gate_up.shape[1] % 2 == 0, "glu: input must be contiguous [T, 2F]")
     T, F2 = gate_up.shape
     out = torch.empty(T, F2 // 2, dtype=out_dtype or gate_up.dtype, device=gate_up.device)
-    _call("tl_glu", _ptr(gate_up), _code(gate_up, "glu in"), _ptr(out), _code(out, "glu out"), T, F2 // 2,
+    _call("tl_glu", gate_up, _code(gate_up, "glu in"), out, _code(out, "glu out"), T, F2 // 2,
           GLU_ACTIVATIONS[activation], _stream())
     return out
 
@@ -1508,8 +1527,8 @@ def gated_group_norm(o: torch.Tensor, weight: torch.Tensor, gate: torch.Tensor, 
     _f32(weight, "gated_group_norm weight", N)
     _check(gate_act in _GATE_ACTS and group > 0 and N % group == 0, "gated_group_norm: bad group or gate")
     out = torch.empty(T, N, dtype=out_dtype, device=o.device)
-    _call("tl_gated_group_norm", _ptr(o), o.stride(0) if T > 1 else N, _ptr(weight), _ptr(gate), gate.stride(0) if T > 1 else N,
-          _ptr(out), _code(out, "gated_group_norm out"), T, N, int(group), ctypes.c_float(eps), _GATE_ACTS[gate_act],
+    _call("tl_gated_group_norm", o, o.stride(0) if T > 1 else N, weight, gate, gate.stride(0) if T > 1 else N,
+          out, _code(out, "gated_group_norm out"), T, N, int(group), float(eps), _GATE_ACTS[gate_act],
           _stream())
     return out
 
@@ -1517,13 +1536,13 @@ def gated_group_norm(o: torch.Tensor, weight: torch.Tensor, gate: torch.Tensor, 
 _GATE_ACTS = {"sigmoid": 0, "silu": 1, "silu_first": 2}
 
 
-def _state_ptr(state: torch.Tensor, offset: int) -> tuple[ctypes.c_void_p, int]:
+def _state_ptr(state: torch.Tensor, offset: int) -> tuple[int, int]:
     """(address of element ``offset`` of slot 0, elements from one slot to the next) of a float32
     state arena [slots, n]; the arena may be a block of columns of a wider one (a mixer's share of the
     state that several mixers of a layer keep side by side)."""
     _check(state.dtype == torch.float32 and state.dim() == 2 and state.stride(1) == 1 and 0 <= offset <= state.shape[1],
            "a state arena must be float32 [slots, n] with a slot's values contiguous")
-    return ctypes.c_void_p(state.data_ptr() + 4 * offset), state.stride(0)
+    return _ptr(state) + 4 * offset, state.stride(0)
 
 
 def token_shift(h: torch.Tensor, mu: torch.Tensor, ctx, state: torch.Tensor, offset: int) -> torch.Tensor:
@@ -1538,8 +1557,8 @@ def token_shift(h: torch.Tensor, mu: torch.Tensor, ctx, state: torch.Tensor, off
     _check(offset + W <= state.shape[1], "token_shift: the kept row does not fit the state")
     prev, stride = _state_ptr(state, offset)
     out = torch.empty(mu.shape[0], T, W, dtype=h.dtype, device=h.device)
-    _call("tl_token_shift", _ptr(h), _code(h, "token_shift"), _ptr(ctx.seq_of_token), _ptr(ctx.q_start), _ptr(ctx.state_slots),
-          prev, ctypes.c_longlong(stride), _ptr(mu), _ptr(out), T, ctx.num_seqs, W, mu.shape[0], _stream())
+    _call("tl_token_shift", h, _code(h, "token_shift"), ctx.seq_of_token, ctx.q_start, ctx.state_slots,
+          prev, stride, mu, out, T, ctx.num_seqs, W, mu.shape[0], _stream())
     return out
 
 
@@ -1551,7 +1570,7 @@ def gelu_token_gate(z: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, col
     _i32(ids, "ids", T)
     _check(table.dim() == 2 and table.is_contiguous() and col0 + D <= table.shape[1], "gelu_token_gate: bad table")
     out = torch.empty(T, D, dtype=table.dtype, device=z.device)
-    _call("tl_gelu_token_gate", _ptr(z), _ptr(table), _code(table, "gelu_token_gate table"), _ptr(ids), _ptr(out), T, D,
+    _call("tl_gelu_token_gate", z, table, _code(table, "gelu_token_gate table"), ids, out, T, D,
           table.shape[1], int(col0), table.shape[0], _stream())
     return out
 
@@ -1587,8 +1606,8 @@ def latent_prepare(proj: torch.Tensor, pos: torch.Tensor, freq: torch.Tensor, ma
     ld = lambda t: t.stride(0) if T > 1 else max(t.shape[1], t.stride(0))
     q_plain = torch.empty(T, heads * dim, dtype=k_cache.dtype, device=proj.device)
     q_lat = torch.empty(T, heads * D, dtype=k_cache.dtype, device=proj.device)
-    _call("tl_latent_prepare", _ptr(q), ld(q), _ptr(down), ld(down), _ptr(pos), _ptr(freq), ctypes.c_float(mag),
-          _ptr(norm_weight), ctypes.c_float(eps), _ptr(slots), _ptr(q_plain), _ptr(q_lat), _ptr(k_cache), _ptr(v_cache),
+    _call("tl_latent_prepare", q, ld(q), down, ld(down), pos, freq, float(mag),
+          norm_weight, float(eps), slots, q_plain, q_lat, k_cache, v_cache,
           _code(k_cache, "latent_prepare cache"), T, heads, dim, rot, rank, D, page, _stream())
     return q_plain, q_lat
 
@@ -1612,8 +1631,8 @@ def wide_row_attention(q: torch.Tensor, k_cache: torch.Tensor, tables: torch.Ten
     _i32(seq_of_token, "seq_of_token", T)
     _i32(pos, "pos", T)
     out = torch.empty_like(q)
-    _call("tl_attention_wide", _ptr(q), _ptr(k_cache), _code(q, "wide_row_attention"), _ptr(tables), tables.shape[1],
-          _ptr(seq_of_token), _ptr(pos), _ptr(out), T, heads, D, page, ctypes.c_float(scale), int(window or 0), _stream())
+    _call("tl_attention_wide", q, k_cache, _code(q, "wide_row_attention"), tables, tables.shape[1],
+          seq_of_token, pos, out, T, heads, D, page, float(scale), int(window or 0), _stream())
     return out
 
 
@@ -1623,7 +1642,7 @@ def head_gate(o: torch.Tensor, gate: torch.Tensor, heads: int) -> torch.Tensor:
     T = o.shape[0]
     _check(o.is_contiguous() and o.shape[1] % heads == 0 and gate.dtype == torch.float32 and gate.stride(1) == 1
            and tuple(gate.shape) == (T, heads), "head_gate: bad shapes")
-    _call("tl_head_gate", _ptr(o), _code(o, "head_gate"), _ptr(gate), gate.stride(0) if T > 1 else heads, T, heads,
+    _call("tl_head_gate", o, _code(o, "head_gate"), gate, gate.stride(0) if T > 1 else heads, T, heads,
           o.shape[1] // heads, _stream())
     return o
 
@@ -1639,10 +1658,10 @@ def batched_linear(a: torch.Tensor, weights: torch.Tensor, out: torch.Tensor) ->
            and a.stride(2) == 1 and out.stride(2) == 1 and a.dtype == weights.dtype == out.dtype, "batched_linear: bad shapes")
     if T == 0:
         return out
-    _call("tl_gemm_generic_batched", _ptr(a), _code(a, "batched_linear"), _ptr(weights), _code(weights, "batched_linear"),
-          _ptr(out), _code(out, "batched_linear"), T, N, K, a.stride(0) if T > 1 else max(K, a.stride(0)),
-          out.stride(0) if T > 1 else max(N, out.stride(0)), B, ctypes.c_longlong(a.stride(1)),
-          ctypes.c_longlong(N * K), ctypes.c_longlong(out.stride(1)), _stream())
+    _call("tl_gemm_generic_batched", a, _code(a, "batched_linear"), weights, _code(weights, "batched_linear"),
+          out, _code(out, "batched_linear"), T, N, K, a.stride(0) if T > 1 else max(K, a.stride(0)),
+          out.stride(0) if T > 1 else max(N, out.stride(0)), B, a.stride(1),
+          N * K, out.stride(1), _stream())
     return out
 
 
@@ -1711,14 +1730,14 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ctx, st
         S = ctx.num_seqs
         ws = torch.empty(S * chunks * heads * (dk * dv + 1), dtype=torch.float32, device=q.device)
         n_state = S * chunks * heads * dk * dv
-        _call("tl_ssd_chunked", _ptr(q), ld(q), _ptr(k), ld(k), _ptr(v), ld(v), _ptr(steps), ld(steps), _ptr(rate_log),
-              _ptr(step_bias), _ptr(skip), share, st, ctypes.c_longlong(stride), _ptr(ctx.state_slots), _ptr(ctx.q_start),
-              _ptr(out), heads * dv, _ptr(ws[:n_state]), _ptr(ws[n_state:]), S, chunks, heads, dk, dv, _stream())
+        _call("tl_ssd_chunked", q, ld(q), k, ld(k), v, ld(v), steps, ld(steps), rate_log,
+              step_bias, skip, share, st, stride, ctx.state_slots, ctx.q_start,
+              out, heads * dv, ws[:n_state], ws[n_state:], S, chunks, heads, dk, dv, _stream())
         return out
-    _call("tl_linear_recurrence", _ptr(q), ld(q), _ptr(k), ld(k), _ptr(v), ld(v), _ptr(wlog), ld(wlog) if per_token else 0,
-          _ptr(decay), _ptr(bonus), per_token, _ptr(skip if per_token == 2 else None), share,
-          st, ctypes.c_longlong(stride), _ptr(ctx.state_slots),
-          _ptr(ctx.q_start), _ptr(out), heads * dv, ctx.num_seqs, heads, dk, dv, 1 if silu_inputs else 0,
+    _call("tl_linear_recurrence", q, ld(q), k, ld(k), v, ld(v), wlog, ld(wlog) if per_token else 0,
+          decay, bonus, per_token, skip if per_token == 2 else None, share,
+          st, stride, ctx.state_slots,
+          ctx.q_start, out, heads * dv, ctx.num_seqs, heads, dk, dv, 1 if silu_inputs else 0,
           int(facts.max_query_len) if facts is not None else 0, _stream())
     return out
 
@@ -1795,9 +1814,9 @@ def conv_unit(x: torch.Tensor, taps: torch.Tensor, ctx, state: torch.Tensor, off
     _check(offset + (K - 1) * C <= state.shape[1], "conv_unit: the kept inputs do not fit the state")
     kept, stride = _state_ptr(state, offset)
     out = torch.empty(T, C, dtype=out_dtype, device=x.device)
-    _call("tl_conv_unit", _ptr(x), x.stride(0) if T > 1 else max(C, x.stride(0)), _ptr(taps), _ptr(bias), kept, ctypes.c_longlong(stride),
-          _ptr(ctx.state_slots), _ptr(ctx.seq_of_token), _ptr(ctx.q_start), _ptr(out), _code(out, "conv_unit out"), C, T, ctx.num_seqs, C, K, int(unit),
-          int(n_unit), int(n_scaled), ctypes.c_float(scale), ctypes.c_float(eps),
+    _call("tl_conv_unit", x, x.stride(0) if T > 1 else max(C, x.stride(0)), taps, bias, kept, stride,
+          ctx.state_slots, ctx.seq_of_token, ctx.q_start, out, _code(out, "conv_unit out"), C, T, ctx.num_seqs, C, K, int(unit),
+          int(n_unit), int(n_scaled), float(scale), float(eps),
           2 if ctx.facts.decode_only and T == ctx.num_seqs else 1, _stream())
     return out
 
@@ -1832,21 +1851,21 @@ def delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, b: torch.Tenso
     st, stride = _state_ptr(state, state_offset)
     out = torch.empty(T, heads * dv, dtype=torch.float32, device=q.device)
     ld = lambda t: t.stride(0) if T > 1 else max(t.shape[1], t.stride(0))
-    head = (_ptr(q), ld(q), _ptr(k), ld(k), _ptr(v), ld(v), _ptr(b), ld(b), _ptr(a), ld(a), _ptr(rate_log), _ptr(step_bias), share, st,
-            ctypes.c_longlong(stride), _ptr(ctx.state_slots), _ptr(ctx.q_start))
+    head = (q, ld(q), k, ld(k), v, ld(v), b, ld(b), a, ld(a), rate_log, step_bias, share, st,
+            stride, ctx.state_slots, ctx.q_start)
     if chunks is not None and library().tl_delta_chunked_takes(dk, dv):
         _check_chunks(chunks, ctx.num_seqs, "delta_rule")
         fn = library().tl_delta_chunked_workspace
         fn.restype = ctypes.c_longlong
         ws = torch.empty(chunks.count * heads * fn(dk, dv), dtype=torch.float32, device=q.device)
-        _call("tl_delta_chunked", *head, _ptr(chunks.seq), _ptr(chunks.row), _ptr(chunks.first), _ptr(ws), _ptr(out), heads * dv,
+        _call("tl_delta_chunked", *head, chunks.seq, chunks.row, chunks.first, ws, out, heads * dv,
               ctx.num_seqs, chunks.count, heads, dk, dv, _stream())
         if not chunks.walked:
             return out
         walk_upto = WALK_TOKENS
     else:
         walk_upto = 0
-    _call("tl_delta_walk", *head, _ptr(out), heads * dv, ctx.num_seqs, heads, dk, dv, walk_upto, _stream())
+    _call("tl_delta_walk", *head, out, heads * dv, ctx.num_seqs, heads, dk, dv, walk_upto, _stream())
     return out
 
 
@@ -1886,9 +1905,9 @@ def matrix_lstm(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_in: torc
     st, stride = _state_ptr(state, state_offset)
     out = torch.empty(T, heads * dv, dtype=torch.float32, device=q.device)
     ld = lambda t: t.stride(0) if T > 1 else max(t.shape[1], t.stride(0))
-    head = (_ptr(q), ld(q), _ptr(k), ld(k), _ptr(v), ld(v), _ptr(gate_in), ld(gate_in), _ptr(gate_forget), ld(gate_forget), _ptr(bias_in),
-            _ptr(bias_forget), ctypes.c_float(cap), ctypes.c_float(q_scale), ctypes.c_float(floor), st, ctypes.c_longlong(stride),
-            _ptr(ctx.state_slots), _ptr(ctx.q_start))
+    head = (q, ld(q), k, ld(k), v, ld(v), gate_in, ld(gate_in), gate_forget, ld(gate_forget), bias_in,
+            bias_forget, float(cap), float(q_scale), float(floor), st, stride,
+            ctx.state_slots, ctx.q_start)
     walk_upto = 0
     if chunks is not None:
         _check_chunks(chunks, ctx.num_seqs, "matrix_lstm")
@@ -1898,12 +1917,12 @@ def matrix_lstm(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_in: torc
         ws = torch.empty(n * fn(dk, dv), dtype=torch.float32, device=q.device)
         ws_g = torch.empty(2 * n, dtype=torch.float64, device=q.device)
         ws_m = torch.empty(n, dtype=torch.float32, device=q.device)
-        _call("tl_mlstm_chunked", *head, _ptr(chunks.seq), _ptr(chunks.row), _ptr(chunks.first), _ptr(ws), _ptr(ws_g), _ptr(ws_m), _ptr(out),
+        _call("tl_mlstm_chunked", *head, chunks.seq, chunks.row, chunks.first, ws, ws_g, ws_m, out,
               heads * dv, ctx.num_seqs, chunks.count, heads, dk, dv, _stream())
         if not chunks.walked:
             return out
         walk_upto = WALK_TOKENS
-    _call("tl_mlstm_walk", *head, _ptr(out), heads * dv, ctx.num_seqs, heads, dk, dv, walk_upto, _stream())
+    _call("tl_mlstm_walk", *head, out, heads * dv, ctx.num_seqs, heads, dk, dv, walk_upto, _stream())
     return out
 
 
@@ -1942,9 +1961,9 @@ def selective_scan(dt_raw: torch.Tensor, dt_bias: torch.Tensor | None, x: torch.
         ws_s = torch.empty(chunks.count * N * inner, dtype=torch.float32, device=x.device)
         ws_dt = torch.empty(chunks.count * inner, dtype=torch.float32, device=x.device)
     seq, row, first = (chunks.seq, chunks.row, chunks.first) if chunks is not None else (None, None, None)
-    _call("tl_selective_scan", _ptr(dt_raw), ld(dt_raw), _ptr(dt_bias), _ptr(x), ld(x), _ptr(z), ld(z), _ptr(bc), ld(bc), _ptr(a2),
-          _ptr(skip), st, ctypes.c_longlong(stride), _ptr(ctx.state_slots), _ptr(ctx.q_start), _ptr(seq), _ptr(row), _ptr(first),
-          _ptr(ws_s), _ptr(ws_dt), _ptr(out), _code(x, "selective_scan"), inner, ctx.num_seqs,
+    _call("tl_selective_scan", dt_raw, ld(dt_raw), dt_bias, x, ld(x), z, ld(z), bc, ld(bc), a2,
+          skip, st, stride, ctx.state_slots, ctx.q_start, seq, row, first,
+          ws_s, ws_dt, out, _code(x, "selective_scan"), inner, ctx.num_seqs,
           chunks.count if chunks is not None else 0, inner, N, WALK_TOKENS if chunks is not None and chunks.walked else 0, _stream())
     return out
 
@@ -1982,11 +2001,11 @@ def moe_route(logits: torch.Tensor, top: int, weighting: str = "softmax_top", sc
     if weighting == "sigmoid_grouped":
         if not (groups > 0 and E % groups == 0 and 0 < keep <= groups and top <= keep * (E // groups) and groups <= 64):
             raise KernelError(f"moe_route: {E} experts in {groups} groups of which {keep} are kept do not give {top} choices")
-        _call("tl_moe_route_grouped", _ptr(logits), ldl, _ptr(ids), _ptr(weights), T, E, int(top), int(groups), int(keep),
-              _ptr(correction), _stream())
+        _call("tl_moe_route_grouped", logits, ldl, ids, weights, T, E, int(top), int(groups), int(keep),
+              correction, _stream())
         return ids, weights
-    _call("tl_moe_route", _ptr(logits), ldl, _ptr(ids), _ptr(weights), T, E, int(top),
-          ROUTER_WEIGHTINGS[weighting], ctypes.c_float(scale), _stream())
+    _call("tl_moe_route", logits, ldl, ids, weights, T, E, int(top),
+          ROUTER_WEIGHTINGS[weighting], float(scale), _stream())
     return ids, weights
 
 
@@ -2071,17 +2090,17 @@ def _experts_pass(h, ldh, ids, weights, shared, shared_gate, rows, out, gate_up,
     max_tiles = P // BM + E
     order = torch.empty(P, dtype=torch.int32, device=h.device)
     tiles = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=h.device)
-    _call("tl_moe_sort", _ptr(ids), _ptr(order), _ptr(tiles), P, E, BM, _stream())
+    _call("tl_moe_sort", ids, order, tiles, P, E, BM, _stream())
     act = torch.empty(P, F, dtype=h.dtype, device=h.device)
-    _call("tl_moe_gemm", _ptr(h), _code(h, "moe_experts input"), ldh, _ptr(gate_up),
-          _code(gate_up, "moe_experts weights"), _ptr(act), _code(act, "moe_experts"), F, _ptr(order), _ptr(tiles), max_tiles, E, BM,
-          top, F, K, 1 if gated else 2, ctypes.c_float(limit), ctypes.c_float(alpha), ctypes.c_float(shift), _stream())
+    _call("tl_moe_gemm", h, _code(h, "moe_experts input"), ldh, gate_up,
+          _code(gate_up, "moe_experts weights"), act, _code(act, "moe_experts"), F, order, tiles, max_tiles, E, BM,
+          top, F, K, 1 if gated else 2, float(limit), float(alpha), float(shift), _stream())
     y = torch.empty(P, N, dtype=torch.float32, device=h.device) if rows is None else rows
-    _call("tl_moe_gemm", _ptr(act), _code(act, "moe_experts"), F, _ptr(down), _code(down, "moe_experts weights"), _ptr(y), F32, N,
-          _ptr(order), _ptr(tiles), max_tiles, E, BM, top, N, F, 0, ctypes.c_float(0.0), ctypes.c_float(0.0), ctypes.c_float(0.0),
+    _call("tl_moe_gemm", act, _code(act, "moe_experts"), F, down, _code(down, "moe_experts weights"), y, F32, N,
+          order, tiles, max_tiles, E, BM, top, N, F, 0, 0.0, 0.0, 0.0,
           _stream())
     if rows is None:
-        _call("tl_moe_combine", _ptr(y), _ptr(weights), _ptr(shared), _ptr(shared_gate), ldg, _ptr(out), T, N, top, _stream())
+        _call("tl_moe_combine", y, weights, shared, shared_gate, ldg, out, T, N, top, _stream())
 
 
 # ---------------------------------------------------------------------------------------------
@@ -2110,8 +2129,8 @@ def causal_conv(x: torch.Tensor, taps: torch.Tensor, bias: torch.Tensor | None, 
     _check(offset + (K - 1) * C <= state.shape[1], "causal_conv: the kept inputs do not fit the state")
     kept, stride = _state_ptr(state, offset)
     out = torch.empty(T, C, dtype=out_dtype, device=x.device)
-    _call("tl_causal_conv", _ptr(x), x.stride(0) if T > 1 else max(C, x.stride(0)), _ptr(taps), _ptr(bias), kept,
-          ctypes.c_longlong(stride), _ptr(ctx.state_slots), _ptr(ctx.seq_of_token), _ptr(ctx.q_start), _ptr(out),
+    _call("tl_causal_conv", x, x.stride(0) if T > 1 else max(C, x.stride(0)), taps, bias, kept,
+          stride, ctx.state_slots, ctx.seq_of_token, ctx.q_start, out,
           _code(out, "causal_conv out"), C, T, ctx.num_seqs, C, K, 1 if act == "silu" else 0,
           2 if ctx.facts.decode_only and T == ctx.num_seqs else 1, _stream())
     return out
@@ -2142,9 +2161,9 @@ def gated_scan(gates: torch.Tensor, bias_r: torch.Tensor | None, bias_i: torch.T
     st, stride = _state_ptr(state, offset)
     out = torch.empty(T, W, dtype=out_dtype, device=u.device)
     ld = lambda t: t.stride(0) if T > 1 else max(W, t.stride(0))
-    _call("tl_gated_scan", _ptr(gates), ctypes.c_void_p(gates.data_ptr() + 4 * bw), 2 * W, _ptr(bias_r), _ptr(bias_i), _ptr(u),
-          ld(u), _ptr(y), ld(y), _ptr(lam), ctypes.c_float(c), st, ctypes.c_longlong(stride), _ptr(ctx.state_slots),
-          _ptr(ctx.q_start), _ptr(out), _code(out, "gated_scan out"), W, ctx.num_seqs, W, bw, 2 * bw, _stream())
+    _call("tl_gated_scan", gates, gates.data_ptr() + 4 * bw, 2 * W, bias_r, bias_i, u,
+          ld(u), y, ld(y), lam, float(c), st, stride, ctx.state_slots,
+          ctx.q_start, out, _code(out, "gated_scan out"), W, ctx.num_seqs, W, bw, 2 * bw, _stream())
     return out
 
 
@@ -2172,8 +2191,8 @@ def qk_norm_store(proj: torch.Tensor, pos: torch.Tensor, q_weight: torch.Tensor 
         _f32(q_weight, "qk_norm_store q weight", heads * dim)
         _f32(k_weight, "qk_norm_store k weight", kv_heads * dim)
     q = torch.empty(T, heads * D, dtype=out_dtype, device=proj.device)
-    _call("tl_qk_norm_store", _ptr(proj), proj.stride(0) if T > 1 else proj.shape[1], _ptr(pos), _ptr(q_weight), _ptr(k_weight),
-          ctypes.c_float(eps), ctypes.c_float(temp_coef), int(temp_every), _ptr(slots), _ptr(q), _ptr(k_cache), _ptr(v_cache),
+    _call("tl_qk_norm_store", proj, proj.stride(0) if T > 1 else proj.shape[1], pos, q_weight, k_weight,
+          float(eps), float(temp_coef), int(temp_every), slots, q, k_cache, v_cache,
           _code(q, "qk_norm_store"), T, heads, kv_heads, dim, vdim, D, page, _stream())
     return q
 
@@ -2219,11 +2238,11 @@ def head_norm_rotate_store(proj: torch.Tensor, pos: torch.Tensor, q_weight: torc
                and tuple(first_values.shape) == (T, kv_heads * vdim), "head_norm_rotate_store: the values mixed in must be float32 [T, kv_heads * vdim]")
         ldf = first_values.stride(0) if T > 1 else max(first_values.shape[1], first_values.stride(0))
     q = torch.empty(T, heads * D, dtype=out_dtype, device=proj.device)
-    _call("tl_head_norm_rotate_store", _ptr(proj), proj.stride(0) if T > 1 else proj.shape[1], _ptr(pos), _ptr(q_weight),
-          _ptr(k_weight), ctypes.c_float(eps), _ptr(freq), ctypes.c_float(mag), rot, _ptr(slots), _ptr(q), _ptr(k_cache),
-          _ptr(v_cache), _code(q, "head_norm_rotate_store"), T, heads, kv_heads, dim, vdim, D, page,
+    _call("tl_head_norm_rotate_store", proj, proj.stride(0) if T > 1 else proj.shape[1], pos, q_weight,
+          k_weight, float(eps), freq, float(mag), rot, slots, q, k_cache,
+          v_cache, _code(q, "head_norm_rotate_store"), T, heads, kv_heads, dim, vdim, D, page,
           1 if values_from_keys else 0, 1 if q_weight is not None else 2 if plain_norm else 0, 1 if halves else 0,
-          _ptr(first_values), ldf, ctypes.c_float(mix), _stream())
+          first_values, ldf, float(mix), _stream())
     return q
 
 
@@ -2271,10 +2290,10 @@ def conv_rotate_store(proj: torch.Tensor, taps: torch.Tensor, ctx, state: torch.
     q = torch.empty(T, heads * head_size, dtype=out_dtype, device=proj.device)
     kept, stride = _state_ptr(state, offset)
     one_launch = ctx.facts.decode_only and T == ctx.num_seqs and (rot == 0 or dim % 2 == 0)
-    _call("tl_conv_rotate_store", _ptr(proj), proj.stride(0) if T > 1 else max(C, proj.stride(0)), _ptr(taps), kept,
-          ctypes.c_longlong(stride), _ptr(ctx.state_slots), _ptr(ctx.seq_of_token), _ptr(ctx.q_start), _ptr(ctx.pos), _ptr(freq),
-          ctypes.c_float(mag), rot, _ptr(slots) if k_heads else _ptr(None), _ptr(q), _ptr(k_cache) if k_heads else _ptr(None),
-          _ptr(v_cache) if k_heads else _ptr(None), _code(q, "conv_rotate_store"), T, ctx.num_seqs, heads, k_heads, dim, v_heads,
+    _call("tl_conv_rotate_store", proj, proj.stride(0) if T > 1 else max(C, proj.stride(0)), taps, kept,
+          stride, ctx.state_slots, ctx.seq_of_token, ctx.q_start, ctx.pos, freq,
+          float(mag), rot, slots if k_heads else None, q, k_cache if k_heads else None,
+          v_cache if k_heads else None, _code(q, "conv_rotate_store"), T, ctx.num_seqs, heads, k_heads, dim, v_heads,
           vdim, head_size, max(v_repeat, 1), page, K, 2 if one_launch else 1, _stream())
     return q
 
@@ -2290,6 +2309,6 @@ def diff_combine(a: torch.Tensor, heads: int, kv_heads: int, vdim: int, head_siz
     _check(a.dim() == 2 and a.stride(1) == 1 and a.shape[1] == 2 * heads * head_size and heads % kv_heads == 0 and vdim <= head_size,
            "diff_combine: bad shapes")
     out = torch.empty(T, heads * vdim, dtype=a.dtype, device=a.device)
-    _call("tl_diff_combine", _ptr(a), a.stride(0) if T > 1 else a.shape[1], _ptr(out), _code(a, "diff_combine"), T, heads, kv_heads,
-          vdim, head_size, ctypes.c_float(lam), ctypes.c_float(eps), ctypes.c_float(post), _stream())
+    _call("tl_diff_combine", a, a.stride(0) if T > 1 else a.shape[1], out, _code(a, "diff_combine"), T, heads, kv_heads,
+          vdim, head_size, float(lam), float(eps), float(post), _stream())
     return out

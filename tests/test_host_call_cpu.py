@@ -1,0 +1,46 @@
+"""How Python's arguments reach a C entry point (csrc/host_call.hip): by a callback of a known signature, on the CPU."""
+import ctypes
+
+import pytest
+import torch
+
+from tensorline_amd.ops import kernels
+
+
+class Pair(ctypes.Structure):
+    _fields_ = [("a", ctypes.c_void_p), ("b", ctypes.c_float)]
+
+
+def enter(kinds, *args):
+    """What a callee with parameters of ``kinds`` is given for ``args``, and the status that comes back."""
+    seen = []
+    c = ctypes.CFUNCTYPE(ctypes.c_int, *kinds)(lambda *a: (seen.extend(a), -7)[1])
+    kernels._entry_point("tl_last_error")            # (loads the module)
+    status = kernels._enter(ctypes.cast(c, ctypes.c_void_p).value, *args)
+    return seen, status
+
+
+def test_arguments_of_every_kind_in_any_order():
+    t, pair = torch.arange(5.0), Pair(3, 0.25)
+    i, q, f, p = ctypes.c_int, ctypes.c_longlong, ctypes.c_float, ctypes.c_void_p
+    kinds = [p, f, q, i, p, f, i, i, q, f, ctypes.c_uint32, i, p, p, f, q, f]
+    args = [t, 0.1, -(1 << 40), -3, None, 2.5, True, ctypes.c_int(-9), ctypes.c_longlong(1 << 50), ctypes.c_float(-1.5),
+            ctypes.c_uint32(0xffffffff), 1 << 31, pair, ctypes.c_void_p(0x7fff12345678), 1e30, t[2:].data_ptr(), -0.0]
+    seen, status = enter(kinds, *args)
+    want = [t.data_ptr(), ctypes.c_float(0.1).value, -(1 << 40), -3, None, 2.5, 1, -9, 1 << 50, -1.5, 0xffffffff, -(1 << 31),
+            ctypes.addressof(pair), 0x7fff12345678, ctypes.c_float(1e30).value, t.data_ptr() + 8, 0.0]
+    assert seen == want and status == -7
+
+
+def test_as_many_arguments_as_there_is_room_for():
+    seen, _ = enter([ctypes.c_int] * 56 + [ctypes.c_float] * 8, *range(56), *[k + 0.5 for k in range(8)])
+    assert seen == list(range(56)) + [k + 0.5 for k in range(8)]
+    for args in ([0] * 57, [0.0] * 9):
+        with pytest.raises(TypeError):
+            enter([], *args)
+
+
+@pytest.mark.parametrize("bad", ["text", b"", ctypes.c_double(1.0), [1], object(), (ctypes.c_int * 2)()])
+def test_other_arguments_are_refused(bad):
+    with pytest.raises((TypeError, AttributeError)):
+        enter([ctypes.c_void_p], bad)
