@@ -161,6 +161,24 @@ def test_state_slots():
     m.check()
 
 
+def test_state_of_several_layers_side_by_side():
+    """Layers' state (one-dimensional and not, of two types) shares a row per request: pieces do not meet, start at multiples of 64
+    values, and a slot that is handed out is zero in all of them where the others' stay."""
+    needs = [StateNeed((3,)), None, StateNeed((2, 5)), StateNeed((130,)), StateNeed((7,), "int32")]
+    m = manager([None] * 5, states=needs, max_requests=2)
+    s0, s1 = m.add_request("a"), m.add_request("b")
+    for i, need in enumerate(needs):
+        if need is not None:
+            assert tuple(m.state[i].shape) == (3, *need.shape) and m.state[i].storage_offset() % 64 == 0 and m.state[i][0].is_contiguous()
+            m.state[i].fill_(i + 1)
+    assert all((m.state[i] == i + 1).all() for i, need in enumerate(needs) if need is not None)
+    m.release("a")
+    assert m.add_request("c") == s0
+    for i, need in enumerate(needs):
+        if need is not None:
+            assert (m.state[i][s0] == 0).all() and (m.state[i][s1] == i + 1).all() and (m.state[i][m.scratch_slot] == i + 1).all()
+
+
 def test_prefix_sharing_through_the_manager():
     m = manager([keys_and_values(1, 8)], prefix_caching=True)
     toks = list(range(11))
