@@ -410,11 +410,13 @@ extern "C" int tl_gemm_generic(const void* A, int a_dtype, const void* W, int w_
 }
 
 // A batch of bfloat16 products on v_mfma_f32_16x16x32_bf16 (products exact, sums in float), for the small matrices that are
-// applied per head (a latent's: 192 x 128): a wave has 32 rows of A by 64 of W and takes its fragments straight from memory
+// applied per head (a latent's: 192 x 128): a wave has 32 or 64 rows of A by 64 of W and takes its fragments straight from memory
 // (lane 16 g + c: row c, eight k from 8 g on), the four waves of a work-group the same 64 rows of W, which an L1 then holds.
-// What a head's matrix is read from is L2 (48 KB a head), what bounds it is A and C: 2,048 rows of 32 heads take 28 us for
-// 192 x 128 and 26 for 128 x 192, where the float instruction took 86 and 55 through LDS.  One order of summation per element whatever the rows: k in steps of 32 from 0 up.
+// What a head's matrix is read from is L2 (48 KB a head), what bounds it is A, C and the reading of W by every wave again: 2,048 rows of 32
+// heads take 22 us for 192 x 128 and 19 for 128 x 192 with 64 rows a wave and results by 16 bytes (ROWS), where they took 25 and 24 with 32 rows and
+// two bytes (200 rows of 16 times 1,024 x 1,024 46 -> 31), and 86 and 55 on the float instruction through LDS.  One order of summation per element whatever the rows: k in steps of 32 from 0 up.
 typedef __bf16 gg_bf16x8 __attribute__((ext_vector_type(8)));
+template <int MB, bool ROWS>
 __global__ __launch_bounds__(GG_THREADS) void gemm_batched_bf16_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                                       bf16_t* __restrict__ C, int M, int N, int K, int lda, int ldc,
                                                                       long long a_bs, long long w_bs, long long c_bs) {
@@ -422,49 +424,63 @@ __global__ __launch_bounds__(GG_THREADS) void gemm_batched_bf16_kernel(const bf1
     W += (size_t)blockIdx.z * w_bs;
     C += (size_t)blockIdx.z * c_bs;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
-    const int m0 = (blockIdx.y * 4 + wave) * 32, n0 = blockIdx.x * 64;
+    const int m0 = (blockIdx.y * 4 + wave) * 16 * MB, n0 = blockIdx.x * 64;
     if (m0 >= M) return;
-    const bf16_t* ap[2];
+    const bf16_t* ap[MB];
     const bf16_t* wp[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) ap[i] = A + (size_t)min(m0 + i * 16 + c, M - 1) * lda + 8 * g;    // a row that is not there: the
+    for (int i = 0; i < MB; ++i) ap[i] = A + (size_t)min(m0 + i * 16 + c, M - 1) * lda + 8 * g;    // a row that is not there: the
 #pragma unroll
-    for (int j = 0; j < 4; ++j) wp[j] = W + (size_t)min(n0 + j * 16 + c, N - 1) * K + 8 * g;      // last one, not written back
-    gg_f32x4 acc[2][4];
+    for (int j = 0; j < 4; ++j) wp[j] = W + (size_t)min(n0 + (ROWS ? (c >> 2) * 16 + j * 4 + (c & 3) : j * 16 + c), N - 1) * K + 8 * g;   // last one, not written back
+    gg_f32x4 acc[MB][4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = (gg_f32x4){0.f, 0.f, 0.f, 0.f};
     auto step = [&](int k0, bool here) {
-        uint4 a[2], w[4];
+        uint4 a[MB], w[4];
         const uint4 zero = make_uint4(0, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) a[i] = here ? *reinterpret_cast<const uint4*>(ap[i] + k0) : zero;
+        for (int i = 0; i < MB; ++i) a[i] = here ? *reinterpret_cast<const uint4*>(ap[i] + k0) : zero;
 #pragma unroll
         for (int j = 0; j < 4; ++j) w[j] = here ? *reinterpret_cast<const uint4*>(wp[j] + k0) : zero;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MB; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gg_bf16x8, a[i]), __builtin_bit_cast(gg_bf16x8, w[j]),
-                                                                    acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gg_bf16x8, ROWS ? w[j] : a[i]),
+                                                                    __builtin_bit_cast(gg_bf16x8, ROWS ? a[i] : w[j]), acc[i][j], 0, 0, 0);
     };
     const int whole = K / 32 * 32;
 #pragma unroll 4
     for (int k0 = 0; k0 < whole; k0 += 32) step(k0, true);
     if (whole < K) step(whole, whole + 8 * g < K);           // K is a multiple of eight: a lane's piece is there or not
+    if constexpr (ROWS) {              // a lane has row c of a block of rows and the sixteen columns from n0 + 16 g on, four of each block j
+        const int n = n0 + 16 * g;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MB; ++i) {
+            const int m = m0 + i * 16 + c;
+            if (m >= M || n >= N) continue;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int m = m0 + i * 16 + 4 * g + v;
-            if (m >= M) continue;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int n = n0 + j * 16 + c;
-                if (n < N) C[(size_t)m * ldc + n] = tl_from_float<bf16_t>(acc[i][j][v]);
-            }
+            for (int j = 0; j < 4; j += 2)
+                *reinterpret_cast<uint4*>(C + (size_t)m * ldc + n + 4 * j) =
+                    make_uint4(tl_pack_bf16(acc[i][j][0], acc[i][j][1]), tl_pack_bf16(acc[i][j][2], acc[i][j][3]),
+                               tl_pack_bf16(acc[i][j + 1][0], acc[i][j + 1][1]), tl_pack_bf16(acc[i][j + 1][2], acc[i][j + 1][3]));
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int m = m0 + i * 16 + 4 * g + v;
+                if (m >= M) continue;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int n = n0 + j * 16 + c;
+                    if (n < N) C[(size_t)m * ldc + n] = tl_from_float<bf16_t>(acc[i][j][v]);
+                }
+            }
+    }
 }
 
 // `batch` products of the same shape in one launch: product b reads A + b * a_bs (row stride lda),
@@ -485,8 +501,17 @@ extern "C" int tl_gemm_generic_batched(const void* A, int a_dtype, const void* W
     // 5.4, x 448 7.3 and 7.1, x 512 7.4 and 7.7, x 640 7.6 and 8.8, 64 x 1,024 7.7 and 12.2.
     if (a_dtype == TL_BF16 && w_dtype == TL_BF16 && c_dtype == TL_BF16 && K % 8 == 0 && K <= (M <= 16 ? 512 : 1024) && lda % 8 == 0 && a_bs % 8 == 0 &&
         w_bs % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && tl_ceil_div(M, 128) <= 65535) {
-        hipLaunchKernelGGL(gemm_batched_bf16_kernel, dim3(tl_ceil_div(N, 64), tl_ceil_div(M, 128), batch), dim3(GG_THREADS), 0, stream,
-                           (const bf16_t*)A, (const bf16_t*)W, (bf16_t*)C, M, N, K, lda, ldc, a_bs, w_bs, c_bs);
+        // whole aligned sixteens of columns; and 64 rows a wave where that leaves enough waves, which a short K needs more of (600 rows of 32
+        // heads of 192 x 128 10.0 and 11.9 us with 32 and 64 rows a wave, 2,048 23.5 and 22.1; 900 of 128 x 192 12.8 and 9.6)
+        const bool rows = N % 16 == 0 && (uintptr_t)C % 16 == 0 && ldc % 8 == 0 && c_bs % 8 == 0;
+        const bool tall = rows && (double)tl_ceil_div(N, 64) * tl_ceil_div(M, 256) * batch >= (K >= 192 ? 256 : 512);
+#define GO(MB, ROWS)                                                                                                                  \
+    hipLaunchKernelGGL((gemm_batched_bf16_kernel<MB, ROWS>), dim3(tl_ceil_div(N, 64), tl_ceil_div(M, 64 * MB), batch), dim3(GG_THREADS), 0, \
+                       stream, (const bf16_t*)A, (const bf16_t*)W, (bf16_t*)C, M, N, K, lda, ldc, a_bs, w_bs, c_bs)
+        if (tall) GO(4, true);
+        else if (rows) GO(2, true);
+        else GO(2, false);
+#undef GO
         TL_CHECK_LAUNCH("tl_gemm_generic_batched");
         return 0;
     }

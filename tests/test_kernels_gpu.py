@@ -1664,6 +1664,49 @@ def test_batched_linear_bfloat16(T, B, N, Kd):
         assert bool((wide[:, :, [0, 1, N + 2]] == 7.0).all())
 
 
+@pytest.mark.parametrize("T,B,N,Kd", [(1, 2, 16, 8), (31, 3, 48, 40), (33, 2, 192, 128), (130, 1, 112, 96), (2049, 32, 128, 192), (257, 32, 272, 192),
+                                      (1300, 43, 128, 128)])
+def test_batched_linear_by_whole_rows_and_not(T, B, N, Kd):
+    """Results that are whole aligned sixteens of columns are stored by 16 bytes, from 64 rows a wave where there are many: the same
+    bits as through a result that is not aligned, and within a float sum of the product in 64 bits; nothing beside them is written."""
+    torch.manual_seed(T + N)
+    w, a = torch.randn(B, N, Kd, device=DEV).to(torch.bfloat16), torch.randn(T, B, Kd, device=DEV).to(torch.bfloat16)
+    wide = [torch.full((T, B, N + pad), 7.0, dtype=torch.bfloat16, device=DEV) for pad in (16, 3)]
+    got, other = K().batched_linear(a, w, wide[0][:, :, 8:N + 8]), K().batched_linear(a, w, wide[1][:, :, 2:N + 2])
+    assert torch.equal(got, other)
+    for b in {0, B - 1}:
+        want, size = a[:, b].double() @ w[b].double().T, a[:, b].double().abs() @ w[b].double().abs().T
+        assert bool(((got[:, b].double() - want).abs() <= 2.0 ** -8 * want.abs() + (Kd + 8) * 2.0 ** -24 * size).all())
+    assert bool((wide[0][:, :, :8] == 7.0).all()) and bool((wide[0][:, :, N + 8:] == 7.0).all()) and bool((wide[1][:, :, [0, 1, N + 2]] == 7.0).all())
+
+
+@pytest.mark.parametrize("W,skew", [(4, 0), (1020, 0), (1024, 1), (1028, 0), (2050, 0), (2048, 0)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_token_shift_by_quads_and_not(W, skew, dtype):
+    """Rows of whole aligned quads and others: the formula in float, a sequence's first row against what its slot keeps, which its last row
+    becomes."""
+    import types
+    torch.manual_seed(W)
+    dt, lens = getattr(torch, dtype), [3, 1, 7]
+    T, starts = sum(lens), [0, 3, 4, 11]
+    h = torch.randn(T * W + skew, device=DEV).to(dt)[skew:].view(T, W)
+    mu = torch.randn(5, W, device=DEV)
+    slots = [2, 0, 1]
+    dev = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    ctx = types.SimpleNamespace(num_tokens=T, num_seqs=3, seq_of_token=dev([0] * 3 + [1] + [2] * 7), q_start=dev(starts), state_slots=dev(slots))
+    state = torch.randn(4, W + 9, device=DEV)
+    before = torch.empty(T, W, device=DEV)
+    before[1:] = h[:-1].float()
+    for s in range(3):
+        before[starts[s]] = state[slots[s], 5:5 + W]
+    want = torch.stack([(h.float() + (before - h.float()) * mu[m]).to(dt) for m in range(5)])
+    want_state = state.clone()
+    for s in range(3):
+        want_state[slots[s], 5:5 + W] = h[starts[s + 1] - 1].float()
+    got = K().token_shift(h, mu, ctx, state, 5)
+    assert torch.equal(got, want) and torch.equal(state, want_state)
+
+
 @pytest.mark.parametrize("nq,nkv,d,bs,lens,q_lens,kw", [
     (12, 2, 128, 16, [3200, 40, 1, 300, 129], [70, 40, 1, 1, 129], {}),                 # behind a long context, beside one-token requests
     (12, 2, 128, 16, [3200, 40], [70, 40], dict(pads=3)),                               # beside padding sequences
