@@ -383,20 +383,29 @@ def add_rmsnorm(x: torch.Tensor, residual: "torch.Tensor | ShareSum | None", wei
     return out
 
 
+def _ordered(weight: torch.Tensor, step: int) -> torch.Tensor:
+    """[N, K] as [ceil(N/16), ceil(K/step), 4, 16, step/4], zero where it pads; a quarter of a step is 16 bytes."""
+    N, K = weight.shape
+    if weight.is_cuda and weight.is_contiguous() and N > 0 and K > 0 and K % (step // 4) == 0 and weight.data_ptr() % 16 == 0:
+        out = torch.empty(-(-N // 16), -(-K // step), 4, 16, step // 4, dtype=weight.dtype, device=weight.device)
+        _call("tl_order_weight", weight, out, N, K // (step // 4), _stream())
+        return out
+    Np, Kp = -(-N // 16) * 16, -(-K // step) * step
+    if (Np, Kp) != (N, K):
+        padded = torch.zeros(Np, Kp, dtype=weight.dtype, device=weight.device)
+        padded[:N, :K] = weight
+    else:
+        padded = weight
+    return padded.view(Np // 16, 16, Kp // step, 4, step // 4).permute(0, 2, 3, 1, 4).contiguous()
+
+
 def shuffle_weight(weight: torch.Tensor) -> torch.Tensor | None:
     """The copy of a bfloat16 [N, K] matrix that the few-row kernel streams: [ceil(N/16) tiles,
     ceil(K/32) chunks, 64 lanes, 8 values], lane 16*g + r holding row r of the tile at k = 32*chunk +
     8*g .. +8, zero where it pads.  None for matrices that kernel does not take."""
     if weight.dtype != torch.bfloat16 or weight.dim() != 2 or weight.shape[1] % 8:
         return None
-    N, K = weight.shape
-    Np, Kp = -(-N // 16) * 16, -(-K // 32) * 32
-    if (Np, Kp) != (N, K):
-        padded = torch.zeros(Np, Kp, dtype=weight.dtype, device=weight.device)
-        padded[:N, :K] = weight
-    else:
-        padded = weight
-    return padded.view(Np // 16, 16, Kp // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+    return _ordered(weight, 32)
 
 
 def shuffle_weight_float(weight: torch.Tensor) -> torch.Tensor | None:
@@ -406,19 +415,12 @@ def shuffle_weight_float(weight: torch.Tensor) -> torch.Tensor | None:
     is 1 KB of consecutive memory instead of 16 pieces of 64 bytes.  None for other matrices."""
     if weight.dtype != torch.float32 or weight.dim() != 2:
         return None
-    N, K = weight.shape
-    Np, Kp = -(-N // 16) * 16, -(-K // 16) * 16
-    if (Np, Kp) != (N, K):
-        padded = torch.zeros(Np, Kp, dtype=weight.dtype, device=weight.device)
-        padded[:N, :K] = weight
-    else:
-        padded = weight
-    return padded.view(Np // 16, 16, Kp // 16, 4, 4).permute(0, 2, 3, 1, 4).contiguous()
+    return _ordered(weight, 16)
 
 
 def weight_ranges(shuffled: torch.Tensor | None, N: int, K: int) -> torch.Tensor | None:
     """What the float product of more than 16 rows has to know of an [N, K] matrix ahead of it, from its copy by
-    :func:`shuffle_weight_float`: 8 bytes per row and 2,048 values (its largest value's exponent and its norm, gemm_float.hip).  One pass
+    :func:`shuffle_weight_float`: 4 bytes per row and 2,048 values (the power of two that its largest is multiplied by, gemm_float.hip).  One pass
     over the copy; a product that is not given them makes them itself.  None for a copy that is no float one, or not on the GPU."""
     if shuffled is None or shuffled.dtype != torch.float32 or not shuffled.is_cuda:
         return None
@@ -427,6 +429,19 @@ def weight_ranges(shuffled: torch.Tensor | None, N: int, K: int) -> torch.Tensor
     out = torch.empty(library().tl_gemm_float_ranges_size(N, K), dtype=torch.int32, device=shuffled.device)
     _call("tl_gemm_float_ranges", shuffled, out, N, K, _stream())
     return out
+
+
+def shuffle_weight_float_and_ranges(weight: torch.Tensor) -> tuple[torch.Tensor | None, torch.Tensor | None]:
+    """:func:`shuffle_weight_float` and :func:`weight_ranges` of it, in one pass over a matrix that is on the GPU, contiguous and aligned."""
+    if not (weight.is_cuda and weight.dtype == torch.float32 and weight.dim() == 2 and weight.is_contiguous() and weight.numel() > 0
+            and weight.shape[1] % 4 == 0 and weight.data_ptr() % 16 == 0):
+        shuffled = shuffle_weight_float(weight)
+        return shuffled, weight_ranges(shuffled, *weight.shape[:2])
+    N, K = weight.shape
+    shuffled = torch.empty(-(-N // 16), -(-K // 16), 4, 16, 4, dtype=torch.float32, device=weight.device)
+    ranges = torch.empty(library().tl_gemm_float_ranges_size(N, K), dtype=torch.int32, device=weight.device)
+    _call("tl_gemm_float_order", weight, shuffled, ranges, N, K, _stream())
+    return shuffled, ranges
 
 
 def _check_shuffled(shuffled: torch.Tensor, N: int, K: int) -> None:

@@ -87,8 +87,7 @@ class Linear:
         many-row products read that copy, the others hand the row-major one to the library: twice the
         bytes, for which 288 GB of HBM has room."""
         self.shuffled = kernels.shuffle_weight(self.weight)
-        self.shuffled_float = kernels.shuffle_weight_float(self.weight)
-        self.ranges = kernels.weight_ranges(self.shuffled_float, *self.weight.shape)
+        self.shuffled_float, self.ranges = kernels.shuffle_weight_float_and_ranges(self.weight)
         return self
 
     def tensors_kept(self) -> list[torch.Tensor]:

@@ -1664,6 +1664,23 @@ def test_batched_linear_bfloat16(T, B, N, Kd):
         assert bool((wide[:, :, [0, 1, N + 2]] == 7.0).all())
 
 
+@pytest.mark.parametrize("N,Kd", [(1, 8), (16, 32), (17, 40), (33, 520), (48, 512), (100, 1032), (40, 4104), (16 * 65535 + 5, 8)])
+@pytest.mark.parametrize("dtype,step", [("bfloat16", 32), ("float32", 16)])
+def test_ordered_copy_of_a_matrix(N, Kd, dtype, step):
+    """The matrix-core ordered copy, made on the GPU or (rows that are not contiguous) by torch: the definition, zeros where it pads."""
+    w = torch.randn(N, Kd, device=DEV).to(getattr(torch, dtype))
+    make = K().shuffle_weight if dtype == "bfloat16" else K().shuffle_weight_float
+    padded = torch.zeros(-(-N // 16) * 16, -(-Kd // step) * step, dtype=w.dtype, device=DEV)
+    padded[:N, :Kd] = w
+    want = padded.view(-1, 16, padded.shape[1] // step, 4, step // 4).permute(0, 2, 3, 1, 4)
+    assert torch.equal(make(w), want)
+    assert torch.equal(make(torch.cat([w, w], 1)[:, :Kd]), want)
+    if dtype == "float32":
+        w[N // 2].zero_()
+        sh, ranges = K().shuffle_weight_float_and_ranges(w)
+        assert torch.equal(sh, make(w)) and torch.equal(ranges, K().weight_ranges(sh, N, Kd))
+
+
 @pytest.mark.parametrize("T,B,N,Kd", [(1, 2, 16, 8), (31, 3, 48, 40), (33, 2, 192, 128), (130, 1, 112, 96), (2049, 32, 128, 192), (257, 32, 272, 192),
                                       (1300, 43, 128, 128)])
 def test_batched_linear_by_whole_rows_and_not(T, B, N, Kd):
