@@ -1,56 +1,52 @@
-// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float for more than 16 rows, on the half-precision matrix
-// instruction (v_mfma_f32_32x32x16_f16): the 32-bit path's product of prompts and large batches.
+// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float for more than 16 rows, on the bfloat16 matrix
+// instruction (v_mfma_f32_32x32x16_bf16): the 32-bit path's product of prompts and large batches.
 //
-// A float is the sum of two halves of 11 significant bits, each rounded to nearest, the second the rest of the first (splitting floats
-// into shorter ones so that products are exact is Dekker's, Numerische Mathematik 18, 1971): 22 to 23 bits with the second one's
-// sign, off by 4e-8 of the float in the mean.  Halves reach from 2^-24 to 2^16, so the values of a segment of a row (FS_SEG k) are
-// multiplied by a power of two that brings its largest into [2^14, 2^15), which comes out again of the segment's sum.  Of the four
-// partial products the three with a first part in them are taken, small ones first, each exact; the one left out comes to 2^-22 of the
-// product at most, 4e-8 in the mean.  What the result is off the exact one, 2-norm, 256 rows, here / three bfloat16 parts and six products
-// on v_mfma_f32_32x32x16_bf16, as it was before / v_mfma_f32_16x16x4_f32, in 1e-7:
-//                                    K = 64              128                 896                 3,584               18,944
-//   normal numbers                   1.13 1.09 1.44      1.44 1.64 2.05      3.36 4.52 5.36      4.79 6.67 10.7      5.24 7.61 24.5
-//   positive (uniform in [0, 1))     0.65 0.83 1.14      0.92 1.24 1.58      2.57 2.93 4.20      2.66 2.75 8.43      1.42 1.43 20.8
-//   one column 3,000 times the rest  1.35 1.06 1.64      1.64 1.51 2.34      3.87 3.88 6.16      4.61 4.57 12.3      6.74 6.85 28.3
-//   fifth powers of normal numbers   1.22 1.25 1.56      1.53 1.60 2.09      3.43 4.13 5.12      4.81 5.80 10.2      5.24 6.49 23.1
-// Half the products are half the roundings of the sums, which is more than the parts lose from K = 896 on.  Products of a K below
-// 64 go to the float instruction.
+// A float times 2^24 is exactly the sum of three bfloat16 numbers (8 + 8 + 8 significant bits; each is the rest of the
+// one before, rounded to nearest, so the rests have either sign; splitting floats into shorter ones so that products
+// are exact is Dekker's, Numerische Mathematik 18, 1971).  The factor keeps the last part of the smallest
+// float a normal bfloat16: without it floats below 2^-110 lost their rests (4.6e-4 of a value of 1e-37).  It comes out
+// again as 2^-48 of a segment's sum, and costs 1 to 3% (2,048 rows of 37,888 x 3,584: 2.79 ms against 2.75).
 //
-// Values below 2^-18 of their segment's largest lose bits of the second half: it is off by up to 2^-25 after scaling, 2^-40 of the
-// largest.  Beside the sum of the other products that is nothing, unless those cancel or vanish (a column that is zero where the row
-// is large).  So a result below FS_SMALL sqrt(length of the segment), which is 2^20 times what such values can be off by in the worst
-// case and 2^23 times what they usually are, is computed again from the floats, one at a time: some 2 in 100,000 of normal
-// numbers' products; results of segments that are all zero are not.
+// Of the nine partial products of two such sums the six with a first part in them and the product of the two second parts
+// are taken, small ones first, each exact; the three left out come to at most 2^-24 of the product they
+// belong to (a second part is up to 2^-8 of its float, a third up to 2^-17) and 1e-8 of it on average, and a sum of K
+// products takes roundings of that size at every step whatever the instruction.  What the result is off the exact one,
+// 2-norm, 256 rows, six products here / eight of the nine / v_mfma_f32_16x16x4_f32:
+//                                    K = 16                  896                     3,584                   18,944
+//   normal numbers                   3.4e-8 3.3e-8 7.3e-8    4.6e-7 4.6e-7 5.4e-7    6.7e-7 6.7e-7 1.1e-6    7.6e-7 7.6e-7 2.5e-6
+//   positive (uniform in [0, 1))     3.3e-8 3.3e-8 6.2e-8    2.9e-7 2.9e-7 4.2e-7    2.8e-7 2.8e-7 8.4e-7    1.4e-7 1.4e-7 2.1e-6
+//   one column 3,000 times the rest  5.9e-8 5.9e-8 8.4e-8    3.9e-7 3.9e-7 6.2e-7    4.6e-7 4.6e-7 1.3e-6    6.9e-7 6.9e-7 2.9e-6
+// The two more products cost 20% (gate/up of 2,048 rows 2.74 -> 3.34 ms) and change nothing from K = 16 on; below, where a
+// result is a handful of products, the matrix instruction's own last addition is the error (K = 1: 3.4e-8 with six or eight,
+// 2.6e-8 on the float instruction), and products of a K below 64 go to the float instruction.  Six bfloat16 products take 6 / 16 of the
+// matrix cores' time of one on the float instruction (2.5 PFLOP/s against 157 TFLOP/s).
 //
 // What is split where: the rows of A once, by a pass of its own, into the order in which the product reads
-// them (fs_split_kernel); W, which may be most of the GPU's memory, stays float and is split in registers by the wave that owns its
-// columns, from the matrix-core ordered copy that the few-row product streams as well.  The powers of two of W's rows are asked for
-// beforehand (tl_gemm_float_ranges), once for a matrix that is kept.  A wave owns 32 columns and all the rows of its work-group
-// (up to 256): 40 vector instructions beside 3 matrix instructions per 32 x 32 block and 16 k.
+// them (fs_split_kernel: 4 bytes read and 6 written per value); W, which may be most of the GPU's memory,
+// stays float and is split in registers by the wave that owns its columns, from the matrix-core ordered copy
+// that the few-row product streams as well.  A wave owns 32 or 64 columns and all the rows of its work-group
+// (up to 128): 52 vector instructions per 32 columns beside 6 matrix instructions per 32 x 32 block and 16 k.
 //
-// Per step of 16 k a work-group holds 2 KB of A per 32 rows and 8 KB of W in LDS, in the layout the fragments are read in (a fragment is
-// 1 KB, lane after lane: no bank conflicts), fetched two or three steps ahead by global_load_lds; one barrier per step.  A step's weights are
-// split, and its first rows read, between the products of the step before.
-// What bounds it at thousands of rows: the power that products of random halves take; 2,048 rows of 37,888 x 3,584 1.85 ms (300 TFLOP/s,
-// 0.9 PFLOP/s of half products; three bfloat16 parts 2.80), all ones 1.55, halves that are bfloat16 numbers 1.67.  With W split ahead by a pass of
-// its own and both operands straight from LDS, tiles of 256 x 256, the products alone take 1.53, with the pass and its 0.5 GB of
-// workspace 1.74: not kept.  At a few hundred rows: the chain barrier - reads - products of a step, and rounds that do not come out even (513 rows of
-// 17,920 x 1,536 225 -> 147 us, 256 of 3,584 x 18,944 270 -> 168, 33 of 2,048 x 1,536 43 -> 28).
+// Per step of 16 k a work-group holds 3 KB of A per 32 rows and 2 KB of W per 32 columns of a wave in LDS, in the
+// layout the fragments are read in (a fragment is 1 KB, lane after lane: no bank conflicts), fetched one or two
+// steps ahead by global_load_lds; one barrier per step.  What bounds it: the matrix cores are busy half of the time
+// (200 TFLOP/s are 1.2 PFLOP/s of bfloat16 products), the rest is the splitting of W, which does not overlap with them,
+// and LDS reads (a fragment of A feeds six products of a column block).
 //
 // One output element is summed in one fixed order whatever the number of rows or the tile: k in segments of
-// FS_SEG at absolute k, within a segment steps of 16 upwards with the three partial products of a step in one
+// FS_SEG at absolute k, within a segment steps of 16 upwards with the six partial products of a step in one
 // order, the segments' sums added in ascending order.  Few tiles (few rows of a narrow matrix) are spread
 // over the GPU by segments, whose sums a second kernel adds in the same order.
 //
-// Values that are not finite make the split itself infinity minus infinity, and sums may pass the largest float: an element whose segment does
-// not come out finite is computed again on the float instruction, so infinities, NaN and sums of any size give what they give
-// there.  (A wave takes its blocks of 32 x 32 in turn: 2.5 ms for 2,048 rows of 4,608 x 3,584 with an infinity in every row, 0.4 without.)
+// Values that are not finite, and those of 2^104 and more, which the factor takes past the largest bfloat16, make the
+// split itself infinity minus infinity, and sums of 2^80 and more pass the largest float where the sums themselves do
+// not: an element whose segment does not come out finite is computed again on the float instruction, so infinities,
+// NaN and sums of any size give what they give there.  (A wave takes its blocks of 32 x 32 in
+// turn: 2.5 ms for 2,048 rows of 4,608 x 3,584 with an infinity in every row, 0.4 without.)
 #include "common.h"
 
-#include <type_traits>
-
-typedef _Float16 fs_half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 fs_half2 __attribute__((ext_vector_type(2)));
+typedef __bf16 fs_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 fs_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float fs_f32x2 __attribute__((ext_vector_type(2)));
 typedef float fs_f32x16 __attribute__((ext_vector_type(16)));
 
@@ -60,153 +56,64 @@ typedef float fs_f32x16 __attribute__((ext_vector_type(16)));
 #define FS_WAVES 4
 #define FS_CUS 256
 #define FS_MOST_SUMS (512LL << 18)       // floats at most of the segments' sums (512 MB): beyond, K stays whole
-#define FS_TOP 14                        // a segment's largest value is brought to [2^14, 2^15)
-#define FS_MOST_UP 126                   // by a factor that is a normal float
-#define FS_SMALL 0x1.6ap9f               // times the root of a segment's length: results below are computed again
+#define FS_UP 0x1p24f                    // factor of both operands
+#define FS_DOWN 0x1p-48f
 #define FS_RAW_K 2048                    // at most 32 aligned rows of a K up to this are split where they are used (RAW)
 #define FS_RAW_GROUP 4                   // steps whose weights a wave asks for together
 #define FS_RAW_CHUNK 24                  // steps whose rows are in LDS at a time
 
-// The exponent of a segment's factor; FS_ZERO where all its values are zero.
-#define FS_ZERO 127
-__device__ __forceinline__ int fs_up(float most) {       // (what lies below 2^-112 takes the largest factor)
-    return most == 0.f ? FS_ZERO : min(FS_TOP + 127 - (int)(__float_as_uint(most) >> 23 & 255u), FS_MOST_UP);
-}
-__device__ __forceinline__ float fs_factor(int up) { return __uint_as_float((uint32_t)(up + 127) << 23); }
-
-// over the eight lanes that have a row (lanes 8 r .. 8 r + 7), without trips through LDS
-#define FS_MOVED(V, CTRL) __builtin_amdgcn_update_dpp(0, (int)(V), CTRL, 0xf, 0xf, true)
-__device__ __forceinline__ float fs_group_most(float v) {
-    v = fmaxf(v, __int_as_float(FS_MOVED(__float_as_int(v), 0xB1)));       // quad_perm 1, 0, 3, 2
-    v = fmaxf(v, __int_as_float(FS_MOVED(__float_as_int(v), 0x4E)));       // quad_perm 2, 3, 0, 1
-    return fmaxf(v, __int_as_float(FS_MOVED(__float_as_int(v), 0x141)));   // row_half_mirror
-}
-
-// two floats as two halves, rounded to nearest even, and what is left of each
+// two floats as two bfloat16, rounded to nearest even, and what is left of each
 __device__ __forceinline__ uint32_t fs_take(float& a, float& b) {
     const fs_f32x2 v = {a, b};
-    const fs_half2 h = __builtin_convertvector(v, fs_half2);
-    const uint32_t bits = __builtin_bit_cast(uint32_t, h);
-    // a - h, exact; the compiler makes a conversion and a subtraction of it
-    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel_hi:[1,0,0]" : "+v"(a) : "v"(bits));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(b) : "v"(bits));
-    return bits;
+    const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, fs_bf16x2));
+    a -= __uint_as_float(p << 16);
+    b -= __uint_as_float(p & 0xffff0000u);
+    return p;
 }
-__device__ __forceinline__ uint32_t fs_rest(float a, float b) {
-    const fs_f32x2 v = {a, b};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, fs_half2));
-}
-// floats, their factor applied, as twice as many halves
-__device__ __forceinline__ void fs_split4(float4 x, uint2& hi, uint2& lo) {
+// floats times FS_UP as three times as many bfloat16
+__device__ __forceinline__ void fs_split4(float4 x, uint2& hi, uint2& mid, uint2& lo) {
+    x.x *= FS_UP, x.y *= FS_UP, x.z *= FS_UP, x.w *= FS_UP;
     hi = make_uint2(fs_take(x.x, x.y), fs_take(x.z, x.w));
-    lo = make_uint2(fs_rest(x.x, x.y), fs_rest(x.z, x.w));
+    mid = make_uint2(fs_take(x.x, x.y), fs_take(x.z, x.w));
+    lo = make_uint2(fs_take(x.x, x.y), fs_take(x.z, x.w));
 }
-__device__ __forceinline__ void fs_split8(float4 x, float4 y, uint4& hi, uint4& lo) {
+__device__ __forceinline__ void fs_split8(float4 x, float4 y, uint4& hi, uint4& mid, uint4& lo) {
+    x.x *= FS_UP, x.y *= FS_UP, x.z *= FS_UP, x.w *= FS_UP, y.x *= FS_UP, y.y *= FS_UP, y.z *= FS_UP, y.w *= FS_UP;
     hi = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
-    lo = make_uint4(fs_rest(x.x, x.y), fs_rest(x.z, x.w), fs_rest(y.x, y.y), fs_rest(y.z, y.w));
-}
-__device__ __forceinline__ void fs_times(float4& x, float f) { x.x *= f, x.y *= f, x.z *= f, x.w *= f; }
-__device__ __forceinline__ float fs_most(float4 x) { return fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))); }
-
-// A as the product reads it: [ceil(M/32) blocks][ceil(K/16) steps][2 parts][64 lanes][8 values], lane l the row
-// l % 32 of the block at k = 16 step + 8 (l / 32) .. + 8; zero beyond M and K; and the rows' ranges [segments][32 ceil(M/32)].
-// A work-group per eight rows and segment, whose values wait in registers until their rows' largest is known: a wave has 64 k of
-// each row (every fourth 64), a lane eight.
-#define FS_SPLIT_WAVES 4
-__global__ __launch_bounds__(FS_SPLIT_WAVES * 64) void fs_split_kernel(const float* __restrict__ A, uint4* __restrict__ out,
-                                                                     int* __restrict__ ranges, int M, int K, int lda, int steps,
-                                                                     int vec) {
-    constexpr int EACH = FS_SEG / 64 / FS_SPLIT_WAVES;
-    __shared__ float most_of[FS_SPLIT_WAVES][8];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane >> 3, unit = lane & 7;
-    const int seg = blockIdx.x, row = blockIdx.y * 8 + r, s1 = min((seg + 1) * FS_SEG_STEPS, steps);
-    const int s0 = seg * FS_SEG_STEPS + wave * 4 + (unit >> 1);         // this lane's steps: s0, s0 + 16, ..
-    float4 x[EACH], y[EACH];
-    const float* line = A + (size_t)min(row, M - 1) * lda;
-#pragma unroll
-    for (int i = 0; i < EACH; ++i) {
-        const int k = (s0 + i * 4 * FS_SPLIT_WAVES) * FS_STEP + 8 * (unit & 1);
-        x[i] = y[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (row < M && s0 + i * 4 * FS_SPLIT_WAVES < s1) {
-            const float* p = line + k;
-            if (vec && k + 8 <= K) {
-                x[i] = *reinterpret_cast<const float4*>(p);
-                y[i] = *reinterpret_cast<const float4*>(p + 4);
-            } else {
-                x[i].x = k < K ? p[0] : 0.f;
-                x[i].y = k + 1 < K ? p[1] : 0.f;
-                x[i].z = k + 2 < K ? p[2] : 0.f;
-                x[i].w = k + 3 < K ? p[3] : 0.f;
-                y[i].x = k + 4 < K ? p[4] : 0.f;
-                y[i].y = k + 5 < K ? p[5] : 0.f;
-                y[i].z = k + 6 < K ? p[6] : 0.f;
-                y[i].w = k + 7 < K ? p[7] : 0.f;
-            }
-        }
-    }
-    float most = 0.f;
-#pragma unroll
-    for (int i = 0; i < EACH; ++i) most = fmaxf(most, fmaxf(fs_most(x[i]), fs_most(y[i])));
-    most = fs_group_most(most);
-    if (unit == 0) most_of[wave][r] = most;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < FS_SPLIT_WAVES; ++w) most = fmaxf(most, most_of[w][r]);
-    const int up = fs_up(most);
-    const float f = fs_factor(up);
-    if (threadIdx.x < 64 && unit == 0) ranges[(size_t)seg * gridDim.y * 8 + row] = up;
-    uint4* to = out + (size_t)(row >> 5) * steps * 128 + (unit & 1) * 32 + (row & 31);
-#pragma unroll
-    for (int i = 0; i < EACH; ++i) {
-        fs_times(x[i], f);
-        fs_times(y[i], f);
-        if (s0 + i * 4 * FS_SPLIT_WAVES < s1) {
-            uint4 hi, lo;
-            fs_split8(x[i], y[i], hi, lo);
-            uint4* o = to + (size_t)(s0 + i * 4 * FS_SPLIT_WAVES) * 128;
-            o[0] = hi;
-            o[64] = lo;
-        }
-    }
+    mid = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
+    lo = make_uint4(fs_take(x.x, x.y), fs_take(x.z, x.w), fs_take(y.x, y.y), fs_take(y.z, y.w));
 }
 
-// The ranges of a matrix, [segments][16 ceil(N/16)], from its ordered copy, or (ORDER: from W [N, 4 units], aligned) with that copy, which is then
-// one pass over W and not another one behind it: 37,888 x 3,584 229 us where the copy alone takes 198 and the ranges from it 103.
-// A work-group per 16 rows and segment.
-#define FS_RANGE_WAVES 8
-template <bool ORDER>
-__global__ __launch_bounds__(FS_RANGE_WAVES * 64) void fs_ranges_kernel(const float4* __restrict__ W, float4* __restrict__ Ws, int* __restrict__ ranges,
-                                                                      int N, int units, int tiles, int steps) {
-    constexpr int EACH = FS_SEG_STEPS / FS_RANGE_WAVES;
-    __shared__ float most_of[FS_RANGE_WAVES][16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, tile = blockIdx.x, seg = blockIdx.y;
-    const int s0 = seg * FS_SEG_STEPS + wave, s1 = min((seg + 1) * FS_SEG_STEPS, steps);
-    float4 x[EACH];
-#pragma unroll
-    for (int i = 0; i < EACH; ++i) {
-        const int s = s0 + i * FS_RANGE_WAVES, u = s * 4 + (lane >> 4);
-        x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if constexpr (ORDER) {
-            if (s < s1 && u < units && tile * 16 + r < N) x[i] = W[(size_t)(tile * 16 + r) * units + u];
+// A as the product reads it: [ceil(M/32) blocks][ceil(K/16) steps][3 parts][64 lanes][8 values], lane l the row
+// l % 32 of the block at k = 16 step + 8 (l / 32) .. + 8; zero beyond M and K.  A wave per (block, step).
+__global__ __launch_bounds__(256) void fs_split_kernel(const float* __restrict__ A, uint4* __restrict__ out, int M, int K, int lda,
+                                                       int steps, int vec) {
+    const int lane = threadIdx.x & 63, step = blockIdx.x * 4 + (threadIdx.x >> 6), block = blockIdx.y;
+    if (step >= steps) return;
+    const int row = block * 32 + (lane & 31), k = step * FS_STEP + 8 * (lane >> 5);
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f), y = x;
+    if (row < M) {
+        const float* p = A + (size_t)row * lda + k;
+        if (vec && k + 8 <= K) {
+            x = *reinterpret_cast<const float4*>(p);
+            y = *reinterpret_cast<const float4*>(p + 4);
         } else {
-            if (s < s1) x[i] = Ws[((size_t)tile * steps + s) * 64 + lane];
+            x.x = k < K ? p[0] : 0.f;
+            x.y = k + 1 < K ? p[1] : 0.f;
+            x.z = k + 2 < K ? p[2] : 0.f;
+            x.w = k + 3 < K ? p[3] : 0.f;
+            y.x = k + 4 < K ? p[4] : 0.f;
+            y.y = k + 5 < K ? p[5] : 0.f;
+            y.z = k + 6 < K ? p[6] : 0.f;
+            y.w = k + 7 < K ? p[7] : 0.f;
         }
     }
-    if constexpr (ORDER) {
-#pragma unroll
-        for (int i = 0; i < EACH; ++i)
-            if (s0 + i * FS_RANGE_WAVES < s1) Ws[((size_t)tile * steps + s0 + i * FS_RANGE_WAVES) * 64 + lane] = x[i];
-    }
-    float most = 0.f;
-#pragma unroll
-    for (int i = 0; i < EACH; ++i) most = fmaxf(most, fs_most(x[i]));
-    most = fmaxf(most, __shfl_xor(most, 16));
-    most = fmaxf(most, __shfl_xor(most, 32));
-    if (lane < 16) most_of[wave][r] = most;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < FS_RANGE_WAVES; ++w) most = fmaxf(most, most_of[w][r]);
-    if (threadIdx.x < 16) ranges[((size_t)seg * tiles + tile) * 16 + r] = fs_up(most);
+    uint4 hi, mid, lo;
+    fs_split8(x, y, hi, mid, lo);
+    uint4* o = out + ((size_t)block * steps + step) * 192 + lane;
+    o[0] = hi;
+    o[64] = mid;
+    o[128] = lo;
 }
 
 // tl_load_to_lds, the address made a scalar; waited for where FS_LANDED says so
@@ -217,38 +124,37 @@ __device__ __forceinline__ void fs_load_to_lds(const void* g, void* lds_base) {
 #define FS_LANDED(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory")
 
 #define FS_MUL_ONE(ACC, A_, W_)                                                                                              \
-    ACC = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(fs_half8, A_), __builtin_bit_cast(fs_half8, W_), ACC, 0, 0, 0);
+    ACC = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fs_bf16x8, A_), __builtin_bit_cast(fs_bf16x8, W_), ACC, 0, 0, 0);
 
-// MB blocks of 32 rows, FS_WAVES waves side by side with 32 columns each.  PARTS: blockIdx.y is a segment
+// MB blocks of 32 rows, FS_WAVES waves side by side with NB blocks of 32 columns each.  PARTS: blockIdx.y is a segment
 // of K and C the workspace [segments][M][N]; else the whole K, C holding the sum of the segments so far (a lane reads
 // and writes its own elements only).
 // Work-groups of one XCD (every eighth in the order of their ids) take the row tiles of one column tile in turn, so
 // that W is fetched into an L2 once and the rows are what its work-groups share at a time.
 // RAW (17 to 32 rows, 16-byte aligned, K a multiple of four and one segment): one launch, the rows split by the work-group that
-// uses them.  What bounds such a product is the chain of one element's products, three a step that wait for each other, and ahead of it
-// waits for memory: the rows once for their largest values, and again by chunks.  A wave's eight rows come by whole lines
+// uses them.  What bounds such a product is the chain of one element's products, six a step that wait for each other (0.25 us a
+// step with what lies between), and ahead of it a launch and two waits for memory.  So a wave's eight rows come by whole lines
 // of 128 bytes, a chunk of 24 steps at a time with the next one on its way, and go to LDS as parts once; the weights go from memory to
 // registers, three groups of four steps ahead, and the next step's are split between a step's products, where nothing else would
-// run; a barrier per chunk.  17 and 32 rows, us, parts beforehand / here / three bfloat16 parts: 1,152 x 896 23, 24 / 17, 18 / 17, 18;
-// 2,048 x 1,536 34, 35 / 26, 27 / 26, 27; 17,920 x 1,536 37, 38 / 33, 34 / 32, 33; 9,728 x 896 26, 27 / 21, 22 / 19, 20; 1,024 x 64 9, 10 / 5.5, 5.9 / 4.7,
-// 5.1.  (All chunks' loads at once: slower, 46 us at 17,920 x 1,536.)
-template <int MB, int STAGES, bool PARTS, bool RAW>
-__global__ __launch_bounds__(FS_WAVES * 64, 2) void fs_gemm_kernel(
-    const uint4* __restrict__ As, const int* __restrict__ row_ranges, const float* __restrict__ A, const float* __restrict__ Ws,
-    const int* __restrict__ column_ranges, const float* __restrict__ bias, float* __restrict__ C, int M, int N, int K, int lda, int ldc,
-    int steps) {
+// run; a barrier per chunk.  17 and 32 rows of 1,152 x K, us: parts beforehand / here / the float instruction: K = 64 7.2, 7.9 /
+// 5.3, 5.9 / 4.8, 5.1; 128 8.6, 9.4 / 6.2, 6.8 / 6.4, 6.7; 256 11.7, 12.4 / 8.1, 8.7 / 9.7, 10.1; 896 26, 27 / 18, 19 / 26, 27;
+// 2,048 52, 53 / 35, 36 / 56, 56.  (Waves that fetched and split 16 k at a time between barriers: 64 5.2, 128 7.1, 256 11.1; left to
+// the compiler, the splitting ran ahead of the products: 2,048 40.)
+template <int MB, int NB, int STAGES, bool PARTS, bool RAW>
+__global__ __launch_bounds__(FS_WAVES * 64, MB * NB > 8 ? 1 : 2) void fs_gemm_kernel(
+    const uint4* __restrict__ As, const float* __restrict__ A, const float* __restrict__ Ws, const float* __restrict__ bias,
+    float* __restrict__ C, int M, int N, int K, int lda, int ldc, int steps) {
     extern __shared__ uint4 fs_lds[];
-    __shared__ int raw_ranges[RAW ? 32 : 1];
-    static_assert(!RAW || (MB == 1 && !PARTS), "unsplit rows come in one block, with the whole of a short K");
+    static_assert(!RAW || (MB == 1 && NB == 1 && !PARTS), "unsplit rows come in one block, with the whole of a short K");
     static_assert(FS_RAW_K <= FS_SEG && FS_RAW_CHUNK % (3 * FS_RAW_GROUP) == 0 && FS_RAW_CHUNK % 2 == 0, "RAW: one segment, whole turns of three groups");
-    constexpr int CHUNKS = MB * 2, LA = (CHUNKS + FS_WAVES - 1) / FS_WAVES, LW = 2, STAGE = (CHUNKS + FS_WAVES * LW) * 64;
-    constexpr int BN = FS_WAVES * 32;
+    constexpr int CHUNKS = MB * 3, LA = (CHUNKS + FS_WAVES - 1) / FS_WAVES, LW = NB * 2, STAGE = (CHUNKS + FS_WAVES * LW) * 64;
+    constexpr int BN = FS_WAVES * NB * 32;
     const int blocks = (M + 31) / 32, mtiles = (blocks + MB - 1) / MB, ntiles = (N + BN - 1) / BN;
     const int local = blockIdx.x >> 3;
     const int nt = (local / mtiles) * 8 + (blockIdx.x & 7), mt = local % mtiles;
     if (nt >= ntiles) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b0 = mt * MB, n0 = (nt * FS_WAVES + wave) * 32;
+    const int b0 = mt * MB, n0 = (nt * FS_WAVES + wave) * NB * 32;
     const int first = PARTS ? blockIdx.y * FS_SEG_STEPS : 0;
     const int last = PARTS ? min(first + FS_SEG_STEPS, steps) : steps;
 
@@ -257,7 +163,7 @@ __global__ __launch_bounds__(FS_WAVES * 64, 2) void fs_gemm_kernel(
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
         const int c = min(wave + i * FS_WAVES, CHUNKS - 1);            // a wave without a piece of its own repeats the last one
-        ap[i] = As + ((size_t)min(b0 + c / 2, blocks - 1) * steps + first) * 128 + (c % 2) * 64 + lane;
+        ap[i] = As + ((size_t)min(b0 + c / 3, blocks - 1) * steps + first) * 192 + (c % 3) * 64 + lane;
     }
 #pragma unroll
     for (int j = 0; j < LW; ++j)
@@ -271,21 +177,19 @@ __global__ __launch_bounds__(FS_WAVES * 64, 2) void fs_gemm_kernel(
         for (int j = 0; j < LW; ++j) fs_load_to_lds(wp[j], stage + (CHUNKS + wave * LW + j) * 64);
         if (++ahead < last) {
 #pragma unroll
-            for (int i = 0; i < LA; ++i) ap[i] += 128;
+            for (int i = 0; i < LA; ++i) ap[i] += 192;
 #pragma unroll
             for (int j = 0; j < LW; ++j) wp[j] += 64;
         }
     };
-    // this lane's column's range of the segment of step s; its factor is applied as the weights are split
-    auto column_of = [&](int s) { return column_ranges[(size_t)(s / FS_SEG_STEPS) * ((N + 15) / 16 * 16) + min(n0 + (lane & 31), N - 1)]; };
-    int column = column_of(first);
-    float factor = fs_factor(column);
-    fs_f32x16 acc[MB];
+    fs_f32x16 acc[MB][NB];
     auto clear = [&]() {
 #pragma unroll
         for (int i = 0; i < MB; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     };
     // this lane holds rows 8 (r / 4) + 4 (lane / 32) + r % 4 of a block and one column
     float* out = PARTS ? C + (size_t)blockIdx.y * M * N : C;
@@ -293,86 +197,49 @@ __global__ __launch_bounds__(FS_WAVES * 64, 2) void fs_gemm_kernel(
     const int row0 = b0 * 32 + 4 * (lane >> 5);
     auto store = [&](int s0, int s1) {       // the sums over steps [s0, s1), a segment
         const bool first_seg = s0 == 0, last_seg = s1 == steps;
-        const bool inside = RAW && M == MB * 32 && n0 + 32 <= N;           // no element's place is looked at
-        int row = row0, n = n0 + (lane & 31);
-        asm volatile("" : "+v"(row), "+v"(n));         // addresses and bounds are made here, not kept through the loop over k
-        const int* ranges = RAW ? raw_ranges + row : row_ranges + (size_t)(s0 / FS_SEG_STEPS) * blocks * 32 + row;
-        const float b = !PARTS && bias && last_seg && n < N ? bias[n] : 0.f;
-        // elements to compute again, sixteen bits per block: those that are not finite, and those so small that what the
-        // halves lose of the smallest values could show (but where all of a row or column is zero)
-        const float least = column == FS_ZERO ? 0.f : FS_SMALL * __builtin_amdgcn_sqrtf((float)min(FS_SEG, K - s0 * FS_STEP));
-        uint32_t again[(MB + 1) / 2], small[(MB + 1) / 2];
+        const bool inside = RAW && M == MB * 32 && n0 + NB * 32 <= N;      // no element's place is looked at
+        int row = row0, col = n0 + (lane & 31);
+        asm volatile("" : "+v"(row), "+v"(col));       // addresses and bounds are made here, not kept through the loop over k
+        uint32_t again[(MB * NB + 1) / 2];             // elements to compute again: sixteen bits per block
 #pragma unroll
-        for (int u = 0; u < (MB + 1) / 2; ++u) again[u] = small[u] = 0;
-        int rows[2][16];                               // of a block's rows, asked for a block ahead
-        auto ranges_of = [&](int i) {
+        for (int u = 0; u < (MB * NB + 1) / 2; ++u) again[u] = 0;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) rows[i & 1][r] = ranges[(RAW || b0 + i < blocks ? i : 0) * 32 + 8 * (r >> 2) + (r & 3)];
-        };
-        ranges_of(0);
+        for (int j = 0; j < NB; ++j) {
+            const int n = col + j * 32;
+            const float b = !PARTS && bias && last_seg && n < N ? bias[n] : 0.f;
+            float* o = out + (size_t)row * ld + n;
 #pragma unroll
-        for (int i = 0; i < MB; ++i) {
-            if (!RAW && b0 + i >= blocks) break;
-            if (i + 1 < MB) ranges_of(i + 1);
-            asm volatile("" ::: "memory");
+            for (int i = 0; i < MB; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {              // four rows at a time: a few addresses and sums in registers
-                float* o = out + (size_t)(row + i * 32 + 8 * q) * ld + n;
+                for (int q = 0; q < 4; ++q) {          // four rows at a time: a few addresses and sums in registers
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int up = rows[i & 1][4 * q + r];
-                    const float sum = acc[i][4 * q + r], v = __builtin_amdgcn_ldexpf(sum, -(up + column));
-                    if (inside || (n < N && row + i * 32 + 8 * q + r < M)) {
-                        const bool finite = fabsf(v) < INFINITY, low = finite && fabsf(sum) < least && up != FS_ZERO;
-                        const bool fine = finite && !low;                  // else the sum so far stays where it is
-                        const uint32_t bit = 1u << ((i & 1) * 16 + 4 * q + r);
-                        again[i / 2] |= finite ? 0u : bit;
-                        small[i / 2] |= low ? bit : 0u;
-                        const float so_far = !PARTS && !first_seg ? o[r * ld] : 0.f;
-                        o[r * ld] = fine ? (!PARTS && !first_seg ? so_far + v : v) + b : so_far;
+                    for (int r = 0; r < 4; ++r) {
+                        const float v = acc[i][j][4 * q + r] * FS_DOWN;
+                        if (inside || (n < N && row + i * 32 + 8 * q + r < M)) {
+                            const bool fine = fabsf(v) < INFINITY;         // else the sum so far stays where it is
+                            again[(i * NB + j) / 2] |= fine ? 0u : 1u << (((i * NB + j) & 1) * 16 + 4 * q + r);
+                            const float so_far = !PARTS && !first_seg ? o[r * ld] : 0.f;
+                            o[r * ld] = fine ? (!PARTS && !first_seg ? so_far + v : v) + b : so_far;
+                        }
                     }
+                    o += 8 * ld;
+                    asm volatile("" ::: "memory");
                 }
-                asm volatile("" ::: "memory");
-            }
-        }
-        // the small ones, one at a time: a lane every 64th k
-        for (int i = 0; i < MB; ++i) {
-            uint32_t marks = 0;
-#pragma unroll
-            for (int u = 0; u < (MB + 1) / 2; ++u) marks = i >> 1 == u ? small[u] : marks;
-            marks = marks >> (i & 1) * 16 & 0xffffu;
-            for (uint64_t holders = __ballot(marks != 0); holders; holders = __ballot(marks != 0)) {
-                const int holder = __builtin_ctzll(holders), r = __builtin_ctz(__builtin_amdgcn_readlane((int)marks, holder));
-                const int m = (b0 + i) * 32 + 4 * (holder >> 5) + 8 * (r >> 2) + (r & 3), col = n0 + (holder & 31);
-                const float* a = A + (size_t)m * lda;
-                const float* w = Ws + ((size_t)(col >> 4) * steps * 64 + (col & 15)) * 4;
-                const int end = min(s1 * FS_STEP, K);
-                float v = 0.f;
-#pragma unroll 8
-                for (int k = s0 * FS_STEP + lane; k < end; k += 64)
-                    v = __builtin_fmaf(a[k], w[(size_t)(k >> 4) * 256 + (k >> 2 & 3) * 64 + (k & 3)], v);
-                v = tl_wave_sum(v);
-                if (lane == holder) {
-                    float* o = out + (size_t)m * ld + col;
-                    *o = (!PARTS && !first_seg ? *o + v : v) + b;
-                    marks &= marks - 1;
-                }
-            }
         }
         bool any = false;
 #pragma unroll
-        for (int u = 0; u < (MB + 1) / 2; ++u) any |= again[u] != 0;
+        for (int u = 0; u < (MB * NB + 1) / 2; ++u) any |= again[u] != 0;
         if (!__any(any)) return;
-        // those that are not finite from the values themselves, on the float instruction
-        for (int i = 0; i < MB; ++i) {
+        // the marked elements from the values themselves
+        for (int block = 0; block < MB * NB; ++block) {
             uint32_t marks = 0;
 #pragma unroll
-            for (int u = 0; u < (MB + 1) / 2; ++u) marks = i >> 1 == u ? again[u] : marks;
-            marks = marks >> (i & 1) * 16 & 0xffffu;
+            for (int u = 0; u < (MB * NB + 1) / 2; ++u) marks = block >> 1 == u ? again[u] : marks;
+            marks = marks >> (block & 1) * 16 & 0xffffu;
             if (!__any(marks != 0)) continue;
             int here = lane;
             asm volatile("" : "+v"(here));             // nothing of this is made ahead of the loop over k
-            const int n = n0 + (here & 31), half = here >> 5;
+            const int i = block / NB, n = n0 + block % NB * 32 + (here & 31), half = here >> 5;
             const float* a = A + (size_t)min((b0 + i) * 32 + (here & 31), M - 1) * lda + half;        // rows and columns that
             const float* w = Ws + ((size_t)min(n >> 4, (N + 15) / 16 - 1) * steps * 64 + (n & 15)) * 4 + half;   // are not there: others
             fs_f32x16 sum;
@@ -388,6 +255,7 @@ __global__ __launch_bounds__(FS_WAVES * 64, 2) void fs_gemm_kernel(
 #pragma unroll
                 for (int t = 0; t < 8; ++t) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(av[t], wv[t], sum, 0, 0, 0);
             }
+            const float b = !PARTS && bias && last_seg && n < N ? bias[n] : 0.f;
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 if (marks >> r & 1) {
@@ -411,96 +279,72 @@ __global__ __launch_bounds__(FS_WAVES * 64, 2) void fs_gemm_kernel(
                 to[u][1] = wl[at + 16];
             }
         };
-        // One step's products, each of which waits for the one before; between them the next step's rows are read and its weights split.
-        uint4 x[2], a[2];
-        auto step = [&](const uint4* next_rows, const float4 (&next)[2]) {
-            uint4 b[2];
+        // One step's products, each of which waits for the one before, and between them the splitting of the next step's weights.
+        uint4 x[3];
+        auto step = [&](const uint4* rows_of, const float4 (&next)[2]) {
+            uint4 a[3];
 #pragma unroll
-            for (int p = 0; p < 2; ++p) b[p] = next_rows[p * 64];
+            for (int p = 0; p < 3; ++p) a[p] = rows_of[p * 64];
             float f[8] = {next[0].x, next[0].y, next[0].z, next[0].w, next[1].x, next[1].y, next[1].z, next[1].w};
-            uint32_t y[8];
-            auto take = [&](int t) { y[t] = t < 4 ? fs_take(f[2 * t], f[2 * t + 1]) : fs_rest(f[2 * (t & 3)], f[2 * (t & 3) + 1]); };
+            uint32_t y[12];
+            auto take = [&](int t) { y[t] = fs_take(f[2 * (t & 3)], f[2 * (t & 3) + 1]); };
 #define FS_AMONG(PA, PW, ...)                   \
-    FS_MUL_ONE(acc[0], a[PA], x[PW])            \
+    FS_MUL_ONE(acc[0][0], a[PA], x[PW])         \
     __VA_ARGS__;                                \
     __builtin_amdgcn_sched_barrier(0);
-            FS_AMONG(0, 1, _Pragma("unroll") for (int i = 0; i < 8; ++i) f[i] *= factor; take(0); take(1))
-            FS_AMONG(1, 0, take(2); take(3); take(4))
-            FS_AMONG(0, 0, take(5); take(6); take(7))
+            FS_AMONG(0, 2, _Pragma("unroll") for (int i = 0; i < 8; ++i) f[i] *= FS_UP; take(0))
+            FS_AMONG(2, 0, take(1); take(2))
+            FS_AMONG(1, 1, take(3); take(4))
+            FS_AMONG(0, 1, take(5); take(6))
+            FS_AMONG(1, 0, take(7); take(8))
+            FS_AMONG(0, 0, take(9); take(10); take(11))
 #undef FS_AMONG
 #pragma unroll
-            for (int p = 0; p < 2; ++p) x[p] = make_uint4(y[4 * p], y[4 * p + 1], y[4 * p + 2], y[4 * p + 3]), a[p] = b[p];
+            for (int p = 0; p < 3; ++p) x[p] = make_uint4(y[4 * p], y[4 * p + 1], y[4 * p + 2], y[4 * p + 3]);
         };
-        // (behind a chunk's last step lie rows of the chunk before, or nothing: read and not used)
         auto multiply = [&](float4 (&from)[FS_RAW_GROUP][2], const float4 (&then)[FS_RAW_GROUP][2], int s, int c0) {
-            const uint4* rows_of = fs_lds + (s - c0) * 128 + lane;
+            const uint4* rows_of = fs_lds + (s - c0) * 192 + lane;
 #pragma unroll
             for (int u = 0; u < FS_RAW_GROUP; ++u)
-                if (s + u < steps)
-                    step(rows_of + (s + u - c0 + 1 < FS_RAW_CHUNK && s + u + 1 < steps ? (u + 1) * 128 : 0),
-                         u + 1 < FS_RAW_GROUP ? from[u + 1 < FS_RAW_GROUP ? u + 1 : 0] : then[0]);
+                if (s + u < steps) step(rows_of + u * 192, u + 1 < FS_RAW_GROUP ? from[u + 1 < FS_RAW_GROUP ? u + 1 : 0] : then[0]);
             ask(from, s + 3 * FS_RAW_GROUP);
         };
         // Rows: a wave has eight of them, a lane 16 bytes of one in a line of 128 (two steps), so that no line is asked for twice.
         constexpr int LINES = FS_RAW_CHUNK / 2;
         const int row = wave * 8 + (lane >> 3), unit = 4 * (lane & 7);
         const float* al = A + (size_t)min(row, M - 1) * lda;
-        uint2* part = reinterpret_cast<uint2*>(fs_lds) + ((lane >> 2 & 1) * 128 + (lane >> 1 & 1) * 32 + row) * 2 + (lane & 1);
+        uint2* part = reinterpret_cast<uint2*>(fs_lds) + ((lane >> 2 & 1) * 192 + (lane >> 1 & 1) * 32 + row) * 2 + (lane & 1);
         float4 rows[LINES];
-        auto ask_rows = [&](float4 (&to)[LINES], int c0) {
+        auto ask_rows = [&](int c0) {
 #pragma unroll
             for (int i = 0; i < LINES; ++i)
-                if (c0 + 2 * i < steps) to[i] = *reinterpret_cast<const float4*>(al + min((c0 + 2 * i) * FS_STEP + unit, K - 4));
+                if (c0 + 2 * i < steps) rows[i] = *reinterpret_cast<const float4*>(al + min((c0 + 2 * i) * FS_STEP + unit, K - 4));
         };
-        auto ask_first = [&]() {
 #pragma unroll
-            for (int g = 0; g < 3; ++g) {
+        for (int i = 0; i < LINES; ++i) rows[i] = zero;
+        ask_rows(0);
 #pragma unroll
-                for (int u = 0; u < FS_RAW_GROUP; ++u) w[g][u][0] = w[g][u][1] = zero;
-                ask(w[g], g * FS_RAW_GROUP);
-            }
-        };
-        // the rows' largest values first: the chunks from the last to the first, which stays
-        float most = 0.f;
-        auto most_of = [&](const float4 (&of)[LINES], int c0) {
+        for (int g = 0; g < 3; ++g) {
 #pragma unroll
-            for (int i = 0; i < LINES; ++i)
-                if ((c0 + 2 * i) * FS_STEP + unit < K) most = fmaxf(most, fs_most(of[i]));
-        };
-        for (int c0 = (steps - 1) / FS_RAW_CHUNK * FS_RAW_CHUNK; c0 > 0; c0 -= FS_RAW_CHUNK) {
-            ask_rows(rows, c0);
-            most_of(rows, c0);
+            for (int u = 0; u < FS_RAW_GROUP; ++u) w[g][u][0] = w[g][u][1] = zero;
+            ask(w[g], g * FS_RAW_GROUP);
         }
-        ask_rows(rows, 0);
-        ask_first();
-        most_of(rows, 0);
-        most = fs_group_most(most);
-        const int up = fs_up(most);
-        const float row_factor = fs_factor(up);
-        if ((lane & 7) == 0) raw_ranges[row] = up;       // (behind barriers by the time it is read)
         for (int c0 = 0; c0 < steps; c0 += FS_RAW_CHUNK) {
             const int here = min(steps - c0, FS_RAW_CHUNK);
             if (c0) __syncthreads();                     // every wave has read the rows before
 #pragma unroll
             for (int i = 0; i < LINES; ++i)
                 if (2 * i < here) {
-                    float4 f = (c0 + 2 * i) * FS_STEP + unit < K && row < M ? rows[i] : zero;
-                    fs_times(f, row_factor);
-                    uint2 hi, lo;
-                    fs_split4(f, hi, lo);
-                    uint2* to = part + i * 512;
+                    uint2 hi, mid, lo;
+                    fs_split4((c0 + 2 * i) * FS_STEP + unit < K ? rows[i] : zero, hi, mid, lo);
+                    uint2* to = part + i * 768;
                     to[0] = hi;
-                    to[128] = lo;
+                    to[128] = mid;
+                    to[256] = lo;
                 }
-            if (c0 + FS_RAW_CHUNK < steps) ask_rows(rows, c0 + FS_RAW_CHUNK);
-            if (c0 == 0) {
-                fs_times(w[0][0][0], factor);
-                fs_times(w[0][0][1], factor);
-                fs_split8(w[0][0][0], w[0][0][1], x[0], x[1]);
-            }
+            if (c0 + FS_RAW_CHUNK < steps) ask_rows(c0 + FS_RAW_CHUNK);
+            if (c0 == 0) fs_split8(w[0][0][0], w[0][0][1], x[0], x[1], x[2]);
             __syncthreads();
-#pragma unroll
-            for (int p = 0; p < 2; ++p) a[p] = fs_lds[p * 64 + lane];
             for (int s = c0; s < c0 + here; s += 3 * FS_RAW_GROUP) {
                 multiply(w[0], w[1], s, c0);
                 if (s + FS_RAW_GROUP < c0 + here) multiply(w[1], w[2], s + FS_RAW_GROUP, c0);
@@ -510,88 +354,47 @@ __global__ __launch_bounds__(FS_WAVES * 64, 2) void fs_gemm_kernel(
         store(0, steps);
         return;
     }
-    // A step's weights are split, and its first rows read, while the step before is multiplied; within a step the next rows are read
-    // while some are multiplied, two blocks in turn where there are two, so that a product does not wait for the one before it.
-    constexpr int IB = MB == 1 ? 1 : 2, GROUPS = MB / IB;
     for (int i = 0; i < STAGES - 1; ++i) fetch(i);
-    const int wfrag = (CHUNKS + wave * LW) * 64 + ((lane >> 4) & 1) * 64 + (lane >> 5) * 32 + (lane & 15);
-    auto rows_of = [&](int buf, int g, uint4 (&to)[IB][2]) {
-#pragma unroll
-        for (int b = 0; b < IB; ++b)
-#pragma unroll
-            for (int p = 0; p < 2; ++p) to[b][p] = fs_lds[buf * STAGE + ((g * IB + b) * 2 + p) * 64 + lane];
-    };
-    uint4 a[2][IB][2], w[2][2];
-    FS_LANDED((STAGES - 2) * (LA + LW));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    {
-        float4 x = __builtin_bit_cast(float4, fs_lds[wfrag]), y = __builtin_bit_cast(float4, fs_lds[wfrag + 16]);
-        fs_times(x, factor);
-        fs_times(y, factor);
-        fs_split8(x, y, w[0][0], w[0][1]);
-        rows_of(0, 0, a[0]);
-    }
     int buf = 0;
-    auto step = [&](auto parity, float factor) {       // factor: the next step's
-        constexpr int S = decltype(parity)::value, A0 = GROUPS & 1 ? S : 0;     // which registers the step's first rows are in
-        FS_LANDED((STAGES - 3) * (LA + LW));       // step s + 1 is here; later ones may be on their way
+    const int wfrag = (CHUNKS + wave * LW) * 64 + ((lane >> 4) & 1) * 64 + (lane >> 5) * 32 + (lane & 15);
+    for (int s = first; s < last; ++s) {
+        FS_LANDED((STAGES - 2) * (LA + LW));   // step s is here; later ones may be on their way
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        const int next = buf == STAGES - 1 ? 0 : buf + 1;
-        float4 x = __builtin_bit_cast(float4, fs_lds[next * STAGE + wfrag]), y = __builtin_bit_cast(float4, fs_lds[next * STAGE + wfrag + 16]);
         fetch(buf == 0 ? STAGES - 1 : buf - 1);   // the buffer of step s - 1, which every wave has read
-        float f[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-        uint32_t u[8];
-        auto take = [&](int t) { u[t] = t < 4 ? fs_take(f[2 * t], f[2 * t + 1]) : fs_rest(f[2 * (t & 3)], f[2 * (t & 3) + 1]); };
+        const uint4* stage = fs_lds + buf * STAGE;
+        uint4 w[NB][3];
 #pragma unroll
-        for (int g = 0; g < GROUPS; ++g) {
-            if (g + 1 < GROUPS) rows_of(buf, g + 1, a[(A0 + g + 1) & 1]);
-            else rows_of(next, 0, a[(A0 + g + 1) & 1]);
-            const uint4 (&rows)[IB][2] = a[(A0 + g) & 1];
-#define FS_MUL(T, PA, PW)                                                                                                    \
-    _Pragma("unroll") for (int b = 0; b < IB; ++b) FS_MUL_ONE(acc[g * IB + b], rows[b][PA], w[S][PW])                         \
-    if (g == 0 && T == 0) { _Pragma("unroll") for (int i = 0; i < 8; ++i) f[i] *= factor; }                                   \
-    _Pragma("unroll") for (int t = (g * 3 + T) * 8 / (GROUPS * 3); t < (g * 3 + T + 1) * 8 / (GROUPS * 3); ++t) take(t);       \
-    __builtin_amdgcn_sched_barrier(0);
-            FS_MUL(0, 0, 1)
-            FS_MUL(1, 1, 0)
-            FS_MUL(2, 0, 0)
+        for (int j = 0; j < NB; ++j)
+            fs_split8(__builtin_bit_cast(float4, stage[wfrag + j * 128]), __builtin_bit_cast(float4, stage[wfrag + j * 128 + 16]),
+                      w[j][0], w[j][1], w[j][2]);
+        // two blocks' products in turn, so that none waits for the one before it
+        constexpr int IB = NB > 1 || MB == 1 ? 1 : 2;
+#pragma unroll
+        for (int i = 0; i < MB; i += IB) {
+            uint4 a[IB][3];
+#pragma unroll
+            for (int b = 0; b < IB; ++b)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) a[b][p] = stage[((i + b) * 3 + p) * 64 + lane];
+#define FS_MUL(PA, PW)                                                                                                       \
+    _Pragma("unroll") for (int b = 0; b < IB; ++b) _Pragma("unroll") for (int j = 0; j < NB; ++j) FS_MUL_ONE(acc[i + b][j], a[b][PA], w[j][PW])
+            FS_MUL(0, 2)
+            FS_MUL(2, 0)
+            FS_MUL(1, 1)
+            FS_MUL(0, 1)
+            FS_MUL(1, 0)
+            FS_MUL(0, 0)
 #undef FS_MUL
         }
-#pragma unroll
-        for (int p = 0; p < 2; ++p) w[S ^ 1][p] = make_uint4(u[4 * p], u[4 * p + 1], u[4 * p + 2], u[4 * p + 3]);
-        buf = next;
-    };
-    int s = first;
-    auto steps_to = [&](int end, float then) __attribute__((always_inline)) {          // then: the factor behind them
-        for (; s + 2 <= end; s += 2) {
-            step(std::integral_constant<int, 0>(), factor);
-            step(std::integral_constant<int, 1>(), s + 2 < end ? factor : then);
-        }
-        if (s < end) {                   // (an odd segment is the last)
-            step(std::integral_constant<int, 0>(), factor);
-            ++s;
-        }
-    };
-    if constexpr (PARTS) {
-        steps_to(last, factor);
-        FS_LANDED(0);                    // nothing may land in LDS that is no longer this work-group's
-        store(first, last);
-        return;
-    }
-    while (s < last) {                   // a segment at a time
-        const int s0 = s, s1 = min(s + FS_SEG_STEPS, last), next = s1 < last ? column_of(s1) : column;
-        asm volatile("" ::"v"(next));    // here before the loop, where a wait for it would wait for the steps on their way
-        steps_to(s1, fs_factor(next));
-        if (s == last) FS_LANDED(0);
-        store(s0, s);
-        if (s < last) {
+        if (!PARTS && (s + 1) % FS_SEG_STEPS == 0 && s + 1 < last) {
+            store(s + 1 - FS_SEG_STEPS, s + 1);
             clear();
-            column = next;
-            factor = fs_factor(next);
         }
+        buf = buf == STAGES - 1 ? 0 : buf + 1;
     }
+    FS_LANDED(0);                        // nothing may land in LDS that is no longer this work-group's
+    store(PARTS ? first : (last - 1) / FS_SEG_STEPS * FS_SEG_STEPS, last);
 }
 
 // The segments' sums in ascending order, as the product adds them where it has the whole K.  VEC: four columns a
@@ -617,16 +420,17 @@ __global__ __launch_bounds__(256) void fs_add_kernel(const float* __restrict__ p
     }
 }
 
-// The tiles (row blocks of a wave) as a fitted time: a step of 16 k takes a work-group `alone` us when its CU has nothing else (the
-// chain barrier - reads - products), and a CU gets through one in `shared` us when it holds as many as fit.  The tile, and whether K is
-// dealt out by segments, is the least estimate: 2.8% longer than the best choice in the mean over eleven matrices of 64 to 18,944 k x
-// nineteen row counts, 25% at most (1,700 rows of 3,584 x 3,584).  E.g. at 2,048 rows down (3,584 x 18,944) takes 0.96 ms with K dealt
-// out, 1.46 without; at 40 rows 74 to 86 us and 440 to 920.
+// The tiles (row blocks and column blocks of a wave) with what was measured on the products of 7B and 0.5B models: a step of
+// 16 k takes a work-group `alone` us when its CU has nothing else (the chain barrier - reads - products), and a CU gets
+// through one in `shared` us when it holds as many as fit.  The tile, and whether K is dealt out by segments, is the
+// least estimate; e.g. at 2,048 rows gate/up (37,888 x 3,584) 2.8 ms in tiles of 128 x 256 (200 TFLOP/s; tiles of 256 rows
+// 3.1, of 128 x 128 3.0), down (3,584 x 18,944) 1.55 ms with K dealt out (1.66 against 1.72 when both were tried), where the float
+// instruction takes 4.8 and 2.8; at 40 rows down takes 93 us dealt out (97 against 480).
 struct FsTile {
-    int mb, fit;
+    int mb, nb, fit;
     double alone, shared;
 };
-static const FsTile fs_tiles[] = {{8, 2, 1.30, 0.83}, {4, 2, 0.70, 0.48}, {2, 3, 0.55, 0.25}, {1, 4, 0.29, 0.18}};
+static const FsTile fs_tiles[] = {{4, 2, 2, 1.90, 1.36}, {4, 1, 2, 0.95, 0.71}, {2, 1, 3, 0.56, 0.41}, {1, 1, 4, 0.43, 0.26}};
 
 static int fs_choose(int M, int N, int K, bool* parts) {
     const int blocks = tl_ceil_div(M, 32), steps = tl_ceil_div(K, FS_STEP), nseg = tl_ceil_div(K, FS_SEG);
@@ -635,12 +439,12 @@ static int fs_choose(int M, int N, int K, bool* parts) {
     for (int t = 0; t < 4; ++t) {
         const FsTile& z = fs_tiles[t];
         if (z.mb > 1 && z.mb / 2 >= blocks) continue;                  // half of it holds all the rows
-        const double tiles = (double)tl_ceil_div(blocks, z.mb) * tl_ceil_div(N, FS_WAVES * 32);
+        const double tiles = (double)tl_ceil_div(blocks, z.mb) * tl_ceil_div(N, FS_WAVES * 32 * z.nb);
         for (int cut = 0; cut < (nseg > 1 && nseg <= 65535 && (long long)M * N <= FS_MOST_SUMS / nseg ? 2 : 1); ++cut) {
             const double each = tiles * (cut ? nseg : 1) / FS_CUS, whole = (double)(long long)(each + 0.999999);
             const double on_a_cu = whole < 4 ? whole : each + 0.5, turns = (double)(long long)((whole + z.fit - 1) / z.fit);
             const double step = turns * z.alone > on_a_cu * z.shared ? turns * z.alone : on_a_cu * z.shared;
-            const double us = step * steps / (cut ? nseg : 1) + (cut ? 4.7 + 8.0 * M * N * nseg / 6e6 : 0.0);
+            const double us = step * steps / (cut ? nseg : 1) + (cut ? 4.0 + 8.0 * M * N * nseg / 6e6 : 0.0);
             if (us < cost) cost = us, best = t, *parts = cut != 0;
         }
     }
@@ -672,38 +476,11 @@ extern "C" long long tl_gemm_float_split_workspace(int M, int N, int K) {
     return parts ? (long long)tl_ceil_div(K, FS_SEG) * M * N : 0;
 }
 
-// 32-bit numbers of the ranges of a matrix [N, K], and the ranges from its ordered copy.
-extern "C" long long tl_gemm_float_ranges_size(int N, int K) {
-    return N > 0 && K > 0 ? (long long)tl_ceil_div(K, FS_SEG) * tl_ceil_div(N, 16) * 16 : 0;
-}
-extern "C" int tl_gemm_float_ranges(const float* Ws, void* ranges, int N, int K, hipStream_t stream) {
-    TL_CHECK_ARG(N > 0 && K > 0 && tl_ceil_div(K, FS_SEG) <= 65535, "tl_gemm_float_ranges: bad sizes N=%d K=%d", N, K);
-    TL_CHECK_ARG((uintptr_t)Ws % 16 == 0 && (uintptr_t)ranges % 4 == 0, "tl_gemm_float_ranges: the weight copy must be 16-byte aligned");
-    hipLaunchKernelGGL(fs_ranges_kernel<false>, dim3(tl_ceil_div(N, 16), tl_ceil_div(K, FS_SEG)), dim3(FS_RANGE_WAVES * 64), 0, stream, nullptr,
-                       (float4*)Ws, (int*)ranges, N, 0, tl_ceil_div(N, 16), tl_ceil_div(K, FS_STEP));
-    TL_CHECK_LAUNCH("tl_gemm_float_ranges");
-    return 0;
-}
-// The ordered copy Ws of W [N, K] (contiguous, K a multiple of four), and its ranges.
-extern "C" int tl_gemm_float_order(const float* W, float* Ws, void* ranges, int N, int K, hipStream_t stream) {
-    TL_CHECK_ARG(N > 0 && K > 0 && K % 4 == 0 && tl_ceil_div(K, FS_SEG) <= 65535, "tl_gemm_float_order: bad sizes N=%d K=%d", N, K);
-    TL_CHECK_ARG((uintptr_t)W % 16 == 0 && (uintptr_t)Ws % 16 == 0 && (uintptr_t)ranges % 4 == 0, "tl_gemm_float_order: the matrix and its copy must be 16-byte aligned");
-    hipLaunchKernelGGL(fs_ranges_kernel<true>, dim3(tl_ceil_div(N, 16), tl_ceil_div(K, FS_SEG)), dim3(FS_RANGE_WAVES * 64), 0, stream,
-                       (const float4*)W, (float4*)Ws, (int*)ranges, N, K / 4, tl_ceil_div(N, 16), tl_ceil_div(K, FS_STEP));
-    TL_CHECK_LAUNCH("tl_gemm_float_order");
-    return 0;
-}
-
-// Bytes of `split` for M rows of K.
-extern "C" long long tl_gemm_float_split_bytes(int M, int K) {
-    return M > 0 && K > 0 ? (long long)tl_ceil_div(M, 32) * (tl_ceil_div(K, FS_STEP) * 2048ll + tl_ceil_div(K, FS_SEG) * 128ll) : 0;
-}
-
 // A float [M, K] with row stride lda; Ws float [ceil(N/16), ceil(K/16), 64, 4] (the matrix-core ordered copy of W, zero
-// where it pads); ranges: tl_gemm_float_ranges of it; split: workspace of tl_gemm_float_split_bytes, or null where
+// where it pads); split: workspace of ceil(M/32) * ceil(K/16) * 3 KB, or null where
 // tl_gemm_float_split_takes_rows says that the rows are split where they are used; ws: tl_gemm_float_split_workspace floats.
-extern "C" int tl_gemm_float_split(const float* A, const float* Ws, const void* ranges, const float* bias, float* C, void* split, float* ws,
-                                   int M, int N, int K, int lda, int ldc, hipStream_t stream) {
+extern "C" int tl_gemm_float_split(const float* A, const float* Ws, const float* bias, float* C, void* split, float* ws, int M,
+                                   int N, int K, int lda, int ldc, hipStream_t stream) {
     TL_CHECK_ARG(M >= 0 && N > 0 && K > 0, "tl_gemm_float_split: bad sizes M=%d N=%d K=%d", M, N, K);
     TL_CHECK_ARG(lda >= K && ldc >= N, "tl_gemm_float_split: row strides lda=%d ldc=%d too small for K=%d N=%d", lda, ldc, K, N);
     TL_CHECK_ARG((uintptr_t)Ws % 16 == 0 && (uintptr_t)split % 16 == 0, "tl_gemm_float_split: the weight copy and the workspace must be 16-byte aligned");
@@ -712,34 +489,31 @@ extern "C" int tl_gemm_float_split(const float* A, const float* Ws, const void* 
     TL_CHECK_ARG(blocks <= 65535, "tl_gemm_float_split: %d rows are too many for one launch", M);
     bool parts = false;
     const int tile = fs_choose(M, N, K, &parts);
-    const int mtiles = tl_ceil_div(blocks, fs_tiles[tile].mb), ntiles = tl_ceil_div(N, FS_WAVES * 32);
+    const int mtiles = tl_ceil_div(blocks, fs_tiles[tile].mb), ntiles = tl_ceil_div(N, FS_WAVES * 32 * fs_tiles[tile].nb);
     const long long grid = (long long)mtiles * tl_ceil_div(ntiles, 8) * 8;
     TL_CHECK_ARG(grid < (1ll << 31), "tl_gemm_float_split: M=%d N=%d are too many tiles for one launch", M, N);
     TL_CHECK_ARG(!parts || ws, "tl_gemm_float_split: no workspace for the segments' sums");
     const int vec = ((uintptr_t)A % 16 == 0 && lda % 4 == 0) ? 1 : 0;
     TL_CHECK_ARG(split || (tl_gemm_float_split_takes_rows(M, N, K, lda) && vec && tile == 3 && !parts),
                  "tl_gemm_float_split: M=%d K=%d lda=%d need a workspace for the rows' parts", M, K, lda);
-    TL_CHECK_ARG(ranges && (uintptr_t)ranges % 4 == 0, "tl_gemm_float_split: no ranges of the matrix");
-    int* rows = split ? (int*)((uint4*)split + (size_t)blocks * steps * 128) : nullptr;
     if (split)
-        hipLaunchKernelGGL(fs_split_kernel, dim3(nseg, blocks * 4), dim3(FS_SPLIT_WAVES * 64), 0, stream, A, (uint4*)split, rows, M, K, lda, steps,
-                           vec);
-#define FS_GO(MB, ST, P, RAW, LDS)                                                                                           \
-    hipLaunchKernelGGL((fs_gemm_kernel<MB, ST, P, RAW>), dim3((unsigned)grid, P ? nseg : 1), dim3(FS_WAVES * 64), LDS, stream, \
-                       (const uint4*)split, rows, A, Ws, (const int*)ranges, bias, P ? ws : C, M, N, K, lda, ldc, steps)
-#define FS_GO_P(MB, ST)                                                               \
-    if (parts) FS_GO(MB, ST, true, false, ST * (MB * 2 + FS_WAVES * 2) * 1024); \
-    else FS_GO(MB, ST, false, false, ST * (MB * 2 + FS_WAVES * 2) * 1024)
+        hipLaunchKernelGGL(fs_split_kernel, dim3(tl_ceil_div(steps, 4), blocks), dim3(256), 0, stream, A, (uint4*)split, M, K, lda, steps, vec);
+#define FS_GO(MB, NB, ST, P, RAW, LDS)                                                                                           \
+    hipLaunchKernelGGL((fs_gemm_kernel<MB, NB, ST, P, RAW>), dim3((unsigned)grid, P ? nseg : 1), dim3(FS_WAVES * 64), LDS, stream, \
+                       (const uint4*)split, A, Ws, bias, P ? ws : C, M, N, K, lda, ldc, steps)
+#define FS_GO_P(MB, NB, ST)                                                               \
+    if (parts) FS_GO(MB, NB, ST, true, false, ST * (MB * 3 + FS_WAVES * NB * 2) * 1024); \
+    else FS_GO(MB, NB, ST, false, false, ST * (MB * 3 + FS_WAVES * NB * 2) * 1024)
     if (tile == 0) {
-        FS_GO_P(8, 3);
+        FS_GO_P(4, 2, 2);
     } else if (tile == 1) {
-        FS_GO_P(4, 4);
+        FS_GO_P(4, 1, 3);
     } else if (tile == 2) {
-        FS_GO_P(2, 4);
+        FS_GO_P(2, 1, 3);
     } else if (split) {
-        FS_GO_P(1, 4);
+        FS_GO_P(1, 1, 3);
     } else {
-        FS_GO(1, 1, false, true, (steps < FS_RAW_CHUNK ? (steps + 1) / 2 * 2 : FS_RAW_CHUNK) * 2048);
+        FS_GO(1, 1, 1, false, true, (steps < FS_RAW_CHUNK ? (steps + 1) / 2 * 2 : FS_RAW_CHUNK) * 3072);
     }
 #undef FS_GO_P
 #undef FS_GO

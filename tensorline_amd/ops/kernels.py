@@ -47,8 +47,7 @@ def library() -> ctypes.CDLL:
                 except OSError as e:
                     raise KernelError(f"cannot load the HIP kernel library {path}: {e}") from e
                 lib.tl_last_error.restype = ctypes.c_char_p
-                for name in ("tl_gemm_float_split_workspace", "tl_gemm_float_split_bytes", "tl_gemm_float_ranges_size"):
-                    getattr(lib, name).restype = ctypes.c_longlong
+                lib.tl_gemm_float_split_workspace.restype = ctypes.c_longlong
                 _lib = lib
     return _lib
 
@@ -418,32 +417,6 @@ def shuffle_weight_float(weight: torch.Tensor) -> torch.Tensor | None:
     return _ordered(weight, 16)
 
 
-def weight_ranges(shuffled: torch.Tensor | None, N: int, K: int) -> torch.Tensor | None:
-    """What the float product of more than 16 rows has to know of an [N, K] matrix ahead of it, from its copy by
-    :func:`shuffle_weight_float`: 4 bytes per row and 2,048 values (the power of two that its largest is multiplied by, gemm_float.hip).  One pass
-    over the copy; a product that is not given them makes them itself.  None for a copy that is no float one, or not on the GPU."""
-    if shuffled is None or shuffled.dtype != torch.float32 or not shuffled.is_cuda:
-        return None
-    _check_shuffled(shuffled, N, K)
-    _on_gpu(shuffled)
-    out = torch.empty(library().tl_gemm_float_ranges_size(N, K), dtype=torch.int32, device=shuffled.device)
-    _call("tl_gemm_float_ranges", shuffled, out, N, K, _stream())
-    return out
-
-
-def shuffle_weight_float_and_ranges(weight: torch.Tensor) -> tuple[torch.Tensor | None, torch.Tensor | None]:
-    """:func:`shuffle_weight_float` and :func:`weight_ranges` of it, in one pass over a matrix that is on the GPU, contiguous and aligned."""
-    if not (weight.is_cuda and weight.dtype == torch.float32 and weight.dim() == 2 and weight.is_contiguous() and weight.numel() > 0
-            and weight.shape[1] % 4 == 0 and weight.data_ptr() % 16 == 0):
-        shuffled = shuffle_weight_float(weight)
-        return shuffled, weight_ranges(shuffled, *weight.shape[:2])
-    N, K = weight.shape
-    shuffled = torch.empty(-(-N // 16), -(-K // 16), 4, 16, 4, dtype=torch.float32, device=weight.device)
-    ranges = torch.empty(library().tl_gemm_float_ranges_size(N, K), dtype=torch.int32, device=weight.device)
-    _call("tl_gemm_float_order", weight, shuffled, ranges, N, K, _stream())
-    return shuffled, ranges
-
-
 def _check_shuffled(shuffled: torch.Tensor, N: int, K: int) -> None:
     if shuffled.dtype == torch.float32:
         if not (shuffled.is_contiguous() and tuple(shuffled.shape) == (-(-N // 16), -(-K // 16), 4, 16, 4)):
@@ -538,8 +511,7 @@ def _norm_args(owed: NormedRows | None, sink: NormSink | None, M: int, N: int, d
 def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tensor | None = None,
            out_dtype: torch.dtype | None = None, out: torch.Tensor | None = None,
            shuffled: torch.Tensor | None = None, sink: NormSink | None = None,
-           keep_shares: bool = False, act: str | None = None,
-           ranges: torch.Tensor | None = None) -> "torch.Tensor | NormedRows | ShareSum":
+           keep_shares: bool = False, act: str | None = None) -> "torch.Tensor | NormedRows | ShareSum":
     """``a @ weight.T + bias``: a [M, K] (rows may be strided), weight [N, K], bias float32 [N].
     ``shuffled``: the copy of ``weight`` made by :func:`shuffle_weight`, which few-row bfloat16
     products stream instead of ``weight``.  ``a`` may be :class:`NormedRows` and ``sink`` a
@@ -547,8 +519,7 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
     kernel (:func:`can_defer_norm` rows, a shuffled copy).  ``keep_shares``: the caller takes a
     :class:`ShareSum` where the product is computed in shares of K (many rows, a long K).  ``act`` "relu2":
     the result is ``max(y, 0)^2`` in ``out_dtype``, computed in float32: in the few-row bfloat16 kernel's or the many-row tiles'
-    epilogue where one of them runs the product, by a pass of its own otherwise.  ``ranges``: :func:`weight_ranges` of a float
-    ``shuffled``."""
+    epilogue where one of them runs the product, by a pass of its own otherwise."""
     if act is not None:
         _check(act == "relu2" and not isinstance(a, NormedRows) and sink is None and out is None and not keep_shares,
                "linear: the activation is 'relu2', on a plain product")
@@ -575,7 +546,7 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
             if plan:
                 _on_gpu(a, weight, bias, shuffled)
                 return _tiles(a, shuffled, bias, out_dtype or a.dtype, M, weight.shape[0], K, lda, plan, act=1)
-        return relu_squared(linear(a, weight, bias, out_dtype=torch.float32, shuffled=shuffled, ranges=ranges), out_dtype or a.dtype)
+        return relu_squared(linear(a, weight, bias, out_dtype=torch.float32, shuffled=shuffled), out_dtype or a.dtype)
     owed = a if isinstance(a, NormedRows) else None
     if owed is not None:
         a = owed.rows
@@ -623,7 +594,7 @@ def linear(a: torch.Tensor | NormedRows, weight: torch.Tensor, bias: torch.Tenso
     ldc = out.stride(0) if M > 1 else N
     if shuffled is not None:
         _check_shuffled(shuffled, N, K)
-    return _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled, ranges)
+    return _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled)
 
 
 MAX_KEY_SPLITS = 1024    # key splits the attention merge kernel takes
@@ -633,7 +604,7 @@ FLOAT_DECODE_SPLIT_KEYS = 128   # the same where its float form without LDS tile
 SKINNY_MAX_ROWS = 16     # rows the few-row kernel serves (one 16-row MFMA tile)
 ROWS64_MAX_ROWS = 64     # rows the 17..64-row kernel serves; above that gemm_tiles.hip or the library
 FLOAT_SPLIT_MAX_ROWS = 65535 * 32   # rows one launch of the float product of more than 16 rows takes
-FLOAT_SPLIT_BYTES = 512 << 20   # at six bytes a value; the parts take four: more rows go in several launches
+FLOAT_SPLIT_BYTES = 512 << 20   # at most this much for the parts of a launch's rows: more rows go in several launches
 FLOAT_SPLIT_MIN_K = 64   # below: the float instruction (_float_split)
 
 
@@ -660,29 +631,26 @@ def _few_rows_go_to_rows64(N: int, K: int) -> bool:
     return 2 <= rounds <= 3 and tiles < 0.75 * rounds * 256 and rounds * steps >= 150
 
 
-def _float_split(a, shuffled, ranges, bias, out, M, N, K, lda, ldc):
-    """More than 16 float rows: every float as the sum of two halves on the half-precision matrix instruction,
+def _float_split(a, shuffled, bias, out, M, N, K, lda, ldc):
+    """More than 16 float rows: every float as the sum of three bfloat16 numbers on the bfloat16 matrix instruction,
     the weight from its matrix-core ordered copy.  Every matrix with the copy and a K of 64 or more goes here, whatever its
     rows beyond 16, so that a row's bits do not depend on how many others come along.  Measured, us here and on the float
-    instruction: 33 rows of 1,152 K = 64 8.7 and 8.2, 128 9.6 and 11.5, 896 21 and 51; 128 rows K = 64 8.8 and 16.5, 896 21 and
-    89; 1,000 rows of 9,728 K = 896 90 and 204.  17 and 32 rows: K = 64 5.5, 5.9 and 4.8, 5.1, 128 6.5, 6.6 and 6.4, 6.7, 896 17, 18
-    and 26, 27: below K = 128 they pay up to a fifth for the one order of summation.  (Below K = 16 the float instruction's error is the
-    smaller one, too: gemm_float.hip.)"""
+    instruction, N = 1,152: 33 rows K = 16 7.0 and 5.8, 64 8.2 and 8.2, 128 9.8 and 11.5, 896 28 and 51; 128 rows K = 16 6.9
+    and 12.2, 64 8.3 and 16.5, 896 29 and 89; 1,000 rows of 9,728 K = 16 25 and 18, 64 31 and 30, 128 39 and 43, 896 130 and
+    204.  17 and 32 rows: K = 64 5.3, 5.9 and 4.8, 5.1, 100 6.1, 6.7 and 6.0, 6.3, 128 6.2, 6.8 and 6.4, 6.7, 256 8.1, 8.7 and 9.7,
+    10.1, 896 18, 19 and 26, 27, 2,048 35, 36 and 56, 56, 4,864 54 and 147: below K = 100 they pay up to a fifth for the one order of
+    summation.  (Below K = 16 the float
+    instruction's error is the smaller one, too: gemm_float.hip.)"""
     most = max(128, FLOAT_SPLIT_BYTES // (-(-K // 16) * 96) // 128 * 128)
     split = ws = None
     if M > 32 or a.data_ptr() % 16 or not library().tl_gemm_float_split_takes_rows(M, N, K, lda):
-        split = torch.empty(library().tl_gemm_float_split_bytes(min(M, most), K), dtype=torch.uint8, device=a.device)
-    if ranges is None:
-        ranges = weight_ranges(shuffled, N, K)
-    elif not (ranges.dtype == torch.int32 and ranges.is_contiguous() and ranges.device == a.device
-              and ranges.numel() == library().tl_gemm_float_ranges_size(N, K)):
-        raise KernelError(f"linear: the ranges do not belong to a [{N}, {K}] matrix")
+        split = torch.empty(-(-min(M, most) // 32) * -(-K // 16) * 1536, dtype=torch.int16, device=a.device)
     for r in range(0, M, most):
         m = min(M - r, most)
         floats = library().tl_gemm_float_split_workspace(m, N, K)
         if floats and (ws is None or ws.numel() < floats):
             ws = torch.empty(floats, dtype=torch.float32, device=a.device)
-        _call("tl_gemm_float_split", a[r:], shuffled, ranges, bias, out[r:], split, ws, m, N, K, lda, ldc, _stream())
+        _call("tl_gemm_float_split", a[r:], shuffled, bias, out[r:], split, ws, m, N, K, lda, ldc, _stream())
     return out
 
 
@@ -730,7 +698,7 @@ def _tiles(a, shuffled, bias, out_dtype, M, N, K, lda, plan: int, keep_shares: b
     return ShareSum(ws) if kept else out
 
 
-def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None, ranges=None) -> torch.Tensor:
+def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None) -> torch.Tensor:
     """bfloat16 with few rows: the streaming MFMA kernels.  float32 with the matrix-core ordered copy: the few-row kernel,
     or (more than 16 rows, a K of 64 or more) the float product on the bfloat16 instruction.  The rest: the plain tiled
     kernel.  (bfloat16 with many rows went to gemm_tiles.hip or the library before this; the reference uses a library:
@@ -747,7 +715,7 @@ def _linear_dispatch(a, weight, bias, out, M, N, K, lda, ldc, shuffled=None, ran
         return out
     if (shuffled is not None and shuffled.dtype == torch.float32 and a.dtype == torch.float32 and out.dtype == torch.float32
             and SKINNY_MAX_ROWS < M <= FLOAT_SPLIT_MAX_ROWS and K >= FLOAT_SPLIT_MIN_K):
-        return _float_split(a, shuffled, ranges, bias, out, M, N, K, lda, ldc)
+        return _float_split(a, shuffled, bias, out, M, N, K, lda, ldc)
     _call("tl_gemm_generic", a, _code(a, "linear input"), weight, _code(weight, "linear weight"),
           bias, out, _code(out, "linear output"), M, N, K, lda, ldc, _stream())
     return out
@@ -855,11 +823,11 @@ def tune_library_linear(rows: int, weight: torch.Tensor, out_dtype: torch.dtype,
 
 
 def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
-                   shuffled: torch.Tensor | None = None, activation: str = "silu", ranges: torch.Tensor | None = None) -> torch.Tensor:
+                   shuffled: torch.Tensor | None = None, activation: str = "silu") -> torch.Tensor:
     """``silu(h Wg^T) * (h Wu^T)`` for a fused [2I, K] weight (gate rows first): one kernel for
     bfloat16 rows where it reads the ``shuffled`` copy (few rows, or what gemm_tiles.hip takes), product then SiLU-multiply otherwise.
     ``h`` may be :class:`NormedRows` (few-row kernel only).  ``activation`` "gelu_tanh": the tanh form of GELU
-    passes the gate instead of SiLU (in the streaming kernels' epilogues, or by a pass over the product).  ``ranges``: as :func:`linear`'s."""
+    passes the gate instead of SiLU (in the streaming kernels' epilogues, or by a pass over the product)."""
     if not (activation in GLU_ACTIVATIONS):
         raise KernelError(f"swiglu_gate_up: unknown activation {activation!r}")
     if activation != "silu":
@@ -889,7 +857,7 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
             if plan:
                 _on_gpu(h, gate_up_weight, shuffled)
                 return _tiles(h, shuffled, None, h.dtype, M, 2 * I, K, lda, plan, gated=True, act=2)
-        return glu(linear(h, gate_up_weight, shuffled=shuffled, ranges=ranges), activation, h.dtype)
+        return glu(linear(h, gate_up_weight, shuffled=shuffled), activation, h.dtype)
     owed = h if isinstance(h, NormedRows) else None
     if owed is not None:
         h = owed.rows
@@ -914,7 +882,7 @@ def swiglu_gate_up(h: torch.Tensor | NormedRows, gate_up_weight: torch.Tensor,
         plan = _tiles_plan(h, shuffled, M, 2 * I, K, lda, gated=True)
         if plan:
             return _tiles(h, shuffled, None, h.dtype, M, 2 * I, K, lda, plan, gated=True)
-    return silu_mul(linear(owed if owed is not None else h, gate_up_weight, shuffled=shuffled, ranges=ranges))
+    return silu_mul(linear(owed if owed is not None else h, gate_up_weight, shuffled=shuffled))
 
 
 def _check_caches(k_cache, v_cache, dtype, num_kv_heads, head_dim, who: str) -> None:

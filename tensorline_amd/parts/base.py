@@ -70,7 +70,6 @@ class Linear:
         self.bias: torch.Tensor | None = None
         self.shuffled: torch.Tensor | None = None     # the copy few-row bfloat16 products stream
         self.shuffled_float: torch.Tensor | None = None   # the same for a float32 weight (the 32-bit path's products)
-        self.ranges: torch.Tensor | None = None       # what products of many rows ask of that copy
 
     def tensors(self) -> dict[str, TensorDecl]:
         out = {self.weight_name: TensorDecl((self.out_features, self.in_features), "normal", self.std, "compute")}
@@ -87,11 +86,11 @@ class Linear:
         many-row products read that copy, the others hand the row-major one to the library: twice the
         bytes, for which 288 GB of HBM has room."""
         self.shuffled = kernels.shuffle_weight(self.weight)
-        self.shuffled_float, self.ranges = kernels.shuffle_weight_float_and_ranges(self.weight)
+        self.shuffled_float = kernels.shuffle_weight_float(self.weight)
         return self
 
     def tensors_kept(self) -> list[torch.Tensor]:
-        return [t for t in (self.weight, self.bias, self.shuffled, self.shuffled_float, self.ranges) if t is not None]
+        return [t for t in (self.weight, self.bias, self.shuffled, self.shuffled_float) if t is not None]
 
     def in_library(self, out_dtype: torch.dtype, form: str = "plain") -> tuple:
         """This matrix for :meth:`Part.library_products`; ``form``: what its product's kernel does with the sums."""
@@ -102,17 +101,10 @@ class Linear:
         """The matrix-core ordered copy few-row products stream, of whichever type the weight has."""
         return self.shuffled if self.shuffled is not None else self.shuffled_float
 
-    @property
-    def copies(self) -> dict[str, torch.Tensor]:
-        """What a product may read in the matrix's place, by the names that :func:`kernels.linear` gives it."""
-        if self.ranges is None:
-            return {"shuffled": self.streamed}
-        return {"shuffled": self.shuffled_float, "ranges": self.ranges}
-
     def __call__(self, x, out_dtype: torch.dtype | None = None, sink=None, with_bias: bool = True,
                  keep_shares: bool = False, act: str | None = None):
         return kernels.linear(x, self.weight, self.bias if with_bias else None, out_dtype=out_dtype,
-                              sink=sink, keep_shares=keep_shares, act=act, **self.copies)
+                              shuffled=self.streamed, sink=sink, keep_shares=keep_shares, act=act)
 
 
 def fuse_linears(name: str, parts: list[Linear]) -> Linear:

@@ -154,7 +154,7 @@ class RoutedExperts(Part):
         shared = None
         if self.shared_down is not None:
             if self.activation == "swiglu":       # SiLU rides on the few-row product, as in the dense feed-forward
-                act = kernels.swiglu_gate_up(h, self.shared_gate_up.weight, **self.shared_gate_up.copies)
+                act = kernels.swiglu_gate_up(h, self.shared_gate_up.weight, self.shared_gate_up.streamed)
             else:
                 act = kernels.clamp_glu(self.shared_gate_up(h, out_dtype=torch.float32), self.shared_limit, self.alpha, self.dtype)
             shared = self.shared_down(act, out_dtype=torch.float32)

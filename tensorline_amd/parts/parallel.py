@@ -60,7 +60,7 @@ class ParallelMixers(Part):
             self.fused = fuse_linears(self.prefix + "in", firsts)
             self._split = firsts[0].out_features
             for lin in firsts:            # the fused copy is the one that is kept
-                lin.weight = lin.bias = lin.shuffled = lin.shuffled_float = lin.ranges = None
+                lin.weight = lin.bias = lin.shuffled = lin.shuffled_float = None
 
     def weight_tensors(self):
         return (self.fused.tensors_kept() if self.fused is not None else []) + [t for m in self.sides for t in m.weight_tensors()]

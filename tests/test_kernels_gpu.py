@@ -1675,10 +1675,6 @@ def test_ordered_copy_of_a_matrix(N, Kd, dtype, step):
     want = padded.view(-1, 16, padded.shape[1] // step, 4, step // 4).permute(0, 2, 3, 1, 4)
     assert torch.equal(make(w), want)
     assert torch.equal(make(torch.cat([w, w], 1)[:, :Kd]), want)
-    if dtype == "float32":
-        w[N // 2].zero_()
-        sh, ranges = K().shuffle_weight_float_and_ranges(w)
-        assert torch.equal(sh, make(w)) and torch.equal(ranges, K().weight_ranges(sh, N, Kd))
 
 
 @pytest.mark.parametrize("T,B,N,Kd", [(1, 2, 16, 8), (31, 3, 48, 40), (33, 2, 192, 128), (130, 1, 112, 96), (2049, 32, 128, 192), (257, 32, 272, 192),
@@ -1969,10 +1965,10 @@ def test_17_to_64_rows_in_tiles_of_what_is_there(M, N, Kd):
 
 
 @pytest.mark.parametrize("M,N,Kd", [(17, 130, 64), (32, 300, 2048), (33, 129, 2064), (97, 2051, 4112), (300, 1000, 896), (700, 5000, 2050)])
-def test_linear_float_where_halves_lose_the_smallest_values(M, N, Kd):
+def test_linear_float_where_large_values_meet_zeros(M, N, Kd):
     """Rows whose large values meet zeros in the matrix, and the other way round, so that a result is made of values 2^-30 of their
-    segment's largest, which a half no longer holds: the bound of K float multiply-adds all the same.  Rows and columns of zeros give zeros,
-    and a row has the same bits whatever rows come along and whether the matrix' ranges are given or made."""
+    row's largest: the bound of K float multiply-adds all the same.  A value that is picked out of a row comes out as it is, rows and
+    columns of zeros give zeros, and a row has the same bits whatever rows come along."""
     torch.manual_seed(M + Kd)
     a, w, b = torch.randn(M, Kd, device=DEV), torch.randn(N, Kd, device=DEV), torch.randn(N, device=DEV)
     a[1, ::2] *= 2.0 ** 30                                   # meets columns that are zero there
@@ -1984,18 +1980,47 @@ def test_linear_float_where_halves_lose_the_smallest_values(M, N, Kd):
     w[8, Kd - 1] = 1.0                                       # picks one value out of every row, the smallest too
     a[6, Kd - 1], a[9, Kd - 1] = 2.0 ** -30, 2.0 ** -100
     ws = K().shuffle_weight_float(w)
-    ranges = K().weight_ranges(ws, N, Kd)
     got = K().linear(a, w, b, shuffled=ws)
     want, size = a.double() @ w.double().T + b.double(), a.double().abs() @ w.double().abs().T + b.double().abs()
     assert bool(((got.double() - want).abs() <= (Kd + 8) * 2.0 ** -24 * size).all())
-    plain_sums = K().linear(a, w, shuffled=ws, ranges=ranges)
+    plain_sums = K().linear(a, w, shuffled=ws)
     assert bool((plain_sums[4] == 0).all()) and bool((plain_sums[:, 7] == 0).all())
-    small = plain_sums[:, 8].double() - a[:, Kd - 1].double()        # of one product each, within the float's last place
-    assert bool((small.abs() <= 2.0 ** -22 * a[:, Kd - 1].double().abs()).all())
-    assert torch.equal(K().linear(a, w, b, shuffled=ws, ranges=ranges), got)
-    assert torch.equal(K().linear(a[:17], w, b, shuffled=ws, ranges=ranges), got[:17])
-    with pytest.raises(K().KernelError):
-        K().linear(a, w, b, shuffled=ws, ranges=ranges[1:])
+    assert torch.equal(plain_sums[:, 8], a[:, Kd - 1])
+    assert torch.equal(K().linear(a[:17], w, b, shuffled=ws), got[:17])
+
+
+@pytest.mark.parametrize("M", [17, 32, 40, 200])
+@pytest.mark.parametrize("Kd", [64, 80, 896, 2048])
+def test_linear_float_keeps_all_bits_of_small_values(M, Kd):
+    """Values 2^-17 to 2^-25 of their row's largest, which meets a zero, all of one sign and with the same last bits, so that what is lost of
+    each would add up: the sum is off by what its own roundings make of it, six a step of 16 k, each at most 2^-24 of it and of either
+    sign (four times the root of their number), and 2^-22 for the partial products that are left out.  The roles of both operands."""
+    torch.manual_seed(Kd + M)
+    limit = 2.0 ** -22 + 4.0 * math.sqrt(6 * Kd / 16) * 2.0 ** -24
+    small = torch.empty(M, Kd, dtype=torch.float64)
+    for r in range(M):                                       # multiples of 2^-38, all 2^-40 off one
+        c = 2.0 ** -(17 + r % 9) * (1.0 + 0.9 * torch.rand((), dtype=torch.float64))
+        small[r] = (c * 2.0 ** 38).floor() * 2.0 ** -38 + torch.randint(0, 4, (Kd,)) * 2.0 ** -38 + 2.0 ** -40
+    small[:, 0] = 1.0
+    small = small.float().to(DEV)
+    ones = torch.ones(48, Kd, device=DEV)
+    ones[:, 0] = 0.0
+    want = small.double()[:, 1:].sum(1, keepdim=True)
+    for a, w in ((small, ones), (ones, small)):
+        got = K().linear(a, w, shuffled=K().shuffle_weight_float(w))
+        off = (got if a is small else got.T).double() / want - 1.0
+        assert off.shape == (M, 48) and off.abs().max().item() <= limit
+
+
+def test_linear_float_of_more_rows_than_fit_a_grid_by_eights():
+    """524,300 rows of a short K, one launch: every row the bits of the same row in a call of a few hundred."""
+    M, N, Kd = 65535 * 8 + 20, 16, 64
+    torch.manual_seed(5)
+    a, w = torch.randn(M, Kd, device=DEV), torch.randn(N, Kd, device=DEV)
+    ws = K().shuffle_weight_float(w)
+    got = K().linear(a, w, shuffled=ws)
+    for r in (0, M // 2, M - 300):
+        assert torch.equal(got[r:r + 300], K().linear(a[r:r + 300].contiguous(), w, shuffled=ws))
 
 
 @pytest.mark.parametrize("nq,nkv,d,bs", [(4, 4, 64, 4), (14, 2, 64, 16), (28, 4, 128, 16), (3, 1, 128, 8), (40, 2, 64, 128), (130, 1, 128, 16)])
