@@ -928,8 +928,8 @@ extern "C" int tl_glu(const void* gu, int in_dtype, void* out, int out_dtype, in
 // A work-group per token and a share of the heads (of queries, keys or values, in that order); LANES lanes take a head, a lane the
 // pairs LANES apart of it.  What bounds large steps is the instructions of a head, most of them the same for all its lanes (the sum, the
 // root and quotient of the norm, addresses): sixteen lanes to a head give them to four heads of a wave at once, 2,048 tokens of 32 query,
-// 8 key and 8 value heads of 128 35 -> 26 us with a norm, 27 -> 23 without, where a wave took one head at a time.  Small steps are bound by a wave's chain, and
-// 64 lanes to a head make it short: 16 tokens 3.4 against 4.1 us; 128 tokens 7.3 us either way.  The sum of squares adds pairs 64 apart, then 32, 16 .. 1
+// 8 key and 8 value heads of 128 37 -> 28 us with a norm, 29 -> 24 without, where a wave takes one head at a time.  Small steps are bound by a wave's chain, and
+// 64 lanes to a head make it short: 16 tokens 3.4 against 4.1 us (the line: tl_head_lanes).  The sum of squares adds pairs 64 apart, then 32, 16 .. 1
 // apart in both.  A work-group computes the token's cosines and sines once, into LDS.  Steps of many tokens leave the values to a kernel of their own (n_units then ends with the keys): written a token at
 // a time they are single numbers a page apart, written for sixteen neighbouring tokens at a time they are runs.
 template <typename T, int D_MAX, int LANES>
@@ -941,6 +941,7 @@ __global__ __launch_bounds__(256) void head_norm_rotate_store_kernel(
     constexpr int NQ = D_MAX / 2 / LANES;                          // pairs of a lane
     __shared__ float cs[128], sn[128];
     const int t = blockIdx.x, m = threadIdx.x % LANES;
+    if (LANES == 64 && halves) pairs = 0;                          // a head's lanes would part ways
     const float* row = proj + (size_t)t * ldp;
     const float p = freq ? (float)pos[t] : 0.f;
     for (int i = threadIdx.x; 2 * i < rot; i += 256) {
@@ -968,12 +969,23 @@ __global__ __launch_bounds__(256) void head_norm_rotate_store_kernel(
             const bool apart = halves && (is_q || is_k) && 2 * i < rot;
             ca[j] = apart ? i : 2 * i;
             cb[j] = apart ? i + (rot >> 1) : 2 * i + 1;
-            if (pairs && !apart) {
-                const float2 v = ca[j] < n ? *reinterpret_cast<const float2*>(x + ca[j]) : make_float2(0.f, 0.f);
-                raw[2 * j] = v.x, raw[2 * j + 1] = v.y;
-            } else {
+        }
+        if (LANES == 64 && !pairs) {                              // (apart from the other form, whose loads would wait for each other with it)
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) {
                 raw[2 * j] = ca[j] < n ? x[ca[j]] : 0.f;
                 raw[2 * j + 1] = cb[j] < n ? x[cb[j]] : 0.f;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) {
+                if (pairs && cb[j] == ca[j] + 1) {
+                    const float2 v = ca[j] < n ? *reinterpret_cast<const float2*>(x + ca[j]) : make_float2(0.f, 0.f);
+                    raw[2 * j] = v.x, raw[2 * j + 1] = v.y;
+                } else {
+                    raw[2 * j] = ca[j] < n ? x[ca[j]] : 0.f;
+                    raw[2 * j + 1] = cb[j] < n ? x[cb[j]] : 0.f;
+                }
             }
         }
         const float* w = norm == 1 ? (is_q ? wq : is_k ? wk : nullptr) : nullptr;
@@ -1008,38 +1020,52 @@ __global__ __launch_bounds__(256) void head_norm_rotate_store_kernel(
         }
         T* at = is_q ? q_out + ((size_t)t * H + head) * D : k_cache + ((size_t)slot * G + head) * D;
         T* vat = v_cache + ((size_t)pg * G + head) * D * page + within;
-        if (keep) {
-#pragma unroll
-            for (int j = 0; j < NQ; ++j) {
-                const int i = m + LANES * j;
-                float a = raw[2 * j] * rstd, b = raw[2 * j + 1] * rstd;
-                if (w) {
-                    a = ca[j] < n ? a * by[2 * j] : 0.f;
-                    b = cb[j] < n ? b * by[2 * j + 1] : 0.f;
-                }
-                if ((is_q || is_k) && 2 * i + 1 < rot) {
-                    const float ra = a * cs[i] - b * sn[i], rb = b * cs[i] + a * sn[i];
-                    a = ra;
-                    b = rb;
-                }
-                if (is_q || is_k) {                               // zeros beyond the head's values
-                    if (pairs && cb[j] == ca[j] + 1) {            // neighbours: one store (D is even)
-                        if (ca[j] < D) {
-                            if constexpr (sizeof(T) == 4) *reinterpret_cast<float2*>(at + ca[j]) = make_float2(a, b);
-                            else *reinterpret_cast<uint32_t*>(at + ca[j]) = tl_pack_bf16(a, b);
-                        }
-                    } else {
-                        if (ca[j] < D) at[ca[j]] = tl_from_float<T>(a);
-                        if (cb[j] < D) at[cb[j]] = tl_from_float<T>(b);
-                    }
-                    if (is_k && v_from_k) {
-                        if (ca[j] < D) vat[(size_t)ca[j] * page] = tl_from_float<T>(raw[2 * j]);
-                        if (cb[j] < D) vat[(size_t)cb[j] * page] = tl_from_float<T>(raw[2 * j + 1]);
+        auto turn = [&](int j, float& a, float& b) {
+            const int i = m + LANES * j;
+            a = raw[2 * j] * rstd, b = raw[2 * j + 1] * rstd;
+            if (w) {
+                a = ca[j] < n ? a * by[2 * j] : 0.f;
+                b = cb[j] < n ? b * by[2 * j + 1] : 0.f;
+            }
+            if ((is_q || is_k) && 2 * i + 1 < rot) {
+                const float ra = a * cs[i] - b * sn[i], rb = b * cs[i] + a * sn[i];
+                a = ra;
+                b = rb;
+            }
+        };
+        auto put = [&](int j, float a, float b) {                 // zeros beyond the head's values
+            if (is_q || is_k) {
+                if (pairs && cb[j] == ca[j] + 1) {                // neighbours: one store (D is even)
+                    if (ca[j] < D) {
+                        if constexpr (sizeof(T) == 4) *reinterpret_cast<float2*>(at + ca[j]) = make_float2(a, b);
+                        else *reinterpret_cast<uint32_t*>(at + ca[j]) = tl_pack_bf16(a, b);
                     }
                 } else {
-                    if (ca[j] < D) vat[(size_t)ca[j] * page] = tl_from_float<T>(a);
-                    if (cb[j] < D) vat[(size_t)cb[j] * page] = tl_from_float<T>(b);
+                    if (ca[j] < D) at[ca[j]] = tl_from_float<T>(a);
+                    if (cb[j] < D) at[cb[j]] = tl_from_float<T>(b);
                 }
+                if (is_k && v_from_k) {
+                    if (ca[j] < D) vat[(size_t)ca[j] * page] = tl_from_float<T>(raw[2 * j]);
+                    if (cb[j] < D) vat[(size_t)cb[j] * page] = tl_from_float<T>(raw[2 * j + 1]);
+                }
+            } else {
+                if (ca[j] < D) vat[(size_t)ca[j] * page] = tl_from_float<T>(a);
+                if (cb[j] < D) vat[(size_t)cb[j] * page] = tl_from_float<T>(b);
+            }
+        };
+        if (!keep) continue;
+        if constexpr (LANES == 64) {
+            float y[2 * NQ];
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) turn(j, y[2 * j], y[2 * j + 1]);
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) put(j, y[2 * j], y[2 * j + 1]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) {
+                float a, b;
+                turn(j, a, b);
+                put(j, a, b);
             }
         }
     }
@@ -1066,6 +1092,13 @@ __global__ __launch_bounds__(256) void head_values_store_kernel(const float* __r
                     tl_from_float<T>(c + e >= dv ? 0.f : y0 ? (1.0f - lam) * x[c + e] + lam * y0[c + e] : x[c + e]);
 }
 
+// Lanes to a head of a step of T tokens with `units` heads each in rows of D.  Us with 64 and 16 lanes, queries and keys normed: 128 tokens of 16 heads of 64
+// 6.6 and 6.9, 200 7.0 and 7.0, 512 9.7 and 7.3; of 12 heads of 128 384 tokens level, 512 0.87 of the time; of 36 160 tokens level, 384 0.77; five heads
+// leave eleven of a work-group's sixteen places empty: level at best, 2,048 tokens 1.06 without a norm.  Rows beyond 128 give a lane of
+// sixteen eight pairs, whose chain is longer than what is saved (T tokens of 12 heads of 256 200 9.2 and 10.7, 2,048 without a norm 21.1
+// and 21.9, of three 1.4 times as long).
+extern "C" int tl_head_lanes(int T, int units, int D) { return D <= 128 && units >= 6 && T >= 128 && (long long)T * units >= 4608 ? 16 : 64; }
+
 extern "C" int tl_head_norm_rotate_store(const float* proj, int ldp, const int32_t* pos, const float* wq, const float* wk,
                                          float eps, const float* freq, float mag, int rot, const int32_t* slots, void* q_out,
                                          void* k_cache, void* v_cache, int dtype, int T, int H, int G, int d, int dv, int D,
@@ -1083,16 +1116,16 @@ extern "C" int tl_head_norm_rotate_store(const float* proj, int ldp, const int32
     if (T == 0) return 0;
     const bool values_apart = !v_from_k && G > 0 && G <= 65535 && T >= 64;
     const int units = H + G + (v_from_k || values_apart ? 0 : G);
-    const bool few = T < 128;
-    dim3 grid(T, tl_ceil_div(units, few ? 4 : 16)), block(256);
+    const int lanes = tl_head_lanes(T, units, D);
+    dim3 grid(T, tl_ceil_div(units, lanes == 16 || T >= 512 ? 16 : 4)), block(256);
     TL_CHECK_ARG(grid.y <= 65535, "tl_head_norm_rotate_store: too many heads");
     const size_t two = 2 * (dtype == TL_F32 ? sizeof(float) : sizeof(bf16_t));
     // neighbours go by one access
     const int pairs = D % 2 == 0 && d % 2 == 0 && dv % 2 == 0 && ldp % 2 == 0 && (uintptr_t)proj % 8 == 0 && (uintptr_t)q_out % two == 0 &&
                       (uintptr_t)k_cache % two == 0;
 #define GO(TT)                                                                                                         \
-    hipLaunchKernelGGL((few ? D <= 128 ? head_norm_rotate_store_kernel<TT, 128, 64> : head_norm_rotate_store_kernel<TT, 256, 64>                \
-                            : D <= 128 ? head_norm_rotate_store_kernel<TT, 128, 16> : head_norm_rotate_store_kernel<TT, 256, 16>), grid, block, 0, stream, proj, ldp, pos, wq, wk, eps, freq, mag, \
+    hipLaunchKernelGGL((D > 128 ? head_norm_rotate_store_kernel<TT, 256, 64> : lanes == 64 ? head_norm_rotate_store_kernel<TT, 128, 64>         \
+                                                                             : head_norm_rotate_store_kernel<TT, 128, 16>), grid, block, 0, stream, proj, ldp, pos, wq, wk, eps, freq, mag, \
                        rot, slots, (TT*)q_out, (TT*)k_cache, (TT*)v_cache, H, G, d, dv, D, page, v_from_k, norm, halves, units, first, ldf, lam, pairs)
     if (dtype == TL_F32) GO(float);
     else if (dtype == TL_BF16) GO(bf16_t);

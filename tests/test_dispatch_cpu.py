@@ -245,3 +245,13 @@ def test_products_bound_by_their_weights_take_the_tiles_that_keep_the_cus_least_
     plan = K.library().tl_gemm_tiles_plan
     for N, Kd in ((152064, 3584), (151936, 1536), (131072, 5120)):
         assert all(plan(M, N, Kd, 0, 0) == 256 + 2 for M in (65, 96, 128)) and plan(192, N, Kd, 0, 0) == 256 + 6      # of 128 and 192 rows
+
+
+def test_heads_have_the_lanes_that_are_faster():
+    """Rows of heads past 128, a few heads and small steps: 64 lanes a head; many heads of up to 128: sixteen."""
+    lanes = K.library().tl_head_lanes
+    for T, units, D in ((128, 12, 256), (2048, 12, 256), (2048, 40, 256), (2048, 32, 192), (2048, 5, 64), (512, 5, 128), (128, 16, 64), (200, 12, 128),
+                        (100, 64, 128), (1, 40, 128)):
+        assert lanes(T, units, D) == 64, (T, units, D)
+    for T, units, D in ((512, 16, 64), (512, 12, 128), (160, 36, 128), (200, 24, 128), (2048, 7, 64), (2048, 48, 96)):
+        assert lanes(T, units, D) == 16, (T, units, D)

@@ -2173,9 +2173,10 @@ def test_four_values_at_a_time_and_one(what, rows, width):
 @pytest.mark.parametrize("halves", [False, True])
 @pytest.mark.parametrize("d,dv,D,turned", [(128, 128, 128, 64), (50, 40, 64, 20), (63, 63, 63, 30), (200, 256, 256, 200)])
 def test_heads_of_small_and_large_steps_alike(d, dv, D, turned, halves):
-    """A head has 64 lanes in steps of up to 127 tokens and 16 in larger ones, accesses of two numbers where sizes and addresses are even:
-    the same bits of queries, keys and values."""
-    H, G, T, page = 5, 2, 128, 16
+    """A head of up to 128 dimensions has 64 lanes in a small step and 16 in a large one, accesses of two numbers where sizes and addresses are
+    even: the same bits of queries, keys and values."""
+    H, G, T, page, few = 5, 2, 672, 16, 300
+    assert [K().library().tl_head_lanes(t, H + G, D) for t in (few, T)] == ([64, 16] if D <= 128 else [64, 64])
     torch.manual_seed(d)
     cols = (H + G) * d + G * dv
     proj, wide = torch.randn(T, cols + cols % 2, device=DEV), torch.empty(T, cols + 3 - cols % 2, device=DEV)
@@ -2188,10 +2189,10 @@ def test_heads_of_small_and_large_steps_alike(d, dv, D, turned, halves):
         t = x.shape[0]
         kc, vc = torch.zeros(T // page, page, G, D, dtype=torch.bfloat16, device=DEV), torch.zeros(T // page, G, D, page, dtype=torch.bfloat16, device=DEV)
         q = K().head_norm_rotate_store(x, n[:t], w[0].contiguous(), w[1].contiguous(), 1e-5, freq, 1.1, kc, vc, slots[:t], H, G, d, dv, False, torch.bfloat16, halves=halves)
-        return q, kc.view(-1, G, D)[1:], vc.permute(0, 3, 1, 2).reshape(-1, G, D)[1:]      # (slot 0 is the last token's)
-    (q, kc, vc), (q1, kc1, vc1), (q2, kc2, vc2) = run(proj), run(wide[:, 1:cols + 1]), run(proj[:T - 1])
+        return q, kc.view(-1, G, D), vc.permute(0, 3, 1, 2).reshape(-1, G, D)
+    (q, kc, vc), (q1, kc1, vc1), (q2, kc2, vc2) = run(proj), run(wide[:, 1:cols + 1]), run(proj[:few])
     assert torch.equal(q, q1) and torch.equal(kc, kc1) and torch.equal(vc, vc1)
-    assert torch.equal(q[:T - 1], q2) and torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    assert torch.equal(q[:few], q2) and torch.equal(kc[T - few:], kc2[T - few:]) and torch.equal(vc[T - few:], vc2[T - few:])   # (token i's slot: T - 1 - i)
     x = proj[:, :H * d].double().view(T, H, d)
     x = x / torch.sqrt(x.square().mean(2, keepdim=True) + 1e-5) * w[0].double()
     angle = (n.unsqueeze(1).float() * freq).double()
