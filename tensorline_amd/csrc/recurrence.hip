@@ -28,8 +28,7 @@
 // Steps that bring portions of more than a chunk (HELP) have a second four waves to a work-group, one to a SIMD, that bring the chunks to LDS
 // (SiLU and decays among it), and add up and write the outputs of the chunk before, while the first four do nothing but walk: what a token
 // costs is then the walk's instructions and reads alone.  Sequences of 803, 211 and 507 tokens, us: 16 heads of 128 x 128 with one decay 219 -> 138,
-// 32 of 64 x 64 with a decay per channel 127 -> 87; one of 2,048 547 -> 291 and 317 -> 187.  Where more work-groups come than CUs hold two of, the
-// second four waves are in the way (40 sequences of 33 tokens 104 and 118, eight of 100 61 and 59 or 84 and 96), and one chunk leaves them nothing to do.
+// 32 of 64 x 64 with a decay per channel 127 -> 87; one of 2,048 547 -> 291 and 317 -> 187.  Where they are in the way: tl_linear_recurrence_helps.
 #include "common.h"
 
 #include <math.h>
@@ -38,7 +37,7 @@
 #define REC_COLS 16
 #define REC_HELP_DK 128        // (beyond, LDS does not hold two chunks)
 #define REC_HELP_TOKENS 16
-#define REC_HELP_GROUPS 512
+#define REC_CUS 256
 
 __device__ __forceinline__ float rec_silu(float z) { return z / (1.0f + expf(-z)); }
 
@@ -226,17 +225,29 @@ __global__ __launch_bounds__(HELP ? 512 : 256) void linear_recurrence_kernel(
 
 extern "C" int tl_linear_recurrence_takes(int dk) { return dk > 0 && dk <= REC_MAX_DK ? 1 : 0; }
 
+// Whether a launch has the second four waves: S sequences of `tokens` together and `longest` at most (0: not known), form as per_token below.
+// One chunk leaves them nothing to do, and two work-groups to a CU have to hold all (40 sequences of 33 tokens without and with them 104 and 118 us, eight of 100 61 and 59
+// or 84 and 96).  With a decay per channel and keys past 64 the chunks of one fill more than half of a CU's LDS (85 KB): what comes second
+// waits for a whole round, at 0.56 of the time a token, and is worth it where one sequence is long and the others are not (16 heads of 128 x 128, four
+// sequences of 40 tokens 22 and 27 us, of 19, 19, 13 and 2 13 and 17; of 75, 218, 686 and 311 0.65 of the time, of 803, 211 and 507 254 and 149).
+extern "C" int tl_linear_recurrence_helps(int S, int tokens, int longest, int H, int dk, int dv, int form) {
+    const long long groups = (long long)tl_ceil_div(dv, REC_COLS) * H * S;
+    if (longest <= REC_HELP_TOKENS || dk > REC_HELP_DK || groups > 2 * REC_CUS) return 0;
+    if (form != 1 || dk <= 64 || groups <= REC_CUS) return 1;
+    return longest >= 64 && 2LL * longest * S >= 3LL * tokens ? 1 : 0;
+}
+
 // q, k [T, >= H*dk], v [T, >= H*dv] float with row strides; per_token 0: decay [H]; per_token 1: wlog
 // [T, >= H*dk] with row stride ldw, bonus [H, dk] or null; per_token 2: q, k [T, >= (H/share)*dk], wlog the
 // steps [T, >= H], decay rate_log [H], bonus step_bias [H] or null, skip [H] or null.  state: float, a
 // request's [H, dk, dv] at state + slot * state_stride.  out float [T, >= H*dv].  S sequences, rows
-// q_start[s] .. q_start[s+1]; longest: the most tokens that one of them brings, 0 where the caller does not know.
+// q_start[s] .. q_start[s+1], `tokens` in all; longest: the most tokens that one of them brings, 0 where the caller does not know.
 extern "C" int tl_linear_recurrence(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
                                     const float* wlog, int ldw, const float* decay, const float* bonus, int per_token,
                                     const float* skip, int share,
                                     float* state, long long state_stride, const int32_t* state_slots,
                                     const int32_t* q_start, float* out, int ldo, int S, int H, int dk, int dv,
-                                    int silu_inputs, int longest, hipStream_t stream) {
+                                    int silu_inputs, int tokens, int longest, hipStream_t stream) {
     TL_CHECK_ARG(S >= 0 && H > 0 && dv > 0, "tl_linear_recurrence: bad sizes S=%d H=%d dv=%d", S, H, dv);
     TL_CHECK_ARG(tl_linear_recurrence_takes(dk), "tl_linear_recurrence: a key size of %d is not served (at most %d)", dk, REC_MAX_DK);
     TL_CHECK_ARG(per_token >= 0 && per_token <= 2, "tl_linear_recurrence: unknown form %d", per_token);
@@ -251,7 +262,7 @@ extern "C" int tl_linear_recurrence(const float* q, int ldq, const float* k, int
     TL_CHECK_ARG(H <= 65535 && S <= 65535, "tl_linear_recurrence: too many heads or sequences for one launch");
     if (S == 0) return 0;
     const dim3 grid(tl_ceil_div(dv, REC_COLS), H, S);
-    const bool help = longest > REC_HELP_TOKENS && dk <= REC_HELP_DK && (long long)grid.x * H * S <= REC_HELP_GROUPS;
+    const bool help = tl_linear_recurrence_helps(S, tokens, longest, H, dk, dv, per_token) != 0;
     const dim3 block(help ? 512 : 256);
 #define GO_MODE(R, MODE, HELP)                                                                                          \
     hipLaunchKernelGGL((linear_recurrence_kernel<R, MODE, HELP>), grid, block, 0, stream, q, ldq, k, ldk, v, ldv, wlog, ldw, \

@@ -1721,7 +1721,7 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ctx, st
           decay, bonus, per_token, skip if per_token == 2 else None, share,
           st, stride, ctx.state_slots,
           ctx.q_start, out, heads * dv, ctx.num_seqs, heads, dk, dv, 1 if silu_inputs else 0,
-          int(facts.max_query_len) if facts is not None else 0, _stream())
+          T, int(facts.max_query_len) if facts is not None else 0, _stream())
     return out
 
 

@@ -255,3 +255,17 @@ def test_heads_have_the_lanes_that_are_faster():
         assert lanes(T, units, D) == 64, (T, units, D)
     for T, units, D in ((512, 16, 64), (512, 12, 128), (160, 36, 128), (200, 24, 128), (2048, 7, 64), (2048, 48, 96)):
         assert lanes(T, units, D) == 16, (T, units, D)
+
+
+def test_recurrences_have_helping_waves_where_that_is_faster():
+    """One to a CU (a decay per channel, keys past 64): a second round of work-groups only beside one long sequence."""
+    helps = lambda lens, H, dk, dv, form: K.library().tl_linear_recurrence_helps(len(lens), sum(lens), max(lens), H, dk, dv, form)
+    for lens, H, dk, dv in (([40] * 4, 16, 128, 128), ([17] * 8, 8, 96, 96), ([64] * 16, 8, 128, 64), ([1] * 15 + [20], 8, 128, 64), ([19, 19, 13, 2], 16, 128, 128),
+                            ([1, 4, 17], 16, 80, 128), ([500] * 4, 16, 128, 128), ([600, 600, 600, 120], 16, 128, 128)):
+        assert not helps(lens, H, dk, dv, 1), (lens, H, dk, dv)
+        assert helps(lens, H, dk, dv, 0) and helps(lens, H, dk, dv, 2) and helps(lens, H, 64, dv, 1)
+    for lens, H, dk, dv in (([17], 16, 128, 128), ([803, 211, 507], 16, 128, 128), ([75, 218, 686, 311], 16, 128, 128), ([40] * 4, 8, 96, 96)):
+        assert helps(lens, H, dk, dv, 1), (lens, H, dk, dv)
+    for form in (0, 1, 2):
+        assert not helps([16] * 4, 4, 64, 64, form) and not helps([300], 4, 144, 64, form) and not helps([40] * 40, 16, 64, 128, form)
+        assert not K.library().tl_linear_recurrence_helps(1, 100, 0, 4, 64, 64, form)
