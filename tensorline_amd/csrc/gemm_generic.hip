@@ -483,6 +483,15 @@ __global__ __launch_bounds__(GG_THREADS) void gemm_batched_bf16_kernel(const bf1
     }
 }
 
+// Whether a wave of such a product has 64 rows: where that leaves enough waves, which a short K needs more of (600 rows of 32 heads of 192 x
+// 128 10.0 and 11.9 us with 32 and 64 rows a wave, 2,048 23.5 and 22.1; 900 of 128 x 192 12.8 and 9.6), and where the rows fill them: 16 of 1,024 x
+// 1,024 take 16.6 and 20.8 us for 17 rows, 19.0 and 22.2 for 64, 22 and 23 for 96, 27 and 23 for 128; 257 to 384 rows are three
+// work-groups or two with a wave or two in the second, level in time (60 and 61 us) unless the two are one round of the GPU (4 of 2,048 x 1,024 46 and 32).
+extern "C" int tl_gemm_batched_tall(int M, int N, int K, int batch) {
+    const double groups = (double)tl_ceil_div(N, 64) * tl_ceil_div(M, 256) * batch;
+    return M >= 128 && groups >= (K >= 192 ? 256 : 512) && (tl_ceil_div(M, 128) != 3 || groups <= 256) ? 1 : 0;
+}
+
 // `batch` products of the same shape in one launch: product b reads A + b * a_bs (row stride lda),
 // W + b * w_bs ([N, K] contiguous) and writes C + b * c_bs (row stride ldc); strides in elements.
 // Each is summed as tl_gemm_generic sums it, or (aligned bfloat16) in steps of 32 k from 0 upwards on the bfloat16
@@ -501,10 +510,9 @@ extern "C" int tl_gemm_generic_batched(const void* A, int a_dtype, const void* W
     // 5.4, x 448 7.3 and 7.1, x 512 7.4 and 7.7, x 640 7.6 and 8.8, 64 x 1,024 7.7 and 12.2.
     if (a_dtype == TL_BF16 && w_dtype == TL_BF16 && c_dtype == TL_BF16 && K % 8 == 0 && K <= (M <= 16 ? 512 : 1024) && lda % 8 == 0 && a_bs % 8 == 0 &&
         w_bs % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && tl_ceil_div(M, 128) <= 65535) {
-        // whole aligned sixteens of columns; and 64 rows a wave where that leaves enough waves, which a short K needs more of (600 rows of 32
-        // heads of 192 x 128 10.0 and 11.9 us with 32 and 64 rows a wave, 2,048 23.5 and 22.1; 900 of 128 x 192 12.8 and 9.6)
+        // whole aligned sixteens of columns
         const bool rows = N % 16 == 0 && (uintptr_t)C % 16 == 0 && ldc % 8 == 0 && c_bs % 8 == 0;
-        const bool tall = rows && (double)tl_ceil_div(N, 64) * tl_ceil_div(M, 256) * batch >= (K >= 192 ? 256 : 512);
+        const bool tall = rows && tl_gemm_batched_tall(M, N, K, batch);
 #define GO(MB, ROWS)                                                                                                                  \
     hipLaunchKernelGGL((gemm_batched_bf16_kernel<MB, ROWS>), dim3(tl_ceil_div(N, 64), tl_ceil_div(M, 64 * MB), batch), dim3(GG_THREADS), 0, \
                        stream, (const bf16_t*)A, (const bf16_t*)W, (bf16_t*)C, M, N, K, lda, ldc, a_bs, w_bs, c_bs)

@@ -269,3 +269,13 @@ def test_recurrences_have_helping_waves_where_that_is_faster():
     for form in (0, 1, 2):
         assert not helps([16] * 4, 4, 64, 64, form) and not helps([300], 4, 144, 64, form) and not helps([40] * 40, 16, 64, 128, form)
         assert not K.library().tl_linear_recurrence_helps(1, 100, 0, 4, 64, 64, form)
+
+
+def test_products_per_head_have_tall_waves_where_rows_fill_them():
+    """64 rows a wave: not for few rows, whatever the batch, nor for three work-groups' rows, nor where waves are few."""
+    tall = K.library().tl_gemm_batched_tall
+    for M, N, Kd, batch in ((1, 1024, 1024, 16), (17, 1024, 1024, 16), (64, 256, 1024, 64), (96, 512, 512, 32), (300, 1024, 1024, 16), (384, 256, 1024, 64), (600, 192, 128, 32),
+                            (128, 128, 512, 32), (2048, 96, 64, 4)):
+        assert not tall(M, N, Kd, batch), (M, N, Kd, batch)
+    for M, N, Kd, batch in ((128, 1024, 1024, 16), (256, 512, 512, 32), (300, 2048, 1024, 4), (400, 1024, 768, 16), (600, 1024, 1024, 16), (2048, 192, 128, 32), (2049, 128, 192, 32)):
+        assert tall(M, N, Kd, batch), (M, N, Kd, batch)
