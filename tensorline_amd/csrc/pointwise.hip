@@ -32,6 +32,12 @@ template <> struct pw_quad<bf16_t> {
     }
 };
 static bool pw_quads(const void* p, int dtype) { return (uintptr_t)p % (dtype == TL_F32 ? 16 : 8) == 0; }
+// log2 of the threads that share a row of so many quads in a work-group of 256; narrow rows leave room for more of them
+static int pw_row_threads(int quads) {
+    int log2 = 0;
+    while (log2 < 8 && 1 << log2 < quads) ++log2;
+    return log2;
+}
 
 // ---- residual add + Dynamic Tanh ---------------------------------------------------------------
 // Without `rows`: x[r] += residual[r] (float, written back); out[r] = tanh(alpha x[r]) * w + b.
@@ -78,7 +84,8 @@ extern "C" int tl_add_dyt(float* x, const void* res, int res_dtype, const float*
                           void* out, int out_dtype, const int32_t* rows, int n, int H, hipStream_t stream) {
     TL_CHECK_ARG(n >= 0 && H > 0, "tl_add_dyt: bad sizes n=%d H=%d", n, H);
     if (n == 0) return 0;
-    const bool quads = H % 4 == 0 && pw_quads(x, TL_F32) && pw_quads(res, res_dtype) && pw_quads(w, TL_F32) && pw_quads(b, TL_F32) && pw_quads(out, out_dtype);
+    // (rows of up to 128 have a thread a number, whose chain is shorter: 4,096 of 64 3.5 us, 3.8 by quads)
+    const bool quads = H > 128 && H % 4 == 0 && pw_quads(x, TL_F32) && pw_quads(res, res_dtype) && pw_quads(w, TL_F32) && pw_quads(b, TL_F32) && pw_quads(out, out_dtype);
     const dim3 grid(n), block(quads ? (H >= 2048 ? 512 : H >= 1024 ? 256 : 128) : H >= 1024 ? 256 : 128);
 #define GO(R, O)                                                                                                                             \
     if (quads) hipLaunchKernelGGL((add_dyt_quad_kernel<R, O>), grid, block, 0, stream, x, (const R*)res, w, b, alpha, (O*)out, rows, H);       \
@@ -180,12 +187,13 @@ __global__ void clamp_glu_kernel(const I* __restrict__ gu, O* __restrict__ out, 
 }
 
 // Four columns a thread, and the sigmoid of middling numbers in its short form (the same bits): 1,521 rows of 2,048, floats to
-// bfloat16 7.2 -> 4.2 us.
+// bfloat16 7.2 -> 4.2 us.  A work-group has as many rows as there is room for (1 << log2 threads to a row): 4,096 rows of 64
+// 3.1 us, 4.3 with a work-group each.
 template <typename I, typename O>
-__global__ __launch_bounds__(256) void clamp_glu_quad_kernel(const I* __restrict__ gu, O* __restrict__ out, int F, float limit, float alpha) {
-    const int c = (blockIdx.y * 256 + threadIdx.x) * 4;
-    const size_t t = blockIdx.x;
-    const bool here = c < F;
+__global__ __launch_bounds__(256) void clamp_glu_quad_kernel(const I* __restrict__ gu, O* __restrict__ out, int T, int F, float limit, float alpha, int log2) {
+    const int c = (int)((blockIdx.y << log2) + (threadIdx.x & ((1 << log2) - 1))) * 4;
+    const size_t t = ((size_t)blockIdx.x << (8 - log2)) + (threadIdx.x >> log2);
+    const bool here = c < F && t < T;
     float4 g = make_float4(0.f, 0.f, 0.f, 0.f), u = g;
     if (here) g = pw_quad<I>::load(gu + t * 2 * F + c), u = pw_quad<I>::load(gu + t * 2 * F + F + c);
     float gv[4] = {g.x, g.y, g.z, g.w}, uv[4] = {u.x, u.y, u.z, u.w};
@@ -214,9 +222,10 @@ extern "C" int tl_clamp_glu(const void* gu, int in_dtype, void* out, int out_dty
     TL_CHECK_ARG(T >= 0 && F > 0, "tl_clamp_glu: bad sizes");
     if (T == 0) return 0;
     const bool quads = F % 4 == 0 && tl_ceil_div(F, 1024) <= 65535 && pw_quads(gu, in_dtype) && pw_quads(out, out_dtype);
-    const dim3 grid = quads ? dim3(T, tl_ceil_div(F, 1024)) : dim3((unsigned)(((size_t)T * F + 255) / 256)), block(256);
+    const int log2 = pw_row_threads(F / 4);
+    const dim3 grid = quads ? dim3(tl_ceil_div(T, 256 >> log2), tl_ceil_div(F, 1024)) : dim3((unsigned)(((size_t)T * F + 255) / 256)), block(256);
 #define GO(I, O)                                                                                                                  \
-    if (quads) hipLaunchKernelGGL((clamp_glu_quad_kernel<I, O>), grid, block, 0, stream, (const I*)gu, (O*)out, F, limit, alpha);   \
+    if (quads) hipLaunchKernelGGL((clamp_glu_quad_kernel<I, O>), grid, block, 0, stream, (const I*)gu, (O*)out, T, F, limit, alpha, log2); \
     else hipLaunchKernelGGL((clamp_glu_kernel<I, O>), grid, block, 0, stream, (const I*)gu, (O*)out, T, F, limit, alpha)
     if (in_dtype == TL_F32 && out_dtype == TL_F32) { GO(float, float); }
     else if (in_dtype == TL_F32 && out_dtype == TL_BF16) { GO(float, bf16_t); }
@@ -577,11 +586,11 @@ __global__ void head_gate_kernel(T* __restrict__ o, const float* __restrict__ ga
 }
 
 // Four numbers of a head at a time, its gate worked out once for them: 2,048 tokens of 32 heads of 128
-// 14.2 -> 7.3 us, 16 tokens 5.2 -> 1.9.
+// 14.2 -> 7.3 us, 16 tokens 5.2 -> 1.9.  Several narrow tokens to a work-group, as above: 4,096 of one head of 64 3.0 us, 4.1 with a work-group each.
 template <typename T>
-__global__ __launch_bounds__(256) void head_gate_quad_kernel(T* __restrict__ o, const float* __restrict__ gate, int ldg, int H, int dv) {
-    const int t = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
-    if (c >= H * dv) return;
+__global__ __launch_bounds__(256) void head_gate_quad_kernel(T* __restrict__ o, const float* __restrict__ gate, int ldg, int tokens, int H, int dv, int log2) {
+    const int t = (int)((blockIdx.y << (8 - log2)) + (threadIdx.x >> log2)), c = (int)((blockIdx.x << log2) + (threadIdx.x & ((1 << log2) - 1))) * 4;
+    if (t >= tokens || c >= H * dv) return;
     const float s = pw_sigmoid(gate[(size_t)t * ldg + c / dv]);
     T* at = o + (size_t)t * H * dv + c;
     const float4 v = pw_quad<T>::load(at);
@@ -593,9 +602,10 @@ extern "C" int tl_head_gate(void* o, int dtype, const float* gate, int ldg, int 
     if (T == 0) return 0;
     const dim3 grid(T), block(256);
     if (dv % 4 == 0 && T <= 65535 && pw_quads(o, dtype) && (dtype == TL_F32 || dtype == TL_BF16)) {
-        const dim3 quads(tl_ceil_div(H * dv, 1024), T);
-        if (dtype == TL_F32) hipLaunchKernelGGL(head_gate_quad_kernel<float>, quads, block, 0, stream, (float*)o, gate, ldg, H, dv);
-        else hipLaunchKernelGGL(head_gate_quad_kernel<bf16_t>, quads, block, 0, stream, (bf16_t*)o, gate, ldg, H, dv);
+        const int log2 = pw_row_threads(H * dv / 4);
+        const dim3 quads(tl_ceil_div(H * dv, 1024), tl_ceil_div(T, 256 >> log2));
+        if (dtype == TL_F32) hipLaunchKernelGGL(head_gate_quad_kernel<float>, quads, block, 0, stream, (float*)o, gate, ldg, T, H, dv, log2);
+        else hipLaunchKernelGGL(head_gate_quad_kernel<bf16_t>, quads, block, 0, stream, (bf16_t*)o, gate, ldg, T, H, dv, log2);
     }
     else if (dtype == TL_F32) hipLaunchKernelGGL(head_gate_kernel<float>, grid, block, 0, stream, (float*)o, gate, ldg, H, dv);
     else if (dtype == TL_BF16) hipLaunchKernelGGL(head_gate_kernel<bf16_t>, grid, block, 0, stream, (bf16_t*)o, gate, ldg, H, dv);

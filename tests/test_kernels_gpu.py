@@ -2170,6 +2170,28 @@ def test_four_values_at_a_time_and_one(what, rows, width):
     torch.testing.assert_close(got[0].double(), want, rtol=2 ** -8, atol=2e-6)
 
 
+@pytest.mark.parametrize("rows,width", [(1, 4), (255, 4), (257, 4), (65, 16), (33, 64), (17, 68), (3, 512), (5, 516), (2, 1024), (3, 1028)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_narrow_rows_share_a_work_group(rows, width, dtype):
+    """The clamped gate and the gate of heads over rows from one quad to more than a work-group's 256: the bits of one number at a time, and
+    nothing beside the rows is written."""
+    k, dt = K(), getattr(torch, dtype)
+    torch.manual_seed(rows + width)
+    gu, heads = 4.0 * torch.randn(rows, 2 * width, device=DEV), 1 if width % 16 else width // 16
+    room = torch.empty(gu.numel() + 1, dtype=dt, device=DEV)
+    room[1:] = gu.to(dt).flatten()
+    assert torch.equal(k.clamp_glu(gu.to(dt), 7.0, 1.702), k.clamp_glu(room[1:].view(rows, 2 * width), 7.0, 1.702))
+    gate, x = torch.randn(rows, heads, device=DEV), torch.randn(rows, width, device=DEV).to(dt)
+    both = torch.full((2, rows * width + 8), 3.0, dtype=dt, device=DEV)
+    outs = []
+    for room, off in zip(both, (4, 5)):                      # (a row of `both` starts at a whole quad)
+        o = room[off:off + rows * width].view(rows, width)
+        o.copy_(x)
+        outs.append(k.head_gate(o, gate, heads))
+        assert bool((room[:off] == 3.0).all()) and bool((room[off + rows * width:] == 3.0).all())
+    assert torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("halves", [False, True])
 @pytest.mark.parametrize("d,dv,D,turned", [(128, 128, 128, 64), (50, 40, 64, 20), (63, 63, 63, 30), (200, 256, 256, 200)])
 def test_heads_of_small_and_large_steps_alike(d, dv, D, turned, halves):
