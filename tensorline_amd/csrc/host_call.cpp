@@ -1,4 +1,5 @@
-// Python's way into the library's C entry points: `enter(address, *arguments)` of the module that this library also is.
+// Python's way into the kernel library's C entry points: `enter(address, *arguments)`, a Python module of its own, so that the library neither
+// needs Python's headers to be built nor its symbols to be loaded.  Without this module ctypes does the same (kernels.py).
 //
 // What bounds a small eager step is the host: 11 to 18 us a launch, of which ctypes' conversions, with an object made around every pointer,
 // stream, float and 64-bit number, took some 3.  Here an argument is converted where it stands: a tensor is its address, None
@@ -14,7 +15,6 @@
 
 #include <stdint.h>
 
-#ifndef __HIP_DEVICE_COMPILE__
 #if !defined(__x86_64__) || defined(_WIN32)
 #error "the calls are made for the System V convention of x86-64"
 #endif
@@ -103,10 +103,9 @@ static PyMethodDef hc_methods[] = {
     {"enter", (PyCFunction)(void (*)(void))hc_enter, METH_FASTCALL, "enter(address, *arguments): the status that a C entry point returns"},
     {nullptr, nullptr, 0, nullptr},
 };
-static PyModuleDef hc_module = {PyModuleDef_HEAD_INIT, "libtensorline_hip", nullptr, -1, hc_methods, nullptr, nullptr, nullptr, nullptr};
+static PyModuleDef hc_module = {PyModuleDef_HEAD_INIT, "tensorline_call", nullptr, -1, hc_methods, nullptr, nullptr, nullptr, nullptr};
 
-PyMODINIT_FUNC PyInit_libtensorline_hip(void) {
+PyMODINIT_FUNC PyInit_tensorline_call(void) {
     hc_data_ptr = PyUnicode_InternFromString("data_ptr");
     return hc_data_ptr ? PyModule_Create(&hc_module) : nullptr;
 }
-#endif

@@ -4,6 +4,8 @@
 ``libtensorline_hip.so`` next to this file (or, when that folder cannot be written, under the
 temporary folder).  A stamp file records the hash of the sources a library was built from; a
 library whose stamp does not match the sources is rebuilt on load, so stale code is never run.
+``csrc/host_call.cpp``, Python's way into it, is a small module beside it, one for each kind of
+Python; where it cannot be built (no headers of Python, another machine than x86-64) it is left out.
 """
 from __future__ import annotations
 
@@ -19,9 +21,12 @@ from concurrent.futures import ThreadPoolExecutor
 
 OFFLOAD_ARCH = "gfx950"
 LIB_NAME = "libtensorline_hip.so"
+CALL_NAME = f"tensorline_call.{sysconfig.get_config_var('SOABI') or 'abi'}.so"
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(_HERE), "csrc")
+CALL_SOURCE = os.path.join(CSRC, "host_call.cpp")
+CALL_FLAGS = ["-x", "c++", "-O3", "-fPIC", "-std=c++17", "-shared"]
 
 # -packed-fp32-ops off: the compiler otherwise forms packed float instructions from scalar code.
 HIPCC_FLAGS = [
@@ -46,7 +51,6 @@ def _headers() -> list[str]:
 def source_hash() -> str:
     h = hashlib.sha256()
     h.update(" ".join(HIPCC_FLAGS).encode())
-    h.update((sysconfig.get_config_var("SOABI") or "").encode())      # host_call.hip is Python's as well
     for path in sources() + _headers():
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as f:
@@ -76,6 +80,21 @@ def find_built() -> str | None:
         lib = os.path.join(d, LIB_NAME)
         if os.path.isfile(lib) and _stamp_ok(lib, want):
             return lib
+    return None
+
+
+def _call_hash() -> str:
+    with open(CALL_SOURCE, "rb") as f:
+        return hashlib.sha256(" ".join([CALL_NAME, *CALL_FLAGS]).encode() + f.read()).hexdigest()
+
+
+def find_call() -> str | None:
+    """Path of a module for this Python that matches the current source, or None."""
+    want = _call_hash()
+    for d in _candidate_dirs():
+        path = os.path.join(d, CALL_NAME)
+        if os.path.isfile(path) and _stamp_ok(path, want):
+            return path
     return None
 
 
@@ -122,7 +141,7 @@ def build(verbose: bool = True, jobs: int | None = None) -> str:
 
     def compile_one(src: str) -> str:
         obj = os.path.join(obj_dir, os.path.basename(src)[:-4] + ".o")
-        cmd = [hipcc, *HIPCC_FLAGS, "-I", CSRC, "-I", sysconfig.get_paths()["include"], "-c", src, "-o", obj]
+        cmd = [hipcc, *HIPCC_FLAGS, "-I", CSRC, "-c", src, "-o", obj]
         proc = subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, env=env, text=True)
         last = time.time()
         while True:
@@ -152,7 +171,34 @@ def build(verbose: bool = True, jobs: int | None = None) -> str:
     with open(lib + ".stamp", "w", encoding="utf-8") as f:
         f.write(want + "\n")
     _say(f"built {lib} in {time.time() - t0:.0f} s", verbose)
+    build_call(verbose=verbose)
     return lib
+
+
+def build_call(verbose: bool = True) -> str | None:
+    """Compile the module that calls the library's entry points, for this Python.  Returns its path, or None where that does not go:
+    the calls go through ctypes then, some 3 us longer each."""
+    try:
+        out_dir = _writable_dir()
+        path = os.path.join(out_dir, CALL_NAME)
+        tmp = path + f".tmp{os.getpid()}"
+        cmd = [find_hipcc(), *CALL_FLAGS, "-I", sysconfig.get_paths()["include"], CALL_SOURCE, "-o", tmp]
+        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, env={"HOME": out_dir, **os.environ}, text=True)
+        if res.returncode != 0:
+            raise BuildError(f"hipcc failed on {CALL_SOURCE}:\n{res.stdout}")
+        os.replace(tmp, path)
+        with open(path + ".stamp", "w", encoding="utf-8") as f:
+            f.write(_call_hash() + "\n")
+    except (BuildError, OSError) as e:
+        _say(f"{CALL_NAME} is left out, kernels are called through ctypes: {e}", verbose)
+        return None
+    _say(f"built {path}", verbose)
+    return path
+
+
+def ensure_call(verbose: bool = True) -> str | None:
+    """The module for the current source and Python: the built one if there is one, else build it now; None where that does not go."""
+    return find_call() or build_call(verbose=verbose)
 
 
 def ensure_built(verbose: bool = True) -> str:

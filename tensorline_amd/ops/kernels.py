@@ -72,14 +72,43 @@ _enter = None
 
 
 def _entry_point(name: str) -> int:
-    """The address of a C entry point, for ``_enter``: ``enter(address, *arguments)`` of the library as a Python module (host_call.hip)."""
+    """The address of a C entry point, for ``_enter``: ``enter(address, *arguments)`` of the module that host_call.cpp is, or its twin here."""
     global _enter
     lib = library()
     if _enter is None:
-        loader = importlib.machinery.ExtensionFileLoader("libtensorline_hip", lib._name)
-        _enter = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader)).enter
+        path = _build.ensure_call()
+        if path is not None:
+            loader = importlib.machinery.ExtensionFileLoader("tensorline_call", path)
+            _enter = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader)).enter
+        else:
+            _enter = _enter_by_ctypes
     address = _entry_points[name] = ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
     return address
+
+
+_by_ctypes: dict[int, object] = {}      # functions, by address
+
+
+def _as_ctypes(a):
+    if a is None or isinstance(a, int):
+        return ctypes.c_longlong(a or 0)           # (a 32-bit parameter takes the low half)
+    if isinstance(a, float):
+        return ctypes.c_float(a)
+    if isinstance(a, ctypes.Structure):
+        return ctypes.byref(a)
+    if isinstance(a, ctypes._SimpleCData) and not isinstance(a, ctypes.c_double):
+        return a
+    if isinstance(a, torch.Tensor):
+        return ctypes.c_void_p(a.data_ptr())
+    raise TypeError(f"a kernel takes no argument of type {type(a).__name__}")
+
+
+def _enter_by_ctypes(address: int, *args) -> int:
+    """What the module's ``enter`` does, where there is no module."""
+    fn = _by_ctypes.get(address)
+    if fn is None:
+        fn = _by_ctypes[address] = ctypes.CFUNCTYPE(ctypes.c_int)(address)
+    return fn(*map(_as_ctypes, args))
 
 
 def _call(name: str, *args) -> None:

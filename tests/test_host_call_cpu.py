@@ -1,10 +1,12 @@
-"""How Python's arguments reach a C entry point (csrc/host_call.hip): by a callback of a known signature, on the CPU."""
+"""How Python's arguments reach a C entry point (csrc/host_call.cpp): by a callback of a known signature, on the CPU."""
 import ctypes
+import re
+import subprocess
 
 import pytest
 import torch
 
-from tensorline_amd.ops import kernels
+from tensorline_amd.ops import build, kernels
 
 
 class Pair(ctypes.Structure):
@@ -44,3 +46,28 @@ def test_as_many_arguments_as_there_is_room_for():
 def test_other_arguments_are_refused(bad):
     with pytest.raises((TypeError, AttributeError)):
         enter([ctypes.c_void_p], bad)
+
+
+def test_the_same_without_the_module(monkeypatch):
+    """Through ctypes: the same parameters are filled, the same arguments refused."""
+    kernels._entry_point("tl_last_error")
+    monkeypatch.setattr(kernels, "_enter", kernels._enter_by_ctypes)
+    test_arguments_of_every_kind_in_any_order()
+    seen, _ = enter([ctypes.c_int] * 56 + [ctypes.c_float] * 8, *range(56), *[k + 0.5 for k in range(8)])
+    assert seen == list(range(56)) + [k + 0.5 for k in range(8)]
+    for bad in ("text", b"", ctypes.c_double(1.0), [1], object(), (ctypes.c_int * 2)()):
+        test_other_arguments_are_refused(bad)
+
+
+def test_the_module_is_left_out_where_it_cannot_be_built(monkeypatch, tmp_path):
+    """No headers of Python: the library is built without them and loads without Python's symbols, calls go through ctypes."""
+    assert all(build.CALL_SOURCE != src for src in build.sources())
+    symbols = subprocess.run(["nm", "-D", "--undefined-only", build.ensure_built()], capture_output=True, text=True, check=True).stdout
+    assert "hipLaunchKernel" in symbols and not re.search(r"\b_?Py[A-Z_]", symbols)
+    monkeypatch.setattr(build, "_candidate_dirs", lambda: [str(tmp_path)])
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path / "none")})
+    assert build.find_call() is None and build.ensure_call(verbose=False) is None
+    monkeypatch.setattr(kernels, "_enter", None)
+    monkeypatch.setattr(build, "ensure_built", lambda: None)
+    kernels._entry_point("tl_last_error")
+    assert kernels._enter is kernels._enter_by_ctypes
