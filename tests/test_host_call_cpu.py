@@ -1,4 +1,5 @@
 """How Python's arguments reach a C entry point (csrc/host_call.cpp): by a callback of a known signature, on the CPU."""
+import ast
 import ctypes
 import re
 import subprocess
@@ -71,3 +72,66 @@ def test_the_module_is_left_out_where_it_cannot_be_built(monkeypatch, tmp_path):
     monkeypatch.setattr(build, "ensure_built", lambda: None)
     kernels._entry_point("tl_last_error")
     assert kernels._enter is kernels._enter_by_ctypes
+
+
+def _signatures():
+    """(name, a letter for each parameter: f float, w anything else) of the library's entry points that return a status."""
+    out = {}
+    for path in build.sources():
+        with open(path, encoding="utf-8") as f:
+            text = re.sub(r"//[^\n]*", "", f.read())
+        for name, params in re.findall(r'extern "C" int (tl_\w+)\(([^)]*)\)', text):
+            kinds = []
+            for p in params.split(","):
+                assert "*" in p or "double" not in p, (name, p)
+                kinds.append("f" if re.match(r"\s*(const\s+)?float\s+\w+\s*$", p) else "w")
+            out[name] = "".join(kinds)
+    return out
+
+
+def _kinds(args, scope, returns):
+    """The letters of a call's arguments: a float is a float literal, ``float(..)``, or a name that such a value was given to."""
+    out = ""
+    for a in args:
+        if isinstance(a, ast.Starred):
+            given = scope.get(a.value.id)
+            assert isinstance(given, ast.Tuple), f"line {a.lineno}: what *{a.value.id} holds is not seen"
+            out += _kinds(given.elts, scope, returns)
+        else:
+            if isinstance(a, ast.Name) and a.id in scope:
+                a = scope[a.id]
+            is_float = (isinstance(a, ast.Constant) and isinstance(a.value, float)) or (
+                isinstance(a, ast.Call) and isinstance(a.func, ast.Name) and a.func.id == "float")
+            out += "f" if is_float else "w"
+    return out
+
+
+def test_every_call_has_the_arguments_its_entry_point_takes():
+    """Neither the module nor ctypes knows an entry point's parameters: the calls in kernels.py are held against the sources, number
+    and kind of every argument."""
+    signatures, seen = _signatures(), 0
+    tree = ast.parse(open(kernels.__file__, encoding="utf-8").read())
+    functions = [n for n in tree.body if isinstance(n, ast.FunctionDef)]
+    returns = {f.name: [r.value for r in ast.walk(f) if isinstance(r, ast.Return) and r.value is not None] for f in functions}
+    for f in functions:
+        scope = {}                                       # names that hold a tuple or a float, in this function
+        for n in ast.walk(f):
+            if isinstance(n, ast.Assign):
+                for target in n.targets:
+                    if isinstance(target, ast.Name) and isinstance(n.value, (ast.Tuple, ast.Call)):
+                        scope[target.id] = n.value
+                    elif isinstance(target, ast.Tuple) and isinstance(n.value, ast.Call) and isinstance(n.value.func, ast.Name):
+                        for i, name in enumerate(target.elts):
+                            tuples = {ast.dump(ast.Tuple([ast.Constant(c) for c in _kinds(r.elts[i].elts, {}, returns)], ast.Load())): r.elts[i]
+                                      for r in returns.get(n.value.func.id, []) if isinstance(r, ast.Tuple) and isinstance(r.elts[i], ast.Tuple)}
+                            assert len(tuples) <= 1, f"line {n.lineno}: {name.id} holds arguments of several kinds"
+                            for given in tuples.values():
+                                scope[name.id] = given
+        for n in ast.walk(f):
+            if isinstance(n, ast.Call) and isinstance(n.func, ast.Name) and n.func.id == "_call" and isinstance(n.args[0], ast.Constant):
+                got = _kinds(n.args[1:], scope, returns)
+                assert got == signatures[n.args[0].value], f"kernels.py:{n.lineno}: {n.args[0].value} is given {got}"
+                seen += 1
+    assert seen > 50
+    wrong = ast.parse("_call('tl_scale_cap', z, n, scale, float(cap), _stream())").body[0].value
+    assert _kinds(wrong.args[1:], {}, returns) != signatures["tl_scale_cap"]
