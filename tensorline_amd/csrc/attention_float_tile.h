@@ -1,7 +1,8 @@
 // Float attention of steps with prompt portions (the 32-bit path's prefill): head sizes 64 and 128, pages of a power of two of at
 // least four tokens, no cap and no bias.  Products on v_mfma_f32_32x32x16_bf16, every float as the exact sum of three bfloat16 numbers
-// (8 + 8 + 8 significant bits, each the rest of the one before; Dekker, Numerische Mathematik 18, 1971), the six of the nine
-// partial products that matter, each exact, sums in float: nothing is held in 16 bits that the three parts together would not give back.
+// (8 + 8 + 8 significant bits, each the rest of the one before; Dekker, Numerische Mathematik 18, 1971).  Of the nine partial products of
+// two floats six are taken, each exact, with sums in float; the three left out (second by third part, third by second and by third) are at most 2^-24 of the
+// product they belong to.  Off 64 bits by 3.4e-7 in the 2-norm where the float instruction was by 4.5e-7 (2,048 tokens, 28 / 4 heads of 128).
 //
 // A work-group of four waves takes 128 columns, (token, query head) pairs of one sequence and key/value head in the order of the
 // tokens, a wave 32 of them; keys go by tiles of 32 at absolute multiples of 32.  A tile's keys, then its values, go from the cache
@@ -10,8 +11,9 @@
 // column, so the softmax crosses lanes once, and the weights are the second operand of the product with the values where they
 // are, if the values' fragments have their keys in the same order, which the split sees to.
 //
-// A tile that holds infinities, NaN or numbers beyond 2^60, or none above 2^-40 but zeros, and a wave's queries that do, go to the float
-// instruction (v_mfma_f32_32x32x2_f32) instead, from the cache, for the same result layout.
+// A tile that holds infinities, NaN or numbers beyond 2^60, or none above 2^-40 but zeros, goes to the float instruction
+// (v_mfma_f32_32x32x2_f32) instead, from the cache, for the same result layout; so does a column whose query does, and its neighbours stay as they are.
+// A column's bits do not depend on how its sequence is cut, then, unless a key or value behind its own position makes its tile such a one.
 //
 // What bounds it: a tile is a chain of some 4 us for a wave that has its SIMD to itself, 1.6 of them 96 matrix instructions, 0.9 some 430 vector
 // instructions (the splits of keys, values and weights 260 of them), the rest waits for values, fragments and the two barriers, which a second
@@ -91,7 +93,7 @@ __global__ __launch_bounds__(AFT_WAVES * 64, 2) void attn_float_tile_kernel(
     const float sign = scale < 0.f ? -1.f : 1.f, to_exp = fabsf(scale) * 1.44269504088896340736f;
 
     uint4 qf[KS][3];
-    bool odd_queries;
+    bool odd_query;                                      // this lane's column
     {
         const float* qrow = q + (size_t)(t0 + (real ? column / G : 0)) * q_stride + (size_t)(kvh * G + (real ? column % G : 0)) * D + 8 * h;
         float z = 0.f;
@@ -111,8 +113,11 @@ __global__ __launch_bounds__(AFT_WAVES * 64, 2) void attn_float_tile_kernel(
             aft_split(x, qf[ks]);
             if (ks < QL) qparts[(wave * QL + ks) * 64 + lane] = qf[ks][2];
         }
-        odd_queries = aft_odd(z);
+        const tl_u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(z), __float_as_uint(z), false, false);
+        z = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+        odd_query = !(z < 0x1p120f) || (z > 0.f && z < 0x1p-80f);
     }
+    const bool odd_queries = __any(odd_query);
     __syncthreads();
     int k_hi = 0, k_lo = 0x7fffffff;
 #pragma unroll
@@ -187,10 +192,11 @@ __global__ __launch_bounds__(AFT_WAVES * 64, 2) void attn_float_tile_kernel(
         const bool sees = k0 < w_hi && (k0 + AFT_KT > w_lo || k0 < mask.first);
         aft_f32x16 sc, sc2;
         if (sees) {
-            int slow = odd_queries;
+            int slow = 0;
 #pragma unroll
             for (int w = 0; w < AFT_WAVES; ++w) slow |= odd_keys[w];
-            if (__builtin_amdgcn_readfirstlane(slow) == 0) {
+            slow = __builtin_amdgcn_readfirstlane(slow);
+            if (slow == 0) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sc[r] = sc2[r] = 0.f;
                 uint4 a[2][3];
@@ -214,9 +220,10 @@ __global__ __launch_bounds__(AFT_WAVES * 64, 2) void attn_float_tile_kernel(
                 }
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sc[r] += sc2[r];
-            } else {
+            }
+            if (slow || odd_queries) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+                for (int r = 0; r < 16; ++r) sc2[r] = 0.f;
                 int here = lane & 31;
                 asm volatile("" : "+v"(here));           // nothing of this is made ahead of the loop
                 const bool there = k0 + here < k_hi;
@@ -224,7 +231,9 @@ __global__ __launch_bounds__(AFT_WAVES * 64, 2) void attn_float_tile_kernel(
                 const float* kp = k_cache + ((size_t)page_of(k0 + here) * bs + (last(k0 + here) & (bs - 1))) * nkv * D + (size_t)kvh * D + h;
                 const float* qp = q + (size_t)(t0 + (c < columns ? c / G : 0)) * q_stride + (size_t)(kvh * G + (c < columns ? c % G : 0)) * D + h;
                 for (int kk = 0; kk < D / 2; ++kk)       // head dimension 2 kk + h
-                    sc = __builtin_amdgcn_mfma_f32_32x32x2f32(there ? kp[2 * kk] : 0.f, c < columns ? qp[2 * kk] * sign : 0.f, sc, 0, 0, 0);
+                    sc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(there ? kp[2 * kk] : 0.f, c < columns ? qp[2 * kk] * sign : 0.f, sc2, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sc[r] = slow || odd_query ? sc2[r] : sc[r];
             }
         }
         // this tile's values, asked for as late as there is something to do until they come (registers)

@@ -2036,7 +2036,7 @@ def test_float_attention_of_prompt_portions(nq, nkv, d, bs, kw):
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("what", ["cut", "strided", "not finite", "tiny", "huge"])
 def test_float_attention_of_prompt_portions_at_their_limits(d, what):
-    """A position's bits do not depend on how its sequence is cut, nor on rows' strides.  Infinities and NaN in a key, a value or a query give
+    """A position's bits do not depend on how its sequence is cut (of finite numbers that are neither all tiny nor huge), nor on rows' strides.  Infinities and NaN in a key, a value or a query give
     what plain float arithmetic gives, in the tiles and columns that see them, and every other column stays as it is; values of
     2^-70 and 2^70 are as close to 64 bits as others."""
     torch.manual_seed(d)
@@ -2089,6 +2089,44 @@ def test_float_attention_of_prompt_portions_at_their_limits(d, what):
         q[40, 2 * d + 3] = float("nan")
         after, before = run(0, n).view(n, nq, d), None
         assert bool(after[40, 2].isnan().all()) and int(after.isnan().sum()) == d
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("odd", [float("nan"), float("inf"), 2.0 ** 70, 2.0 ** -60])
+def test_float_attention_beside_queries_of_another_size(d, odd):
+    """A query with NaN, an infinity or a number past 2^60, or a tiny one as a whole, leaves the bits of its neighbours among a wave's columns as they
+    are, however the sequence is cut; itself as close to 64 bits as others where its scores are numbers."""
+    from tensorline_amd.engine.batch import StepFacts
+    torch.manual_seed(d)
+    nq, nkv, bs, n = 6, 2, 16, 120
+    kc, vc = torch.randn(8, bs, nkv, d, device=DEV), torch.randn(8, nkv, d, bs, device=DEV)
+    table = torch.randperm(8, device=DEV).to(torch.int32)[None].contiguous()
+    q = torch.randn(n, nq, d, device=DEV)
+    def run(q, lo, hi):
+        i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+        facts = StepFacts(max_context=hi, max_query_len=hi - lo, decode_only=False, num_seqs=1, q_lens=[hi - lo], starts=[lo])
+        return K().paged_attention(q[lo:hi].reshape(hi - lo, nq * d), kc, vc, table, i32(*[0] * (hi - lo)), i32(*range(lo, hi)), nq, nkv, d, d ** -0.5,
+                                   q_start=i32(0, hi - lo), ctx_start=i32(lo), plan=facts).view(hi - lo, nq, d)
+    before, other = run(q, 0, n), q.clone()
+    at = ((3, 0), (40, 2), (41, 3), (90, 5))
+    for t, h in at:
+        if odd < 1.0:
+            other[t, h] *= odd
+        else:
+            other[t, h, 7] = odd
+    after, mine = run(other, 0, n), torch.zeros(n, nq, dtype=torch.bool, device=DEV)
+    for t, h in at:
+        mine[t, h] = True
+    assert torch.equal(after[~mine], before[~mine])
+    for cut in (20, 50, 100):
+        cuts = torch.cat((run(other, 0, cut), run(other, cut, n)))
+        assert torch.equal(cuts[~mine], before[~mine]) and torch.equal(cuts[mine].isnan(), after[mine].isnan())
+        assert odd != odd or torch.equal(cuts[mine].nan_to_num(), after[mine].nan_to_num())
+    if odd < 1.0:
+        rows = table[0].long()
+        kf, vf = kc[rows].view(-1, nkv, d)[:n].double().cpu(), vc[rows].permute(0, 3, 1, 2).reshape(-1, nkv, d)[:n].double().cpu()
+        want = plain.causal_attention(other.double().cpu(), kf, vf, d ** -0.5).to(DEV)
+        torch.testing.assert_close(after.double(), want, atol=2e-5, rtol=2e-5)
 
 
 @pytest.mark.parametrize("form", ["decay", "channels", "steps"])
