@@ -414,7 +414,8 @@ def add_rmsnorm(x: torch.Tensor, residual: "torch.Tensor | ShareSum | None", wei
 def _ordered(weight: torch.Tensor, step: int) -> torch.Tensor:
     """[N, K] as [ceil(N/16), ceil(K/step), 4, 16, step/4], zero where it pads; a quarter of a step is 16 bytes."""
     N, K = weight.shape
-    if weight.is_cuda and weight.is_contiguous() and N > 0 and K > 0 and K % (step // 4) == 0 and weight.data_ptr() % 16 == 0:
+    if (weight.is_cuda and weight.is_contiguous() and N > 0 and K > 0 and K % (step // 4) == 0 and weight.data_ptr() % 16 == 0
+            and weight.get_device() == torch._C._cuda_getDevice()):          # (a matrix of another GPU than the current one goes to torch)
         out = torch.empty(-(-N // 16), -(-K // step), 4, 16, step // 4, dtype=weight.dtype, device=weight.device)
         _call("tl_order_weight", weight, out, N, K // (step // 4), _stream())
         return out

@@ -1677,6 +1677,17 @@ def test_ordered_copy_of_a_matrix(N, Kd, dtype, step):
     assert torch.equal(make(torch.cat([w, w], 1)[:, :Kd]), want)
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_ordered_copy_of_a_matrix_on_another_gpu(dtype, monkeypatch):
+    """Where the matrix is not on the current GPU, whose stream a kernel of ours would run on, the copy is torch's, the same."""
+    w = torch.randn(33, 72, device=DEV).to(getattr(torch, dtype))
+    make = K().shuffle_weight if dtype == "bfloat16" else K().shuffle_weight_float
+    want, calls = make(w), []
+    monkeypatch.setattr(K(), "_call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 1)
+    assert torch.equal(make(w), want) and not calls
+
+
 @pytest.mark.parametrize("T,B,N,Kd", [(1, 2, 16, 8), (31, 3, 48, 40), (33, 2, 192, 128), (130, 1, 112, 96), (2049, 32, 128, 192), (257, 32, 272, 192),
                                       (1300, 43, 128, 128)])
 def test_batched_linear_by_whole_rows_and_not(T, B, N, Kd):
