@@ -11,7 +11,7 @@
 // column, so the softmax crosses lanes once, and the weights are the second operand of the product with the values where they
 // are, if the values' fragments have their keys in the same order, which the split sees to.
 //
-// A tile that holds infinities, NaN or numbers beyond 2^60, or none above 2^-40 but zeros, goes to the float instruction
+// A tile that holds infinities, NaN or numbers beyond 2^60, or none above 2^-40 but zeros, or of values one below 2^-110, goes to the float instruction
 // (v_mfma_f32_32x32x2_f32) instead, from the cache, for the same result layout; so does a column whose query does, and its neighbours stay as they are.
 // A column's bits do not depend on how its sequence is cut, then, unless a key or value behind its own position makes its tile such a one.
 //
@@ -49,12 +49,20 @@ __device__ __forceinline__ void aft_split(float (&x)[8], uint4 (&to)[3]) {
     to[2] = make_uint4(aft_rest(x[0], x[1]), aft_rest(x[2], x[3]), aft_rest(x[4], x[5]), aft_rest(x[6], x[7]));
 }
 // the sum of squares shows infinities, NaN and numbers past 2^60, and that those that are not zero are below 2^-40 (below 2^-75 it does not, but
-// three parts hold numbers down to 2^-110)
+// three parts hold numbers down to 2^-110, and keys below that give scores of nothing with any query that has parts)
 __device__ __forceinline__ void aft_squares(const float (&x)[8], float& z) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) z = __builtin_fmaf(x[i], x[i], z);
 }
 __device__ __forceinline__ bool aft_odd(float z) { return __any(!(z < 0x1p120f)) || (__any(z > 0.f) && !__any(z >= 0x1p-80f)); }
+
+// A value below 2^-110 that is not zero: a head dimension may have no others, and the third part no longer holds its last bits (up to 6e-3 of a
+// value of 2^-126).  The smallest of twice a number's bits less one, in which zero comes last.
+__device__ __forceinline__ void aft_least(const float (&x)[8], uint32_t& least) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) least = min(least, (__float_as_uint(x[i]) << 1) - 1u);
+}
+__device__ __forceinline__ bool aft_tiny(uint32_t least) { return __any(least < (__float_as_uint(0x1p-110f) << 1) - 1u); }
 
 #define AFT_MUL(ACC, A_, B_) \
     ACC = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(aft_bf16x8, A_), __builtin_bit_cast(aft_bf16x8, B_), ACC, 0, 0, 0)
@@ -279,6 +287,7 @@ __global__ __launch_bounds__(AFT_WAVES * 64, 2) void attn_float_tile_kernel(
         }
         {
             float z = 0.f;
+            uint32_t least = ~0u;
 #pragma unroll
             for (int u = 0; u < VU; ++u) {
                 const int unit = wave * VU + u;
@@ -289,12 +298,13 @@ __global__ __launch_bounds__(AFT_WAVES * 64, 2) void attn_float_tile_kernel(
                     for (int e = 0; e < 8; ++e) x[e] = k0 + 16 * (unit & 1) + 8 * (e >> 2) + 4 * h + (e & 3) < k_hi ? x[e] : 0.f;
                 }
                 aft_squares(x, z);
+                aft_least(x, least);
                 uint4 parts[3];
                 aft_split(x, parts);
 #pragma unroll
                 for (int t = 0; t < 3; ++t) vparts[(unit * 3 + t) * 64 + lane] = parts[t];
             }
-            const bool odd = aft_odd(z);
+            const bool odd = aft_odd(z) || aft_tiny(least);
             if (lane == 0) odd_values[wave] = odd;
         }
         // the next tile's keys

@@ -2140,6 +2140,28 @@ def test_float_attention_beside_queries_of_another_size(d, odd):
         torch.testing.assert_close(after.double(), want, atol=2e-5, rtol=2e-5)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("size", [-20, -76, -109, -112, -118, -126])
+@pytest.mark.parametrize("dims", ["one", "all"])
+def test_float_attention_of_values_of_every_size(d, size, dims):
+    """A head dimension whose values are all some power of two, down to the smallest normal float, beside others or alone: as close to 64 bits as any,
+    where what is left of 24 bits is a normal float (a result below 2^-126 is off by up to 2^-149)."""
+    torch.manual_seed(d)
+    nq, bs, n = 2, 16, 96
+    kc, vc = torch.randn(6, bs, nq, d, device=DEV), torch.rand(6, nq, d, bs, device=DEV) + 1.0
+    at = slice(None) if dims == "all" else 5
+    vc[:, :, at] *= 2.0 ** size
+    table, q = torch.randperm(6, device=DEV).to(torch.int32)[None].contiguous(), torch.randn(n, nq, d, device=DEV)
+    from tensorline_amd.engine.batch import StepFacts
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    facts = StepFacts(max_context=n, max_query_len=n, decode_only=False, num_seqs=1, q_lens=[n], starts=[0])
+    got = K().paged_attention(q.view(n, nq * d), kc, vc, table, i32([0] * n), i32(list(range(n))), nq, nq, d, d ** -0.5,
+                              q_start=i32([0, n]), ctx_start=i32([0]), plan=facts).view(n, nq, d)
+    rows = table[0].long()
+    want = plain.causal_attention(q.double().cpu(), kc[rows].view(-1, nq, d).double().cpu(), vc[rows].permute(0, 3, 1, 2).reshape(-1, nq, d).double().cpu(), d ** -0.5).to(DEV)
+    torch.testing.assert_close(got.double()[:, :, at] * 2.0 ** -size, want[:, :, at] * 2.0 ** -size, atol=2.0 ** (-149 - size), rtol=2e-6)
+
+
 @pytest.mark.parametrize("form", ["decay", "channels", "steps"])
 @pytest.mark.parametrize("dk,dv", [(16, 16), (24, 40), (64, 64), (128, 17)])
 def test_recurrences_of_portions_with_helping_waves(form, dk, dv):
