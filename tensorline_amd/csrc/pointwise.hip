@@ -1064,7 +1064,7 @@ __global__ __launch_bounds__(256) void head_norm_rotate_store_kernel(
             }
         };
         if (!keep) continue;
-        if constexpr (LANES == 64) {
+        if (LANES == 64 && !pairs) {                              // (single stores come together behind the rotation)
             float y[2 * NQ];
 #pragma unroll
             for (int j = 0; j < NQ; ++j) turn(j, y[2 * j], y[2 * j + 1]);
