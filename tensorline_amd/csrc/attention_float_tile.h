@@ -13,6 +13,7 @@
 //
 // A tile that holds infinities, NaN or numbers beyond 2^60, or none above 2^-40 but zeros, or of values one below 2^-110, goes to the float instruction
 // (v_mfma_f32_32x32x2_f32) instead, from the cache, for the same result layout; so does a column whose query does, and its neighbours stay as they are.
+// (Weights below 2^-110 of a column's largest so far keep fewer bits, off by 2^-134 of that one.)
 // A column's bits do not depend on how its sequence is cut, then, unless a key or value behind its own position makes its tile such a one.
 //
 // What bounds it: a tile is a chain of some 4 us for a wave that has its SIMD to itself, 1.6 of them 96 matrix instructions, 0.9 some 430 vector
